@@ -110,6 +110,7 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 _build_failure = None
 
 
@@ -155,6 +156,29 @@ def load():
             raise RuntimeError(f"libtlq.so ABI version {lib.tlq_abi_version()} != expected {ABI_VERSION}")
         _lib = lib
     return _lib
+
+
+def host():
+    """The extension module tlq_host (csrc/host_calls.cpp), bound to the loaded libtlq: builds kernel objects' native calls.
+    Like the library it has no substitute: if it cannot be loaded this raises."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is None:
+            import importlib.machinery
+            import importlib.util
+
+            path = _build.HOST_PATH
+            if not os.path.exists(path):
+                _build.build_library(force=False)
+            spec = importlib.util.spec_from_file_location("tlq_host", path, loader=importlib.machinery.ExtensionFileLoader("tlq_host", path))
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES})
+            _host = mod
+    return _host
 
 
 def last_error() -> str:
@@ -211,18 +235,3 @@ def tuning(w4a16_tile: int = 0, i8_tile: int = 0, gemv: tuple = None, skinny: tu
                 lib.tlq_tune_gemv_depth(0)
             if skinny:
                 lib.tlq_tune_w4a16_skinny(0, 0)
-
-
-def scratch(nbytes: int, device, stream: int):
-    """A per-call workspace of `nbytes` bytes from torch's caching allocator, safe to hand to a kernel launched on the raw
-    stream `stream`: the allocator orders reuse of a block by the stream that was current when it was allocated, so when
-    the launch stream is another one the block is recorded on it (otherwise the block could be handed out again, on the
-    current stream, while the kernel still writes it).  None for nbytes == 0."""
-    import torch
-
-    if not nbytes:
-        return None
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    if stream and stream != torch.cuda.current_stream(ws.device).cuda_stream:
-        ws.record_stream(torch.cuda.ExternalStream(stream, device=ws.device))
-    return ws

@@ -1,11 +1,12 @@
-"""Builds libtlq.so (HIP kernels + C ABI) for gfx950 with hipcc, in-tree.
+"""Builds libtlq.so (HIP kernels + C ABI) for gfx950 with hipcc and tlq_host.so (the extension module that calls it), in-tree.
 
     python -m tilelang_ascend_amd.build [--force]
 
 Mirrors the role of the reference's LibraryGenerator.compile_lib
 (tilelang/jit/adapter/libgen.py:106-232: write source, shell out to the device compiler,
 produce a .so that ctypes loads), except that the kernels are fixed sources rather than
-generated ones, so there is one library for all operators.
+generated ones, so there is one library for all operators (and one extension module in the place of the reference's Cython
+wrapper, tilelang/jit/adapter/cython/cython_wrapper.pyx).
 """
 from __future__ import annotations
 
@@ -25,6 +26,7 @@ INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 LIB_PATH = os.path.join(LIB_DIR, "libtlq.so")
+HOST_PATH = os.path.join(LIB_DIR, "tlq_host.so")
 
 ARCH = "gfx950"
 SOURCES = [
@@ -65,6 +67,11 @@ HIPCC_FLAGS = [
 ]
 
 
+# the extension module through which Python makes the calls (csrc/host_calls.cpp): host code against torch's C++ headers
+HOST_SOURCE = "host_calls.cpp"
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{INCLUDE_DIR}"]
+
+
 def hipcc_path() -> str:
     for cand in (os.environ.get("HIPCC"), shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
         if cand and os.path.exists(cand):
@@ -76,7 +83,7 @@ def source_fingerprint() -> str:
     """sha256 over kernel sources, headers and flags -- the analogue of the reference's kernel
     cache key (tilelang/cache/kernel_cache.py:71-117: hash of source + target + options)."""
     h = hashlib.sha256()
-    h.update(" ".join(HIPCC_FLAGS).encode())
+    h.update(" ".join(HIPCC_FLAGS + HOST_FLAGS).encode())
     names = sorted(os.listdir(CSRC_DIR)) + ["../../include/tlq.h", "../../include/tlq_debug.h"]
     for name in names:
         path = os.path.join(CSRC_DIR, name)
@@ -100,6 +107,26 @@ def _compile_one(src: str, verbose: bool) -> str:
     if verbose and out.strip():
         print(out)
     return obj
+
+
+def _compile_host() -> str:
+    """tlq_host.so for the running interpreter and torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = HOST_PATH + ".tmp"
+    rocm = os.path.dirname(os.path.dirname(hipcc_path()))
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    includes = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = [shutil.which("g++") or "g++", *HOST_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in includes), os.path.join(CSRC_DIR, HOST_SOURCE), "-o", tmp, f"-L{torch_lib}",
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"Compilation Failed! {' '.join(cmd)}\n{res.stdout}")
+    return tmp
 
 
 STAMP_PATH = os.path.join(LIB_DIR, "libtlq.fingerprint")
@@ -153,20 +180,23 @@ def _build_locked(force: bool, verbose: bool, jobs: int) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     stamp = STAMP_PATH
     fp = source_fingerprint()
-    if not force and is_current():
+    if not force and is_current() and os.path.exists(HOST_PATH):
         return LIB_PATH
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC_DIR, s))]
     missing = sorted(set(SOURCES) - set(srcs))
     if missing:
         raise RuntimeError(f"kernel sources missing: {missing}")
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host)
         objs = list(pool.map(lambda s: _compile_one(s, verbose), srcs))
+        host_tmp = host.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc_path(), "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp, *objs]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"Compilation Failed! {' '.join(cmd)}\n{res.stdout}")
     os.replace(tmp, LIB_PATH)
+    os.replace(host_tmp, HOST_PATH)
     with open(stamp, "w") as f:
         f.write(fp + "\n")
     return LIB_PATH

@@ -3,6 +3,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
+
 #include "tlq_common.h"
 
 namespace tlq {
@@ -69,8 +71,15 @@ const char* tlq_debug_launch_log_text(void) { return tlq::g_log; }
 int tlq_device_cu_count(void) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
+  // (every plan of a kernel choice asks, a dozen times per call: the count of a device does not change while it is there)
+  static std::atomic<int> counts[64];
+  if (dev >= 0 && dev < 64) {
+    const int known = counts[dev].load(std::memory_order_relaxed);
+    if (known > 0) return known;
+  }
   int n = 0;
   if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  if (dev >= 0 && dev < 64) counts[dev].store(n, std::memory_order_relaxed);
   return n;
 }
 

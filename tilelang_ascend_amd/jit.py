@@ -5,6 +5,8 @@ Reference behaviour mirrored here (paths relative to the reference checkout):
 * ``@tilelang.jit(out_idx=..., workspace_idx=..., pass_configs=...)`` decorates a *factory*;
   calling the factory returns a kernel, memoised per ``(args, sorted kwargs)``
   (tilelang/jit/__init__.py:197-247).
+* the ordinary call runs in an extension module (csrc/host_calls.cpp), as the reference's runs in Cython; ``forward`` below
+  is the same contract in Python, for an explicit stream, another device, and to name what is wrong with a call;
 * ``kernel(*inputs, stream=-1)`` consumes the parameters that are neither outputs nor
   workspaces positionally, allocates outputs with ``torch.empty(shape, dtype,
   device=inputs[0].device)``, validates contiguity / device / dtype, launches on the current
@@ -48,6 +50,9 @@ ABI_DTYPE = {
     torch.int32: _abi.I32,
 }
 
+# the extension module's type codes: those of the C ABI, and one for packed weights
+_NATIVE_DTYPE = {name: ABI_DTYPE.get(t, 5) for name, t in TORCH_DTYPES.items()}
+
 
 class PassConfigKey(str, enum.Enum):
     """Names of tilelang/transform/pass_config.py:8-79 that the quantized-matmul examples pass.
@@ -73,13 +78,26 @@ class Param:
 
 
 @dataclass
+class NativeCall:
+    """The call of one C entry point, made by the extension module: which one (``kind``) and its integers in the order
+    csrc/host_calls.cpp takes them (-1: the size of the symbolic dimension), the scalar zero point where there is one.
+    tuning: choices of _abi.tuning that are applied around the call.  before: run once, before the first call."""
+
+    kind: str
+    ints: Tuple[int, ...]
+    zero: float = 0.0
+    tuning: Optional[Dict[str, Any]] = None
+    before: Optional[Callable[[], None]] = None
+
+
+@dataclass
 class KernelSpec:
-    """What a factory hands to ``jit``: the parameter list in the reference's order and the
-    launch function ``launch(tensors, symbols, stream)`` that calls the C ABI."""
+    """What a factory hands to ``jit``: the parameter list in the reference's order and the launch: a NativeCall, or a
+    function ``launch(tensors, symbols, stream)``."""
 
     name: str
     params: List[Param]
-    launch: Callable[[List[Optional[torch.Tensor]], Dict[str, int], int], None]
+    launch: Union[NativeCall, Callable[[List[Optional[torch.Tensor]], Dict[str, int], int], None]]
     attrs: Dict[str, Any] = field(default_factory=dict)
 
 
@@ -114,6 +132,8 @@ class JITKernel:
         self.execution_backend = execution_backend
         self.input_idx = [i for i in range(n) if i not in self.result_idx and i not in self.workspace_idx]
         self._tuner_result = None
+        self._plan = None
+        self._fast = self._first_call
 
     # -- introspection kept for drop-in use ----------------------------------------------
     @property
@@ -133,6 +153,34 @@ class JITKernel:
         return Profiler(self)
 
     # -- the launch contract -----------------------------------------------------------------
+    def _native_plan(self):
+        """The extension module's Plan of this kernel (its parameter list and call), made once."""
+        if self._plan is None:
+            call = self.spec.launch
+            if call.before is not None:
+                call.before()
+            params = tuple((tuple(p.shape), _NATIVE_DTYPE[p.dtype], 2 if i in self.workspace_idx else 1 if i in self.result_idx else 0)
+                           for i, p in enumerate(self.params))
+            self._plan = _abi.host().Plan(call.kind, params, tuple(int(i) for i in call.ints), float(call.zero))
+        return self._plan
+
+    def _first_call(self, *args):
+        """From the first call on ``_fast`` is the Plan itself: the ordinary call in native code, NotImplemented for
+        everything that ``forward`` has to look at."""
+        call = self.spec.launch
+        if not isinstance(call, NativeCall) or call.tuning or not torch.cuda.is_available():
+            return NotImplemented
+        torch.cuda.current_stream()  # (initialises torch's GPU state, which the extension module takes for granted)
+        self._fast = self._native_plan()
+        return self._fast(*args)
+
+    def _launch(self, tensors, symbols, stream):
+        call = self.spec.launch
+        if not isinstance(call, NativeCall):
+            return call(tensors, symbols, stream)
+        with _abi.tuning(**(call.tuning or {})):
+            self._native_plan().launch(tensors, stream)
+
     def _resolve(self, inputs: Sequence[torch.Tensor]) -> Dict[str, int]:
         symbols: Dict[str, int] = {}
         for pos, pi in enumerate(self.input_idx):
@@ -205,12 +253,16 @@ class JITKernel:
                 f"Buffer device mismatch for parameter {self.params[0].name}: expected a ROCm device ('cuda'), got {device}"
             )
         with torch.cuda.device(device):
-            self.spec.launch(tensors, symbols, stream)
+            self._launch(tensors, symbols, stream)
         if len(self.result_idx) == 1:
             return tensors[self.result_idx[0]]
         return [tensors[i] for i in self.result_idx]
 
     def __call__(self, *args, stream: int = -1):
+        if stream == -1:
+            out = self._fast(*args)
+            if out is not NotImplemented:
+                return out
         return self.forward(list(args), stream=stream)
 
 

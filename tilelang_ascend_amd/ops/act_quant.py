@@ -18,8 +18,7 @@ from __future__ import annotations
 
 from typing import Literal
 
-from .. import _abi
-from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, Param, PassConfigKey, jit
+from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, NativeCall, Param, PassConfigKey, jit
 
 _PASS_CONFIGS = {
     PassConfigKey.TL_ASCEND_AUTO_SYNC: True,
@@ -34,12 +33,6 @@ def act_quant_kernel_int8_optimized(N: int, block_M: int = 32, block_N: int = 32
     if N <= 0:
         raise ValueError("N must be positive")
     tin = ABI_DTYPE[TORCH_DTYPES[in_dtype]]
-
-    def launch(t, sym, stream):
-        X, Y, S = t
-        _abi.check(_abi.load().tlq_act_quant_i8(_abi.ptr(X), _abi.ptr(Y), _abi.ptr(S), sym["M"], N, tin,
-                                                1 if round_scale else 0, stream))
-
     return KernelSpec("act_quant_kernel_int8_optimized",
                       [Param("X", ("M", N), in_dtype), Param("Y", ("M", N), "int8"), Param("S", ("M",), "float32")],
-                      launch, {"block": (block_M, block_N), "round_scale": bool(round_scale)})
+                      NativeCall("act_quant", (N, tin, bool(round_scale))), {"block": (block_M, block_N), "round_scale": bool(round_scale)})

@@ -17,7 +17,7 @@ from typing import Optional, Union
 import torch
 
 from .. import _abi
-from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, Param, PassConfigKey, jit
+from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, NativeCall, Param, PassConfigKey, jit
 
 _PASS_CONFIGS = {
     PassConfigKey.TL_ASCEND_AUTO_CV_COMBINE: True,
@@ -48,6 +48,10 @@ def unpack_int4(tensor: torch.Tensor, out_dtype: torch.dtype = torch.int8, sign_
     """uint8 [N, K/2] -> [N, K] of out_dtype (int8 / float16 / bfloat16).  Element k of row n is
     nibble k % 2 of byte k // 2, low nibble first.  sign_mode: 'unsigned' (0..15), 'twos'
     (two's complement -8..7), 'offset8' (u-8), 'offset7' (u-7)."""
+    if isinstance(tensor, torch.Tensor) and tensor.is_cuda and out_dtype in ABI_DTYPE and sign_mode in _SIGN_MODES:
+        out = _abi.host().unpack(tensor, ABI_DTYPE[out_dtype], _SIGN_MODES[sign_mode])  # the ordinary call
+        if out is not NotImplemented:
+            return out
     if tensor.dtype != torch.uint8 or tensor.dim() != 2:
         raise ValueError(f"packed weights must be a 2-D uint8 tensor, got {tensor.dtype} {tuple(tensor.shape)}")
     if not tensor.is_contiguous():
@@ -84,10 +88,14 @@ def dequantize_w4(B_packed: torch.Tensor, scales: Optional[torch.Tensor] = None,
     """W[n, k] = rn( rn(T(u[n,k]) - z[n, k//g]) * s[n, k//g] ), T = dtype, as a [N, K] tensor.
     scales: [N, K/g] of dtype or None (=1).  zeros: None (=0), a number, or [N, K/g] of dtype.
     weight_layout: "plain", or "interleaved" for words repacked by interleave_weight(target float16)."""
+    z_t, z_s = _split_zero(zeros)
+    if isinstance(B_packed, torch.Tensor) and B_packed.is_cuda and dtype in (torch.float16, torch.bfloat16) and weight_layout in _LAYOUTS:
+        out = _abi.host().dequantize(B_packed, scales, z_t, z_s, group_size, ABI_DTYPE[dtype], _LAYOUTS[weight_layout])  # the ordinary call
+        if out is not NotImplemented:
+            return out
     _require_cuda(B_packed, "B_packed")
     N, Kp = B_packed.shape
     K = Kp * 2
-    z_t, z_s = _split_zero(zeros)
     _check_group_tensor(scales, "scales", N, K, group_size, dtype)
     _check_group_tensor(z_t, "zeros", N, K, group_size, dtype)
     out = torch.empty(N, K, dtype=dtype, device=B_packed.device)
@@ -125,38 +133,30 @@ def _check_group_tensor(t, name, N, K, group, dtype):
 def fp16_gemm(M: int, N: int, K: int, block_M: int, block_N: int, block_K: int):
     """fine_grained.py:60-115: C[M,N] f16 = A[M,K] f16 . B[K,N] f16, fp32 accumulate.  The block
     sizes are accepted for signature compatibility; tiling is chosen by the library."""
-
-    def launch(t, sym, stream):
-        A, B, C = t
-        lib = _abi.load()
-        # few activation rows: K slices with their fp32 matrices in a workspace (allocated per call, like the
-        # reference's workspace_idx buffers); 0 bytes for every other shape
-        ws_bytes = lib.tlq_f16_workspace_bytes(1, M, N, K)
-        ws = _abi.scratch(ws_bytes, A.device, stream)
-        _abi.check(lib.tlq_gemm_f16_ws(_abi.ptr(A), _abi.ptr(B), _abi.ptr(C), _abi.ptr(ws), ws_bytes, 1, M, N, K, _abi.F16,
-                                       _abi.F16, _abi.B_KN, stream))
-
+    # (few activation rows: K slices with their fp32 matrices in a workspace, allocated per call like the reference's
+    # workspace_idx buffers)
     return KernelSpec("fp16_gemm", [Param("A", (M, K), "float16"), Param("B", (K, N), "float16"),
-                                    Param("C", (M, N), "float16")], launch,
+                                    Param("C", (M, N), "float16")], NativeCall("f16", (M, N, K)),
                       {"block": (block_M, block_N, block_K)})
 
 
 @jit(out_idx=[-1], pass_configs=_PASS_CONFIGS)
 def int8_gemm(M: int, N: int, K: int, block_M: int, block_N: int, block_K: int):
     """fine_grained.py:118-173: C[M,N] i32 = A[M,K] i8 . B[K,N] i8, int32 accumulate (exact)."""
-
-    def launch(t, sym, stream):
-        A, B, C = t
-        _abi.check(_abi.load().tlq_gemm_i8(_abi.ptr(A), _abi.ptr(B), _abi.ptr(C), 1, M, N, K, _abi.B_KN, stream))
-
     return KernelSpec("int8_gemm", [Param("A", (M, K), "int8"), Param("B", (K, N), "int8"),
-                                    Param("C", (M, N), "int32")], launch,
+                                    Param("C", (M, N), "int32")], NativeCall("i8", (M, N, K)),
                       {"block": (block_M, block_N, block_K)})
 
 
 # ------------------------------------------------------------------------------------------
 # fused W4A16
 # ------------------------------------------------------------------------------------------
+def _load_tuned_choices() -> None:
+    from ..autotuner import ensure_w4a16_choices_loaded
+
+    ensure_w4a16_choices_loaded()  # (once per process: the device's persisted tuned choices, if any)
+
+
 @jit(out_idx=[-1], pass_configs=_PASS_CONFIGS)
 def w4a16_gemm(M: int, N: int, K: int, block_M: int = 128, block_N: int = 256, block_K: int = 64,
                in_dtype: str = "float16", out_dtype: str = "float16", group_size: int = 128,
@@ -177,7 +177,7 @@ def w4a16_gemm(M: int, N: int, K: int, block_M: int = 128, block_N: int = 256, b
     TLQ_TUNED_CHOICES=0).  A workspace
     (split-K partial sums or the [N, K] dequantised weights) is taken from torch's stream-ordered allocator on every
     call, as the reference allocates its workspace_idx buffers per call, so launches on different streams do not share one;
-    when the launch stream (forward(stream=...)) is not torch's current stream the block is recorded on it (_abi.scratch).
+    when the launch stream (forward(stream=...)) is not torch's current stream the block is recorded on it.
     weight_layout: "plain" (general_compress order) or "interleaved" (B_packed went through interleave_weight for the
     float16 target, e.g. quantize.gpu.pack_int4(..., interleave="float16")); interleaved weights are read by the "gemv" (one row,
     two fp16 rows), "decode", "stream" and panel kernels and the two passes, with results bit-identical to the plain layout
@@ -205,37 +205,11 @@ def w4a16_gemm(M: int, N: int, K: int, block_M: int = 128, block_N: int = 256, b
         params.append(Param("zeros", (N, G), in_dtype))
     params.append(Param("C", (M, N), out_dtype))
     tin, tout = ABI_DTYPE[TORCH_DTYPES[in_dtype]], ABI_DTYPE[TORCH_DTYPES[out_dtype]]
-    algo_code = _ALGOS[algo]
-    layout_code = _LAYOUTS[weight_layout]
-
-    def launch(t, sym, stream):
-        A, Bp = t[0], t[1]
-        i = 2
-        S = Z = None
-        if with_scales:
-            S = t[i]
-            i += 1
-        if zeros_tensor:
-            Z = t[i]
-            i += 1
-        C = t[i]
-        lib = _abi.load()
-        ws = None
-        if algo == "auto":
-            from ..autotuner import ensure_w4a16_choices_loaded
-            ensure_w4a16_choices_loaded()  # (once per process: the device's persisted tuned choices, if any)
-        # what the named family asks for ("auto": the rule-based choice and any tuned choice for this shape)
-        ws_bytes = lib.tlq_w4a16_workspace_bytes_for(M, N, K, algo_code)
-        if layout_code != _abi.W_PLAIN and algo == "auto" and M > 256:
-            ws_bytes = max(ws_bytes, N * K * 2)
-        if ws_bytes:
-            ws = _abi.scratch(ws_bytes, A.device, stream)
-        with _abi.tuning(w4a16_tile=tile, gemv=gemv_tuning, skinny=skinny_tuning):
-            _abi.check(lib.tlq_gemm_w4a16_layout_ws(_abi.ptr(A), _abi.ptr(Bp), _abi.ptr(S), _abi.ptr(Z), _abi.ptr(C), M, N, K,
-                                                    group_size, zero_scalar, tin, tout, algo_code, layout_code, _abi.ptr(ws),
-                                                    ws_bytes, stream))
-
-    return KernelSpec("w4a16_gemm", params, launch,
+    tuning = {k: v for k, v in (("w4a16_tile", tile), ("gemv", gemv_tuning), ("skinny", skinny_tuning)) if v}
+    # the workspace is what the named family asks for ("auto": the rule-based choice and any tuned choice for this shape)
+    call = NativeCall("w4a16", (M, N, K, group_size, tin, tout, _ALGOS[algo], _LAYOUTS[weight_layout], with_scales, zeros_tensor),
+                      zero_scalar, tuning, _load_tuned_choices if algo == "auto" else None)
+    return KernelSpec("w4a16_gemm", params, call,
                       {"block": (block_M, block_N, block_K), "group": group_size, "zeros": zeros, "algo": algo,
                        "tile": tile, "gemv_tuning": gemv_tuning, "skinny_tuning": skinny_tuning,
                        "weight_layout": weight_layout})
@@ -258,17 +232,20 @@ def dequant_gemm_fp16_wrapper(M: int, N: int, K: int, block_M: int, block_N: int
 
     def wrapper(A: torch.Tensor, B_packed: torch.Tensor, scales: Optional[torch.Tensor] = None,
                 zeros: Union[None, float, int, torch.Tensor] = None):
-        on_cpu = A.device.type != "cuda"
         z_is_tensor = isinstance(zeros, torch.Tensor)
         key = (scales is not None, "tensor" if z_is_tensor else zeros)
-        if key not in kernels:
-            kernels[key] = w4a16_gemm(M, N, K, block_M, block_N, block_K, input_dtype, output_dtype, group_size,
-                                      scales is not None, key[1], algo, weight_layout=weight_layout)
-        args = [A, B_packed] + ([scales] if scales is not None else []) + ([zeros] if z_is_tensor else [])
-        if on_cpu:
-            args = [a.cuda() for a in args]
-        C = kernels[key](*args)
-        return C.cpu() if on_cpu else C
+        kernel = kernels.get(key)
+        if kernel is None:
+            kernel = kernels[key] = w4a16_gemm(M, N, K, block_M, block_N, block_K, input_dtype, output_dtype, group_size,
+                                               scales is not None, key[1], algo, weight_layout=weight_layout)
+        args = [A, B_packed]
+        if scales is not None:
+            args.append(scales)
+        if z_is_tensor:
+            args.append(zeros)
+        if A.is_cuda:
+            return kernel(*args)
+        return kernel(*[a.cuda() for a in args]).cpu()
 
     return wrapper
 
@@ -292,11 +269,6 @@ def dequant_gemm_int8_wrapper(M: int, N: int, K: int, block_M: int, block_N: int
 
 @jit(out_idx=[-1], pass_configs=_PASS_CONFIGS)
 def _w4a8_kernel(M: int, N: int, K: int, sign_mode: str):
-    mode = _SIGN_MODES[sign_mode]
-
-    def launch(t, sym, stream):
-        A, Bp, C = t
-        _abi.check(_abi.load().tlq_gemm_w4a8(_abi.ptr(A), _abi.ptr(Bp), _abi.ptr(C), M, N, K, mode, stream))
-
+    call = NativeCall("w4a8", (M, N, K, _SIGN_MODES[sign_mode]))
     return KernelSpec("w4a8_gemm", [Param("A", (M, K), "int8"), Param("B_packed", (N, K // 2), "uint8"),
-                                    Param("C", (M, N), "int32")], launch, {"sign": sign_mode})
+                                    Param("C", (M, N), "int32")], call, {"sign": sign_mode})

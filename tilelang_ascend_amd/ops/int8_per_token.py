@@ -18,7 +18,7 @@ from typing import Literal
 
 from .. import _abi
 from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, Param, PassConfigKey, jit
-from .quant_matmul import w8a8_launch
+from .quant_matmul import w8a8_call
 
 _PASS_CONFIGS = {
     PassConfigKey.TL_ASCEND_AUTO_SYNC: True,
@@ -41,16 +41,11 @@ def int8_gemm_kernel_corrected(N: int, K: int, block_M: int = 32, block_N: int =
     if in_dtype != "int8" or accum_dtype != "int32" or scale_dtype != "float32":
         raise ValueError("only int8 inputs, int32 accumulation and float32 scales are supported")
     tout = ABI_DTYPE[TORCH_DTYPES[out_dtype]]
-
-    def launch(t, sym, stream):
-        A, B, sa, sb, C, _ws = t
-        with _abi.tuning(i8_tile=tile):
-            w8a8_launch(A, B, sa, sb, C, 1, sym["M"], N, K, N, _abi.B_NK, tout, stream)
-
+    call = w8a8_call(1, -1, N, K, N, _abi.B_NK, tout, True, {"i8_tile": tile} if tile else None)
     return KernelSpec("int8_gemm_kernel_corrected",
                       [Param("A", ("M", K), in_dtype), Param("B", (N, K), in_dtype),
                        Param("scale_a", ("M",), scale_dtype), Param("scale_b", (N,), scale_dtype),
-                       Param("C", ("M", N), out_dtype), Param("workspace_1", ("M", N), accum_dtype)], launch,
+                       Param("C", ("M", N), out_dtype), Param("workspace_1", ("M", N), accum_dtype)], call,
                       {"block": (block_M, block_N, block_K), "tile": tile})
 
 
@@ -62,14 +57,9 @@ def quant_batch_matmul_per_token(Batch: int, M: int, N: int, K: int, block_M: in
     the batched layout of example_quant_batch_matmul.py:38-40 with the sequential two-scale
     epilogue of deepseek_v4/int8_gemm.py:97-99."""
     tout = ABI_DTYPE[TORCH_DTYPES[out_dtype]]
-
-    def launch(t, sym, stream):
-        A, B, sa, sb, C, _ws = t
-        with _abi.tuning(i8_tile=tile):
-            w8a8_launch(A, B, sa, sb, C, Batch, M, N, K, N, _abi.B_KN, tout, stream)
-
+    call = w8a8_call(Batch, M, N, K, N, _abi.B_KN, tout, True, {"i8_tile": tile} if tile else None)
     return KernelSpec("quant_batch_matmul_per_token",
                       [Param("A", (Batch, M, K), "int8"), Param("B", (Batch, K, N), "int8"),
                        Param("scale_a", (Batch, M), "float32"), Param("scale_b", (N,), "float32"),
-                       Param("C", (Batch, M, N), out_dtype), Param("workspace_1", (Batch, M, N), "int32")], launch,
+                       Param("C", (Batch, M, N), out_dtype), Param("workspace_1", (Batch, M, N), "int32")], call,
                       {"block": (block_M, block_N, block_K), "tile": tile})

@@ -13,8 +13,7 @@ no output index -- C is accumulated in place by atomic adds and must be zeroed b
 """
 from __future__ import annotations
 
-from .. import _abi
-from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, Param, PassConfigKey, jit
+from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, NativeCall, Param, PassConfigKey, jit
 
 _DT = {"float16": "float16", "bfloat16": "bfloat16", "float32": "float32", "float": "float32"}
 
@@ -25,12 +24,8 @@ def simple_gemv(N: int, K: int, block_N: int, block_K: int, dtype: str = "float1
         raise ValueError("dtype must be float16, bfloat16 or float32 and accum_dtype float32")
     dt = _DT[dtype]
     code = ABI_DTYPE[TORCH_DTYPES[dt]]
-
-    def launch(t, sym, stream):
-        x, A, y = t
-        _abi.check(_abi.load().tlq_gemv(_abi.ptr(x), _abi.ptr(A), _abi.ptr(y), N, K, code, code, stream))
-
-    return KernelSpec("simple_gemv", [Param("x", (K,), dt), Param("A", (N, K), dt), Param("y", (N,), dt)], launch,
+    call = NativeCall("gemv", (N, K, code))
+    return KernelSpec("simple_gemv", [Param("x", (K,), dt), Param("A", (N, K), dt), Param("y", (N,), dt)], call,
                       {"block": (block_N, block_K)})
 
 
@@ -42,14 +37,9 @@ def gemm_splitk(M: int, N: int, K: int, block_M: int, block_N: int, block_K: int
     if split_k < 1 or K % split_k:
         raise ValueError(f"split_k={split_k} must divide K={K}")
     code = ABI_DTYPE[TORCH_DTYPES[dtype]]
-
-    def launch(t, sym, stream):
-        A, B, C = t
-        _abi.check(_abi.load().tlq_gemm_f16_splitk(_abi.ptr(A), _abi.ptr(B), _abi.ptr(C), M, N, K, split_k, code, _abi.B_KN,
-                                                   stream))
-
+    call = NativeCall("splitk", (M, N, K, split_k, code))
     return KernelSpec("gemm_splitk", [Param("A", (M, K), dtype), Param("B", (K, N), dtype), Param("C", (M, N), "float32")],
-                      launch, {"block": (block_M, block_N, block_K), "split_k": split_k})
+                      call, {"block": (block_M, block_N, block_K), "split_k": split_k})
 
 
 @jit(out_idx=[-1], pass_configs={PassConfigKey.TL_ASCEND_AUTO_CV_COMBINE: True, PassConfigKey.TL_ASCEND_AUTO_SYNC: True,
@@ -61,11 +51,6 @@ def batch_matmul(B: int, M: int, N: int, K: int, block_M: int, block_N: int, K_L
     if dtype not in ("float16", "bfloat16") or _DT[accum_dtype] != "float32":
         raise ValueError("dtype must be float16 or bfloat16 and accum_dtype float")
     code = ABI_DTYPE[TORCH_DTYPES[dtype]]
-
-    def launch(t, sym, stream):
-        A, Bm, C = t
-        _abi.check(_abi.load().tlq_gemm_f16_batched(_abi.ptr(A), _abi.ptr(Bm), _abi.ptr(C), B, M, N, K, code, code, _abi.B_KN,
-                                                    stream))
-
+    call = NativeCall("f16_batched", (B, M, N, K, code))
     return KernelSpec("batch_matmul", [Param("A_mat", (B, M, K), dtype), Param("B_mat", (B, K, N), dtype),
-                                       Param("C_mat", (B, M, N), dtype)], launch, {"block": (block_M, block_N, K_L1)})
+                                       Param("C_mat", (B, M, N), dtype)], call, {"block": (block_M, block_N, K_L1)})

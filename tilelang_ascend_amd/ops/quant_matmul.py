@@ -11,7 +11,7 @@ The reference writes acc to the global workspace and re-reads it on the vector c
 (:66-68); here the rescale runs on the MFMA accumulators.  Only with one batch and few
 activation rows, where the output tiles are too few to fill the machine, K is cut into
 slices that write int32 matrices into a workspace and a second pass sums and rescales
-them (``w8a8_launch``) -- the same values bit for bit.
+them (``w8a8_call``) -- the same values bit for bit.
 """
 from __future__ import annotations
 
@@ -20,7 +20,7 @@ from typing import Literal
 import torch
 
 from .. import _abi
-from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, Param, PassConfigKey, jit
+from ..jit import ABI_DTYPE, TORCH_DTYPES, KernelSpec, NativeCall, Param, PassConfigKey, jit
 
 _PASS_CONFIGS = {
     PassConfigKey.TL_ASCEND_AUTO_SYNC: True,
@@ -38,16 +38,12 @@ def _check_types(scale_size, in_dtype, out_dtype, accum_dtype, scale_dtype):
         raise ValueError(f"out_dtype must be float16, bfloat16 or float32, got {out_dtype}")
 
 
-def w8a8_launch(A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_code, stream):
+def w8a8_call(batch, M, N, K, n_scale_b, b_layout, out_code, with_scale_a, tuning=None) -> NativeCall:
     """One W8A8 launch with the int32 workspace the library asks for (the reference's workspace_idx buffer,
     example_quant_batch_matmul.py:28,42): allocated per call on A's device like the reference's, and only where the
     library cuts K into slices (one batch, few activation rows); otherwise the rescale stays fused and nothing is
     allocated."""
-    lib = _abi.load()
-    ws_bytes = lib.tlq_w8a8_workspace_bytes(batch, M, N, K)
-    ws = _abi.scratch(ws_bytes, A.device, stream)
-    _abi.check(lib.tlq_gemm_w8a8_ws(_abi.ptr(A), _abi.ptr(B), _abi.ptr(scale_a), _abi.ptr(scale_b), _abi.ptr(C), _abi.ptr(ws),
-                                    ws_bytes, batch, M, N, K, n_scale_b, b_layout, out_code, stream))
+    return NativeCall("w8a8", (batch, M, N, K, n_scale_b, b_layout, out_code, with_scale_a), tuning=tuning)
 
 
 @jit(out_idx=[3], workspace_idx=[4], pass_configs=_PASS_CONFIGS)
@@ -61,15 +57,11 @@ def simple_quant_batch_matmul(Batch: int, M: int, N: int, K: int, scale_size: Li
     _check_types(scale_size, in_dtype, out_dtype, accum_dtype, scale_dtype)
     N_scale = N if scale_size == "N" else 1
     tout = ABI_DTYPE[TORCH_DTYPES[out_dtype]]
-
-    def launch(t, sym, stream):
-        A, B, scale, C, _ws = t
-        w8a8_launch(A, B, None, scale, C, Batch, M, N, K, N_scale, _abi.B_KN, tout, stream)
-
+    call = w8a8_call(Batch, M, N, K, N_scale, _abi.B_KN, tout, False)
     return KernelSpec("simple_quant_batch_matmul",
                       [Param("A", (Batch, M, K), in_dtype), Param("B", (Batch, K, N), in_dtype),
                        Param("scale", (N_scale,), scale_dtype), Param("C", (Batch, M, N), out_dtype),
-                       Param("workspace_1", (Batch, M, N), accum_dtype)], launch,
+                       Param("workspace_1", (Batch, M, N), accum_dtype)], call,
                       {"block": (block_M, block_N, block_K), "scale_size": scale_size})
 
 
@@ -84,13 +76,9 @@ def simple_quant_matmul(M: int, N: int, K: int, scale_size: Literal["1", "N"],
     _check_types(scale_size, in_dtype, out_dtype, accum_dtype, scale_dtype)
     N_scale = N if scale_size == "N" else 1
     tout = ABI_DTYPE[TORCH_DTYPES[out_dtype]]
-
-    def launch(t, sym, stream):
-        A, B, scale, C, _ws = t
-        w8a8_launch(A, B, None, scale, C, 1, M, N, K, N_scale, _abi.B_KN, tout, stream)
-
+    call = w8a8_call(1, M, N, K, N_scale, _abi.B_KN, tout, False)
     return KernelSpec("simple_quant_matmul",
                       [Param("A", (M, K), in_dtype), Param("B", (K, N), in_dtype),
                        Param("scale", (N_scale,), scale_dtype), Param("C", (M, N), out_dtype),
-                       Param("workspace_1", (M, N), accum_dtype)], launch,
+                       Param("workspace_1", (M, N), accum_dtype)], call,
                       {"block": (block_M, block_N, block_K), "scale_size": scale_size})

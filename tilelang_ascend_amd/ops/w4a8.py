@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from .. import _abi
-from ..jit import KernelSpec, Param, PassConfigKey, jit
+from ..jit import KernelSpec, NativeCall, Param, PassConfigKey, jit
 from .dequant_gemm import unpack_int4
 
 PASS_CONFIGS = {
@@ -28,15 +28,9 @@ PASS_CONFIGS = {
 @jit(out_idx=[-1], pass_configs=PASS_CONFIGS)
 def w4a8_gemm_cv(M, N, K):
     """C[M,N] i32 = A[M,K] i8 . twos_complement_unpack(B_packed)[N,K]^T (exact)."""
-
-    def launch(t, sym, stream):
-        A, Bp, workspace, C = t
-        ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None and workspace.is_contiguous() else 0
-        _abi.check(_abi.load().tlq_gemm_w4a8_ws(_abi.ptr(A), _abi.ptr(Bp), _abi.ptr(workspace) if ws_bytes else None, ws_bytes,
-                                                _abi.ptr(C), M, N, K, _abi.S4_TWOS, stream))
-
     return KernelSpec("w4a8_gemm_cv", [Param("A", (M, K), "int8"), Param("B_packed", (N, K // 2), "uint8"),
-                                       Param("workspace", (N, K), "int8"), Param("C", (M, N), "int32")], launch)
+                                       Param("workspace", (N, K), "int8"), Param("C", (M, N), "int32")],
+                      NativeCall("w4a8_ws", (M, N, K, _abi.S4_TWOS)))
 
 
 def torch_convert(tensor: torch.Tensor) -> torch.Tensor:

@@ -13,6 +13,7 @@ import torch
 from .. import _abi
 
 _INTERLEAVE = {None: 0, "none": 0, "float16": 1, "int8": 2}
+_STORAGE = {torch.int8: _abi.I8, torch.uint8: 5}
 _DT = {torch.float16: _abi.F16, torch.bfloat16: _abi.BF16}
 
 
@@ -25,6 +26,10 @@ def pack_int4(values: torch.Tensor, interleave: Optional[str] = None, storage_dt
     interleave: None, "float16" or "int8" (the target_dtype of interleave_weight)."""
     if interleave not in _INTERLEAVE:
         raise ValueError('interleave must be None, "float16" or "int8"')
+    if isinstance(values, torch.Tensor) and values.is_cuda and storage_dtype in _STORAGE:
+        out = _abi.host().pack(values, _INTERLEAVE[interleave], _STORAGE[storage_dtype])  # the ordinary call
+        if out is not NotImplemented:
+            return out
     if values.dtype not in (torch.int8, torch.uint8) or values.dim() != 2:
         raise ValueError("values must be a 2-D int8 or uint8 tensor")
     if not values.is_cuda or not values.is_contiguous():
@@ -39,6 +44,10 @@ def pack_int4(values: torch.Tensor, interleave: Optional[str] = None, storage_dt
 def quantize_sym4(W: torch.Tensor, group_size: int = -1) -> Tuple[torch.Tensor, torch.Tensor]:
     """W fp16 / bf16 [N, K] on the GPU -> (q - 8 as int8 [N, K], scales [N, K // group_size] in W's dtype):
     s = max|w| / 8 per group, q = clamp(round(w / s) + 8, 0, 16).  group_size -1 means one group per row."""
+    if isinstance(W, torch.Tensor) and W.is_cuda and W.dim() == 2:
+        out = _abi.host().quantize(W, W.shape[1] if group_size == -1 else group_size)  # the ordinary call
+        if out is not NotImplemented:
+            return out
     if W.dtype not in _DT or W.dim() != 2:
         raise ValueError("W must be a 2-D float16 or bfloat16 tensor")
     if not W.is_cuda or not W.is_contiguous():
