@@ -49,6 +49,9 @@ int tlq_debug_check_panel256_addressing(int64_t M, int64_t N, int64_t K, int64_t
 int tlq_debug_panel256_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out);
 /* The schedule alone over `steps` steps, with the kernel's own wait counts (negative arguments) or others (to see them fail). */
 int tlq_debug_check_panel256_schedule(int steps, int wait_w, int wait_a);
+/* What the small-tile kernel (one launch, wavefronts split K) would take for a problem: plan_out receives int64 activation rows and weight
+ * rows per work-group, wavefronts, estimated nanoseconds; returns 1 when it applies. */
+int tlq_debug_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, void* plan_out);
 /* The middle-M panel kernel (TLQ_ALGO_PANELM): its plan (plan_out: int64 tiles_m, tiles_n, K slices, steps per slice, activation
  * rows per work-group). */
 int tlq_debug_panelm_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out);
@@ -114,8 +117,9 @@ void tlq_tune_w4a16_panelm_rows(int rows);                   /* activation rows 
 void tlq_tune_w4a16_panel_slice(int steps);                  /* K slice of the panel kernels in steps of 128 values (0 = their own plan) */
 void tlq_tune_w4a16_tile(int block_m);                      /* 16|32|64|128|256 */
 void tlq_tune_w4a16_split(int slices);                       /* K slices of the tile kernel, 16 < M < 256 with a workspace */
-void tlq_tune_w4a16_skinny(int waves, int row_tiles);       /* wavefronts per group 1..16; 16-row tiles per wavefront 1|2,
-                                                               +10 = never stage through LDS, +20 = stage whenever possible */
+void tlq_tune_w4a16_skinny(int waves, int row_tiles);       /* wavefronts per group 1..16; 16-row weight tiles per work-group 1|2|4, +100*(1|2|4):
+                                                               16-row activation tiles, +10 = never the small-tile kernel, +20 = that
+                                                               kernel whenever it applies */
 void tlq_tune_i8_tile(int block_m);                         /* 32|128|256 */
 void tlq_tune_f16_split(int slices);                        /* K slices of tlq_gemm_f16_ws: 0 = automatic, 1 = never, n = up to n */
 int tlq_debug_f16_split(int64_t M, int64_t N, int64_t K);  /* K slices tlq_gemm_f16_ws takes for one batch of this shape */

@@ -39,6 +39,7 @@ SOURCES = [
     "gemv_plain.hip",
     "gemv_w4a16.hip",
     "gemm_w4a16.hip",
+    "gemm_w4a16_small.hip",
     "gemm_w4a16_stream.hip",
     "gemm_w4a16_panel.hip",
     "gemm_w4a16_panel256.hip",

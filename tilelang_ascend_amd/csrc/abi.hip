@@ -41,6 +41,11 @@ static void log_launch(const char* what, const char* detail) {
 // returned an error without the count moving has refused its arguments and launched nothing.
 static thread_local uint64_t g_launches = 0;
 uint64_t launch_count() { return g_launches; }
+bool launch_log_on() { return g_log_on; }
+
+static std::atomic<uint64_t> g_generation{0};
+uint64_t tuning_generation() { return g_generation.load(std::memory_order_acquire); }
+void tuning_changed() { g_generation.fetch_add(1, std::memory_order_acq_rel); }
 
 bool check_launch(const char* what, const char* detail) {
   ++g_launches;

@@ -28,6 +28,14 @@ int gemm_w4a16_stream(const void* A, const void* Wp, const void* scales, const v
                       float* partial, hipStream_t st);
 int gemm_w4a16_skinny(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, hipStream_t st);
+struct SmallPlan {
+  bool ok;
+  int mt, rt, waves;
+  double us;
+};
+SmallPlan w4a16_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros, int force_waves, int force_rt, int force_mt);
+int gemm_w4a16_small(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N, int64_t K, int64_t group,
+                     float zero_scalar, int in_dtype, int out_dtype, int w_layout, const SmallPlan& p, const char* what, hipStream_t st);
 int gemm_f16_plain(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype,
                    int out_dtype, int b_layout, hipStream_t st);
 int gemm_f16_splitk(const void* A, const void* B, float* C, int64_t M, int64_t N, int64_t K, int64_t split_k,
@@ -176,13 +184,13 @@ void tlq_tune_gemm_slots(int mode) { tlq::g_gemm_slots = mode < 0 ? 0 : (mode > 
 int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused) {
   return tlq::prefer_small_tiles(batch, M, N, fused ? 0.65 : 0.72) ? 128 : 256;
 }
-void tlq_tune_gemm_tile(int tile) { tlq::g_gemm_f16_tile = (tile == 128 || tile == 256) ? tile : 0; }
+void tlq_tune_gemm_tile(int tile) { tlq::tuning_changed(), tlq::g_gemm_f16_tile = (tile == 128 || tile == 256) ? tile : 0; }
 void tlq_tune_w4a16_stream(int on) { tlq::g_w4a16_stream = on != 0; }
-void tlq_tune_w4a16_stream_slice(int steps) { tlq::g_stream_slice_steps = steps; }
+void tlq_tune_w4a16_stream_slice(int steps) { tlq::tuning_changed(), tlq::g_stream_slice_steps = steps; }
 void tlq_tune_w4a16_decode(int on) { tlq::g_w4a16_decode = on != 0; }
 void tlq_tune_w4a16_panel(int mode) { tlq::g_w4a16_panel = mode != 0 ? 1 : 0; }
-void tlq_tune_w4a16_panel_slice(int steps) { tlq::g_panel_slice_steps = tlq::g_panel2_slice_steps = tlq::g_panelm_slice_steps = steps < 0 ? 0 : steps; }
-void tlq_tune_w4a16_panelm_rows(int rows) { tlq::g_panelm_rows = (rows == 64 || rows == 128) ? rows : 0; }
+void tlq_tune_w4a16_panel_slice(int steps) { tlq::tuning_changed(), tlq::g_panel_slice_steps = tlq::g_panel2_slice_steps = tlq::g_panelm_slice_steps = steps < 0 ? 0 : steps; }
+void tlq_tune_w4a16_panelm_rows(int rows) { tlq::tuning_changed(), tlq::g_panelm_rows = (rows == 64 || rows == 128) ? rows : 0; }
 
 int tlq_debug_panel_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out) {
   if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return 0;
@@ -214,6 +222,15 @@ int tlq_debug_panelm_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cu
   return p.ok ? 1 : 0;
 }
 
+int tlq_debug_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, void* plan_out) {
+  const SmallPlan p = w4a16_small_plan(M, N, K, group, nullptr, nullptr, 0, 0, 0);
+  if (plan_out) {
+    int64_t* o = (int64_t*)plan_out;
+    o[0] = 16 * p.mt, o[1] = 16 * p.rt, o[2] = p.waves, o[3] = (int64_t)(p.us * 1000.0);
+  }
+  return p.ok ? 1 : 0;
+}
+
 int tlq_debug_decode_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out) {
   const DecodePlan p = w4a16_decode_plan(M, N, K, group, cus);
   if (plan_out) {
@@ -232,6 +249,23 @@ static bool skinny_leaves_cus_idle(int64_t N) {
   if (tile_fill(1, 16, N, 16) < 0.8) return true;
   const int64_t wgs = ceil_div(N, (int64_t)16), places = 2 * cu_count_or_default();
   return wgs > places / 2 && (double)wgs / (double)(ceil_div(wgs, places) * places) < 0.8;
+}
+// Where the small-tile kernel (gemm_w4a16_small.hip: one launch, wavefronts split K) is ahead of a family by estimate.  The
+// families' own times were fitted to the same 520 problems (10 - 11 % rms each; G: billions of products, G16: the same with M rounded up
+// to 16 rows); with these bars it never lost more than 5 % to the family it replaces and won 1.43 x on average over the
+// streaming kernel's share of them, 1.47 x over the two passes'.
+static double giga(double m, int64_t N, int64_t K) { return m * (double)N * (double)K * 1e-9; }
+static double up16(int64_t M) { return (double)ceil_div(M, (int64_t)16) * 16.0; }
+static bool small_beats_stream(const SmallPlan& p, int64_t M, int64_t N, int64_t K) {
+  return p.ok && g_stream_slice_steps <= 0 && p.us < 0.95 * (11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K);
+}
+// above 512 rows (the two passes, or the panel kernels with their head and tail): only while the whole call stays short
+static bool small_beats_panels(const SmallPlan& p, int64_t M, int64_t N, int64_t K) {
+  return p.ok && p.us < 13.0 && p.us < 0.9 * (14.9 + 3.6 * giga(up16(M), N, K) + 0.79e-3 * (double)K);
+}
+// the decode kernel over chunks of K, whose second launch adds the chunks
+static bool small_beats_decode_chunks(const SmallPlan& p, int64_t M, int64_t N, int64_t K) {
+  return p.ok && p.us < 0.95 * (5.2 + 0.67 * giga((double)M, N, K) + 4.36 * giga(up16(M), N, K) + 0.023e-6 * (double)N * (double)K + 0.25e-3 * (double)K);
 }
 static bool decode_preferred(int64_t M, int64_t N, int64_t K) { return M > 2 || (M == 2 && N * K >= ((int64_t)1 << 24)); }
 
@@ -446,8 +480,13 @@ int64_t tlq_w4a16_workspace_bytes_for(int64_t M, int64_t N, int64_t K, int algo)
 }
 
 static int64_t w4a16_kernel_workspace_bytes(int64_t M, int64_t N, int64_t K);
+static int64_t w4a16_workspace_bytes_now(int64_t M, int64_t N, int64_t K);
 int64_t tlq_w4a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (N <= 0 || K <= 0) return 0;
+  static thread_local PlanTable<int64_t> known;
+  return known.get(M, N, K, 0, [&] { return w4a16_workspace_bytes_now(M, N, K); });
+}
+static int64_t w4a16_workspace_bytes_now(int64_t M, int64_t N, int64_t K) {
   int64_t need = w4a16_kernel_workspace_bytes(M, N, K);
   // (a weight-row count that is no multiple of four: what the multiple of 16 below asks for, then its packed result, sized for fp32)
   if (ragged_rows_apply(M, N)) need = ragged_head(N) == 0 ? 0 : (w4a16_kernel_workspace_bytes(M, ragged_head(N), K) + 15) / 16 * 16 + ragged_result_bytes(M, N, 4);
@@ -717,6 +756,15 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       set_error("%s", "");
     }
   }
+  // Many rows on so few and short weight rows that the whole call is a matter of latency: the small-tile kernel
+  if (algo == TLQ_ALGO_AUTO && M > 512 && M < kMaxDim && N >= 1 && N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && w_packed && C && aligned16(A) &&
+      aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
+      (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
+    const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+    if (small_beats_panels(small, M, N, K))
+      return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
+                              (hipStream_t)stream);
+  }
   // Above 512 rows the panel kernels are the fast path, and they take row counts that are multiples of four (their direct
   // loads move four activation rows).  Any other count -- prompt lengths are what they are -- runs as its multiple of four
   // below through the same choice plus the last one to three rows through the small-M kernels, which is one short launch
@@ -776,6 +824,12 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     // Two of its work-groups share a CU, so that holds for rounds of twice the CU count as well: N = 10240, K = 8192
     // (640 work-groups on 512 places): 15 against 20 - 26 us; N = 12288, K = 6144 (768): 14 - 15 against 17 - 21 us;
     // N = 17408, K = 5120 (1088): 17 - 19 against 20 - 24 us; with 512 or 960 work-groups the skinny kernel is ahead)
+    if (algo == TLQ_ALGO_AUTO && dp.ok && dp.chunks > 1 && args_ok) {
+      const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+      if (small_beats_decode_chunks(small, M, N, K))
+        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
+                                (hipStream_t)stream);
+    }
     if (dp.ok && dp.chunks > 1 && (algo == TLQ_ALGO_DECODE || M > 16 || K > 16384 || N * (K / 2) >= ((int64_t)64 << 20) || skinny_leaves_cus_idle(N)) && args_ok && (M * N) % 4 == 0 && workspace && aligned16(workspace) &&
         workspace_bytes >= (int64_t)dp.chunks * M * N * 4)
       return gemm_w4a16_decode(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, dp,
@@ -860,6 +914,13 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
                          (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) && (M * N) % 4 == 0 &&
                          ((uintptr_t)scales & 1) == 0 && ((uintptr_t)zeros & 1) == 0 && K > 0 && fits32(M, K * 2) && fits32(N, K / 2);
     const bool ws_ok = sp.ok && (sp.split == 1 || (workspace && aligned16(workspace) && workspace_bytes >= (int64_t)sp.split * M * N * 4));
+    // (on the family's behalf, asked for by name too: the interleaved layout takes the same kernel at the same sizes)
+    if (sp.ok && args_ok) {
+      const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+      if (small_beats_stream(small, M, N, K))
+        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(stream)",
+                                (hipStream_t)stream);
+    }
     if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && panel256_beats_stream(M, N, K, group, sp)) {
       const int rc = try_panel256(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, workspace,
                                   workspace_bytes, stream);
@@ -1062,6 +1123,12 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
   }
   if (algo != TLQ_ALGO_TWO_PASS) {
     const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
+    if (sp.ok && (M * N) % 4 == 0) {
+      const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+      if (small_beats_stream(small, M, N, K))
+        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(stream)",
+                                (hipStream_t)stream);
+    }
     const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));
     // (129 .. 512 rows: the 256-row kernel where its estimate beats the streaming kernel's, as for the plain layout)
     if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && panel256_beats_stream(M, N, K, group, sp)) {
@@ -1155,7 +1222,7 @@ int tlq_gemm_f16_ws(const void* A, const void* B, void* C, void* workspace, int6
   return gemm_f16_slices(A, B, C, (float*)workspace, M, N, K, split, in_dtype, out_dtype, b_layout, (hipStream_t)stream);
 }
 
-void tlq_tune_f16_split(int slices) { g_f16_split = slices; }
+void tlq_tune_f16_split(int slices) { tlq::tuning_changed(), g_f16_split = slices; }
 int tlq_debug_f16_split(int64_t M, int64_t N, int64_t K) { return f16_split_choice(1, M, N, K); }
 
 int tlq_gemm_f16_splitk(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t split_k,

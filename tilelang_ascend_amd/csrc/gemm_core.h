@@ -1011,8 +1011,8 @@ int launch_gemm(const typename AL::Params& pa, const typename WL::Params& pw, co
   }
   kern<<<(unsigned)blocks, WM * WN * 64, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, KT, k_tail, (int)tiles_m,
                                                           (int)tiles_n, g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows, kt_total);
-  char detail[96];
-  snprintf(detail, sizeof(detail), "gemm_mfma_kernel %dx%d tiles, two stages%s", BM, BN, WL::DIRECT ? "" : ", weights through registers");
+  char detail[96] = "";
+  if (launch_log_on()) snprintf(detail, sizeof(detail), "gemm_mfma_kernel %dx%d tiles, two stages%s", BM, BN, WL::DIRECT ? "" : ", weights through registers");
   return check_launch(what, detail) ? 0 : 1;
 }
 

@@ -410,8 +410,8 @@ static int launch_stream(const void* A, const void* Wp, const void* scales, cons
   kern<<<dim3(p.n_blocks, p.split, p.m_blocks), 512, lds_bytes, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales,
                                                                      (const T*)zeros, C, partial, (int)M, (int)N, (int)K, gshift,
                                                                      zero_scalar, out_dtype, p.slice_steps);
-  char detail[64];
-  snprintf(detail, sizeof(detail), "w4a16_stream_kernel, %d activation rows per work-group", 16 * TM);
+  char detail[64] = "";
+  if (launch_log_on()) snprintf(detail, sizeof(detail), "w4a16_stream_kernel, %d activation rows per work-group", 16 * TM);
   return check_launch("tlq_gemm_w4a16(stream)", detail) ? 0 : 1;
 }
 

@@ -14,6 +14,42 @@ namespace tlq {
 void set_error(const char* fmt, ...);
 bool check_launch(const char* what, const char* detail = nullptr);
 uint64_t launch_count();
+bool launch_log_on();  // (texts that only the log wants are made only then)
+
+// ---- plans already worked out ------------------------------------------------------------
+// A number that changes whenever something a plan depends on may have changed: the tuning hooks, the table of tuned choices.
+uint64_t tuning_generation();
+void tuning_changed();
+// A small direct-mapped table per thread for functions of a few sizes that a call asks for again and again (workspace sizes,
+// launch plans: 1 - 3 us of host time where a whole launch takes 3).  An entry holds while the generation and the compute-unit
+// count are those it was made with.
+template <class Value>
+class PlanTable {
+  struct Entry {
+    uint64_t generation = ~(uint64_t)0;
+    int64_t key[5];
+    Value value;
+  };
+  Entry e_[64];
+
+ public:
+  template <class Make>
+  const Value& get(int64_t a, int64_t b, int64_t c, int64_t d, Make make) {
+    const int64_t key[5] = {a, b, c, d, tlq_device_cu_count()};
+    uint64_t h = 0;
+    for (int64_t k : key) h = (h ^ (uint64_t)k) * 0x9e3779b97f4a7c15ull, h ^= h >> 29;
+    Entry& e = e_[h & 63];
+    const uint64_t now = tuning_generation();
+    bool same = e.generation == now;
+    for (int i = 0; i < 5; ++i) same = same && e.key[i] == key[i];
+    if (!same) {
+      e.value = make();
+      for (int i = 0; i < 5; ++i) e.key[i] = key[i];
+      e.generation = now;
+    }
+    return e.value;
+  }
+};
 
 #define TLQ_REQUIRE(cond, ...)      \
   do {                              \

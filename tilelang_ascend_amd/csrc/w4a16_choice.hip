@@ -75,6 +75,7 @@ int tlq_w4a16_choice_set(int64_t M, int64_t N, int64_t K, int64_t group, int in_
   else
     t[key] = algo;
   g_choice_count.store((int64_t)t.size(), std::memory_order_release);
+  tuning_changed();
   return 0;
 }
 
@@ -87,6 +88,7 @@ void tlq_w4a16_choice_clear(void) {
   std::unique_lock<std::shared_mutex> lk(g_choice_lock);
   choice_table().clear();
   g_choice_count.store(0, std::memory_order_release);
+  tuning_changed();
 }
 
 int64_t tlq_w4a16_choice_count(void) { return tlq::g_choice_count.load(std::memory_order_acquire); }
@@ -142,6 +144,7 @@ int tlq_w4a16_choice_load(const char* path) {
   auto& t = choice_table();
   for (const auto& kv : incoming) t[kv.first] = kv.second;
   g_choice_count.store((int64_t)t.size(), std::memory_order_release);
+  tuning_changed();
   return 0;
 }
 
