@@ -120,6 +120,11 @@ void tlq_tune_w4a16_split(int slices);                       /* K slices of the 
 void tlq_tune_w4a16_skinny(int waves, int row_tiles);       /* wavefronts per group 1..16; 16-row weight tiles per work-group 1|2|4, +100*(1|2|4):
                                                                16-row activation tiles, +10 = never the small-tile kernel, +20 = that
                                                                kernel whenever it applies */
+void tlq_tune_small(int waves, int tiles);                  /* the small-tile kernel of the int8, W4A8 and plain 16-bit products: tiles =
+                                                               10 * activation tiles + weight tiles (1|2|4 each), < 0 = never; 0, 0 = by estimate */
+/* What that kernel would take: kind 0 weights [N, K] (int8), 1 int8 [K, N], 2 16-bit [K, N], 3 packed int4 [N, K / 2]; row_bytes: bytes of K of an
+ * activation row; plan_out as in tlq_debug_small_plan. */
+int tlq_debug_small_tile(int kind, int64_t batch, int64_t M, int64_t N, int64_t row_bytes, void* plan_out);
 void tlq_tune_i8_tile(int block_m);                         /* 32|128|256 */
 void tlq_tune_f16_split(int slices);                        /* K slices of tlq_gemm_f16_ws: 0 = automatic, 1 = never, n = up to n */
 int tlq_debug_f16_split(int64_t M, int64_t N, int64_t K);  /* K slices tlq_gemm_f16_ws takes for one batch of this shape */

@@ -1,0 +1,133 @@
+"""The small-tile kernel of the int8, W4A8 and plain 16-bit products (csrc/gemm_small.h): every tile and weight layout, ragged rows and
+columns, one wavefront to all, batches, every epilogue and sign convention -- integers bit for bit, 16-bit results against fp32."""
+import ctypes
+import re
+import subprocess
+
+import pytest
+import torch
+
+from helpers import assert_bit_equal, check_float_output, gen
+from tilelang_ascend_amd import _abi, build
+
+CODE = {torch.float16: _abi.F16, torch.bfloat16: _abi.BF16, torch.float32: _abi.F32}
+
+
+@pytest.fixture
+def lib():
+    yield _abi.load()
+    _abi.load().tlq_tune_small(0, 0)
+
+
+def i8(seed, *shape):
+    return torch.randint(-127, 128, shape, dtype=torch.int8, generator=gen(seed))
+
+
+def called(lib, rc):
+    log = lib.tlq_debug_launch_log_text().decode()
+    lib.tlq_debug_launch_log(0)
+    _abi.check(rc)
+    torch.cuda.synchronize()
+    assert "gemm_small_kernel" in log and log.count("[") == 1, log
+
+
+TILES = [(1, 1), (2, 1), (4, 1), (1, 2), (2, 2), (4, 2), (1, 4), (2, 4), (4, 4)]  # activation tiles, weight tiles
+SHAPES = [(1, 16, 128, 1), (17, 48, 256, 2), (33, 80, 640, 3), (64, 272, 1152, 4), (70, 1008, 2048, 8), (5, 144, 4224, 16)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", TILES)
+@pytest.mark.parametrize("M,N,K,waves", SHAPES)
+def test_int8_weights_by_rows_and_packed(lib, rows, cols, M, N, K, waves):
+    P, st = _abi.ptr, torch.cuda.current_stream().cuda_stream
+    print(f"small int8 {rows}x{cols} M={M} N={N} K={K} waves={waves}", flush=True)
+    lib.tlq_tune_small(waves, 10 * rows + cols)
+    A, W, sa, sb = i8(1, M, K), i8(2, N, K), torch.rand(M, generator=gen(3)), torch.rand(N, generator=gen(4))
+    dA, dW, dsa, dsb = A.cuda(), W.cuda(), sa.cuda(), sb.cuda()
+    acc = (A.double() @ W.double().T).to(torch.int32)  # exact
+    C = torch.full((M, N), -1, dtype=torch.int32, device="cuda")
+    lib.tlq_debug_launch_log(1)
+    called(lib, lib.tlq_gemm_i8(P(dA), P(dW), P(C), 1, M, N, K, _abi.B_NK, st))
+    assert torch.equal(C.cpu(), acc)
+    for dt in (torch.float16, torch.bfloat16, torch.float32):
+        out = torch.full((M, N), float("nan"), dtype=dt, device="cuda")
+        lib.tlq_debug_launch_log(1)
+        called(lib, lib.tlq_gemm_w8a8(P(dA), P(dW), P(dsa), P(dsb), P(out), 1, M, N, K, N, _abi.B_NK, CODE[dt], st))
+        assert_bit_equal(out.cpu(), ((acc.float() * sa[:, None]) * sb).to(dt), f"rescaled {dt}")
+    Wp = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=gen(5))
+    dWp = Wp.cuda()
+    u = torch.stack([Wp & 15, Wp >> 4], -1).reshape(N, K).to(torch.int32)
+    for mode, w in ((_abi.U4, u), (_abi.S4_TWOS, torch.where(u >= 8, u - 16, u)), (_abi.S4_OFFSET8, u - 8), (_abi.S4_OFFSET7, u - 7)):
+        lib.tlq_debug_launch_log(1)
+        called(lib, lib.tlq_gemm_w4a8(P(dA), P(dWp), P(C), M, N, K, mode, st))
+        assert torch.equal(C.cpu(), (A.double() @ w.double().T).to(torch.int32)), mode
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2, 4])
+@pytest.mark.parametrize("M,N,K,waves", SHAPES)
+@pytest.mark.parametrize("batch", [1, 3])
+def test_weights_by_columns_in_batches(lib, rows, M, N, K, waves, batch):
+    P, st = _abi.ptr, torch.cuda.current_stream().cuda_stream
+    print(f"small [K, N] {rows} M={M} N={N} K={K} waves={waves} batch={batch}", flush=True)
+    lib.tlq_tune_small(waves, 10 * rows + 4)
+    A, W, sb = i8(11, batch, M, K), i8(12, batch, K, N), torch.rand(1, generator=gen(13))
+    dA, dW, dsb = A.cuda(), W.cuda(), sb.cuda()
+    acc = torch.bmm(A.double(), W.double()).to(torch.int32)
+    C = torch.full((batch, M, N), -1, dtype=torch.int32, device="cuda")
+    lib.tlq_debug_launch_log(1)
+    called(lib, lib.tlq_gemm_i8(P(dA), P(dW), P(C), batch, M, N, K, _abi.B_KN, st))
+    assert torch.equal(C.cpu(), acc)
+    out = torch.full((batch, M, N), float("nan"), dtype=torch.float16, device="cuda")
+    lib.tlq_debug_launch_log(1)
+    called(lib, lib.tlq_gemm_w8a8_ws(P(dA), P(dW), None, P(dsb), P(out), None, 0, batch, M, N, K, 1, _abi.B_KN, _abi.F16, st))
+    assert_bit_equal(out.cpu(), (acc.float() * sb).to(torch.float16), "one scale")
+    for dt in (torch.float16, torch.bfloat16):
+        X, B = torch.randn(batch, M, K, generator=gen(14)).to(dt), torch.randn(batch, K, N, generator=gen(15)).to(dt)
+        D, dX, dB = torch.full((batch, M, N), float("nan"), dtype=dt, device="cuda"), X.cuda(), B.cuda()
+        lib.tlq_debug_launch_log(1)
+        called(lib, lib.tlq_gemm_f16_batched(P(dX), P(dB), P(D), batch, M, N, K, CODE[dt], CODE[dt], _abi.B_KN, st))
+        check_float_output(D.cpu().reshape(batch * M, N), torch.bmm(X.float(), B.float()).reshape(batch * M, N), f"16-bit {dt}")
+
+
+@pytest.mark.gpu
+def test_estimates_take_it_where_it_is_ahead(lib):
+    """The operators' own calls: small problems in one launch, large ones as before."""
+    from tilelang_ascend_amd import ops
+
+    def log_of(kernel, *args):
+        lib.tlq_debug_launch_log(1)
+        kernel(*args)
+        text = lib.tlq_debug_launch_log_text().decode()
+        lib.tlq_debug_launch_log(0)
+        return text
+
+    assert "gemm_small_kernel" in log_of(ops.int8_gemm_kernel_corrected(512, 3328), i8(1, 40, 3328).cuda(), i8(2, 512, 3328).cuda(), torch.rand(40).cuda(), torch.rand(512).cuda())
+    assert "gemm_small_kernel" in log_of(ops.w4a8_gemm_cv(57, 1024, 3840), i8(1, 57, 3840).cuda(), torch.zeros(1024, 1920, dtype=torch.uint8).cuda(), i8(2, 1024, 3840).cuda())
+    assert "gemm_small_kernel" in log_of(ops.batch_matmul(4, 34, 256, 5376, 1, 1, 1), torch.zeros(4, 34, 5376).half().cuda(), torch.zeros(4, 5376, 256).half().cuda())
+    assert "gemm_small_kernel" not in log_of(ops.int8_gemm_kernel_corrected(4096, 4096), i8(1, 2048, 4096).cuda(), i8(2, 4096, 4096).cuda(), torch.rand(2048).cuda(), torch.rand(4096).cuda())
+
+
+def test_plan_keeps_to_the_machine(lib):
+    o = (ctypes.c_int64 * 4)()
+    for kind in range(4):
+        for M in (1, 17, 130, 3000):
+            for N in (16, 1008, 14336):
+                for row_bytes in (128, 11008, 28672):
+                    assert lib.tlq_debug_small_tile(kind, 2, M, N, row_bytes, o) == 1
+                    mt, rt, waves = o[0] // 16, o[1] // 16, o[2]
+                    slot = mt * 2048 + (rt * 2048, 8192, 8192, rt * 1024)[kind]
+                    assert mt in (1, 2, 4) and rt in ((1, 2, 4), (4,), (4,), (1, 2, 4))[kind] and 1 <= waves <= min(16, row_bytes // 128)
+                    assert waves * slot * (4 if slot <= 4096 else 3 if slot <= 8192 else 2) <= 160 * 1024 and (rt * mt <= 4 or waves <= 8)
+        assert lib.tlq_debug_small_tile(kind, 1, 1, 16, 192, o) == 0 and lib.tlq_debug_small_tile(kind, 1, 0, 16, 128, o) == 0
+
+
+def test_no_register_spills(tmp_path):
+    cmd = [build.hipcc_path(), *build.HIPCC_FLAGS, "-Rpass-analysis=kernel-resource-usage", "-c", f"{build.CSRC_DIR}/gemm_small.hip",
+           "-o", str(tmp_path / "out.o")]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout[-2000:]
+    blocks = [b for b in re.split(r"remark: Function Name: ", res.stdout)[1:] if "gemm_small_kernel" in b.split()[0]]
+    assert len(blocks) == 39
+    for b in blocks:
+        assert re.search(r"ScratchSize \[bytes/lane\]: 0\b", b) and re.search(r"VGPRs Spill: 0\b", b), b[:300]

@@ -98,6 +98,8 @@ SIGNATURES = {
     "tlq_tune_w4a16_tile": (None, [_int]),
     "tlq_tune_w4a16_split": (None, [_int]),
     "tlq_tune_w4a16_skinny": (None, [_int, _int]),
+    "tlq_tune_small": (None, [_int, _int]),
+    "tlq_debug_small_tile": (_int, [_int, _i64, _i64, _i64, _i64, _vp]),
     "tlq_tune_i8_tile": (None, [_int]),
     "tlq_tune_i8_split": (None, [_int]),
     "tlq_tune_w4a8_ws": (None, [_int]),

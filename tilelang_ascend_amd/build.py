@@ -47,6 +47,7 @@ SOURCES = [
     "w4a16_choice.hip",
     "gemm_w4a16_decode.hip",
     "gemm_int8.hip",
+    "gemm_small.hip",
     "gemm_f16.hip",
     "gemm_api.hip",
     "gemm_addr_check.hip",

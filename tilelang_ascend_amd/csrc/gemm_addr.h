@@ -45,7 +45,8 @@ __host__ __device__ inline uint32_t rowfrag_off(uint32_t base, int ks, int t) {
 // ---- int8 [K, N] source copied unchanged into a [128 k][BN] tile -------------------------------------
 template <int BN>
 __host__ __device__ inline int kn_swz(int k) {
-  static_assert(BN == 128 || BN == 256, "tile width");
+  static_assert(BN == 64 || BN == 128 || BN == 256, "tile width");
+  if (BN == 64) return ((k >> 2) & 1) | (((k >> 4) & 1) << 1);
   return BN == 256 ? ((k & 7) | (((k >> 4) & 1) << 3)) : (((k >> 1) & 3) | (((k >> 4) & 1) << 2));
 }
 // one wavefront instruction covers 1024 / BN consecutive k rows
@@ -77,17 +78,22 @@ __host__ __device__ inline uint32_t knfrag_off(int lane, int wave_row0, int t) {
 // completes the eight values of an MFMA operand.  16-byte chunks of a k row are XOR-swizzled by an even number, which
 // keeps the 8-byte halves of a chunk together and spreads the eight rows a half-wavefront touches over all banks.
 __host__ __device__ inline int kn16_swz(int k) { return ((k & 3) << 1) | (((k >> 3) & 1) << 3); }
+// (tiles of 64 columns: eight chunks in a row, two rows in the 256 bytes of all banks)
+template <int BN>
+__host__ __device__ inline int kn16_swz_of(int k) {
+  return BN == 64 ? (k & 2) | (((k >> 3) & 1) << 2) : kn16_swz(k);
+}
 // one wavefront instruction covers 512 / BN consecutive k rows
 template <int BN>
 __host__ __device__ inline int kn16_k(int lane, int wave, int j, int waves) {
-  static_assert(BN == 128 || BN == 256, "tile width");
+  static_assert(BN == 64 || BN == 128 || BN == 256, "tile width");
   return (j * waves + wave) * (512 / BN) + lane / (BN / 8);
 }
 template <int BN>
 __host__ __device__ inline uint32_t kn16_voff(int lane, int wave, int j, int waves, int cols_valid, uint32_t ld_bytes) {
   const int k = kn16_k<BN>(lane, wave, j, waves);
   const int pc = lane % (BN / 8);
-  int colb = (pc ^ kn16_swz(k)) * 16;
+  int colb = (pc ^ kn16_swz_of<BN>(k)) * 16;
   colb = colb < cols_valid * 2 ? colb : cols_valid * 2 - 16;  // whole chunks are clamped; those columns are masked at the store
   return (uint32_t)k * ld_bytes + (uint32_t)colb;
 }
@@ -98,7 +104,7 @@ __host__ __device__ inline uint32_t kn16frag_off(int lane, int wave_col0, int t)
   const int i = lane & 15, q = lane >> 4;
   const int krow = 8 * q + (i >> 2);
   const int chunk = (wave_col0 >> 3) + 2 * t + ((i & 3) >> 1);
-  return (uint32_t)(krow * 2 * BN) + (uint32_t)((chunk ^ kn16_swz(krow)) << 4) + (uint32_t)(8 * (i & 1));
+  return (uint32_t)(krow * 2 * BN) + (uint32_t)((chunk ^ kn16_swz_of<BN>(krow)) << 4) + (uint32_t)(8 * (i & 1));
 }
 
 // ---- five-slot schedule (gemm_slots.h): tile t = 2 * stage (+ 1 for the weights) lives in slot t % 5 ----

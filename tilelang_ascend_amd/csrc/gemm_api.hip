@@ -59,6 +59,21 @@ int gemm_w8a8_rescale_splitk(const void* A, const void* B, const void* scale_a, 
                              int64_t M, int64_t N, int64_t K, int64_t n_scale_b, int64_t split, int b_layout, int out_dtype,
                              hipStream_t st);
 
+// the small-tile kernel of these products (gemm_small.hip); kinds of weights: 0 [N, K], 1 int8 [K, N], 2 16-bit [K, N], 3 packed int4 [N, K / 2]
+struct SmallTile {
+  bool ok;
+  int mt, rt, waves;
+  double us;
+};
+SmallTile small_tile_plan(int kind, int64_t batch, int64_t M, int64_t N, int64_t row_bytes);
+bool small_tile_forced();
+int small_i8(const SmallTile& t, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int b_layout, hipStream_t st);
+int small_w8a8(const SmallTile& t, const void* A, const void* B, const void* scale_a, const void* scale_b, void* C, int64_t batch, int64_t M, int64_t N, int64_t K,
+               int64_t n_scale_b, int b_layout, int out_dtype, hipStream_t st);
+int small_w4a8(const SmallTile& t, const void* A, const void* Wp, void* C, int64_t M, int64_t N, int64_t K, int sign_mode, hipStream_t st);
+int small_f16(const SmallTile& t, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype, int out_dtype, hipStream_t st);
+extern thread_local int g_i8_tile, g_i8_split;
+
 struct PanelPlan {
   bool ok;
   int tiles_m, tiles_n, split, slice_steps;
@@ -1170,6 +1185,48 @@ int tlq_gemv_w4a16_batched(const void* A, const void* w_packed, const void* scal
                     (hipStream_t)stream);
 }
 
+// Is the small-tile kernel's estimate below what the kernels with 128-wide tiles take?  Theirs were fitted to the same 970 problems, apart
+// for the calls that cut K into slices (8 - 9 us before anything is multiplied: two or three launches) and those that do not
+// (16-bit and W4A8: 10 and 6 us per thousand of K whatever M and N); 7 - 17 % rms.  With these bars it is ahead by 1.1 - 1.5 x on average on what it
+// takes and lost more than 5 % on 20 of the 970, 27 % at most.
+static bool small_tile_wins(const SmallTile& t, int kind, int64_t batch, int64_t M, int64_t N, int64_t K) {
+  if (!t.ok || small_tile_forced()) return t.ok;
+  const double g = (double)batch * (double)M * (double)N * (double)K * 1e-9, g32 = (double)batch * (double)ceil_div(M, (int64_t)32) * 32.0 * (double)N * (double)K * 1e-9;
+  const double nk = (double)batch * (double)N * (double)K * 1e-6, mn = (double)batch * (double)M * (double)N * 1e-6, k = (double)K * 1e-3;
+  const double tiles_k = (double)batch * (double)ceil_div(M, (int64_t)128) * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6;
+  auto sliced = [&](double pace) { return batch == 1 && slice_choice(M, N, K, true, pace, 0) > 1; };
+  switch (kind) {
+    case 0: return t.us < 0.92 * (sliced(1.0) ? 8.4 + 0.12 * g + 0.065 * nk + 8.7 * mn + 0.12 * k + 0.65 * g32 : 5.1 + 1.4 * g + 0.16 * mn + 2.07 * k);
+    case 1: return t.us < 0.88 * (sliced(1.0) ? 8.6 + 1.84 * g + 0.073 * nk + 0.97 * mn + 0.073 * k + 1.08 * g32
+                                                                           : 4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32);
+    case 2: return t.us < 0.9 * (batch == 1 && slice_choice(M, N, K * 2, true, 1.0, 0) > 1 ? 8.3 + 0.049 * nk + 2.2 * mn + 0.17 * k + 2.9 * g32 + 10.9 * tiles_k
+                                                                     : 3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * tiles_k);
+    default: return t.us < 0.95 * (M <= 256 && sliced(2.5) ? 8.9 + 2.5 * g + 4.7 * mn + 0.24 * k + 6.2 * tiles_k
+                                                                                         : 4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
+  }
+}
+static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t K, int kind) {
+  const SmallTile t{false, 0, 0, 0, 0.0};
+  if (batch < 1 || M < 1 || N < 1 || K < 128 || K % 128 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_i8_tile || g_i8_split) return t;
+  static thread_local PlanTable<SmallTile> known;
+  return known.get(M, N, K, kind + 4 * batch, [&] {
+    SmallTile p = small_tile_plan(kind, batch, M, N, K);
+    p.ok = small_tile_wins(p, kind, batch, M, N, K);
+    return p;
+  });
+}
+static SmallTile small_tile_for_f16(int64_t batch, int64_t M, int64_t N, int64_t K, int b_layout) {
+  const SmallTile t{false, 0, 0, 0, 0.0};
+  if (b_layout != TLQ_B_KN || batch < 1 || M < 1 || N < 1 || K < 64 || K % 64 != 0 || N % 8 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_gemm_f16_tile || g_gemm_slots == 2)
+    return t;
+  static thread_local PlanTable<SmallTile> known;
+  return known.get(M, N, K, batch, [&] {
+    SmallTile p = small_tile_plan(2, batch, M, N, K * 2);
+    p.ok = small_tile_wins(p, 2, batch, M, N, K);
+    return p;
+  });
+}
+
 int tlq_gemm_f16_batched(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype,
                          int out_dtype, int b_layout, void* stream) {
   TLQ_CHECK_DIMS("tlq_gemm_f16");
@@ -1187,6 +1244,7 @@ int tlq_gemm_f16_batched(const void* A, const void* B, void* C, int64_t batch, i
   TLQ_REQUIRE(fits32(M, K * 2) && fits32(N, K * 2), "tlq_gemm_f16: a matrix spans 4 GiB or more");
   TLQ_REQUIRE(batch == 1 || (((M * K) % 8 == 0) && ((M * N) % 8 == 0)),
               "tlq_gemm_f16: every matrix of a batch must start on a 16-byte boundary (M*K and M*N multiples of 8)");
+  if (const SmallTile t = small_tile_for_f16(batch, M, N, K, b_layout); t.ok) return small_f16(t, A, B, C, batch, M, N, K, in_dtype, out_dtype, (hipStream_t)stream);
   return gemm_f16_plain(A, B, C, batch, M, N, K, in_dtype, out_dtype, b_layout, (hipStream_t)stream);
 }
 
@@ -1210,7 +1268,7 @@ int tlq_gemm_f16_ws(const void* A, const void* B, void* C, void* workspace, int6
     split = f16_split_choice(batch, M, N, K);
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;
   }
-  if (split <= 1) return tlq_gemm_f16_batched(A, B, C, batch, M, N, K, in_dtype, out_dtype, b_layout, stream);
+  if (split <= 1 || (g_f16_split == 0 && small_tile_for_f16(batch, M, N, K, b_layout).ok)) return tlq_gemm_f16_batched(A, B, C, batch, M, N, K, in_dtype, out_dtype, b_layout, stream);
   TLQ_REQUIRE(in_dtype == TLQ_F16 || in_dtype == TLQ_BF16, "tlq_gemm_f16_ws: in_dtype must be float16 or bfloat16 (got %d)",
               in_dtype);
   TLQ_REQUIRE(out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32, "tlq_gemm_f16_ws: bad out_dtype %d",
@@ -1253,6 +1311,7 @@ int tlq_gemm_i8(const void* A, const void* B, void* C, int64_t batch, int64_t M,
   TLQ_REQUIRE(A && B && C, "tlq_gemm_i8: null pointer");
   TLQ_REQUIRE(aligned16(A) && aligned16(B) && aligned16(C), "tlq_gemm_i8: pointers must be 16-byte aligned");
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K), "tlq_gemm_i8: a matrix spans 4 GiB or more");
+  if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1); t.ok) return small_i8(t, A, B, C, batch, M, N, K, b_layout, (hipStream_t)stream);
   // few activation rows: K slices add into C itself (int32, exact in any order)
   if (const int split = i8_split_choice(batch, M, N, K, false); split > 1)
     return gemm_i8_i32_splitk(A, B, (int32_t*)C, M, N, K, split, b_layout, (hipStream_t)stream);
@@ -1269,6 +1328,7 @@ int tlq_gemm_w4a8(const void* A, const void* w_packed, void* C, int64_t M, int64
   TLQ_REQUIRE(A && w_packed && C, "tlq_gemm_w4a8: null pointer");
   TLQ_REQUIRE(aligned16(A) && aligned16(w_packed) && aligned16(C), "tlq_gemm_w4a8: pointers must be 16-byte aligned");
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K / 2), "tlq_gemm_w4a8: a matrix spans 4 GiB or more");
+  if (const SmallTile t = small_tile_for_i8(1, M, N, K, 3); t.ok) return small_w4a8(t, A, w_packed, C, M, N, K, sign_mode, (hipStream_t)stream);
   // few activation rows: K slices add into C (int32, exact in any order)
   if (const int split = i8_split_choice(1, M, N, K, false, 2.5); split > 1)
     return gemm_w4a8_i32_splitk(A, w_packed, C, M, N, K, sign_mode, split, nullptr, (hipStream_t)stream);
@@ -1283,6 +1343,7 @@ int tlq_gemm_w4a8_ws(const void* A, const void* w_packed, void* workspace, int64
   // steps -- unpack into the workspace, int8 GEMM on it -- each at its own roofline (M = N = K = 4096: 6 + 66 us against
   // 98 us fused; M = 1024: 37 against 65 us).  Few rows (the unpack pass would cost more than the GEMM): the kernel that
   // unpacks on the way into LDS over K slices, the workspace holding one int32 [M, N] matrix per slice.
+  if (g_w4a8_ws_mode == 0 && small_tile_for_i8(1, M, N, K, 3).ok) return tlq_gemm_w4a8(A, w_packed, C, M, N, K, sign_mode, stream);
   const bool usable = workspace != nullptr && aligned16(workspace) && N > 0 && K > 0 && M > 0 && M < kMaxDim && N < kMaxDim &&
                       K < kMaxDim && fits32(N, K / 2) && fits32(M, K);
   if (usable && K % 32 == 0 && N % 4 == 0 && g_w4a8_ws_mode != 2 && (M <= 256 || g_w4a8_ws_mode == 1)) {
@@ -1322,6 +1383,8 @@ int tlq_gemm_w8a8(const void* A, const void* B, const void* scale_a, const void*
   TLQ_REQUIRE(aligned16(A) && aligned16(B) && aligned16(C), "tlq_gemm_w8a8: pointers must be 16-byte aligned");
   TLQ_REQUIRE(((uintptr_t)scale_a & 3) == 0 && ((uintptr_t)scale_b & 3) == 0, "tlq_gemm_w8a8: scales misaligned");
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K), "tlq_gemm_w8a8: a matrix spans 4 GiB or more");
+  if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1); t.ok)
+    return small_w8a8(t, A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype, (hipStream_t)stream);
   return gemm_w8a8_rescale(A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype,
                            (hipStream_t)stream);
 }
@@ -1347,7 +1410,7 @@ int tlq_gemm_w8a8_ws(const void* A, const void* B, const void* scale_a, const vo
     split = i8_split_choice(batch, M, N, K, true);
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;  // as many slices as the workspace holds
   }
-  if (split <= 1)
+  if (split <= 1 || small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1).ok)
     return tlq_gemm_w8a8(A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype, stream);
   TLQ_REQUIRE(b_layout == TLQ_B_KN || b_layout == TLQ_B_NK, "tlq_gemm_w8a8_ws: bad b_layout %d", b_layout);
   TLQ_REQUIRE(out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32, "tlq_gemm_w8a8_ws: bad out_dtype %d",

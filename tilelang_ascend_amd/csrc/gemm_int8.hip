@@ -109,7 +109,7 @@ static int run_i8(const void* A, const typename WL::Params& pw, const typename E
   return launch_gemm<MmaI8, AL, WL, Epi, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K, st, what, 2);
 }
 
-static thread_local int g_i8_tile = 0;
+thread_local int g_i8_tile = 0;
 
 static int pick_tile(int64_t batch, int64_t M, int64_t N) {
   if (g_i8_tile) return g_i8_tile;
@@ -209,7 +209,7 @@ static int run_i8_splitk(const void* A, const void* B, const typename Epi::Param
   return launch_gemm<MmaI8, AL, WL, Epi, BM, BN, WM, WN>(pa, pw, pe, split, M, N, ks, st, "tlq_gemm_i8 (K slices)", 2, (int)stages);
 }
 
-static thread_local int g_i8_split = 0;  // tlq_tune_i8_split: 0 = automatic, 1 = never, n = that many slices where K allows
+thread_local int g_i8_split = 0;  // tlq_tune_i8_split: 0 = automatic, 1 = never, n = that many slices where K allows
 
 // Number of K slices for one batch of [M,K] x [N,K] (slice_choice in gemm_core.h): `buffers`: every slice has an int32
 // [M,N] matrix of its own, otherwise the slices add into one matrix with atomic adds; `pace`: 2.5 for the loader that
