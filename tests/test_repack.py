@@ -173,3 +173,26 @@ def test_packed_weights_round_trip_through_a_file(tmp_path):
     torch.save({"format": "something else"}, tmp_path / "other.pt")
     with pytest.raises(ValueError):
         load_packed(tmp_path / "other.pt")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_quantizer_scales_of_every_size(dtype):
+    """The quotients by reciprocal and the division behind them: group maxima over the type's whole range (subnormal scales, bfloat16 scales on
+    both sides of 2^-96 and 2^96), values on the ties of the quotient, infinities and NaN."""
+    from tilelang_ascend_amd.quantize import gpu
+
+    g = torch.Generator().manual_seed(11)
+    lo, hi = (-24, 15) if dtype is torch.float16 else (-130, 126)
+    top = torch.exp2(torch.arange(lo, hi, dtype=torch.float64)) * 1.37
+    frac = torch.cat([(torch.arange(-32, 32) + 0.0) / 32, torch.rand(64, generator=g, dtype=torch.float64) * 2 - 1])
+    W = (top[:, None] * frac).to(dtype)
+    W[0, 5], W[1, 9], W[2, 3] = float("nan"), float("inf"), -float("inf")
+    W = W.repeat(1, 2).contiguous()
+    s_want = (W.view(-1, 2, 128).float().abs().nan_to_num(0, float("inf")).amax(2) * 0.125).to(dtype)
+    q, s = gpu.quantize_sym4(W.cuda(), 128)
+    assert torch.equal(s.cpu(), s_want)
+    # IEEE division on the host, rounded to the type, then to the nearest even whole number; NaN and a scale of 0 are the lower bound
+    f = torch.round((W.view(-1, 2, 128).float() / s_want.float()[:, :, None]).to(dtype).float())
+    want = torch.where(f.isnan() | (s_want.float()[:, :, None] == 0), torch.full_like(f, -8.0), f.clamp(-8, 8)).to(torch.int8).view_as(W)
+    assert torch.equal(q.cpu(), want)
