@@ -114,6 +114,7 @@ int gemm_w4a16_decode(const void* A, const void* Wp, const void* scales, const v
                       hipStream_t st);
 
 thread_local int g_gemm_band_rows = 0;
+thread_local int g_gemm_groups = 0;
 thread_local int g_gemm_slots = 1;  // tlq_tune_gemm_slots: 0 = never the five-slot kernel, 1 = where it measured faster, 2 = wherever it can run
 extern thread_local int g_gemm_f16_tile;
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -194,6 +195,7 @@ using namespace tlq;
 
 extern "C" {
 
+void tlq_tune_gemm_groups(int variant) { tlq::tuning_changed(), tlq::g_gemm_groups = variant < 0 || variant > 5 ? 0 : variant; }
 void tlq_tune_gemm_band(int tile_rows) { tlq::g_gemm_band_rows = tile_rows < 0 ? 0 : tile_rows; }
 void tlq_tune_gemm_slots(int mode) { tlq::g_gemm_slots = mode < 0 ? 0 : (mode > 2 ? 2 : mode); }
 int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused) {
@@ -1185,8 +1187,30 @@ int tlq_gemv_w4a16_batched(const void* A, const void* w_packed, const void* scal
                     (hipStream_t)stream);
 }
 
+// The estimate of the 128-row tiles with K over groups of wavefronts (gemm_core.h), where those would run; far off otherwise.
+static double group_tile_us(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes) {
+  double us = 0.0;
+  if (M <= 32 || N < 1 || k_bytes < 1 || !prefer_small_tiles(batch, M, N) || group_tile(kind, batch, M, N, k_bytes, &us) == 0) return 1e30;
+  return us;
+}
+// What a call takes that cuts K into slices over work-groups and adds them in a further launch, by SmallW kind: 8 - 9 us before
+// anything is multiplied.
+static double sliced_us(int kind, int64_t batch, int64_t M, int64_t N, int64_t K) {
+  const double g = (double)batch * (double)M * (double)N * (double)K * 1e-9, g32 = (double)batch * (double)ceil_div(M, (int64_t)32) * 32.0 * (double)N * (double)K * 1e-9;
+  const double nk = (double)batch * (double)N * (double)K * 1e-6, mn = (double)batch * (double)M * (double)N * 1e-6, k = (double)K * 1e-3;
+  const double tiles_k = (double)batch * (double)ceil_div(M, (int64_t)128) * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6;
+  switch (kind) {
+    case 0: return 8.4 + 0.12 * g + 0.065 * nk + 8.7 * mn + 0.12 * k + 0.65 * g32;
+    case 1: return 8.6 + 1.84 * g + 0.073 * nk + 0.97 * mn + 0.073 * k + 1.08 * g32;
+    case 2: return 8.3 + 0.049 * nk + 2.2 * mn + 0.17 * k + 2.9 * g32 + 10.9 * tiles_k;
+    default: return 8.9 + 2.5 * g + 4.7 * mn + 0.24 * k + 6.2 * tiles_k;
+  }
+}
+static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes) {
+  return group_tile_us(tile, 1, M, N, k_bytes) < 0.9 * sliced_us(kind, 1, M, N, K);
+}
 // Is the small-tile kernel's estimate below what the kernels with 128-wide tiles take?  Theirs were fitted to the same 970 problems, apart
-// for the calls that cut K into slices (8 - 9 us before anything is multiplied: two or three launches) and those that do not
+// for the calls that cut K into slices (sliced_us) and those that do not
 // (16-bit and W4A8: 10 and 6 us per thousand of K whatever M and N); 7 - 17 % rms.  With these bars it is ahead by 1.1 - 1.5 x on average on what it
 // takes and lost more than 5 % on 20 of the 970, 27 % at most.
 static bool small_tile_wins(const SmallTile& t, int kind, int64_t batch, int64_t M, int64_t N, int64_t K) {
@@ -1196,13 +1220,12 @@ static bool small_tile_wins(const SmallTile& t, int kind, int64_t batch, int64_t
   const double tiles_k = (double)batch * (double)ceil_div(M, (int64_t)128) * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6;
   auto sliced = [&](double pace) { return batch == 1 && slice_choice(M, N, K, true, pace, 0) > 1; };
   switch (kind) {
-    case 0: return t.us < 0.92 * (sliced(1.0) ? 8.4 + 0.12 * g + 0.065 * nk + 8.7 * mn + 0.12 * k + 0.65 * g32 : 5.1 + 1.4 * g + 0.16 * mn + 2.07 * k);
-    case 1: return t.us < 0.88 * (sliced(1.0) ? 8.6 + 1.84 * g + 0.073 * nk + 0.97 * mn + 0.073 * k + 1.08 * g32
-                                                                           : 4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32);
-    case 2: return t.us < 0.9 * (batch == 1 && slice_choice(M, N, K * 2, true, 1.0, 0) > 1 ? 8.3 + 0.049 * nk + 2.2 * mn + 0.17 * k + 2.9 * g32 + 10.9 * tiles_k
-                                                                     : 3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * tiles_k);
-    default: return t.us < 0.95 * (M <= 256 && sliced(2.5) ? 8.9 + 2.5 * g + 4.7 * mn + 0.24 * k + 6.2 * tiles_k
-                                                                                         : 4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
+    case 0: return t.us < 0.92 * (sliced(1.0) ? sliced_us(0, batch, M, N, K) : 5.1 + 1.4 * g + 0.16 * mn + 2.07 * k) && t.us < 1.05 * group_tile_us(kTileI8NK, batch, M, N, K);
+    case 1: return t.us < 0.88 * (sliced(1.0) ? sliced_us(1, batch, M, N, K) : 4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32) &&
+                   t.us < 1.05 * group_tile_us(kTileI8KN, batch, M, N, K);
+    case 2: return t.us < 0.9 * (batch == 1 && slice_choice(M, N, K * 2, true, 1.0, 0) > 1 ? sliced_us(2, batch, M, N, K) : 3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * tiles_k) &&
+                   t.us < 1.05 * group_tile_us(kTileF16KN, batch, M, N, K * 2);
+    default: return t.us < 0.95 * (M <= 256 && sliced(2.5) ? sliced_us(3, batch, M, N, K) : 4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
   }
 }
 static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t K, int kind) {
@@ -1268,7 +1291,9 @@ int tlq_gemm_f16_ws(const void* A, const void* B, void* C, void* workspace, int6
     split = f16_split_choice(batch, M, N, K);
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;
   }
-  if (split <= 1 || (g_f16_split == 0 && small_tile_for_f16(batch, M, N, K, b_layout).ok)) return tlq_gemm_f16_batched(A, B, C, batch, M, N, K, in_dtype, out_dtype, b_layout, stream);
+  if (g_f16_split == 0 && split > 1 && (small_tile_for_f16(batch, M, N, K, b_layout).ok || groups_beat_slices(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, 2, M, N, K, K * 2)))
+    split = 1;
+  if (split <= 1) return tlq_gemm_f16_batched(A, B, C, batch, M, N, K, in_dtype, out_dtype, b_layout, stream);
   TLQ_REQUIRE(in_dtype == TLQ_F16 || in_dtype == TLQ_BF16, "tlq_gemm_f16_ws: in_dtype must be float16 or bfloat16 (got %d)",
               in_dtype);
   TLQ_REQUIRE(out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32, "tlq_gemm_f16_ws: bad out_dtype %d",
@@ -1313,7 +1338,8 @@ int tlq_gemm_i8(const void* A, const void* B, void* C, int64_t batch, int64_t M,
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K), "tlq_gemm_i8: a matrix spans 4 GiB or more");
   if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1); t.ok) return small_i8(t, A, B, C, batch, M, N, K, b_layout, (hipStream_t)stream);
   // few activation rows: K slices add into C itself (int32, exact in any order)
-  if (const int split = i8_split_choice(batch, M, N, K, false); split > 1)
+  if (const int split = i8_split_choice(batch, M, N, K, false);
+      split > 1 && (g_i8_split || !groups_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
     return gemm_i8_i32_splitk(A, B, (int32_t*)C, M, N, K, split, b_layout, (hipStream_t)stream);
   return gemm_i8_i32(A, B, C, batch, M, N, K, b_layout, (hipStream_t)stream);
 }
@@ -1410,7 +1436,8 @@ int tlq_gemm_w8a8_ws(const void* A, const void* B, const void* scale_a, const vo
     split = i8_split_choice(batch, M, N, K, true);
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;  // as many slices as the workspace holds
   }
-  if (split <= 1 || small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1).ok)
+  if (split <= 1 || small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1).ok ||
+      (!g_i8_split && groups_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
     return tlq_gemm_w8a8(A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype, stream);
   TLQ_REQUIRE(b_layout == TLQ_B_KN || b_layout == TLQ_B_NK, "tlq_gemm_w8a8_ws: bad b_layout %d", b_layout);
   TLQ_REQUIRE(out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32, "tlq_gemm_w8a8_ws: bad out_dtype %d",

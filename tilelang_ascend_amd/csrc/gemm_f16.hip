@@ -88,7 +88,7 @@ struct H16KNLoader {
 // tlq_tune_gemm_tile: 0 = automatic, 128 / 256 = that square tile
 thread_local int g_gemm_f16_tile = 0;
 
-template <class Mma, int BM, int BN, int WM, int WN>
+template <class Mma, int BM, int BN, int WM, int WN, int KG = 1>
 static int run_f16(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int out_dtype,
                    int b_layout, hipStream_t st) {
   constexpr int NT = WM * WN * 64;
@@ -98,16 +98,19 @@ static int run_f16(const void* A, const void* B, void* C, int64_t batch, int64_t
   if (b_layout == TLQ_B_NK) {
     typedef RowLoaderDirect<BN, NT> WL;
     typename WL::Params pw{(const uint8_t*)B, K * 2, N * K * 2, K * 2};
-    return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
+    return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN, KG>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
   }
   if (N % 8 == 0) {  // [K, N] rows are whole 16-byte chunks: copied as they are, transposed by the operand read
     typedef H16KNLoaderDirect<BN, NT> WL;
     H16KNParams pw{(const uint8_t*)B, N * 2, K * N * 2, K};
+    return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN, KG>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
+  }
+  if constexpr (KG == 1) {
+    typedef H16KNLoader<BN, NT> WL;
+    typename WL::Params pw{(const uint8_t*)B, N * 2, K * N * 2, K};
     return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
   }
-  typedef H16KNLoader<BN, NT> WL;
-  typename WL::Params pw{(const uint8_t*)B, N * 2, K * N * 2, K};
-  return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
+  return 1;  // (groups of wavefronts are not asked for there)
 }
 
 // Split-K: slice z of K is "batch" z of the loaders (the batch strides step along K), and every slice
@@ -200,8 +203,12 @@ template <class Mma>
 static int dispatch_f16(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int out_dtype,
                         int b_layout, hipStream_t st) {
   const bool small = g_gemm_f16_tile ? g_gemm_f16_tile == 128 : prefer_small_tiles(batch, M, N);
-  if (small)
-    return run_f16<Mma, 128, 128, 2, 2>(A, B, C, batch, M, N, K, out_dtype, b_layout, st);
+  if (small) {
+    const int variant = b_layout == TLQ_B_NK || N % 8 == 0 ? group_tile(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, batch, M, N, K * 2) : 0;
+#define TLQ_RUN(BM, BN, WM, WN, KG) return run_f16<Mma, BM, BN, WM, WN, KG>(A, B, C, batch, M, N, K, out_dtype, b_layout, st);
+    TLQ_GROUP_TILES(variant, TLQ_RUN)
+#undef TLQ_RUN
+  }
   // (the five-slot kernel only on request: alternating runs on one box have the two-stage loop 3 - 14 % ahead on ten of
   // twelve 16-bit shapes, 2 % behind on the other two)
   if (g_gemm_slots == 2 && b_layout == TLQ_B_NK && K % 64 == 0) {  // whole 128-byte stages

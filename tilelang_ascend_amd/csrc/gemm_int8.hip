@@ -100,13 +100,13 @@ struct W4I8Loader {
 };
 
 // ---- launch helpers -----------------------------------------------------------------------
-template <class WL, class Epi, int BM, int BN, int WM, int WN>
+template <class WL, class Epi, int BM, int BN, int WM, int WN, int KG = 1>
 static int run_i8(const void* A, const typename WL::Params& pw, const typename Epi::Params& pe, int64_t batch,
                   int64_t M, int64_t N, int64_t K, hipStream_t st, const char* what) {
   constexpr int NT = WM * WN * 64;
   typedef RowLoaderDirect<BM, NT> AL;  // activations travel global -> LDS without passing through registers
   typename AL::Params pa{(const uint8_t*)A, K, M * K, K};
-  return launch_gemm<MmaI8, AL, WL, Epi, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K, st, what, 2);
+  return launch_gemm<MmaI8, AL, WL, Epi, BM, BN, WM, WN, KG>(pa, pw, pe, batch, M, N, K, st, what, 2);
 }
 
 thread_local int g_i8_tile = 0;
@@ -131,19 +131,19 @@ static int dispatch_i8(const void* A, const void* B, const typename Epi::Params&
       typename WL::Params pw{(const uint8_t*)B, N, K * N, K};
       return launch_gemm_slots<MmaI8, WL, Epi>(pa, pw, pe, batch, M, N, K, st, what, 2);
     }
-#define TLQ_RUN(BM, BN, WM, WN)                                               \
+#define TLQ_RUN(BM, BN, WM, WN, KG)                                               \
   {                                                                           \
     typedef I8KNLoaderDirect<BN, WM * WN * 64> WL;                            \
     typename WL::Params pw{(const uint8_t*)B, N, K * N, K};                   \
-    return run_i8<WL, Epi, BM, BN, WM, WN>(A, pw, pe, batch, M, N, K, st, what); \
+    return run_i8<WL, Epi, BM, BN, WM, WN, KG>(A, pw, pe, batch, M, N, K, st, what); \
   }
     switch (tile) {
       case 32:
-        TLQ_RUN(32, 128, 1, 4)
+        TLQ_RUN(32, 128, 1, 4, 1)
       case 128:
-        TLQ_RUN(128, 128, 2, 2)
+        TLQ_GROUP_TILES(group_tile(kTileI8KN, batch, M, N, K), TLQ_RUN)
       default:
-        TLQ_RUN(256, 256, 2, 4)
+        TLQ_RUN(256, 256, 2, 4, 1)
     }
 #undef TLQ_RUN
   } else {
@@ -151,19 +151,19 @@ static int dispatch_i8(const void* A, const void* B, const typename Epi::Params&
       typename RowLoaderDirect<256, 512>::Params pa{(const uint8_t*)A, K, M * K, K}, pw{(const uint8_t*)B, K, N * K, K};
       return launch_gemm_slots<MmaI8, RowLoaderDirect<256, 512>, Epi>(pa, pw, pe, batch, M, N, K, st, what, 2);
     }
-#define TLQ_RUN(BM, BN, WM, WN)                                               \
+#define TLQ_RUN(BM, BN, WM, WN, KG)                                               \
   {                                                                           \
     typedef RowLoaderDirect<BN, WM * WN * 64> WL;                             \
     typename WL::Params pw{(const uint8_t*)B, K, N * K, K};                   \
-    return run_i8<WL, Epi, BM, BN, WM, WN>(A, pw, pe, batch, M, N, K, st, what); \
+    return run_i8<WL, Epi, BM, BN, WM, WN, KG>(A, pw, pe, batch, M, N, K, st, what); \
   }
     switch (tile) {
       case 32:
-        TLQ_RUN(32, 128, 1, 4)
+        TLQ_RUN(32, 128, 1, 4, 1)
       case 128:
-        TLQ_RUN(128, 128, 2, 2)
+        TLQ_GROUP_TILES(group_tile(kTileI8NK, batch, M, N, K), TLQ_RUN)
       default:
-        TLQ_RUN(256, 256, 2, 4)
+        TLQ_RUN(256, 256, 2, 4, 1)
     }
 #undef TLQ_RUN
   }
