@@ -1,0 +1,45 @@
+"""W4A16 above 512 rows: where the automatic choice takes the two passes by estimate (row counts that are no multiple of four, many rounds of short
+rows, few output tiles), with room for them and -- the kernels that ran before -- without."""
+import pytest
+import torch
+
+from helpers import gen
+from tilelang_ascend_amd import _abi
+
+# 639: three rows over; 4868: short rows in a round and a sixteenth; 614 / 667: few output tiles; 1037: one row over, two stages of K per step
+SHAPES = [(639, 5680, 896, 128), (4868, 3152, 384, 128), (614, 1392, 2304, 128), (667, 256, 12288, 128), (1037, 3488, 384, 64)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,group", SHAPES)
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tensor", [True, False])
+def test_two_passes_by_estimate(M, N, K, group, dt, tensor):
+    print(f"two passes M={M} N={N} K={K} g={group} {dt} tensor={tensor}", flush=True)
+    lib, P, st = _abi.load(), _abi.ptr, torch.cuda.current_stream().cuda_stream
+    code = _abi.F16 if dt is torch.float16 else _abi.BF16
+    A = torch.randn(M, K, generator=gen(1)).to(dt).cuda()
+    W = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=gen(2)).cuda()
+    S = (torch.rand(N, K // group, generator=gen(3)) * 0.015 + 0.005).to(dt).cuda()
+    Z = torch.randint(6, 10, (N, K // group), generator=gen(4)).to(dt).cuda() if tensor else None
+    u = torch.stack([W & 15, W >> 4], -1).reshape(N, K // group, group).to(dt)
+    w = ((u - (Z[:, :, None] if tensor else torch.tensor(8, dtype=dt, device="cuda"))) * S[:, :, None]).reshape(N, K)  # each operation rounded to dt
+    want, size = A.double() @ w.double().T, A.double().abs() @ w.double().abs().T
+    # fp32 sums of K exact products (partial sums in any order), then the result's own rounding
+    tol = K * 2.0**-24 * size + (2.0**-11 if dt is torch.float16 else 2.0**-8) * (want.abs() + K * 2.0**-24 * size) + 2.0**-25
+    full = lib.tlq_w4a16_workspace_bytes(M, N, K)
+    for size_ws in (full, N * K * 2, 0):
+        ws = torch.empty(size_ws + 16, dtype=torch.uint8, device="cuda")
+        C = torch.full((M, N), float("nan"), dtype=dt, device="cuda")
+        lib.tlq_debug_launch_log(1)
+        rc = lib.tlq_gemm_w4a16_ws(P(A), P(W), P(S), P(Z) if tensor else None, P(C), M, N, K, group, 0.0 if tensor else 8.0, code, code, _abi.ALGO_AUTO,
+                                   P(ws) if size_ws else None, size_ws, st)
+        log = lib.tlq_debug_launch_log_text().decode()
+        lib.tlq_debug_launch_log(0)
+        _abi.check(rc)
+        torch.cuda.synchronize()
+        assert ("dequant_w4" in log) == (size_ws > 0) or lib.tlq_device_cu_count() != 256, log
+        # (without room the last rows go to the GEMV, which applies scale and zero point to the group's sum: its weights are not rounded to dt,
+        # half an ulp each)
+        bound = tol if size_ws else tol + (2.0**-11 if dt is torch.float16 else 2.0**-8) * size
+        assert bool(((C.double() - want).abs() <= bound).all())

@@ -14,6 +14,7 @@ int gemv_w4a16_ring_interleaved(const void* A, const void* Wp, const void* scale
 int gemm_w4a16_mfma(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                     int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, hipStream_t st);
 int64_t w4a16_mid_split(int64_t M, int64_t N, int64_t K, int64_t group);
+int w4a16_split_forced();
 double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group);
 int gemm_w4a16_mfma_splitk(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M,
                            int64_t N, int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype,
@@ -612,6 +613,28 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
   return (double)wgs / (double)(ceil_div(wgs, cus_now) * cus_now) >= kPanel256Fill;
 }
 
+// Above 512 rows: do the two passes beat what the panel kernels would run?  The dequantisation pass costs 3 us and the weights' bytes, the
+// plain GEMM behind it has smaller tiles, K in groups of wavefronts and any row count, while the panel kernels have 8 us per round of
+// work-groups (many rounds of short rows: 4868 x 3152 x 384 bf16 36.9 -> 25.5 us, 6631 x 4608 x 256 38.7 -> 29.8) and leave
+// one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  On 61 problems above
+// 512 rows the bar below takes the two passes on 23, none slower; a bar of one would have lost 2 - 5 % on three more.
+static double plain_nk_us(int64_t M, int64_t N, int64_t K);
+static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
+  const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
+  const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
+  const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
+  if (!p2.ok || N % 8 != 0) return false;
+  auto two_us = [&](int64_t rows) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(rows, N, K); };
+  double panels;
+  if (pm.ok && panelm_estimate_wins(head, N, K, group))
+    panels = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, head, N, cus_now);
+  else if (panel256_fills(head, N, K, group))
+    panels = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, head, N, cus_now);
+  else
+    panels = two_us(head);  // they would not run
+  return 1.1 * two_us(M) < 0.85 * (panels + (head != M ? 5.5 : 0.0));
+}
+
 // The panel kernel (large M, one launch, weights dequantised on the operand read).  Returns -1 when it does not take the
 // problem (nothing launched, no error set), else the launch's return code.
 static int try_panel(const void* A, const void* w_packed, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
@@ -773,6 +796,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       set_error("%s", "");
     }
   }
+  const bool room_for_two_passes = N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && workspace != nullptr && workspace_bytes >= N * K * 2 && aligned16(workspace);
   // Many rows on so few and short weight rows that the whole call is a matter of latency: the small-tile kernel
   if (algo == TLQ_ALGO_AUTO && M > 512 && M < kMaxDim && N >= 1 && N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && w_packed && C && aligned16(A) &&
       aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
@@ -791,7 +815,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       K < kMaxDim && group > 0 && A && C && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
       (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
     const int64_t head = M & ~(int64_t)3;
-    if (w4a16_panel256_plan(head, N, K, group, cu_count_or_default()).ok) {
+    if (w4a16_panel256_plan(head, N, K, group, cu_count_or_default()).ok && !(room_for_two_passes && two_passes_beat_panels(M, N, K, group))) {
       const int rc = tlq_gemm_w4a16_ws(A, w_packed, scales, zeros, C, head, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, workspace,
                                        workspace_bytes, stream);
       if (rc != 0) return rc;
@@ -1005,7 +1029,8 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // 576 and 2048 rows on wide or long matrices (N = 28672, K = 4096, M = 768: 1.40 - 1.54 x; N = 4096, K = 14336, M = 1280:
   // 1.50 - 1.56 x), 0.98 - 0.99 on a few of the largest fp16 problems -- and 2 - 21 % behind below that fill (N = K = 4096,
   // M <= 1024: 96 work-groups).  The 128-row kernel is ahead of it nowhere by more than 4 % and stays an explicit choice.
-  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && K > 0 && group > 0 && N >= 1 && N < kMaxDim && K < kMaxDim && M < kMaxDim) {
+  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && K > 0 && group > 0 && N >= 1 && N < kMaxDim && K < kMaxDim && M < kMaxDim &&
+      !(have && two_passes_beat_panels(M, N, K, group))) {
     // The middle-M kernel's 128-row tiles first where an estimate of both kernels' times says so: rounds of work-groups x
     // (steps per K slice x the time of a step + a fixed part) + the pass over the slices' partial tiles, with the step
     // times measured at a full machine (2.2 us on 128 rows, 3.3 us on 256) and fixed parts of 6 / 8 us.  On ten (N, K)
@@ -1024,7 +1049,11 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       if (rc >= 0) return rc;
     }
   }
-  const bool split_region = w4a16_mid_split(M, N, K, group > 0 ? group : 32) > 1;
+  // (above 512 rows only rows of 13312 values and more: below, the plain GEMM of the two passes, which cuts K over groups of wavefronts
+  // or unevenly over work-groups, is ahead: 614 x 1392 x 2304 28.7 -> 20.6 us, 667 x 256 x 12288 36.8 -> 25.3, 682 x 2288 x 11648
+  // 76.4 -> 66.3; 656 x 2496 x 3712 level)
+  const bool split_region = !(algo == TLQ_ALGO_AUTO && have && M > 512 && K < 13312 && N % 8 == 0 && w4a16_split_forced() == 0) &&
+                            w4a16_mid_split(M, N, K, group > 0 ? group : 32) > 1;
   const bool two_pass = algo == TLQ_ALGO_TWO_PASS ||
                         (algo == TLQ_ALGO_AUTO && have && M >= kTwoPassMinM && N % 8 == 0 && !split_region);
   if (!two_pass && (algo == TLQ_ALGO_AUTO || algo == TLQ_ALGO_MFMA) && M > 16 && workspace && aligned16(workspace) &&
@@ -1206,8 +1235,19 @@ static double sliced_us(int kind, int64_t batch, int64_t M, int64_t N, int64_t K
     default: return 8.9 + 2.5 * g + 4.7 * mn + 0.24 * k + 6.2 * tiles_k;
   }
 }
+static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes);
+static double plain_nk_us(int64_t M, int64_t N, int64_t K) {  // one 16-bit matrix of [N, K] weights
+  const int64_t stages = ceil_div(K * 2, (int64_t)kStageBytes);
+  if (!prefer_small_tiles(1, M, N)) return tile_us(kTileF16NK, 6, 1, M, N, stages);
+  if (f16_split_choice(1, M, N, K) > 1 && !groups_beat_slices(kTileF16NK, 2, M, N, K, K * 2)) return sliced_us(2, 1, M, N, K);
+  double us = 0.0;
+  group_tile(kTileF16NK, 1, M, N, K * 2, &us);
+  return us;
+}
 static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes) {
-  return group_tile_us(tile, 1, M, N, k_bytes) < 0.9 * sliced_us(kind, 1, M, N, K);
+  // (rows of more than 48 stages stay with the slices, which their estimate makes too dear on many activation rows: 3326 x 768 x 5504 44
+  // against 56 us in groups, 947 x 1664 x 6016 36 against 43, 7795 x 256 x 7808 54 against 78)
+  return k_bytes <= 48 * kStageBytes && group_tile_us(tile, 1, M, N, k_bytes) < 0.9 * sliced_us(kind, 1, M, N, K);
 }
 // Is the small-tile kernel's estimate below what the kernels with 128-wide tiles take?  Theirs were fitted to the same 970 problems, apart
 // for the calls that cut K into slices (sliced_us) and those that do not
@@ -1220,11 +1260,11 @@ static bool small_tile_wins(const SmallTile& t, int kind, int64_t batch, int64_t
   const double tiles_k = (double)batch * (double)ceil_div(M, (int64_t)128) * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6;
   auto sliced = [&](double pace) { return batch == 1 && slice_choice(M, N, K, true, pace, 0) > 1; };
   switch (kind) {
-    case 0: return t.us < 0.92 * (sliced(1.0) ? sliced_us(0, batch, M, N, K) : 5.1 + 1.4 * g + 0.16 * mn + 2.07 * k) && t.us < 1.05 * group_tile_us(kTileI8NK, batch, M, N, K);
+    case 0: return t.us < 0.92 * (sliced(1.0) ? sliced_us(0, batch, M, N, K) : 5.1 + 1.4 * g + 0.16 * mn + 2.07 * k) && t.us < 1.15 * group_tile_us(kTileI8NK, batch, M, N, K);
     case 1: return t.us < 0.88 * (sliced(1.0) ? sliced_us(1, batch, M, N, K) : 4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32) &&
-                   t.us < 1.05 * group_tile_us(kTileI8KN, batch, M, N, K);
+                   t.us < 1.15 * group_tile_us(kTileI8KN, batch, M, N, K);
     case 2: return t.us < 0.9 * (batch == 1 && slice_choice(M, N, K * 2, true, 1.0, 0) > 1 ? sliced_us(2, batch, M, N, K) : 3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * tiles_k) &&
-                   t.us < 1.05 * group_tile_us(kTileF16KN, batch, M, N, K * 2);
+                   t.us < 1.15 * group_tile_us(kTileF16KN, batch, M, N, K * 2);
     default: return t.us < 0.95 * (M <= 256 && sliced(2.5) ? sliced_us(3, batch, M, N, K) : 4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
   }
 }

@@ -461,6 +461,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4_t* __re
 // work-group's run of stages is latency bound: aim at one to two work-groups per CU (measured best on the
 // MLP shapes), slices of at least 512 values that are whole stages and whole quantisation groups.  1 = no split.
 static thread_local int g_w4a16_split = 0;  // forced number of K slices for tuning runs (0 = automatic)
+int w4a16_split_forced() { return g_w4a16_split; }
 
 // fraction of the work-group places (256, or 512 for the smaller tiles) that the tile kernel fills with the K cut it would take
 double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group);
