@@ -79,3 +79,35 @@ def test_taken_where_tiles_leave_one_work_group_to_a_cu(lib):
         C, dA, dW = torch.empty(M, N, dtype=torch.float16, device="cuda"), A.cuda(), W.cuda()
         lib.tlq_debug_launch_log(1)
         called(lib, lib.tlq_gemm_f16(P(dA), P(dW), P(C), M, N, K, _abi.F16, _abi.F16, _abi.B_KN, st), groups)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,launches", [(4099, 4096, 1024, 2), (4096, 4096, 1024, 1)])
+def test_rows_of_full_rounds_and_the_rest(lib, M, N, K, launches):
+    """One tile row too many for a round of the machine: the rest of the rows is a launch of its own (checked on a machine of 256 CUs), at the
+    right rows of the activations, the scales and the result."""
+    print(f"full rounds M={M} N={N} K={K}", flush=True)
+    P, st = _abi.ptr, torch.cuda.current_stream().cuda_stream
+    A = torch.randint(-127, 128, (M, K), dtype=torch.int8, generator=gen(1)).cuda()
+    W = torch.randint(-127, 128, (N, K), dtype=torch.int8, generator=gen(2)).cuda()
+    sa, sb = torch.rand(M, generator=gen(3)).cuda(), torch.rand(N, generator=gen(4)).cuda()
+    acc = (A.double() @ W.double().T).to(torch.int32)  # exact
+
+    def count(rc):
+        log = lib.tlq_debug_launch_log_text().decode()
+        lib.tlq_debug_launch_log(0)
+        _abi.check(rc)
+        torch.cuda.synchronize()
+        assert lib.tlq_device_cu_count() != 256 or log.count("[") == launches, log
+
+    C = torch.full((M, N), -1, dtype=torch.int32, device="cuda")
+    lib.tlq_debug_launch_log(1)
+    count(lib.tlq_gemm_i8(P(A), P(W), P(C), 1, M, N, K, _abi.B_NK, st))
+    assert torch.equal(C, acc)
+    for dt in CODE:
+        for scale in (sa, None):
+            out = torch.full((M, N), float("nan"), dtype=dt, device="cuda")
+            lib.tlq_debug_launch_log(1)
+            count(lib.tlq_gemm_w8a8(P(A), P(W), None if scale is None else P(scale), P(sb), P(out), 1, M, N, K, N, _abi.B_NK, CODE[dt], st))
+            want = ((acc.float() if scale is None else acc.float() * scale[:, None]) * sb).to(dt)
+            assert_bit_equal(out.cpu(), want.cpu(), f"rescaled {dt}")

@@ -1290,6 +1290,41 @@ static SmallTile small_tile_for_f16(int64_t batch, int64_t M, int64_t N, int64_t
   });
 }
 
+// A product whose last round of work-groups is nearly empty runs as two launches: the rows of the tiles that fill whole rounds, then
+// the rest by whatever is best for that many rows.  Returns the rows of the first, 0 = one launch.  (4099 rows on 4096 x 4096 int8 are 17 x 16
+// tiles of 256 x 256, a round of 256 and one of 16; one launch took 128 x 128 tiles instead, 96 us; 4096 rows and 3 take
+// 62 us.)
+static int64_t rows_of_full_rounds(TileKind kind, int64_t M, int64_t N, int64_t K) {
+  if (M <= 512 || N < 256 || K % 128 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_gemm_groups || g_gemm_f16_tile || g_i8_tile || g_gemm_slots == 2) return 0;
+  static thread_local PlanTable<int64_t> known;
+  return known.get(M, N, K, kind, [&]() -> int64_t {
+    const bool i8 = kind >= kTileI8KN;
+    const int64_t k_bytes = i8 ? K : 2 * K, stages = k_bytes / kStageBytes, cus = cu_count_or_default();
+    auto one_us = [&](int64_t rows) {
+      double us = 0.0;
+      if (!prefer_small_tiles(1, rows, N)) return tile_us(kind, 6, 1, rows, N, stages);
+      group_tile(kind, 1, rows, N, k_bytes, &us);
+      return us;
+    };
+    auto rest_us = [&](int64_t rows) {
+      const double us = one_us(rows);
+      if (kind == kTileF16NK) return us;
+      const SmallTile t = i8 ? small_tile_for_i8(1, rows, N, K, kind == kTileI8NK ? 0 : 1) : small_tile_for_f16(1, rows, N, K, TLQ_B_KN);
+      return t.ok && t.us < us ? t.us : us;
+    };
+    double best = 0.87 * one_us(M);
+    int64_t head = 0;
+    for (const int64_t tile : {(int64_t)256, (int64_t)128}) {
+      const int64_t across = ceil_div(N, tile), round = tile == 256 ? cus : 2 * cus, rounds = ceil_div(M, tile) * across / round;
+      const int64_t rows = rounds * round / across * tile;
+      if (rounds == 0 || rows <= 0 || rows >= M || prefer_small_tiles(1, rows, N) != (tile == 128)) continue;
+      const double us = one_us(rows) + 1.5 + rest_us(M - rows);
+      if (us < best) best = us, head = rows;
+    }
+    return head;
+  });
+}
+
 int tlq_gemm_f16_batched(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype,
                          int out_dtype, int b_layout, void* stream) {
   TLQ_CHECK_DIMS("tlq_gemm_f16");
@@ -1308,6 +1343,11 @@ int tlq_gemm_f16_batched(const void* A, const void* B, void* C, int64_t batch, i
   TLQ_REQUIRE(batch == 1 || (((M * K) % 8 == 0) && ((M * N) % 8 == 0)),
               "tlq_gemm_f16: every matrix of a batch must start on a 16-byte boundary (M*K and M*N multiples of 8)");
   if (const SmallTile t = small_tile_for_f16(batch, M, N, K, b_layout); t.ok) return small_f16(t, A, B, C, batch, M, N, K, in_dtype, out_dtype, (hipStream_t)stream);
+  if (const int64_t head = batch == 1 ? rows_of_full_rounds(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, M, N, K) : 0; head > 0) {
+    if (const int rc = tlq_gemm_f16_batched(A, B, C, 1, head, N, K, in_dtype, out_dtype, b_layout, stream)) return rc;
+    return tlq_gemm_f16_batched((const uint8_t*)A + head * K * 2, B, (uint8_t*)C + head * N * (out_dtype == TLQ_F32 ? 4 : 2), 1, M - head, N, K, in_dtype, out_dtype, b_layout,
+                                stream);
+  }
   return gemm_f16_plain(A, B, C, batch, M, N, K, in_dtype, out_dtype, b_layout, (hipStream_t)stream);
 }
 
@@ -1381,6 +1421,10 @@ int tlq_gemm_i8(const void* A, const void* B, void* C, int64_t batch, int64_t M,
   if (const int split = i8_split_choice(batch, M, N, K, false);
       split > 1 && (g_i8_split || !groups_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
     return gemm_i8_i32_splitk(A, B, (int32_t*)C, M, N, K, split, b_layout, (hipStream_t)stream);
+  if (const int64_t head = batch == 1 ? rows_of_full_rounds(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, M, N, K) : 0; head > 0) {
+    if (const int rc = tlq_gemm_i8(A, B, C, 1, head, N, K, b_layout, stream)) return rc;
+    return tlq_gemm_i8((const uint8_t*)A + head * K, B, (int32_t*)C + head * N, 1, M - head, N, K, b_layout, stream);
+  }
   return gemm_i8_i32(A, B, C, batch, M, N, K, b_layout, (hipStream_t)stream);
 }
 
@@ -1451,6 +1495,11 @@ int tlq_gemm_w8a8(const void* A, const void* B, const void* scale_a, const void*
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K), "tlq_gemm_w8a8: a matrix spans 4 GiB or more");
   if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1); t.ok)
     return small_w8a8(t, A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype, (hipStream_t)stream);
+  if (const int64_t head = batch == 1 ? rows_of_full_rounds(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, M, N, K) : 0; head > 0) {
+    if (const int rc = tlq_gemm_w8a8(A, B, scale_a, scale_b, C, 1, head, N, K, n_scale_b, b_layout, out_dtype, stream)) return rc;
+    return tlq_gemm_w8a8((const uint8_t*)A + head * K, B, scale_a ? (const float*)scale_a + head : nullptr, scale_b,
+                         (uint8_t*)C + head * N * (out_dtype == TLQ_F32 ? 4 : 2), 1, M - head, N, K, n_scale_b, b_layout, out_dtype, stream);
+  }
   return gemm_w8a8_rescale(A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype,
                            (hipStream_t)stream);
 }
