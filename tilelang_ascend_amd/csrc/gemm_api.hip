@@ -617,7 +617,7 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 // plain GEMM behind it has smaller tiles, K in groups of wavefronts and any row count, while the panel kernels have 8 us per round of
 // work-groups (many rounds of short rows: 4868 x 3152 x 384 bf16 36.9 -> 25.5 us, 6631 x 4608 x 256 38.7 -> 29.8) and leave
 // one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  On 61 problems above
-// 512 rows the bar below takes the two passes on 23, none slower; a bar of one would have lost 2 - 5 % on three more.
+// 512 rows the bar below takes the two passes on 22, none slower; a bar of one would have lost 2 - 5 % on three more.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
 static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
   const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
@@ -626,7 +626,9 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
   if (!p2.ok || N % 8 != 0) return false;
   auto two_us = [&](int64_t rows) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(rows, N, K); };
   double panels;
-  if (pm.ok && panelm_estimate_wins(head, N, K, group))
+  const bool middle = pm.ok && panelm_estimate_wins(head, N, K, group);
+  if (middle && N > 512) return false;  // (against the middle-M kernel and its tail measured on up to 512 weight rows, one or two of its tiles)
+  if (middle)
     panels = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, head, N, cus_now);
   else if (panel256_fills(head, N, K, group))
     panels = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, head, N, cus_now);
