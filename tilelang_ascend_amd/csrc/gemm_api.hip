@@ -287,6 +287,35 @@ static bool small_beats_decode_chunks(const SmallPlan& p, int64_t M, int64_t N, 
 }
 static bool decode_preferred(int64_t M, int64_t N, int64_t K) { return M > 2 || (M == 2 && N * K >= ((int64_t)1 << 24)); }
 
+// The kernel of tlq_gemm_w4a16 by its rules (up to 64 rows; more rows come here only where every kernel above wants a workspace).
+static bool w4a16_decode_in_one_chunk(const DecodePlan& dp, const void* scales, const void* zeros) {
+  return dp.ok && dp.chunks == 1 && (((uintptr_t)scales | (uintptr_t)zeros) & 3) == 0;
+}
+static int w4a16_few_rows_choice(int64_t M, int64_t N, int64_t K, int64_t group, int in_dtype, const void* scales, const void* zeros, bool decode_ok) {
+  // The skinny kernel takes the same time for every M up to 16 (the weights bound it); the GEMV kernels grow with
+  // M.  Measured crossovers: fp16 GEMV wins at M = 1, and at M = 2 while K <= 4096; the bf16 GEMV dequantises
+  // element by element and wins only at M = 1 in its register-resident form (rows of up to 16384 values: level with the
+  // skinny kernel on 4096 weight rows, 15 against 25 us on 5120 rows of 13824 values).
+  const bool skinny_ok = M <= 64 && K % 128 == 0 && fits32(M, K * 2) && fits32(N, K / 2);
+  // two fp16 activation rows on many weight rows: the ring GEMV (8.9 against 10.3 us for the decode kernel at
+  // 11008 x 4096, 5.2 against 6.2 us at 8192 x 2048; with 4096 rows, one per wavefront, the decode kernel is 5 % ahead)
+  if (M == 2 && N >= 8192 && gemv_ring_applies(M, N, K, group, in_dtype, scales, zeros)) return TLQ_ALGO_GEMV;
+  if (decode_preferred(M, N, K) && decode_ok && g_w4a16_decode) return TLQ_ALGO_DECODE;
+  if (M > 4) return skinny_ok ? TLQ_ALGO_SKINNY : TLQ_ALGO_MFMA;
+  if (!skinny_ok) return TLQ_ALGO_GEMV;
+  if (in_dtype == TLQ_BF16) return (M == 1 && K <= 16384 && (group & (group - 1)) == 0) ? TLQ_ALGO_GEMV : TLQ_ALGO_SKINNY;
+  return ((M == 1 && K <= 16384) || (M == 2 && K <= 4096)) ? TLQ_ALGO_GEMV : TLQ_ALGO_SKINNY;  // (longer rows: no register-resident GEMV)
+}
+// Do the last M % 4 of many rows, run by themselves, go to the fp16 GEMV kernels?  Those apply scale and zero point to fp32 sums of
+// exact products, where every other kernel multiplies weights rounded to 16 bits: rows that have had that precision keep it.
+static bool last_rows_take_f16_gemv(int64_t M, int64_t N, int64_t K, int64_t group, int in_dtype, const void* scales, const void* zeros) {
+  const int64_t rows = M & 3;
+  if (rows == 0 || in_dtype != TLQ_F16) return false;
+  if (w4a16_choice_lookup(rows, N, K, group, in_dtype) == TLQ_ALGO_GEMV) return true;
+  const DecodePlan dp = w4a16_decode_plan(rows, N, K, group, cu_count_or_default());
+  return w4a16_few_rows_choice(rows, N, K, group, in_dtype, scales, zeros, w4a16_decode_in_one_chunk(dp, scales, zeros)) == TLQ_ALGO_GEMV;
+}
+
 int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, const void* zeros, void* C, int64_t M,
                    int64_t N, int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int algo,
                    void* stream) {
@@ -328,33 +357,13 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
   // The decode kernel (M <= 32): without a workspace only rows of up to 4096 values (one chunk of K).  Its scale / zero
   // gathers read aligned dwords: the tensors must start on a dword boundary (their length is checked by the plan).
   const DecodePlan dp = M <= 32 ? w4a16_decode_plan(M, N, K, group, cu_count_or_default()) : DecodePlan{false, 0, 0, 0, 0, 0};
-  const bool decode_ok = dp.ok && dp.chunks == 1 && (((uintptr_t)scales | (uintptr_t)zeros) & 3) == 0;
+  const bool decode_ok = w4a16_decode_in_one_chunk(dp, scales, zeros);
+  if (algo == TLQ_ALGO_AUTO) algo = w4a16_few_rows_choice(M, N, K, group, in_dtype, scales, zeros, decode_ok);
   if (algo == TLQ_ALGO_DECODE) {
     TLQ_REQUIRE(decode_ok, "tlq_gemm_w4a16: the decode kernel needs 1 <= M <= 32, K %% 256 == 0, K <= 4096 without a workspace, a power-of-two "
                 "group and dword-aligned scale / zero tensors (M=%lld N=%lld K=%lld group=%lld)", (long long)M, (long long)N, (long long)K,
                 (long long)group);
     return gemm_w4a16_decode(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, dp, nullptr, st);
-  }
-  if (algo == TLQ_ALGO_AUTO) {
-    // The skinny kernel takes the same time for every M up to 16 (the weights bound it); the GEMV kernels grow with
-    // M.  Measured crossovers: fp16 GEMV wins at M = 1, and at M = 2 while K <= 4096; the bf16 GEMV dequantises
-    // element by element and wins only at M = 1 in its register-resident form (rows of up to 16384 values: level with the
-    // skinny kernel on 4096 weight rows, 15 against 25 us on 5120 rows of 13824 values).
-    const bool skinny_ok = M <= 64 && K % 128 == 0 && fits32(M, K * 2) && fits32(N, K / 2);
-    // two fp16 activation rows on many weight rows: the ring GEMV (8.9 against 10.3 us for the decode kernel at
-    // 11008 x 4096, 5.2 against 6.2 us at 8192 x 2048; with 4096 rows, one per wavefront, the decode kernel is 5 % ahead)
-    if (M == 2 && N >= 8192 && gemv_ring_applies(M, N, K, group, in_dtype, scales, zeros))
-      return gemv_w4a16(A, w_packed, scales, zeros, C, 1, M, N, K, group, zero_scalar, in_dtype, out_dtype, st);
-    if (decode_preferred(M, N, K) && decode_ok && g_w4a16_decode)
-      return gemm_w4a16_decode(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, dp, nullptr, st);
-    if (M > 4)
-      algo = skinny_ok ? TLQ_ALGO_SKINNY : TLQ_ALGO_MFMA;
-    else if (!skinny_ok)
-      algo = TLQ_ALGO_GEMV;
-    else if (in_dtype == TLQ_BF16)
-      algo = (M == 1 && K <= 16384 && (group & (group - 1)) == 0) ? TLQ_ALGO_GEMV : TLQ_ALGO_SKINNY;
-    else
-      algo = ((M == 1 && K <= 16384) || (M == 2 && K <= 4096)) ? TLQ_ALGO_GEMV : TLQ_ALGO_SKINNY;  // (longer rows: no register-resident GEMV)
   }
   if (algo == TLQ_ALGO_SKINNY) {
     TLQ_REQUIRE(M <= 64, "tlq_gemm_w4a16: the skinny kernel handles M <= 64 (got %lld)", (long long)M);
@@ -799,8 +808,20 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     }
   }
   const bool room_for_two_passes = N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && workspace != nullptr && workspace_bytes >= N * K * 2 && aligned16(workspace);
+  // Above 512 rows the panel kernels are the fast path, and they take row counts that are multiples of four (their direct
+  // loads move four activation rows).  Any other count -- prompt lengths are what they are -- runs as its multiple of four
+  // below through the same choice plus the last one to three rows through the small-M kernels, which is one short launch
+  // more instead of the two passes for everything (measured: M = 1001, N = 14336, K = 4096: 147 us in one piece, 128 us for
+  // 1000 rows; M = 2049, N = K = 8192: 392 against 249 us; M = 601, N = K = 8192: 164 against 120 us; the tail takes 6 - 15 us).
+  // One launch or two passes for all rows instead, where their estimates say so -- but not where the last rows belong to the fp16
+  // GEMV kernels, whose results are closer to exact arithmetic.
+  const bool head_and_tail = algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && (M & 3) != 0 && M < kMaxDim && N >= 16 && N % 16 == 0 &&
+                             N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && C && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
+                             (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) &&
+                             w4a16_panel256_plan(M & ~(int64_t)3, N, K, group, cu_count_or_default()).ok;
+  const bool keep_tail = head_and_tail && last_rows_take_f16_gemv(M, N, K, group, in_dtype, scales, zeros);
   // Many rows on so few and short weight rows that the whole call is a matter of latency: the small-tile kernel
-  if (algo == TLQ_ALGO_AUTO && M > 512 && M < kMaxDim && N >= 1 && N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && w_packed && C && aligned16(A) &&
+  if (algo == TLQ_ALGO_AUTO && !keep_tail && M > 512 && M < kMaxDim && N >= 1 && N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && w_packed && C && aligned16(A) &&
       aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
       (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
     const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
@@ -808,23 +829,14 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                               (hipStream_t)stream);
   }
-  // Above 512 rows the panel kernels are the fast path, and they take row counts that are multiples of four (their direct
-  // loads move four activation rows).  Any other count -- prompt lengths are what they are -- runs as its multiple of four
-  // below through the same choice plus the last one to three rows through the small-M kernels, which is one short launch
-  // more instead of the two passes for everything (measured: M = 1001, N = 14336, K = 4096: 147 us in one piece, 128 us for
-  // 1000 rows; M = 2049, N = K = 8192: 392 against 249 us; M = 601, N = K = 8192: 164 against 120 us; the tail takes 6 - 15 us).
-  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && (M & 3) != 0 && M < kMaxDim && N >= 16 && N % 16 == 0 && N < kMaxDim && K > 0 &&
-      K < kMaxDim && group > 0 && A && C && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
-      (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
+  if (head_and_tail && (keep_tail || !(room_for_two_passes && two_passes_beat_panels(M, N, K, group)))) {
     const int64_t head = M & ~(int64_t)3;
-    if (w4a16_panel256_plan(head, N, K, group, cu_count_or_default()).ok && !(room_for_two_passes && two_passes_beat_panels(M, N, K, group))) {
-      const int rc = tlq_gemm_w4a16_ws(A, w_packed, scales, zeros, C, head, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, workspace,
-                                       workspace_bytes, stream);
-      if (rc != 0) return rc;
-      const int64_t out_bytes = out_dtype == TLQ_F32 ? 4 : 2;
-      return tlq_gemm_w4a16((const uint8_t*)A + head * K * 2, w_packed, scales, zeros, (uint8_t*)C + head * N * out_bytes, M - head, N, K, group,
-                            zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, stream);
-    }
+    const int rc = tlq_gemm_w4a16_ws(A, w_packed, scales, zeros, C, head, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, workspace,
+                                     workspace_bytes, stream);
+    if (rc != 0) return rc;
+    const int64_t out_bytes = out_dtype == TLQ_F32 ? 4 : 2;
+    return tlq_gemm_w4a16((const uint8_t*)A + head * K * 2, w_packed, scales, zeros, (uint8_t*)C + head * N * out_bytes, M - head, N, K, group,
+                          zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, stream);
   }
   if (algo == TLQ_ALGO_PANELM) {
     const int rc = try_panelm(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, workspace, workspace_bytes, stream);
