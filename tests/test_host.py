@@ -213,6 +213,61 @@ def test_build_lock_is_exclusive_and_stale_libraries_are_detected(tmp_path, monk
     assert not build.is_stale() and build.is_current()
 
 
+def test_build_records_do_not_depend_on_where_the_checkout_lies(tmp_path, monkeypatch):
+    import shutil
+
+    from tilelang_ascend_amd import build
+
+    want, want_host = build.source_fingerprint(), build.host_fingerprint()
+    shutil.copytree(build.CSRC_DIR, tmp_path / "pkg" / "csrc")
+    shutil.copytree(build.INCLUDE_DIR, tmp_path / "include")
+    monkeypatch.setattr(build, "CSRC_DIR", str(tmp_path / "pkg" / "csrc"))
+    monkeypatch.setattr(build, "INCLUDE_DIR", str(tmp_path / "include"))
+    moved = lambda flags: [f for f in flags if not f.startswith("-I")] + [f"-I{tmp_path}/include"]  # noqa: E731
+    monkeypatch.setattr(build, "HIPCC_FLAGS", moved(build.HIPCC_FLAGS))
+    monkeypatch.setattr(build, "HOST_FLAGS", moved(build.HOST_FLAGS))
+    assert build.source_fingerprint() == want and build.host_fingerprint() == want_host
+    with open(tmp_path / "include" / "tlq.h", "a") as f:
+        f.write("/* changed */\n")
+    assert build.source_fingerprint() != want and build.host_fingerprint() != want_host
+
+
+def test_extension_module_belongs_to_one_interpreter_and_one_torch(tmp_path, monkeypatch):
+    """Its record names them, it is rebuilt alone, and a compiler that cannot build it leaves libtlq.so in place."""
+    from tilelang_ascend_amd import build
+
+    for name in ("LIB_DIR", "OBJ_DIR"):
+        monkeypatch.setattr(build, name, str(tmp_path))
+    for name, file in (("LIB_PATH", "libtlq.so"), ("STAMP_PATH", "libtlq.fingerprint"), ("HOST_PATH", "tlq_host.so"), ("HOST_STAMP_PATH", "tlq_host.fingerprint")):
+        monkeypatch.setattr(build, name, str(tmp_path / file))
+
+    def compiled(name):
+        (tmp_path / name).write_bytes(b"")
+        return str(tmp_path / name)
+
+    built = []
+    monkeypatch.setattr(build, "_build_locked", lambda verbose, jobs: built.append("lib") or build._install(compiled("lib.tmp"), build.LIB_PATH, build.STAMP_PATH, build.source_fingerprint()))
+    monkeypatch.setattr(build, "_compile_host", lambda: built.append("host") or compiled("host.tmp"))
+    assert build.is_host_stale()
+    build.build_library(force=False)
+    assert sorted(built) == ["host", "lib"] and not build.is_host_stale() and build.is_current()
+    monkeypatch.setattr(torch, "__version__", "0.0.other")
+    assert build.is_host_stale() and build.is_current()
+    build.build_library(force=False)
+    assert sorted(built) == ["host", "host", "lib"] and not build.is_host_stale()
+    (tmp_path / "tlq_host.fingerprint").unlink()
+    assert not build.is_host_stale()  # no record: cannot be judged
+    (tmp_path / "libtlq.so").unlink()
+
+    def cannot():
+        raise RuntimeError("no headers")
+
+    monkeypatch.setattr(build, "_compile_host", cannot)
+    with pytest.raises(RuntimeError, match="no headers"):
+        build.build_library()
+    assert build.is_current()
+
+
 def test_tile_choice_by_machine_fill():
     """128 x 128 or 256 x 256 output tiles: the choice follows how full each makes the machine (256 CUs without a GPU),
     the small tiles' fill weighted by their pace.  The table is what was measured faster on an MI355X."""

@@ -116,6 +116,7 @@ _lock = threading.Lock()
 _lib = None
 _host = None
 _build_failure = None
+_host_failure = None
 
 
 def library_path() -> str:
@@ -142,7 +143,7 @@ def load():
             if _build_failure is not None:  # one attempt per process: sources that do not compile fail every caller at once
                 raise RuntimeError(f"libtlq.so at {path} is {state} and could not be built ({_build_failure})")
             try:
-                path = _build.build_library(force=False)
+                path = _build.build_library(force=False, host=False)
             except Exception as e:  # noqa: BLE001
                 _build_failure = e
                 raise RuntimeError(
@@ -175,8 +176,15 @@ def host():
             import importlib.util
 
             path = _build.HOST_PATH
-            if not os.path.exists(path):
-                _build.build_library(force=False)
+            global _host_failure
+            if _host_failure is not None:  # one attempt per process, as for the library
+                raise RuntimeError(f"tlq_host.so at {path} could not be built ({_host_failure})")
+            if _build.is_host_stale():
+                try:
+                    _build.build_host()
+                except Exception as e:  # noqa: BLE001
+                    _host_failure = e
+                    raise RuntimeError(f"tlq_host.so at {path} could not be built ({e}); run `python -m tilelang_ascend_amd.build`") from e
             spec = importlib.util.spec_from_file_location("tlq_host", path, loader=importlib.machinery.ExtensionFileLoader("tlq_host", path))
             mod = importlib.util.module_from_spec(spec)
             spec.loader.exec_module(mod)

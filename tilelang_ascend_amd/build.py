@@ -27,6 +27,8 @@ LIB_DIR = os.path.join(PKG_DIR, "lib")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 LIB_PATH = os.path.join(LIB_DIR, "libtlq.so")
 HOST_PATH = os.path.join(LIB_DIR, "tlq_host.so")
+STAMP_PATH = os.path.join(LIB_DIR, "libtlq.fingerprint")
+HOST_STAMP_PATH = os.path.join(LIB_DIR, "tlq_host.fingerprint")
 
 ARCH = "gfx950"
 SOURCES = [
@@ -81,19 +83,34 @@ def hipcc_path() -> str:
     raise RuntimeError("hipcc not found: cannot build libtlq.so")
 
 
-def source_fingerprint() -> str:
-    """sha256 over kernel sources, headers and flags -- the analogue of the reference's kernel
-    cache key (tilelang/cache/kernel_cache.py:71-117: hash of source + target + options)."""
+def _fingerprint(flags, paths) -> str:
+    """sha256 over flags and file contents.  Include folders are left out: they say where the checkout lies, not what is built
+    (a checkout that is moved, or reached through another path, keeps its libraries)."""
     h = hashlib.sha256()
-    h.update(" ".join(HIPCC_FLAGS + HOST_FLAGS).encode())
-    names = sorted(os.listdir(CSRC_DIR)) + ["../../include/tlq.h", "../../include/tlq_debug.h"]
-    for name in names:
-        path = os.path.join(CSRC_DIR, name)
+    h.update(" ".join(f for f in flags if not f.startswith("-I")).encode())
+    for path in paths:
         if os.path.isfile(path):
-            h.update(name.encode())
+            h.update(os.path.basename(path).encode())
             with open(path, "rb") as f:
                 h.update(f.read())
     return h.hexdigest()
+
+
+def source_fingerprint() -> str:
+    """sha256 over kernel sources, headers and flags -- the analogue of the reference's kernel
+    cache key (tilelang/cache/kernel_cache.py:71-117: hash of source + target + options)."""
+    names = [n for n in sorted(os.listdir(CSRC_DIR)) if n != HOST_SOURCE]
+    return _fingerprint(HIPCC_FLAGS, [os.path.join(CSRC_DIR, n) for n in names] + [os.path.join(INCLUDE_DIR, n) for n in ("tlq.h", "tlq_debug.h")])
+
+
+def host_fingerprint() -> str:
+    """The same for the extension module, which also belongs to one interpreter and one torch."""
+    import sysconfig
+
+    import torch
+
+    flags = HOST_FLAGS + [str(sysconfig.get_config_var("SOABI")), torch.__version__]
+    return _fingerprint(flags, [os.path.join(CSRC_DIR, HOST_SOURCE), os.path.join(INCLUDE_DIR, "tlq.h")])
 
 
 def _compile_one(src: str, verbose: bool) -> str:
@@ -122,7 +139,8 @@ def _compile_host() -> str:
     rocm = os.path.dirname(os.path.dirname(hipcc_path()))
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     includes = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
-    cmd = [shutil.which("g++") or "g++", *HOST_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+    compiler = shutil.which("g++") or os.path.join(rocm, "bin", "amdclang++")
+    cmd = [compiler, *HOST_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f"-isystem{p}" for p in includes), os.path.join(CSRC_DIR, HOST_SOURCE), "-o", tmp, f"-L{torch_lib}",
            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -131,16 +149,17 @@ def _compile_host() -> str:
     return tmp
 
 
-STAMP_PATH = os.path.join(LIB_DIR, "libtlq.fingerprint")
+def _record(path: str):
+    try:
+        with open(path) as f:
+            return f.read().strip() or None
+    except OSError:
+        return None
 
 
 def built_fingerprint():
     """Fingerprint the library on disk was built from (None when there is no record)."""
-    try:
-        with open(STAMP_PATH) as f:
-            return f.read().strip() or None
-    except OSError:
-        return None
+    return _record(STAMP_PATH)
 
 
 def is_current() -> bool:
@@ -154,6 +173,14 @@ def is_stale() -> bool:
         return True
     fp = built_fingerprint()
     return fp is not None and fp != source_fingerprint()
+
+
+def is_host_stale() -> bool:
+    """The same for the extension module: absent, or built from other sources, for another interpreter or another torch."""
+    if not os.path.exists(HOST_PATH):
+        return True
+    fp = _record(HOST_STAMP_PATH)
+    return fp is not None and fp != host_fingerprint()
 
 
 @contextlib.contextmanager
@@ -170,38 +197,49 @@ def build_lock():
             fcntl.flock(f, fcntl.LOCK_UN)
 
 
-def build_library(force: bool = True, verbose: bool = False, jobs: int = 6) -> str:
-    """Compile every kernel source for gfx950 and link libtlq.so.  With force=False an
-    up-to-date library (matching fingerprint) is reused.  Holds the build lock throughout; a process that waited
+def build_library(force: bool = True, verbose: bool = False, jobs: int = 6, host: bool = True) -> str:
+    """Compile every kernel source for gfx950 and link libtlq.so, then (host=True) the extension module that calls it.  With
+    force=False what is up to date (matching record) is reused.  libtlq.so needs hipcc alone and is in place before the
+    extension module, which needs torch's headers as well, is awaited.  Holds the build lock throughout; a process that waited
     for another one's build finds the library current and (force=False) returns at once."""
+    with build_lock(), ThreadPoolExecutor(max_workers=1) as side:
+        module = side.submit(_compile_host) if host and (force or is_host_stale()) else None
+        if force or not is_current():
+            _build_locked(verbose, jobs)
+        if module is not None:
+            _install(module.result(), HOST_PATH, HOST_STAMP_PATH, host_fingerprint())
+    return LIB_PATH
+
+
+def build_host() -> str:
+    """The extension module alone, where it is absent or belongs to other sources, another interpreter or another torch."""
     with build_lock():
-        return _build_locked(force, verbose, jobs)
+        if is_host_stale():
+            _install(_compile_host(), HOST_PATH, HOST_STAMP_PATH, host_fingerprint())
+    return HOST_PATH
 
 
-def _build_locked(force: bool, verbose: bool, jobs: int) -> str:
+def _install(tmp: str, path: str, stamp: str, fingerprint: str) -> None:
+    os.replace(tmp, path)
+    with open(stamp, "w") as f:
+        f.write(fingerprint + "\n")
+
+
+def _build_locked(verbose: bool, jobs: int) -> None:
     os.makedirs(OBJ_DIR, exist_ok=True)
-    stamp = STAMP_PATH
     fp = source_fingerprint()
-    if not force and is_current() and os.path.exists(HOST_PATH):
-        return LIB_PATH
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC_DIR, s))]
     missing = sorted(set(SOURCES) - set(srcs))
     if missing:
         raise RuntimeError(f"kernel sources missing: {missing}")
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        host = pool.submit(_compile_host)
         objs = list(pool.map(lambda s: _compile_one(s, verbose), srcs))
-        host_tmp = host.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc_path(), "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp, *objs]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"Compilation Failed! {' '.join(cmd)}\n{res.stdout}")
-    os.replace(tmp, LIB_PATH)
-    os.replace(host_tmp, HOST_PATH)
-    with open(stamp, "w") as f:
-        f.write(fp + "\n")
-    return LIB_PATH
+    _install(tmp, LIB_PATH, STAMP_PATH, fp)
 
 
 if __name__ == "__main__":
