@@ -1,4 +1,5 @@
 """The native calls (csrc/host_calls.cpp): the same result as the Python path, and everything out of the ordinary left to it."""
+import copy
 import threading
 
 import pytest
@@ -18,6 +19,18 @@ def test_plan_checks_its_description_and_leaves_host_tensors_alone():
                           ("w4a8", (((4, -8), _abi.I8, 0),) + params[1:], (4, 4, 8, 0)), ("w4a8", (((4, 8), 77, 0),) + params[1:], (4, 4, 8, 0))):
         with pytest.raises(ValueError):
             Plan(kind, p, ints, 0.0)
+
+
+def test_kernel_objects_are_copied_after_their_plan_is_made():
+    kernel = ops.w4a16_gemm(3, 64, 256, group_size=128, zeros="tensor")
+    kernel._fast = kernel._native_plan()  # what the first call on a GPU does
+    holder = torch.nn.Module()
+    holder.kernel = kernel
+    for twin in (copy.deepcopy(kernel), copy.copy(kernel), copy.deepcopy(holder).kernel):
+        assert twin is not kernel and twin.params == kernel.params and twin.result_idx == kernel.result_idx
+        assert twin._plan is None and twin._fast == twin._first_call
+        assert twin._native_plan() is not kernel._plan
+    assert kernel._fast is kernel._plan
 
 
 def _calls():

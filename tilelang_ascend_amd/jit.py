@@ -135,6 +135,15 @@ class JITKernel:
         self._plan = None
         self._fast = self._first_call
 
+    def __getstate__(self):
+        # a copy makes a native plan of its own at its first call: a Plan holds nothing of the kernel's and cannot be copied
+        return {k: v for k, v in self.__dict__.items() if k not in ("_plan", "_fast")}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._plan = None
+        self._fast = self._first_call
+
     # -- introspection kept for drop-in use ----------------------------------------------
     @property
     def out_idx(self):
