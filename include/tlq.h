@@ -70,7 +70,8 @@ enum {
   TLQ_ALGO_AUTO = 0,
   TLQ_ALGO_GEMV = 1, /* split-K wavefront GEMV (M <= 16) */
   TLQ_ALGO_MFMA = 2, /* LDS-staged MFMA dequant-GEMM */
-  TLQ_ALGO_SKINNY = 3, /* M <= 64: weights stream from HBM through the dequantiser into MFMA operands, no LDS tile */
+  TLQ_ALGO_SKINNY = 3, /* M <= 64: weights stream from HBM through the dequantiser into MFMA operands, no LDS tile (up to 16 rows and with
+                        * power-of-two groups the small-tile kernel, TLQ_ALGO_SMALL) */
   TLQ_ALGO_TWO_PASS = 4, /* tlq_gemm_w4a16_ws only: dequantise into the workspace, then the plain GEMM */
   TLQ_ALGO_STREAM = 5, /* tlq_gemm_w4a16_ws only: 17 <= M <= 512, weights streamed once per 128 activation rows through a deep
                        * ring of direct loads, dequantised in registers; K slices add up through the workspace */
@@ -96,6 +97,10 @@ enum {
                        * zero points are small integers, unfolded from the first window that is not).  K % 128 == 0, M % 4 == 0,
                        * N % 16 == 0, power-of-two group >= 64 with (K / group) % 8 == 0, 16-byte aligned scale / zero tensors;
                        * plain word layout.  Workspace: the fp32 partial tiles where K is cut into slices */
+  ,
+  TLQ_ALGO_SMALL = 11 /* (10 names no family) problems that large tiles do not fill: 16, 32 or 64 activation rows x 16, 32 or 64 weight rows per work-group,
+                       * whose wavefronts split K; one launch, no workspace, any M.  K % 128 == 0, power-of-two group >= 32,
+                       * dword-aligned scale / zero tensors of an even number of values */
 };
 
 int tlq_abi_version(void);

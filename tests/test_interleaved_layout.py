@@ -93,11 +93,11 @@ def test_two_passes_and_automatic_choice_on_interleaved_words(in_dtype, out_dtyp
     dt = DT[in_dtype]
     A = torch.randn(M, K, generator=gen(73)).to(dt)
     Wp, s, z = make_w4(N, K, group, dt, "int", seed=74)
-    # what the automatic choice takes for interleaved words: the streaming kernel for 300 rows on 1024 weight rows (the
-    # tile kernels of the two passes would leave most of the machine idle), the two passes for 1024 rows
+    # what the automatic choice takes for interleaved words: the small-tile kernel for 300 rows on 1024 weight rows of 512
+    # values (the tile kernels of the two passes would leave most of the machine idle), the two passes for 1024 rows
     # (448 rows on 5120 x 13824: two tiles of the 256-row kernel against four streaming blocks, by estimate)
     # (80 rows on 81920 weight rows: 160 work-groups of the 128-row panel kernel in one round)
-    taken = {300: _abi.ALGO_STREAM, 1024: _abi.ALGO_TWO_PASS, 448: _abi.ALGO_PANEL256, 80: _abi.ALGO_PANEL}[M]
+    taken = {300: _abi.ALGO_SMALL, 1024: _abi.ALGO_TWO_PASS, 448: _abi.ALGO_PANEL256, 80: _abi.ALGO_PANEL}[M]
     for algo, plain_algo in ((_abi.ALGO_TWO_PASS, _abi.ALGO_TWO_PASS), (_abi.ALGO_AUTO, taken)):
         rc, plain = run_layout(A, Wp, s, z, group, _abi.W_PLAIN, plain_algo, DT[out_dtype])
         assert rc == 0, _abi.last_error()

@@ -36,22 +36,22 @@ def cases():
 
     return [
         # M, N, K, group, the kernel the automatic choice is meant to take
-        (256, 256, 256, 128, _abi.ALGO_MFMA),      # the reference's own CPU-runnable case: one launch of the tile kernel
-        (128, 1024, 512, 128, _abi.ALGO_MFMA),
-        (64, 1024, 1024, 128, _abi.ALGO_SKINNY),
-        (48, 4096, 1024, 64, _abi.ALGO_SKINNY),
+        (256, 256, 256, 128, _abi.ALGO_SMALL),     # the reference's own CPU-runnable case: one launch of the small-tile kernel
+        (128, 1024, 512, 128, _abi.ALGO_SMALL),
+        (64, 1024, 1024, 128, _abi.ALGO_SMALL),
+        (48, 4096, 1024, 64, _abi.ALGO_SMALL),
         (24, 4096, 4096, 128, _abi.ALGO_DECODE),
         (32, 1024, 2048, 32, _abi.ALGO_DECODE),
         (2, 8192, 2048, 64, _abi.ALGO_GEMV),       # ring kernel, two activation rows
         (2, 4096, 4096, 128, _abi.ALGO_DECODE),    # 4096 rows: one per wavefront, the decode kernel is ahead
-        (64, 4096, 4096, 128, _abi.ALGO_STREAM),   # large enough for K slices and a second launch
-        (256, 1024, 1024, 128, _abi.ALGO_STREAM),
+        (64, 4096, 4096, 128, _abi.ALGO_SMALL),    # still ahead of K slices and a second launch (10.5 against 16.9 us)
+        (256, 1024, 1024, 128, _abi.ALGO_SMALL),
         (16, 5120, 5120, 128, _abi.ALGO_DECODE),   # rows of 5120 values, 320 tiles of 16 weight rows (more than CUs): decode kernel on K chunks
         (512, 4096, 2048, 128, _abi.ALGO_STREAM),  # 512 rows on 4096 weight rows: the tile kernels would fill half the machine
         (384, 10240, 2048, 128, _abi.ALGO_STREAM),  # three blocks of 128 activation rows: streaming kernel whatever the tile kernels' fill
         (512, 8192, 2048, 128, _abi.ALGO_STREAM),   # four blocks, 32 x 4 x 2 = 256 streaming work-groups: they fit the machine at once
         (512, 8192, 1024, 128, _abi.ALGO_MFMA),     # short rows, one round of 128 x 128 tiles: the tile kernel in one launch (19 against 23 us)
-        (48, 8192, 1024, 128, _abi.ALGO_SKINNY),    # short rows, 33 .. 64 activation rows, up to 2^24 weights: the skinny kernel's one launch
+        (48, 8192, 1024, 128, _abi.ALGO_SMALL),     # short rows, 33 .. 64 activation rows, up to 2^24 weights: one launch
         (112, 32768, 4096, 128, _abi.ALGO_PANELM),    # one tile of 128 rows on 2^27 weights or more: the middle-M kernel
         (144, 50304, 4096, 128, _abi.ALGO_PANEL256),  # two streaming blocks of 96 rows in two rounds against one round of 256-row tiles, by estimate
         (448, 5120, 13824, 128, _abi.ALGO_PANEL256),  # 108 groups per row (the middle-M kernel wants multiples of eight): two 256-row tiles against four streaming blocks by estimate

@@ -75,7 +75,7 @@ def test_interleaved_words_with_one_group_per_row(M, N, K, zeros_kind):
     A = torch.randn(M, K, generator=gen(960 + M)).half()
     Wp, s, z = make_w4(N, K, K, torch.float16, zeros_kind, seed=961 + M)
     # (the kernel that reads interleaved words at this size, by name on the plain ones: the sums must be added in the same order)
-    plain = run(A, Wp, s, z, K, algo=_abi.ALGO_DECODE if M <= 32 else _abi.ALGO_STREAM)
+    plain = run(A, Wp, s, z, K, algo={16: _abi.ALGO_DECODE, 64: _abi.ALGO_SMALL, 300: _abi.ALGO_SMALL}[M])
     Wi = ref.interleave_weight(Wp.view(torch.int8), 4, "float16").view(torch.uint8).contiguous()
     dA, dW, dS, dZ = A.cuda(), Wi.cuda(), s.cuda(), z.cuda()
     need = max(lib.tlq_w4a16_workspace_bytes(M, N, K), 16)

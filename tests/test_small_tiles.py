@@ -15,18 +15,19 @@ from tilelang_ascend_amd import _abi, build
 CODE = {torch.float16: _abi.F16, torch.bfloat16: _abi.BF16, torch.float32: _abi.F32}
 
 
-def run(A, Wp, s, z, group, algo, out_dtype=None, layout=_abi.W_PLAIN):
+def run(A, Wp, s, z, group, algo, out_dtype=None, layout=_abi.W_PLAIN, workspace=0):
     lib, P = _abi.load(), _abi.ptr
     (M, K), N = A.shape, Wp.shape[0]
     out_dtype = out_dtype or A.dtype
     zt = z.cuda() if torch.is_tensor(z) else None
     dA, dW, dS = A.cuda(), Wp.cuda(), s.cuda()
     C = torch.full((M, N), float("nan"), dtype=out_dtype, device="cuda")
+    ws = torch.empty(workspace, dtype=torch.uint8, device="cuda") if workspace else None
     print(f"small tiles M={M} N={N} K={K} g={group} algo={algo} layout={layout}", flush=True)
     lib.tlq_debug_launch_log(1)
     rc = lib.tlq_gemm_w4a16_layout_ws(P(dA), P(dW), P(dS), P(zt), P(C), M, N, K, group, 0.0 if zt is not None or z is None else float(z),
-                                      CODE[A.dtype], CODE[out_dtype], algo, layout, None, 0, torch.cuda.current_stream().cuda_stream)
-    run.log = lib.tlq_debug_launch_log_text().decode()
+                                      CODE[A.dtype], CODE[out_dtype], algo, layout, P(ws), workspace, torch.cuda.current_stream().cuda_stream)
+    run.log = lib.tlq_debug_launch_log_text().decode().strip()
     lib.tlq_debug_launch_log(0)
     _abi.check(rc)
     torch.cuda.synchronize()
@@ -59,18 +60,57 @@ def test_every_tile_against_the_oracle(in_dtype, rows, cols, M, N, K, group, zer
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,group,algo", [(40, 1024, 3072, 128, "STREAM"), (200, 300, 1024, 64, "STREAM"), (130, 528, 512, 32, "MFMA"),
-                                              (700, 256, 384, 128, "AUTO"), (603, 272, 1280, 64, "AUTO"), (9, 336, 8320, 128, "AUTO")])
-def test_families_hand_small_problems_over(M, N, K, group, algo):
-    """Named families and the automatic choice run it where its estimate is lower; repacked words give the bits of plain ones."""
+@pytest.mark.parametrize("M,N,K,group", [(40, 1024, 3072, 128), (200, 300, 1024, 64), (130, 528, 512, 32), (700, 256, 384, 128), (603, 272, 1280, 64),
+                                         (9, 336, 8320, 128)])
+def test_automatic_choice_runs_it_on_small_problems(M, N, K, group):
+    """Where its estimate is lower; the same bits by its own name, and on repacked words."""
     A = torch.randn(M, K, generator=gen(M)).half()
     Wp, s, z = make_w4(N, K, group, torch.float16, "int", seed=N)
-    got = run(A, Wp, s, z, group, getattr(_abi, "ALGO_" + algo))
+    got = run(A, Wp, s, z, group, _abi.ALGO_AUTO)
     assert "w4a16_small_kernel" in run.log, run.log
+    check_float_output(got, w4a16_reference(A, Wp, s, z, group), f"{M}x{N}x{K}")
+    assert_bit_equal(run(A, Wp, s, z, group, _abi.ALGO_SMALL), got, "by name")
+    Wi = ref.interleave_weight(Wp.view(torch.int8), 4, "float16").view(torch.uint8).contiguous()
+    assert_bit_equal(run(A, Wi, s, z, group, _abi.ALGO_SMALL, layout=_abi.W_INTERLEAVED_F16), got, "interleaved words")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [_abi.W_PLAIN, _abi.W_INTERLEAVED_F16])
+@pytest.mark.parametrize("M,N,K,group,algo,kernel", [
+    (40, 1024, 768, 128, "STREAM", "w4a16_stream_kernel"), (200, 300, 256, 64, "STREAM", "w4a16_stream_kernel"), (130, 528, 512, 32, "MFMA", "tlq_gemm_w4a16(mfma)"),
+    (256, 256, 256, 128, "MFMA", "tlq_gemm_w4a16(mfma)"), (40, 1024, 768, 128, "SKINNY", "w4a16_skinny_kernel"), (64, 512, 512, 64, "SKINNY", "w4a16_skinny_kernel"),
+    (130, 528, 512, 32, "SMALL", "w4a16_small_kernel")])
+def test_families_asked_for_by_name_run_themselves(layout, M, N, K, group, algo, kernel):
+    """Also on problems that the automatic choice gives to the small-tile kernel."""
+    if layout != _abi.W_PLAIN and algo in ("MFMA", "SKINNY"):
+        pytest.skip("does not read repacked words")
+    A = torch.randn(M, K, generator=gen(M)).half()
+    Wp, s, z = make_w4(N, K, group, torch.float16, "int", seed=N)
+    Wl = Wp if layout == _abi.W_PLAIN else ref.interleave_weight(Wp.view(torch.int8), 4, "float16").view(torch.uint8).contiguous()
+    workspace = _abi.load().tlq_w4a16_workspace_bytes_for(M, N, K, getattr(_abi, "ALGO_" + algo)) if algo == "STREAM" else 0
+    got = run(A, Wl, s, z, group, getattr(_abi, "ALGO_" + algo), layout=layout, workspace=workspace)
+    assert kernel in run.log and (algo == "SMALL") == ("w4a16_small_kernel" in run.log), run.log
     check_float_output(got, w4a16_reference(A, Wp, s, z, group), f"{algo} {M}x{N}x{K}")
-    if algo == "STREAM":
-        Wi = ref.interleave_weight(Wp.view(torch.int8), 4, "float16").view(torch.uint8).contiguous()
-        assert_bit_equal(run(A, Wi, s, z, group, _abi.ALGO_STREAM, layout=_abi.W_INTERLEAVED_F16), got, "interleaved words")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [_abi.W_PLAIN, _abi.W_INTERLEAVED_F16])
+def test_streaming_kernel_by_name_is_refused_without_room_for_its_slices(layout):
+    M, N, K, group = 64, 1024, 4096, 128
+    assert _abi.load().tlq_w4a16_workspace_bytes_for(M, N, K, _abi.ALGO_STREAM) > 0
+    A, (Wp, s, z) = torch.zeros(M, K).half(), make_w4(N, K, group, torch.float16, "int", seed=1)
+    with pytest.raises(RuntimeError, match="streaming kernel"):
+        run(A, Wp, s, z, group, _abi.ALGO_STREAM, layout=layout)
+    assert run.log == ""
+
+
+def test_small_family_refuses_what_its_kernel_does_not_read():
+    lib, fake = _abi.load(), ctypes.c_void_p(1 << 20)
+    for N, K, group in ((64, 192, 64), (64, 384, 96), (1, 128, 128)):  # K in whole k-blocks, power-of-two groups, an even number of scales
+        rc = lib.tlq_gemm_w4a16(fake, fake, fake, None, fake, 40, N, K, group, 8.0, _abi.F16, _abi.F16, _abi.ALGO_SMALL, None)
+        assert rc != 0 and "small-tile kernel needs" in _abi.last_error()
+        rc = lib.tlq_gemm_w4a16_layout_ws(fake, fake, fake, None, fake, 40, N, K, group, 8.0, _abi.F16, _abi.F16, _abi.ALGO_SMALL, _abi.W_INTERLEAVED_F16, None, 0, None)
+        assert rc != 0 and "small-tile kernel needs" in _abi.last_error()
 
 
 def test_plan_keeps_to_the_machine():

@@ -115,9 +115,14 @@ def test_stream_rejects_what_it_cannot_do():
 def test_automatic_choice_takes_the_streaming_kernel_and_agrees_with_it():
     from tilelang_ascend_amd import _abi
 
-    M, N, K, group = 64, 4096, 4096, 128  # (small problems and short rows at this M -- K <= 2048 on up to 2^24 weights -- go to single-launch kernels instead)
+    M, N, K, group = 64, 14336, 4096, 128  # (small problems, 64 rows on 4096 x 4096 among them, go to single-launch kernels instead)
     A = torch.randn(M, K, generator=gen(54)).to(torch.float16)
     Wp, s, z = make_w4(N, K, group, torch.float16, "int", seed=55)
     a = run_stream(A, Wp, s, z, group)
+    lib = _abi.load()
+    lib.tlq_debug_launch_log(1)
     b = run_stream(A, Wp, s, z, group, algo=_abi.ALGO_AUTO)
+    log = lib.tlq_debug_launch_log_text().decode()
+    lib.tlq_debug_launch_log(0)
+    assert "w4a16_stream_kernel" in log, log
     assert_bit_equal(a, b, "auto vs stream")

@@ -19,7 +19,7 @@ F16, BF16, F32, I8, I32 = 0, 1, 2, 3, 4
 U4, S4_TWOS, S4_OFFSET8, S4_OFFSET7 = 0, 1, 2, 3
 B_KN, B_NK = 0, 1
 W_PLAIN, W_INTERLEAVED_F16 = 0, 1
-ALGO_AUTO, ALGO_GEMV, ALGO_MFMA, ALGO_SKINNY, ALGO_TWO_PASS, ALGO_STREAM, ALGO_DECODE, ALGO_PANEL, ALGO_PANEL256, ALGO_PANELM = 0, 1, 2, 3, 4, 5, 6, 7, 8, 9
+ALGO_AUTO, ALGO_GEMV, ALGO_MFMA, ALGO_SKINNY, ALGO_TWO_PASS, ALGO_STREAM, ALGO_DECODE, ALGO_PANEL, ALGO_PANEL256, ALGO_PANELM, ALGO_SMALL = 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 11
 ABI_VERSION = 1
 
 _vp, _i64, _int, _f32, _cstr = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float, ctypes.c_char_p

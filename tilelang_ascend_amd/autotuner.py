@@ -334,7 +334,7 @@ def autotune(func: Callable = None, *, configs: Union[Sequence[dict], Callable],
 # ``cache.clear_cache()`` removes and which ``ops.w4a16_gemm`` installs once per process.
 
 W4A16_FAMILIES = {"gemv": 1, "mfma": 2, "skinny": 3, "two_pass": 4, "stream": 5, "decode": 6, "panel": 7, "panel256": 8,
-                  "panelm": 9}
+                  "panelm": 9, "small": 11}
 _choices_lock = threading.Lock()
 _choices_loaded = False
 

@@ -15,6 +15,8 @@ int gemm_w4a16_mfma(const void* A, const void* Wp, const void* scales, const voi
                     int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, hipStream_t st);
 int64_t w4a16_mid_split(int64_t M, int64_t N, int64_t K, int64_t group);
 int w4a16_split_forced();
+bool w4a16_tile_forced();
+bool w4a16_skinny_forced();
 double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group);
 int gemm_w4a16_mfma_splitk(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M,
                            int64_t N, int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype,
@@ -194,6 +196,10 @@ using namespace tlq;
   TLQ_REQUIRE(M >= 0 && N >= 0 && K >= 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim, name ": bad shape M=%lld N=%lld K=%lld", \
               (long long)M, (long long)N, (long long)K)
 
+#define TLQ_SMALL_NEEDS(name)                                                                                       \
+  name ": the small-tile kernel needs K %% 128 == 0, a power-of-two group >= 32, dword-aligned scale / zero tensors of an even " \
+       "number of values and matrices below 4 GiB (M=%lld N=%lld K=%lld group=%lld)"
+
 extern "C" {
 
 void tlq_tune_gemm_groups(int variant) { tlq::tuning_changed(), tlq::g_gemm_groups = variant < 0 || variant > 5 ? 0 : variant; }
@@ -285,6 +291,16 @@ static bool small_beats_panels(const SmallPlan& p, int64_t M, int64_t N, int64_t
 static bool small_beats_decode_chunks(const SmallPlan& p, int64_t M, int64_t N, int64_t K) {
   return p.ok && p.us < 0.95 * (5.2 + 0.67 * giga((double)M, N, K) + 4.36 * giga(up16(M), N, K) + 0.023e-6 * (double)N * (double)K + 0.25e-3 * (double)K);
 }
+// The skinny kernel on 17 .. 64 rows (12.8 -> 7.8 us for M = 64 on 5120 x 1280, level where the launch is all there is) and the tile
+// kernel (4 us + 1.5 us per 128 values of K whatever M and N: 21.5 -> 5.9 us for 116 rows on 368 x 1280, 256 x 256 x 256 6.8 -> 5.4 us):
+// the family the automatic choice runs in their place.
+static int small_or(int algo, int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros) {
+  if (algo == TLQ_ALGO_SKINNY ? M <= 16 || w4a16_skinny_forced() : algo != TLQ_ALGO_MFMA || N % 4 != 0 || w4a16_tile_forced()) return algo;
+  const SmallPlan p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+  const double theirs = algo == TLQ_ALGO_SKINNY ? 0.95 * (5.2 + 7.0 * giga((double)M, N, K) + 4.1 * giga(up16(M), N, K) + 0.3e-3 * (double)K)
+                                                : 0.9 * (3.9 + 11.6e-3 * (double)K + 0.94 * giga((double)M, N, K) + 0.116e-6 * (double)M * (double)N);
+  return p.ok && p.us < theirs ? TLQ_ALGO_SMALL : algo;
+}
 static bool decode_preferred(int64_t M, int64_t N, int64_t K) { return M > 2 || (M == 2 && N * K >= ((int64_t)1 << 24)); }
 
 // The kernel of tlq_gemm_w4a16 by its rules (up to 64 rows; more rows come here only where every kernel above wants a workspace).
@@ -324,13 +340,13 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
               in_dtype);
   TLQ_REQUIRE(out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32,
               "tlq_gemm_w4a16: out_dtype must be float16, bfloat16 or float32 (got %d)", out_dtype);
-  TLQ_REQUIRE((algo >= TLQ_ALGO_AUTO && algo <= TLQ_ALGO_SKINNY) || algo == TLQ_ALGO_DECODE, "tlq_gemm_w4a16: bad algo %d", algo);
+  TLQ_REQUIRE((algo >= TLQ_ALGO_AUTO && algo <= TLQ_ALGO_SKINNY) || algo == TLQ_ALGO_DECODE || algo == TLQ_ALGO_SMALL, "tlq_gemm_w4a16: bad algo %d", algo);
   if (M == 0 || N == 0) return 0;
   if (algo == TLQ_ALGO_AUTO) {
     // a tuned choice for this call signature (tlq_w4a16_choice_set) goes first; where that kernel refuses the call (its
     // shape or alignment rules: nothing launched), the rules below decide as if there were none
     const int chosen = w4a16_choice_lookup(M, N, K, group, in_dtype);
-    if ((chosen >= TLQ_ALGO_GEMV && chosen <= TLQ_ALGO_SKINNY) || chosen == TLQ_ALGO_DECODE) {
+    if ((chosen >= TLQ_ALGO_GEMV && chosen <= TLQ_ALGO_SKINNY) || chosen == TLQ_ALGO_DECODE || chosen == TLQ_ALGO_SMALL) {
       const uint64_t before = launch_count();
       const int rc = tlq_gemm_w4a16(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, chosen, stream);
       if (rc == 0 || launch_count() != before) return rc;
@@ -358,7 +374,12 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
   // gathers read aligned dwords: the tensors must start on a dword boundary (their length is checked by the plan).
   const DecodePlan dp = M <= 32 ? w4a16_decode_plan(M, N, K, group, cu_count_or_default()) : DecodePlan{false, 0, 0, 0, 0, 0};
   const bool decode_ok = w4a16_decode_in_one_chunk(dp, scales, zeros);
-  if (algo == TLQ_ALGO_AUTO) algo = w4a16_few_rows_choice(M, N, K, group, in_dtype, scales, zeros, decode_ok);
+  if (algo == TLQ_ALGO_AUTO) algo = small_or(w4a16_few_rows_choice(M, N, K, group, in_dtype, scales, zeros, decode_ok), M, N, K, group, scales, zeros);
+  if (algo == TLQ_ALGO_SMALL) {
+    const SmallPlan p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+    TLQ_REQUIRE(p.ok, TLQ_SMALL_NEEDS("tlq_gemm_w4a16"), (long long)M, (long long)N, (long long)K, (long long)group);
+    return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, p, "tlq_gemm_w4a16(small)", st);
+  }
   if (algo == TLQ_ALGO_DECODE) {
     TLQ_REQUIRE(decode_ok, "tlq_gemm_w4a16: the decode kernel needs 1 <= M <= 32, K %% 256 == 0, K <= 4096 without a workspace, a power-of-two "
                 "group and dword-aligned scale / zero tensors (M=%lld N=%lld K=%lld group=%lld)", (long long)M, (long long)N, (long long)K,
@@ -502,7 +523,7 @@ int64_t tlq_w4a16_workspace_bytes_for(int64_t M, int64_t N, int64_t K, int algo)
     case TLQ_ALGO_PANEL:
     case TLQ_ALGO_PANEL256: return panel_workspace_bytes(M, N, K);
     case TLQ_ALGO_PANELM: return panelm_workspace_bytes(M, N, K);
-    default: return 0;  // GEMV, skinny: no workspace
+    default: return 0;  // GEMV, skinny, small tiles: no workspace
   }
 }
 
@@ -782,7 +803,7 @@ static int run_ragged_rows(const void* A, const void* w_packed, const void* scal
 int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, const void* zeros, void* C, int64_t M,
                       int64_t N, int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int algo,
                       void* workspace, int64_t workspace_bytes, void* stream) {
-  TLQ_REQUIRE(algo >= TLQ_ALGO_AUTO && algo <= TLQ_ALGO_PANELM, "tlq_gemm_w4a16_ws: bad algo %d", algo);
+  TLQ_REQUIRE((algo >= TLQ_ALGO_AUTO && algo <= TLQ_ALGO_PANELM) || algo == TLQ_ALGO_SMALL, "tlq_gemm_w4a16_ws: bad algo %d", algo);
   if (algo != TLQ_ALGO_TWO_PASS) {  // (not for the two passes by name: their dequantisation pass takes any group as it is)
     RowValues rv;
     const int wrote = write_out_row_values(scales, zeros, M, N, K, group, in_dtype, workspace, workspace_bytes, stream, rv);
@@ -922,7 +943,8 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     const int64_t tiles128 = ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128);
     if (M >= 96 && M <= 512 && N % 4 == 0 && tiles128 <= cu_count_or_default() &&
         (K <= 512 || (K <= 768 && tiles128 >= 96) || (K <= 1024 && tiles128 >= (group < 64 ? 192 : 96)) || (K <= 1536 && tiles128 >= 128 && (M == 128 || M > 192))))  // (129 .. 192 rows: the streaming kernel's blocks of 96 rows are level there)
-      return tlq_gemm_w4a16(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_MFMA, stream);
+      return tlq_gemm_w4a16(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype,
+                            small_or(TLQ_ALGO_MFMA, M, N, K, group, scales, zeros), stream);
     // 17 .. 32 activation rows whose K is one chunk of the decode kernel: that kernel, which needs no workspace
     // (M = 32, N = 14336, K = 4096: 16.8 against 20 us for the streaming kernel)
     if (M > 16 && M <= 32 && g_w4a16_decode && group > 0) {
@@ -969,11 +991,10 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
                          (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) && (M * N) % 4 == 0 &&
                          ((uintptr_t)scales & 1) == 0 && ((uintptr_t)zeros & 1) == 0 && K > 0 && fits32(M, K * 2) && fits32(N, K / 2);
     const bool ws_ok = sp.ok && (sp.split == 1 || (workspace && aligned16(workspace) && workspace_bytes >= (int64_t)sp.split * M * N * 4));
-    // (on the family's behalf, asked for by name too: the interleaved layout takes the same kernel at the same sizes)
-    if (sp.ok && args_ok) {
+    if (algo == TLQ_ALGO_AUTO && sp.ok && args_ok) {
       const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_stream(small, M, N, K))
-        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(stream)",
+        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
     }
     if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && panel256_beats_stream(M, N, K, group, sp)) {
@@ -1106,8 +1127,9 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
     return tlq_gemm_w4a16_ws(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, algo, workspace,
                              workspace_bytes, stream);
   TLQ_CHECK_DIMS("tlq_gemm_w4a16_layout_ws");
-  TLQ_REQUIRE(algo == TLQ_ALGO_AUTO || algo == TLQ_ALGO_GEMV || algo == TLQ_ALGO_STREAM || algo == TLQ_ALGO_TWO_PASS || algo == TLQ_ALGO_DECODE || algo == TLQ_ALGO_PANEL || algo == TLQ_ALGO_PANEL256,
-              "tlq_gemm_w4a16_layout_ws: interleaved weights are read by the ring GEMV, the decode kernel, the streaming kernel, the panel kernels and the two passes (algo %d)", algo);
+  TLQ_REQUIRE(algo == TLQ_ALGO_AUTO || algo == TLQ_ALGO_GEMV || algo == TLQ_ALGO_STREAM || algo == TLQ_ALGO_TWO_PASS || algo == TLQ_ALGO_DECODE || algo == TLQ_ALGO_PANEL || algo == TLQ_ALGO_PANEL256 ||
+                  algo == TLQ_ALGO_SMALL,
+              "tlq_gemm_w4a16_layout_ws: interleaved weights are read by the ring GEMV, the decode kernel, the small-tile kernel, the streaming kernel, the panel kernels and the two passes (algo %d)", algo);
   TLQ_REQUIRE(in_dtype == TLQ_F16 || in_dtype == TLQ_BF16, "tlq_gemm_w4a16_layout_ws: in_dtype must be float16 or bfloat16 (got %d)", in_dtype);
   TLQ_REQUIRE(out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32, "tlq_gemm_w4a16_layout_ws: bad out_dtype %d", out_dtype);
   if (M == 0 || N == 0) return 0;
@@ -1132,6 +1154,11 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
     if (taken) return rc;
   }
   const bool ws_aligned = workspace && aligned16(workspace);
+  if (algo == TLQ_ALGO_SMALL) {
+    const SmallPlan p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+    TLQ_REQUIRE(p.ok, TLQ_SMALL_NEEDS("tlq_gemm_w4a16_layout_ws"), (long long)M, (long long)N, (long long)K, (long long)group);
+    return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, p, "tlq_gemm_w4a16(small)", (hipStream_t)stream);
+  }
   // one or two activation rows: the ring GEMV where the plain layout takes it too (one row; two fp16 rows on 8192 weight
   // rows or more), or when asked for by name
   if (M <= 2 && (algo == TLQ_ALGO_GEMV || (algo == TLQ_ALGO_AUTO && (M == 1 || N >= 8192)))) {
@@ -1183,10 +1210,10 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
   }
   if (algo != TLQ_ALGO_TWO_PASS) {
     const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
-    if (sp.ok && (M * N) % 4 == 0) {
+    if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0) {
       const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_stream(small, M, N, K))
-        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(stream)",
+        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
     }
     const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));

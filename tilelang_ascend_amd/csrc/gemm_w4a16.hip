@@ -386,14 +386,11 @@ template <typename T, bool FOLD>
 static int dispatch_skinny(const W4Args& a) {
   const int64_t row_tiles = ceil_div(a.N, 16);
   const int KB = (int)(a.K / 128);
-  // power-of-two groups: the small-tile kernel, operands staged through wavefront-private LDS (asked for by name with forced
-  // variants, and automatically up to 16 rows and wherever its estimate is below this kernel's: 12.8 -> 7.8 us for M = 64 on
-  // 5120 x 1280, level where the launch is all there is)
-  if (g_skinny_lds != 0) {
-    const bool by_name = g_skinny_lds == 1 || a.M <= 16;
-    const SmallPlan p = w4a16_small_plan(a.M, a.N, a.K, a.group, a.scales, a.zeros, by_name ? g_skinny_waves : 0, by_name ? g_skinny_rt : 0, g_skinny_mt);
-    const double g16 = (double)ceil_div(a.M, (int64_t)16) * 16.0 * (double)a.N * (double)a.K * 1e-9, g = (double)a.M * (double)a.N * (double)a.K * 1e-9;
-    if (p.ok && (by_name || (!g_skinny_waves && !g_skinny_rt && p.us < 0.95 * (5.2 + 7.0 * g + 4.1 * g16 + 0.3e-3 * (double)a.K))))
+  // up to 16 rows and power-of-two groups: operands staged through wavefront-private LDS, which is the small-tile kernel with
+  // tiles of 16 activation rows (more rows: only where a tuning hook asks for it)
+  if (g_skinny_lds == 1 || (a.M <= 16 && g_skinny_lds != 0)) {
+    const SmallPlan p = w4a16_small_plan(a.M, a.N, a.K, a.group, a.scales, a.zeros, g_skinny_waves, g_skinny_rt, g_skinny_mt);
+    if (p.ok)
       return gemm_w4a16_small(a.A, a.Wp, a.scales, a.zeros, a.C, a.M, a.N, a.K, a.group, a.zero_scalar, std::is_same<T, half_t>::value ? TLQ_F16 : TLQ_BF16, a.out_dtype,
                               TLQ_W_PLAIN, p, "tlq_gemm_w4a16(skinny)", a.st);
   }
@@ -462,6 +459,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4_t* __re
 // MLP shapes), slices of at least 512 values that are whole stages and whole quantisation groups.  1 = no split.
 static thread_local int g_w4a16_split = 0;  // forced number of K slices for tuning runs (0 = automatic)
 int w4a16_split_forced() { return g_w4a16_split; }
+bool w4a16_tile_forced() { return g_w4a16_tile != 0; }
+bool w4a16_skinny_forced() { return g_skinny_waves != 0 || g_skinny_rt != 0 || g_skinny_lds >= 0; }
 
 // fraction of the work-group places (256, or 512 for the smaller tiles) that the tile kernel fills with the K cut it would take
 double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group);
@@ -537,13 +536,6 @@ int gemm_w4a16_mfma(const void* A, const void* Wp, const void* scales, const voi
   // An integer zero point shared by the whole matrix folds exactly into the unpack bias.
   const bool fold = zeros == nullptr && zero_scalar == (float)(int)zero_scalar && zero_scalar >= -256.0f &&
                     zero_scalar <= 256.0f;
-  // Too few tiles to matter: the small-tile kernel where its estimate is below this kernel's (4 us + 1.5 us per 128 values of K whatever
-  // M and N: 21.5 -> 5.9 us for 116 rows on 368 x 1280, 256 x 256 x 256 6.8 -> 5.4 us)
-  if (g_w4a16_tile == 0) {
-    const SmallPlan p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
-    if (p.ok && p.us < 0.9 * (3.9 + 11.6e-3 * (double)K + 0.94e-9 * (double)M * (double)N * (double)K + 0.116e-6 * (double)M * (double)N))
-      return gemm_w4a16_small(A, Wp, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, p, "tlq_gemm_w4a16(mfma)", st);
-  }
   const W4Args a{A, Wp, scales, zeros, C, M, N, K, group, zero_scalar, out_dtype, st};
   if (in_dtype == TLQ_F16) return fold ? dispatch_w4a16<half_t, true>(a) : dispatch_w4a16<half_t, false>(a);
   return fold ? dispatch_w4a16<bf16_t, true>(a) : dispatch_w4a16<bf16_t, false>(a);

@@ -36,7 +36,7 @@ std::unordered_map<ChoiceKey, int, ChoiceHash>& choice_table() {
 }
 std::atomic<int64_t> g_choice_count{0};  // entries in the table: the launch path looks nothing up while it is 0
 
-bool valid_algo(int algo) { return algo >= TLQ_ALGO_AUTO && algo <= TLQ_ALGO_PANELM; }
+bool valid_algo(int algo) { return (algo >= TLQ_ALGO_AUTO && algo <= TLQ_ALGO_PANELM) || algo == TLQ_ALGO_SMALL; }
 
 }  // namespace
 

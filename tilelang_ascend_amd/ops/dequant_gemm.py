@@ -27,7 +27,8 @@ _PASS_CONFIGS = {
 }
 _SIGN_MODES = {"unsigned": _abi.U4, "twos": _abi.S4_TWOS, "offset8": _abi.S4_OFFSET8, "offset7": _abi.S4_OFFSET7}
 _ALGOS = {"auto": _abi.ALGO_AUTO, "gemv": _abi.ALGO_GEMV, "mfma": _abi.ALGO_MFMA, "skinny": _abi.ALGO_SKINNY,
-          "two_pass": _abi.ALGO_TWO_PASS, "stream": _abi.ALGO_STREAM, "decode": _abi.ALGO_DECODE, "panel": _abi.ALGO_PANEL, "panel256": _abi.ALGO_PANEL256, "panelm": _abi.ALGO_PANELM}
+          "two_pass": _abi.ALGO_TWO_PASS, "stream": _abi.ALGO_STREAM, "decode": _abi.ALGO_DECODE, "panel": _abi.ALGO_PANEL, "panel256": _abi.ALGO_PANEL256, "panelm": _abi.ALGO_PANELM,
+          "small": _abi.ALGO_SMALL}
 # arrangement of the 4-bit fields in each 32-bit word: general_compress order, or interleave_weight(target float16)
 _LAYOUTS = {"plain": _abi.W_PLAIN, "interleaved": _abi.W_INTERLEAVED_F16}
 
@@ -169,6 +170,8 @@ def w4a16_gemm(M: int, N: int, K: int, block_M: int = 128, block_N: int = 256, b
     (a [N,K/group_size] in_dtype input follows).  C [M,N] out_dtype, fp32 accumulate.
     algo: "auto" | "gemv" (split-K wavefront kernel, M <= 16) | "decode" (M <= 32, K % 256 == 0: persistent work-groups with the
     activations in registers: what "auto" does for 3 <= M <= 16) | "skinny" (M <= 64) | "mfma" (LDS-staged MFMA kernel)
+    | "small" (tiles of 16 - 64 activation rows x 16 - 64 weight rows in one launch, K % 128 == 0: what "auto" does for problems too
+    small to fill the machine with large tiles)
     | "stream" (wavefront-private packed weights dequantised in registers, 17 <= M <= 512: what "auto" does up to
     M = 384) | "panel" (large M in one launch: packed weights copied to LDS as they are and dequantised on the MFMA operand
     read; what "auto" does from 513 to 2048 rows where its work-groups fill the machine) | "two_pass" (dequantise into a
@@ -180,7 +183,7 @@ def w4a16_gemm(M: int, N: int, K: int, block_M: int = 128, block_N: int = 256, b
     when the launch stream (forward(stream=...)) is not torch's current stream the block is recorded on it.
     weight_layout: "plain" (general_compress order) or "interleaved" (B_packed went through interleave_weight for the
     float16 target, e.g. quantize.gpu.pack_int4(..., interleave="float16")); interleaved weights are read by the "gemv" (one row,
-    two fp16 rows), "decode", "stream" and panel kernels and the two passes, with results bit-identical to the plain layout
+    two fp16 rows), "decode", "small", "stream" and panel kernels and the two passes, with results bit-identical to the plain layout
     (the GEMV: to the rounding of its fp32 sums).
     tile: rows of activations per work-group of the MFMA kernel (16, 32, 64, 128, 256; 0 = chosen by the
     library); gemv_tuning = (rows_per_wave, waves, blocks_per_cu, depth) and skinny_tuning = (waves,
