@@ -104,6 +104,21 @@ def test_streaming_kernel_by_name_is_refused_without_room_for_its_slices(layout)
     assert run.log == ""
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,group,layout,error", [
+    (700, 258, 384, 128, _abi.W_PLAIN, "N % 4"), (2420, 85, 256, 32, _abi.W_PLAIN, "N % 4"),  # rows over a multiple of four of weights: with the packed result's room only
+    (40, 1024, 3072, 128, _abi.W_INTERLEAVED_F16, "workspace"), (364, 512, 3840, 32, _abi.W_INTERLEAVED_F16, "workspace")])
+def test_automatic_choice_refuses_without_a_workspace_what_wants_one(M, N, K, group, layout, error):
+    """Calls that the other kernels refuse for lack of room are not accepted because the small-tile kernel needs none."""
+    A, (Wp, s, z) = torch.zeros(M, K).half(), make_w4(N, K, group, torch.float16, "int", seed=1)
+    with pytest.raises(RuntimeError, match=error):
+        run(A, Wp, s, z, group, _abi.ALGO_AUTO, layout=layout)
+    assert run.log == ""
+    need = max(_abi.load().tlq_w4a16_workspace_bytes(M, N, K), N * K * 2)
+    run(A, Wp, s, z, group, _abi.ALGO_AUTO, layout=layout, workspace=need)
+    assert "w4a16_small_kernel" in run.log, run.log
+
+
 def test_small_family_refuses_what_its_kernel_does_not_read():
     lib, fake = _abi.load(), ctypes.c_void_p(1 << 20)
     for N, K, group in ((64, 192, 64), (64, 384, 96), (1, 128, 128)):  # K in whole k-blocks, power-of-two groups, an even number of scales

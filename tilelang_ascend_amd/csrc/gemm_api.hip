@@ -842,7 +842,8 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
                              w4a16_panel256_plan(M & ~(int64_t)3, N, K, group, cu_count_or_default()).ok;
   const bool keep_tail = head_and_tail && last_rows_take_f16_gemv(M, N, K, group, in_dtype, scales, zeros);
   // Many rows on so few and short weight rows that the whole call is a matter of latency: the small-tile kernel
-  if (algo == TLQ_ALGO_AUTO && !keep_tail && M > 512 && M < kMaxDim && N >= 1 && N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && w_packed && C && aligned16(A) &&
+  // (weight-row counts that are no multiple of four need the room of run_ragged_rows above, whatever the number of rows)
+  if (algo == TLQ_ALGO_AUTO && !keep_tail && M > 512 && M < kMaxDim && N >= 1 && N % 4 == 0 && N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && w_packed && C && aligned16(A) &&
       aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
       (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
     const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
@@ -1210,20 +1211,25 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
   }
   if (algo != TLQ_ALGO_TWO_PASS) {
     const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
-    if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0) {
+    const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));
+    const bool room_for_two_passes = ws_aligned && workspace_bytes >= N * K * 2;
+    // (no tile kernel reads this layout: the alternative is the two passes)
+    const bool stream_taken = ws_ok && (algo == TLQ_ALGO_STREAM || M <= 384 || (int64_t)sp.m_blocks * sp.n_blocks * sp.split <= cu_count_or_default() ||
+                                        tile_fill(1, M, N, 128) < 0.65 || !room_for_two_passes);
+    // the small-tile kernel in the place of either, for calls that bring the workspace those want: without it they are refused
+    if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (stream_taken || (room_for_two_passes && N % 8 == 0))) {
       const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_stream(small, M, N, K))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
     }
-    const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));
     // (129 .. 512 rows: the 256-row kernel where its estimate beats the streaming kernel's, as for the plain layout)
     if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && panel256_beats_stream(M, N, K, group, sp)) {
       const int rc = try_panel256(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, workspace,
                                   workspace_bytes, stream);
       if (rc >= 0) return rc;
     }
-    if (ws_ok && (algo == TLQ_ALGO_STREAM || M <= 384 || (int64_t)sp.m_blocks * sp.n_blocks * sp.split <= cu_count_or_default() || tile_fill(1, M, N, 128) < 0.65 || !(ws_aligned && workspace_bytes >= N * K * 2)))  // (no tile kernel reads this layout: the alternative is the two passes)
+    if (stream_taken)
       return gemm_w4a16_stream(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, sp,
                                (float*)workspace, (hipStream_t)stream);
     TLQ_REQUIRE(algo != TLQ_ALGO_STREAM, "tlq_gemm_w4a16_layout_ws: the streaming kernel does not take M=%lld N=%lld K=%lld group=%lld "
