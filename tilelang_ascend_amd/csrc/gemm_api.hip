@@ -2,6 +2,7 @@
 // Every shape assumption a kernel makes is checked here, before anything is launched.
 #include "tlq_common.h"
 #include "gemm_core.h"
+#include "small_tiles.h"
 
 namespace tlq {
 int gemv_w4a16(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t batch, int64_t M,
@@ -31,14 +32,6 @@ int gemm_w4a16_stream(const void* A, const void* Wp, const void* scales, const v
                       float* partial, hipStream_t st);
 int gemm_w4a16_skinny(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, hipStream_t st);
-struct SmallPlan {
-  bool ok;
-  int mt, rt, waves;
-  double us;
-};
-SmallPlan w4a16_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros, int force_waves, int force_rt, int force_mt);
-int gemm_w4a16_small(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N, int64_t K, int64_t group,
-                     float zero_scalar, int in_dtype, int out_dtype, int w_layout, const SmallPlan& p, const char* what, hipStream_t st);
 int gemm_f16_plain(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype,
                    int out_dtype, int b_layout, hipStream_t st);
 int gemm_f16_splitk(const void* A, const void* B, float* C, int64_t M, int64_t N, int64_t K, int64_t split_k,
@@ -62,19 +55,6 @@ int gemm_w8a8_rescale_splitk(const void* A, const void* B, const void* scale_a, 
                              int64_t M, int64_t N, int64_t K, int64_t n_scale_b, int64_t split, int b_layout, int out_dtype,
                              hipStream_t st);
 
-// the small-tile kernel of these products (gemm_small.hip); kinds of weights: 0 [N, K], 1 int8 [K, N], 2 16-bit [K, N], 3 packed int4 [N, K / 2]
-struct SmallTile {
-  bool ok;
-  int mt, rt, waves;
-  double us;
-};
-SmallTile small_tile_plan(int kind, int64_t batch, int64_t M, int64_t N, int64_t row_bytes);
-bool small_tile_forced();
-int small_i8(const SmallTile& t, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int b_layout, hipStream_t st);
-int small_w8a8(const SmallTile& t, const void* A, const void* B, const void* scale_a, const void* scale_b, void* C, int64_t batch, int64_t M, int64_t N, int64_t K,
-               int64_t n_scale_b, int b_layout, int out_dtype, hipStream_t st);
-int small_w4a8(const SmallTile& t, const void* A, const void* Wp, void* C, int64_t M, int64_t N, int64_t K, int sign_mode, hipStream_t st);
-int small_f16(const SmallTile& t, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype, int out_dtype, hipStream_t st);
 extern thread_local int g_i8_tile, g_i8_split;
 
 struct PanelPlan {
@@ -247,7 +227,7 @@ int tlq_debug_panelm_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cu
 }
 
 int tlq_debug_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, void* plan_out) {
-  const SmallPlan p = w4a16_small_plan(M, N, K, group, nullptr, nullptr, 0, 0, 0);
+  const SmallTile p = w4a16_small_plan(M, N, K, group, nullptr, nullptr, 0, 0, 0);
   if (plan_out) {
     int64_t* o = (int64_t*)plan_out;
     o[0] = 16 * p.mt, o[1] = 16 * p.rt, o[2] = p.waves, o[3] = (int64_t)(p.us * 1000.0);
@@ -280,15 +260,15 @@ static bool skinny_leaves_cus_idle(int64_t N) {
 // streaming kernel's share of them, 1.47 x over the two passes'.
 static double giga(double m, int64_t N, int64_t K) { return m * (double)N * (double)K * 1e-9; }
 static double up16(int64_t M) { return (double)ceil_div(M, (int64_t)16) * 16.0; }
-static bool small_beats_stream(const SmallPlan& p, int64_t M, int64_t N, int64_t K) {
+static bool small_beats_stream(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
   return p.ok && g_stream_slice_steps <= 0 && p.us < 0.95 * (11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K);
 }
 // above 512 rows (the two passes, or the panel kernels with their head and tail): only while the whole call stays short
-static bool small_beats_panels(const SmallPlan& p, int64_t M, int64_t N, int64_t K) {
+static bool small_beats_panels(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
   return p.ok && p.us < 13.0 && p.us < 0.9 * (14.9 + 3.6 * giga(up16(M), N, K) + 0.79e-3 * (double)K);
 }
 // the decode kernel over chunks of K, whose second launch adds the chunks
-static bool small_beats_decode_chunks(const SmallPlan& p, int64_t M, int64_t N, int64_t K) {
+static bool small_beats_decode_chunks(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
   return p.ok && p.us < 0.95 * (5.2 + 0.67 * giga((double)M, N, K) + 4.36 * giga(up16(M), N, K) + 0.023e-6 * (double)N * (double)K + 0.25e-3 * (double)K);
 }
 // The skinny kernel on 17 .. 64 rows (12.8 -> 7.8 us for M = 64 on 5120 x 1280, level where the launch is all there is) and the tile
@@ -296,7 +276,7 @@ static bool small_beats_decode_chunks(const SmallPlan& p, int64_t M, int64_t N, 
 // the family the automatic choice runs in their place.
 static int small_or(int algo, int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros) {
   if (algo == TLQ_ALGO_SKINNY ? M <= 16 || w4a16_skinny_forced() : algo != TLQ_ALGO_MFMA || N % 4 != 0 || w4a16_tile_forced()) return algo;
-  const SmallPlan p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+  const SmallTile p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
   const double theirs = algo == TLQ_ALGO_SKINNY ? 0.95 * (5.2 + 7.0 * giga((double)M, N, K) + 4.1 * giga(up16(M), N, K) + 0.3e-3 * (double)K)
                                                 : 0.9 * (3.9 + 11.6e-3 * (double)K + 0.94 * giga((double)M, N, K) + 0.116e-6 * (double)M * (double)N);
   return p.ok && p.us < theirs ? TLQ_ALGO_SMALL : algo;
@@ -376,7 +356,7 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
   const bool decode_ok = w4a16_decode_in_one_chunk(dp, scales, zeros);
   if (algo == TLQ_ALGO_AUTO) algo = small_or(w4a16_few_rows_choice(M, N, K, group, in_dtype, scales, zeros, decode_ok), M, N, K, group, scales, zeros);
   if (algo == TLQ_ALGO_SMALL) {
-    const SmallPlan p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+    const SmallTile p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
     TLQ_REQUIRE(p.ok, TLQ_SMALL_NEEDS("tlq_gemm_w4a16"), (long long)M, (long long)N, (long long)K, (long long)group);
     return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, p, "tlq_gemm_w4a16(small)", st);
   }
@@ -846,7 +826,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   if (algo == TLQ_ALGO_AUTO && !keep_tail && M > 512 && M < kMaxDim && N >= 1 && N % 4 == 0 && N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && w_packed && C && aligned16(A) &&
       aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
       (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
-    const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+    const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
     if (small_beats_panels(small, M, N, K))
       return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                               (hipStream_t)stream);
@@ -902,7 +882,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     // (640 work-groups on 512 places): 15 against 20 - 26 us; N = 12288, K = 6144 (768): 14 - 15 against 17 - 21 us;
     // N = 17408, K = 5120 (1088): 17 - 19 against 20 - 24 us; with 512 or 960 work-groups the skinny kernel is ahead)
     if (algo == TLQ_ALGO_AUTO && dp.ok && dp.chunks > 1 && args_ok) {
-      const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+      const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_decode_chunks(small, M, N, K))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
@@ -993,7 +973,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
                          ((uintptr_t)scales & 1) == 0 && ((uintptr_t)zeros & 1) == 0 && K > 0 && fits32(M, K * 2) && fits32(N, K / 2);
     const bool ws_ok = sp.ok && (sp.split == 1 || (workspace && aligned16(workspace) && workspace_bytes >= (int64_t)sp.split * M * N * 4));
     if (algo == TLQ_ALGO_AUTO && sp.ok && args_ok) {
-      const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+      const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_stream(small, M, N, K))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
@@ -1156,7 +1136,7 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
   }
   const bool ws_aligned = workspace && aligned16(workspace);
   if (algo == TLQ_ALGO_SMALL) {
-    const SmallPlan p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+    const SmallTile p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
     TLQ_REQUIRE(p.ok, TLQ_SMALL_NEEDS("tlq_gemm_w4a16_layout_ws"), (long long)M, (long long)N, (long long)K, (long long)group);
     return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, p, "tlq_gemm_w4a16(small)", (hipStream_t)stream);
   }
@@ -1218,7 +1198,7 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
                                         tile_fill(1, M, N, 128) < 0.65 || !room_for_two_passes);
     // the small-tile kernel in the place of either, for calls that bring the workspace those want: without it they are refused
     if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (stream_taken || (room_for_two_passes && N % 8 == 0))) {
-      const SmallPlan small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+      const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_stream(small, M, N, K))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);

@@ -13,10 +13,9 @@
 //   weights stored [K, N] (RT = 4):          [128 or 64 k rows][64 columns] as they are, eight loads, transposed by the read
 #pragma once
 #include "gemm_core.h"
+#include "small_tiles.h"
 
 namespace tlq {
-
-enum SmallW { kSmallNK = 0, kSmallKN8 = 1, kSmallKN16 = 2, kSmallW4 = 3 };
 
 template <SmallW W, int RT, int MT>
 struct SmallCfg {

@@ -4,12 +4,6 @@
 
 namespace tlq {
 
-struct SmallTile {
-  bool ok;
-  int mt, rt, waves;
-  double us;  // estimated time of a call
-};
-
 static thread_local int g_small_waves = 0, g_small_tiles = 0;  // tuning and tests: forced variant; tiles < 0: never
 
 static constexpr int small_slot(SmallW w, int rt, int mt) { return mt * 2048 + (w == kSmallNK ? rt * 2048 : (w == kSmallW4 ? rt * 1024 : 8192)); }
@@ -64,7 +58,6 @@ static SmallTile small_tile_now(int kind, int64_t batch, int64_t M, int64_t N, i
   return best;
 }
 
-// kind: SmallW; row_bytes: bytes of K in an activation row
 SmallTile small_tile_plan(int kind, int64_t batch, int64_t M, int64_t N, int64_t row_bytes) {
   if (g_small_tiles < 0 || batch < 1 || M < 1 || N < 16 || row_bytes < 128 || row_bytes % 128 != 0) return SmallTile{false, 0, 0, 0, 0.0};
   return small_tile_now(kind, batch, M, N, row_bytes / 128);
@@ -129,7 +122,6 @@ int small_w4a8(const SmallTile& t, const void* A, const void* Wp, void* C, int64
   return launch_tile<MmaI8, kSmallW4, EpiInt32>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
 }
 
-// [K, N] weights
 int small_f16(const SmallTile& t, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype, int out_dtype, hipStream_t st) {
   EpiFloat::Params pe{C, N, M * N, out_dtype};
   const SmallParams p = small_params(A, B, M, N, K * 2, N * 2, N * K * 2);

@@ -21,17 +21,9 @@
 // bfloat16 roundings, v_cvt_pk_bf16_f32 to pack pairs in k order.
 #include "gemm_core.h"
 #include "expand8.h"
+#include "small_tiles.h"
 
 namespace tlq {
-
-struct SmallPlan {
-  bool ok;
-  int mt, rt, waves;
-  double us;
-};
-SmallPlan w4a16_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros, int force_waves, int force_rt, int force_mt);
-int gemm_w4a16_small(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N, int64_t K, int64_t group,
-                     float zero_scalar, int in_dtype, int out_dtype, int w_layout, const SmallPlan& p, const char* what, hipStream_t st);
 
 template <typename T, bool FOLD, int ROWS, int NT>
 struct W4Loader {
@@ -389,7 +381,7 @@ static int dispatch_skinny(const W4Args& a) {
   // up to 16 rows and power-of-two groups: operands staged through wavefront-private LDS, which is the small-tile kernel with
   // tiles of 16 activation rows (more rows: only where a tuning hook asks for it)
   if (g_skinny_lds == 1 || (a.M <= 16 && g_skinny_lds != 0)) {
-    const SmallPlan p = w4a16_small_plan(a.M, a.N, a.K, a.group, a.scales, a.zeros, g_skinny_waves, g_skinny_rt, g_skinny_mt);
+    const SmallTile p = w4a16_small_plan(a.M, a.N, a.K, a.group, a.scales, a.zeros, g_skinny_waves, g_skinny_rt, g_skinny_mt);
     if (p.ok)
       return gemm_w4a16_small(a.A, a.Wp, a.scales, a.zeros, a.C, a.M, a.N, a.K, a.group, a.zero_scalar, std::is_same<T, half_t>::value ? TLQ_F16 : TLQ_BF16, a.out_dtype,
                               TLQ_W_PLAIN, p, "tlq_gemm_w4a16(skinny)", a.st);

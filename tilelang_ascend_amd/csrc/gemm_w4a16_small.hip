@@ -20,6 +20,7 @@
 // interleave_weight (tilelang/quantize/utils.py:73-101, fp16 target); the same sums, so the same bits.
 #include "expand8.h"
 #include "gemm_core.h"
+#include "small_tiles.h"
 
 namespace tlq {
 
@@ -262,30 +263,24 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
   }
 }
 
-struct SmallPlan {
-  bool ok;
-  int mt, rt, waves;
-  double us;  // estimated time of a call
-};
-
 // Tile, wavefronts per work-group (the cut of K) and an estimate of the call's time, or ok = false where the kernel does not
 // apply.  The estimate: a launch, then rounds of the work-groups the machine holds at once (LDS and registers) x the longest
 // chain of k-blocks in a wavefront, plus what a CU does for its share of the tiles: dequantising (the vector rate) and
 // operand traffic and multiplications per 16 x 16 tile and k-block.  Fitted to 520 problems (M 2 .. 700, N 256 .. 14400,
 // K 256 .. 14336, both types, groups of 64 and 128, zero-point tensor or scalar) x up to 24 forced variants each: 12 % rms over all
 // variants; the variant it picks is 2.4 % behind the fastest on average.
-static SmallPlan small_plan_now(int64_t M, int64_t N, int64_t K, int force_waves, int force_rt, int force_mt);
-SmallPlan w4a16_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros, int force_waves, int force_rt, int force_mt) {
-  SmallPlan best{false, 0, 0, 0, 0.0};
+static SmallTile small_plan_now(int64_t M, int64_t N, int64_t K, int force_waves, int force_rt, int force_mt);
+SmallTile w4a16_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros, int force_waves, int force_rt, int force_mt) {
+  SmallTile best{false, 0, 0, 0, 0.0};
   if (M < 1 || N < 1 || K < 128 || K % 128 != 0 || group < 32 || (group & (group - 1)) != 0 || K % group != 0) return best;
   // (the scale / zero gathers read aligned dwords: the tensors must start and end on a dword boundary; 32-bit offsets)
   if ((((uintptr_t)scales | (uintptr_t)zeros) & 3) != 0 || ((N * (K / group)) & 1) != 0) return best;
   if (M * K * 2 >= ((int64_t)1 << 32) || N * (K / 2) >= ((int64_t)1 << 32) || N * (K / group) >= ((int64_t)1 << 31)) return best;
-  static thread_local PlanTable<SmallPlan> known;
+  static thread_local PlanTable<SmallTile> known;
   return known.get(M, N, K, force_waves * 100 + force_rt * 10 + force_mt, [&] { return small_plan_now(M, N, K, force_waves, force_rt, force_mt); });
 }
-static SmallPlan small_plan_now(int64_t M, int64_t N, int64_t K, int force_waves, int force_rt, int force_mt) {
-  SmallPlan best{false, 0, 0, 0, 0.0};
+static SmallTile small_plan_now(int64_t M, int64_t N, int64_t K, int force_waves, int force_rt, int force_mt) {
+  SmallTile best{false, 0, 0, 0, 0.0};
   int cus = tlq_device_cu_count();
   if (cus <= 0) cus = 256;
   const int64_t KB = K / 128;
@@ -305,7 +300,7 @@ static SmallPlan small_plan_now(int64_t M, int64_t N, int64_t K, int force_waves
         if (held < 1) held = 1;
         const double rounds = (double)ceil_div(blocks, cus * held), per_cu = (double)ceil_div(blocks, (int64_t)cus) * (double)KB;
         const double us = 2.8 + rounds * (1.15 + 0.163 * (double)ceil_div(KB, w) + 0.034 * (double)w) + per_cu * (0.027 * rt + 0.0298 * rt * mt);
-        if (!best.ok || us < best.us * 0.995) best = SmallPlan{true, mt, rt, (int)w, us};
+        if (!best.ok || us < best.us * 0.995) best = SmallTile{true, mt, rt, (int)w, us};
       }
     }
   }
@@ -342,7 +337,7 @@ static int launch_small(const SmallArgs& a, int waves) {
 }
 
 template <typename T, bool FOLD, int LAYOUT>
-static int dispatch_small(const SmallArgs& a, const SmallPlan& p) {
+static int dispatch_small(const SmallArgs& a, const SmallTile& p) {
 #define TLQ_SMALL(RT, MT) \
   if (p.rt == RT && p.mt == MT) return launch_small<T, FOLD, LAYOUT, RT, MT>(a, p.waves);
   TLQ_SMALL(1, 1) TLQ_SMALL(2, 1) TLQ_SMALL(4, 1) TLQ_SMALL(1, 2) TLQ_SMALL(2, 2) TLQ_SMALL(4, 2) TLQ_SMALL(1, 4) TLQ_SMALL(2, 4) TLQ_SMALL(4, 4)
@@ -351,9 +346,8 @@ static int dispatch_small(const SmallArgs& a, const SmallPlan& p) {
   return 1;
 }
 
-// `what`: the entry point and family on whose behalf the kernel runs, for the launch log and error texts
 int gemm_w4a16_small(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N, int64_t K, int64_t group,
-                     float zero_scalar, int in_dtype, int out_dtype, int w_layout, const SmallPlan& p, const char* what, hipStream_t st) {
+                     float zero_scalar, int in_dtype, int out_dtype, int w_layout, const SmallTile& p, const char* what, hipStream_t st) {
   // An integer zero point shared by the whole matrix folds exactly into the unpack bias.
   const bool fold = zeros == nullptr && zero_scalar == (float)(int)zero_scalar && zero_scalar >= -256.0f && zero_scalar <= 256.0f;
   int gshift = 0;
