@@ -52,6 +52,10 @@ int tlq_debug_check_panel256_schedule(int steps, int wait_w, int wait_a);
 /* What the small-tile kernel (one launch, wavefronts split K) would take for a problem: plan_out receives int64 activation rows and weight
  * rows per work-group, wavefronts, estimated nanoseconds; returns 1 when it applies. */
 int tlq_debug_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, void* plan_out);
+/* The addresses and the ring of both small-tile kernels on the corner tiles of a problem.  kind as for tlq_debug_small_tile, 4 = W4A16 with
+ * groups of `group` values (else ignored); row_bytes: bytes of K of an activation row; rows, cols: of a work-group's tile.  extra_in_flight is added to
+ * every wait's count of loads (0 = the kernels' own; more: to see the walk fail). */
+int tlq_debug_check_small_addressing(int kind, int64_t M, int64_t N, int64_t row_bytes, int64_t group, int rows, int cols, int waves, int extra_in_flight);
 /* The middle-M panel kernel (TLQ_ALGO_PANELM): its plan (plan_out: int64 tiles_m, tiles_n, K slices, steps per slice, activation
  * rows per work-group). */
 int tlq_debug_panelm_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out);

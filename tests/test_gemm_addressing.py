@@ -87,3 +87,27 @@ def test_streaming_kernel_addressing(tm, depth):
         _ok(lib.tlq_debug_check_stream_addressing(M, N, K, tm, depth))
     assert lib.tlq_debug_check_stream_addressing(64, 256, 100, tm, depth) != 0   # K not a multiple of 128
     assert lib.tlq_debug_check_stream_addressing(64, 1 << 22, 4096, tm, depth) != 0  # packed weights of 8 GiB
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2, 3, 4])
+def test_small_tile_kernels_addressing_and_schedule(kind):
+    """Both small-tile kernels: loads inside their matrices (rows past them clamped), operand reads on the cells that hold what they
+    multiply, scales and zero points of the right group, and rings whose waits cover what is read and whose loads overwrite
+    nothing still to be read; with one load more left in flight the walk fails."""
+    lib = _abi.load()
+    unit = 256 if kind == 4 else 128
+    for rows in (16, 32, 64):
+        for cols in ((64,) if kind in (1, 2) else (16, 32, 64)):
+            for M, N, steps, group, waves in ((1, 16, 1, 128, 1), (17, 48, 5, 32, 2), (33, 80, 7, 64, 3), (70, 1008, 16, 256, 4), (5, 144, 33, 128, 8),
+                                              (200, 272, 16, 2048, 1), (1000, 4096, 40, 32, 5), (64, 136 if kind == 2 else 144, 24, 512, 8)):
+                group = min(group, 128 * steps & -(128 * steps))  # (a power of two that divides K)
+                wave_lds = {0: 2 * 128 * (rows + cols), 1: 2 * (128 * rows + 8192), 2: 2 * (128 * rows + 8192), 3: 2 * (128 * rows + 64 * cols),
+                            4: 2 * (256 * rows + 64 * cols + 32 * cols)}[kind]
+                waves = min(waves, 160 * 1024 // (2 * wave_lds))
+                _ok(lib.tlq_debug_check_small_addressing(kind, M, N, unit * steps, group, rows, cols, waves, 0))
+                if steps > waves:
+                    assert lib.tlq_debug_check_small_addressing(kind, M, N, unit * steps, group, rows, cols, waves, 1) != 0
+                    assert "in flight" in _abi.last_error()
+    assert lib.tlq_debug_check_small_addressing(kind, 16, 16, unit + 64, 32, 16, 64, 1, 0) != 0        # a part of a step
+    assert lib.tlq_debug_check_small_addressing(kind, 1 << 21, 64, unit * 16, 32, 16, 64, 1, 0) != 0    # activations of 4 GiB and more
+    assert lib.tlq_debug_check_small_addressing(kind, 64, 64, unit * 64, 32, 64, 64, 16, 0) != 0        # more LDS than there is

@@ -75,6 +75,7 @@ SIGNATURES = {
     "tlq_debug_panel256_plan": (_int, [_i64, _i64, _i64, _i64, _int, _vp]),
     "tlq_debug_check_panel256_schedule": (_int, [_int, _int, _int]),
     "tlq_debug_small_plan": (_int, [_i64, _i64, _i64, _i64, _vp]),
+    "tlq_debug_check_small_addressing": (_int, [_int, _i64, _i64, _i64, _i64, _int, _int, _int, _int]),
     "tlq_debug_panelm_plan": (_int, [_i64, _i64, _i64, _i64, _int, _vp]),
     "tlq_debug_check_panelm_addressing": (_int, [_i64, _i64, _i64, _i64, _int, _int]),
     "tlq_debug_check_panelm_schedule": (_int, [_int, _int, _int, _int, _int]),

@@ -425,5 +425,30 @@ __host__ __device__ inline int ring_younger_rows(int i, int my_rows, int depth) 
   return y < depth - 1 ? y : depth - 1;
 }
 
+// ---- small-tile kernels (gemm_small.h, gemm_w4a16_small.hip) ------------------------------------------------------
+// Wavefront w of W owns the steps small_first(w) .. small_first(w + 1) - 1 of a tile and runs them through a ring of D slots of
+// its own: the first D steps are issued ahead, step i + D once the contents of step i are in registers.  At the top of step i the
+// loads of the steps behind it, small_younger of them, may be outstanding.
+__host__ __device__ inline int small_first(int wave, int waves, int steps) { return (int)(((int64_t)wave * steps) / waves); }
+__host__ __device__ inline int small_younger(int i, int n, int D) { return n - 1 - i < D - 1 ? n - 1 - i : D - 1; }
+// gemm_small.h, steps of 128 bytes of K: 2 KB per 16 activation rows, then the weights (kind: SmallW)
+__host__ __device__ constexpr int small_w_tile(int kind, int rt) { return kind == 0 ? rt * 2048 : (kind == 3 ? rt * 1024 : 8192); }
+__host__ __device__ constexpr int small_slot_bytes(int kind, int rt, int mt) { return mt * 2048 + small_w_tile(kind, rt); }
+__host__ __device__ constexpr int small_depth(int slot_bytes) { return slot_bytes <= 4096 ? 4 : (slot_bytes <= 8192 ? 3 : 2); }
+// gemm_w4a16_small.hip, steps of 128 values of K, D = 2: rt [16 rows][64 B] packed tiles, then 4 KB per 16 activation rows; behind the
+// two slots two buffers of gathered scales and zero points, [rt][scale | zero][64 dwords] each.  A gather covers four consecutive
+// groups of a tile's 16 rows (lane: row r16, group q), dwords that hold a row's group and one of its neighbours.
+__host__ __device__ constexpr int smallw_slot_bytes(int rt, int mt) { return rt * 1024 + mt * 4096; }
+__host__ __device__ constexpr int smallw_sc_bytes(int rt) { return rt * 2 * 256; }
+__host__ __device__ inline int smallw_sc_base(int kb, int gshift) { return ((kb << 7) >> gshift) & ~3; }
+__host__ __device__ inline int smallw_sc_buf(int kb, int gshift) { return (smallw_sc_base(kb, gshift) >> 2) & 1; }
+__host__ __device__ inline bool smallw_new_period(int kb, int kb0, int gshift) { return kb == kb0 || smallw_sc_base(kb, gshift) != smallw_sc_base(kb - 1, gshift); }
+__host__ __device__ inline uint64_t smallw_sc_elem(int lane, int base, uint32_t row_g, int groups) {
+  const int g = base + (lane >> 4);
+  return (uint64_t)row_g + (uint64_t)(g < groups ? g : groups - 1);
+}
+__host__ __device__ inline int smallw_group(int lane, int kb, int gshift) { return ((kb << 7) + ((lane >> 4) << 5)) >> gshift; }
+__host__ __device__ inline int smallw_sc_cell(int lane, int kb, int gshift) { return (lane & 15) + 16 * (smallw_group(lane, kb, gshift) - smallw_sc_base(kb, gshift)); }
+
 }  // namespace addr
 }  // namespace tlq

@@ -966,6 +966,179 @@ int check_decode_ring(int my_tiles) {
   return 0;
 }
 
+// Small-tile kernels.  kind 0 .. 3: gemm_small.h (SmallW), 4: gemm_w4a16_small.hip (group: values per scale; scales and zero points both
+// there).  Tiles of 16 mt activation rows x 16 rt weight rows; the corner tiles of the grid (first and last in either direction: the
+// ones whose rows are clamped) are walked whole, every wavefront, step, load instruction and lane: each load inside its matrix and on
+// the bytes that its row and chunk name, each operand read on cells that hold what it multiplies and whose load has been waited for,
+// no load into a cell that is still to be read.  extra: added to every wait's count of loads in flight (to see the walk fail).
+int check_small(int kind, int64_t M, int64_t N, int64_t row_bytes, int64_t group, int mt, int rt, int waves, int extra) {
+  const bool wide = kind == 4;  // W4A16
+  const int step_bytes = wide ? 256 : 128;
+  CHECK_OR_FAIL(kind >= 0 && kind <= 4 && (mt == 1 || mt == 2 || mt == 4) && (rt == 1 || rt == 2 || rt == 4), "small tiles: kind %d, %d x %d", kind, mt, rt);
+  CHECK_OR_FAIL(M >= 1 && N >= 1 && row_bytes >= step_bytes && row_bytes % step_bytes == 0, "small tiles: bad shape");
+  CHECK_OR_FAIL((kind != 1 && kind != 2) || (rt == 4 && N % (kind == 1 ? 16 : 8) == 0), "small tiles: [K, N] weights come in tiles of 64 columns, whole chunks");
+  const int steps = (int)(row_bytes / step_bytes);
+  CHECK_OR_FAIL(waves >= 1 && waves <= 16 && waves <= steps, "small tiles: %d wavefronts", waves);
+  const int64_t K = kind == 2 || wide ? row_bytes / 2 : row_bytes;  // values
+  const int64_t w_row = kind == 0 ? row_bytes : kind == 1 ? N : kind == 2 ? 2 * N : K / 2, w_extent = kind == 1 || kind == 2 ? K * w_row : N * w_row;
+  const int64_t a_extent = M * row_bytes;
+  CHECK_OR_FAIL(a_extent < ((int64_t)1 << 32) && w_extent < ((int64_t)1 << 32), "small tiles: a matrix spans 4 GiB or more");
+  int gshift = 0;
+  if (wide) {
+    while (((int64_t)1 << gshift) < group) ++gshift;
+    CHECK_OR_FAIL(group >= 32 && ((int64_t)1 << gshift) == group && K % group == 0 && (N * (K / group)) % 2 == 0, "small tiles: bad group");
+  }
+  const int groups = wide ? (int)(K / group) : 0;
+  const int slot_bytes = wide ? addr::smallw_slot_bytes(rt, mt) : addr::small_slot_bytes(kind, rt, mt), D = wide ? 2 : addr::small_depth(slot_bytes);
+  const int w_at = wide ? 0 : mt * 2048, a_at = wide ? rt * 1024 : 0;  // where the weights / activations of a slot begin
+  const int sc_bytes = wide ? addr::smallw_sc_bytes(rt) : 0;
+  CHECK_OR_FAIL((int64_t)waves * (D * slot_bytes + 2 * sc_bytes) <= 160 * 1024, "small tiles: LDS");
+  const int step_loads = slot_bytes / 1024;
+
+  struct Cell {
+    int step = -1, load = -1;
+    int64_t row = -1, at = -1;  // row of the matrix (k row of [K, N] weights), byte offset in that row's step (or in the k row)
+  };
+  struct Pair {
+    int64_t dword = -1;
+    int load = -1, last_kb = -1;  // the last step that reads it
+  };
+  const int64_t tiles_m = ceil_div(M, (int64_t)16 * mt), tiles_n = ceil_div(N, (int64_t)16 * rt);
+  for (int64_t tm : {(int64_t)0, tiles_m - 1})
+    for (int64_t tn : {(int64_t)0, tiles_n - 1})
+      for (int wave = 0; wave < waves; ++wave) {
+        const int m_base = (int)(tm * 16 * mt), n_base = (int)(tn * 16 * rt);
+        const int s0 = addr::small_first(wave, waves, steps), n = addr::small_first(wave + 1, waves, steps) - s0;
+        CHECK_OR_FAIL(n >= 1 && (wave > 0 || s0 == 0) && (wave + 1 < waves || s0 + n == steps), "small tiles: the cut of K");
+        std::vector<Cell> cells(D * slot_bytes / 16);
+        std::vector<Pair> pairs(2 * sc_bytes / 4);
+        int issued = 0, landed = 0, read_steps = 0;  // loads issued / known to have landed; steps whose operands are in registers
+        auto a_row = [&](int r) { return m_base + r < M ? (int64_t)m_base + r : M - 1; };
+        auto w_row_of = [&](int r) { return n_base + r < N ? (int64_t)n_base + r : N - 1; };
+        auto put = [&](int slot, int at, int lane, const char* what, int step, int64_t row, int64_t byte, int64_t off, int64_t want, int64_t extent) -> int {
+          CHECK_OR_FAIL(off == want && off >= 0 && off + 16 <= extent, "small tiles: %s load at byte %lld (step %d lane %d), row %lld byte %lld lies at %lld of %lld", what,
+                        (long long)off, step, lane, (long long)row, (long long)byte, (long long)want, (long long)extent);
+          CHECK_OR_FAIL(at >= 0 && at + 1024 <= slot_bytes, "small tiles: %s load lands outside its slot", what);
+          Cell& c = cells[(slot * slot_bytes + at) / 16 + lane];
+          CHECK_OR_FAIL(c.step < 0 || c.step - s0 < read_steps, "small tiles: a load of step %d overwrites step %d, which is still to be read", step, c.step);
+          c.step = step, c.load = issued, c.row = row, c.at = byte;
+          return 0;
+        };
+        auto issue_period = [&](int kb) -> int {
+          const int base = addr::smallw_sc_base(kb, gshift), buf = addr::smallw_sc_buf(kb, gshift);
+          int last = kb;  // the steps of this wavefront that share the gather
+          while (last + 1 < s0 + n && addr::smallw_sc_base(last + 1, gshift) == base) ++last;
+          for (int t = 0; t < rt; ++t)
+            for (int z = 0; z < 2; ++z, ++issued)
+              for (int lane = 0; lane < 64; ++lane) {
+                const int64_t row = w_row_of(t * 16 + (lane & 15)), byte = (int64_t)((addr::smallw_sc_elem(lane, base, (uint32_t)row * (uint32_t)groups, groups) * 2u) & ~(uint64_t)3);
+                CHECK_OR_FAIL(byte >= 0 && byte + 4 <= N * groups * 2, "small tiles: scale gather at byte %lld of %lld", (long long)byte, (long long)(N * groups * 2));
+                Pair& p = pairs[buf * (sc_bytes / 4) + (t * 2 + z) * 64 + lane];
+                CHECK_OR_FAIL(p.dword < 0 || p.last_kb - s0 < read_steps, "small tiles: a gather for step %d overwrites one that step %d still reads", kb, p.last_kb);
+                p.dword = byte / 4, p.load = issued, p.last_kb = last;
+              }
+          return 0;
+        };
+        auto issue = [&](int i) -> int {
+          const int s = s0 + i, slot = i % D;
+          if (wide && addr::smallw_new_period(s, s0, gshift))
+            if (int rc = issue_period(s)) return rc;
+          const int w_loads = (slot_bytes - (wide ? mt * 4096 : mt * 2048)) / 1024;
+          for (int j = 0; j < w_loads; ++j, ++issued)
+            for (int lane = 0; lane < 64; ++lane) {
+              int64_t row, byte, off, want;
+              if (kind == 0) {
+                row = w_row_of(addr::rd_row(lane, 0, j, 1)), byte = addr::rd_chunk(lane) * 16;
+                off = (int64_t)(uint32_t)(addr::rd_voff(lane, 0, j, 1, (int)(N - n_base), (uint32_t)w_row) + (uint32_t)n_base * (uint32_t)w_row) + (int64_t)s * 128;
+                want = row * w_row + (int64_t)s * 128 + byte;
+              } else if (kind == 3 || wide) {
+                row = w_row_of(j * 16 + addr::sw_row(lane)), byte = addr::sw_piece(lane) * 16;
+                off = (int64_t)(uint32_t)((uint32_t)row * (uint32_t)w_row + (uint32_t)byte) + (int64_t)s * 64;
+                want = row * w_row + (int64_t)s * 64 + byte;
+              } else {
+                const int kr = kind == 1 ? 128 : 64;
+                row = kind == 1 ? addr::kn_k<64>(lane, 0, j, 1) : addr::kn16_k<64>(lane, 0, j, 1);
+                const uint32_t v = kind == 1 ? addr::kn_voff<64>(lane, 0, j, 1, (int)(N - n_base), (uint32_t)w_row) : addr::kn16_voff<64>(lane, 0, j, 1, (int)(N - n_base), (uint32_t)w_row);
+                CHECK_OR_FAIL(row < kr, "small tiles: k row %lld of a step", (long long)row);
+                byte = (int64_t)v - row * w_row;
+                CHECK_OR_FAIL(byte >= 0 && n_base * (kind == 1 ? 1 : 2) + byte + 16 <= w_row, "small tiles: a load past the end of its k row");
+                off = (int64_t)(uint32_t)(v + (uint32_t)(n_base * (kind == 1 ? 1 : 2))) + (int64_t)s * kr * w_row;
+                want = ((int64_t)s * kr + row) * w_row + n_base * (kind == 1 ? 1 : 2) + byte;
+              }
+              if (int rc = put(slot, w_at + j * 1024, lane, "weight", s, row, byte, off, want, w_extent)) return rc;
+            }
+          const int a_loads = (wide ? 4 : 2) * mt;
+          for (int j = 0; j < a_loads; ++j, ++issued)
+            for (int lane = 0; lane < 64; ++lane) {
+              const int64_t row = a_row(wide ? addr::sa_row(lane, j) : addr::rd_row(lane, 0, j, 1)), byte = (wide ? addr::sa_chunk(lane, j) : addr::rd_chunk(lane)) * 16;
+              const int64_t off = (wide ? (int64_t)(uint32_t)(((uint32_t)row * (uint32_t)K) * 2u + (uint32_t)byte)
+                                        : (int64_t)(uint32_t)(addr::rd_voff(lane, 0, j, 1, (int)(M - m_base), (uint32_t)row_bytes) + (uint32_t)m_base * (uint32_t)row_bytes)) +
+                                  (int64_t)s * step_bytes;
+              if (int rc = put(slot, a_at + j * 1024, lane, "activation", s, row, byte, off, row * row_bytes + (int64_t)s * step_bytes + byte, a_extent)) return rc;
+            }
+          return 0;
+        };
+        auto find = [&](uint32_t off, int bytes, int slot, int step, const char* what, int64_t row, int64_t byte, int lane) -> int {
+          CHECK_OR_FAIL(off % bytes == 0 && off + bytes <= (uint32_t)slot_bytes, "small tiles: %s operand read at %u", what, off);
+          const Cell& c = cells[(slot * slot_bytes + off) / 16];
+          CHECK_OR_FAIL(c.step == step && c.load < landed, "small tiles: %s operand of step %d lane %d: the cell holds step %d, %s", what, step, lane, c.step,
+                        c.load < landed ? "landed" : "which may be in flight");
+          CHECK_OR_FAIL(row < 0 || (c.row == row && c.at + off % 16 == byte), "small tiles: %s operand of lane %d finds row %lld byte %lld, expects %lld byte %lld", what, lane,
+                        (long long)c.row, (long long)(c.at + off % 16), (long long)row, (long long)byte);
+          return 0;
+        };
+        for (int i = 0; i < D && i < n; ++i)
+          if (int rc = issue(i)) return rc;
+        for (int i = 0; i < n; ++i) {
+          const int kb = s0 + i, younger = addr::small_younger(i, n, D);
+          int outstanding = younger * step_loads + extra;
+          if (wide && younger && addr::smallw_new_period(kb + 1, s0, gshift)) outstanding += 2 * rt;
+          if (issued - outstanding > landed) landed = issued - outstanding;
+          const int slot = i % D;
+          for (int lane = 0; lane < 64; ++lane) {
+            const int r16 = lane & 15, q = lane >> 4;
+            for (int t = 0; t < mt; ++t)
+              for (int ks = 0; ks < (wide ? 4 : 2); ++ks) {
+                const uint32_t off = wide ? (uint32_t)a_at + addr::sa_frag_off(lane, 0, ks) + t * 4096 : (uint32_t)(addr::row_lds_off(r16, kind == 3 ? 2 * q + ks : q + 4 * ks) + t * 2048);
+                if (int rc = find(off, 16, slot, kb, "activation", a_row(t * 16 + r16), 16 * (wide ? 4 * q + ks : kind == 3 ? 2 * q + ks : q + 4 * ks), lane)) return rc;
+              }
+            for (int t = 0; t < rt; ++t) {
+              if (kind == 3 || wide) {
+                if (int rc = find((uint32_t)w_at + addr::sw_frag_off(lane) + t * 1024, 16, slot, kb, "weight", w_row_of(t * 16 + r16), 16 * q, lane)) return rc;
+              } else if (kind == 0) {
+                for (int ks = 0; ks < 2; ++ks)
+                  if (int rc = find((uint32_t)(w_at + addr::row_lds_off(r16, q + 4 * ks) + t * 2048), 16, slot, kb, "weight", w_row_of(t * 16 + r16), 16 * (q + 4 * ks), lane)) return rc;
+              } else {
+                for (int ks = 0; ks < 2; ++ks)
+                  for (int h = 0; h < 2; ++h) {
+                    const bool in = n_base + t * 16 < N;  // columns past the matrix: any loaded cell
+                    const uint32_t off = kind == 1 ? addr::knfrag_off<64>(lane, 0, t) + (uint32_t)(ks * 64 * 64 + h * 8 * 64) : addr::kn16frag_off<64>(lane, 0, t) + (uint32_t)(ks * 32 * 128 + h * 4 * 128);
+                    const int k = kind == 1 ? 16 * q + (r16 >> 1) + 8 * h + 64 * ks : 8 * q + (r16 >> 2) + 4 * h + 32 * ks;
+                    const int64_t byte = kind == 1 ? t * 16 + 8 * (r16 & 1) : 2 * (t * 16 + 4 * (r16 & 3));
+                    const bool col_in = kind == 1 ? in : n_base + t * 16 + 4 * (r16 & 3) < N;
+                    if (int rc = find((uint32_t)w_at + off, 8, slot, kb, "weight", col_in ? k : -1, byte, lane)) return rc;
+                  }
+              }
+              if (wide) {
+                const int g = addr::smallw_group(lane, kb, gshift), cell = addr::smallw_sc_cell(lane, kb, gshift);
+                CHECK_OR_FAIL(g < groups && cell >= 0 && cell < 64, "small tiles: scale cell %d of group %d", cell, g);
+                const int64_t elem = w_row_of(t * 16 + r16) * groups + g;
+                for (int z = 0; z < 2; ++z) {
+                  const Pair& p = pairs[addr::smallw_sc_buf(kb, gshift) * (sc_bytes / 4) + (t * 2 + z) * 64 + cell];
+                  CHECK_OR_FAIL(p.dword == elem / 2 && p.load < landed && p.last_kb >= kb, "small tiles: scale of step %d lane %d: the cell holds dword %lld, expects %lld (%s)", kb, lane,
+                                (long long)p.dword, (long long)(elem / 2), p.load < landed ? "landed" : "may be in flight");
+                }
+              }
+            }
+          }
+          read_steps = i + 1;
+          if (i + D < n)
+            if (int rc = issue(i + D)) return rc;
+        }
+      }
+  return 0;
+}
+
 }  // namespace
 }  // namespace tlq
 
@@ -1158,6 +1331,10 @@ int tlq_debug_check_slots_schedule(int stages, int loads_per_tile) {
 
 int tlq_debug_check_gemv_ring_addressing(int64_t M, int64_t N, int64_t K, int64_t group, int rows_per_block, int waves, int depth) {
   return check_gemv_ring(M, N, K, group, rows_per_block, waves, depth);
+}
+
+int tlq_debug_check_small_addressing(int kind, int64_t M, int64_t N, int64_t row_bytes, int64_t group, int rows, int cols, int waves, int extra_in_flight) {
+  return check_small(kind, M, N, row_bytes, group, rows / 16, cols / 16, waves, extra_in_flight);
 }
 
 }  // extern "C"

@@ -20,9 +20,10 @@ namespace tlq {
 template <SmallW W, int RT, int MT>
 struct SmallCfg {
   static constexpr int A_TILE = MT * 2048;
-  static constexpr int W_TILE = W == kSmallNK ? RT * 2048 : (W == kSmallW4 ? RT * 1024 : 8192);
-  static constexpr int SLOT = A_TILE + W_TILE;
-  static constexpr int D = SLOT <= 4096 ? 4 : (SLOT <= 8192 ? 3 : 2);  // steps in the ring
+  static constexpr int W_TILE = addr::small_w_tile(W, RT);
+  static constexpr int SLOT = addr::small_slot_bytes(W, RT, MT);
+  static constexpr int D = addr::small_depth(SLOT);  // steps in the ring
+  static_assert(SLOT == A_TILE + W_TILE, "the two parts of a slot");
   static constexpr int LDS = D * SLOT;                                  // per wavefront
   static constexpr int LOADS = SLOT / 1024;                             // direct loads per step
   static constexpr int MAX_WAVES = RT * MT <= 4 ? 16 : 8;
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(RT* MT <= 4 ? 1024 : 512) void gemm_small_kernel(Sm
   uint8_t* const mine = smem + wave * Cfg::LDS;
   const uint32_t mine_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)mine);
   const int n_base = blockIdx.x * (16 * RT), m_base = blockIdx.y * (16 * MT), batch = blockIdx.z;
-  const int s0 = (int)(((int64_t)wave * p.steps) / waves), s1 = (int)(((int64_t)(wave + 1) * p.steps) / waves);
+  const int s0 = addr::small_first(wave, waves, p.steps), s1 = addr::small_first(wave + 1, waves, p.steps);
   const int n_steps = s1 - s0;
   const uint8_t* const a_base = p.a + batch * p.a_batch;
   const uint8_t* const w_base = p.w + batch * p.w_batch;
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(RT* MT <= 4 ? 1024 : 512) void gemm_small_kernel(Sm
     if (d < n_steps) issue(s0 + d, d);
   int slot = 0;
   for (int i = 0; i < n_steps; ++i) {
-    const int younger = n_steps - 1 - i < D - 1 ? n_steps - 1 - i : D - 1;  // steps issued behind this one
+    const int younger = addr::small_younger(i, n_steps, D);  // steps issued behind this one
     if (D >= 4 && younger == 3)
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D >= 4 ? 3 * L : 0) : "memory");
     else if (D >= 3 && younger == 2)

@@ -6,10 +6,9 @@ namespace tlq {
 
 static thread_local int g_small_waves = 0, g_small_tiles = 0;  // tuning and tests: forced variant; tiles < 0: never
 
-static constexpr int small_slot(SmallW w, int rt, int mt) { return mt * 2048 + (w == kSmallNK ? rt * 2048 : (w == kSmallW4 ? rt * 1024 : 8192)); }
 static constexpr int small_lds(SmallW w, int rt, int mt) {
-  const int slot = small_slot(w, rt, mt);
-  return slot * (slot <= 4096 ? 4 : (slot <= 8192 ? 3 : 2));
+  const int slot = addr::small_slot_bytes(w, rt, mt);
+  return slot * addr::small_depth(slot);
 }
 
 // The estimate, in microseconds: a launch, rounds of the work-groups the machine holds at once (LDS and registers) x the longest chain

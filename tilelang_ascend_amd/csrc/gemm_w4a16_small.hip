@@ -35,7 +35,7 @@ struct SmallMma<bf16_t> {
   typedef MmaBF16 type;
 };
 
-constexpr int small_wave_lds(int rt, int mt) { return 2 * (rt * 1024 + mt * 4096) + 2 * (rt * 2 * 256); }
+constexpr int small_wave_lds(int rt, int mt) { return 2 * addr::smallw_slot_bytes(rt, mt) + 2 * addr::smallw_sc_bytes(rt); }
 constexpr int small_max_waves(int mt) { return mt == 1 ? 16 : 8; }
 
 template <typename T, bool FOLD, int LAYOUT, int RT, int MT>
@@ -45,8 +45,8 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
                                                                 float zero_scalar, int out_dtype) {
   typedef typename SmallMma<T>::type Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
-  constexpr int SLOT = RT * 1024 + MT * 4096;  // RT weight tiles + MT activation tiles
-  constexpr int SC = RT * 2 * 256;        // [rt][scale | zero][64 dwords]
+  constexpr int SLOT = addr::smallw_slot_bytes(RT, MT);  // RT weight tiles + MT activation tiles
+  constexpr int SC = addr::smallw_sc_bytes(RT);          // [rt][scale | zero][64 dwords]
   constexpr int WAVE_LDS = 2 * SLOT + 2 * SC;
   constexpr int NI = RT + 4 * MT;         // direct loads per k-block
   extern __shared__ __align__(16) uint8_t smem[];
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
   const int n_base = blockIdx.x * (16 * RT), m_base = blockIdx.y * (16 * MT);
   const int groups = K >> gshift;
   const int KB = K >> 7;
-  const int kb0 = (int)(((int64_t)wave * KB) / waves), kb1 = (int)(((int64_t)(wave + 1) * KB) / waves);
+  const int kb0 = addr::small_first(wave, waves, KB), kb1 = addr::small_first(wave + 1, waves, KB);
   const int nkb = kb1 - kb0;
   const bool has_s = scales != nullptr, has_z = zeros != nullptr;
   const int NS = RT * ((has_s ? 1 : 0) + (has_z ? 1 : 0));  // gathers per scale period (uniform)
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
   // ---- per-lane source offsets of the direct loads ----
   uint32_t voff_w[RT], voff_a[4 * MT], row_g[RT];
   {
-    const int rho = lane >> 2, piece = (lane & 3) ^ ((rho >> 1) & 3);  // lands on row lane/4, physical piece lane%4
+    const int rho = addr::sw_row(lane), piece = addr::sw_piece(lane);  // lands on row lane/4, physical piece lane%4
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       int n = n_base + rt * 16 + rho;
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
     }
   }
   // ---- per-lane LDS offsets of the fragment reads ----
-  const uint32_t fo_w = (uint32_t)(r16 * 64 + ((q ^ ((r16 >> 1) & 3)) << 4));
+  const uint32_t fo_w = addr::sw_frag_off(lane);
   uint32_t fo_a[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) fo_a[j] = (uint32_t)(RT * 1024) + addr::sa_frag_off(lane, 0, j);
@@ -106,12 +106,10 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
   };
   // four consecutive groups (base .. base+3) of the 16 rows of every tile: lane (row r16, group q)
   auto issue_sc = [&](int base, int buf) {
-    int g = base + q;
-    g = g < groups ? g : groups - 1;
     const uint32_t l0 = mine_lds + (uint32_t)(2 * SLOT + buf * SC);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      const uint64_t e2 = ((uint64_t)row_g[rt] + (uint64_t)g) * 2u;
+      const uint64_t e2 = addr::smallw_sc_elem(lane, base, row_g[rt], groups) * 2u;
       if (has_s) {
         const uint64_t a = ((uint64_t)(uintptr_t)scales + e2) & ~(uint64_t)3;
         asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(l0 + (rt * 2 + 0) * 256), "v"(a) : "memory");
@@ -122,9 +120,9 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
       }
     }
   };
-  auto sc_base = [&](int kb) { return ((kb << 7) >> gshift) & ~3; };
-  auto new_period = [&](int kb) { return NS > 0 && (kb == kb0 || sc_base(kb) != sc_base(kb - 1)); };
-  auto sc_buf = [&](int kb) { return (sc_base(kb) >> 2) & 1; };
+  auto sc_base = [&](int kb) { return addr::smallw_sc_base(kb, gshift); };
+  auto new_period = [&](int kb) { return NS > 0 && addr::smallw_new_period(kb, kb0, gshift); };
+  auto sc_buf = [&](int kb) { return addr::smallw_sc_buf(kb, gshift); };
 
   typename Mma::acc_t acc[RT][MT];
 #pragma unroll
@@ -164,9 +162,8 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
       const uint8_t* slot = mine + (i & 1) * SLOT;
       T sv[RT], zv[RT];
       {
-        const int g = ((kb << 7) + (q << 5)) >> gshift;
-        const int rel = g - sc_base(kb);
-        const uint8_t* sc = mine + 2 * SLOT + sc_buf(kb) * SC + (r16 + 16 * rel) * 4;
+        const int g = addr::smallw_group(lane, kb, gshift);
+        const uint8_t* sc = mine + 2 * SLOT + sc_buf(kb) * SC + addr::smallw_sc_cell(lane, kb, gshift) * 4;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           const uint32_t sh = (((uint32_t)row_g[rt] + (uint32_t)g) & 1u) * 16u;
