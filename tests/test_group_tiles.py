@@ -79,6 +79,11 @@ def test_taken_where_tiles_leave_one_work_group_to_a_cu(lib):
         C, dA, dW = torch.empty(M, N, dtype=torch.float16, device="cuda"), A.cuda(), W.cuda()
         lib.tlq_debug_launch_log(1)
         called(lib, lib.tlq_gemm_f16(P(dA), P(dW), P(C), M, N, K, _abi.F16, _abi.F16, _abi.B_KN, st), groups)
+    # (280 tiles of 128 x 128; 504 of 128 x 64 would be two rounds)
+    A, W = torch.randn(8, 780, 1024, generator=gen(1)).half().cuda(), torch.randn(8, 1024, 528, generator=gen(2)).half().cuda()
+    C = torch.empty(8, 780, 528, dtype=torch.float16, device="cuda")
+    lib.tlq_debug_launch_log(1)
+    called(lib, lib.tlq_gemm_f16_batched(P(A), P(W), P(C), 8, 780, 528, 1024, _abi.F16, _abi.F16, _abi.B_KN, st), False)
 
 
 @pytest.mark.gpu

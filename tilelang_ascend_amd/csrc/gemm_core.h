@@ -1010,13 +1010,17 @@ static constexpr TileCost kTileCost[4][6] = {
     {{2.4, 1.4, 1.10, 0.70}, {1.0, 4.0, 1.05, 0}, {2.1, 2.9, 0.84, 0}, {2.7, 2.2, 0.84, 0}, {3.0, 1.9, 1.06, 0}, {0.0, 5.3, 1.25, 0}},
     {{2.0, 3.4, 1.23, 0.72}, {0.4, 5.0, 1.10, 0}, {1.2, 3.6, 0.98, 0}, {1.7, 2.8, 0.90, 0}, {2.2, 2.0, 1.36, 0}, {0.0, 7.3, 1.32, 0}},
     {{0.3, 6.2, 1.02, 0.60}, {1.6, 4.8, 0.99, 0}, {3.4, 2.5, 0.81, 0}, {3.2, 2.8, 0.79, 0}, {3.9, 1.6, 1.05, 0}, {0.0, 8.8, 1.13, 0}}};
-inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int64_t N, int64_t stages) {  // variant 1, kGroup*, 6
-  static constexpr int kRows[6] = {128, 128, 128, 64, 64, 256}, kCols[6] = {128, 128, 64, 128, 64, 256}, kGroups[6] = {1, 2, 2, 2, 4, 1};
+inline int64_t tile_blocks(int variant, int64_t batch, int64_t M, int64_t N) {  // variant 1, kGroup*, 6
+  static constexpr int kRows[6] = {128, 128, 128, 64, 64, 256}, kCols[6] = {128, 128, 64, 128, 64, 256};
+  return batch * ceil_div(M, (int64_t)kRows[variant - 1]) * ceil_div(N, (int64_t)kCols[variant - 1]);
+}
+inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int64_t N, int64_t stages) {
+  static constexpr int kGroups[6] = {1, 2, 2, 2, 4, 1};
   const int v = variant - 1;
   int cus = tlq_device_cu_count();
   if (cus <= 0) cus = 256;
   const TileCost& c = kTileCost[kind][v];
-  const int64_t blocks = batch * ceil_div(M, (int64_t)kRows[v]) * ceil_div(N, (int64_t)kCols[v]);
+  const int64_t blocks = tile_blocks(variant, batch, M, N);
   const double run = c.fixed + c.step * (double)ceil_div(stages, (int64_t)kGroups[v]);
   const int64_t rounds = blocks / (2 * cus), rest = blocks % (2 * cus);  // two plain 128 x 128 work-groups share a CU
   const double us = variant != 1 ? run * (double)ceil_div(blocks, (int64_t)cus)
@@ -1027,15 +1031,22 @@ inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int6
   const double floor_us = memory > product ? memory : product;
   return c.launch + (us > floor_us ? us : floor_us);
 }
-// The variant for a problem that would run 128 x 128 tiles: 0 = those, or one of kGroup*, where its estimate is clearly below.
+// The variant for a problem that would run 128 x 128 tiles: 0 = those, or one of kGroup*, where its work-groups run in one round (they
+// have a CU each) and its estimate is clearly below.  On 4800 problems (1200 per operand layout, ranges as above, up to 1100 tiles of
+// 128 x 128) with every variant forced on each: taken on 2725, 1.26 - 1.39 x over the plain tiles on average over all, more than 5 % behind on
+// one (0.89).  Without the bound of one round 71 were, 0.64 at worst (fp16 8 x 780 x 528 x 10752 234 us in two rounds of
+// 128 x 64 tiles, 160 in plain ones): the estimates miss what two work-groups of the plain kernel on a CU give each other.
 inline int group_tile(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes, double* us = nullptr) {
   const int64_t stages = ceil_div(k_bytes, (int64_t)kStageBytes);
   if (g_gemm_groups > 1) return stages >= 4 ? g_gemm_groups : 0;
   int best = 0;
   double best_us = tile_us(kind, 1, batch, M, N, stages);
   if (g_gemm_groups == 0 && stages >= 4 && M >= 64) {  // (fewer rows were not measured)
+    int cus = tlq_device_cu_count();
+    if (cus <= 0) cus = 256;
     double bar = best_us * 0.94;
     for (int v = kGroup128x128; v <= kGroup64x64; ++v) {
+      if (tile_blocks(v, batch, M, N) > cus) continue;
       const double t = tile_us(kind, v, batch, M, N, stages);
       if (t < bar) best = v, best_us = bar = t;
     }
