@@ -131,3 +131,47 @@ def test_no_register_spills(tmp_path):
     assert len(blocks) == 39
     for b in blocks:
         assert re.search(r"ScratchSize \[bytes/lane\]: 0\b", b) and re.search(r"VGPRs Spill: 0\b", b), b[:300]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what,B,M,N,K,small", [
+    # where it measured ahead of what runs without it ...
+    ("w4a8", 1, 57, 1024, 3840, True), ("w4a8", 1, 128, 4096, 11008, True), ("i8 NK", 1, 257, 1232, 8576, True), ("w8a8 NK", 1, 32, 4096, 14336, True),
+    ("f16", 4, 34, 256, 5376, True),
+    # ... and behind: K over groups of wavefronts, few rows in K slices, [K, N] weights of many columns
+    ("i8 NK", 8, 1009, 160, 3456, False), ("w4a8", 1, 1374, 1184, 5376, False), ("f16", 3, 231, 1376, 8576, False), ("i8 KN", 1, 14, 704, 5760, False),
+    ("w8a8 KN", 1, 89, 11440, 6528, False)])
+def test_choice_against_the_larger_tiles(lib, what, B, M, N, K, small):
+    """With the workspace that the entry points ask for, on a machine of 256 CUs."""
+    P, st = _abi.ptr, torch.cuda.current_stream().cuda_stream
+    print(f"choice {what} B={B} M={M} N={N} K={K}", flush=True)
+    nk = what.endswith("NK")
+    if what == "f16":
+        A, W = torch.randn(B, M, K, generator=gen(1)).half().cuda(), torch.randn(B, K, N, generator=gen(2)).half().cuda()
+    else:
+        A, W = i8(1, B, M, K).cuda(), (torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=gen(2)) if what == "w4a8" else i8(2, B, *((N, K) if nk else (K, N)))).cuda()
+    C = torch.empty(B, M, N, dtype=torch.float16 if what == "f16" else torch.float32 if what.startswith("w8a8") else torch.int32, device="cuda")
+    need = {"w8a8": lib.tlq_w8a8_workspace_bytes(B, M, N, K), "w4a8": N * K, "f16": lib.tlq_f16_workspace_bytes(B, M, N, K)}.get(what.split()[0], 0)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    layout = _abi.B_NK if nk else _abi.B_KN
+    lib.tlq_debug_launch_log(1)
+    if what == "w4a8":
+        rc = lib.tlq_gemm_w4a8_ws(P(A), P(W), P(ws), need, P(C), M, N, K, _abi.U4, st)
+    elif what == "f16":
+        rc = lib.tlq_gemm_f16_ws(P(A), P(W), P(C), P(ws), need, B, M, N, K, _abi.F16, _abi.F16, layout, st)
+    elif what.startswith("w8a8"):
+        rc = lib.tlq_gemm_w8a8_ws(P(A), P(W), None, None, P(C), P(ws), need, B, M, N, K, 1, layout, _abi.F32, st)
+    else:
+        rc = lib.tlq_gemm_i8(P(A), P(W), P(C), B, M, N, K, layout, st)
+    log = lib.tlq_debug_launch_log_text().decode()
+    lib.tlq_debug_launch_log(0)
+    _abi.check(rc)
+    torch.cuda.synchronize()
+    assert ("gemm_small_kernel" in log) == small or lib.tlq_device_cu_count() != 256, log
+    if what == "w4a8":
+        W = torch.stack([W & 15, W >> 4], -1).reshape(1, N, K)
+    want = torch.bmm(A.double(), W.double().transpose(1, 2).contiguous() if nk or what == "w4a8" else W.double())
+    if what == "f16":
+        assert bool(((C.double() - want).abs() <= 2.0**-11 * want.abs() + K * 2.0**-24 * torch.bmm(A.double().abs(), W.double().abs()) * 1.001 + 2.0**-25).all())
+    else:
+        assert torch.equal(C.double(), want.float().double())

@@ -1276,32 +1276,66 @@ static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, in
   // against 56 us in groups, 947 x 1664 x 6016 36 against 43, 7795 x 256 x 7808 54 against 78)
   return k_bytes <= 48 * kStageBytes && group_tile_us(tile, 1, M, N, k_bytes) < 0.9 * sliced_us(kind, 1, M, N, K);
 }
-// Is the small-tile kernel's estimate below what the kernels with 128-wide tiles take?  Theirs were fitted to the same 970 problems, apart
-// for the calls that cut K into slices (sliced_us) and those that do not
-// (16-bit and W4A8: 10 and 6 us per thousand of K whatever M and N); 7 - 17 % rms.  With these bars it is ahead by 1.1 - 1.5 x on average on what it
-// takes and lost more than 5 % on 20 of the 970, 27 % at most.
-static bool small_tile_wins(const SmallTile& t, int kind, int64_t batch, int64_t M, int64_t N, int64_t K) {
+// The products that may take the small-tile kernel: weights as stored (the first four: SmallW), int32 results, or rescaled ones
+// (W8A8), W4A8 where the caller brought the room to unpack the weights first.
+enum SmallUse { kUseI8NK = kSmallNK, kUseI8KN = kSmallKN8, kUseF16KN = kSmallKN16, kUseW4A8 = kSmallW4, kUseW4A8TwoSteps = 4, kUseW8A8NK = 5, kUseW8A8KN = 6 };
+static SmallW small_weights(SmallUse use) { return use == kUseW8A8NK ? kSmallNK : use == kUseW8A8KN ? kSmallKN8 : use == kUseW4A8TwoSteps ? kSmallW4 : (SmallW)use; }
+// Is the small-tile kernel ahead of what would run in its place?  Two things its own estimate leaves out come on top: the activations' trip from
+// memory (at 2.5 TB/s: every tile of weight rows asks for them again) and, with 16-bit weights, that theirs cannot take less than
+// a copy.  The other side, by what would run: calls that cut K into slices over work-groups (sliced_us), up to 32 rows a fit to the 32-row
+// tiles, else the tiles' own estimates -- plain, with K over groups of wavefronts, 256 x 256 --, for W4A8 in two steps behind the
+// unpack pass.  The bars are fitted to problems (M 1 .. 8192, N 64 .. 14400, K 128 .. 14336, one to eight batches) timed with the
+// small-tile kernel, without it and by the choice.  On 9000 others, 1500 per use, it is taken on 5206, ahead by 1.40 - 1.80 x on average
+// and more than 5 % behind on 135 (81 by more than 10 %); the choice is 0.4 - 1.6 % behind the faster of both on average.  (The rule
+// before, without the two additions and with bars of 0.88 - 1.15 of a fit to the plain tiles: 428 of 4693, 2 - 8 % --
+// 8 x 1009 x 160 x 3456 int8 35.8 us against 15.0, W4A8 1374 x 1184 x 5376 47.8 against 28.1.)
+struct SmallBars {
+  double few_sliced, sliced, few, plain, groups;
+};
+static constexpr SmallBars kSmallBars[7] = {
+    // <= 32 rows, K slices   K slices   <= 32 rows   tiles   tiles with K in groups
+    {0.84, 1.5, 1.15, 1.03, 0.92},  // int8 [N, K]
+    {0.74, 1.05, 1.05, 1.0, 1.0},   // int8 [K, N]
+    {0.8, 1.04, 1.02, 1.0, 1.0},    // 16-bit [K, N]
+    {1.04, 1.0, 0.93, 0.93, 0.93},  // W4A8
+    {1.04, 1.0, 0.93, 1.0, 1.0},    // W4A8 in two steps
+    {0.84, 0.95, 1.12, 0.9, 0.88},  // W8A8 [N, K]
+    {0.74, 0.9, 1.0, 0.88, 0.92}};  // W8A8 [K, N]
+static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int64_t M, int64_t N, int64_t K) {
   if (!t.ok || small_tile_forced()) return t.ok;
+  const SmallW w = small_weights(use);
+  const SmallBars& bar = kSmallBars[use];
   const double g = (double)batch * (double)M * (double)N * (double)K * 1e-9, g32 = (double)batch * (double)ceil_div(M, (int64_t)32) * 32.0 * (double)N * (double)K * 1e-9;
   const double nk = (double)batch * (double)N * (double)K * 1e-6, mn = (double)batch * (double)M * (double)N * 1e-6, k = (double)K * 1e-3;
-  const double tiles_k = (double)batch * (double)ceil_div(M, (int64_t)128) * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6;
-  auto sliced = [&](double pace) { return batch == 1 && slice_choice(M, N, K, true, pace, 0) > 1; };
-  switch (kind) {
-    case 0: return t.us < 0.92 * (sliced(1.0) ? sliced_us(0, batch, M, N, K) : 5.1 + 1.4 * g + 0.16 * mn + 2.07 * k) && t.us < 1.15 * group_tile_us(kTileI8NK, batch, M, N, K);
-    case 1: return t.us < 0.88 * (sliced(1.0) ? sliced_us(1, batch, M, N, K) : 4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32) &&
-                   t.us < 1.15 * group_tile_us(kTileI8KN, batch, M, N, K);
-    case 2: return t.us < 0.9 * (batch == 1 && slice_choice(M, N, K * 2, true, 1.0, 0) > 1 ? sliced_us(2, batch, M, N, K) : 3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * tiles_k) &&
-                   t.us < 1.15 * group_tile_us(kTileF16KN, batch, M, N, K * 2);
-    default: return t.us < 0.95 * (M <= 256 && sliced(2.5) ? sliced_us(3, batch, M, N, K) : 4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
-  }
+  const int64_t k_bytes = w == kSmallKN16 ? 2 * K : K, stages = ceil_div(k_bytes, (int64_t)kStageBytes);
+  double us = t.us + (double)batch * (double)M * (double)k_bytes / 2.5e6;
+  if (w == kSmallKN16 && us < 1.05 * nk * 2.0 / 5.0) us = 1.05 * nk * 2.0 / 5.0;
+  const bool packed = w == kSmallW4;
+  const TileKind tile = w == kSmallKN16 ? kTileF16KN : w == kSmallKN8 ? kTileI8KN : kTileI8NK;
+  const bool adds = use == kUseI8NK || use == kUseI8KN;  // (their slices add into the result itself)
+  if (packed ? M <= 256 && slice_choice(M, N, k_bytes, true, 2.5, 0) > 1
+             : batch == 1 && slice_choice(M, N, k_bytes, !adds, 1.0, 0) > 1 && !groups_beat_slices(tile, w, M, N, K, k_bytes))
+    return us < (M <= 32 ? bar.few_sliced : bar.sliced) * sliced_us(w, batch, M, N, K);
+  if (packed && use != kUseW4A8TwoSteps) return us < bar.few * (4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
+  if (M <= 32 && w == kSmallNK) return us < bar.few * (5.1 + 1.4 * g + 0.16 * mn + 2.07 * k);
+  if (M <= 32 && w == kSmallKN8) return us < bar.few * (4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32);
+  if (M <= 32 && w == kSmallKN16) return us < bar.few * (3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * (double)batch * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6);
+  const double unpack_us = packed ? 2.6 + nk * 1.5 / 4.5 : 0.0;
+  if (packed && i8_split_choice(1, M, N, K, false) > 1 && !groups_beat_slices(kTileI8NK, 0, M, N, K, K))
+    return us < bar.sliced * (unpack_us + 2.0 * sliced_us(0, 1, M, N, K));  // (slices that add into the result take twice those with matrices of their own)
+  if (!prefer_small_tiles(batch, M, N)) return us < bar.plain * (unpack_us + tile_us(tile, 6, batch, M, N, stages));
+  double tiles_us = 0.0;
+  const bool groups = group_tile(tile, batch, M, N, k_bytes, &tiles_us) != 0;
+  if (groups && us < 5.6 && us < 1.1 * (unpack_us + tiles_us)) return true;  // (no more than a launch: nothing to lose)
+  return us < (groups ? bar.groups : bar.plain) * (unpack_us + tiles_us);
 }
-static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t K, int kind) {
+static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t K, SmallUse use) {
   const SmallTile t{false, 0, 0, 0, 0.0};
   if (batch < 1 || M < 1 || N < 1 || K < 128 || K % 128 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_i8_tile || g_i8_split) return t;
   static thread_local PlanTable<SmallTile> known;
-  return known.get(M, N, K, kind + 4 * batch, [&] {
-    SmallTile p = small_tile_plan(kind, batch, M, N, K);
-    p.ok = small_tile_wins(p, kind, batch, M, N, K);
+  return known.get(M, N, K, use + 8 * batch, [&] {
+    SmallTile p = small_tile_plan(small_weights(use), batch, M, N, K);
+    p.ok = small_tile_wins(p, use, batch, M, N, K);
     return p;
   });
 }
@@ -1312,7 +1346,7 @@ static SmallTile small_tile_for_f16(int64_t batch, int64_t M, int64_t N, int64_t
   static thread_local PlanTable<SmallTile> known;
   return known.get(M, N, K, batch, [&] {
     SmallTile p = small_tile_plan(2, batch, M, N, K * 2);
-    p.ok = small_tile_wins(p, 2, batch, M, N, K);
+    p.ok = small_tile_wins(p, kUseF16KN, batch, M, N, K);
     return p;
   });
 }
@@ -1336,7 +1370,7 @@ static int64_t rows_of_full_rounds(TileKind kind, int64_t M, int64_t N, int64_t 
     auto rest_us = [&](int64_t rows) {
       const double us = one_us(rows);
       if (kind == kTileF16NK) return us;
-      const SmallTile t = i8 ? small_tile_for_i8(1, rows, N, K, kind == kTileI8NK ? 0 : 1) : small_tile_for_f16(1, rows, N, K, TLQ_B_KN);
+      const SmallTile t = i8 ? small_tile_for_i8(1, rows, N, K, kind == kTileI8NK ? kUseI8NK : kUseI8KN) : small_tile_for_f16(1, rows, N, K, TLQ_B_KN);
       return t.ok && t.us < us ? t.us : us;
     };
     double best = 0.87 * one_us(M);
@@ -1443,7 +1477,7 @@ int tlq_gemm_i8(const void* A, const void* B, void* C, int64_t batch, int64_t M,
   TLQ_REQUIRE(A && B && C, "tlq_gemm_i8: null pointer");
   TLQ_REQUIRE(aligned16(A) && aligned16(B) && aligned16(C), "tlq_gemm_i8: pointers must be 16-byte aligned");
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K), "tlq_gemm_i8: a matrix spans 4 GiB or more");
-  if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1); t.ok) return small_i8(t, A, B, C, batch, M, N, K, b_layout, (hipStream_t)stream);
+  if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? kUseI8NK : kUseI8KN); t.ok) return small_i8(t, A, B, C, batch, M, N, K, b_layout, (hipStream_t)stream);
   // few activation rows: K slices add into C itself (int32, exact in any order)
   if (const int split = i8_split_choice(batch, M, N, K, false);
       split > 1 && (g_i8_split || !groups_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
@@ -1465,7 +1499,7 @@ int tlq_gemm_w4a8(const void* A, const void* w_packed, void* C, int64_t M, int64
   TLQ_REQUIRE(A && w_packed && C, "tlq_gemm_w4a8: null pointer");
   TLQ_REQUIRE(aligned16(A) && aligned16(w_packed) && aligned16(C), "tlq_gemm_w4a8: pointers must be 16-byte aligned");
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K / 2), "tlq_gemm_w4a8: a matrix spans 4 GiB or more");
-  if (const SmallTile t = small_tile_for_i8(1, M, N, K, 3); t.ok) return small_w4a8(t, A, w_packed, C, M, N, K, sign_mode, (hipStream_t)stream);
+  if (const SmallTile t = small_tile_for_i8(1, M, N, K, kUseW4A8); t.ok) return small_w4a8(t, A, w_packed, C, M, N, K, sign_mode, (hipStream_t)stream);
   // few activation rows: K slices add into C (int32, exact in any order)
   if (const int split = i8_split_choice(1, M, N, K, false, 2.5); split > 1)
     return gemm_w4a8_i32_splitk(A, w_packed, C, M, N, K, sign_mode, split, nullptr, (hipStream_t)stream);
@@ -1480,9 +1514,12 @@ int tlq_gemm_w4a8_ws(const void* A, const void* w_packed, void* workspace, int64
   // steps -- unpack into the workspace, int8 GEMM on it -- each at its own roofline (M = N = K = 4096: 6 + 66 us against
   // 98 us fused; M = 1024: 37 against 65 us).  Few rows (the unpack pass would cost more than the GEMM): the kernel that
   // unpacks on the way into LDS over K slices, the workspace holding one int32 [M, N] matrix per slice.
-  if (g_w4a8_ws_mode == 0 && small_tile_for_i8(1, M, N, K, 3).ok) return tlq_gemm_w4a8(A, w_packed, C, M, N, K, sign_mode, stream);
   const bool usable = workspace != nullptr && aligned16(workspace) && N > 0 && K > 0 && M > 0 && M < kMaxDim && N < kMaxDim &&
                       K < kMaxDim && fits32(N, K / 2) && fits32(M, K);
+  const bool two_steps = usable && workspace_bytes >= N * K && K % 16 == 0 && N % 16 == 0 && fits32(N, K) &&
+                         (M > 64 || g_w4a8_ws_mode == 2);
+  if (g_w4a8_ws_mode == 0 && small_tile_for_i8(1, M, N, K, two_steps ? kUseW4A8TwoSteps : kUseW4A8).ok)
+    return tlq_gemm_w4a8(A, w_packed, C, M, N, K, sign_mode, stream);
   if (usable && K % 32 == 0 && N % 4 == 0 && g_w4a8_ws_mode != 2 && (M <= 256 || g_w4a8_ws_mode == 1)) {
     int split = i8_split_choice(1, M, N, K, true, 2.5);
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;
@@ -1493,8 +1530,6 @@ int tlq_gemm_w4a8_ws(const void* A, const void* w_packed, void* workspace, int64
       return gemm_w4a8_i32_splitk(A, w_packed, C, M, N, K, sign_mode, split, (int32_t*)workspace, (hipStream_t)stream);
     }
   }
-  const bool two_steps = usable && workspace_bytes >= N * K && K % 16 == 0 && N % 16 == 0 && fits32(N, K) &&
-                         (M > 64 || g_w4a8_ws_mode == 2);
   if (!two_steps) return tlq_gemm_w4a8(A, w_packed, C, M, N, K, sign_mode, stream);
   TLQ_REQUIRE(sign_mode >= TLQ_U4 && sign_mode <= TLQ_S4_OFFSET7, "tlq_gemm_w4a8_ws: bad sign_mode %d", sign_mode);
   TLQ_REQUIRE(A && w_packed && C && aligned16(w_packed), "tlq_gemm_w4a8_ws: null or misaligned pointer");
@@ -1520,7 +1555,7 @@ int tlq_gemm_w8a8(const void* A, const void* B, const void* scale_a, const void*
   TLQ_REQUIRE(aligned16(A) && aligned16(B) && aligned16(C), "tlq_gemm_w8a8: pointers must be 16-byte aligned");
   TLQ_REQUIRE(((uintptr_t)scale_a & 3) == 0 && ((uintptr_t)scale_b & 3) == 0, "tlq_gemm_w8a8: scales misaligned");
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K), "tlq_gemm_w8a8: a matrix spans 4 GiB or more");
-  if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1); t.ok)
+  if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? kUseW8A8NK : kUseW8A8KN); t.ok)
     return small_w8a8(t, A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype, (hipStream_t)stream);
   if (const int64_t head = batch == 1 ? rows_of_full_rounds(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, M, N, K) : 0; head > 0) {
     if (const int rc = tlq_gemm_w8a8(A, B, scale_a, scale_b, C, 1, head, N, K, n_scale_b, b_layout, out_dtype, stream)) return rc;
@@ -1552,7 +1587,7 @@ int tlq_gemm_w8a8_ws(const void* A, const void* B, const void* scale_a, const vo
     split = i8_split_choice(batch, M, N, K, true);
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;  // as many slices as the workspace holds
   }
-  if (split <= 1 || small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? 0 : 1).ok ||
+  if (split <= 1 || small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? kUseW8A8NK : kUseW8A8KN).ok ||
       (!g_i8_split && groups_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
     return tlq_gemm_w8a8(A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype, stream);
   TLQ_REQUIRE(b_layout == TLQ_B_KN || b_layout == TLQ_B_NK, "tlq_gemm_w8a8_ws: bad b_layout %d", b_layout);
