@@ -254,32 +254,42 @@ static bool skinny_leaves_cus_idle(int64_t N) {
   const int64_t wgs = ceil_div(N, (int64_t)16), places = 2 * cu_count_or_default();
   return wgs > places / 2 && (double)wgs / (double)(ceil_div(wgs, places) * places) < 0.8;
 }
-// Where the small-tile kernel (gemm_w4a16_small.hip: one launch, wavefronts split K) is ahead of a family by estimate.  The
-// families' own times were fitted to the same 520 problems (10 - 11 % rms each; G: billions of products, G16: the same with M rounded up
-// to 16 rows); with these bars it never lost more than 5 % to the family it replaces and won 1.43 x on average over the
-// streaming kernel's share of them, 1.47 x over the two passes'.
+// Where the small-tile kernel (gemm_w4a16_small.hip: one launch, wavefronts split K) is ahead of a family by estimate (G: billions of
+// products, G16: the same with M rounded up to 16 rows).  The plan's estimate leaves out the activations' trip from memory and the store
+// of the result (fitted: 1.6 and 3.2 times what they take at 5 TB/s; 11 % rms on 2700 problems with them, 0.23 too low on average
+// and 17 % above 512 rows without).  Against the kernels it replaces, on 3500 problems (M 2 .. 8192, N 128 .. 14400, K 128 .. 14336,
+// groups of 32 - 256, both types) not used for the fit: taken on 1944, ahead by 1.6 x on average up to 700 rows and by 1.8 x
+// above 500, more than 5 % behind on 27 and 19 % at most (without the two terms 131 of 2138, 2.7 x at most: 6980 x 912 x 128 22.2 us
+// against 8.2 in the tile kernel).
 static double giga(double m, int64_t N, int64_t K) { return m * (double)N * (double)K * 1e-9; }
 static double up16(int64_t M) { return (double)ceil_div(M, (int64_t)16) * 16.0; }
-static bool small_beats_stream(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
-  return p.ok && g_stream_slice_steps <= 0 && p.us < 0.95 * (11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K);
+static double small_us(const SmallTile& p, int64_t M, int64_t N, int64_t K) { return p.us + 0.64e-6 * (double)M * (double)K + 1.28e-6 * (double)M * (double)N; }
+static double fused_tile_us(int64_t M, int64_t N, int64_t K) {  // the W4A16 tile kernel where it has few tiles: 4 us + 1.5 us per 128 values of K
+  return 3.9 + 11.6e-3 * (double)K + 0.94 * giga((double)M, N, K) + 0.116e-6 * (double)M * (double)N;
 }
-// above 512 rows (the two passes, or the panel kernels with their head and tail): only while the whole call stays short
-static bool small_beats_panels(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
-  return p.ok && p.us < 13.0 && p.us < 0.9 * (14.9 + 3.6 * giga(up16(M), N, K) + 0.79e-3 * (double)K);
+static bool small_beats_stream(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
+  return p.ok && g_stream_slice_steps <= 0 && small_us(p, M, N, K) < 0.99 * (11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K);
+}
+// above 512 rows: the tile kernel on up to 2^19 weights -- and the launch for the last M % 4 rows, 4 us, where they run apart --, else the
+// two passes or the panel kernels, which are level with them or ahead; only while the whole call stays short
+static double two_passes_us(int64_t M, int64_t N, int64_t K);
+static bool small_beats_panels(const SmallTile& p, int64_t M, int64_t N, int64_t K, bool head_and_tail) {
+  if (!p.ok || p.us >= 13.0) return false;
+  const double us = small_us(p, M, N, K);
+  return us < (N * K <= ((int64_t)1 << 19) ? 0.95 * (fused_tile_us(M, N, K) + (head_and_tail ? 4.0 : 0.0)) : 0.95 * two_passes_us(M, N, K));
 }
 // the decode kernel over chunks of K, whose second launch adds the chunks
 static bool small_beats_decode_chunks(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
   return p.ok && p.us < 0.95 * (5.2 + 0.67 * giga((double)M, N, K) + 4.36 * giga(up16(M), N, K) + 0.023e-6 * (double)N * (double)K + 0.25e-3 * (double)K);
 }
 // The skinny kernel on 17 .. 64 rows (12.8 -> 7.8 us for M = 64 on 5120 x 1280, level where the launch is all there is) and the tile
-// kernel (4 us + 1.5 us per 128 values of K whatever M and N: 21.5 -> 5.9 us for 116 rows on 368 x 1280, 256 x 256 x 256 6.8 -> 5.4 us):
-// the family the automatic choice runs in their place.
+// kernel (21.5 -> 5.9 us for 116 rows on 368 x 1280, 256 x 256 x 256 6.8 -> 5.4 us): the family the automatic choice runs in their place.
 static int small_or(int algo, int64_t M, int64_t N, int64_t K, int64_t group, const void* scales, const void* zeros) {
   if (algo == TLQ_ALGO_SKINNY ? M <= 16 || w4a16_skinny_forced() : algo != TLQ_ALGO_MFMA || N % 4 != 0 || w4a16_tile_forced()) return algo;
   const SmallTile p = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
   const double theirs = algo == TLQ_ALGO_SKINNY ? 0.95 * (5.2 + 7.0 * giga((double)M, N, K) + 4.1 * giga(up16(M), N, K) + 0.3e-3 * (double)K)
-                                                : 0.9 * (3.9 + 11.6e-3 * (double)K + 0.94 * giga((double)M, N, K) + 0.116e-6 * (double)M * (double)N);
-  return p.ok && p.us < theirs ? TLQ_ALGO_SMALL : algo;
+                                                : 0.95 * fused_tile_us(M, N, K);
+  return p.ok && (algo == TLQ_ALGO_SKINNY ? p.us : small_us(p, M, N, K)) < theirs ? TLQ_ALGO_SMALL : algo;
 }
 static bool decode_preferred(int64_t M, int64_t N, int64_t K) { return M > 2 || (M == 2 && N * K >= ((int64_t)1 << 24)); }
 
@@ -629,12 +639,12 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 // one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  On 61 problems above
 // 512 rows the bar below takes the two passes on 22, none slower; a bar of one would have lost 2 - 5 % on three more.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
+static double two_passes_us(int64_t M, int64_t N, int64_t K) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(M, N, K); }
 static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
   const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
   const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
   const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
   if (!p2.ok || N % 8 != 0) return false;
-  auto two_us = [&](int64_t rows) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(rows, N, K); };
   double panels;
   const bool middle = pm.ok && panelm_estimate_wins(head, N, K, group);
   if (middle && N > 512) return false;  // (against the middle-M kernel and its tail measured on up to 512 weight rows, one or two of its tiles)
@@ -643,8 +653,8 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
   else if (panel256_fills(head, N, K, group))
     panels = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, head, N, cus_now);
   else
-    panels = two_us(head);  // they would not run
-  return 1.1 * two_us(M) < 0.85 * (panels + (head != M ? 5.5 : 0.0));
+    panels = two_passes_us(head, N, K);  // they would not run
+  return 1.1 * two_passes_us(M, N, K) < 0.85 * (panels + (head != M ? 5.5 : 0.0));
 }
 
 // The panel kernel (large M, one launch, weights dequantised on the operand read).  Returns -1 when it does not take the
@@ -827,7 +837,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
       (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
     const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
-    if (small_beats_panels(small, M, N, K))
+    if (small_beats_panels(small, M, N, K, head_and_tail))
       return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                               (hipStream_t)stream);
   }
