@@ -636,8 +636,10 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 // Above 512 rows: do the two passes beat what the panel kernels would run?  The dequantisation pass costs 3 us and the weights' bytes, the
 // plain GEMM behind it has smaller tiles, K in groups of wavefronts and any row count, while the panel kernels have 8 us per round of
 // work-groups (many rounds of short rows: 4868 x 3152 x 384 bf16 36.9 -> 25.5 us, 6631 x 4608 x 256 38.7 -> 29.8) and leave
-// one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  On 61 problems above
-// 512 rows the bar below takes the two passes on 22, none slower; a bar of one would have lost 2 - 5 % on three more.
+// one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  On 1500 problems
+// (M 513 .. 8192, N 128 .. 14400, K 256 .. 19200, half of the row counts odd) the bar below takes the two passes on 278, ahead by 1.15 - 1.32 x
+// on average, more than 3 % behind on five (12 % at most), on 1500 others 277 and three (4 %); a bar of 0.9 for 0.85 takes 453, 48 of them behind.  The estimates of both
+// panel kernels are 13 - 19 % high there (11 % rms), that of the two passes 4 % (16 - 23 %), which the bar takes in.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
 static double two_passes_us(int64_t M, int64_t N, int64_t K) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(M, N, K); }
 static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
@@ -647,7 +649,6 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
   if (!p2.ok || N % 8 != 0) return false;
   double panels;
   const bool middle = pm.ok && panelm_estimate_wins(head, N, K, group);
-  if (middle && N > 512) return false;  // (against the middle-M kernel and its tail measured on up to 512 weight rows, one or two of its tiles)
   if (middle)
     panels = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, head, N, cus_now);
   else if (panel256_fills(head, N, K, group))
