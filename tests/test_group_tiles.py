@@ -87,10 +87,10 @@ def test_taken_where_tiles_leave_one_work_group_to_a_cu(lib):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,launches", [(4099, 4096, 1024, 2), (4096, 4096, 1024, 1)])
+@pytest.mark.parametrize("M,N,K,launches", [(4099, 4096, 1024, 2), (4096, 4096, 1024, 1), (7314, 2384, 384, 1), (7314, 2384, 768, 2)])
 def test_rows_of_full_rounds_and_the_rest(lib, M, N, K, launches):
     """One tile row too many for a round of the machine: the rest of the rows is a launch of its own (checked on a machine of 256 CUs), at the
-    right rows of the activations, the scales and the result."""
+    right rows of the activations, the scales and the result.  Not on rows of fewer than six 128-byte stages, where it is behind one launch."""
     print(f"full rounds M={M} N={N} K={K}", flush=True)
     P, st = _abi.ptr, torch.cuda.current_stream().cuda_stream
     A = torch.randint(-127, 128, (M, K), dtype=torch.int8, generator=gen(1)).cuda()

@@ -1365,13 +1365,17 @@ static SmallTile small_tile_for_f16(int64_t batch, int64_t M, int64_t N, int64_t
 // A product whose last round of work-groups is nearly empty runs as two launches: the rows of the tiles that fill whole rounds, then
 // the rest by whatever is best for that many rows.  Returns the rows of the first, 0 = one launch.  (4099 rows on 4096 x 4096 int8 are 17 x 16
 // tiles of 256 x 256, a round of 256 and one of 16; one launch took 128 x 128 tiles instead, 96 us; 4096 rows and 3 take
-// 62 us.)
+// 62 us.)  Not on rows of fewer than six 128-byte stages, where a launch more is a larger part than the 1.5 us below: 300 random problems
+// that two launches were estimated to win ran, against one, 0.93 as fast on rows of one to three stages (25 of 33 more than 3 % behind;
+// int8 7314 x 2384 x 384 26.7 us for 22.6), 1.01 on four or five (8 of 30 behind), 1.06 on six or seven (1 of 14), 1.1 on eight to
+// fifteen (2 of 55) and 1.2 beyond (none of 168).
 static int64_t rows_of_full_rounds(TileKind kind, int64_t M, int64_t N, int64_t K) {
   if (M <= 512 || N < 256 || K % 128 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_gemm_groups || g_gemm_f16_tile || g_i8_tile || g_gemm_slots == 2) return 0;
   static thread_local PlanTable<int64_t> known;
   return known.get(M, N, K, kind, [&]() -> int64_t {
     const bool i8 = kind >= kTileI8KN;
     const int64_t k_bytes = i8 ? K : 2 * K, stages = k_bytes / kStageBytes, cus = cu_count_or_default();
+    if (stages < 6) return 0;
     auto one_us = [&](int64_t rows) {
       double us = 0.0;
       if (!prefer_small_tiles(1, rows, N)) return tile_us(kind, 6, 1, rows, N, stages);
