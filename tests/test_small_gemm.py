@@ -175,3 +175,18 @@ def test_choice_against_the_larger_tiles(lib, what, B, M, N, K, small):
         assert bool(((C.double() - want).abs() <= 2.0**-11 * want.abs() + K * 2.0**-24 * torch.bmm(A.double().abs(), W.double().abs()) * 1.001 + 2.0**-25).all())
     else:
         assert torch.equal(C.double(), want.float().double())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,unpacked", [(257, 512, 512, True), (300, 1040, 512, True), (600, 256, 1024, True), (256, 512, 512, False)])
+def test_w4a8_above_256_rows_leaves_the_unpacked_weights_in_the_workspace(lib, M, N, K, unpacked):
+    """What tlq.h says of a workspace that holds the int8 [N, K] matrix, also on problems that the small-tile kernel would win."""
+    print(f"w4a8 workspace M={M} N={N} K={K}", flush=True)
+    P, st = _abi.ptr, torch.cuda.current_stream().cuda_stream
+    A, Wp = i8(1, M, K), torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=gen(2))
+    u = torch.stack([Wp & 15, Wp >> 4], -1).reshape(N, K).to(torch.int8)
+    W = torch.where(u >= 8, u - 16, u)
+    dA, dW, ws, C = A.cuda(), Wp.cuda(), torch.full((N, K), 99, dtype=torch.int8, device="cuda"), torch.full((M, N), -1, dtype=torch.int32, device="cuda")
+    _abi.check(lib.tlq_gemm_w4a8_ws(P(dA), P(dW), P(ws), N * K, P(C), M, N, K, _abi.S4_TWOS, st))
+    assert torch.equal(C.cpu(), (A.double() @ W.double().T).to(torch.int32))  # exact
+    assert torch.equal(ws.cpu(), W) == unpacked

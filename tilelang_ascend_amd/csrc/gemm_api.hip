@@ -1533,7 +1533,8 @@ int tlq_gemm_w4a8_ws(const void* A, const void* w_packed, void* workspace, int64
                       K < kMaxDim && fits32(N, K / 2) && fits32(M, K);
   const bool two_steps = usable && workspace_bytes >= N * K && K % 16 == 0 && N % 16 == 0 && fits32(N, K) &&
                          (M > 64 || g_w4a8_ws_mode == 2);
-  if (g_w4a8_ws_mode == 0 && small_tile_for_i8(1, M, N, K, two_steps ? kUseW4A8TwoSteps : kUseW4A8).ok)
+  // (above 256 rows the caller finds the unpacked weights in a workspace that holds them, also where the small-tile kernel is faster)
+  if (g_w4a8_ws_mode == 0 && !(two_steps && M > 256) && small_tile_for_i8(1, M, N, K, two_steps ? kUseW4A8TwoSteps : kUseW4A8).ok)
     return tlq_gemm_w4a8(A, w_packed, C, M, N, K, sign_mode, stream);
   if (usable && K % 32 == 0 && N % 4 == 0 && g_w4a8_ws_mode != 2 && (M <= 256 || g_w4a8_ws_mode == 1)) {
     int split = i8_split_choice(1, M, N, K, true, 2.5);
