@@ -1288,7 +1288,8 @@ static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, in
   return k_bytes <= 48 * kStageBytes && group_tile_us(tile, 1, M, N, k_bytes) < 0.9 * sliced_us(kind, 1, M, N, K);
 }
 // The products that may take the small-tile kernel: weights as stored (the first four: SmallW), int32 results, or rescaled ones
-// (W8A8), W4A8 where the caller brought the room to unpack the weights first.
+// (W8A8), W4A8 where the caller brought the room to unpack the weights first (65 to 256 rows: above, that is what runs; the figures
+// below count such problems of any number of rows).
 enum SmallUse { kUseI8NK = kSmallNK, kUseI8KN = kSmallKN8, kUseF16KN = kSmallKN16, kUseW4A8 = kSmallW4, kUseW4A8TwoSteps = 4, kUseW8A8NK = 5, kUseW8A8KN = 6 };
 static SmallW small_weights(SmallUse use) { return use == kUseW8A8NK ? kSmallNK : use == kUseW8A8KN ? kSmallKN8 : use == kUseW4A8TwoSteps ? kSmallW4 : (SmallW)use; }
 // Is the small-tile kernel ahead of what would run in its place?  Two things its own estimate leaves out come on top: the activations' trip from

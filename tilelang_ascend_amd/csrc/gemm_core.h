@@ -777,7 +777,7 @@ __device__ __forceinline__ TileCoord tile_of_block(int tiles_m, int tiles_n, int
 // ---- the kernel -----------------------------------------------------------------------------
 // KG > 1: the work-group is KG groups of WM x WN wavefronts, each with two LDS stages of its own, that run the same tile over
 // KG consecutive parts of K in step and meet in LDS at the end (group g writes tile rows g of KG of every wavefront
-// tile).  See k_groups_pay for when and why.
+// tile).  See group_tile for when and why.
 template <class Mma, class AL, class WL, class Epi, int BM, int BN, int WM, int WN, int KG = 1>
 __global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void gemm_mfma_kernel(
     typename AL::Params pa, typename WL::Params pw, typename Epi::Params pe, int M, int N, int kt_each, int k_tail,

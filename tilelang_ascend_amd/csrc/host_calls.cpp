@@ -1,16 +1,17 @@
 // The calls of the operators, from Python arguments to the C entry points of libtlq, in native code.
 //
 // What a small operator costs is the host: a decode GEMV runs 6 us on the GPU, and checking its arguments, allocating its
-// output and workspace and making the call took 23 us in Python (MI355X box; torch's own one-launch operators take 4.0 us).
+// output and workspace and making the call took 23 us in Python (torch's own one-launch operators take 4.0 us).
 // Here the same steps are one extension call of 4 - 5 us with one launch (1 x 11008 x 4096: 22.5 -> 6.1 us a call, which is the
 // kernel): a Plan is built once per kernel object from its parameter list, and calling it checks the tensors, allocates
 // outputs (and the workspace the entry point asks for) from torch's caching allocator on the current stream, releases the
 // interpreter lock and calls the entry point.
 //
-// A Plan does the ordinary call only.  Whatever is not ordinary -- a wrong type or shape, a tensor on another device, anything
-// that ends in an error -- comes back as NotImplemented with nothing done, and the Python path of the caller takes over: it
-// names the error, or runs the call on the other device.  Nothing here keeps state between calls, so any number of threads and
-// streams may use one Plan.
+// A Plan does the ordinary call only.  Whatever its checks do not let through -- a wrong type or shape, a tensor on another
+// device, an allocation that fails -- comes back as NotImplemented with nothing done, and the Python path of the caller takes
+// over: it names the error, or runs the call on the other device.  What passes the checks is called once: where the entry point refuses it, the entry point's
+// message is raised from here, as that path would.  Nothing here keeps state between calls, so any number of threads and streams may
+// use one Plan.
 #include <Python.h>
 #include <structmember.h>
 
