@@ -169,10 +169,12 @@ int tlq_decode_lowbit_interleaved(const void* src, const void* scales, const voi
  * A: [M,K] in_dtype (TLQ_F16 / TLQ_BF16); C: [M,N] out_dtype (TLQ_F16 / TLQ_BF16 / TLQ_F32).
  * Requires K % 64 == 0 and group % 32 == 0 (group divides K).  The MFMA kernel additionally needs
  * N % 4 == 0 and a power-of-two group (32, 64, 128, ...); the GEMV kernel (M <= 16) takes any such group;
- * the skinny kernel (M <= 64) needs K % 128 == 0.  TLQ_ALGO_AUTO: M = 1 GEMV (fp16; bf16 up to K = 8192; fp16 also M = 2 with
+ * the skinny kernel (M <= 64) needs K % 128 == 0.  TLQ_ALGO_AUTO: M = 1 GEMV (rows of up to 16384 values; fp16 also M = 2 with
  * K <= 4096), otherwise the decode kernel (TLQ_ALGO_DECODE) where M <= 32, K % 256 == 0, K <= 4096, the group is a power of two and the
  * scale / zero tensors are dword aligned, else M <= 64 skinny where its conditions hold (else GEMV up to M = 4), else -- more than
- * 64 rows -- what tlq_gemm_w4a16_ws takes when it is given no workspace: the streaming and panel kernels where they do not cut K, else MFMA. */
+ * 64 rows -- what tlq_gemm_w4a16_ws takes when it is given no workspace: the streaming and panel kernels where they do not cut K, else
+ * MFMA.  In the place of the decode, skinny, streaming, panel or MFMA kernel it takes the small-tile kernel (TLQ_ALGO_SMALL) where that
+ * kernel's conditions hold and its estimate is ahead of theirs.  A family named by `algo` runs itself or the call is refused. */
 int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, const void* zeros, void* C, int64_t M,
                    int64_t N, int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int algo,
                    void* stream);
@@ -185,10 +187,14 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
  * workspace, then the plain GEMM on it (itself over K slices, kept behind the dequantised matrix, where it has few output
  * tiles) -- which is the structure of the reference's own wrapper (example_dequant_gemm_fine_grained.py:176-223 unpacks,
  * then calls fp16_gemm) and is faster than converting the weights again in every row block of the fused kernel.  The
- * workspace holds nothing between calls.
- * algo: as tlq_gemm_w4a16, or TLQ_ALGO_TWO_PASS to force the two passes (workspace required).
- * With TLQ_ALGO_AUTO and more than 512 rows, a row count that is no multiple of four runs as two calls on the stream: the
- * multiple of four below (the large-M kernels take such counts only), then the last one to three rows.
+ * workspace holds nothing between calls.  TLQ_ALGO_AUTO takes the small-tile kernel in one launch, with no workspace, in the place of
+ * any of these on problems that leave the others' tiles few or short, by estimates of both.
+ * algo: as tlq_gemm_w4a16, or a family that only this entry point has (TLQ_ALGO_TWO_PASS, _STREAM, _PANEL, _PANEL256, _PANELM).
+ * With TLQ_ALGO_AUTO and more than 512 rows, a row count that is no multiple of four runs in one launch of the small-tile kernel or in
+ * the two passes where their estimates say so; otherwise as two calls on the stream: the multiple of four below (the panel kernels
+ * take such counts only), then the last one to three rows.  Always as two calls where those last rows, run by themselves, go to the
+ * fp16 GEMV kernels: they apply scale and zero point to fp32 sums of exact products, and their rows are the only ones of the
+ * result whose weights are not rounded to in_dtype.
  * One scale / zero point per weight row (group == K) on rows whose length is no power of two: the kernels over K slices take
  * power-of-two groups, so the per-row values are first written out per group of min(K & -K, 1024) values into the last
  * 2 * align16(N * K / group * 2) + 16 bytes of the workspace (tlq_w4a16_workspace_bytes counts them) and the call runs with
@@ -214,8 +220,8 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
  * tlq_pack_int4(interleave = 1)); TLQ_W_PLAIN is tlq_gemm_w4a16_ws itself.  Consumers of the repacked layout: the ring GEMV
  * (one activation row, or two fp16 rows; K <= 4096, (K / group) % 8 == 0; TLQ_ALGO_GEMV or the automatic choice), the
  * decode kernel (M <= 32, K % 256 == 0), the streaming kernel (17 <= M <= 512; the fp16 decode saves the four byte permutes
- * per word that only undo the plain layout), the panel kernels and the two passes (M >= 256 with a workspace of N * K
- * 16-bit values).  Other shapes are rejected.  Results are bit-identical to the plain layout on the same logical weights,
+ * per word that only undo the plain layout), the small-tile kernel (any M; TLQ_ALGO_SMALL, or the automatic choice in the place of the
+ * decode and streaming kernels), the panel kernels and the two passes (M >= 256 with a workspace of N * K 16-bit values).  Other shapes are rejected.  Results are bit-identical to the plain layout on the same logical weights,
  * except for the GEMV, whose dot products pair neighbouring elements instead of elements four apart: there the two
  * layouts agree to the rounding of the fp32 sums (and bit for bit on one-hot activations).  One scale / zero point per row on
  * rows whose length is no power of two is written out per group into the workspace's tail as in tlq_gemm_w4a16_ws, and ragged
@@ -320,8 +326,9 @@ int tlq_gemm_w4a8(const void* A, const void* w_packed, void* C, int64_t M, int64
  * (example_dequant_gemm_w4a8.py:27,69-106 unpacks into it on the vector cores, :108-120 multiplies from it).  With many
  * activation rows (M > 256) and a usable workspace (N * K bytes, 16-byte aligned, K and N multiples of 16) the weights
  * are unpacked into it and the int8 GEMM runs on it, as in the reference; the workspace then holds the unpacked
- * weights.  With few rows the unpack stays fused and K is cut into slices, the workspace holding one int32 [M, N] matrix
- * per slice (as many slices as fit).  Otherwise this is tlq_gemm_w4a8.  The result is the same in every case. */
+ * weights.  With few rows the unpack stays fused: one launch of the small-tile kernel, which leaves the workspace alone, where its
+ * estimate is ahead, otherwise K is cut into slices, the workspace holding one int32 [M, N] matrix per slice (as many slices as
+ * fit), or, from 65 rows on where K has no cut, the two steps.  Otherwise this is tlq_gemm_w4a8.  The result is the same in every case. */
 int tlq_gemm_w4a8_ws(const void* A, const void* w_packed, void* workspace, int64_t workspace_bytes, void* C, int64_t M,
                      int64_t N, int64_t K, int sign_mode, void* stream);
 
