@@ -6,8 +6,9 @@ The reference unpacks on the vector cores into a caller-supplied int8 [N, K] glo
 and then runs the cube GEMM; so does this one from 257 activation rows on when the workspace
 (third positional, as the reference's callers pass it) is a usable int8 [N, K] buffer: an unpack
 kernel at the HBM roofline and the int8 GEMM, which together beat the kernel that unpacks on the
-way into LDS.  With fewer rows the unpack pass would cost more than the GEMM: the fused kernel
-runs over slices of K and keeps one int32 [M, N] matrix per slice in the workspace.
+way into LDS.  With fewer rows the unpack pass would cost more than the GEMM: the small-tile
+kernel in one launch, or the fused kernel over slices of K, which keeps one int32 [M, N] matrix
+per slice in the workspace.
 """
 from __future__ import annotations
 
