@@ -87,6 +87,17 @@ def test_automatic_choice_leaves_many_results_of_short_rows_to_larger_tiles(M, N
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,kernel", [(64, 4096, 14336, "w4a16_stream_kernel"), (48, 4096, 4096, "w4a16_small_kernel"), (24, 8192, 10368, "w4a16_small_kernel")])
+def test_long_shares_of_large_matrices_go_to_the_streaming_kernel(M, N, K, kernel):
+    """Small tiles are level there while a cache holds the weights and 1.2 x slower from memory (on a machine of 256 CUs)."""
+    A = torch.randn(M, K, generator=gen(M)).half()
+    Wp, s, z = make_w4(N, K, 128, torch.float16, "int", seed=N)
+    got = run(A, Wp, s, z, 128, _abi.ALGO_AUTO, workspace=_abi.load().tlq_w4a16_workspace_bytes(M, N, K))
+    assert kernel in run.log or _abi.load().tlq_device_cu_count() != 256, run.log
+    check_float_output(got, w4a16_reference(A, Wp, s, z, 128), f"{M}x{N}x{K}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("layout", [_abi.W_PLAIN, _abi.W_INTERLEAVED_F16])
 @pytest.mark.parametrize("M,N,K,group,algo,kernel", [
     (40, 1024, 768, 128, "STREAM", "w4a16_stream_kernel"), (200, 300, 256, 64, "STREAM", "w4a16_stream_kernel"), (130, 528, 512, 32, "MFMA", "tlq_gemm_w4a16(mfma)"),

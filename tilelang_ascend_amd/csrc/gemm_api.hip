@@ -267,8 +267,17 @@ static double small_us(const SmallTile& p, int64_t M, int64_t N, int64_t K) { re
 static double fused_tile_us(int64_t M, int64_t N, int64_t K) {  // the W4A16 tile kernel where it has few tiles: 4 us + 1.5 us per 128 values of K
   return 3.9 + 11.6e-3 * (double)K + 0.94 * giga((double)M, N, K) + 0.116e-6 * (double)M * (double)N;
 }
+// The streaming kernel.  The figures above are of weights that a cache still holds (three sets in turn); from memory the small-tile kernel,
+// with two steps in flight to a wavefront, takes 0.09 us more per step of a wavefront's share of K and 0.08 us per MB of weights (fitted,
+// 0.7 us rms on 900 problems), the streaming kernel 1 us and 0.01.  So where a wavefront has 24 steps and more on 16 MB of weights and
+// more, it has to be ahead by more than the estimates are off: on the 32 of 23000 problems (M 17 .. 200, N 1024 .. 9600, K 3072 .. 14336)
+// that this changes the streaming kernel is 2 % behind from a cache and 1.21 x ahead from memory (64 x 4096 x 14336 27.4 -> 24.8 us
+// and 32.6 -> 26.9).  With shorter shares small tiles are ahead from a cache by less than they are behind from memory (22 and 23 steps: 3 %
+// and 14 %), on fewer rows by more (18 x 7856 x 9344 18.4 against 24.7 us, and 22.5 against 25.6).
 static bool small_beats_stream(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
-  return p.ok && g_stream_slice_steps <= 0 && small_us(p, M, N, K) < 0.99 * (11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K);
+  if (!p.ok || g_stream_slice_steps > 0) return false;
+  const bool long_shares = M > 32 && ceil_div(K / 128, (int64_t)p.waves) >= 24 && N * K >= ((int64_t)32 << 20);
+  return small_us(p, M, N, K) < (long_shares ? 0.85 : 0.99) * (11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K);
 }
 // above 512 rows: the tile kernel on up to 2^19 weights -- and the launch for the last M % 4 rows, 4 us, where they run apart --, else the
 // two passes or the panel kernels, which are level with them or ahead; only while the whole call stays short
