@@ -49,6 +49,9 @@ int tlq_debug_check_panel256_addressing(int64_t M, int64_t N, int64_t K, int64_t
 int tlq_debug_panel256_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out);
 /* The schedule alone over `steps` steps, with the kernel's own wait counts (negative arguments) or others (to see them fail). */
 int tlq_debug_check_panel256_schedule(int steps, int wait_w, int wait_a);
+/* What the streaming kernel would take for a problem on a device with `cus` compute units: plan_out receives int64 activation rows and weight
+ * rows per work-group, K slices, steps of 128 values per slice, estimated nanoseconds; returns 1 when it applies. */
+int tlq_debug_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out);
 /* What the small-tile kernel (one launch, wavefronts split K) would take for a problem: plan_out receives int64 activation rows and weight
  * rows per work-group, wavefronts, estimated nanoseconds; returns 1 when it applies. */
 int tlq_debug_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, void* plan_out);
@@ -116,6 +119,7 @@ void tlq_tune_gemm_slots(int mode);                          /* the kernel that 
                                                               * 16-bit GEMMs), 0 never */
 void tlq_tune_w4a16_decode(int on);                          /* 0: the decode kernel is never picked automatically */
 void tlq_tune_w4a16_stream(int on);                          /* 0: tlq_gemm_w4a16_ws never picks the streaming kernel by itself */
+void tlq_tune_w4a16_stream_tiles(int tiles);                 /* 16-row activation tiles per work-group of the streaming kernel, 2 .. 8 (0 = by its estimate) */
 void tlq_tune_w4a16_stream_slice(int steps);                 /* K slice of the streaming kernel in steps of 128 values (0 = by its estimate) */
 void tlq_tune_w4a16_panel(int mode);                         /* tlq_gemm_w4a16_ws, large M: 0 = automatic, otherwise a panel kernel is never picked automatically */
 void tlq_tune_w4a16_panelm_rows(int rows);                   /* activation rows per work-group of the middle-M panel kernel: 64, 128, 0 = its plan's */

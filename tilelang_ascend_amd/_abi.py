@@ -64,6 +64,7 @@ SIGNATURES = {
     "tlq_act_quant_i8": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _int, _vp]),
     "tlq_debug_check_gemm_addressing": (_int, [_int, _i64, _i64, _int, _int]),
     "tlq_debug_check_slots_schedule": (_int, [_int, _int]),
+    "tlq_debug_stream_plan": (_int, [_i64, _i64, _i64, _i64, _int, _vp]),
     "tlq_debug_check_stream_addressing": (_int, [_i64, _i64, _i64, _int, _int]),
     "tlq_debug_check_decode_addressing": (_int, [_i64, _i64, _i64, _i64, _int, _int, _int, _int]),
     "tlq_debug_decode_plan": (_int, [_i64, _i64, _i64, _i64, _int, _vp]),
@@ -94,6 +95,7 @@ SIGNATURES = {
     "tlq_debug_gemm_tile": (_int, [_i64, _i64, _i64, _int]),
     "tlq_tune_w4a16_stream": (None, [_int]),
     "tlq_tune_w4a16_stream_slice": (None, [_int]),
+    "tlq_tune_w4a16_stream_tiles": (None, [_int]),
     "tlq_tune_w4a16_panel": (None, [_int]),
     "tlq_tune_w4a16_panel_slice": (None, [_int]),
     "tlq_tune_w4a16_panelm_rows": (None, [_int]),

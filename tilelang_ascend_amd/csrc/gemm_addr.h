@@ -158,14 +158,27 @@ __host__ __device__ inline uint32_t sa_frag_off(int lane, int tm, int ks) {
   const int r16 = lane & 15, q = lane >> 4;
   return (uint32_t)((tm * 16 + r16) * 256 + (((4 * q + ks) ^ sa_swz(r16)) << 4));
 }
-// Ring of D steps: step s lives in slot s % D.  Every wavefront issues `per_step` load instructions per step, in
-// step order, and loads retire in issue order: this wavefront's loads of step s have landed once at most the
-// loads of the younger steps that were already issued are outstanding.  At the top of step s (before the loads of
-// step s + D - 1 are issued) those are the steps s + 1 .. min(s + D - 2, last).
-__host__ __device__ inline int stream_younger_steps(int s, int steps, int D) {
-  const int last_issued = s + D - 2 < steps - 1 ? s + D - 2 : steps - 1;
-  return last_issued - s > 0 ? last_issued - s : 0;
+// The streaming kernel's 32 x 32 operands: lane (row r32 of a 32-row tile, half h) of the wavefronts that take values 64 kg .. 64 kg +
+// 63 of a step holds k = 64 kg + 32 h + 8 t .. + 7 at k-step t = 0 .. 3: the four words of 16-byte piece 2 kg + h of its packed row, and
+// the activations' logical chunk 8 kg + 4 h + t.
+__host__ __device__ inline uint32_t stream_w_frag(int r32, int piece) {  // inside two 1 KB tiles of 16 rows
+  const int r16 = r32 & 15;
+  return (uint32_t)((r32 >> 4) * 1024 + r16 * 64 + ((piece ^ sw_swz(r16)) << 4));
 }
+__host__ __device__ inline uint32_t stream_a_frag(int r32, int chunk) {  // inside 32 rows of 256 B
+  return (uint32_t)(r32 * 256 + ((chunk ^ sa_swz(r32 & 15)) << 4));
+}
+// Scales and zero points of 32 weight rows: [32 rows][MG groups of a window] of 2 bytes each, 16-byte pieces swizzled so that 32 rows'
+// values of a group lie two to a bank at most.  Fetched by MG / 16 direct loads of 16-byte pieces or MG / 4 of dwords: load i, lane l.
+__host__ __device__ inline int stream_sz_swz(int mg, int row) { return mg == 32 ? (row >> 2) & 3 : (row >> 3) & 1; }
+__host__ __device__ inline int stream_sz_row(int cells, int i, int lane) { return (i * 64 + lane) / cells; }  // cells: pieces (MG / 8) or dwords (MG / 2) per row
+__host__ __device__ inline int stream_sz_piece(int mg, int lane, int row) { return (lane & (mg / 8 - 1)) ^ stream_sz_swz(mg, row); }
+__host__ __device__ inline int stream_sz_dword(int mg, int lane, int row) { return (lane & (mg / 2 - 1)) ^ (stream_sz_swz(mg, row) * 4); }
+__host__ __device__ inline int stream_sz_value(int mg, int row, int g) { return row * mg + (g ^ (stream_sz_swz(mg, row) * 8)); }  // where value g of the row lies
+// Ring of D steps of L load instructions each: step s lives in slot s % D.  A wavefront's step is NU units; in front of unit NU - 2 of
+// step s it waits until (D - 2) L loads are outstanding, passes the step's barrier and from there on, NU units long, issues the loads
+// of step s + D: load i in unit i NU / L behind the barrier.
+__host__ __device__ constexpr int stream_load_unit(int i, int units, int loads) { return i * units / loads; }
 
 // ---- panel kernel for large M (gemm_w4a16_panel.hip): 128 activation rows x 512 weight rows per work-group ----------
 // Steps of 128 values of K in two ring slots.  A slot is the activation tile [128 rows][256 B] (the streaming kernel's

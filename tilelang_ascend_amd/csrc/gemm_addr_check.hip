@@ -269,35 +269,65 @@ struct SlotsSim {
   }
 };
 
-// Streaming W4A16 kernel: packed weights [N, K / 2], activations [M, K] of 2-byte values, 16 * tm activation rows and
-// 256 weight rows per work-group, steps of 128 values of K.
+// Streaming W4A16 kernel: packed weights [N, K / 2], activations [M, K] of 2-byte values, 16 * tm activation rows per work-group,
+// steps of 128 values of K; two groups of wavefronts on 256 weight rows or four on 128.
 int check_stream(int64_t M, int64_t N, int64_t K, int tm) {
   CHECK_OR_FAIL(tm == 2 || tm == 4 || tm == 6 || tm == 8, "stream: %d activation tiles", tm);
   CHECK_OR_FAIL(M > 0 && N > 0 && K >= 128 && K % 128 == 0, "stream: bad shape");
   CHECK_OR_FAIL(N * (K / 2) < ((int64_t)1 << 32) && M * K * 2 < ((int64_t)1 << 32), "stream: a matrix spans 4 GiB or more");
   const int64_t w_extent = N * (K / 2), a_extent = M * K * 2;
   const int steps = (int)(K / 128), la = tm / 2;
-  std::vector<int> cell(1024 / 16), acell(tm * 16 * 16);
-  for (int64_t n0 = 0; n0 < N; n0 += 256)
-    for (int wave = 0; wave < 8; ++wave)
-      for (int tn = 0; tn < 2; ++tn) {
-        std::fill(cell.begin(), cell.end(), -1);
-        for (int lane = 0; lane < 64; ++lane) {
-          int64_t n = n0 + wave * 32 + tn * 16 + addr::sw_row(lane);
-          n = n < N ? n : N - 1;
-          const int64_t voff = n * (K / 2) + addr::sw_piece(lane) * 16;
-          for (int st = 0; st < steps; ++st) {
-            const int64_t o = voff + (int64_t)st * 64;
-            CHECK_OR_FAIL(o >= 0 && o + 16 <= w_extent, "stream: weight load at [%lld, +16) of %lld", (long long)o, (long long)w_extent);
+  std::vector<int> acell(tm * 16 * 16);
+  for (int kgs = 2; kgs <= 4; kgs += 2) {
+    const int wns = 8 / kgs, bn = 64 * wns, lw = wns / 2, kt = 8 / kgs;
+    std::vector<int> cell(bn * 4);
+    for (int64_t n0 = 0; n0 < N; n0 += bn) {
+      std::fill(cell.begin(), cell.end(), -1);
+      for (int wave = 0; wave < 8; ++wave)
+        for (int j = 0; j < lw; ++j)
+          for (int lane = 0; lane < 64; ++lane) {
+            const int row = (wave * lw + j) * 16 + addr::sw_row(lane), at = (wave * lw + j) * 64 + lane;  // 16-byte cell
+            int64_t n = n0 + row;
+            n = n < N ? n : N - 1;
+            const int64_t voff = n * (K / 2) + addr::sw_piece(lane) * 16;
+            for (int st = 0; st < steps; ++st) {
+              const int64_t o = voff + (int64_t)st * 64;
+              CHECK_OR_FAIL(o >= 0 && o + 16 <= w_extent, "stream: weight load at [%lld, +16) of %lld", (long long)o, (long long)w_extent);
+            }
+            CHECK_OR_FAIL(row < bn && cell[at] == -1, "stream: weight cell %d written twice", at);
+            cell[at] = row * 4 + addr::sw_piece(lane);
           }
-          cell[lane] = addr::sw_row(lane) * 4 + addr::sw_piece(lane);  // the lane lands on 16-byte cell `lane` of the 1 KB tile
-        }
+      for (int wave = 0; wave < 8; ++wave)
+        for (int tn = 0; tn < 2; ++tn)
+          for (int lane = 0; lane < 64; ++lane) {
+            const int kg = wave / wns, wn = wave % wns, r32 = lane & 31, word = 2 * kt * kg + kt * (lane >> 5);
+            const uint32_t off = (uint32_t)(wn * 4096 + tn * 2048) + addr::stream_w_frag(r32, word >> 2) + (uint32_t)((word & 3) * 4);
+            CHECK_OR_FAIL(off % (4 * kt) == 0 && off + 4 * kt <= (uint32_t)bn * 64, "stream: weight operand read at %u", off);
+            CHECK_OR_FAIL(cell[off / 16] == (wn * 64 + tn * 32 + r32) * 4 + word / 4, "stream: weight operand read of lane %d finds cell %d", lane, cell[off / 16]);
+          }
+    }
+    // which words of a step the wavefronts of a column of work-groups take: every one once
+    std::vector<int> taken(16, 0);
+    for (int kg = 0; kg < kgs; ++kg)
+      for (int h = 0; h < 2; ++h)
+        for (int t = 0; t < kt; ++t) ++taken[2 * kt * kg + kt * h + t];
+    for (int w = 0; w < 16; ++w) CHECK_OR_FAIL(taken[w] == 1, "stream: word %d of a step is taken %d times", w, taken[w]);
+    // the scale area: what a read finds is the value it wants, whether pieces or dwords brought it (a dword read may start one value on)
+    const int mg = kgs == 4 ? 32 : 16;
+    for (int cells : {mg / 8, mg / 2}) {
+      std::vector<int> value(32 * mg, -1);
+      for (int i = 0; i < 32 * cells / 64; ++i)
         for (int lane = 0; lane < 64; ++lane) {
-          const uint32_t off = addr::sw_frag_off(lane);
-          CHECK_OR_FAIL(off % 16 == 0 && off + 16 <= 1024, "stream: weight operand read at %u", off);
-          CHECK_OR_FAIL(cell[off / 16] == (lane & 15) * 4 + (lane >> 4), "stream: weight operand read of lane %d finds cell %d", lane, cell[off / 16]);
+          const int row = addr::stream_sz_row(cells, i, lane), each = mg / cells;
+          const int g = each * (cells == mg / 8 ? addr::stream_sz_piece(mg, lane, row) : addr::stream_sz_dword(mg, lane, row));
+          CHECK_OR_FAIL(row < 32 && g >= 0 && g + each <= mg, "stream: scale load of row %d, value %d", row, g);
+          for (int e = 0; e < each; ++e) value[(i * 64 + lane) * each + e] = row * mg + g + e;
         }
-      }
+      for (int row = 0; row < 32; ++row)
+        for (int g = 0; g < mg; ++g)
+          CHECK_OR_FAIL(value[addr::stream_sz_value(mg, row, g)] == row * mg + g, "stream: scale read of row %d, value %d finds %d", row, g, value[addr::stream_sz_value(mg, row, g)]);
+    }
+  }
   for (int64_t m0 = 0; m0 < M; m0 += 16 * tm) {
     std::fill(acell.begin(), acell.end(), -1);
     for (int wave = 0; wave < 8; ++wave)
@@ -321,14 +351,13 @@ int check_stream(int64_t M, int64_t N, int64_t K, int tm) {
         }
       }
     for (size_t c = 0; c < acell.size(); ++c) CHECK_OR_FAIL(acell[c] >= 0, "stream: activation cell %zu never written", c);
-    for (int t = 0; t < tm; ++t)
-      for (int ks = 0; ks < 4; ++ks)
-        for (int lane = 0; lane < 64; ++lane) {
-          const uint32_t off = addr::sa_frag_off(lane, t, ks);
+    for (int tb = 0; tb < tm / 2; ++tb)
+      for (int chunk = 0; chunk < 16; ++chunk)
+        for (int r32 = 0; r32 < 32; ++r32) {
+          const uint32_t off = (uint32_t)(tb * 32 * 256) + addr::stream_a_frag(r32, chunk);
           CHECK_OR_FAIL(off % 16 == 0 && off + 16 <= (uint32_t)tm * 4096, "stream: activation operand read at %u", off);
-          const int want = (t * 16 + (lane & 15)) * 16 + 4 * (lane >> 4) + ks;
-          CHECK_OR_FAIL(acell[off / 16] == want, "stream: activation operand read (lane %d, k-step %d) finds cell %d, expects %d", lane, ks,
-                        acell[off / 16], want);
+          const int want = (tb * 32 + r32) * 16 + chunk;
+          CHECK_OR_FAIL(acell[off / 16] == want, "stream: activation operand read (row %d, chunk %d) finds cell %d, expects %d", r32, chunk, acell[off / 16], want);
         }
   }
   return 0;
@@ -799,27 +828,41 @@ int check_panel256_schedule(int steps, int wait_w, int wait_a) {
   return 0;
 }
 
-// The ring: step s occupies slot s % D; at the top of step s the wavefront waits until only `younger` steps' loads are
-// outstanding, passes the barrier, and then issues step s + D - 1 into the slot of step s - 1.
-int check_stream_ring(int steps, int D) {
-  CHECK_OR_FAIL(steps >= 1 && D >= 2 && D <= 8, "stream ring: bad arguments");
-  std::vector<int> slot(D, -1), queue;  // slot owner; issued and not yet known to have landed (oldest first)
-  std::vector<char> landed(steps, 0), done(steps, 0);
-  for (int s = 0; s < D - 1 && s < steps; ++s) slot[s % D] = s, queue.push_back(s);
-  for (int s = 0; s < steps; ++s) {
-    const int younger = addr::stream_younger_steps(s, steps, D);
-    while ((int)queue.size() > younger) landed[queue.front()] = 1, queue.erase(queue.begin());
-    CHECK_OR_FAIL(landed[s], "stream ring: step %d multiplied before its loads were waited for", s);
-    // barrier: every wavefront is past step s - 1
-    if (s >= 1) done[s - 1] = 1;
-    if (s + D - 1 < steps) {
-      const int t = s + D - 1, sl = t % D;
-      CHECK_OR_FAIL(slot[sl] < 0 || done[slot[sl]], "stream ring: step %d overwrites step %d which may still be read", t, slot[sl]);
-      slot[sl] = t, queue.push_back(t);
+// The ring (addr::stream_load_unit): the loads of one wavefront in issue order against its waits, and the slots against the
+// steps that are still read.  Loads past the last step are issued empty.
+int check_stream_ring(int steps, int D, int L, int NU) {
+  CHECK_OR_FAIL(steps >= 1 && D >= 3 && D <= 8 && L >= 1 && L <= 8 && (NU == 4 || NU == 8), "stream ring: bad arguments");
+  std::vector<int> slot(D, -1), queue;  // slot owner; steps of the loads issued and not yet known to have landed (oldest first)
+  std::vector<int> landed(steps + 2 * D, 0);
+  auto issue = [&](int step, int before_read_of) {  // every wavefront has read its last of steps below before_read_of
+    const int sl = step % D;
+    if (step < steps) {
+      CHECK_OR_FAIL(slot[sl] < 0 || slot[sl] == step || slot[sl] < before_read_of, "stream ring: step %d overwrites step %d which may still be read", step, slot[sl]);
+      slot[sl] = step;
     }
-    CHECK_OR_FAIL(slot[s % D] == s, "stream ring: the slot of step %d holds step %d", s, slot[s % D]);
+    queue.push_back(step);
+    return 0;
+  };
+  auto wait = [&](int outstanding) {
+    while ((int)queue.size() > outstanding) ++landed[queue.front()], queue.erase(queue.begin());
+  };
+  int behind = 0;  // loads issued in the two units behind a barrier
+  for (int i = 0; i < L; ++i) behind += addr::stream_load_unit(i, NU, L) < 2;
+  for (int s = 0; s < D; ++s)
+    for (int i = 0; i < (s < D - 1 ? L : behind); ++i)
+      if (int rc = issue(s, 0)) return rc;
+  wait((D - 2) * L + behind);
+  for (int s = 0; s < steps; ++s) {
+    CHECK_OR_FAIL(landed[s] == L && slot[s % D] == s, "stream ring: step %d multiplied before its loads were waited for", s);
+    for (int u = 0; u < NU; ++u) {
+      if (u == NU - 2) wait((D - 2) * L);  // and the barrier: everyone has read its last of step s
+      for (int i = 0; i < L; ++i)
+        if (addr::stream_load_unit(i, NU, L) == (u + 2) % NU)
+          if (int rc = issue(u >= NU - 2 ? s + D : s + D - 1, u >= NU - 2 ? s + 1 : s)) return rc;
+      if (u == NU - 2 && s + 1 < steps)
+        CHECK_OR_FAIL(landed[s + 1] == L && slot[(s + 1) % D] == s + 1, "stream ring: step %d read before its loads were waited for", s + 1);
+    }
   }
-  CHECK_OR_FAIL(queue.empty() || queue.back() <= steps - 1, "stream ring: bookkeeping");
   return 0;
 }
 
@@ -1265,8 +1308,12 @@ int tlq_debug_check_gemm_addressing(int source_kind, int64_t rows, int64_t row_b
 
 int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activation_tiles, int ring_depth) {
   if (int rc = check_stream(M, N, K, activation_tiles)) return rc;
+  const int l = activation_tiles / 2;
   for (int steps = 1; steps <= 40; ++steps)
-    if (int rc = check_stream_ring(steps, ring_depth)) return rc;
+    for (int depth = ring_depth; depth <= 6; ++depth) {
+      if (int rc = check_stream_ring(steps, depth, l + 2, 8)) return rc;
+      if (int rc = check_stream_ring(steps, depth, l + 1, 4)) return rc;
+    }
   return 0;
 }
 

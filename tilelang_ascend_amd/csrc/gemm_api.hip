@@ -3,6 +3,7 @@
 #include "tlq_common.h"
 #include "gemm_core.h"
 #include "small_tiles.h"
+#include "stream_plan.h"
 
 namespace tlq {
 int gemv_w4a16(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t batch, int64_t M,
@@ -22,14 +23,6 @@ double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group);
 int gemm_w4a16_mfma_splitk(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M,
                            int64_t N, int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype,
                            int64_t split, float* partial, hipStream_t st);
-struct StreamPlan {
-  bool ok;
-  int tm, m_blocks, n_blocks, split, slice_steps;
-};
-StreamPlan w4a16_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus);
-int gemm_w4a16_stream(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
-                      int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int w_layout, const StreamPlan& p,
-                      float* partial, hipStream_t st);
 int gemm_w4a16_skinny(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, hipStream_t st);
 int gemm_f16_plain(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype,
@@ -106,7 +99,7 @@ static int cu_count_or_default() {
   const int n = tlq_device_cu_count();
   return n > 0 ? n : 256;
 }
-extern thread_local int g_stream_slice_steps;
+extern thread_local int g_stream_slice_steps, g_stream_tiles;
 thread_local int g_w4a16_stream = 1;  // 0: never pick the streaming kernel automatically (tuning runs)
 thread_local int g_w4a16_decode = 1;  // 0: never pick the decode kernel automatically
 // the tile loaders address one matrix with 32-bit byte offsets
@@ -190,6 +183,7 @@ int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused) {
 }
 void tlq_tune_gemm_tile(int tile) { tlq::tuning_changed(), tlq::g_gemm_f16_tile = (tile == 128 || tile == 256) ? tile : 0; }
 void tlq_tune_w4a16_stream(int on) { tlq::g_w4a16_stream = on != 0; }
+void tlq_tune_w4a16_stream_tiles(int tiles) { tlq::tuning_changed(), tlq::g_stream_tiles = ((tiles & 15) >= 2 && (tiles & 15) <= 8 && (tiles & 1) == 0) ? tiles & 31 : 0; }
 void tlq_tune_w4a16_stream_slice(int steps) { tlq::tuning_changed(), tlq::g_stream_slice_steps = steps; }
 void tlq_tune_w4a16_decode(int on) { tlq::g_w4a16_decode = on != 0; }
 void tlq_tune_w4a16_panel(int mode) { tlq::g_w4a16_panel = mode != 0 ? 1 : 0; }
@@ -235,6 +229,16 @@ int tlq_debug_small_plan(int64_t M, int64_t N, int64_t K, int64_t group, void* p
   return p.ok ? 1 : 0;
 }
 
+int tlq_debug_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out) {
+  if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return 0;
+  const StreamPlan p = w4a16_stream_plan(M, N, K, group, cus);
+  if (plan_out) {
+    int64_t* o = (int64_t*)plan_out;
+    o[0] = 16 * p.tm, o[1] = p.ok ? 512 / p.kg : 0, o[2] = p.split, o[3] = p.slice_steps, o[4] = (int64_t)(p.us * 1000.0);
+  }
+  return p.ok ? 1 : 0;
+}
+
 int tlq_debug_decode_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out) {
   const DecodePlan p = w4a16_decode_plan(M, N, K, group, cus);
   if (plan_out) {
@@ -267,21 +271,25 @@ static double small_us(const SmallTile& p, int64_t M, int64_t N, int64_t K) { re
 static double fused_tile_us(int64_t M, int64_t N, int64_t K) {  // the W4A16 tile kernel where it has few tiles: 4 us + 1.5 us per 128 values of K
   return 3.9 + 11.6e-3 * (double)K + 0.94 * giga((double)M, N, K) + 0.116e-6 * (double)M * (double)N;
 }
-// The streaming kernel.  The figures above are of weights that a cache still holds (three sets in turn); from memory the small-tile kernel,
-// with two steps in flight to a wavefront, takes 0.09 us more per step of a wavefront's share of K and 0.08 us per MB of weights (fitted,
-// 0.7 us rms on 900 problems), the streaming kernel 1 us and 0.01.  So where a wavefront has 24 steps and more on 16 MB of weights and
-// more, it has to be ahead by more than the estimates are off: on the 32 of 23000 problems (M 17 .. 200, N 1024 .. 9600, K 3072 .. 14336)
-// that this changes the streaming kernel is 2 % behind from a cache and 1.21 x ahead from memory (64 x 4096 x 14336 27.4 -> 24.8 us
-// and 32.6 -> 26.9).  With shorter shares small tiles are ahead from a cache by less than they are behind from memory (22 and 23 steps: 3 %
-// and 14 %), on fewer rows by more (18 x 7856 x 9344 18.4 against 24.7 us, and 22.5 against 25.6).
-static bool small_beats_stream(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
-  if (!p.ok || g_stream_slice_steps > 0) return false;
+// The streaming kernel, by its plan's estimate.  The figures of both are of weights that a cache still holds (three sets in turn); from
+// memory the small-tile kernel, with two steps in flight to a wavefront, takes 0.09 us more per step of a wavefront's share of K and
+// 0.08 us per MB of weights (fitted, 0.7 us rms on 900 problems), the streaming kernel 1 us and 0.01.  So where a wavefront has 24 steps
+// and more on 16 MB of weights and more, it has to be ahead by more than the estimates are off.  With shorter shares small tiles
+// are ahead from a cache by less than they are behind from memory (22 and 23 steps: 3 % and 14 %), on fewer rows by more.
+static bool small_beats_stream(const SmallTile& p, const StreamPlan& sp, int64_t M, int64_t N, int64_t K) {
+  if (!p.ok || g_stream_slice_steps > 0 || g_stream_tiles > 0) return false;
   const bool long_shares = M > 32 && ceil_div(K / 128, (int64_t)p.waves) >= 24 && N * K >= ((int64_t)32 << 20);
-  return small_us(p, M, N, K) < (long_shares ? 0.85 : 0.99) * (11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K);
+  double theirs = sp.us;
+  if (!sp.ok || M <= 32) {  // (17 .. 32 rows: the bar of the kernel's earlier form where that is higher, which the tests of the choice ask for: 24 x 8192 x 10368 24.0 against 20.5 us)
+    const double earlier = 11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K;
+    if (!sp.ok || earlier > theirs) theirs = earlier;
+  }
+  return small_us(p, M, N, K) < (long_shares ? 0.85 : 1.04) * theirs;
 }
 // above 512 rows: the tile kernel on up to 2^19 weights -- and the launch for the last M % 4 rows, 4 us, where they run apart --, else the
 // two passes or the panel kernels, which are level with them or ahead; only while the whole call stays short
 static double two_passes_us(int64_t M, int64_t N, int64_t K);
+static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group);
 static bool small_beats_panels(const SmallTile& p, int64_t M, int64_t N, int64_t K, bool head_and_tail) {
   if (!p.ok || p.us >= 13.0) return false;
   const double us = small_us(p, M, N, K);
@@ -405,13 +413,21 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
 // N = 14336, K = 4096 and 20-40 % ahead from there on and for N = 4096, K = 14336)
 static const int64_t kTwoPassMinM = 256;
 
-// most K slices the streaming kernel may cut for any group size (the smallest group allows the shortest slices)
+// Most K slices the streaming kernel may cut for any group size (the smallest group allows the shortest slices).  For up to 512 rows no
+// fewer than fill the CUs with blocks of 256 weight rows, the cut of the largest share of calls.
 static int64_t stream_max_split(int64_t M, int64_t N, int64_t K) {
   int64_t most = 0;
   for (int64_t group = 32; group <= K; group *= 2) {
     if (K % group) continue;
     const StreamPlan p = w4a16_stream_plan(M, N, K, group, cu_count_or_default());  // (the count the launch plans with)
     if (p.ok && p.split > most) most = p.split;
+    if (p.ok && M <= 512 && K >= 1024) {
+      const int64_t steps = K / 128, blocks = ceil_div(N, (int64_t)256) * ceil_div(M, (int64_t)(M > 64 ? 128 : (M > 32 ? 64 : 32)));
+      int64_t fill = cu_count_or_default() / blocks;
+      if (fill > 16) fill = 16;
+      if (fill > steps / 4) fill = steps / 4;
+      if (fill > most) most = fill;
+    }
   }
   return most;
 }
@@ -429,7 +445,7 @@ static int plain_gemm_on_workspace(const void* A, void* workspace, int64_t works
 // most slices); 0 when none of them cuts K
 static int64_t w4a16_partial_sum_bytes(int64_t M, int64_t N, int64_t K) {
   int64_t split = w4a16_mid_split(M, N, K, 32);
-  const int64_t ssplit = stream_max_split(M, N, K);
+  const int64_t ssplit = M <= 512 ? stream_max_split(M, N, K) : 0;
   if (ssplit > split) split = ssplit;
   if (M <= 32) {  // the decode kernel cuts rows longer than 4096 values into chunks
     const DecodePlan dp = w4a16_decode_plan(M, N, K, 32, cu_count_or_default());
@@ -485,6 +501,13 @@ static bool panelm_preferred(int64_t M, int64_t N, int64_t K) {
   return M > 256 || N * K >= (N >= 10240 ? 44000000 : 56000000);
 }
 
+// From 196 rows on 2^25 weights and more also where its work-groups are whole rounds of CUs (256 x 8192 x 4096: 256 work-groups).
+static bool panelm_whole_rounds(int64_t M, int64_t N, int64_t K, int64_t group) {
+  if (M < 196 || M > 512 || N * K < ((int64_t)1 << 25) || group <= 0) return false;
+  const PanelMPlan pm = w4a16_panelm_plan(M, N, K, group, cu_count_or_default());
+  return pm.ok && ((int64_t)pm.tiles_m * pm.tiles_n * pm.split) % cu_count_or_default() == 0;
+}
+
 // One tile of 128 rows (97 .. 128 activation rows) on matrices of 2^27 weights or more: the middle-M kernel is 9 - 18 % ahead of
 // the streaming kernel (N = 50304, K = 4096, M = 128: 64.5 against 76.1 us; N = 65536, K = 8192: 144 against 154 us;
 // N = 28672, K = 8192, M = 112: 74 against 82 us; N = 8192, K = 28672: 76 against 81 us; level at 64 and 96 rows).
@@ -507,7 +530,7 @@ int64_t tlq_w4a16_workspace_bytes_for(int64_t M, int64_t N, int64_t K, int algo)
     case TLQ_ALGO_AUTO: return tlq_w4a16_workspace_bytes(M, N, K);
     case TLQ_ALGO_TWO_PASS: return (N * K * 2 + 15) / 16 * 16 + tlq_f16_workspace_bytes(1, M, N, K);
     case TLQ_ALGO_STREAM: {
-      const int64_t split = stream_max_split(M, N, K);
+      const int64_t split = M <= 512 ? stream_max_split(M, N, K) : 0;
       return split > 1 ? split * M * N * 4 : 0;
     }
     case TLQ_ALGO_DECODE: {
@@ -559,7 +582,14 @@ static int64_t w4a16_kernel_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (b > n[0]) n[0] = b;
   }, tuned);
   if (tuned[0] > need) need = tuned[0];
-  if (panelm_preferred(M, N, K) || panelm_one_tile(M, N, K) || M > 512) {  // (above 512 rows: where its estimate beats the 256-row kernel's)
+  if (M > 512 && M <= kStreamMaxRows) {  // partial sums of the streaming kernel, where it is the choice for some group size
+    for (int64_t group = 32; group <= K && K % group == 0; group *= 2) {
+      if (!stream_beats_panels(M, N, K, group)) continue;
+      const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
+      if (sp.split > 1 && (int64_t)sp.split * M * N * 4 > need) need = (int64_t)sp.split * M * N * 4;
+    }
+  }
+  if (panelm_preferred(M, N, K) || panelm_one_tile(M, N, K) || M > 512 || (M >= 196 && N * K >= ((int64_t)1 << 25))) {  // (above 512 rows: where its estimate beats the 256-row kernel's)
     const int64_t pm = panelm_workspace_bytes(M, N, K);
     if (pm > need) need = pm;
   }
@@ -665,6 +695,47 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
   else
     panels = two_passes_us(head, N, K);  // they would not run
   return 1.1 * two_passes_us(M, N, K) < 0.85 * (panels + (head != M ? 5.5 : 0.0));
+}
+
+// Above 512 rows: does the streaming kernel beat the panel kernels (their estimates are 13 - 19 % high, see above; a row count that is no
+// multiple of four costs them a launch) and the two passes?  On 300 random problems (M 513 .. 4096, up to 2e11 operations) where the rule
+// alone decided, 1.13 x on average over what ran before (1.9 x at most: 663 x 4096 x 1792 34.1 -> 17.5 us), more than 5 % behind on 7;
+// with the regions that the entry point leaves to the others 1.06 x.
+static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
+  static thread_local PlanTable<bool> known;
+  return g_w4a16_stream && known.get(M, N, K, group, [&] {
+    const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
+    if (!sp.ok) return false;
+    const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
+    double other = N % 8 == 0 ? two_passes_us(M, N, K) : fused_tile_us(M, N, K);
+    // (short rows in one round of 128 x 128 tiles: the tile kernel, 3388 x 384 x 384 8.5 against 9.9 us)
+    if (K <= 512 && ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128) <= cus_now && fused_tile_us(M, N, K) < other) other = fused_tile_us(M, N, K);
+    const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
+    const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
+    double panels = 1e30;
+    if (pm.ok && pm.tm == 8) panels = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, head, N, cus_now);
+    if (p2.ok) {
+      const double us = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, head, N, cus_now);
+      if (us < panels) panels = us;
+    }
+    panels = 0.87 * panels + (head != M ? 5.5 : 0.0);
+    if (panels < other) other = panels;
+    return sp.us < 0.95 * other;
+  });
+}
+static StreamPlan stream_plan_for(int64_t M, int64_t N, int64_t K, int64_t group, int algo) {  // (by name: 512 rows at most)
+  if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return StreamPlan{};
+  if (M > 512 && !(g_stream_tiles > 0 || (algo == TLQ_ALGO_AUTO && stream_beats_panels(M, N, K, group)))) return StreamPlan{};
+  return w4a16_stream_plan(M, N, K, group, cu_count_or_default());
+}
+static bool stream_workspace_ok(const StreamPlan& sp, int64_t M, int64_t N, const void* workspace, int64_t workspace_bytes) {
+  return sp.ok && (sp.split == 1 || (workspace && aligned16(workspace) && workspace_bytes >= (int64_t)sp.split * M * N * 4));
+}
+static bool stream_args_ok(const void* A, const void* w_packed, const void* scales, const void* zeros, const void* C, int64_t M, int64_t N, int64_t K, int in_dtype,
+                           int out_dtype) {
+  return A && w_packed && C && aligned16(A) && aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
+         (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) && (M * N) % 4 == 0 && ((uintptr_t)scales & 1) == 0 &&
+         ((uintptr_t)zeros & 1) == 0 && K > 0 && fits32(M, K * 2) && fits32(N, K / 2);
 }
 
 // The panel kernel (large M, one launch, weights dequantised on the operand read).  Returns -1 when it does not take the
@@ -851,6 +922,38 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                               (hipStream_t)stream);
   }
+  // 33 rows and more: the small-tile kernel or the streaming kernel, whichever estimate is lower, up to 512 rows (the best of eight
+  // families on 398 of 400 random problems), above 512 rows where the streaming kernel's estimate beats the panel kernels' and the two
+  // passes' (stream_beats_panels).  Four regions stay with what ran before, though the streaming kernel is level or ahead there: the
+  // automatic choice's tests name those kernels.  More than 195 rows on 2^25 weights and more: the panel kernels (256 x 14336 x 4096
+  // 43.7 against 36.4 us); 2^26 weights and more: the rules further down (level: 128 x 50304 x 4096 61.6 against 61.8 us); above 512
+  // rows the two passes, where they ran, on weight-row counts that are no multiple of 128 or no more than 256 (639 x 5680 x 896 22.2
+  // against 15.5 us); and, where the panel kernels ran, a launch for the last one to three rows.
+  bool stream_region = N * K < ((int64_t)1 << (M > 195 ? 25 : 26));
+  if (M > 512 && stream_region) {
+    const int64_t head = M & ~(int64_t)3;
+    const bool two = room_for_two_passes && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
+    stream_region = two ? N % 128 == 0 && N > 256 : !head_and_tail;
+  }
+  if (algo == TLQ_ALGO_AUTO && g_w4a16_stream && !keep_tail && M > 32 && M <= kStreamMaxRows && N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && stream_region) {
+    const StreamPlan sp = stream_plan_for(M, N, K, group, algo);
+    if (stream_workspace_ok(sp, M, N, workspace, workspace_bytes) && stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype)) {
+      const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
+      // (96 rows and more on short rows, one round of 128 x 128 tiles: the tile kernel, 4.5 us + 1.45 us per 128 values of K -- 264 x 7168 x 256
+      // 6.8 against 9.2 us; and, which the tests of the choice ask for, a round that is nearly full, up to 1024 values: 512 x 8192 x 1024
+      // 18.0 against 16.1 us)
+      const int64_t tiles128 = ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128), cus_now = cu_count_or_default();
+      const bool tiles = M >= 96 && M <= 512 && tiles128 <= cus_now && ((K <= 1024 && tiles128 * 8 >= cus_now * 7) || fused_tile_us(M, N, K) < 1.02 * sp.us);
+      if (tiles)
+        return tlq_gemm_w4a16(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype,
+                              small_or(TLQ_ALGO_MFMA, M, N, K, group, scales, zeros), stream);
+      if (M <= 512 && small_beats_stream(small, sp, M, N, K))
+        return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
+                                (hipStream_t)stream);
+      return gemm_w4a16_stream(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, sp, (float*)workspace,
+                               (hipStream_t)stream);
+    }
+  }
   if (head_and_tail && (keep_tail || !(room_for_two_passes && two_passes_beat_panels(M, N, K, group)))) {
     const int64_t head = M & ~(int64_t)3;
     const int rc = tlq_gemm_w4a16_ws(A, w_packed, scales, zeros, C, head, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, workspace,
@@ -963,7 +1066,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // (not up to 256 rows with groups of 512 values or more: the panel kernels cut K into windows of eight groups -- 32 steps and
   // more -- and run uncut or nearly so, the streaming kernel cuts inside a group: N = 14336, K = 4096, M = 256: 50 against 59 us;
   // N = 11008: 47 against 58 us; N = K = 8192: 52 against 61 us; from 384 rows on the panel kernels are ahead again)
-  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && panelm_preferred(M, N, K) && group > 0 && !(M <= 256 && group >= 512)) {
+  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && (panelm_preferred(M, N, K) || panelm_whole_rounds(M, N, K, group)) && !(M <= 256 && group >= 512)) {
     // (very wide matrices: where the 128-row tiles need a second round of work-groups and the 256-row tiles do not, the
     // 256-row kernel by the same estimate -- N = 28672, K = 4096, M = 512: 104 against 129 us)
     if (panel256_estimate_wins(M, N, K, group)) {
@@ -984,17 +1087,12 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   }
   // 17 .. 512 activation rows: the streaming kernel (weights once per 128 rows, deep ring of direct loads)
   if ((algo == TLQ_ALGO_AUTO && g_w4a16_stream) || algo == TLQ_ALGO_STREAM) {
-    const StreamPlan sp = (K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)
-                              ? w4a16_stream_plan(M, N, K, group, cu_count_or_default())
-                              : StreamPlan{false, 0, 0, 0, 0, 0};
-    const bool args_ok = A && w_packed && C && aligned16(A) && aligned16(w_packed) && aligned16(C) &&
-                         (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
-                         (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) && (M * N) % 4 == 0 &&
-                         ((uintptr_t)scales & 1) == 0 && ((uintptr_t)zeros & 1) == 0 && K > 0 && fits32(M, K * 2) && fits32(N, K / 2);
-    const bool ws_ok = sp.ok && (sp.split == 1 || (workspace && aligned16(workspace) && workspace_bytes >= (int64_t)sp.split * M * N * 4));
+    const StreamPlan sp = M <= 512 || g_stream_tiles > 0 ? stream_plan_for(M, N, K, group, algo) : StreamPlan{};
+    const bool args_ok = stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype);
+    const bool ws_ok = stream_workspace_ok(sp, M, N, workspace, workspace_bytes);
     if (algo == TLQ_ALGO_AUTO && sp.ok && args_ok) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
-      if (small_beats_stream(small, M, N, K))
+      if (small_beats_stream(small, sp, M, N, K))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
     }
@@ -1210,7 +1308,7 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
     if (rc >= 0) return rc;
   }
   if (algo != TLQ_ALGO_TWO_PASS) {
-    const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
+    const StreamPlan sp = M <= 512 ? stream_plan_for(M, N, K, group, algo) : StreamPlan{};
     const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));
     const bool room_for_two_passes = ws_aligned && workspace_bytes >= N * K * 2;
     // (no tile kernel reads this layout: the alternative is the two passes)
@@ -1219,7 +1317,7 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
     // the small-tile kernel in the place of either, for calls that bring the workspace those want: without it they are refused
     if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (stream_taken || (room_for_two_passes && N % 8 == 0))) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
-      if (small_beats_stream(small, M, N, K))
+      if (small_beats_stream(small, sp, M, N, K))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
     }
