@@ -199,6 +199,12 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
       for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[tn][tb][i] = 0.0f;
+    if constexpr (TB <= 2 && !MANY) {  // (made here and not where they are first used)
+#pragma unroll
+      for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) asm volatile("" : "+v"(acc[tn][tb]));
+    }
   };
   StreamMagic mg;
   static_cast<NibbleMagic&>(mg) = make_nibble_magic();
@@ -270,15 +276,14 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
         if (has_z && my_z) dma4(l_sz + (uint32_t)(Cfg::SZ / 2 + i * 256), voff, (const uint8_t*)zeros);
       }
     }
+    // Two steps now, the rest behind the barrier: a CU takes the loads in at 64 bytes a cycle, and the wavefronts that issue them wait for
+    // that -- with the whole ring ahead of the barrier step 0 had long landed when they got there (2200 - 4700 cycles to issue).
 #pragma unroll
-    for (int s = 0; s < D; ++s)
-      static_for<0, Cfg::L>([&](auto ic) {
-        if (s < D - 1 || decltype(ic)::value < Cfg::LB) issue1(w0 + s, w0 + wsteps, s, ic);
-      });
+    for (int s = 0; s < 2; ++s) static_for<0, Cfg::L>([&](auto ic) { issue1(w0 + s, w0 + wsteps, s, ic); });
     __builtin_amdgcn_sched_barrier(0);
     if (wide || dwords) {
-      // loads return in issue order: with the ring's loads still in flight the scales have landed
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * Cfg::L + Cfg::LB) : "memory");
+      // loads return in issue order: with the two steps' loads still in flight the scales have landed
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * Cfg::L) : "memory");
       if (!has_s || !has_z) {  // an absent tensor is the constant 1 / the scalar zero point
         const uint32_t ws = (uint32_t)bitcast<uint16_t>(one) * 0x10001u, wz = (uint32_t)bitcast<uint16_t>(zs) * 0x10001u;
         const uint4_t cs{ws, ws, ws, ws}, cz{wz, wz, wz, wz};
@@ -317,11 +322,17 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
           if (my_z) *(T*)(sz + Cfg::SZ / 2 + addr::stream_sz_value(MG, tn * 16 + r16, g) * 2) = pre_z[tn][i];
         }
     }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 2) * Cfg::L + Cfg::LB) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Cfg::L) : "memory");
     __syncthreads();  // the window's scales and its step 0 are complete for every wavefront
+#pragma unroll
+    for (int s = 2; s < D; ++s)
+      static_for<0, Cfg::L>([&](auto ic) {
+        if (s < D - 1 || decltype(ic)::value < Cfg::LB) issue1(w0 + s, w0 + wsteps, s, ic);
+      });
     // small integer zero points fold exactly into the unpack bias (a quarter of the conversion arithmetic less); decided
     // once per wavefront and window, on the zero points of the 64 rows it multiplies
-    bool integral = true;
+    uint32_t fraction = 0;  // not zero for a fraction or a NaN
+    float largest = 0.0f;
 #pragma unroll
     for (int p = 0; p < 2 * (MG / 16); ++p) {
       const uint4_t v = *(const uint4_t*)(sz_read + (p & 1) * Cfg::SZ + Cfg::SZ / 2 + (p >> 1) * 1024 + lane * 16);
@@ -331,9 +342,11 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const float zf = to_float(bitcast<T>((uint16_t)(w[i] >> (16 * e))));
-          integral = integral && zf == __builtin_rintf(zf) && zf >= -256.0f && zf <= 256.0f;
+          fraction |= bitcast<uint32_t>(__builtin_amdgcn_fractf(zf));
+          largest = __builtin_fmaxf(largest, __builtin_fabsf(zf));
         }
     }
+    const bool integral = fraction == 0 && largest <= 256.0f;
     return __builtin_amdgcn_ballot_w64(integral) == ~0ull;
   };
   // The steps of a window.  A wavefront's step is eight units of TB MFMAs (unit u: k-step u / 2 of its four, weight tile u % 2).
@@ -411,8 +424,9 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
   // One copy of the loops per dequantiser: a choice inside a loop would make the two paths meet with the accumulators
   // in different registers.
   if constexpr (!MANY) {
+    if constexpr (TB <= 2) clear();  // (while the first loads are on their way; more sums would not stay in registers across them)
     const bool fold = fetch(0, steps);
-    clear();
+    if constexpr (TB > 2) clear();
     if (fold)
       multiply(0, steps, std::true_type{});
     else
