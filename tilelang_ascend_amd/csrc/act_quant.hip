@@ -2,7 +2,7 @@
 //   amax[m]  = max(max_n |x[m, n]|, 1e-4)
 //   scale[m] = amax / 127                      (round_scale: the next power of two, 2^ceil(log2(amax / 127)))
 //   y[m, n]  = int8( rint( clamp(x[m, n] / scale[m], -127, 127) ) )      rint = round half to even
-// HBM bound: one wavefront (many rows) or one work-group (few or long rows) owns a row, reads it once
+// HBM bound: one wavefront (many rows), one work-group (long rows) or several (few long rows) own a row, reads it once
 // into registers with 16-byte loads, reduces the maximum across lanes, and writes 8 int8 per lane and
 // chunk.  Rows longer than 32768 values, or of a length that is no multiple of 8, are read twice.
 #include "tlq_common.h"
@@ -15,7 +15,8 @@ __device__ __forceinline__ float to_float<float>(float v) {
 }
 
 // Eight consecutive values, kept as loaded (16 or 32 bytes) and widened to float on use.  The input is read once:
-// non-temporal loads (M = 16384, N = 4096: 38.2 instead of 40.0 us; with the resident grid 36.1 us).  The output is
+// non-temporal loads (M = 16384, N = 4096: 38.2 instead of 40.0 us; with the resident grid 36.1 us) -- but for load_shared, whose
+// values other work-groups read too.  The output is
 // stored normally: non-temporal stores save another microsecond here and cost the W8A8 GEMM that reads the output next
 // 4 - 14 us (16384 x 4096 x 4096: quantiser + GEMM 291 against 279 us).
 template <typename T>
@@ -24,6 +25,7 @@ template <>
 struct Raw8<half_t> {
   half8_t v;
   __device__ __forceinline__ void load(const half_t* p) { v = __builtin_nontemporal_load((const half8_t*)p); }
+  __device__ __forceinline__ void load_shared(const half_t* p) { v = *(const half8_t*)p; }
   __device__ __forceinline__ float get(int i) const { return (float)v[i]; }
 };
 template <>
@@ -31,6 +33,10 @@ struct Raw8<bf16_t> {
   uint32_t w[4];
   __device__ __forceinline__ void load(const bf16_t* p) {
     const uint4_t q = __builtin_nontemporal_load((const uint4_t*)p);
+    w[0] = q.x, w[1] = q.y, w[2] = q.z, w[3] = q.w;
+  }
+  __device__ __forceinline__ void load_shared(const bf16_t* p) {
+    const uint4_t q = *(const uint4_t*)p;
     w[0] = q.x, w[1] = q.y, w[2] = q.z, w[3] = q.w;
   }
   __device__ __forceinline__ float get(int i) const {
@@ -44,6 +50,7 @@ struct Raw8<float> {
     a = __builtin_nontemporal_load((const float4_t*)p);
     b = __builtin_nontemporal_load((const float4_t*)(p + 4));
   }
+  __device__ __forceinline__ void load_shared(const float* p) { a = *(const float4_t*)p, b = *(const float4_t*)(p + 4); }
   __device__ __forceinline__ float get(int i) const { return i < 4 ? a[i] : b[i - 4]; }
 };
 
@@ -72,6 +79,14 @@ __device__ __forceinline__ uint32_t quant1(float x, float scale, float rcp) {
   const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, scale, x), rcp, q0);
   const float q = __builtin_rintf(fminf(fmaxf(q1, -127.0f), 127.0f));
   return (uint32_t)(int)q & 0xffu;
+}
+
+template <typename R>
+__device__ __forceinline__ uint2_t quant8(const R& r, float scale, float rcp) {
+  uint2_t o;
+  o.x = quant1(r.get(0), scale, rcp) | quant1(r.get(1), scale, rcp) << 8 | quant1(r.get(2), scale, rcp) << 16 | quant1(r.get(3), scale, rcp) << 24;
+  o.y = quant1(r.get(4), scale, rcp) | quant1(r.get(5), scale, rcp) << 8 | quant1(r.get(6), scale, rcp) << 16 | quant1(r.get(7), scale, rcp) << 24;
+  return o;
 }
 
 // N % 8 == 0.  WPR wavefronts of a 256-lane work-group share one row (1: four rows per work-group,
@@ -115,15 +130,48 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const T* __restrict
     for (int c = 0; c < CH; ++c) {
       const int ci = c * lanes + sub * 64 + lane;
       if (live && ci < chunks) {
-        uint2_t o;
-        o.x = quant1(r[c].get(0), scale, rcp) | quant1(r[c].get(1), scale, rcp) << 8 | quant1(r[c].get(2), scale, rcp) << 16 |
-              quant1(r[c].get(3), scale, rcp) << 24;
-        o.y = quant1(r[c].get(4), scale, rcp) | quant1(r[c].get(5), scale, rcp) << 8 | quant1(r[c].get(6), scale, rcp) << 16 |
-              quant1(r[c].get(7), scale, rcp) << 24;
-        *(uint2_t*)(y + ci * 8) = o;  // plain store: the GEMM that follows finds the output in the last-level cache
+        *(uint2_t*)(y + ci * 8) = quant8(r[c], scale, rcp);  // plain store: the GEMM that follows finds the output in the last-level cache
       }
     }
   }
+}
+
+// Few long rows: `parts` work-groups (grid y) per row.  Each reads the whole row for its maximum -- from L2 for all but the first, and two
+// vector instructions a value -- and quantises chunks part, part + parts, ... of 8 values, ten instructions a value, one or
+// two chunks per lane.  One work-group per row left seven of eight CUs idle at M = 32 and each of its lanes 56 values of both kinds:
+// 32 x 14336 bf16 4.1 -> 2.9 us, 128 x 16384 7.1 -> 3.6, 256 x 14336 7.1 -> 4.6 and, on rows of one chunk per lane, 512 x 4096 3.9 -> 3.4 (back to
+// back in a graph); from three rows per CU on it is level, from four long ones behind (1000 x 14336 11.2 against 11.6).
+template <typename T, int CH, int OC>
+__global__ __launch_bounds__(512) void act_quant_parts_kernel(const T* __restrict__ X, int8_t* __restrict__ Y, float* __restrict__ S, int N, int round_scale) {
+  __shared__ float part[8];
+  const int tid = threadIdx.x, chunks = N >> 3;
+  const int64_t m = blockIdx.x;
+  const T* x = X + m * N;
+  const int parts = (int)gridDim.y, own = tid * parts + (int)blockIdx.y;  // the first of the lane's chunks
+  Raw8<T> r[CH], mine[OC];
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if (c * 512 + tid < chunks) r[c].load_shared(x + (c * 512 + tid) * 8);
+#pragma unroll
+  for (int c = 0; c < OC; ++c)
+    if (c * 512 * parts + own < chunks) mine[c].load_shared(x + (c * 512 * parts + own) * 8);
+  float amax = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if (c * 512 + tid < chunks)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(r[c].get(i)));
+  amax = wave_max(amax);
+  if ((tid & 63) == 0) part[tid >> 6] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 8; ++w) amax = fmaxf(amax, part[w]);
+  const float scale = row_scale(amax, round_scale);
+  if (tid == 0 && blockIdx.y == 0) S[m] = scale;
+  const float rcp = 1.0f / scale;
+#pragma unroll
+  for (int c = 0; c < OC; ++c)
+    if (c * 512 * parts + own < chunks) *(uint2_t*)(Y + m * N + (c * 512 * parts + own) * 8) = quant8(mine[c], scale, rcp);
 }
 
 // Any N: two passes over the row, one value per lane and step.
@@ -176,6 +224,24 @@ static int run_act_quant(const void* Xv, void* Yv, void* Sv, int64_t M, int64_t 
   if (vec) {
     // one wavefront per row while a lane then holds at most 8 chunks and there are rows enough to
     // fill the chip that way; otherwise the four wavefronts of a work-group split the row
+    int cus = tlq_device_cu_count();
+    if (cus <= 0) cus = 256;
+    int parts = 8;
+    while (parts > 1 && M * parts > cus) parts /= 2;
+    const int64_t chunks = N / 8;
+    if (M <= (int64_t)2 * cus && N >= 4096 && chunks <= 512 * 4) {
+      const dim3 grid((unsigned)M, (unsigned)parts);
+      const int own = (int)ceil_div(chunks, (int64_t)512 * parts);
+#define TLQ_AQP(CH, OC) act_quant_parts_kernel<T, CH, OC><<<grid, 512, 0, st>>>(X, Y, S, (int)N, round_scale)
+      if (chunks <= 512)
+        TLQ_AQP(1, 1);
+      else if (chunks <= 1024)
+        own == 1 ? TLQ_AQP(2, 1) : TLQ_AQP(2, 2);
+      else
+        own == 1 ? TLQ_AQP(4, 1) : (own == 2 ? TLQ_AQP(4, 2) : TLQ_AQP(4, 4));
+#undef TLQ_AQP
+      return check_launch("tlq_act_quant_i8", "act_quant kernel") ? 0 : 1;
+    }
     const int per_lane1 = (int)ceil_div(N, (int64_t)512);
     const int cap1 = sizeof(T) == 4 ? 4 : 8;
     if (per_lane1 <= cap1 && M >= 4096)
