@@ -63,11 +63,11 @@ SmallTile small_tile_plan(int kind, int64_t batch, int64_t M, int64_t N, int64_t
 }
 bool small_tile_forced() { return g_small_tiles > 0; }
 
-template <class Mma, SmallW W, class Epi, int RT, int MT>
+template <class Mma, SmallW W, class Epi, int RT, int MT, bool TIMES16>
 static int launch_one(const SmallParams& p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, int waves, const char* what, hipStream_t st) {
   typedef SmallCfg<W, RT, MT> Cfg;
   static_assert(Cfg::LDS == small_lds(W, RT, MT), "the plan's LDS");
-  auto kern = gemm_small_kernel<Mma, W, Epi, RT, MT>;
+  auto kern = gemm_small_kernel<Mma, W, Epi, RT, MT, TIMES16>;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -82,10 +82,10 @@ static int launch_one(const SmallParams& p, const typename Epi::Params& pe, int6
   return check_launch(what, "gemm_small_kernel") ? 0 : 1;
 }
 
-template <class Mma, SmallW W, class Epi>
+template <class Mma, SmallW W, class Epi, bool TIMES16 = false>
 static int launch_tile(const SmallTile& t, const SmallParams& p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, const char* what, hipStream_t st) {
 #define TLQ_ONE(RT, MT) \
-  if (t.rt == RT && t.mt == MT) return launch_one<Mma, W, Epi, RT, MT>(p, pe, batch, M, N, t.waves, what, st);
+  if (t.rt == RT && t.mt == MT) return launch_one<Mma, W, Epi, RT, MT, TIMES16>(p, pe, batch, M, N, t.waves, what, st);
   if constexpr (W == kSmallNK || W == kSmallW4) {
     TLQ_ONE(1, 1) TLQ_ONE(2, 1) TLQ_ONE(1, 2) TLQ_ONE(2, 2) TLQ_ONE(1, 4) TLQ_ONE(2, 4)
   }
@@ -118,6 +118,8 @@ int small_w4a8(const SmallTile& t, const void* A, const void* Wp, void* C, int64
   EpiInt32::Params pe{(int32_t*)C, N, M * N};
   SmallParams p = small_params(A, Wp, M, N, K, K / 2, 0);
   p.sign_mode = sign_mode;
+  if ((sign_mode == TLQ_S4_TWOS || sign_mode == TLQ_S4_OFFSET8) && K <= kTimes16MaxK)
+    return launch_tile<MmaI8, kSmallW4, EpiInt32, true>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
   return launch_tile<MmaI8, kSmallW4, EpiInt32>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
 }
 
