@@ -1397,8 +1397,16 @@ static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, in
 // The products that may take the small-tile kernel: weights as stored (the first four: SmallW), int32 results, or rescaled ones
 // (W8A8), W4A8 where the caller brought the room to unpack the weights first (65 to 256 rows: above, that is what runs; the figures
 // below count such problems of any number of rows).
-enum SmallUse { kUseI8NK = kSmallNK, kUseI8KN = kSmallKN8, kUseF16KN = kSmallKN16, kUseW4A8 = kSmallW4, kUseW4A8TwoSteps = 4, kUseW8A8NK = 5, kUseW8A8KN = 6 };
-static SmallW small_weights(SmallUse use) { return use == kUseW8A8NK ? kSmallNK : use == kUseW8A8KN ? kSmallKN8 : use == kUseW4A8TwoSteps ? kSmallW4 : (SmallW)use; }
+enum SmallUse { kUseI8NK = kSmallNK, kUseI8KN = kSmallKN8, kUseF16KN = kSmallKN16, kUseW4A8 = kSmallW4, kUseW4A8TwoSteps = 4, kUseW8A8NK = 5, kUseW8A8KN = 6,
+                // the two of W4A8 with weights multiplied as 16 times their value
+                kUseW4A8Times16 = 7, kUseW4A8TwoStepsTimes16 = 8 };
+static SmallW small_weights(SmallUse use) {
+  return use == kUseW8A8NK ? kSmallNK : use == kUseW8A8KN ? kSmallKN8 : use == kUseW4A8TwoSteps || use >= kUseW4A8Times16 ? kSmallW4 : (SmallW)use;
+}
+static SmallUse w4a8_use(bool two_steps, int sign_mode, int64_t K) {
+  if (small_w4a8_times16(sign_mode, K)) return two_steps ? kUseW4A8TwoStepsTimes16 : kUseW4A8Times16;
+  return two_steps ? kUseW4A8TwoSteps : kUseW4A8;
+}
 // Is the small-tile kernel ahead of what would run in its place?  Two things its own estimate leaves out come on top: the activations' trip from
 // memory (at 2.5 TB/s: every tile of weight rows asks for them again) and, with 16-bit weights, that theirs cannot take less than
 // a copy.  The other side, by what would run: calls that cut K into slices over work-groups (sliced_us), up to 32 rows a fit to the 32-row
@@ -1411,7 +1419,7 @@ static SmallW small_weights(SmallUse use) { return use == kUseW8A8NK ? kSmallNK 
 struct SmallBars {
   double few_sliced, sliced, few, plain, groups;
 };
-static constexpr SmallBars kSmallBars[7] = {
+static constexpr SmallBars kSmallBars[9] = {
     // <= 32 rows, K slices   K slices   <= 32 rows   tiles   tiles with K in groups
     {0.84, 1.5, 1.15, 1.03, 0.92},  // int8 [N, K]
     {0.74, 1.05, 1.05, 1.0, 1.0},   // int8 [K, N]
@@ -1419,7 +1427,9 @@ static constexpr SmallBars kSmallBars[7] = {
     {1.04, 1.0, 0.93, 0.93, 0.93},  // W4A8
     {1.04, 1.0, 0.93, 1.0, 1.0},    // W4A8 in two steps
     {0.84, 0.95, 1.12, 0.9, 0.88},  // W8A8 [N, K]
-    {0.74, 0.9, 1.0, 0.88, 0.92}};  // W8A8 [K, N]
+    {0.74, 0.9, 1.0, 0.88, 0.92},   // W8A8 [K, N]
+    {1.04, 1.0, 0.93, 0.93, 0.93},  // W4A8 times 16
+    {1.04, 1.0, 0.93, 1.0, 1.0}};   // the same in two steps
 static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int64_t M, int64_t N, int64_t K) {
   if (!t.ok || small_tile_forced()) return t.ok;
   const SmallW w = small_weights(use);
@@ -1435,7 +1445,7 @@ static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int
   if (packed ? M <= 256 && slice_choice(M, N, k_bytes, true, 2.5, 0) > 1
              : batch == 1 && slice_choice(M, N, k_bytes, !adds, 1.0, 0) > 1 && !groups_beat_slices(tile, w, M, N, K, k_bytes))
     return us < (M <= 32 ? bar.few_sliced : bar.sliced) * sliced_us(w, batch, M, N, K);
-  if (packed && use != kUseW4A8TwoSteps) return us < bar.few * (4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
+  if (packed && use != kUseW4A8TwoSteps && use != kUseW4A8TwoStepsTimes16) return us < bar.few * (4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
   if (M <= 32 && w == kSmallNK) return us < bar.few * (5.1 + 1.4 * g + 0.16 * mn + 2.07 * k);
   if (M <= 32 && w == kSmallKN8) return us < bar.few * (4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32);
   if (M <= 32 && w == kSmallKN16) return us < bar.few * (3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * (double)batch * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6);
@@ -1452,8 +1462,8 @@ static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t 
   const SmallTile t{false, 0, 0, 0, 0.0};
   if (batch < 1 || M < 1 || N < 1 || K < 128 || K % 128 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_i8_tile || g_i8_split) return t;
   static thread_local PlanTable<SmallTile> known;
-  return known.get(M, N, K, use + 8 * batch, [&] {
-    SmallTile p = small_tile_plan(small_weights(use), batch, M, N, K);
+  return known.get(M, N, K, use + 16 * batch, [&] {
+    SmallTile p = small_tile_plan(use >= kUseW4A8Times16 ? (int)kSmallW4Times16 : (int)small_weights(use), batch, M, N, K);
     p.ok = small_tile_wins(p, use, batch, M, N, K);
     return p;
   });
@@ -1622,7 +1632,7 @@ int tlq_gemm_w4a8(const void* A, const void* w_packed, void* C, int64_t M, int64
   TLQ_REQUIRE(A && w_packed && C, "tlq_gemm_w4a8: null pointer");
   TLQ_REQUIRE(aligned16(A) && aligned16(w_packed) && aligned16(C), "tlq_gemm_w4a8: pointers must be 16-byte aligned");
   TLQ_REQUIRE(fits32(M, K) && fits32(N, K / 2), "tlq_gemm_w4a8: a matrix spans 4 GiB or more");
-  if (const SmallTile t = small_tile_for_i8(1, M, N, K, kUseW4A8); t.ok) return small_w4a8(t, A, w_packed, C, M, N, K, sign_mode, (hipStream_t)stream);
+  if (const SmallTile t = small_tile_for_i8(1, M, N, K, w4a8_use(false, sign_mode, K)); t.ok) return small_w4a8(t, A, w_packed, C, M, N, K, sign_mode, (hipStream_t)stream);
   // few activation rows: K slices add into C (int32, exact in any order)
   if (const int split = i8_split_choice(1, M, N, K, false, 2.5); split > 1)
     return gemm_w4a8_i32_splitk(A, w_packed, C, M, N, K, sign_mode, split, nullptr, (hipStream_t)stream);
@@ -1642,7 +1652,7 @@ int tlq_gemm_w4a8_ws(const void* A, const void* w_packed, void* workspace, int64
   const bool two_steps = usable && workspace_bytes >= N * K && K % 16 == 0 && N % 16 == 0 && fits32(N, K) &&
                          (M > 64 || g_w4a8_ws_mode == 2);
   // (above 256 rows the caller finds the unpacked weights in a workspace that holds them, also where the small-tile kernel is faster)
-  if (g_w4a8_ws_mode == 0 && !(two_steps && M > 256) && small_tile_for_i8(1, M, N, K, two_steps ? kUseW4A8TwoSteps : kUseW4A8).ok)
+  if (g_w4a8_ws_mode == 0 && !(two_steps && M > 256) && small_tile_for_i8(1, M, N, K, w4a8_use(two_steps, sign_mode, K)).ok)
     return tlq_gemm_w4a8(A, w_packed, C, M, N, K, sign_mode, stream);
   if (usable && K % 32 == 0 && N % 4 == 0 && g_w4a8_ws_mode != 2 && (M <= 256 || g_w4a8_ws_mode == 1)) {
     int split = i8_split_choice(1, M, N, K, true, 2.5);

@@ -54,9 +54,8 @@ __device__ __forceinline__ uint2_t small_expand8(uint32_t v, int sign_mode) {
 }
 // Two's complement nibbles as int8 of 16 times their value -- a nibble in the upper half of its byte is its own sign extension: 5
 // instructions a word against 11 - 13 -- ; `flip` turns offset-8 nibbles into two's complement (u ^ 8 == u - 8).  The sums are
-// 16 times the result, and exact, while 16 x 8 x 128 K < 2^31.  Expanding was what bounded the tiles: 128 x 4096 x 11008 (86 steps per CU)
+// 16 times the result, and exact, while 16 x 8 x 128 K < 2^31 (small_w4a8_times16).  Expanding was what bounded the tiles: 128 x 4096 x 11008 (86 steps per CU)
 // 20.3 us before, 14.7 now; the other two conventions stay as they were.
-static constexpr int64_t kTimes16MaxK = 131071;
 __device__ __forceinline__ uint2_t small_expand8_times16(uint32_t v, uint32_t flip) {
   v ^= flip;
   const uint32_t lo = (v << 4) & 0xf0f0f0f0u, hi = v & 0xf0f0f0f0u;

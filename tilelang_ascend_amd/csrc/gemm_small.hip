@@ -16,19 +16,23 @@ static constexpr int small_lds(SmallW w, int rt, int mt) {
 // the weights' trip from memory -- once, and again for every further tile of activation rows.  Fitted per kind to 970 problems (M 1 .. 1500,
 // N 256 .. 14400, K 256 .. 14336, one to eight batches) x up to 45 forced variants each: 14 - 22 % rms over all variants; the
 // variant it picks is 4 - 5 % behind the fastest on average.
+// Packed int4 weights multiplied as 16 times their value (kSmallW4Times16) have a row of their own: the one before it is 1.37 x what they
+// take.  700 problems (M 1 .. 1500, N 256 .. 14336, K 256 .. 14336) x up to 36 variants, the adding of the wavefronts' tiles as a further term:
+// 11 % rms; 6.5 % for the variant it picks, which is 3.4 % behind the fastest on average (3.9 with the other row).
 struct SmallCost {
-  double launch, round, step, rt, rt_mt, store, again, weights;
+  double launch, round, step, rt, rt_mt, store, again, weights, sums;
 };
-static constexpr SmallCost kSmallCost[4] = {{3.4, 1.33, 0.049, 0.0028, 0.0092, 0.047, 0.19, 0.29},   // int8 [N, K] (rt: stands for mt here)
-                                            {2.4, 1.57, 0.112, 0.0, 0.0112, 0.080, 0.29, 1.35},      // int8 [K, N]
-                                            {1.75, 1.43, 0.085, 0.0045, 0.0106, 0.020, 0.22, 0.58},  // 16-bit [K, N]
-                                            {3.0, 0.71, 0.391, 0.0444, 0.0118, 0.046, 0.0, 0.0}};    // packed int4
+static constexpr SmallCost kSmallCost[5] = {{3.4, 1.33, 0.049, 0.0028, 0.0092, 0.047, 0.19, 0.29, 0.0},   // int8 [N, K] (rt: stands for mt here)
+                                            {2.4, 1.57, 0.112, 0.0, 0.0112, 0.080, 0.29, 1.35, 0.0},      // int8 [K, N]
+                                            {1.75, 1.43, 0.085, 0.0045, 0.0106, 0.020, 0.22, 0.58, 0.0},  // 16-bit [K, N]
+                                            {3.0, 0.71, 0.391, 0.0444, 0.0118, 0.046, 0.0, 0.0, 0.0},    // packed int4
+                                            {2.01, 0.815, 0.1635, 0.0058, 0.0086, 0.0339, 0.147, 0.344, 0.0159}};  // the same, times 16
 
 static SmallTile small_tile_now(int kind, int64_t batch, int64_t M, int64_t N, int64_t steps) {
   SmallTile best{false, 0, 0, 0, 0.0};
   int cus = tlq_device_cu_count();
   if (cus <= 0) cus = 256;
-  const SmallW w = (SmallW)kind;
+  const SmallW w = kind == kSmallW4Times16 ? kSmallW4 : (SmallW)kind;
   for (int mt = 1; mt <= 4; mt *= 2) {
     if (g_small_tiles > 0 ? mt != g_small_tiles / 10 : mt > 1 && mt * 8 >= M) continue;  // (half of the tile would be padding)
     for (int rt = 1; rt <= 4; rt *= 2) {
@@ -48,7 +52,7 @@ static SmallTile small_tile_now(int kind, int64_t batch, int64_t M, int64_t N, i
         const SmallCost& c = kSmallCost[kind];
         const double w_mb5 = (double)batch * (double)N * (double)steps * (w == kSmallW4 ? 64.0 : 128.0) / 5e6;  // us at 5 TB/s
         const double us = c.launch + rounds * (c.round + c.step * (double)ceil_div(steps, wv)) + per_cu * (c.rt * (w == kSmallNK ? mt : rt) + c.rt_mt * rt * mt) +
-                          c.store * (double)ceil_div(blocks, (int64_t)cus) * rt * mt + w_mb5 * (c.weights + c.again * (double)(tiles_m - 1));
+                          (c.store + (wv > 1 ? c.sums * (double)wv : 0.0)) * (double)ceil_div(blocks, (int64_t)cus) * rt * mt + w_mb5 * (c.weights + c.again * (double)(tiles_m - 1));
         if (!best.ok || us < best.us * 0.995) best = SmallTile{true, mt, rt, (int)wv, us};
       }
     }
@@ -118,7 +122,7 @@ int small_w4a8(const SmallTile& t, const void* A, const void* Wp, void* C, int64
   EpiInt32::Params pe{(int32_t*)C, N, M * N};
   SmallParams p = small_params(A, Wp, M, N, K, K / 2, 0);
   p.sign_mode = sign_mode;
-  if ((sign_mode == TLQ_S4_TWOS || sign_mode == TLQ_S4_OFFSET8) && K <= kTimes16MaxK)
+  if (small_w4a8_times16(sign_mode, K))
     return launch_tile<MmaI8, kSmallW4, EpiInt32, true>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
   return launch_tile<MmaI8, kSmallW4, EpiInt32>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
 }

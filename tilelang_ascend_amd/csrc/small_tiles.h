@@ -20,6 +20,9 @@ int gemm_w4a16_small(const void* A, const void* Wp, const void* scales, const vo
 
 // The int8, W4A8 and plain 16-bit products, by how their weights are stored
 enum SmallW { kSmallNK = 0 /* int8 [N, K] */, kSmallKN8 = 1 /* int8 [K, N] */, kSmallKN16 = 2 /* 16-bit [K, N] */, kSmallW4 = 3 /* packed int4 [N, K / 2] */ };
+// how the packed weights are multiplied (gemm_small.h); a kind of its own for small_tile_plan, which prices it
+enum { kSmallW4Times16 = 4 };
+inline bool small_w4a8_times16(int sign_mode, int64_t K) { return (sign_mode == TLQ_S4_TWOS || sign_mode == TLQ_S4_OFFSET8) && K <= 131071; }
 SmallTile small_tile_plan(int kind, int64_t batch, int64_t M, int64_t N, int64_t row_bytes);  // row_bytes: bytes of K in an activation row
 bool small_tile_forced();
 int small_i8(const SmallTile& t, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int b_layout, hipStream_t st);
