@@ -1,12 +1,14 @@
 """The small-tile kernel multiplies two's complement and offset-8 int4 weights as 16 times their value while 16 x 8 x 128 K fits 31
 bits: exact at the largest sums that allows, on either side of that length, with one wavefront and with several."""
 import ctypes
+import re
+import subprocess
 
 import pytest
 import torch
 
 from helpers import assert_bit_equal, gen
-from tilelang_ascend_amd import _abi
+from tilelang_ascend_amd import _abi, build
 
 
 @pytest.mark.gpu
@@ -32,3 +34,14 @@ def test_largest_sums(mode, low, M, N, K, waves, tiles):
         lib.tlq_tune_small(0, 0)
     torch.cuda.synchronize()
     assert_bit_equal(C.cpu(), want, f"W4A8 mode {mode} {M}x{N}x{K}")
+
+
+def test_no_register_spills(tmp_path):
+    cmd = [build.hipcc_path(), *build.HIPCC_FLAGS, "-Rpass-analysis=kernel-resource-usage", "-c", f"{build.CSRC_DIR}/gemm_small_w4a8.hip",
+           "-o", str(tmp_path / "out.o")]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout[-2000:]
+    blocks = [b for b in re.split(r"remark: Function Name: ", res.stdout)[1:] if "gemm_small_kernel" in b.split()[0]]
+    assert len(blocks) == 9
+    for b in blocks:
+        assert re.search(r"ScratchSize \[bytes/lane\]: 0\b", b) and re.search(r"VGPRs Spill: 0\b", b), b[:300]

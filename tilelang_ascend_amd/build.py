@@ -50,6 +50,7 @@ SOURCES = [
     "gemm_w4a16_decode.hip",
     "gemm_int8.hip",
     "gemm_small.hip",
+    "gemm_small_w4a8.hip",
     "gemm_f16.hip",
     "gemm_api.hip",
     "gemm_addr_check.hip",

@@ -249,4 +249,48 @@ __global__ __launch_bounds__(RT* MT <= 4 ? 1024 : 512) void gemm_small_kernel(Sm
   }
 }
 
+constexpr int small_lds(SmallW w, int rt, int mt) {
+  const int slot = addr::small_slot_bytes(w, rt, mt);
+  return slot * addr::small_depth(slot);
+}
+
+template <class Mma, SmallW W, class Epi, int RT, int MT, bool TIMES16>
+int launch_one(const SmallParams& p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, int waves, const char* what, hipStream_t st) {
+  typedef SmallCfg<W, RT, MT> Cfg;
+  static_assert(Cfg::LDS == small_lds(W, RT, MT), "the plan's LDS");
+  auto kern = gemm_small_kernel<Mma, W, Epi, RT, MT, TIMES16>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) {
+      set_error("%s: cannot reserve LDS: %s", what, hipGetErrorString(e));
+      return 1;
+    }
+    attr_set = true;
+  }
+  const dim3 blocks((unsigned)ceil_div(N, (int64_t)16 * RT), (unsigned)ceil_div(M, (int64_t)16 * MT), (unsigned)batch);
+  kern<<<blocks, waves * 64, (size_t)waves * Cfg::LDS, st>>>(p, pe, (int)M, (int)N);
+  return check_launch(what, "gemm_small_kernel") ? 0 : 1;
+}
+
+template <class Mma, SmallW W, class Epi, bool TIMES16 = false>
+int launch_tile(const SmallTile& t, const SmallParams& p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, const char* what, hipStream_t st) {
+#define TLQ_ONE(RT, MT) \
+  if (t.rt == RT && t.mt == MT) return launch_one<Mma, W, Epi, RT, MT, TIMES16>(p, pe, batch, M, N, t.waves, what, st);
+  if constexpr (W == kSmallNK || W == kSmallW4) {
+    TLQ_ONE(1, 1) TLQ_ONE(2, 1) TLQ_ONE(1, 2) TLQ_ONE(2, 2) TLQ_ONE(1, 4) TLQ_ONE(2, 4)
+  }
+  TLQ_ONE(4, 1) TLQ_ONE(4, 2) TLQ_ONE(4, 4)
+#undef TLQ_ONE
+  set_error("%s: no such tile", what);
+  return 1;
+}
+
+inline SmallParams small_params(const void* A, const void* B, int64_t M, int64_t N, int64_t row_bytes, int64_t w_row, int64_t w_bytes) {
+  return SmallParams{(const uint8_t*)A, (const uint8_t*)B, M * row_bytes, w_bytes, (int)row_bytes, (int)w_row, (int)(row_bytes / 128), 0};
+}
+
+// W4A8 with weights multiplied as 16 times their value (gemm_small_w4a8.hip)
+int small_w4a8_times16_launch(const SmallTile& t, const SmallParams& p, const EpiInt32::Params& pe, int64_t M, int64_t N, hipStream_t st);
+
 }  // namespace tlq

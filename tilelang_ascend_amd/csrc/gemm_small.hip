@@ -6,11 +6,6 @@ namespace tlq {
 
 static thread_local int g_small_waves = 0, g_small_tiles = 0;  // tuning and tests: forced variant; tiles < 0: never
 
-static constexpr int small_lds(SmallW w, int rt, int mt) {
-  const int slot = addr::small_slot_bytes(w, rt, mt);
-  return slot * addr::small_depth(slot);
-}
-
 // The estimate, in microseconds: a launch, rounds of the work-groups the machine holds at once (LDS and registers) x the longest chain
 // of steps in a wavefront, what a CU does per step of its share of the tiles (operand reads, multiplications), what it stores, and
 // the weights' trip from memory -- once, and again for every further tile of activation rows.  Fitted per kind to 970 problems (M 1 .. 1500,
@@ -67,42 +62,6 @@ SmallTile small_tile_plan(int kind, int64_t batch, int64_t M, int64_t N, int64_t
 }
 bool small_tile_forced() { return g_small_tiles > 0; }
 
-template <class Mma, SmallW W, class Epi, int RT, int MT, bool TIMES16>
-static int launch_one(const SmallParams& p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, int waves, const char* what, hipStream_t st) {
-  typedef SmallCfg<W, RT, MT> Cfg;
-  static_assert(Cfg::LDS == small_lds(W, RT, MT), "the plan's LDS");
-  auto kern = gemm_small_kernel<Mma, W, Epi, RT, MT, TIMES16>;
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e != hipSuccess) {
-      set_error("%s: cannot reserve LDS: %s", what, hipGetErrorString(e));
-      return 1;
-    }
-    attr_set = true;
-  }
-  const dim3 blocks((unsigned)ceil_div(N, (int64_t)16 * RT), (unsigned)ceil_div(M, (int64_t)16 * MT), (unsigned)batch);
-  kern<<<blocks, waves * 64, (size_t)waves * Cfg::LDS, st>>>(p, pe, (int)M, (int)N);
-  return check_launch(what, "gemm_small_kernel") ? 0 : 1;
-}
-
-template <class Mma, SmallW W, class Epi, bool TIMES16 = false>
-static int launch_tile(const SmallTile& t, const SmallParams& p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, const char* what, hipStream_t st) {
-#define TLQ_ONE(RT, MT) \
-  if (t.rt == RT && t.mt == MT) return launch_one<Mma, W, Epi, RT, MT, TIMES16>(p, pe, batch, M, N, t.waves, what, st);
-  if constexpr (W == kSmallNK || W == kSmallW4) {
-    TLQ_ONE(1, 1) TLQ_ONE(2, 1) TLQ_ONE(1, 2) TLQ_ONE(2, 2) TLQ_ONE(1, 4) TLQ_ONE(2, 4)
-  }
-  TLQ_ONE(4, 1) TLQ_ONE(4, 2) TLQ_ONE(4, 4)
-#undef TLQ_ONE
-  set_error("%s: no such tile", what);
-  return 1;
-}
-
-static SmallParams small_params(const void* A, const void* B, int64_t M, int64_t N, int64_t row_bytes, int64_t w_row, int64_t w_bytes) {
-  return SmallParams{(const uint8_t*)A, (const uint8_t*)B, M * row_bytes, w_bytes, (int)row_bytes, (int)w_row, (int)(row_bytes / 128), 0};
-}
-
 int small_i8(const SmallTile& t, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int b_layout, hipStream_t st) {
   EpiInt32::Params pe{(int32_t*)C, N, M * N};
   const SmallParams p = small_params(A, B, M, N, K, b_layout == TLQ_B_NK ? K : N, N * K);
@@ -122,8 +81,7 @@ int small_w4a8(const SmallTile& t, const void* A, const void* Wp, void* C, int64
   EpiInt32::Params pe{(int32_t*)C, N, M * N};
   SmallParams p = small_params(A, Wp, M, N, K, K / 2, 0);
   p.sign_mode = sign_mode;
-  if (small_w4a8_times16(sign_mode, K))
-    return launch_tile<MmaI8, kSmallW4, EpiInt32, true>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
+  if (small_w4a8_times16(sign_mode, K)) return small_w4a8_times16_launch(t, p, pe, M, N, st);
   return launch_tile<MmaI8, kSmallW4, EpiInt32>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
 }
 
