@@ -929,13 +929,15 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // 43.7 against 36.4 us); 2^26 weights and more: the rules further down (level: 128 x 50304 x 4096 61.6 against 61.8 us); above 512
   // rows the two passes, where they ran, on weight-row counts that are no multiple of 128 or no more than 256 (639 x 5680 x 896 22.2
   // against 15.5 us); and, where the panel kernels ran, a launch for the last one to three rows.
-  bool stream_region = N * K < ((int64_t)1 << (M > 195 ? 25 : 26));
-  if (M > 512 && stream_region) {
+  bool stream_region = algo == TLQ_ALGO_AUTO && g_w4a16_stream && !keep_tail && M > 32 && M <= kStreamMaxRows && N > 0 && K > 0 && group > 0 && N < kMaxDim && K < kMaxDim &&
+                       N * K < ((int64_t)1 << (M > 195 ? 25 : 26));
+  // (the estimate first: it is kept per shape, the choice among the others is not and takes 1.8 us of host time)
+  if (M > 512 && stream_region && (stream_region = g_stream_tiles > 0 || stream_beats_panels(M, N, K, group))) {
     const int64_t head = M & ~(int64_t)3;
     const bool two = room_for_two_passes && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
     stream_region = two ? N % 128 == 0 && N > 256 : !head_and_tail;
   }
-  if (algo == TLQ_ALGO_AUTO && g_w4a16_stream && !keep_tail && M > 32 && M <= kStreamMaxRows && N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && stream_region) {
+  if (stream_region) {
     const StreamPlan sp = stream_plan_for(M, N, K, group, algo);
     if (stream_workspace_ok(sp, M, N, workspace, workspace_bytes) && stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype)) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
