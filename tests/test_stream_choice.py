@@ -1,0 +1,54 @@
+"""W4A16 on 129 to 512 rows: where the automatic choice, in both word layouts, takes the streaming kernel and where one of the others, at problems where
+the prices that the rules put on the streaming kernel were those of another geometry.  Seen in the launch log and, bit for bit, in the named
+kernel's result.  The times beside the problems: the kernel that is to run, then the one that ran."""
+import pytest
+import torch
+
+from helpers import assert_bit_equal
+from tilelang_ascend_amd import _abi
+
+KERNEL = {_abi.ALGO_STREAM: "w4a16_stream_kernel", _abi.ALGO_PANEL256: "w4a16_panel256_kernel"}
+
+
+def run(M, N, K, group, layout, algo, dtype=torch.float16):
+    lib, P, st = _abi.load(), _abi.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g, device="cuda", dtype=dtype)
+    W = torch.randint(0, 256, (N, K // 2), generator=g, device="cuda", dtype=torch.uint8)
+    S = (torch.rand(N, K // group, generator=g, device="cuda") * 0.015 + 0.005).to(dtype)
+    Z = torch.randint(6, 10, (N, K // group), generator=g, device="cuda").to(dtype)
+    need = int(lib.tlq_w4a16_workspace_bytes(M, N, K) if algo == _abi.ALGO_AUTO else lib.tlq_w4a16_workspace_bytes_for(M, N, K, algo))
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    C = torch.full((M, N), float("nan"), dtype=dtype, device="cuda")
+    code = _abi.F16 if dtype is torch.float16 else _abi.BF16
+    print(f"stream choice M={M} N={N} K={K} g={group} layout={layout} algo={algo} {dtype}", flush=True)
+    lib.tlq_debug_launch_log(1)
+    rc = lib.tlq_gemm_w4a16_layout_ws(P(A), P(W), P(S), P(Z), P(C), M, N, K, group, 0.0, code, code, algo, layout, P(ws) if need else None, need, st)
+    log = lib.tlq_debug_launch_log_text().decode()
+    lib.tlq_debug_launch_log(0)
+    _abi.check(rc)
+    torch.cuda.synchronize()
+    return C, log
+
+
+def check(M, N, K, group, layout, algo, dtype=torch.float16):
+    got, log = run(M, N, K, group, layout, _abi.ALGO_AUTO, dtype)
+    if _abi.load().tlq_device_cu_count() != 256:
+        pytest.skip("the choices are those of 256 compute units")
+    assert KERNEL[algo] in log, log
+    assert_bit_equal(got.cpu(), run(M, N, K, group, layout, algo, dtype)[0].cpu(), f"{M}x{N}x{K} g{group} layout {layout}: automatic choice vs the named kernel")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,N,K,group,algo", [
+    # against the 256-row panel kernel: plans of four groups of wavefronts (blocks of 128 weight rows)
+    (256, 11008, 5504, 128, _abi.ALGO_STREAM),   # 45.4, 71.2 us
+    (384, 8192, 6912, 128, _abi.ALGO_STREAM),    # 53.2, 69.8
+    (512, 4096, 11008, 64, _abi.ALGO_STREAM),    # 61.0, 72.3
+    (256, 5120, 13824, 128, _abi.ALGO_STREAM),   # 49.4, 65.4
+    (512, 6144, 14720, 128, _abi.ALGO_PANEL256), # 87.7 (the streaming kernel 105.1)
+    (448, 18944, 3584, 64, _abi.ALGO_PANEL256),  # 82.7 (100.4), two groups
+])
+def test_against_the_256_row_kernel(M, N, K, group, layout, algo):
+    check(M, N, K, group, layout, algo)

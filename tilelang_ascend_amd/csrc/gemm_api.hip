@@ -642,21 +642,22 @@ static bool panel256_estimate_wins(int64_t M, int64_t N, int64_t K, int64_t grou
   return est_2 < 0.9 * est_m;
 }
 
-// 257 .. 512 rows: does the 256-row kernel beat the streaming kernel's blocks of 128 rows by the same estimate (a streaming
-// step of a 128-row block: 2.2 us, fixed part 8 us)?  It matters where the middle-M kernel does not take K (group counts
-// that are no multiple of eight) and four blocks of 128 rows meet two tiles of 256: N = 5120, K = 13824, M = 448 - 512:
-// 82 - 85 against 102 us; N = 3584, K = 18944: 81 - 85 against 102 - 106 us; N = 18944, K = 3584: 82 against 118 - 128 us;
-// on 30 measured cases the estimated ratio is 4 - 25 % above the measured one, hence the bar of 0.95 (N = 8192, K = 6912,
-// where the 256-row kernel is 2 - 5 % ahead, stays with the streaming kernel; N = 4096, K = 11008, where it is 6 % behind, too).
+// 129 .. 512 rows: does the 256-row kernel beat the streaming kernel?  It matters where the middle-M kernel does not take K (group
+// counts that are no multiple of eight) and four blocks of 128 rows meet two tiles of 256.  Two prices of the streaming kernel:
+//   * Blocks of 256 weight rows (two groups of wavefronts): rounds x (2.2 us a step of 128 rows, 1.75 of 96, + 8), bar 0.95: 448 x 5120 x
+//     13824 82 against 80 - 84 us, 448 x 18944 x 3584 82 against 100, 144 x 50304 x 4096 in two blocks of 96 rows.
+//   * Blocks of 128 weight rows (four groups) make twice the work-groups at a third of that time a step: by the plan's own estimate, with
+//     the 256-row kernel's at 0.9 (it is 18 % high at the median).  On 434 problems (groups of 32 - 1024, both types) 0.1 % behind the faster
+//     kernel on average, more than 3 % on 6; the price above sent 256 x 11008 x 5504 (44 against 71 us), 512 x 4096 x 11008 (61 against 72)
+//     and 165 others to the slower one (1.11 x on average).  The 256-row kernel is ahead from some 400 rows on 6000 x 12000 on: 512 x 6144 x 14720 88 against 105 us.
 static bool panel256_beats_stream(int64_t M, int64_t N, int64_t K, int64_t group, const StreamPlan& sp) {
-  // (256 rows: one tile against two blocks -- N = 151936, K = 3584: 278 against 333 us; 129 .. 192 rows in two blocks of 96
-  // rows, 1.75 us a step, on very wide matrices: N = 50304 .. 128256, K = 4096 .. 8192, M = 160: 100 - 238 against 128 - 277 us)
   if (M <= 128 || !sp.ok || (sp.tm != 8 && sp.tm != 6)) return false;
   const int64_t cus_now = cu_count_or_default();
   const Panel2Plan p2 = w4a16_panel256_plan(M, N, K, group, (int)cus_now);
   if (!p2.ok) return false;
-  const double est_s = panel_estimate_us(sp.m_blocks, sp.n_blocks, sp.split, sp.slice_steps, sp.tm == 8 ? 2.2 : 1.75, 8.0, M, N, cus_now);
   const double est_2 = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, M, N, cus_now);
+  if (sp.kg == 4) return 0.9 * est_2 < sp.us;
+  const double est_s = panel_estimate_us(sp.m_blocks, sp.n_blocks, sp.split, sp.slice_steps, sp.tm == 8 ? 2.2 : 1.75, 8.0, M, N, cus_now);
   return est_2 < 0.95 * est_s;
 }
 
