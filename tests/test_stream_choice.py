@@ -49,6 +49,8 @@ def check(M, N, K, group, layout, algo, dtype=torch.float16):
     (256, 5120, 13824, 128, _abi.ALGO_STREAM),   # 49.4, 65.4
     (512, 6144, 14720, 128, _abi.ALGO_PANEL256), # 87.7 (the streaming kernel 105.1)
     (448, 18944, 3584, 64, _abi.ALGO_PANEL256),  # 82.7 (100.4), two groups
+    (472, 20352, 1152, 32, _abi.ALGO_PANEL256),  # 32.0 (39.7), short rows of a wide matrix
+    (316, 24960, 256, 128, _abi.ALGO_PANEL256),  # 16.8 (20.2)
 ])
 def test_against_the_256_row_kernel(M, N, K, group, layout, algo):
     check(M, N, K, group, layout, algo)

@@ -652,13 +652,16 @@ static bool panel256_estimate_wins(int64_t M, int64_t N, int64_t K, int64_t grou
 //     and 165 others to the slower one (1.11 x on average).  The 256-row kernel is ahead from some 400 rows on 6000 x 12000 on: 512 x 6144 x 14720 88 against 105 us.
 static bool panel256_beats_stream(int64_t M, int64_t N, int64_t K, int64_t group, const StreamPlan& sp) {
   if (M <= 128 || !sp.ok || (sp.tm != 8 && sp.tm != 6)) return false;
-  const int64_t cus_now = cu_count_or_default();
-  const Panel2Plan p2 = w4a16_panel256_plan(M, N, K, group, (int)cus_now);
-  if (!p2.ok) return false;
-  const double est_2 = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, M, N, cus_now);
-  if (sp.kg == 4) return 0.9 * est_2 < sp.us;
-  const double est_s = panel_estimate_us(sp.m_blocks, sp.n_blocks, sp.split, sp.slice_steps, sp.tm == 8 ? 2.2 : 1.75, 8.0, M, N, cus_now);
-  return est_2 < 0.95 * est_s;
+  static thread_local PlanTable<bool> known;
+  return known.get(M, N, K, group, [&] {
+    const int64_t cus_now = cu_count_or_default();
+    const Panel2Plan p2 = w4a16_panel256_plan(M, N, K, group, (int)cus_now);
+    if (!p2.ok) return false;
+    const double est_2 = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, M, N, cus_now);
+    if (sp.kg == 4) return 0.9 * est_2 < sp.us;
+    const double est_s = panel_estimate_us(sp.m_blocks, sp.n_blocks, sp.split, sp.slice_steps, sp.tm == 8 ? 2.2 : 1.75, 8.0, M, N, cus_now);
+    return est_2 < 0.95 * est_s;
+  });
 }
 
 // The automatic choice takes the 256-row panel kernel where the last round of its work-groups fills more than half of the CUs
@@ -940,7 +943,10 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   }
   if (stream_region) {
     const StreamPlan sp = stream_plan_for(M, N, K, group, algo);
-    if (stream_workspace_ok(sp, M, N, workspace, workspace_bytes) && stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype)) {
+    // (129 .. 512 rows where the 256-row kernel's estimate is ahead: on short rows of wide matrices, 472 x 20352 x 1152 in groups of 32 32.0 against
+    // 39.7 us, 316 x 24960 x 256 16.8 against 20.2; it runs further down)
+    const bool panel = M <= 512 && !g_w4a16_panel && panel256_beats_stream(M, N, K, group, sp);
+    if (!panel && stream_workspace_ok(sp, M, N, workspace, workspace_bytes) && stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype)) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       // (96 rows and more on short rows, one round of 128 x 128 tiles: the tile kernel, 4.5 us + 1.45 us per 128 values of K -- 264 x 7168 x 256
       // 6.8 against 9.2 us; and, which the tests of the choice ask for, a round that is nearly full, up to 1024 values: 512 x 8192 x 1024
