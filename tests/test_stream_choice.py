@@ -54,3 +54,20 @@ def check(M, N, K, group, layout, algo, dtype=torch.float16):
 ])
 def test_against_the_256_row_kernel(M, N, K, group, layout, algo):
     check(M, N, K, group, layout, algo)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,N,K,group,dtype", [
+    # against the tile kernel over K slices and the two passes: more work-groups than compute units, group counts that the panel kernels do not take
+    (318, 24192, 8576, 128, torch.float16),   # 213, 300 and 333 us
+    (295, 23424, 3968, 128, torch.bfloat16),  # 93, 129, 142
+    (407, 19968, 2048, 256, torch.float16),   # 50, 80, 64
+    (319, 3200, 12800, 32, torch.float16),    # 51, 89, 74
+    (384, 20480, 1920, 32, torch.bfloat16),   # 38, 92, 53
+    (446, 8192, 7680, 32, torch.float16),     # 61, 108, 105
+])
+def test_against_k_slices_and_two_passes(M, N, K, group, layout, dtype):
+    if layout and dtype is torch.bfloat16:
+        pytest.skip("repacked words are for float16")
+    check(M, N, K, group, layout, _abi.ALGO_STREAM, dtype)

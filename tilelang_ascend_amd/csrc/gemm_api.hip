@@ -19,7 +19,6 @@ int64_t w4a16_mid_split(int64_t M, int64_t N, int64_t K, int64_t group);
 int w4a16_split_forced();
 bool w4a16_tile_forced();
 bool w4a16_skinny_forced();
-double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group);
 int gemm_w4a16_mfma_splitk(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M,
                            int64_t N, int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype,
                            int64_t split, float* partial, hipStream_t st);
@@ -1110,50 +1109,11 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
                                   workspace_bytes, stream);
       if (rc >= 0) return rc;
     }
-    // measured on the MLP shapes: 20 - 35 % ahead of the tile kernel up to 256 rows, level with it at 512 -- unless the
-    // tile kernels cannot fill the machine there (M = 512 on 4096 weight rows: 128 tiles of 128 x 128; K = 11008: 89
-    // against 137 us for the two passes, K = 4096: 34 against 43 us)
-    // (rows of more than 8192 values that the tile kernel can cut into enough K slices stay with it: N = 5120, K = 13824:
-    // 101 against 127 us)
-    // When the partial sums of many short K slices (split x M x N x 4 bytes, written and read back) outweigh the packed
-    // weights, the tile kernel, which cuts K as it likes, is ahead.  (Since a slice of the streaming kernel may run over
-    // several windows of 16 groups its plan seldom cuts that short.)
-    // (Only where the partial sums are tens of MB: on 4096 weight rows, or below, the streaming kernel stays ahead.)
-    // And only where the tile kernel finds a K cut that fills the machine: rows of 11008 = 2 x 43 x 128 values can only be halved.
-    // Up to three blocks of 128 activation rows the streaming kernel is level with or ahead of the tile kernel over K
-    // slices on 18 of 20 (N, K) pairs (N = 10240, K = 8192, M = 384: 93 against 155 us; the other two are 4 % behind);
-    // with four blocks only while its work-groups fit the machine at once (N = 8192, K = 4096, M = 512: 51 against 59 us;
-    // N = 13824, K = 5120, 432 work-groups: 114 against 99 us).
-    // Its weak spot: somewhat more work-groups than CUs (one work-group per CU: the second round runs half empty).  Where
-    // K has no cut for the tile kernel either, the two passes, whose plain GEMM cuts K unevenly, are ahead then:
-    // N = 4096, K = 11008 (86 steps: 288 work-groups at M = 384, 384 at M = 512): 69 against 82 us, 78 against 87 us.
-    const int64_t stream_wgs = (int64_t)sp.m_blocks * sp.n_blocks * sp.split;
-    const int64_t cus_now = cu_count_or_default();
-    const bool thin_second_round = M > 256 && have && N % 8 == 0 && stream_wgs > cus_now && stream_wgs * 2 <= cus_now * 3 &&
-                                   w4a16_mid_split(M, N, K, group) <= 1;
-    // A K cut of the tile kernel into long slices -- 3072 values or more per work-group -- does not pay between 192 and 256 rows
-    // either: N = 28672, K = 8192, M = 192: 154 against 122 us for the streaming kernel; N = 8192, K = 28672: 156 against 121 us.
-    // With groups of 32 values, where neither the middle-M kernel nor long windows are to be had, it does (N = 8192, K = 28672,
-    // bf16, M = 196 - 252: 139 - 147 against 153 - 156 us).
-    const int64_t tile_split = group < 64 && M >= 192 && M <= 256 ? w4a16_mid_split(M, N, K, group) : 1;
-    const bool long_tile_slices = tile_split > 1 && K / tile_split >= 3072 && w4a16_mid_fill(M, N, K, group) >= 0.85 &&
-                                  workspace != nullptr && workspace_bytes >= tile_split * M * N * 4;
-    // Groups of 32 values give the streaming kernel windows of four steps, each with a round trip to memory of its own:
-    // from 320 rows on, the tile kernel over K slices is 2 - 11 % ahead wherever its cut fills the machine (N = 4096,
-    // K = 14336, M = 384: 77 against 84 us; N = 5120, K = 13824: 89 against 97 us); where it cannot cut K (rows of 11008
-    // values) the streaming kernel is far ahead (64 against 160 us) and stays.
-    const bool short_windows = group < 64 && M > 256 && sp.ok && (int64_t)sp.slice_steps * 128 > 2 * 16 * group &&
-                               w4a16_mid_split(M, N, K, group) > 1 && w4a16_mid_fill(M, N, K, group) >= 0.8;
-    const bool stream_first = ((M <= 384 && !thin_second_round) || stream_wgs <= cus_now) && !long_tile_slices && !short_windows;
-    const bool slices_too_short = group < 128 && (int64_t)sp.split * M * 4 >= K && (int64_t)sp.split * M * N * 4 > ((int64_t)40 << 20) &&
-                                  w4a16_mid_fill(M, N, K, group) >= 0.66;
-    // One full tile height of the tile kernel (97 .. 128 rows) on up to 2^23 weights: the tile kernel over K slices is ahead of the
-    // streaming kernel (128 rows, seven (N, K) pairs, fp16 and bf16: 13.6 - 18.2 against 15.3 - 18.8 us; level at 96 rows and
-    // at 4096 x 4096, a third behind from 160 rows on).
-    const bool tile_band = algo == TLQ_ALGO_AUTO && M > 96 && M <= 128 && N * K <= ((int64_t)1 << 23) && w4a16_mid_split(M, N, K, group) > 1 &&
-                           workspace != nullptr && workspace_bytes >= w4a16_mid_split(M, N, K, group) * M * N * 4;
-    if (sp.ok && args_ok && ws_ok && !tile_band &&
-        (algo == TLQ_ALGO_STREAM || (stream_first && !slices_too_short) || (!slices_too_short && !thin_second_round && !long_tile_slices && !short_windows && tile_fill(1, M, N, 128) < 0.65 && (K <= 8192 || w4a16_mid_split(M, N, K, group) <= 1))))
+    // What is left, the tile kernel over K slices and the two passes, is behind on 783 of 796 problems (33 .. 512 rows, 2^25 .. 2^29 weights,
+    // groups of 32 - 4096, both types): 318 x 24192 x 8576 213 us against 300 and 333, 407 x 19968 x 2048 50 against 80 and 64, 319 x 3200 x 12800
+    // in groups of 32 51 against 89 and 74.  On ten of the others the 256-row kernel, asked above, is ahead of all three; the last three (groups of 32;
+    // 5, 6 and 17 % ahead) do not carry a rule.
+    if (sp.ok && args_ok && ws_ok)
       return gemm_w4a16_stream(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, sp, (float*)workspace,
                                (hipStream_t)stream);
     if (algo == TLQ_ALGO_STREAM) {
@@ -1320,11 +1280,9 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
     const StreamPlan sp = M <= 512 ? stream_plan_for(M, N, K, group, algo) : StreamPlan{};
     const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));
     const bool room_for_two_passes = ws_aligned && workspace_bytes >= N * K * 2;
-    // (no tile kernel reads this layout: the alternative is the two passes)
-    const bool stream_taken = ws_ok && (algo == TLQ_ALGO_STREAM || M <= 384 || (int64_t)sp.m_blocks * sp.n_blocks * sp.split <= cu_count_or_default() ||
-                                        tile_fill(1, M, N, 128) < 0.65 || !room_for_two_passes);
+    // (no tile kernel reads this layout: the alternative is the two passes, which are behind: 512 x 8192 x 4096 39 against 56 us)
     // the small-tile kernel in the place of either, for calls that bring the workspace those want: without it they are refused
-    if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (stream_taken || (room_for_two_passes && N % 8 == 0))) {
+    if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (ws_ok || (room_for_two_passes && N % 8 == 0))) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_stream(small, sp, M, N, K))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(small)",
@@ -1336,7 +1294,7 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
                                   workspace_bytes, stream);
       if (rc >= 0) return rc;
     }
-    if (stream_taken)
+    if (ws_ok)
       return gemm_w4a16_stream(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, sp,
                                (float*)workspace, (hipStream_t)stream);
     TLQ_REQUIRE(algo != TLQ_ALGO_STREAM, "tlq_gemm_w4a16_layout_ws: the streaming kernel does not take M=%lld N=%lld K=%lld group=%lld "

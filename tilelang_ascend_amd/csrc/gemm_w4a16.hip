@@ -454,9 +454,6 @@ int w4a16_split_forced() { return g_w4a16_split; }
 bool w4a16_tile_forced() { return g_w4a16_tile != 0; }
 bool w4a16_skinny_forced() { return g_skinny_waves != 0 || g_skinny_rt != 0 || g_skinny_lds >= 0; }
 
-// fraction of the work-group places (256, or 512 for the smaller tiles) that the tile kernel fills with the K cut it would take
-double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group);
-
 int f16_split_choice(int64_t batch, int64_t M, int64_t N, int64_t K);  // gemm_f16.hip
 
 int64_t w4a16_mid_split(int64_t M, int64_t N, int64_t K, int64_t group) {
@@ -486,13 +483,6 @@ int64_t w4a16_mid_split(int64_t M, int64_t N, int64_t K, int64_t group) {
   for (int64_t s = want < 16 ? want : 16; s >= 2; --s)
     if (K % s == 0 && (K / s) % unit == 0 && K / s >= 512) return (M > 256 && tiles * s * 3 < places * 2) ? 1 : s;
   return 1;
-}
-
-double w4a16_mid_fill(int64_t M, int64_t N, int64_t K, int64_t group) {
-  const int64_t bm = M <= 32 ? 32 : (M <= 64 ? 64 : (M <= 128 ? 128 : 256)), bn = (M <= 32 || (M > 64 && M <= 128)) ? 128 : 256;
-  const int64_t tiles = ceil_div(M, bm) * ceil_div(N, bn), places = bm == 256 ? 256 : 512;
-  const double f = (double)(tiles * w4a16_mid_split(M, N, K, group)) / (double)places;
-  return f > 1.0 ? 1.0 : f;
 }
 
 void launch_splitk_reduce(const float* partial, void* C, int64_t M, int64_t N, int split, int out_dtype, hipStream_t st) {
