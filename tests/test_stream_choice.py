@@ -1,6 +1,8 @@
 """W4A16 on 129 to 512 rows: where the automatic choice, in both word layouts, takes the streaming kernel and where one of the others, at problems where
 the prices that the rules put on the streaming kernel were those of another geometry.  Seen in the launch log and, bit for bit, in the named
 kernel's result.  The times beside the problems: the kernel that is to run, then the one that ran."""
+import ctypes
+
 import pytest
 import torch
 
@@ -71,3 +73,18 @@ def test_against_k_slices_and_two_passes(M, N, K, group, layout, dtype):
     if layout and dtype is torch.bfloat16:
         pytest.skip("repacked words are for float16")
     check(M, N, K, group, layout, _abi.ALGO_STREAM, dtype)
+
+
+@pytest.mark.parametrize("M,N,K,group", [
+    (188, 18128, 3200, 64),  # 284 work-groups of 96 x 128 rows 49.6 us, 142 of 96 x 256 35.0
+    (133, 18432, 1920, 32),  # 288 35.7, 144 25.4
+    (223, 17408, 5248, 32),  # 272 96.6, 204 69.0
+    (472, 8352, 4992, 32),   # 264 92.1, 165 70.0
+    (69, 23296, 8064, 64),   # 364 in four K slices 80.2, 182 in two 61.4
+    (47, 32896, 3840, 64),   # 257 51.9, 129 39.7
+])
+def test_plans_leave_no_few_work_groups_for_a_second_round(M, N, K, group):
+    plan = (ctypes.c_int64 * 5)()
+    assert _abi.load().tlq_debug_stream_plan(M, N, K, group, 256, plan) == 1
+    rows, weight_rows, slices, steps, _ = plan
+    assert -(-M // rows) * -(-N // weight_rows) * slices <= 256 and slices * steps >= K // 128

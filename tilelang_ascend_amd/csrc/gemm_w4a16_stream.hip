@@ -623,16 +623,17 @@ __global__ __launch_bounds__(256) void w4a16_stream_reduce_kernel(const float4_t
 thread_local int g_stream_tiles = 0;  // tuning and tests: 16-row activation tiles per work-group (2, 4, 6, 8), + 16 for four groups of wavefronts (0: the estimate below)
 thread_local int g_stream_slice_steps = 0;  // tuning and tests: steps of 128 values of K per slice (0: the estimate below)
 
-// The launch with the lowest estimate.  Per round of work-groups, one to a CU (rounds counted half whole, half as they fill: the last one
-// runs beside the others' ends): a fixed part and its steps; a further window of scales restarts the ring; K slices cost a second
-// launch and their partial sums' way to memory and back; then the products of the padded problem (power), the result, the weights and
-// the activations.  Fitted to 1865 timed configurations of 1050 problems (M 17 .. 4096, N 256 .. 19200, K 512 .. 14336, groups of
-// 64 - 256, both types, up to 2e11 operations): 6.7 % rms, and the choice among the configurations timed of a problem 1.5 % behind its
-// best on average (22 % at most, more than 5 % on 19 of 158).
+// The launch with the lowest estimate.  Per round of work-groups, one to a CU: a fixed part and its steps; a further window of scales
+// restarts the ring; K slices cost a second launch and their partial sums' way to memory and back; then the products of the padded
+// problem (power), the result, the weights and the activations.  Fitted to 1865 timed configurations of 1050 problems (M 17 .. 4096, N 256 ..
+// 19200, K 512 .. 14336, groups of 64 - 256, both types, up to 2e11 operations), the choice among the configurations timed of a problem 1.5 % behind
+// its best on average (22 % at most, more than 5 % on 19 of 158); on 3338 others (M 17 .. 512, N .. 33000, K .. 18944) 5 % high and 7.9 % rms.
+// Rounds are whole: counted half by how full the last one is, as they were, plans with a few work-groups in a second round looked 15 - 20 % shorter
+// than they are (188 x 18128 x 3200 284 work-groups in 49.6 us, 142 in 35.0): 575 problems that this moves 1.08 x on average, 27 of them 3 % and more behind.
 static double stream_us(int64_t M, int64_t N, int64_t K, int tm, int kg, int64_t m_blocks, int64_t n_blocks, int64_t slice_steps, int64_t slices, int64_t windows, int64_t cus) {
   static const double kStep[2][4] = {{0.73, 0.83, 0.95, 1.15}, {0.355, 0.47, 0.61, 0.68}};  // us per step of 128 values of K: [groups][32-row blocks]
   const int64_t blocks = m_blocks * n_blocks * slices;
-  const double fill = (double)blocks / (double)cus, rounds = 0.5 * (double)ceil_div(blocks, cus) + 0.5 * (fill > 1.0 ? fill : 1.0);
+  const double rounds = (double)ceil_div(blocks, cus);
   return 1.95 + rounds * ((kg == 4 ? 4.45 : 3.0) + (double)slice_steps * kStep[kg == 4][tm / 2 - 1] + 2.9 * (double)(windows - 1)) +
          (slices > 1 ? 2.36 + 1.7e-6 * (double)slices * (double)M * (double)N : 0.0) + 0.385e-9 * (double)(m_blocks * tm * 16) * (double)(n_blocks * (512 / kg)) * (double)K +
          0.6e-6 * (double)M * (double)N + 0.022e-6 * (double)N * (double)K + 0.086e-6 * (double)M * (double)K;
