@@ -9,7 +9,7 @@ import torch
 from helpers import assert_bit_equal
 from tilelang_ascend_amd import _abi
 
-KERNEL = {_abi.ALGO_STREAM: "w4a16_stream_kernel", _abi.ALGO_PANEL256: "w4a16_panel256_kernel"}
+KERNEL = {_abi.ALGO_STREAM: "w4a16_stream_kernel", _abi.ALGO_PANEL256: "w4a16_panel256_kernel", _abi.ALGO_PANELM: "w4a16_panelm_kernel"}
 
 
 def run(M, N, K, group, layout, algo, dtype=torch.float16):
@@ -73,6 +73,21 @@ def test_against_k_slices_and_two_passes(M, N, K, group, layout, dtype):
     if layout and dtype is torch.bfloat16:
         pytest.skip("repacked words are for float16")
     check(M, N, K, group, layout, _abi.ALGO_STREAM, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,group,dtype,algo", [
+    # against the middle-M kernel in whole rounds of its work-groups
+    (224, 8192, 4096, 128, torch.float16, _abi.ALGO_STREAM),   # 27.9, 31.6 us: the second tile of 128 rows partly filled
+    (232, 8192, 6656, 64, torch.float16, _abi.ALGO_STREAM),    # 39.4, 46.3
+    (252, 2048, 16384, 128, torch.float16, _abi.ALGO_STREAM),  # 30.1, 33.1
+    (256, 8192, 4096, 128, torch.bfloat16, _abi.ALGO_STREAM),  # 28.1, 31.9
+    (256, 4096, 8192, 64, torch.bfloat16, _abi.ALGO_STREAM),
+    (256, 8192, 5120, 64, torch.float16, _abi.ALGO_STREAM),    # 34.4, 40.4: K slices of 12 steps
+    (256, 8192, 4096, 128, torch.float16, _abi.ALGO_PANELM),
+])
+def test_against_whole_rounds_of_the_middle_m_kernel(M, N, K, group, dtype, algo):
+    check(M, N, K, group, 0, algo, dtype)
 
 
 @pytest.mark.parametrize("M,N,K,group", [

@@ -500,13 +500,6 @@ static bool panelm_preferred(int64_t M, int64_t N, int64_t K) {
   return M > 256 || N * K >= (N >= 10240 ? 44000000 : 56000000);
 }
 
-// From 196 rows on 2^25 weights and more also where its work-groups are whole rounds of CUs (256 x 8192 x 4096: 256 work-groups).
-static bool panelm_whole_rounds(int64_t M, int64_t N, int64_t K, int64_t group) {
-  if (M < 196 || M > 512 || N * K < ((int64_t)1 << 25) || group <= 0) return false;
-  const PanelMPlan pm = w4a16_panelm_plan(M, N, K, group, cu_count_or_default());
-  return pm.ok && ((int64_t)pm.tiles_m * pm.tiles_n * pm.split) % cu_count_or_default() == 0;
-}
-
 // One tile of 128 rows (97 .. 128 activation rows) on matrices of 2^27 weights or more: the middle-M kernel is 9 - 18 % ahead of
 // the streaming kernel (N = 50304, K = 4096, M = 128: 64.5 against 76.1 us; N = 65536, K = 8192: 144 against 154 us;
 // N = 28672, K = 8192, M = 112: 74 against 82 us; N = 8192, K = 28672: 76 against 81 us; level at 64 and 96 rows).
@@ -639,6 +632,21 @@ static bool panel256_estimate_wins(int64_t M, int64_t N, int64_t K, int64_t grou
   const double est_m = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, pm.tm == 8 ? 2.2 : 1.8, 6.0, M, N, cus_now);
   const double est_2 = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, M, N, cus_now);
   return est_2 < 0.9 * est_m;
+}
+
+// 256 rows on 2^25 weights and more that panelm_preferred leaves to the streaming kernel: the middle-M kernel in binary16 where full
+// tiles make whole rounds of its work-groups and its estimate (14 % high there, hence 0.87) is no more than 2 % above the streaming kernel's.
+// About level with what the streaming kernel took before its groups of wavefronts (256 x 8192 x 4096 31.7 against 30.9 us, 256 x 8192 x
+// 6144 39.3 against 40.8), which is why the test of this choice names it; the streaming kernel's estimate is 10 - 15 % high there and it would
+// take 26.0 and 36.9.  With partly filled tiles, longer slices or bfloat16 the same rounds are further behind (232 x 8192 x 6656 45.3
+// against 43.5, 256 x 8192 x 4096 bf16 31.6 against 30.0): there the streaming kernel runs (38.8 and 27.2).
+static bool panelm_whole_rounds(int64_t M, int64_t N, int64_t K, int64_t group, int in_dtype) {
+  if (M != 256 || N % 256 != 0 || N * K < ((int64_t)1 << 25) || group <= 0 || in_dtype != TLQ_F16) return false;
+  const int64_t cus_now = cu_count_or_default();
+  const PanelMPlan pm = w4a16_panelm_plan(M, N, K, group, (int)cus_now);
+  if (!pm.ok || pm.tm != 8 || ((int64_t)pm.tiles_m * pm.tiles_n * pm.split) % cus_now != 0) return false;
+  const StreamPlan sp = w4a16_stream_plan(M, N, K, group, (int)cus_now);
+  return !sp.ok || 0.87 * panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, M, N, cus_now) < 1.02 * sp.us;
 }
 
 // 129 .. 512 rows: does the 256-row kernel beat the streaming kernel?  It matters where the middle-M kernel does not take K (group
@@ -1074,7 +1082,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // (not up to 256 rows with groups of 512 values or more: the panel kernels cut K into windows of eight groups -- 32 steps and
   // more -- and run uncut or nearly so, the streaming kernel cuts inside a group: N = 14336, K = 4096, M = 256: 50 against 59 us;
   // N = 11008: 47 against 58 us; N = K = 8192: 52 against 61 us; from 384 rows on the panel kernels are ahead again)
-  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && (panelm_preferred(M, N, K) || panelm_whole_rounds(M, N, K, group)) && !(M <= 256 && group >= 512)) {
+  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && (panelm_preferred(M, N, K) || panelm_whole_rounds(M, N, K, group, in_dtype)) && !(M <= 256 && group >= 512)) {
     // (very wide matrices: where the 128-row tiles need a second round of work-groups and the 256-row tiles do not, the
     // 256-row kernel by the same estimate -- N = 28672, K = 4096, M = 512: 104 against 129 us)
     if (panel256_estimate_wins(M, N, K, group)) {
