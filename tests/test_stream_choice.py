@@ -103,3 +103,20 @@ def test_plans_leave_no_few_work_groups_for_a_second_round(M, N, K, group):
     assert _abi.load().tlq_debug_stream_plan(M, N, K, group, 256, plan) == 1
     rows, weight_rows, slices, steps, _ = plan
     assert -(-M // rows) * -(-N // weight_rows) * slices <= 256 and slices * steps >= K // 128
+
+
+def test_the_workspace_size_follows_the_switch():
+    """Above 512 rows the size counts the streaming kernel's K slices: one asked for with the kernel off is not handed out once it is on again."""
+    lib = _abi.load()
+    M, N, K = 640, 12, 1664
+    lib.tlq_tune_w4a16_stream(1)
+    on = lib.tlq_w4a16_workspace_bytes(M, N, K)
+    try:
+        lib.tlq_tune_w4a16_stream(0)
+        off = lib.tlq_w4a16_workspace_bytes(M, N, K)
+    finally:
+        lib.tlq_tune_w4a16_stream(1)
+    plan = (ctypes.c_int64 * 5)()
+    assert lib.tlq_debug_stream_plan(M, N, K, 32, lib.tlq_device_cu_count() or 256, plan) == 1
+    assert on >= plan[2] * M * N * 4 > off
+    assert lib.tlq_w4a16_workspace_bytes(M, N, K) == on

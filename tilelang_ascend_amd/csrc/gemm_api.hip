@@ -181,7 +181,7 @@ int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused) {
   return tlq::prefer_small_tiles(batch, M, N, fused ? 0.65 : 0.72) ? 128 : 256;
 }
 void tlq_tune_gemm_tile(int tile) { tlq::tuning_changed(), tlq::g_gemm_f16_tile = (tile == 128 || tile == 256) ? tile : 0; }
-void tlq_tune_w4a16_stream(int on) { tlq::g_w4a16_stream = on != 0; }
+void tlq_tune_w4a16_stream(int on) { tlq::tuning_changed(), tlq::g_w4a16_stream = on != 0; }  // (the workspace size above 512 rows follows it)
 void tlq_tune_w4a16_stream_tiles(int tiles) { tlq::tuning_changed(), tlq::g_stream_tiles = ((tiles & 15) >= 2 && (tiles & 15) <= 8 && (tiles & 1) == 0) ? tiles & 31 : 0; }
 void tlq_tune_w4a16_stream_slice(int steps) { tlq::tuning_changed(), tlq::g_stream_slice_steps = steps; }
 void tlq_tune_w4a16_decode(int on) { tlq::g_w4a16_decode = on != 0; }
