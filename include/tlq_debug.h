@@ -37,6 +37,9 @@ int tlq_debug_check_slots_schedule(int stages, int loads_per_tile);
 /* The same walk for the streaming W4A16 kernel (TLQ_ALGO_STREAM): packed weights [N, K / 2] and 2-byte activations [M, K]
  * with 16 * activation_tiles rows per work-group (2 | 4 | 8), and its ring of `ring_depth` steps for 1 .. 40 steps. */
 int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activation_tiles, int ring_depth);
+/* Its schedule alone over a window of `steps` steps of `loads` load instructions and `units` units (8 with two groups of wavefronts, 4 with
+ * four), with the kernel's own counts of loads that its waits leave outstanding (negative arguments) or others (to see them fail). */
+int tlq_debug_check_stream_schedule(int steps, int depth, int loads, int units, int wait_scales, int wait_first, int wait_step);
 /* The same walk for the panel kernel (TLQ_ALGO_PANEL) with K slices of `slice_steps` steps of 128 values: every direct load of
  * activations, packed weights and scale windows of every work-group, the LDS map and the operand reads; and the plan the
  * library would choose on a device with `cus` compute units: plan_out is a HOST array of four int64 that receives the tiles

@@ -89,6 +89,22 @@ def test_streaming_kernel_addressing(tm, depth):
     assert lib.tlq_debug_check_stream_addressing(64, 1 << 22, 4096, tm, depth) != 0  # packed weights of 8 GiB
 
 
+@pytest.mark.parametrize("blocks,groups,depth", [(1, 2, 6), (2, 2, 4), (3, 2, 3), (4, 2, 3), (1, 4, 6), (2, 4, 6), (3, 4, 4), (4, 4, 3)])
+def test_streaming_kernel_schedule(blocks, groups, depth):
+    """The scales of a window, its first step and every later one are waited for before they are read; one load more left in flight by any
+    of the three waits and the walk fails."""
+    lib, loads, units = _abi.load(), blocks + (2 if groups == 2 else 1), 8 if groups == 2 else 4
+    waits = (2 * loads, loads, (depth - 2) * loads)
+    for steps in (1, 2, 3, 7, 40):
+        _ok(lib.tlq_debug_check_stream_schedule(steps, depth, loads, units, -1, -1, -1))
+        _ok(lib.tlq_debug_check_stream_schedule(steps, depth, loads, units, *waits))
+        for i, what in enumerate(("the scales", "step 0", "step 1")):
+            if steps > 1 or i < 2:
+                wrong = [w + (j == i) for j, w in enumerate(waits)]
+                assert lib.tlq_debug_check_stream_schedule(steps, depth, loads, units, *wrong) != 0
+                assert what in _abi.last_error()
+
+
 @pytest.mark.parametrize("kind", [0, 1, 2, 3, 4])
 def test_small_tile_kernels_addressing_and_schedule(kind):
     """Both small-tile kernels: loads inside their matrices (rows past them clamped), operand reads on the cells that hold what they

@@ -176,9 +176,16 @@ __host__ __device__ inline int stream_sz_piece(int mg, int lane, int row) { retu
 __host__ __device__ inline int stream_sz_dword(int mg, int lane, int row) { return (lane & (mg / 2 - 1)) ^ (stream_sz_swz(mg, row) * 4); }
 __host__ __device__ inline int stream_sz_value(int mg, int row, int g) { return row * mg + (g ^ (stream_sz_swz(mg, row) * 8)); }  // where value g of the row lies
 // Ring of D steps of L load instructions each: step s lives in slot s % D.  A wavefront's step is NU units; in front of unit NU - 2 of
-// step s it waits until (D - 2) L loads are outstanding, passes the step's barrier and from there on, NU units long, issues the loads
-// of step s + D: load i in unit i NU / L behind the barrier.
+// step s it waits until stream_wait_step loads are outstanding, passes the step's barrier and from there on, NU units long, issues the
+// loads of step s + D: load i in unit i NU / L behind the barrier.  A window starts with the loads of its scales, then steps 0 ..
+// kStreamAhead - 1, waits for the scales, waits for step 0, passes a barrier and issues the rest of what a step finds in flight: all of the
+// steps up to D - 2 and the loads of step D - 1 that belong to the two units behind a barrier.
+constexpr int kStreamAhead = 2;
 __host__ __device__ constexpr int stream_load_unit(int i, int units, int loads) { return i * units / loads; }
+__host__ __device__ constexpr int stream_loads_behind(int units, int loads) { return (2 * loads + units - 1) / units; }
+__host__ __device__ constexpr int stream_wait_scales(int loads) { return kStreamAhead * loads; }
+__host__ __device__ constexpr int stream_wait_first(int loads) { return (kStreamAhead - 1) * loads; }
+__host__ __device__ constexpr int stream_wait_step(int depth, int loads) { return (depth - 2) * loads; }
 
 // ---- panel kernel for large M (gemm_w4a16_panel.hip): 128 activation rows x 512 weight rows per work-group ----------
 // Steps of 128 values of K in two ring slots.  A slot is the activation tile [128 rows][256 B] (the streaming kernel's

@@ -828,12 +828,15 @@ int check_panel256_schedule(int steps, int wait_w, int wait_a) {
   return 0;
 }
 
-// The ring (addr::stream_load_unit): the loads of one wavefront in issue order against its waits, and the slots against the
-// steps that are still read.  Loads past the last step are issued empty.
-int check_stream_ring(int steps, int D, int L, int NU) {
+// The ring (addr::stream_load_unit and the waits beside it): the loads of one wavefront in issue order against its waits, and the slots
+// against the steps that are still read, over a window of `steps` steps.  Loads past the last step are issued empty.  (The wait counts
+// are arguments so that a test can show that wrong ones fail.)
+int check_stream_ring(int steps, int D, int L, int NU, int wait_scales, int wait_first, int wait_step) {
   CHECK_OR_FAIL(steps >= 1 && D >= 3 && D <= 8 && L >= 1 && L <= 8 && (NU == 4 || NU == 8), "stream ring: bad arguments");
-  std::vector<int> slot(D, -1), queue;  // slot owner; steps of the loads issued and not yet known to have landed (oldest first)
+  CHECK_OR_FAIL(wait_scales >= 0 && wait_first >= 0 && wait_step >= 0, "stream ring: bad arguments");
+  std::vector<int> slot(D, -1), queue;  // slot owner; steps of the loads issued and not yet known to have landed (oldest first; -1: scales)
   std::vector<int> landed(steps + 2 * D, 0);
+  int scales = 0;
   auto issue = [&](int step, int before_read_of) {  // every wavefront has read its last of steps below before_read_of
     const int sl = step % D;
     if (step < steps) {
@@ -844,18 +847,27 @@ int check_stream_ring(int steps, int D, int L, int NU) {
     return 0;
   };
   auto wait = [&](int outstanding) {
-    while ((int)queue.size() > outstanding) ++landed[queue.front()], queue.erase(queue.begin());
+    while ((int)queue.size() > outstanding) ++(queue.front() < 0 ? scales : landed[queue.front()]), queue.erase(queue.begin());
   };
+  constexpr int kScaleLoads = 2;  // the fewest: a piece of the scales and one of the zero points
+  for (int i = 0; i < kScaleLoads; ++i) queue.push_back(-1);
+  for (int s = 0; s < addr::kStreamAhead; ++s)
+    for (int i = 0; i < L; ++i)
+      if (int rc = issue(s, 0)) return rc;
+  wait(wait_scales);
+  CHECK_OR_FAIL(scales == kScaleLoads, "stream ring: the scales were not waited for");
+  wait(wait_first);  // and the barrier
+  CHECK_OR_FAIL(landed[0] == L, "stream ring: step 0 read before its loads were waited for");
   int behind = 0;  // loads issued in the two units behind a barrier
   for (int i = 0; i < L; ++i) behind += addr::stream_load_unit(i, NU, L) < 2;
-  for (int s = 0; s < D; ++s)
+  CHECK_OR_FAIL(behind == addr::stream_loads_behind(NU, L), "stream ring: %d loads behind a barrier, not %d", behind, addr::stream_loads_behind(NU, L));
+  for (int s = addr::kStreamAhead; s < D; ++s)
     for (int i = 0; i < (s < D - 1 ? L : behind); ++i)
       if (int rc = issue(s, 0)) return rc;
-  wait((D - 2) * L + behind);
   for (int s = 0; s < steps; ++s) {
     CHECK_OR_FAIL(landed[s] == L && slot[s % D] == s, "stream ring: step %d multiplied before its loads were waited for", s);
     for (int u = 0; u < NU; ++u) {
-      if (u == NU - 2) wait((D - 2) * L);  // and the barrier: everyone has read its last of step s
+      if (u == NU - 2) wait(wait_step);  // and the barrier: everyone has read its last of step s
       for (int i = 0; i < L; ++i)
         if (addr::stream_load_unit(i, NU, L) == (u + 2) % NU)
           if (int rc = issue(u >= NU - 2 ? s + D : s + D - 1, u >= NU - 2 ? s + 1 : s)) return rc;
@@ -1306,13 +1318,18 @@ int tlq_debug_check_gemm_addressing(int source_kind, int64_t rows, int64_t row_b
   return 1;
 }
 
+int tlq_debug_check_stream_schedule(int steps, int depth, int loads, int units, int wait_scales, int wait_first, int wait_step) {
+  return check_stream_ring(steps, depth, loads, units, wait_scales < 0 ? addr::stream_wait_scales(loads) : wait_scales,
+                           wait_first < 0 ? addr::stream_wait_first(loads) : wait_first, wait_step < 0 ? addr::stream_wait_step(depth, loads) : wait_step);
+}
+
 int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activation_tiles, int ring_depth) {
   if (int rc = check_stream(M, N, K, activation_tiles)) return rc;
   const int l = activation_tiles / 2;
   for (int steps = 1; steps <= 40; ++steps)
     for (int depth = ring_depth; depth <= 6; ++depth) {
-      if (int rc = check_stream_ring(steps, depth, l + 2, 8)) return rc;
-      if (int rc = check_stream_ring(steps, depth, l + 1, 4)) return rc;
+      if (int rc = tlq_debug_check_stream_schedule(steps, depth, l + 2, 8, -1, -1, -1)) return rc;
+      if (int rc = tlq_debug_check_stream_schedule(steps, depth, l + 1, 4, -1, -1, -1)) return rc;
     }
   return 0;
 }

@@ -70,7 +70,7 @@ struct StreamCfg {
   static constexpr int LW = WN / 2;                           // weight load instructions per wavefront and step (16 rows each)
   static constexpr int L = LA + LW;
   // load i of a step is issued in unit i * NU / L of the NU units that start at the barrier, two units before the step's end
-  static constexpr int LB = (2 * L + NU - 1) / NU;            // loads issued in those two
+  static constexpr int LB = addr::stream_loads_behind(NU, L);  // loads issued in those two
   static_assert(D >= 3 && LDS <= 160 * 1024, "rings fit the CU's LDS");
   static_assert(D * L <= 63, "vmcnt range");
   static_assert(BM * BN * 4 <= RING && (KG == 2 || 2 * BM * BN * 4 <= LDS), "the groups' exchange and the output tile fit the ring");
@@ -279,11 +279,11 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
     // Two steps now, the rest behind the barrier: a CU takes the loads in at 64 bytes a cycle, and the wavefronts that issue them wait for
     // that -- with the whole ring ahead of the barrier step 0 had long landed when they got there (2200 - 4700 cycles to issue).
 #pragma unroll
-    for (int s = 0; s < 2; ++s) static_for<0, Cfg::L>([&](auto ic) { issue1(w0 + s, w0 + wsteps, s, ic); });
+    for (int s = 0; s < addr::kStreamAhead; ++s) static_for<0, Cfg::L>([&](auto ic) { issue1(w0 + s, w0 + wsteps, s, ic); });
     __builtin_amdgcn_sched_barrier(0);
     if (wide || dwords) {
       // loads return in issue order: with the two steps' loads still in flight the scales have landed
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * Cfg::L) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(addr::stream_wait_scales(Cfg::L)) : "memory");
       if (!has_s || !has_z) {  // an absent tensor is the constant 1 / the scalar zero point
         const uint32_t ws = (uint32_t)bitcast<uint16_t>(one) * 0x10001u, wz = (uint32_t)bitcast<uint16_t>(zs) * 0x10001u;
         const uint4_t cs{ws, ws, ws, ws}, cz{wz, wz, wz, wz};
@@ -322,10 +322,10 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
           if (my_z) *(T*)(sz + Cfg::SZ / 2 + addr::stream_sz_value(MG, tn * 16 + r16, g) * 2) = pre_z[tn][i];
         }
     }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Cfg::L) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(addr::stream_wait_first(Cfg::L)) : "memory");
     __syncthreads();  // the window's scales and its step 0 are complete for every wavefront
 #pragma unroll
-    for (int s = 2; s < D; ++s)
+    for (int s = addr::kStreamAhead; s < D; ++s)
       static_for<0, Cfg::L>([&](auto ic) {
         if (s < D - 1 || decltype(ic)::value < Cfg::LB) issue1(w0 + s, w0 + wsteps, s, ic);
       });
@@ -391,7 +391,7 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
       static_for<0, NU>([&](auto uc) {
         constexpr int u = decltype(uc)::value, t = u >> 1, tn = u & 1, v = (u + 1) % NU;
         if constexpr (u == NU - 2) {
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 2) * Cfg::L) : "memory");  // step s + 1
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(addr::stream_wait_step(D, Cfg::L)) : "memory");  // step s + 1
           __syncthreads();
         }
         // the loads of step s + D, spread over the units behind the barrier
