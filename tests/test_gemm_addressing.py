@@ -79,7 +79,7 @@ def test_five_slot_schedule():
 
 @pytest.mark.parametrize("tm,depth", [(2, 5), (4, 4), (6, 3), (8, 3)])
 def test_streaming_kernel_addressing(tm, depth):
-    """Streaming W4A16 kernel: every direct load stays inside the packed weights / the activations (rows past the
+    """Streaming W4A16 kernel: every direct load stays inside the packed weights / the activations / the scale tensors (rows past the
     matrices are clamped), lands on the LDS cell its operand read expects, and the ring never multiplies a step before
     its loads were waited for nor reloads a slot that may still be read."""
     lib = _abi.load()
@@ -87,6 +87,13 @@ def test_streaming_kernel_addressing(tm, depth):
         _ok(lib.tlq_debug_check_stream_addressing(M, N, K, tm, depth))
     assert lib.tlq_debug_check_stream_addressing(64, 256, 100, tm, depth) != 0   # K not a multiple of 128
     assert lib.tlq_debug_check_stream_addressing(64, 1 << 22, 4096, tm, depth) != 0  # packed weights of 8 GiB
+
+
+@pytest.mark.parametrize("N,K", [(4, 128 * 9), (132, 128 * 35), (260, 128 * 67), (300, 128 * 24), (516, 128 * 27), (1000, 128 * 17)])
+def test_streaming_kernel_scale_sources(N, K):
+    """Where the scales come from, on rows of odd and even numbers of groups, in windows and K slices that start on either half of a dword:
+    no load past the tensors, and every read of the scale area finds its row's and group's value."""
+    _ok(_abi.load().tlq_debug_check_stream_addressing(17, N, K, 2, 6))
 
 
 @pytest.mark.parametrize("blocks,groups,depth", [(1, 2, 6), (2, 2, 4), (3, 2, 3), (4, 2, 3), (1, 4, 6), (2, 4, 6), (3, 4, 4), (4, 4, 3)])

@@ -116,3 +116,21 @@ def test_extreme_scales_and_zero_points(s, z):
         got = run(A, Wp, S, Z, group, tiles, 0)
         assert torch.equal(torch.isnan(got), torch.isnan(want))
         assert_bit_equal(torch.nan_to_num(got + 0.0), torch.nan_to_num(want + 0.0), f"scale {s} zero point {z}")
+
+
+@pytest.mark.parametrize("s,z", [(float("inf"), 7.0), (float("nan"), 7.0), (-0.5, 300.0), (0.0, -3.0), (3.0e38, 0.0), (1.2e-38, 8.0)])
+def test_extreme_scales_and_zero_points_in_bfloat16(s, z):
+    """The same in bfloat16: the largest finite scale overflows in the product of scale and weight, the smallest normal one does not vanish."""
+    N, K, group, M = 128, 256, 128, 64
+    A = torch.zeros(M, K, dtype=torch.bfloat16)
+    Wp = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=gen(67))
+    S = torch.full((N, K // group), 0.01, dtype=torch.bfloat16)
+    Z = torch.full((N, K // group), 8.0, dtype=torch.bfloat16)
+    S[5, 0], Z[5, 0] = s, z
+    A[torch.arange(M), torch.arange(M)] = 1.0
+    W = ref.dequant_w4(Wp, S, Z, group, torch.bfloat16)
+    want = (A.double() @ W.double().T).to(torch.bfloat16)
+    for tiles in (4, 20):
+        got = run(A, Wp, S, Z, group, tiles, 0)
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert_bit_equal(torch.nan_to_num(got + 0.0), torch.nan_to_num(want + 0.0), f"scale {s} zero point {z}")

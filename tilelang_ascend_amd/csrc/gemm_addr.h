@@ -158,9 +158,9 @@ __host__ __device__ inline uint32_t sa_frag_off(int lane, int tm, int ks) {
   const int r16 = lane & 15, q = lane >> 4;
   return (uint32_t)((tm * 16 + r16) * 256 + (((4 * q + ks) ^ sa_swz(r16)) << 4));
 }
-// The streaming kernel's 32 x 32 operands: lane (row r32 of a 32-row tile, half h) of the wavefronts that take values 64 kg .. 64 kg +
-// 63 of a step holds k = 64 kg + 32 h + 8 t .. + 7 at k-step t = 0 .. 3: the four words of 16-byte piece 2 kg + h of its packed row, and
-// the activations' logical chunk 8 kg + 4 h + t.
+// The streaming kernel's 32 x 32 operands: lane (row r32 of a 32-row tile, half h) of group kg of KG groups of wavefronts, which take 128 / KG
+// values of a step each, holds at k-step t = 0 .. KT - 1 (KT = 8 / KG) the eight values of word 2 KT kg + KT h + t of its packed row -- KT
+// words, all or half of 16-byte piece (2 KT kg + KT h) / 4 --, and the activations' logical chunk of the same number.
 __host__ __device__ inline uint32_t stream_w_frag(int r32, int piece) {  // inside two 1 KB tiles of 16 rows
   const int r16 = r32 & 15;
   return (uint32_t)((r32 >> 4) * 1024 + r16 * 64 + ((piece ^ sw_swz(r16)) << 4));
@@ -175,6 +175,20 @@ __host__ __device__ inline int stream_sz_row(int cells, int i, int lane) { retur
 __host__ __device__ inline int stream_sz_piece(int mg, int lane, int row) { return (lane & (mg / 8 - 1)) ^ stream_sz_swz(mg, row); }
 __host__ __device__ inline int stream_sz_dword(int mg, int lane, int row) { return (lane & (mg / 2 - 1)) ^ (stream_sz_swz(mg, row) * 4); }
 __host__ __device__ inline int stream_sz_value(int mg, int row, int g) { return row * mg + (g ^ (stream_sz_swz(mg, row) * 8)); }  // where value g of the row lies
+// Where they come from: byte offsets into a tensor [N][groups] of 2-byte values, for a window of G groups from group g0 on.  By 16-byte pieces
+// where all rows' windows are aligned (past the row's end its last piece again), else by dwords from the one that holds the row's first value
+// of the window on (stream_sz_first: it may be that dword's second) and never past the tensor's last dword.
+__host__ __device__ inline bool stream_sz_wide(int groups, int g0) { return ((groups | g0) & 7) == 0; }
+__host__ __device__ inline bool stream_sz_dwords(int mg, int N, int groups, int g0, int G) { return ((N & groups) & 1) == 0 && (((groups | g0) & 1) == 0 || G < mg); }
+__host__ __device__ inline int stream_sz_first(int n, int groups, int g0) { return (n * groups + g0) & 1; }
+__host__ __device__ inline uint32_t stream_sz_piece_voff(int n, int groups, int g0, int piece) {
+  const int last = (groups - g0) / 8 - 1;
+  return ((uint32_t)n * (uint32_t)groups + (uint32_t)g0) * 2u + (uint32_t)((piece < last ? piece : last) * 16);
+}
+__host__ __device__ inline uint32_t stream_sz_dword_voff(int n, int N, int groups, int g0, int dword) {
+  const uint32_t last = (uint32_t)N * (uint32_t)groups * 2u - 4u, voff = ((((uint32_t)n * (uint32_t)groups + (uint32_t)g0) * 2u) & ~3u) + (uint32_t)(dword * 4);
+  return voff < last ? voff : last;
+}
 // Ring of D steps of L load instructions each: step s lives in slot s % D.  A wavefront's step is NU units; in front of unit NU - 2 of
 // step s it waits until stream_wait_step loads are outstanding, passes the step's barrier and from there on, NU units long, issues the
 // loads of step s + D: load i in unit i NU / L behind the barrier.  A window starts with the loads of its scales, then steps 0 ..

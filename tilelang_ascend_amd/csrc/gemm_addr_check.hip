@@ -269,6 +269,59 @@ struct SlotsSim {
   }
 };
 
+// The streaming kernel's scales: every load of every window of K slices of `slice_steps` steps, for the first and last blocks of weight rows, and
+// what the reads of the scale area then find.  `shift`: values by which the tensors lie behind a 16-byte boundary.
+int check_stream_scales(int64_t N, int64_t K, int64_t group, int kgs, int slice_steps, int shift) {
+  const int mg = kgs == 4 ? 32 : 16, bn = 512 / kgs, groups = (int)(K / group), steps_total = (int)(K / 128);
+  CHECK_OR_FAIL(N >= 4 && N % 4 == 0 && K % group == 0 && group >= 32 && N * groups * 2 < ((int64_t)1 << 32) && slice_steps >= 1, "stream scales: bad arguments");
+  int gshift = 0;
+  while (((int64_t)1 << gshift) < group) ++gshift;
+  const int window = gshift >= 7 ? mg << (gshift - 7) : mg >> (7 - gshift);
+  const int64_t extent = N * groups * 2, blocks = (N + bn - 1) / bn;
+  std::vector<int64_t> value(32 * mg);  // what the area holds: index of the value in the tensor
+  for (int64_t b = 0; b < blocks; ++b) {
+    if (b >= 2 && b < blocks - 2) continue;
+    for (int step0 = 0; step0 < steps_total; step0 += slice_steps) {
+      const int steps = steps_total - step0 < slice_steps ? steps_total - step0 : slice_steps;
+      for (int w0 = 0; w0 < steps; w0 += window) {
+        const int wsteps = steps - w0 < window ? steps - w0 : window;
+        const int G = ((wsteps << 7) >> gshift) > 0 ? ((wsteps << 7) >> gshift) : 1, g0 = ((step0 + w0) << 7) >> gshift;
+        CHECK_OR_FAIL(G <= mg && g0 + G <= groups, "stream scales: window of %d groups from %d on of %d", G, g0, groups);
+        const bool wide = (shift & 7) == 0 && addr::stream_sz_wide(groups, g0);
+        const bool dwords = !wide && (shift & 1) == 0 && addr::stream_sz_dwords(mg, (int)N, groups, g0, G);
+        if (!wide && !dwords) continue;  // gathers, one value each
+        for (int block = 0; block < bn / 32; ++block) {
+          std::fill(value.begin(), value.end(), -1);
+          const int cells = wide ? mg / 8 : mg / 2, each = mg / cells;
+          for (int i = 0; i < 32 * cells / 64; ++i)
+            for (int lane = 0; lane < 64; ++lane) {
+              const int row = addr::stream_sz_row(cells, i, lane);
+              int64_t n = b * bn + block * 32 + row;
+              n = n < N ? n : N - 1;
+              const int64_t at = wide ? addr::stream_sz_piece_voff((int)n, groups, g0, addr::stream_sz_piece(mg, lane, row))
+                                      : addr::stream_sz_dword_voff((int)n, (int)N, groups, g0, addr::stream_sz_dword(mg, lane, row));
+              CHECK_OR_FAIL(at % (2 * each) == 0 && at + 2 * each <= extent, "stream scales: load at [%lld, +%d) of %lld", (long long)at, 2 * each, (long long)extent);
+              for (int e = 0; e < each; ++e) value[(i * 64 + lane) * each + e] = at / 2 + e;
+            }
+          for (int row = 0; row < 32; ++row) {
+            const int64_t n = b * bn + block * 32 + row;
+            if (n >= N) continue;
+            const int first = dwords ? addr::stream_sz_first((int)n, groups, g0) : 0;
+            for (int g = 0; g < G; ++g) {
+              CHECK_OR_FAIL(first + g < mg, "stream scales: value %d of a row's %d", first + g, mg);
+              const int64_t found = value[addr::stream_sz_value(mg, row, first + g)];
+              CHECK_OR_FAIL(found == n * groups + g0 + g, "stream scales: row %lld group %d finds value %lld", (long long)n, g0 + g, (long long)found);
+            }
+            // (the kernel works first out once for both weight tiles of a lane)
+            CHECK_OR_FAIL(!dwords || addr::stream_sz_first((int)n + 32, groups, g0) == first, "stream scales: row %lld and the one 32 on start differently", (long long)n);
+          }
+        }
+      }
+    }
+  }
+  return 0;
+}
+
 // Streaming W4A16 kernel: packed weights [N, K / 2], activations [M, K] of 2-byte values, 16 * tm activation rows per work-group,
 // steps of 128 values of K; two groups of wavefronts on 256 weight rows or four on 128.
 int check_stream(int64_t M, int64_t N, int64_t K, int tm) {
@@ -1325,6 +1378,22 @@ int tlq_debug_check_stream_schedule(int steps, int depth, int loads, int units, 
 
 int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activation_tiles, int ring_depth) {
   if (int rc = check_stream(M, N, K, activation_tiles)) return rc;
+  // (K slices as the plans cut them: whole groups, or a power-of-two part of one)
+  for (int64_t group = 32; group <= K; group *= 2) {
+    if (K % group) break;
+    const int unit = group > 128 ? (int)(group / 128) : 1, steps = (int)(K / 128);
+    for (int cut : {1, 2, 3, 5, 16}) {
+      int ss = (steps + cut - 1) / cut;
+      if (ss >= unit)
+        ss = (ss + unit - 1) / unit * unit;
+      else
+        while (ss & (ss - 1)) ++ss;
+      for (int kgs = 2; kgs <= 4; kgs += 2)
+        for (int shift : {0, 2})
+          if (N % 4 == 0)
+            if (int rc = check_stream_scales(N, K, group, kgs, ss, shift)) return rc;
+    }
+  }
   const int l = activation_tiles / 2;
   for (int steps = 1; steps <= 40; ++steps)
     for (int depth = ring_depth; depth <= 6; ++depth) {

@@ -247,31 +247,28 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
     // size: the plan takes slice lengths that divide the group, so the slice lies inside the group of its first step)
     const int G = ((wsteps << 7) >> gshift) > 0 ? ((wsteps << 7) >> gshift) : 1;
     const int g0 = ((step0 + w0) << 7) >> gshift;
-    const bool wide = ((groups | g0) & 7) == 0 && (((uintptr_t)scales | (uintptr_t)zeros) & 15) == 0;  // uniform
-    const bool odd_rows = ((groups | g0) & 1) != 0;  // some row's first group of the window is the second half of a dword
-    const bool dwords = !wide && (((uintptr_t)scales | (uintptr_t)zeros) & 3) == 0 && ((N & groups) & 1) == 0 && (!odd_rows || G < MG);
+    const bool wide = addr::stream_sz_wide(groups, g0) && (((uintptr_t)scales | (uintptr_t)zeros) & 15) == 0;  // uniform
+    const bool dwords = !wide && (((uintptr_t)scales | (uintptr_t)zeros) & 3) == 0 && addr::stream_sz_dwords(MG, N, groups, g0, G);
     // (the same for both weight tiles: 32 rows on, a row starts an even number of values on)
-    first_group = dwords ? ((n0 + wn * 64 + r32) * groups + g0) & 1 : 0;
+    first_group = dwords ? addr::stream_sz_first(n0 + wn * 64 + r32, groups, g0) : 0;
     const uint32_t l_sz = lds0 + (uint32_t)(Cfg::RING + sz_block * Cfg::SZ);
     if (wide) {
 #pragma unroll
       for (int i = 0; i < MG / 16; ++i) {
-        const int row = addr::stream_sz_row(MG / 8, i, lane), piece = addr::stream_sz_piece(MG, lane, row), last = (groups - g0) / 8 - 1;
+        const int row = addr::stream_sz_row(MG / 8, i, lane);
         int n = n0 + sz_block * 32 + row;
         n = n < N ? n : N - 1;
-        const uint32_t voff = ((uint32_t)n * (uint32_t)groups + (uint32_t)g0) * 2u + (uint32_t)((piece < last ? piece : last) * 16);
+        const uint32_t voff = addr::stream_sz_piece_voff(n, groups, g0, addr::stream_sz_piece(MG, lane, row));
         if (has_s && my_s) dma16(l_sz + (uint32_t)(i * 1024), voff, (const uint8_t*)scales);
         if (has_z && my_z) dma16(l_sz + (uint32_t)(Cfg::SZ / 2 + i * 1024), voff, (const uint8_t*)zeros);
       }
     } else if (dwords) {
-      const uint32_t last = (uint32_t)N * (uint32_t)groups * 2u - 4u;
 #pragma unroll
       for (int i = 0; i < MG / 4; ++i) {
         const int row = addr::stream_sz_row(MG / 2, i, lane);
         int n = n0 + sz_block * 32 + row;
         n = n < N ? n : N - 1;
-        uint32_t voff = ((((uint32_t)n * (uint32_t)groups + (uint32_t)g0) * 2u) & ~3u) + (uint32_t)(addr::stream_sz_dword(MG, lane, row) * 4);
-        voff = voff < last ? voff : last;
+        const uint32_t voff = addr::stream_sz_dword_voff(n, N, groups, g0, addr::stream_sz_dword(MG, lane, row));
         if (has_s && my_s) dma4(l_sz + (uint32_t)(i * 256), voff, (const uint8_t*)scales);
         if (has_z && my_z) dma4(l_sz + (uint32_t)(Cfg::SZ / 2 + i * 256), voff, (const uint8_t*)zeros);
       }
