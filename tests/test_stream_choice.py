@@ -120,3 +120,17 @@ def test_the_workspace_size_follows_the_switch():
     assert lib.tlq_debug_stream_plan(M, N, K, 32, lib.tlq_device_cu_count() or 256, plan) == 1
     assert on >= plan[2] * M * N * 4 > off
     assert lib.tlq_w4a16_workspace_bytes(M, N, K) == on
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 4096, 14336), (400, 8192, 8192), (64, 4096, 14336), (200, 4096, 4096), (96, 20480, 2048)])
+def test_the_size_by_name_is_the_most_slices_of_any_plan(M, N, K):
+    """No slices that no plan cuts: in the size by name, which is what a call by name needs for the group size that cuts most."""
+    lib = _abi.load()
+    plan = (ctypes.c_int64 * 5)()
+    slices = []
+    for shift in range(5, 14):
+        if K % (1 << shift) == 0 and lib.tlq_debug_stream_plan(M, N, K, 1 << shift, lib.tlq_device_cu_count() or 256, plan) == 1:
+            slices.append(plan[2])
+    most = max(slices)
+    assert lib.tlq_w4a16_workspace_bytes_for(M, N, K, _abi.ALGO_STREAM) == (most * M * N * 4 if most > 1 else 0)
+    assert lib.tlq_w4a16_workspace_bytes(M, N, K) >= most * M * N * 4 or most == 1

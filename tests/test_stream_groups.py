@@ -11,7 +11,7 @@ from tilelang_ascend_amd import _abi
 pytestmark = pytest.mark.gpu
 
 
-def run(A, Wp, s, z, group, tiles, slice_steps, layout=0, out_dtype=None, shift=0, algo=None):
+def run(A, Wp, s, z, group, tiles, slice_steps, layout=0, out_dtype=None, shift=0, algo=None, exact=False):
     lib, P = _abi.load(), _abi.ptr
     M, K = A.shape
     N = Wp.shape[0]
@@ -32,8 +32,10 @@ def run(A, Wp, s, z, group, tiles, slice_steps, layout=0, out_dtype=None, shift=
     lib.tlq_tune_w4a16_stream_tiles(tiles)
     lib.tlq_tune_w4a16_stream_slice(slice_steps)
     try:
-        need = max(int(lib.tlq_w4a16_workspace_bytes(M, N, K)), 16 * M * N * 4)
-        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        need = int(lib.tlq_w4a16_workspace_bytes(M, N, K))
+        if not exact:  # (forced slices may be more than any plan's)
+            need = max(need, 16 * M * N * 4)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
         lib.tlq_debug_launch_log(1)
         rc = lib.tlq_gemm_w4a16_layout_ws(P(dA), P(dW), P(dS), P(dZ), P(C), M, N, K, group, 0.0 if zt is not None or z is None else float(z), code[A.dtype], code[out_dtype],
                                           _abi.ALGO_STREAM if algo is None else algo, layout, P(ws), need, torch.cuda.current_stream().cuda_stream)
@@ -91,11 +93,11 @@ def test_one_hot_rows_return_the_dequantised_weights(in_dtype, groups, zeros_kin
         assert_bit_equal(run(A, Wp, s, z, group, 8 + groups, steps, layout, out_dtype), want.to(out_dtype), f"{in_dtype} groups {groups} {zeros_kind} -> {out_dtype}, {steps} steps")
 
 
-@pytest.mark.parametrize("M,N,K,group", [(663, 4096, 1792, 128), (1060, 4096, 640, 64), (556, 9216, 512, 256)])
+@pytest.mark.parametrize("M,N,K,group", [(663, 4096, 1792, 128), (1060, 4096, 640, 64), (556, 9216, 512, 256), (640, 896, 4352, 128)])
 def test_automatic_choice_above_512_rows(M, N, K, group):
     A = torch.randn(M, K, generator=gen(65)).half()
     Wp, s, z = make_w4(N, K, group, torch.float16, "int", seed=66)
-    got = run(A, Wp, s, z, group, 0, 0, algo=_abi.ALGO_AUTO)
+    got = run(A, Wp, s, z, group, 0, 0, algo=_abi.ALGO_AUTO, exact=True)
     assert "w4a16_stream_kernel" in run.log or _abi.load().tlq_device_cu_count() != 256, run.log
     check_float_output(got, w4a16_reference(A, Wp, s, z, group), f"{M}x{N}x{K}")
 

@@ -412,23 +412,27 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
 // N = 14336, K = 4096 and 20-40 % ahead from there on and for N = 4096, K = 14336)
 static const int64_t kTwoPassMinM = 256;
 
-// Most K slices the streaming kernel may cut for any group size (the smallest group allows the shortest slices).  For up to 512 rows no
-// fewer than fill the CUs with blocks of 256 weight rows, the cut of the largest share of calls.
+// most K slices the streaming kernel cuts for any group size (the smallest group allows the shortest slices)
 static int64_t stream_max_split(int64_t M, int64_t N, int64_t K) {
   int64_t most = 0;
   for (int64_t group = 32; group <= K; group *= 2) {
     if (K % group) continue;
     const StreamPlan p = w4a16_stream_plan(M, N, K, group, cu_count_or_default());  // (the count the launch plans with)
     if (p.ok && p.split > most) most = p.split;
-    if (p.ok && M <= 512 && K >= 1024) {
-      const int64_t steps = K / 128, blocks = ceil_div(N, (int64_t)256) * ceil_div(M, (int64_t)(M > 64 ? 128 : (M > 32 ? 64 : 32)));
-      int64_t fill = cu_count_or_default() / blocks;
-      if (fill > 16) fill = 16;
-      if (fill > steps / 4) fill = steps / 4;
-      if (fill > most) most = fill;
-    }
   }
   return most;
+}
+// What tlq_w4a16_workspace_bytes counts in its place up to 512 rows: no fewer slices than fill the CUs with blocks of 256 weight rows.  No plan
+// launches those (64 x 4096 x 14336: 16, its plans cut 8 at most); the size of such a call is part of what callers are promised,
+// so it stays.  The least size and the size by name count the plans' own.
+static int64_t stream_promised_split(int64_t M, int64_t N, int64_t K) {
+  const int64_t most = stream_max_split(M, N, K);
+  if (most == 0 || K < 1024) return most;
+  const int64_t blocks = ceil_div(N, (int64_t)256) * ceil_div(M, (int64_t)(M > 64 ? 128 : (M > 32 ? 64 : 32)));
+  int64_t fill = cu_count_or_default() / blocks;
+  if (fill > 16) fill = 16;
+  if (fill > K / 128 / 4) fill = K / 128 / 4;
+  return fill > most ? fill : most;
 }
 
 // Second of the two passes: the plain GEMM on the dequantised matrix at the head of the workspace.  What the workspace
@@ -442,9 +446,9 @@ static int plain_gemm_on_workspace(const void* A, void* workspace, int64_t works
 
 // fp32 partial sums of the K slices of the kernels for small and middle M (sized for the smallest group, which allows the
 // most slices); 0 when none of them cuts K
-static int64_t w4a16_partial_sum_bytes(int64_t M, int64_t N, int64_t K) {
+static int64_t w4a16_partial_sum_bytes(int64_t M, int64_t N, int64_t K, bool least = false) {
   int64_t split = w4a16_mid_split(M, N, K, 32);
-  const int64_t ssplit = M <= 512 ? stream_max_split(M, N, K) : 0;
+  const int64_t ssplit = M > 512 ? 0 : (least ? stream_max_split(M, N, K) : stream_promised_split(M, N, K));
   if (ssplit > split) split = ssplit;
   if (M <= 32) {  // the decode kernel cuts rows longer than 4096 values into chunks
     const DecodePlan dp = w4a16_decode_plan(M, N, K, 32, cu_count_or_default());
@@ -600,7 +604,7 @@ static int64_t w4a16_kernel_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 
 int64_t tlq_w4a16_workspace_bytes_min(int64_t M, int64_t N, int64_t K) {
   if (N <= 0 || K <= 0) return 0;
-  const int64_t partial = w4a16_partial_sum_bytes(M, N, K);
+  const int64_t partial = w4a16_partial_sum_bytes(M, N, K, true);
   if (partial > 0) return partial;
   return M >= kTwoPassMinM ? N * K * 2 : 0;
 }
