@@ -2,9 +2,9 @@
 //   amax[m]  = max(max_n |x[m, n]|, 1e-4)
 //   scale[m] = amax / 127                      (round_scale: the next power of two, 2^ceil(log2(amax / 127)))
 //   y[m, n]  = int8( rint( clamp(x[m, n] / scale[m], -127, 127) ) )      rint = round half to even
-// HBM bound: one wavefront (many rows), one work-group (long rows) or several (few long rows) own a row, reads it once
-// into registers with 16-byte loads, reduces the maximum across lanes, and writes 8 int8 per lane and
-// chunk.  Rows longer than 32768 values, or of a length that is no multiple of 8, are read twice.
+// HBM bound: one wavefront (many rows) or one work-group (long rows) owns a row, reads it once into registers with 16-byte
+// loads, reduces the maximum across lanes, and writes 8 int8 per lane and chunk.  Few long rows are shared by work-groups, each of
+// which reads the whole row.  Rows longer than 32768 values, or of a length that is no multiple of 8, are read twice.
 #include "tlq_common.h"
 
 namespace tlq {
@@ -136,25 +136,29 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const T* __restrict
   }
 }
 
-// Few long rows: `parts` work-groups (grid y) per row.  Each reads the whole row for its maximum -- from L2 for all but the first, and two
-// vector instructions a value -- and quantises chunks part, part + parts, ... of 8 values, ten instructions a value, one or
-// two chunks per lane.  One work-group per row left seven of eight CUs idle at M = 32 and each of its lanes 56 values of both kinds:
+// Few long rows: `parts` work-groups (grid y) per row.  Each reads the whole row for its maximum -- from a cache for all but the first: the
+// last-level one, or L2 where M is a multiple of eight and the row's work-groups land on one XCD (32 x 14336 2.97 us, 31 rows 3.50) --, two
+// vector instructions a value, and quantises chunks part, part + parts, ... of 8 values, ten instructions a value, one or two chunks per lane.  WHOLE: one
+// work-group per row (more rows than half the CUs), which quantises the chunks that it holds (256 x 14336 3.95 -> 3.74 us, 512 x 14336 6.7 -> 6.45
+// against loading them once more).  One work-group per row left seven of eight CUs idle at M = 32 and each of its lanes 56 values of both kinds:
 // 32 x 14336 bf16 4.1 -> 2.9 us, 128 x 16384 7.1 -> 3.6, 256 x 14336 7.1 -> 4.6 and, on rows of one chunk per lane, 512 x 4096 3.9 -> 3.4 (back to
 // back in a graph); from three rows per CU on it is level, from four long ones behind (1000 x 14336 11.2 against 11.6).
-template <typename T, int CH, int OC>
+template <typename T, int CH, int OC, bool WHOLE>
 __global__ __launch_bounds__(512) void act_quant_parts_kernel(const T* __restrict__ X, int8_t* __restrict__ Y, float* __restrict__ S, int N, int round_scale) {
   __shared__ float part[8];
   const int tid = threadIdx.x, chunks = N >> 3;
   const int64_t m = blockIdx.x;
   const T* x = X + m * N;
   const int parts = (int)gridDim.y, own = tid * parts + (int)blockIdx.y;  // the first of the lane's chunks
-  Raw8<T> r[CH], mine[OC];
+  Raw8<T> r[CH], mine[WHOLE ? 1 : OC];
 #pragma unroll
   for (int c = 0; c < CH; ++c)
     if (c * 512 + tid < chunks) r[c].load_shared(x + (c * 512 + tid) * 8);
+  if constexpr (!WHOLE) {
 #pragma unroll
-  for (int c = 0; c < OC; ++c)
-    if (c * 512 * parts + own < chunks) mine[c].load_shared(x + (c * 512 * parts + own) * 8);
+    for (int c = 0; c < OC; ++c)
+      if (c * 512 * parts + own < chunks) mine[c].load_shared(x + (c * 512 * parts + own) * 8);
+  }
   float amax = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c)
@@ -169,9 +173,15 @@ __global__ __launch_bounds__(512) void act_quant_parts_kernel(const T* __restric
   const float scale = row_scale(amax, round_scale);
   if (tid == 0 && blockIdx.y == 0) S[m] = scale;
   const float rcp = 1.0f / scale;
+  if constexpr (WHOLE) {
 #pragma unroll
-  for (int c = 0; c < OC; ++c)
-    if (c * 512 * parts + own < chunks) *(uint2_t*)(Y + m * N + (c * 512 * parts + own) * 8) = quant8(mine[c], scale, rcp);
+    for (int c = 0; c < CH; ++c)
+      if (c * 512 + tid < chunks) *(uint2_t*)(Y + m * N + (c * 512 + tid) * 8) = quant8(r[c], scale, rcp);
+  } else {
+#pragma unroll
+    for (int c = 0; c < OC; ++c)
+      if (c * 512 * parts + own < chunks) *(uint2_t*)(Y + m * N + (c * 512 * parts + own) * 8) = quant8(mine[c], scale, rcp);
+  }
 }
 
 // Any N: two passes over the row, one value per lane and step.
@@ -231,14 +241,13 @@ static int run_act_quant(const void* Xv, void* Yv, void* Sv, int64_t M, int64_t 
     const int64_t chunks = N / 8;
     if (M <= (int64_t)2 * cus && N >= 4096 && chunks <= 512 * 4) {
       const dim3 grid((unsigned)M, (unsigned)parts);
-      const int own = (int)ceil_div(chunks, (int64_t)512 * parts);
-#define TLQ_AQP(CH, OC) act_quant_parts_kernel<T, CH, OC><<<grid, 512, 0, st>>>(X, Y, S, (int)N, round_scale)
+#define TLQ_AQP(CH, OC, WHOLE) act_quant_parts_kernel<T, CH, OC, WHOLE><<<grid, 512, 0, st>>>(X, Y, S, (int)N, round_scale)
       if (chunks <= 512)
-        TLQ_AQP(1, 1);
+        parts == 1 ? TLQ_AQP(1, 1, true) : TLQ_AQP(1, 1, false);
       else if (chunks <= 1024)
-        own == 1 ? TLQ_AQP(2, 1) : TLQ_AQP(2, 2);
+        parts == 1 ? TLQ_AQP(2, 2, true) : TLQ_AQP(2, 1, false);
       else
-        own == 1 ? TLQ_AQP(4, 1) : (own == 2 ? TLQ_AQP(4, 2) : TLQ_AQP(4, 4));
+        parts == 1 ? TLQ_AQP(4, 4, true) : (parts == 2 ? TLQ_AQP(4, 2, false) : TLQ_AQP(4, 1, false));
 #undef TLQ_AQP
       return check_launch("tlq_act_quant_i8", "act_quant kernel") ? 0 : 1;
     }
