@@ -122,7 +122,7 @@ void tlq_tune_gemm_slots(int mode);                          /* the kernel that 
                                                               * 16-bit GEMMs), 0 never */
 void tlq_tune_w4a16_decode(int on);                          /* 0: the decode kernel is never picked automatically */
 void tlq_tune_w4a16_stream(int on);                          /* 0: tlq_gemm_w4a16_ws never picks the streaming kernel by itself */
-void tlq_tune_w4a16_stream_tiles(int tiles);                 /* 16-row activation tiles per work-group of the streaming kernel, 2 .. 8 (0 = by its estimate) */
+void tlq_tune_w4a16_stream_tiles(int tiles);                 /* 16-row activation tiles per work-group of the streaming kernel, 2, 4, 6 or 8, + 16 for four groups of wavefronts over K (128 weight rows per work-group) instead of two (256); 0 = by its estimate */
 void tlq_tune_w4a16_stream_slice(int steps);                 /* K slice of the streaming kernel in steps of 128 values (0 = by its estimate) */
 void tlq_tune_w4a16_panel(int mode);                         /* tlq_gemm_w4a16_ws, large M: 0 = automatic, otherwise a panel kernel is never picked automatically */
 void tlq_tune_w4a16_panelm_rows(int rows);                   /* activation rows per work-group of the middle-M panel kernel: 64, 128, 0 = its plan's */

@@ -132,11 +132,10 @@ __host__ __device__ inline void slots_schedule(int KT, Ops& ops) {
 }
 
 // ---- streaming W4A16 kernel for small and middle M (gemm_w4a16_stream.hip) ---------------------------------------
-// One step is 128 values of K.  A work-group of 8 wavefronts owns 256 weight rows (wavefront w: rows 32 w .. 32 w + 31,
-// two 16-row MFMA tiles) and 16 * TM activation rows.
-// Packed weights: [16 rows][64 B] per MFMA tile, private to the wavefront.  One direct load covers a tile (lane l lands
-// on row l / 4, 16-byte piece l % 4 and fetches logical piece (l % 4) ^ sw_swz(row)); the operand read of lane
-// (row r16, k-group q) takes logical piece q: the four 32-bit words 4 q .. 4 q + 3 = values 32 q .. 32 q + 31 of the step.
+// One step is 128 values of K.  A work-group of 8 wavefronts owns 256 or 128 weight rows and 16 * TM activation rows.
+// Packed weights: tiles of [16 rows][64 B].  One direct load covers a tile (lane l lands on row l / 4, 16-byte piece l % 4
+// and fetches logical piece (l % 4) ^ sw_swz(row)).  The 16-row operand read (small-tile and panel kernels) of lane (row r16,
+// k-group q) takes logical piece q: the four 32-bit words 4 q .. 4 q + 3 = values 32 q .. 32 q + 31 of the step.
 // The swizzles of both tiles were chosen by measuring the 16-byte reads of eight wavefronts over whole families of
 // layouts (every 4 x 4 bit matrix for the activations, 24 row orders x 256 piece swizzles for the weights): with
 // pieces swizzled by row / 4 and chunks by the row number itself a read took 61 clocks instead of 37 in bank conflicts.

@@ -939,11 +939,12 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   }
   // 33 rows and more: the small-tile kernel or the streaming kernel, whichever estimate is lower, up to 512 rows (the best of eight
   // families on 398 of 400 random problems), above 512 rows where the streaming kernel's estimate beats the panel kernels' and the two
-  // passes' (stream_beats_panels).  Four regions stay with what ran before, though the streaming kernel is level or ahead there: the
-  // automatic choice's tests name those kernels.  More than 195 rows on 2^25 weights and more: the panel kernels (256 x 14336 x 4096
-  // 43.7 against 36.4 us); 2^26 weights and more: the rules further down (level: 128 x 50304 x 4096 61.6 against 61.8 us); above 512
-  // rows the two passes, where they ran, on weight-row counts that are no multiple of 128 or no more than 256 (639 x 5680 x 896 22.2
-  // against 15.5 us); and, where the panel kernels ran, a launch for the last one to three rows.
+  // passes' (stream_beats_panels).  The rules further down decide on 2^26 weights and more (2^25 from 196 rows on): the middle-M kernel where
+  // panelm_preferred or panelm_whole_rounds say so, though the streaming kernel is ahead on some of it (256 x 14336 x 4096 43.7 against 36.4
+  // us, which the test of that choice names), then the 128-row, the 256-row or the streaming kernel.  Above 512 rows two regions keep what
+  // ran before the streaming kernel took such calls, though it is level or ahead: the two passes, where they ran, on weight-row counts
+  // that are no multiple of 128 or no more than 256 (639 x 5680 x 896 22.2 against 15.5 us), and, where the panel kernels ran, a launch for
+  // the last one to three rows.  The automatic choice's tests name those kernels too.
   bool stream_region = algo == TLQ_ALGO_AUTO && g_w4a16_stream && !keep_tail && M > 32 && M <= kStreamMaxRows && N > 0 && K > 0 && group > 0 && N < kMaxDim && K < kMaxDim &&
                        N * K < ((int64_t)1 << (M > 195 ? 25 : 26));
   // (the estimate first: it is kept per shape, the choice among the others is not and takes 1.8 us of host time)

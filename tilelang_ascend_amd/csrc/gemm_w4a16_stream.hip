@@ -227,15 +227,15 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
   const uint32_t sz_lane = lds0 + (uint32_t)(Cfg::RING + 2 * wn * Cfg::SZ);
 
   // The slice runs in windows of as many steps as the scale area holds groups for (16 groups: 4, 8, 16 steps for groups
-  // of 32, 64, 128 values, more for larger groups).  Every window fetches its scales and restarts the ring: a memory
+  // of 32, 64, 128 values, more for larger groups; 32 groups, twice as many, with four groups of wavefronts).  Every window fetches its scales and restarts the ring: a memory
   // round trip without multiplications per window, which costs less than a further K slice (a partial tile to write
   // and add, and more work-groups than CUs).
   const int window = __builtin_amdgcn_readfirstlane(gshift >= 7 ? MG << (gshift - 7) : MG >> (7 - gshift));
-  // fetch: the window's scales and zero points and its first D steps; returns whether the zero points are small integers
+  // fetch: the window's scales and zero points and what a step finds in flight of its first D steps; returns whether the zero points are small integers
   auto fetch = [&](int w0, int wsteps) -> bool {
     if (w0 > 0) __syncthreads();  // every wavefront has multiplied the previous window's last steps: the slots are free
 
-    // ---- scales / zero points of this wavefront's 32 rows for the window, and the first D - 1 steps ----
+    // ---- scales / zero points of this wavefront's 32 rows for the window, then the first two steps ----
     // Area of 32 rows: [s | z][32 rows][MG groups], 2 bytes each.  A row's groups of the window are contiguous in memory: where they
     // are 16-byte aligned, MG / 16 direct loads per tensor fetch them in 16-byte pieces (past the row's end its last piece again),
     // issued ahead of the ring so that the first step's wait covers them.  Rows of any other length: MG / 4 direct loads of
@@ -346,11 +346,11 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
     const bool integral = fraction == 0 && largest <= 256.0f;
     return __builtin_amdgcn_ballot_w64(integral) == ~0ull;
   };
-  // The steps of a window.  A wavefront's step is eight units of TB MFMAs (unit u: k-step u / 2 of its four, weight tile u % 2).
-  // While unit u runs, the operand of unit u + 1 is expanded, a few vector instructions behind every MFMA, and the
-  // activation operands of the next k-step are read; units 6 and 7 read those of the next step, its packed words and scales.
-  // The step's one barrier stands in front of unit 6: behind it step s + 1 is complete for everyone, and everyone has read
-  // its last of step s, whose slot takes step s + D.
+  // The steps of a window.  A wavefront's step is NU units of TB MFMAs (unit u: k-step u / 2 of its KT, weight tile u % 2): eight with two
+  // groups of wavefronts, four with four.  While unit u runs, the operand of unit u + 1 is expanded, a few vector instructions
+  // behind every MFMA, and the activation operands of the next k-step are read; the last two units read those of the next step, its
+  // packed words and scales.  The step's one barrier stands in front of those two: behind it step s + 1 is complete for everyone, and
+  // everyone has read its last of step s, whose slot takes step s + D.
   auto multiply = [&](int w0, int wsteps, auto fold_tag) {
     constexpr bool FOLD = decltype(fold_tag)::value;
     typedef StreamExpand<T, FOLD, LAYOUT> Ex;
@@ -699,7 +699,7 @@ static int launch_stream(const void* A, const void* Wp, const void* scales, cons
   return check_launch("tlq_gemm_w4a16(stream)", detail) ? 0 : 1;
 }
 
-// partial: fp32 [split][M][N] workspace, needed when the plan has more than one K slice
+// partial: fp32 [split][N / 4][M][4] workspace, needed when the plan has more than one K slice
 int gemm_w4a16_stream(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int w_layout, const StreamPlan& p,
                       float* partial, hipStream_t st) {
