@@ -112,6 +112,14 @@ def test_streaming_kernel_schedule(blocks, groups, depth):
                 assert what in _abi.last_error()
 
 
+@pytest.mark.parametrize("n_blocks", [1, 3, 7, 8, 9, 32, 61])
+def test_streaming_kernel_order(n_blocks):
+    """Work-group to block, in the order of the grid and by XCD: every block once, also where the blocks are no multiple of eight."""
+    for slices in (1, 2, 3, 8, 13, 16):
+        for m_blocks in (1, 2, 3, 7):
+            _ok(_abi.load().tlq_debug_check_stream_order(n_blocks, slices, m_blocks))
+
+
 @pytest.mark.parametrize("kind", [0, 1, 2, 3, 4])
 def test_small_tile_kernels_addressing_and_schedule(kind):
     """Both small-tile kernels: loads inside their matrices (rows past them clamped), operand reads on the cells that hold what they

@@ -93,6 +93,21 @@ def test_one_hot_rows_return_the_dequantised_weights(in_dtype, groups, zeros_kin
         assert_bit_equal(run(A, Wp, s, z, group, 8 + groups, steps, layout, out_dtype), want.to(out_dtype), f"{in_dtype} groups {groups} {zeros_kind} -> {out_dtype}, {steps} steps")
 
 
+@pytest.mark.parametrize("M,N,K,group,in_dtype,by_xcd", [
+    (403, 1280, 12544, 256, torch.float16, True),   # 33.9 us in the order of the grid, 25.7 by XCD
+    (482, 1024, 16256, 128, torch.float16, True),   # 40.3, 29.1
+    (450, 652, 15360, 64, torch.bfloat16, True),    # blocks of weight rows that are no multiple of eight, the last one cut
+    (250, 14592, 2048, 128, torch.bfloat16, True),  # no K slices
+    (257, 640, 10240, 128, torch.float16, False),   # 16.1, 18.5 by XCD
+])
+def test_order_of_the_work_groups(M, N, K, group, in_dtype, by_xcd):
+    A = torch.randn(M, K, generator=gen(71)).to(in_dtype)
+    Wp, s, z = make_w4(N, K, group, in_dtype, "int", seed=72)
+    got = run(A, Wp, s, z, group, 0, 0)
+    assert ("by XCD" in run.log) == by_xcd or _abi.load().tlq_device_cu_count() != 256, run.log
+    check_float_output(got, w4a16_reference(A, Wp, s, z, group), f"{M}x{N}x{K}")
+
+
 @pytest.mark.parametrize("M,N,K,group", [(663, 4096, 1792, 128), (1060, 4096, 640, 64), (556, 9216, 512, 256), (640, 896, 4352, 128)])
 def test_automatic_choice_above_512_rows(M, N, K, group):
     A = torch.randn(M, K, generator=gen(65)).half()

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "gemm_addr.h"
+#include "stream_plan.h"
 #include "tlq_common.h"
 
 namespace tlq {
@@ -1374,6 +1375,28 @@ int tlq_debug_check_gemm_addressing(int source_kind, int64_t rows, int64_t row_b
 int tlq_debug_check_stream_schedule(int steps, int depth, int loads, int units, int wait_scales, int wait_first, int wait_step) {
   return check_stream_ring(steps, depth, loads, units, wait_scales < 0 ? addr::stream_wait_scales(loads) : wait_scales,
                            wait_first < 0 ? addr::stream_wait_first(loads) : wait_first, wait_step < 0 ? addr::stream_wait_step(depth, loads) : wait_step);
+}
+
+int tlq_debug_check_stream_order(int64_t n_blocks, int64_t slices, int64_t m_blocks) {
+  CHECK_OR_FAIL(n_blocks >= 1 && slices >= 1 && m_blocks >= 1 && n_blocks * slices * m_blocks <= 1 << 20, "stream order: bad arguments");
+  const int64_t total = n_blocks * slices * m_blocks;
+  for (int by_xcd = 0; by_xcd < 2; ++by_xcd) {
+    std::vector<uint8_t> taken(total, 0);
+    std::vector<uint8_t> meets(8 * slices, 0);  // slices that an XCD works on
+    for (int64_t id = 0; id < total; ++id) {
+      const tlq::StreamItem it = tlq::stream_item((uint32_t)id, (uint32_t)n_blocks, (uint32_t)slices, (uint32_t)m_blocks, by_xcd != 0);
+      CHECK_OR_FAIL(it.n >= 0 && it.n < n_blocks && it.slice >= 0 && it.slice < slices && it.m >= 0 && it.m < m_blocks, "stream order: work-group %lld takes block (%d, %d, %d)",
+                    (long long)id, it.n, it.slice, it.m);
+      uint8_t& once = taken[(it.m * slices + it.slice) * n_blocks + it.n];
+      CHECK_OR_FAIL(!once, "stream order: block (%d, %d, %d) taken twice", it.n, it.slice, it.m);
+      once = 1;
+      meets[(id & 7) * slices + it.slice] = 1;
+    }
+    int64_t pairs = 0;
+    for (uint8_t m : meets) pairs += m;
+    CHECK_OR_FAIL(!by_xcd || pairs <= slices + 7, "stream order: %lld pairs of XCD and slice, %lld slices", (long long)pairs, (long long)slices);
+  }
+  return 0;
 }
 
 int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activation_tiles, int ring_depth) {

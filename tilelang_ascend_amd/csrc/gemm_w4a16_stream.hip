@@ -137,7 +137,7 @@ template <typename T, int TB, int KG, int LAYOUT, bool MANY>
 __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restrict__ A, const uint8_t* __restrict__ Wp,
                                                              const T* __restrict__ scales, const T* __restrict__ zeros,
                                                              void* __restrict__ C, float* __restrict__ partial, int M, int N, int K,
-                                                             int gshift, float zero_scalar, int out_dtype, int slice_steps) {
+                                                             int gshift, float zero_scalar, int out_dtype, int slice_steps, int by_xcd) {
   typedef StreamCfg<TB, KG> Cfg;
   typedef StreamMma<T> Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
@@ -147,7 +147,9 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r32 = lane & 31, h = lane >> 5;
   const int kg = wave / WN, wn = wave % WN;  // values 16 KT kg .. of every step; weight rows 64 wn .. 64 wn + 63
-  const int n0 = blockIdx.x * Cfg::BN, m0 = blockIdx.z * Cfg::BM, slice = blockIdx.y;
+  StreamItem item{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
+  if (by_xcd) item = stream_item(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z, true);
+  const int n0 = item.n * Cfg::BN, m0 = item.m * Cfg::BM, slice = item.slice;
   const int steps_total = K >> 7;
   const int step0 = slice * slice_steps;
   const int steps = steps_total - step0 < slice_steps ? steps_total - step0 : slice_steps;
@@ -635,8 +637,21 @@ static double stream_us(int64_t M, int64_t N, int64_t K, int tm, int kg, int64_t
          (slices > 1 ? 2.36 + 1.7e-6 * (double)slices * (double)M * (double)N : 0.0) + 0.385e-9 * (double)(m_blocks * tm * 16) * (double)(n_blocks * (512 / kg)) * (double)K +
          0.6e-6 * (double)M * (double)N + 0.022e-6 * (double)N * (double)K + 0.086e-6 * (double)M * (double)K;
 }
+// The order by XCD where it keeps enough bytes from going into several L2s: the activations, which go into all eight (fewer with fewer blocks
+// of weight rows) instead of the two or so that share a slice, and the weights, which the blocks of activation rows of a slice share.  Blocks of
+// 128 weight rows, twice as many as the kernel had before, had made that 403 x 1280 x 12544 30.1 -> 33.9 us (by XCD 25.7) and 482 x 1024 x 16256 34.4 ->
+// 40.3 (29.1).  On 1524 problems (M 17 .. 3000, N .. 32000, K .. 17920; the line is from 1491 others) it is 3.4 % ahead on average on the 561 beyond the
+// line (4.8 % with K slices, 27 % at most), 3 % and more behind on 5.  Short of the line XCDs whose work-groups all read one slice at a time
+// are up to 13 % behind (257 x 640 x 10240 18.5 against 16.1 us); without slices the two are level there.
+static bool stream_by_xcd(const StreamPlan& p, int64_t M, int64_t N, int64_t K) {
+  auto gcd8 = [](int64_t n) { return n % 8 == 0 ? 8.0 : (n % 4 == 0 ? 4.0 : (n % 2 == 0 ? 2.0 : 1.0)); };
+  const double nb = p.n_blocks, sl = p.split, shares = (sl + 8.0 - gcd8(p.split)) / sl;
+  const double a = 2e-6 * (double)M * (double)K * ((nb < 8.0 ? nb : 8.0) - (nb < shares ? nb : shares));
+  const double meet = 8.0 / gcd8((int64_t)p.n_blocks * p.split), w = 0.5e-6 * (double)N * (double)K * ((p.m_blocks < meet ? p.m_blocks : meet) - 1.0);
+  return a + w > (p.split > 1 ? 40.0 : 12.0);  // MB
+}
 static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group, int64_t cus) {
-  StreamPlan best{false, 0, 0, 0, 0, 0, 2, 0.0};
+  StreamPlan best{false, 0, 0, 0, 0, 0, 2, 0.0, false};
   if (M < 17 || M > kStreamMaxRows || N < 1 || K < 128 || K % 128 != 0 || group < 32 || (group & (group - 1)) != 0 || K % group != 0) return best;
   if (N % 4 != 0) return best;
   const int64_t steps_total = K / 128;
@@ -666,9 +681,10 @@ static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group
         const int64_t slices = ceil_div(steps_total, ss);
         if (slices > 16) continue;  // too many partial sums to add up: the tile kernel with longer slices takes it
         const double us = stream_us(M, N, K, tm, kg, m_blocks, n_blocks, ss, slices, ceil_div(ss, window), cus);
-        if (!best.ok || us < best.us) best = StreamPlan{true, tm, (int)m_blocks, (int)n_blocks, (int)slices, (int)ss, kg, us};
+        if (!best.ok || us < best.us) best = StreamPlan{true, tm, (int)m_blocks, (int)n_blocks, (int)slices, (int)ss, kg, us, false};
       }
     }
+  if (best.ok) best.by_xcd = stream_by_xcd(best, M, N, K);
   return best;
 }
 StreamPlan w4a16_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus) {
@@ -693,9 +709,9 @@ static int launch_stream(const void* A, const void* Wp, const void* scales, cons
     attr_set = true;
   }
   kern<<<dim3(p.n_blocks, p.split, p.m_blocks), 512, lds_bytes, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, partial, (int)M,
-                                                                     (int)N, (int)K, gshift, zero_scalar, out_dtype, p.slice_steps);
-  char detail[64] = "";
-  if (launch_log_on()) snprintf(detail, sizeof(detail), "w4a16_stream_kernel, %d activation rows per work-group", 32 * TB);
+                                                                     (int)N, (int)K, gshift, zero_scalar, out_dtype, p.slice_steps, p.by_xcd);
+  char detail[80] = "";
+  if (launch_log_on()) snprintf(detail, sizeof(detail), "w4a16_stream_kernel, %d activation rows per work-group%s", 32 * TB, p.by_xcd ? ", by XCD" : "");
   return check_launch("tlq_gemm_w4a16(stream)", detail) ? 0 : 1;
 }
 

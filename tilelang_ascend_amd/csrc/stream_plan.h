@@ -13,7 +13,20 @@ struct StreamPlan {
   int split, slice_steps; // K slices, steps of 128 values in each
   int kg;                 // groups of wavefronts over K: 2 (256 weight rows per work-group) or 4 (128)
   double us;              // estimate
+  bool by_xcd;            // the order of the work-groups (stream_item)
 };
+// Which block of weight rows, K slice and block of activation rows work-group `id` of n_blocks x slices x m_blocks takes.  Work-groups go to the
+// eight XCDs round-robin.  Weight rows fastest: with eight blocks of weight rows and more every XCD meets all slices of all activations, and fetches them
+// into its L2.  By XCD: each takes an eighth of the work in a row -- slice after slice, in a slice a run of weight rows with all their activation rows.
+struct StreamItem {
+  int n, slice, m;
+};
+__host__ __device__ inline StreamItem stream_item(uint32_t id, uint32_t n_blocks, uint32_t slices, uint32_t m_blocks, bool by_xcd) {
+  if (!by_xcd) return StreamItem{(int)(id % n_blocks), (int)(id / n_blocks % slices), (int)(id / n_blocks / slices)};
+  const uint32_t total = n_blocks * slices * m_blocks, xcd = id & 7u, rest = total & 7u;
+  const uint32_t at = xcd * (total >> 3) + (xcd < rest ? xcd : rest) + (id >> 3), t = at / m_blocks;
+  return StreamItem{(int)(t % n_blocks), (int)(t / n_blocks), (int)(at % m_blocks)};
+}
 StreamPlan w4a16_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus);
 int gemm_w4a16_stream(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int w_layout, const StreamPlan& p,
