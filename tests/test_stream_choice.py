@@ -90,6 +90,17 @@ def test_against_whole_rounds_of_the_middle_m_kernel(M, N, K, group, dtype, algo
     check(M, N, K, group, 0, algo, dtype)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,dtype", [
+    # against small tiles, groups of 32 with zero points
+    (154, 6016, 3200, torch.float16),   # 25.5, 34.5 us
+    (44, 12224, 3584, torch.bfloat16),  # 20.0, 24.0
+    (213, 4304, 2304, torch.bfloat16),  # 19.8, 23.2
+])
+def test_against_small_tiles_in_groups_of_32(M, N, K, dtype):
+    check(M, N, K, 32, 0, _abi.ALGO_STREAM, dtype)
+
+
 @pytest.mark.parametrize("M,N,K,group", [
     (188, 18128, 3200, 64),  # 284 work-groups of 96 x 128 rows 49.6 us, 142 of 96 x 256 35.0
     (133, 18432, 1920, 32),  # 288 35.7, 144 25.4

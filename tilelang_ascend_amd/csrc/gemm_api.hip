@@ -275,7 +275,10 @@ static double fused_tile_us(int64_t M, int64_t N, int64_t K) {  // the W4A16 til
 // 0.08 us per MB of weights (fitted, 0.7 us rms on 900 problems), the streaming kernel 1 us and 0.01.  So where a wavefront has 24 steps
 // and more on 16 MB of weights and more, it has to be ahead by more than the estimates are off.  With shorter shares small tiles
 // are ahead from a cache by less than they are behind from memory (22 and 23 steps: 3 % and 14 %), on fewer rows by more.
-static bool small_beats_stream(const SmallTile& p, const StreamPlan& sp, int64_t M, int64_t N, int64_t K) {
+// Groups of 32 values: a scale per lane and step and, with a tensor, a zero point, which the small-tile kernel's estimate does not know: 15 % above the
+// others with zero points and 8 % without, the streaming kernel level.  30 of 285 such problems go to the streaming kernel by it, 1.11 x on average (154 x 6016 x
+// 3200 34.5 us with small tiles, 25.5 with the streaming kernel).
+static bool small_beats_stream(const SmallTile& p, const StreamPlan& sp, int64_t M, int64_t N, int64_t K, int64_t group, bool zero_points) {
   if (!p.ok || g_stream_slice_steps > 0 || g_stream_tiles > 0) return false;
   const bool long_shares = M > 32 && ceil_div(K / 128, (int64_t)p.waves) >= 24 && N * K >= ((int64_t)32 << 20);
   double theirs = sp.us;
@@ -283,7 +286,8 @@ static bool small_beats_stream(const SmallTile& p, const StreamPlan& sp, int64_t
     const double earlier = 11.9 + 2.0 * giga((double)M, N, K) + 1.14 * giga(up16(M), N, K) + 0.31e-3 * (double)K;
     if (!sp.ok || earlier > theirs) theirs = earlier;
   }
-  return small_us(p, M, N, K) < (long_shares ? 0.85 : 1.04) * theirs;
+  const double mine = small_us(p, M, N, K) * (group >= 64 ? 1.0 : (zero_points ? 1.15 : 1.08));
+  return mine < (long_shares ? 0.85 : 1.04) * theirs;
 }
 // above 512 rows: the tile kernel on up to 2^19 weights -- and the launch for the last M % 4 rows, 4 us, where they run apart --, else the
 // two passes or the panel kernels, which are level with them or ahead; only while the whole call stays short
@@ -968,7 +972,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       if (tiles)
         return tlq_gemm_w4a16(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype,
                               small_or(TLQ_ALGO_MFMA, M, N, K, group, scales, zeros), stream);
-      if (M <= 512 && small_beats_stream(small, sp, M, N, K))
+      if (M <= 512 && small_beats_stream(small, sp, M, N, K, group, zeros != nullptr))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
       return gemm_w4a16_stream(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, sp, (float*)workspace,
@@ -1113,7 +1117,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     const bool ws_ok = stream_workspace_ok(sp, M, N, workspace, workspace_bytes);
     if (algo == TLQ_ALGO_AUTO && sp.ok && args_ok) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
-      if (small_beats_stream(small, sp, M, N, K))
+      if (small_beats_stream(small, sp, M, N, K, group, zeros != nullptr))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
     }
@@ -1297,7 +1301,7 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
     // the small-tile kernel in the place of either, for calls that bring the workspace those want: without it they are refused
     if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (ws_ok || (room_for_two_passes && N % 8 == 0))) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
-      if (small_beats_stream(small, sp, M, N, K))
+      if (small_beats_stream(small, sp, M, N, K, group, zeros != nullptr))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
     }
