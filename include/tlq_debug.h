@@ -114,7 +114,7 @@ void tlq_tune_gemv_depth(int steps_in_flight);               /* load steps (1 KB
 void tlq_tune_gemv_ring(int on);                             /* 1 (default): a single decode GEMV (1 or 2 activation rows) runs on the
                                                               * ring kernel where it applies; 0: on the kernels it replaced (for one
                                                               * activation row the same results, bit for bit) */
-void tlq_tune_gemm_groups(int variant);                       /* K over groups of wavefronts in the MFMA kernels of 128-row tiles: 0 = automatic, 1 = never, 2 .. 5: 128x128, 128x64, 64x128 tiles x 2, 64x64 x 4 */
+void tlq_tune_gemm_groups(int variant);                       /* the ring kernel in the place of 128-row tiles: 0 = automatic, 1 = never, 2 .. 5: its 128x128, 128x64, 64x128, 64x64 tiles */
 void tlq_tune_gemm_band(int tile_rows);                       /* tile rows per band of the MFMA kernels' tile order (default 4) */
 void tlq_tune_gemm_tile(int tile);                            /* square tile of the plain 16-bit GEMM (and of the second of the two W4A16 passes):
                                                               * 128 | 256, 0 = by the number of output tiles */

@@ -131,6 +131,9 @@ __host__ __device__ inline void slots_schedule(int KT, Ops& ops) {
   }
 }
 
+// ---- ring kernel (gemm_ring.h): slots of one stage of both operand tiles in the CU's 160 KB of LDS ----
+constexpr int ring_slots(int slot_bytes) { return 160 * 1024 / slot_bytes; }
+
 // ---- streaming W4A16 kernel for small and middle M (gemm_w4a16_stream.hip) ---------------------------------------
 // One step is 128 values of K.  A work-group of 8 wavefronts owns 256 or 128 weight rows and 16 * TM activation rows.
 // Packed weights: tiles of [16 rows][64 B].  One direct load covers a tile (lane l lands on row l / 4, 16-byte piece l % 4

@@ -692,7 +692,7 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 }
 
 // Above 512 rows: do the two passes beat what the panel kernels would run?  The dequantisation pass costs 3 us and the weights' bytes, the
-// plain GEMM behind it has smaller tiles, K in groups of wavefronts and any row count, while the panel kernels have 8 us per round of
+// plain GEMM behind it has smaller tiles and any row count, while the panel kernels have 8 us per round of
 // work-groups (many rounds of short rows: 4868 x 3152 x 384 bf16 36.9 -> 25.5 us, 6631 x 4608 x 256 38.7 -> 29.8) and leave
 // one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  On 1500 problems
 // (M 513 .. 8192, N 128 .. 14400, K 256 .. 19200, half of the row counts odd) the bar below takes the two passes on 278, ahead by 1.15 - 1.32 x
@@ -1169,8 +1169,8 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       if (rc >= 0) return rc;
     }
   }
-  // (above 512 rows only rows of 13312 values and more: below, the plain GEMM of the two passes, which cuts K over groups of wavefronts
-  // or unevenly over work-groups, is ahead: 614 x 1392 x 2304 28.7 -> 20.6 us, 667 x 256 x 12288 36.8 -> 25.3, 682 x 2288 x 11648
+  // (above 512 rows only rows of 13312 values and more: below, the plain GEMM of the two passes, in the ring kernel
+  // or over uneven slices of K, is ahead: 614 x 1392 x 2304 28.7 -> 20.6 us, 667 x 256 x 12288 36.8 -> 25.3, 682 x 2288 x 11648
   // 76.4 -> 66.3; 656 x 2496 x 3712 level)
   const bool split_region = !(algo == TLQ_ALGO_AUTO && have && M > 512 && K < 13312 && N % 8 == 0 && w4a16_split_forced() == 0) &&
                             w4a16_mid_split(M, N, K, group > 0 ? group : 32) > 1;
@@ -1345,7 +1345,7 @@ int tlq_gemv_w4a16_batched(const void* A, const void* w_packed, const void* scal
                     (hipStream_t)stream);
 }
 
-// The estimate of the 128-row tiles with K over groups of wavefronts (gemm_core.h), where those would run; far off otherwise.
+// The estimate of the ring kernel (gemm_core.h), where it would run; far off otherwise.
 static double group_tile_us(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes) {
   double us = 0.0;
   if (M <= 32 || N < 1 || k_bytes < 1 || !prefer_small_tiles(batch, M, N) || group_tile(kind, batch, M, N, k_bytes, &us) == 0) return 1e30;
@@ -1374,8 +1374,8 @@ static double plain_nk_us(int64_t M, int64_t N, int64_t K) {  // one 16-bit matr
   return us;
 }
 static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes) {
-  // (rows of more than 48 stages stay with the slices, which their estimate makes too dear on many activation rows: 3326 x 768 x 5504 44
-  // against 56 us in groups, 947 x 1664 x 6016 36 against 43, 7795 x 256 x 7808 54 against 78)
+  // (rows of more than 48 stages stay with the slices, which their estimate makes too dear: int8 [K, N] 131 x 7568 x 7552 27.6 us in slices, 33 - 51
+  // in the ring kernel's tiles, 1856 x 544 x 24064 52.8 against 74)
   return k_bytes <= 48 * kStageBytes && group_tile_us(tile, 1, M, N, k_bytes) < 0.9 * sliced_us(kind, 1, M, N, K);
 }
 // The products that may take the small-tile kernel: weights as stored (the first four: SmallW), int32 results, or rescaled ones
@@ -1394,7 +1394,7 @@ static SmallUse w4a8_use(bool two_steps, int sign_mode, int64_t K) {
 // Is the small-tile kernel ahead of what would run in its place?  Two things its own estimate leaves out come on top: the activations' trip from
 // memory (at 2.5 TB/s: every tile of weight rows asks for them again) and, with 16-bit weights, that theirs cannot take less than
 // a copy.  The other side, by what would run: calls that cut K into slices over work-groups (sliced_us), up to 32 rows a fit to the 32-row
-// tiles, else the tiles' own estimates -- plain, with K over groups of wavefronts, 256 x 256 --, for W4A8 in two steps behind the
+// tiles, else the tiles' own estimates -- plain, of the ring kernel, 256 x 256 --, for W4A8 in two steps behind the
 // unpack pass.  The bars are fitted to problems (M 1 .. 8192, N 64 .. 14400, K 128 .. 14336, one to eight batches) timed with the
 // small-tile kernel, without it and by the choice.  On 9000 others, 1500 per use, it is taken on 5206, ahead by 1.40 - 1.80 x on average
 // and more than 5 % behind on 135 (81 by more than 10 %); the choice is 0.4 - 1.6 % behind the faster of both on average.  (The rule

@@ -246,18 +246,22 @@ struct RowLoaderDirect {
   // may also return through the LDS counter), which serialises the operand reads and LDS stores of the
   // whole stage.  The kernel waits for them by hand (wait_direct) before the barrier that publishes
   // the buffer.
+  __device__ __forceinline__ const uint8_t* stage_src(int kt) const { return uniform_ptr(base + (int64_t)kt * kStageBytes); }
+  __device__ __forceinline__ uint32_t stage_dst(uint8_t* lds) const {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + wave_off);
+  }
+  __device__ __forceinline__ void load_one(int j, const uint8_t* src, uint32_t dst) const {  // of the PER_WAVE loads of a stage
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + addr::direct_lds_off(0, 0, j, WAVES)), "v"(voff[j]), "s"(src)
+                 : "memory");
+  }
   template <bool TAIL>
   __device__ __forceinline__ void gload(Regs& r, int kt, uint8_t* lds_next) const {
-    typedef __attribute__((address_space(3))) uint8_t* lptr_t;
     if (!TAIL) {
       r.pending = false;
-      const uint8_t* sb = uniform_ptr(base + (int64_t)kt * kStageBytes);
-      const uint32_t l0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)lds_next + wave_off);
+      const uint8_t* sb = stage_src(kt);
+      const uint32_t l0 = stage_dst(lds_next);
 #pragma unroll
-      for (int j = 0; j < PER_WAVE; ++j)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l0 + addr::direct_lds_off(0, 0, j, WAVES)),
-                     "v"(voff[j]), "s"(sb)
-                     : "memory");
+      for (int j = 0; j < PER_WAVE; ++j) load_one(j, sb, l0);
     } else {
       r.pending = true;
       const uint8_t* sb = base + (int64_t)kt * kStageBytes;
@@ -331,18 +335,22 @@ struct I8KNLoaderDirect {
   }
   uint32_t ld_;
 
+  __device__ __forceinline__ const uint8_t* stage_src(int kt) const { return uniform_ptr(base + (int64_t)kt * kStageBytes * ld_); }
+  __device__ __forceinline__ uint32_t stage_dst(uint8_t* lds) const {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + wave_off);
+  }
+  __device__ __forceinline__ void load_one(int j, const uint8_t* src, uint32_t dst) const {  // of the PER_WAVE loads of a stage
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + addr::direct_lds_off(0, 0, j, WAVES)), "v"(voff[j]), "s"(src)
+                 : "memory");
+  }
   template <bool TAIL>
   __device__ __forceinline__ void gload(Regs& r, int kt, uint8_t* lds_next) const {
-    typedef __attribute__((address_space(3))) uint8_t* lptr_t;
     if (!TAIL) {
       r.pending = false;
-      const uint8_t* sb = uniform_ptr(base + (int64_t)kt * kStageBytes * ld_);
-      const uint32_t l0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)lds_next + wave_off);
+      const uint8_t* sb = stage_src(kt);
+      const uint32_t l0 = stage_dst(lds_next);
 #pragma unroll
-      for (int j = 0; j < PER_WAVE; ++j)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l0 + addr::direct_lds_off(0, 0, j, WAVES)),
-                     "v"(voff[j]), "s"(sb)
-                     : "memory");
+      for (int j = 0; j < PER_WAVE; ++j) load_one(j, sb, l0);
     } else {
       r.pending = true;
       const uint8_t* sb = base + (int64_t)kt * kStageBytes * ld_;
@@ -407,18 +415,22 @@ struct H16KNLoaderDirect {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) voff[j] = addr::kn16_voff<BN>(lane, wave, j, WAVES, cols_total - col0, ld_);
   }
+  __device__ __forceinline__ const uint8_t* stage_src(int kt) const { return uniform_ptr(base + (int64_t)kt * 64 * ld_); }
+  __device__ __forceinline__ uint32_t stage_dst(uint8_t* lds) const {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + wave_off);
+  }
+  __device__ __forceinline__ void load_one(int j, const uint8_t* src, uint32_t dst) const {  // of the PER_WAVE loads of a stage
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + addr::direct_lds_off(0, 0, j, WAVES)), "v"(voff[j]), "s"(src)
+                 : "memory");
+  }
   template <bool TAIL>
   __device__ __forceinline__ void gload(Regs& r, int kt, uint8_t* lds_next) const {
-    typedef __attribute__((address_space(3))) uint8_t* lptr_t;
     if (!TAIL) {
       r.pending = false;
-      const uint8_t* sb = uniform_ptr(base + (int64_t)kt * 64 * ld_);
-      const uint32_t l0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)lds_next + wave_off);
+      const uint8_t* sb = stage_src(kt);
+      const uint32_t l0 = stage_dst(lds_next);
 #pragma unroll
-      for (int j = 0; j < PER_WAVE; ++j)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l0 + addr::direct_lds_off(0, 0, j, WAVES)), "v"(voff[j]),
-                     "s"(sb)
-                     : "memory");
+      for (int j = 0; j < PER_WAVE; ++j) load_one(j, sb, l0);
     } else {
       r.pending = true;
       const uint8_t* sb = base + (int64_t)kt * 64 * ld_;
@@ -775,23 +787,17 @@ __device__ __forceinline__ TileCoord tile_of_block(int tiles_m, int tiles_n, int
 }
 
 // ---- the kernel -----------------------------------------------------------------------------
-// KG > 1: the work-group is KG groups of WM x WN wavefronts, each with two LDS stages of its own, that run the same tile over
-// KG consecutive parts of K in step and meet in LDS at the end (group g writes tile rows g of KG of every wavefront
-// tile).  See group_tile for when and why.
-template <class Mma, class AL, class WL, class Epi, int BM, int BN, int WM, int WN, int KG = 1>
-__global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void gemm_mfma_kernel(
+template <class Mma, class AL, class WL, class Epi, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(WM* WN * 64, (WM * WN >= 8 ? 2 : 1)) void gemm_mfma_kernel(
     typename AL::Params pa, typename WL::Params pw, typename Epi::Params pe, int M, int N, int kt_each, int k_tail,
     int tiles_m, int tiles_n, int band_rows, int kt_total) {
   constexpr int TM = BM / WM / 16;  // 16-row activation tiles per wave
   constexpr int TN = BN / WN / 16;  // 16-row weight tiles per wave
   constexpr int A_TILE = BM * kStageBytes, W_TILE = BN * kStageBytes;
   extern __shared__ __align__(16) uint8_t smem[];
-  const int lane = threadIdx.x & 63;
-  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int group = KG == 1 ? 0 : wave_all / (WM * WN);  // of wavefronts, by part of K
-  const int wave = KG == 1 ? wave_all : wave_all - group * (WM * WN);
-  const int tid = KG == 1 ? (int)threadIdx.x : wave * 64 + lane;
-  uint8_t* const ldsA0 = smem + group * (2 * (A_TILE + W_TILE));
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint8_t* const ldsA0 = smem;
   uint8_t* const ldsW0 = ldsA0 + 2 * A_TILE;
   const int r16 = lane & 15;
   const int q = lane >> 4;
@@ -800,10 +806,7 @@ __global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void
   const TileCoord tc = tile_of_block<BM, BN>(tiles_m, tiles_n, band_rows);
   const int m0 = tc.m0, n0 = tc.n0, batch = tc.batch;
   // K slices (the "batches" of a split launch) may be uneven: the last one holds what is left of kt_total stages
-  const int kt_tile = kt_total > 0 && kt_total - batch * kt_each < kt_each ? kt_total - batch * kt_each : kt_each;
-  // this group's stages: k0 .. k0 + KT - 1 (at least one: the host launches groups on KG stages and more)
-  const int k0 = KG == 1 ? 0 : group * kt_tile / KG, KT = KG == 1 ? kt_tile : (group + 1) * kt_tile / KG - k0;
-  if (KG > 1 && group + 1 < KG) k_tail = 0;  // only the last group has the partial stage
+  const int KT = kt_total > 0 && kt_total - batch * kt_each < kt_each ? kt_total - batch * kt_each : kt_each;
 
   AL al(pa, batch, m0, M, tid);
   WL wl(pw, batch, n0, N, tid);
@@ -861,20 +864,17 @@ __global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void
 
   // prologue: stage 0 into buffer 0
   if (KT == 1 && k_tail) {
-    al.template gload<true>(ra, k0, ldsA0);
-    wl.template gload<true>(rw, k0, ldsW0);
+    al.template gload<true>(ra, 0, ldsA0);
+    wl.template gload<true>(rw, 0, ldsW0);
   } else {
-    al.template gload<false>(ra, k0, ldsA0);
-    wl.template gload<false>(rw, k0, ldsW0);
+    al.template gload<false>(ra, 0, ldsA0);
+    wl.template gload<false>(rw, 0, ldsW0);
   }
   al.lstore(ra, ldsA0);
   wl.lstore(rw, ldsW0);
   wait_direct();
   __syncthreads();
 
-  // the groups meet at the same barriers: one with a stage less than the longest has one more here
-  if constexpr (KG > 1)
-    for (int i = KT; i < (kt_tile + KG - 1) / KG; ++i) __syncthreads();
   const int last_full = k_tail ? KT - 2 : KT - 1;  // highest stage that is whole (loadable without the tail path)
   if constexpr (WL::PREFETCH2) {
     // Converting loader: the weights of stage t+1 are converted during stage t from registers that were
@@ -884,9 +884,9 @@ __global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void
     auto wload = [&](typename WL::Regs& r, int s) {
       if (s < KT) {
         if (k_tail && s == KT - 1)
-          wl.template gload<true>(r, k0 + s, ldsW0 + (s & 1) * W_TILE);
+          wl.template gload<true>(r, s, ldsW0 + (s & 1) * W_TILE);
         else
-          wl.template gload<false>(r, k0 + s, ldsW0 + (s & 1) * W_TILE);
+          wl.template gload<false>(r, s, ldsW0 + (s & 1) * W_TILE);
       }
     };
     wload(rw_next, 1);
@@ -894,9 +894,9 @@ __global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void
       rw = rw_next;
       wload(rw_next, kt + 2);
       if (k_tail && kt + 1 == KT - 1)
-        al.template gload<true>(ra, k0 + kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
+        al.template gload<true>(ra, kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
       else
-        al.template gload<false>(ra, k0 + kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
+        al.template gload<false>(ra, kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
       stage(kt & 1, std::true_type{});
       wait_direct();
       __syncthreads();
@@ -905,15 +905,15 @@ __global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void
     // Stages 0 .. KT-2 compute and fill.  Only the load of stage KT-1 can be a partial stage.
     int kt = 0;
     for (; kt + 1 <= last_full; ++kt) {
-      al.template gload<false>(ra, k0 + kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
-      wl.template gload<false>(rw, k0 + kt + 1, ldsW0 + ((kt + 1) & 1) * W_TILE);
+      al.template gload<false>(ra, kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
+      wl.template gload<false>(rw, kt + 1, ldsW0 + ((kt + 1) & 1) * W_TILE);
       stage(kt & 1, std::true_type{});
       wait_direct();
       __syncthreads();
     }
     if (kt + 1 < KT) {  // the partial last stage
-      al.template gload<true>(ra, k0 + kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
-      wl.template gload<true>(rw, k0 + kt + 1, ldsW0 + ((kt + 1) & 1) * W_TILE);
+      al.template gload<true>(ra, kt + 1, ldsA0 + ((kt + 1) & 1) * A_TILE);
+      wl.template gload<true>(rw, kt + 1, ldsW0 + ((kt + 1) & 1) * W_TILE);
       stage(kt & 1, std::true_type{});
       wait_direct();
       __syncthreads();
@@ -926,44 +926,8 @@ __global__ __launch_bounds__(WM* WN * KG * 64, (WM * WN * KG >= 8 ? 2 : 1)) void
   // the operand tiles are no longer needed once every wavefront is past its last stage: each wavefront then stages its
   // outputs through its own TM * 16 rows x 128 B of LDS
   static_assert(WM * WN * TM * 16 * kStageBytes <= 2 * (A_TILE + W_TILE), "staging area exceeds the operand tiles");
-  if constexpr (KG == 1) {
-    if constexpr (Epi::STAGED) __syncthreads();
-    write_tile<Epi, TM, TN>(epi, acc, smem + wave * (TM * 16 * kStageBytes), lane, m0 + wave_m0, n0 + wave_n0, M, N);
-  } else {
-    // Part h of every wavefront tile (tile rows h TH .. h TH + TH - 1) is group h's to write: the other groups leave theirs in
-    // LDS, [h][from][wave][TN][TH][64 lanes], and group h adds the KG of them in the order of K (its own, from its
-    // registers, among them).
-    static_assert(TM % KG == 0, "whole tile rows per group");
-    constexpr int TH = TM / KG, PART = TN * TH * 64;
-    typedef typename Mma::acc_t acc_t;
-    static_assert(KG * (KG - 1) * WM * WN * PART * (int)sizeof(acc_t) <= KG * 2 * (A_TILE + W_TILE), "partial sums exceed the operand tiles");
-    acc_t* const sums = (acc_t*)smem + lane;
-    auto part_of = [&](int h, int from) { return ((h * (KG - 1) + (from < h ? from : from - 1)) * (WM * WN) + wave) * PART; };
-    __syncthreads();
-#pragma unroll
-    for (int h = 0; h < KG; ++h)
-      if (h != group)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-          for (int t = 0; t < TH; ++t) sums[part_of(h, group) + (tn * TH + t) * 64] = acc[tn][h * TH + t];
-    __syncthreads();
-    acc_t own[TN][TH];
-#pragma unroll
-    for (int h = 0; h < KG; ++h)
-      if (h == group)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-          for (int t = 0; t < TH; ++t) {
-            acc_t sum = h == 0 ? acc[tn][h * TH + t] : sums[part_of(h, 0) + (tn * TH + t) * 64];
-#pragma unroll
-            for (int from = 1; from < KG; ++from) sum += from == h ? acc[tn][h * TH + t] : sums[part_of(h, from) + (tn * TH + t) * 64];
-            own[tn][t] = sum;
-          }
-    if constexpr (Epi::STAGED) __syncthreads();
-    write_tile<Epi, TH, TN>(epi, own, smem + wave_all * (TH * 16 * kStageBytes), lane, m0 + wave_m0 + group * (TH * 16), n0 + wave_n0, M, N);
-  }
+  if constexpr (Epi::STAGED) __syncthreads();
+  write_tile<Epi, TM, TN>(epi, acc, smem + wave * (TM * 16 * kStageBytes), lane, m0 + wave_m0, n0 + wave_n0, M, N);
 }
 
 // Host-side launcher: sets the dynamic LDS size and launches one work-group per tile.
@@ -989,79 +953,89 @@ inline bool prefer_small_tiles(int64_t batch, int64_t M, int64_t N, double weigh
   return tile_fill(batch, M, N, 128) * weight > tile_fill(batch, M, N, 256);
 }
 
-// ---- K over groups of wavefronts ----
-// A launch of 128 x 128 tiles that gives each CU one work-group at most is paced by what that work-group has in flight: one stage, 32 KB,
-// 0.7 us a trip, whatever else is idle.  With two groups of wavefronts on two parts of K the CU has two stages in flight
-// and two wavefronts on every SIMD, at the cost of one exchange of half a tile through LDS (fp16 1000 x 4096 x 4096, 256 tiles:
-// 49.5 -> 39.7 us).  Narrower tiles do the same where even those would leave CUs idle: 64 x 128, 128 x 64 (two groups), 64 x 64 (four).
-// With more tiles than CUs two work-groups of the plain kernel share a CU and need none of this.
+// ---- launches that give each CU one work-group at most: the ring kernel (gemm_ring.h) ----
+// Its tiles: 128 x 128, and narrower ones where even those would leave CUs idle.
 enum { kGroup128x128 = 2, kGroup128x64 = 3, kGroup64x128 = 4, kGroup64x64 = 5 };
 enum TileKind { kTileF16KN = 0, kTileF16NK = 1, kTileI8KN = 2, kTileI8NK = 3 };
 extern thread_local int g_gemm_groups;  // tuning: 0 = automatic, 1 = never, kGroup* = that variant wherever 128-row tiles are taken
-// Microseconds of a launch: launch + rounds x (fixed + stages x step); `lone`: the step of a plain 128 x 128 work-group that has its CU
-// to itself.  Fitted to 260 problems (M 64 .. 8000, N 256 .. 14000, K 256 .. 14336, one to eight batches), every variant forced on each:
-// 8 - 15 % rms (20 % for 64 x 64 tiles).
+// Microseconds of a launch.  Two-stage kernels: launch + rounds x (fixed + stages x step); `lone`: the step of a plain 128 x 128 work-group
+// that has its CU to itself (260 problems, M 64 .. 8000, N 256 .. 14000, K 256 .. 14336, one to eight batches: 8 - 15 % rms).
 struct TileCost {
   double launch, fixed, step, lone;
 };
-static constexpr TileCost kTileCost[4][6] = {
-    // 128 x 128          128 x 128, 2 groups    128 x 64, 2           64 x 128, 2           64 x 64, 4            256 x 256
-    {{2.4, 1.4, 1.16, 0.74}, {0.0, 2.5, 1.31, 0}, {0.8, 2.1, 0.98, 0}, {1.0, 1.7, 1.01, 0}, {1.6, 1.3, 1.24, 0}, {0.0, 5.3, 1.31, 0}},
-    {{2.4, 1.4, 1.10, 0.70}, {1.0, 4.0, 1.05, 0}, {2.1, 2.9, 0.84, 0}, {2.7, 2.2, 0.84, 0}, {3.0, 1.9, 1.06, 0}, {0.0, 5.3, 1.25, 0}},
-    {{2.0, 3.4, 1.23, 0.72}, {0.4, 5.0, 1.10, 0}, {1.2, 3.6, 0.98, 0}, {1.7, 2.8, 0.90, 0}, {2.2, 2.0, 1.36, 0}, {0.0, 7.3, 1.32, 0}},
-    {{0.3, 6.2, 1.02, 0.60}, {1.6, 4.8, 0.99, 0}, {3.4, 2.5, 0.81, 0}, {3.2, 2.8, 0.79, 0}, {3.9, 1.6, 1.05, 0}, {0.0, 8.8, 1.13, 0}}};
-inline int64_t tile_blocks(int variant, int64_t batch, int64_t M, int64_t N) {  // variant 1, kGroup*, 6
+static constexpr TileCost kTileCost[4][2] = {
+    // 128 x 128                  256 x 256
+    {{2.4, 1.4, 1.16, 0.74}, {0.0, 5.3, 1.31, 0}},
+    {{2.4, 1.4, 1.10, 0.70}, {0.0, 5.3, 1.25, 0}},
+    {{2.0, 3.4, 1.23, 0.72}, {0.0, 7.3, 1.32, 0}},
+    {{0.3, 6.2, 1.02, 0.60}, {0.0, 8.8, 1.13, 0}}};
+// Ring kernel, per round: fixed + stages x (step + shared x the part of the CUs that have a work-group): what the work-groups take from
+// each other, of memory and of the clock, grows with their number.  Fitted to 220 problems per kind (M 33 .. 3000, N 256 .. 14400, 512 ..
+// 28000 bytes of K), every variant that runs in one round forced on each: 7 - 11 % rms; the variant it picks is 2 - 2.6 % behind the best on
+// average.
+struct RingCost {
+  double fixed, step, shared;
+};
+static constexpr RingCost kRingCost[4][4] = {
+    // 128 x 128           128 x 64              64 x 128              64 x 64
+    {{5.26, 0.306, 0.276}, {4.78, 0.219, 0.173}, {4.34, 0.254, 0.164}, {4.89, 0.182, 0.093}},
+    {{5.07, 0.283, 0.262}, {4.70, 0.193, 0.158}, {4.17, 0.224, 0.160}, {4.81, 0.146, 0.097}},
+    {{5.94, 0.365, 0.276}, {5.83, 0.291, 0.211}, {5.14, 0.313, 0.167}, {5.28, 0.258, 0.116}},
+    {{6.08, 0.287, 0.261}, {6.18, 0.193, 0.171}, {5.10, 0.225, 0.164}, {5.50, 0.147, 0.107}}};
+inline int64_t tile_blocks(int variant, int64_t batch, int64_t M, int64_t N) {  // variant 1 (plain 128 x 128), kGroup*, 6 (256 x 256)
   static constexpr int kRows[6] = {128, 128, 128, 64, 64, 256}, kCols[6] = {128, 128, 64, 128, 64, 256};
   return batch * ceil_div(M, (int64_t)kRows[variant - 1]) * ceil_div(N, (int64_t)kCols[variant - 1]);
 }
 inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int64_t N, int64_t stages) {
-  static constexpr int kGroups[6] = {1, 2, 2, 2, 4, 1};
-  const int v = variant - 1;
   int cus = tlq_device_cu_count();
   if (cus <= 0) cus = 256;
-  const TileCost& c = kTileCost[kind][v];
   const int64_t blocks = tile_blocks(variant, batch, M, N);
-  const double run = c.fixed + c.step * (double)ceil_div(stages, (int64_t)kGroups[v]);
-  const int64_t rounds = blocks / (2 * cus), rest = blocks % (2 * cus);  // two plain 128 x 128 work-groups share a CU
-  const double us = variant != 1 ? run * (double)ceil_div(blocks, (int64_t)cus)
-                                 : run * (double)rounds + (rest == 0 ? 0.0 : rest > cus ? run : c.fixed + c.lone * (double)stages);
   const double memory = (double)(batch * (M + N)) * (double)(stages * kStageBytes) / 4.8e6;  // the rate of a copy, whatever the tiles
   // a large product with every CU busy runs at the rate the part sustains under that load: 2.1 POP/s int8, 1.45 PFLOP/s 16-bit
   const double k = (double)(stages * kStageBytes), product = 2.0 * (double)(batch * M) * (double)N * (kind >= kTileI8KN ? k / 2.1e9 : k / 2.9e9);
   const double floor_us = memory > product ? memory : product;
+  if (variant >= kGroup128x128 && variant <= kGroup64x64) {
+    const RingCost& c = kRingCost[kind][variant - kGroup128x128];
+    const double in_round = blocks < cus ? (double)blocks / (double)cus : 1.0;
+    const double us = (double)ceil_div(blocks, (int64_t)cus) * (c.fixed + (double)stages * (c.step + c.shared * in_round));
+    return us > floor_us ? us : floor_us;
+  }
+  const TileCost& c = kTileCost[kind][variant == 1 ? 0 : 1];
+  const double run = c.fixed + c.step * (double)stages;
+  const int64_t rounds = blocks / (2 * cus), rest = blocks % (2 * cus);  // two plain 128 x 128 work-groups share a CU
+  const double us = variant != 1 ? run * (double)ceil_div(blocks, (int64_t)cus)
+                                 : run * (double)rounds + (rest == 0 ? 0.0 : rest > cus ? run : c.fixed + c.lone * (double)stages);
   return c.launch + (us > floor_us ? us : floor_us);
 }
-// The variant for a problem that would run 128 x 128 tiles: 0 = those, or one of kGroup*, where its work-groups run in one round (they
-// have a CU each) and its estimate is clearly below.  On 4800 problems (1200 per operand layout, ranges as above, up to 1100 tiles of
-// 128 x 128) with every variant forced on each: taken on 2725, 1.26 - 1.39 x over the plain tiles on average over all, more than 5 % behind on
-// one (0.89).  Without the bound of one round 71 were, 0.64 at worst (fp16 8 x 780 x 528 x 10752 234 us in two rounds of
-// 128 x 64 tiles, 160 in plain ones): the estimates miss what two work-groups of the plain kernel on a CU give each other.
+// The variant for a problem that would run 128 x 128 tiles: 0 = those, or one of kGroup*, where its work-groups run in one round.  On 880
+// problems (220 per kind, ranges as above) the plain tiles were the fastest on 4, by 3 % at most, so that nothing is asked of the estimate but
+// which of the ring's tiles.  More than one round stays with the plain tiles: two of their work-groups share a CU, and cover each
+// other's barriers (fp16 8 x 780 x 528 x 10752 234 us in two rounds of the 128 x 64 tiles there were before, 160 in plain ones).
 inline int group_tile(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes, double* us = nullptr) {
   const int64_t stages = ceil_div(k_bytes, (int64_t)kStageBytes);
   if (g_gemm_groups > 1) return stages >= 4 ? g_gemm_groups : 0;
   int best = 0;
-  double best_us = tile_us(kind, 1, batch, M, N, stages);
-  if (g_gemm_groups == 0 && stages >= 4 && M >= 64) {  // (fewer rows were not measured)
+  double best_us = 0.0;
+  if (g_gemm_groups == 0 && stages >= 4 && M > 32) {  // (up to 32 rows: not measured)
     int cus = tlq_device_cu_count();
     if (cus <= 0) cus = 256;
-    double bar = best_us * 0.94;
     for (int v = kGroup128x128; v <= kGroup64x64; ++v) {
       if (tile_blocks(v, batch, M, N) > cus) continue;
       const double t = tile_us(kind, v, batch, M, N, stages);
-      if (t < bar) best = v, best_us = bar = t;
+      if (best == 0 || t < best_us) best = v, best_us = t;
     }
   }
-  if (us) *us = best_us;
+  if (us) *us = best != 0 ? best_us : tile_us(kind, 1, batch, M, N, stages);
   return best;
 }
-// One of the variants of run<BM, BN, WM, WN, KG>(); RUN(128, 128, 2, 2, 1) when there is none.
-#define TLQ_GROUP_TILES(variant, RUN)                       \
-  switch (variant) {                                        \
-    case kGroup128x128: RUN(128, 128, 2, 2, 2)              \
-    case kGroup128x64: RUN(128, 64, 2, 2, 2)                \
-    case kGroup64x128: RUN(64, 128, 2, 2, 2)                \
-    case kGroup64x64: RUN(64, 64, 1, 2, 4)                  \
-    default: RUN(128, 128, 2, 2, 1)                         \
+// RUN(tile rows, tile columns, ring kernel or not) for a variant of group_tile()
+#define TLQ_GROUP_TILES(variant, RUN)                \
+  switch (variant) {                                 \
+    case kGroup128x128: RUN(128, 128, true)          \
+    case kGroup128x64: RUN(128, 64, true)            \
+    case kGroup64x128: RUN(64, 128, true)            \
+    case kGroup64x64: RUN(64, 64, true)              \
+    default: RUN(128, 128, false)                    \
   }
 
 // ---- K slices of a one-batch GEMM with few activation rows ---------------------------------------------
@@ -1101,13 +1075,13 @@ inline int slice_choice(int64_t M, int64_t N, int64_t k_bytes, bool buffers, dou
   return (int)best_s;
 }
 
-template <class Mma, class AL, class WL, class Epi, int BM, int BN, int WM, int WN, int KG = 1>
+template <class Mma, class AL, class WL, class Epi, int BM, int BN, int WM, int WN>
 int launch_gemm(const typename AL::Params& pa, const typename WL::Params& pw, const typename Epi::Params& pe,
                 int64_t batch, int64_t M, int64_t N, int64_t k_bytes, hipStream_t st, const char* what, int band_rows = 4,
                 int kt_total = 0) {
   // kt_total > 0: the batches are slices of K of k_bytes each (whole stages), the last one shorter: kt_total stages in all
-  auto kern = gemm_mfma_kernel<Mma, AL, WL, Epi, BM, BN, WM, WN, KG>;
-  constexpr int lds_bytes = KG * 2 * (BM + BN) * kStageBytes;  // two stages for every group
+  auto kern = gemm_mfma_kernel<Mma, AL, WL, Epi, BM, BN, WM, WN>;
+  constexpr int lds_bytes = 2 * (BM + BN) * kStageBytes;
   static bool attr_set = false;  // per instantiation; idempotent, so a race only repeats the call
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
@@ -1126,18 +1100,14 @@ int launch_gemm(const typename AL::Params& pa, const typename WL::Params& pw, co
   }
   const int KT = (int)ceil_div(k_bytes, kStageBytes);
   const int k_tail = (k_bytes % kStageBytes) != 0;
-  if (KG > 1 && (KT < KG || kt_total > 0)) {
-    set_error("%s: %d stages of K for %d groups of wavefronts", what, KT, KG);
-    return 1;
-  }
   if (kt_total > 0 && (k_tail || (batch - 1) * KT >= kt_total || batch * KT < kt_total)) {
     set_error("%s: %lld slices of %d stages do not cover %d stages", what, (long long)batch, KT, kt_total);
     return 1;
   }
-  kern<<<(unsigned)blocks, WM * WN * KG * 64, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, KT, k_tail, (int)tiles_m,
+  kern<<<(unsigned)blocks, WM * WN * 64, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, KT, k_tail, (int)tiles_m,
                                                           (int)tiles_n, g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows, kt_total);
   char detail[96] = "";
-  if (launch_log_on()) snprintf(detail, sizeof(detail), "gemm_mfma_kernel %dx%d tiles, two stages%s%s", BM, BN, KG > 1 ? ", K in groups of wavefronts" : "", WL::DIRECT ? "" : ", weights through registers");
+  if (launch_log_on()) snprintf(detail, sizeof(detail), "gemm_mfma_kernel %dx%d tiles, two stages%s", BM, BN, WL::DIRECT ? "" : ", weights through registers");
   return check_launch(what, detail) ? 0 : 1;
 }
 

@@ -1,6 +1,7 @@
 // Plain fp16 / bf16 GEMM with fp32 accumulation: C[b, M, N] = A[b, M, K] . B[b], B[b] stored [K, N]
 // (transposed on the fly) or [N, K]; the matrices of a batch follow each other densely.
 #include "gemm_core.h"
+#include "gemm_ring.h"
 #include "gemm_slots.h"
 
 namespace tlq {
@@ -88,29 +89,36 @@ struct H16KNLoader {
 // tlq_tune_gemm_tile: 0 = automatic, 128 / 256 = that square tile
 thread_local int g_gemm_f16_tile = 0;
 
-template <class Mma, int BM, int BN, int WM, int WN, int KG = 1>
+template <class L>
+struct Loader {  // names a loader where a type has to be passed as a value
+  typedef L type;
+};
+// RING: the ring kernel (gemm_ring.h: 2 x 2 x 2 wavefronts) instead of the two-stage one
+template <class Mma, int BM, int BN, int WM, int WN, bool RING = false>
 static int run_f16(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int out_dtype,
                    int b_layout, hipStream_t st) {
-  constexpr int NT = WM * WN * 64;
+  constexpr int NT = WM * WN * 64 * (RING ? 2 : 1);
   typedef RowLoaderDirect<BM, NT> AL;
   typename AL::Params pa{(const uint8_t*)A, K * 2, M * K * 2, K * 2};
   EpiFloat::Params pe{C, N, M * N, out_dtype};
+  auto launch = [&](auto loader, const auto& pw) {
+    typedef typename decltype(loader)::type WL;
+    if constexpr (RING)
+      return launch_ring<Mma, AL, WL, EpiFloat, BM, BN>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16", 4);
+    else
+      return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
+  };
   if (b_layout == TLQ_B_NK) {
     typedef RowLoaderDirect<BN, NT> WL;
-    typename WL::Params pw{(const uint8_t*)B, K * 2, N * K * 2, K * 2};
-    return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN, KG>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
+    return launch(Loader<WL>{}, typename WL::Params{(const uint8_t*)B, K * 2, N * K * 2, K * 2});
   }
-  if (N % 8 == 0) {  // [K, N] rows are whole 16-byte chunks: copied as they are, transposed by the operand read
-    typedef H16KNLoaderDirect<BN, NT> WL;
-    H16KNParams pw{(const uint8_t*)B, N * 2, K * N * 2, K};
-    return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN, KG>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
-  }
-  if constexpr (KG == 1) {
+  if (N % 8 == 0)  // [K, N] rows are whole 16-byte chunks: copied as they are, transposed by the operand read
+    return launch(Loader<H16KNLoaderDirect<BN, NT>>{}, H16KNParams{(const uint8_t*)B, N * 2, K * N * 2, K});
+  if constexpr (!RING) {  // (the ring kernel is not asked for there)
     typedef H16KNLoader<BN, NT> WL;
-    typename WL::Params pw{(const uint8_t*)B, N * 2, K * N * 2, K};
-    return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16");
+    return launch(Loader<WL>{}, typename WL::Params{(const uint8_t*)B, N * 2, K * N * 2, K});
   }
-  return 1;  // (groups of wavefronts are not asked for there)
+  return 1;
 }
 
 // Split-K: slice z of K is "batch" z of the loaders (the batch strides step along K), and every slice
@@ -205,7 +213,7 @@ static int dispatch_f16(const void* A, const void* B, void* C, int64_t batch, in
   const bool small = g_gemm_f16_tile ? g_gemm_f16_tile == 128 : prefer_small_tiles(batch, M, N);
   if (small) {
     const int variant = b_layout == TLQ_B_NK || N % 8 == 0 ? group_tile(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, batch, M, N, K * 2) : 0;
-#define TLQ_RUN(BM, BN, WM, WN, KG) return run_f16<Mma, BM, BN, WM, WN, KG>(A, B, C, batch, M, N, K, out_dtype, b_layout, st);
+#define TLQ_RUN(BM, BN, RING) return run_f16<Mma, BM, BN, 2, 2, RING>(A, B, C, batch, M, N, K, out_dtype, b_layout, st);
     TLQ_GROUP_TILES(variant, TLQ_RUN)
 #undef TLQ_RUN
   }

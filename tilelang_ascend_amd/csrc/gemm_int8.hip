@@ -4,6 +4,7 @@
 //   * W4A8: packed int4 weights expanded to int8 on the way into LDS
 // The second operand may be stored [K, N] (transposed on the fly) or [N, K].
 #include "gemm_core.h"
+#include "gemm_ring.h"
 #include "gemm_slots.h"
 
 namespace tlq {
@@ -100,13 +101,17 @@ struct W4I8Loader {
 };
 
 // ---- launch helpers -----------------------------------------------------------------------
-template <class WL, class Epi, int BM, int BN, int WM, int WN, int KG = 1>
+// RING: the ring kernel (gemm_ring.h: 2 x 2 x 2 wavefronts) instead of the two-stage one
+template <class WL, class Epi, int BM, int BN, int WM, int WN, bool RING = false>
 static int run_i8(const void* A, const typename WL::Params& pw, const typename Epi::Params& pe, int64_t batch,
                   int64_t M, int64_t N, int64_t K, hipStream_t st, const char* what) {
-  constexpr int NT = WM * WN * 64;
+  constexpr int NT = WM * WN * 64 * (RING ? 2 : 1);
   typedef RowLoaderDirect<BM, NT> AL;  // activations travel global -> LDS without passing through registers
   typename AL::Params pa{(const uint8_t*)A, K, M * K, K};
-  return launch_gemm<MmaI8, AL, WL, Epi, BM, BN, WM, WN, KG>(pa, pw, pe, batch, M, N, K, st, what, 2);
+  if constexpr (RING)
+    return launch_ring<MmaI8, AL, WL, Epi, BM, BN>(pa, pw, pe, batch, M, N, K, st, what, 2);
+  else
+    return launch_gemm<MmaI8, AL, WL, Epi, BM, BN, WM, WN>(pa, pw, pe, batch, M, N, K, st, what, 2);
 }
 
 thread_local int g_i8_tile = 0;
@@ -131,19 +136,20 @@ static int dispatch_i8(const void* A, const void* B, const typename Epi::Params&
       typename WL::Params pw{(const uint8_t*)B, N, K * N, K};
       return launch_gemm_slots<MmaI8, WL, Epi>(pa, pw, pe, batch, M, N, K, st, what, 2);
     }
-#define TLQ_RUN(BM, BN, WM, WN, KG)                                               \
+#define TLQ_RUN(BM, BN, WM, WN, RING)                                             \
   {                                                                           \
-    typedef I8KNLoaderDirect<BN, WM * WN * 64> WL;                            \
+    typedef I8KNLoaderDirect<BN, WM * WN * 64 * (RING ? 2 : 1)> WL;           \
     typename WL::Params pw{(const uint8_t*)B, N, K * N, K};                   \
-    return run_i8<WL, Epi, BM, BN, WM, WN, KG>(A, pw, pe, batch, M, N, K, st, what); \
+    return run_i8<WL, Epi, BM, BN, WM, WN, RING>(A, pw, pe, batch, M, N, K, st, what); \
   }
     switch (tile) {
       case 32:
-        TLQ_RUN(32, 128, 1, 4, 1)
+        TLQ_RUN(32, 128, 1, 4, false)
       case 128:
-        TLQ_GROUP_TILES(group_tile(kTileI8KN, batch, M, N, K), TLQ_RUN)
+#define TLQ_TILE(BM, BN, RING) TLQ_RUN(BM, BN, 2, 2, RING)
+        TLQ_GROUP_TILES(group_tile(kTileI8KN, batch, M, N, K), TLQ_TILE)
       default:
-        TLQ_RUN(256, 256, 2, 4, 1)
+        TLQ_RUN(256, 256, 2, 4, false)
     }
 #undef TLQ_RUN
   } else {
@@ -151,19 +157,20 @@ static int dispatch_i8(const void* A, const void* B, const typename Epi::Params&
       typename RowLoaderDirect<256, 512>::Params pa{(const uint8_t*)A, K, M * K, K}, pw{(const uint8_t*)B, K, N * K, K};
       return launch_gemm_slots<MmaI8, RowLoaderDirect<256, 512>, Epi>(pa, pw, pe, batch, M, N, K, st, what, 2);
     }
-#define TLQ_RUN(BM, BN, WM, WN, KG)                                               \
+#define TLQ_RUN(BM, BN, WM, WN, RING)                                             \
   {                                                                           \
-    typedef RowLoaderDirect<BN, WM * WN * 64> WL;                             \
+    typedef RowLoaderDirect<BN, WM * WN * 64 * (RING ? 2 : 1)> WL;            \
     typename WL::Params pw{(const uint8_t*)B, K, N * K, K};                   \
-    return run_i8<WL, Epi, BM, BN, WM, WN, KG>(A, pw, pe, batch, M, N, K, st, what); \
+    return run_i8<WL, Epi, BM, BN, WM, WN, RING>(A, pw, pe, batch, M, N, K, st, what); \
   }
     switch (tile) {
       case 32:
-        TLQ_RUN(32, 128, 1, 4, 1)
+        TLQ_RUN(32, 128, 1, 4, false)
       case 128:
-        TLQ_GROUP_TILES(group_tile(kTileI8NK, batch, M, N, K), TLQ_RUN)
+        TLQ_GROUP_TILES(group_tile(kTileI8NK, batch, M, N, K), TLQ_TILE)
+#undef TLQ_TILE
       default:
-        TLQ_RUN(256, 256, 2, 4, 1)
+        TLQ_RUN(256, 256, 2, 4, false)
     }
 #undef TLQ_RUN
   }
