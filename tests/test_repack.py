@@ -77,6 +77,19 @@ def test_quantizer_matches_gen_quant4_arithmetic(dtype, N, K, group):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("chunks,group", [(1, 8), (63, 8), (64, 8), (65, 8), (127, 8), (128, 512), (129, 8), (130, 16), (511, 8), (513, 8), (1028, 32)])
+def test_quantize_chunk_counts(dtype, chunks, group):
+    """Around the 64 and 128 chunks of 8 values that a wavefront takes and the 512 of a work-group."""
+    from tilelang_ascend_amd.quantize import gpu
+
+    W = torch.randn(1, 8 * chunks, generator=torch.Generator().manual_seed(chunks)).to(dtype)
+    q, s = gpu.quantize_sym4(W.cuda(), group)
+    wq, ws = ref.quantize_sym4(W, group)
+    assert torch.equal(s.cpu(), ws) and torch.equal(q.cpu(), wq)
+
+
+@pytest.mark.gpu
 def test_quantize_pack_then_gemm_round_trip():
     """quantise -> pack on the GPU -> W4A16 GEMM with zero point 8 equals the GEMM on the dequantised weights."""
     from tilelang_ascend_amd.ops import w4a16_gemm

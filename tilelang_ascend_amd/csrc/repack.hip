@@ -40,10 +40,10 @@ __device__ __forceinline__ uint32_t interleave8(uint32_t w) {
 
 template <int MODE>
 __global__ __launch_bounds__(256) void pack_int4_kernel(const uint8_t* __restrict__ src, uint32_t* __restrict__ dst,
-                                                       int64_t n_words) {
+                                                       int64_t n_words, int blocks) {
   // a thread packs 16 values (one 16-byte load) into two words (one 8-byte store)
   const int64_t pairs = n_words >> 1;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < pairs; i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < pairs; i += (int64_t)blocks * 256) {
     const uint4_t v = ((const uint4_t*)src)[i];
     uint2_t o;
     o.x = interleave8<MODE>(pack8(v.x, v.y));
@@ -102,19 +102,30 @@ __device__ __forceinline__ int quant_one(float w, float s) {
 // correctly rounded w / s (checked for every pair of float16 values, and of bfloat16 values in the range of s below, that a group can
 // hold).  Scales so small or large that r or a product leaves the range of normal numbers take the division.  Three
 // instructions in place of the dozen and the quarter-rate reciprocal of an IEEE division, which bounded the kernel: 14336 x 4096 float16
-// 51.6 -> 37.6 us (4.7 TB/s) with the loads and the maxima below.
+// 51.6 -> 37.6 us with the loads and the maxima below.
 template <typename T>
 __device__ __forceinline__ uint2_t quant8(const float (&f)[8], float s) {
   uint32_t o[8] = {};
   if (s >= 0x1p-96f && s <= 0x1p96f) {
     const float r = 1.0f / s;
+    auto quotient = [&](int i) {
+      const float q0 = f[i] * r;
+      return __builtin_fmaf(__builtin_fmaf(-q0, s, f[i]), r, q0);
+    };
+    // rounded to T, bounded (NaN becomes the lower bound, as in quant_one), then to the nearest even whole number by the addition, which
+    // leaves its two's complement in the low byte; float16 quotients in pairs
+    if constexpr (std::is_same<T, half_t>::value) {
+      typedef float float2_t __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float q0 = f[i] * r, q = round_T<T>(__builtin_fmaf(__builtin_fmaf(-q0, s, f[i]), r, q0));
-      // bounded (NaN becomes the lower bound, as in quant_one), then to the nearest even whole number by the addition, which leaves its
-      // two's complement in the low byte
-      o[i] = bitcast<uint32_t>(__builtin_amdgcn_fmed3f(q, -8.f, 8.f) + 12582912.f);
+      for (int i = 0; i < 4; ++i) {
+        half2_t q = __builtin_convertvector((float2_t{quotient(2 * i), quotient(2 * i + 1)}), half2_t);
+        q = __builtin_elementwise_min(__builtin_elementwise_max(q, half2_t{-8, -8}), half2_t{8, 8}) + half2_t{1536, 1536};
+        o[i] = bitcast<uint32_t>(q);
+      }
+      return uint2_t{__builtin_amdgcn_perm(o[1], o[0], 0x06040200u), __builtin_amdgcn_perm(o[3], o[2], 0x06040200u)};
     }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = bitcast<uint32_t>(__builtin_amdgcn_fmed3f(round_T<T>(quotient(i)), -8.f, 8.f) + 12582912.f);
     auto bytes = [](const uint32_t* v) {
       return __builtin_amdgcn_perm(__builtin_amdgcn_perm(v[3], v[2], 0x0c0c0400u), __builtin_amdgcn_perm(v[1], v[0], 0x0c0c0400u), 0x05040100u);
     };
@@ -125,22 +136,18 @@ __device__ __forceinline__ uint2_t quant8(const float (&f)[8], float s) {
   return uint2_t{o[0], o[1]};
 }
 
-// LPG = lanes per group (group / 8), a power of two <= 64: the group maximum is a butterfly over LPG lanes.
+// lpg = lanes per group (group / 8), a power of two <= 64: the group maximum is a butterfly over lpg lanes.
 template <typename T>
 __global__ __launch_bounds__(256) void quantize_sym4_kernel(const T* __restrict__ W, int8_t* __restrict__ Q,
-                                                           T* __restrict__ S, int64_t n_chunks, int lpg) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t end = (n_chunks + 63) & ~(int64_t)63;
-  // n_chunks is a multiple of lpg and the grid stride a multiple of 64, so the lanes of a group stay together.  The next chunk is
-  // under way while this one is worked on; the weights are read once and need not stay in the caches.
+                                                           T* __restrict__ S, int64_t n_chunks, int lpg, int blocks) {
+  // A wavefront takes 128 chunks, two per lane and 64 apart, and is done: work-groups that come and go keep loads in flight better than a
+  // resident grid that asks for the next chunks ahead (14336 x 4096, 176 MB, eight work-groups a CU / 32 / one for every 512 chunks: float16 31.8 / 30.8 /
+  // 29.2 us, bfloat16 32.4 / 31.3 / 29.3; one chunk per lane 35.3 / 33.0 / 31.3 and 33.6 / 32.7 / 31.6; four per lane 30.1 and 30.9): 6.0 TB/s, where
+  // a large copy runs at 4.8.  n_chunks is a multiple of lpg, so the lanes of a group stay together.  The weights are read once and need not stay in
+  // the caches.
   typedef uint32_t v4_t __attribute__((ext_vector_type(4)));
   auto load = [&](int64_t c) { return c < n_chunks ? bitcast<uint4_t>(__builtin_nontemporal_load((const v4_t*)W + c)) : uint4_t{0u, 0u, 0u, 0u}; };
-  int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint4_t next = load(c);
-  for (; c < end; c += stride) {
-    const bool live = c < n_chunks;
-    const uint4_t v = next;
-    next = load(c + stride);
+  auto work = [&](int64_t c, const uint4_t& v) {
     float f[8];
     float amax = 0.f;
     widen8<T>(v, f);
@@ -154,20 +161,28 @@ __global__ __launch_bounds__(256) void quantize_sym4_kernel(const T* __restrict_
     if (lpg >= 16) max_dpp(std::integral_constant<int, 0x140>{});
     for (int off = 16; off < lpg; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
     const float s = round_T<T>(amax * 0.125f);
-    if (live) {
+    if (c < n_chunks) {
       if ((c & (lpg - 1)) == 0) S[c >> __builtin_ctz((unsigned)lpg)] = from_float<T>(s);
       ((uint2_t*)Q)[c] = quant8<T>(f, s);
     }
+  };
+  const int64_t stride = (int64_t)blocks * 512;
+  int64_t first = ((int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * 128;
+  const int lane = threadIdx.x & 63;
+  for (; first < n_chunks; first += stride) {
+    const uint4_t a = load(first + lane), b = load(first + 64 + lane);
+    work(first + lane, a);
+    work(first + 64 + lane, b);
   }
 }
 
 // any group size that is a multiple of 8: one wavefront per group, two passes over it
 template <typename T>
 __global__ __launch_bounds__(256) void quantize_sym4_generic_kernel(const T* __restrict__ W, int8_t* __restrict__ Q,
-                                                                   T* __restrict__ S, int64_t n_groups, int group) {
+                                                                   T* __restrict__ S, int64_t n_groups, int group, int blocks) {
   const int lane = threadIdx.x & 63;
-  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t waves = (int64_t)blocks * 4;
   const int cpg = group >> 3;
   for (int64_t g = wave; g < n_groups; g += waves) {
     const uint4_t* w = (const uint4_t*)(W + g * group);
@@ -193,15 +208,13 @@ template <typename T>
 static int run_quantize(const void* W, void* Q, void* S, int64_t N, int64_t K, int64_t group, hipStream_t st) {
   const int64_t n_chunks = N * K / 8, lpg = group / 8;
   if (lpg <= 64 && (lpg & (lpg - 1)) == 0) {
-    const int64_t want = ceil_div(n_chunks, (int64_t)256);
-    // eight work-groups to a CU hold the machine; they walk the rest
-    int cus = tlq_device_cu_count();
-    if (cus <= 0) cus = 256;
-    quantize_sym4_kernel<T><<<(int)(want > cus * 8 ? cus * 8 : want), 256, 0, st>>>((const T*)W, (int8_t*)Q, (T*)S, n_chunks, (int)lpg);
+    const int64_t want = ceil_div(n_chunks, (int64_t)512);
+    const int blocks = (int)(want > 1 << 22 ? 1 << 22 : want);  // (fewer than 2^32 threads)
+    quantize_sym4_kernel<T><<<blocks, 256, 0, st>>>((const T*)W, (int8_t*)Q, (T*)S, n_chunks, (int)lpg, blocks);
   } else {
     const int64_t n_groups = N * (K / group), want = ceil_div(n_groups, (int64_t)4);
-    quantize_sym4_generic_kernel<T><<<(int)(want > 262144 ? 262144 : want), 256, 0, st>>>((const T*)W, (int8_t*)Q, (T*)S, n_groups,
-                                                                                         (int)group);
+    const int blocks = (int)(want > 262144 ? 262144 : want);
+    quantize_sym4_generic_kernel<T><<<blocks, 256, 0, st>>>((const T*)W, (int8_t*)Q, (T*)S, n_groups, (int)group, blocks);
   }
   return check_launch("tlq_quantize_sym4") ? 0 : 1;
 }
@@ -225,11 +238,11 @@ int tlq_pack_int4(const void* values, void* packed, int64_t N, int64_t K, int in
   const int blocks = (int)(want > 262144 ? 262144 : want);
   hipStream_t st = (hipStream_t)stream;
   if (interleave == 0)
-    pack_int4_kernel<0><<<blocks, 256, 0, st>>>((const uint8_t*)values, (uint32_t*)packed, n_words);
+    pack_int4_kernel<0><<<blocks, 256, 0, st>>>((const uint8_t*)values, (uint32_t*)packed, n_words, blocks);
   else if (interleave == 1)
-    pack_int4_kernel<1><<<blocks, 256, 0, st>>>((const uint8_t*)values, (uint32_t*)packed, n_words);
+    pack_int4_kernel<1><<<blocks, 256, 0, st>>>((const uint8_t*)values, (uint32_t*)packed, n_words, blocks);
   else
-    pack_int4_kernel<2><<<blocks, 256, 0, st>>>((const uint8_t*)values, (uint32_t*)packed, n_words);
+    pack_int4_kernel<2><<<blocks, 256, 0, st>>>((const uint8_t*)values, (uint32_t*)packed, n_words, blocks);
   return check_launch("tlq_pack_int4") ? 0 : 1;
 }
 
