@@ -26,3 +26,12 @@ def test_parts_of_a_row(in_dtype, round_scale, M, N):
     y, s = y.cpu(), s.cpu()
     seen = ~torch.isnan(x)
     assert torch.equal(s, want_s.reshape(-1)) and torch.equal(y[seen], want_y[seen])
+
+
+@pytest.mark.parametrize("M,N", [(8200, 4096), (4099, 2056), (4100, 4104)])
+def test_many_rows(M, N):
+    """More rows than work-groups, and row lengths on either side of one wavefront per row."""
+    x = torch.randn(M, N, generator=torch.Generator().manual_seed(M + N)).to(torch.bfloat16)
+    y, s = ops.act_quant_kernel_int8_optimized(N)(x.cuda())
+    want_y, want_s = ref.act_quant_torch(x)
+    assert torch.equal(s.cpu(), want_s.reshape(-1)) and torch.equal(y.cpu(), want_y)

@@ -5,6 +5,8 @@
 // HBM bound: one wavefront (many rows) or one work-group (long rows) owns a row, reads it once into registers with 16-byte
 // loads, reduces the maximum across lanes, and writes 8 int8 per lane and chunk.  Few long rows are shared by work-groups, each of
 // which reads the whole row.  Rows longer than 32768 values, or of a length that is no multiple of 8, are read twice.
+#include <type_traits>
+
 #include "tlq_common.h"
 
 namespace tlq {
@@ -55,9 +57,14 @@ struct Raw8<float> {
 };
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
+  // a row of 16 lanes inside the vector unit (lanes swapped in pairs, in fours, halves of a row and rows mirrored), then rows and halves
+  // of the wavefront swapped: no trip through LDS
+  auto dpp = [&](auto ctrl) { v = fmaxf(v, bitcast<float>(__builtin_amdgcn_update_dpp(0, bitcast<int>(v), decltype(ctrl)::value, 0xf, 0xf, false))); };
+  dpp(std::integral_constant<int, 0xb1>{}), dpp(std::integral_constant<int, 0x4e>{}), dpp(std::integral_constant<int, 0x141>{}), dpp(std::integral_constant<int, 0x140>{});
+  const auto rows = __builtin_amdgcn_permlane16_swap(bitcast<uint32_t>(v), bitcast<uint32_t>(v), false, false);
+  v = fmaxf(bitcast<float>((uint32_t)rows[0]), bitcast<float>((uint32_t)rows[1]));
+  const auto halves = __builtin_amdgcn_permlane32_swap(bitcast<uint32_t>(v), bitcast<uint32_t>(v), false, false);
+  return fmaxf(bitcast<float>((uint32_t)halves[0]), bitcast<float>((uint32_t)halves[1]));
 }
 
 __device__ __forceinline__ float row_scale(float amax, int round_scale) {
@@ -77,15 +84,19 @@ __device__ __forceinline__ float row_scale(float amax, int round_scale) {
 __device__ __forceinline__ uint32_t quant1(float x, float scale, float rcp) {
   const float q0 = x * rcp;
   const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, scale, x), rcp, q0);
-  const float q = __builtin_rintf(fminf(fmaxf(q1, -127.0f), 127.0f));
-  return (uint32_t)(int)q & 0xffu;
+  // bounded (NaN becomes the lower bound), then to the nearest even whole number by the addition, which leaves its two's complement in
+  // the low byte
+  return bitcast<uint32_t>(__builtin_amdgcn_fmed3f(q1, -127.0f, 127.0f) + 12582912.0f);
 }
 
 template <typename R>
 __device__ __forceinline__ uint2_t quant8(const R& r, float scale, float rcp) {
   uint2_t o;
-  o.x = quant1(r.get(0), scale, rcp) | quant1(r.get(1), scale, rcp) << 8 | quant1(r.get(2), scale, rcp) << 16 | quant1(r.get(3), scale, rcp) << 24;
-  o.y = quant1(r.get(4), scale, rcp) | quant1(r.get(5), scale, rcp) << 8 | quant1(r.get(6), scale, rcp) << 16 | quant1(r.get(7), scale, rcp) << 24;
+  auto four = [&](int i) {
+    const uint32_t lo = __builtin_amdgcn_perm(quant1(r.get(i + 1), scale, rcp), quant1(r.get(i), scale, rcp), 0x0c0c0400u);
+    return __builtin_amdgcn_perm(__builtin_amdgcn_perm(quant1(r.get(i + 3), scale, rcp), quant1(r.get(i + 2), scale, rcp), 0x0c0c0400u), lo, 0x05040100u);
+  };
+  o.x = four(0), o.y = four(4);
   return o;
 }
 
@@ -93,7 +104,7 @@ __device__ __forceinline__ uint2_t quant8(const R& r, float scale, float rcp) {
 // 4: one row); a lane keeps CH chunks of 8 values, so the row length is at most 512 * WPR * CH.
 template <typename T, int CH, int WPR>
 __global__ __launch_bounds__(256) void act_quant_rows_kernel(const T* __restrict__ X, int8_t* __restrict__ Y,
-                                                            float* __restrict__ S, int64_t M, int N, int round_scale) {
+                                                            float* __restrict__ S, int64_t M, int N, int round_scale, int blocks) {
   __shared__ float part[2][4];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   constexpr int RPB = 4 / WPR;  // rows per work-group
@@ -101,7 +112,7 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const T* __restrict
   const int chunks = N >> 3;
   int it = 0;
   // every wavefront of a work-group runs the same number of iterations (the barrier below needs that)
-  for (int64_t m0 = (int64_t)blockIdx.x * RPB; m0 < M; m0 += (int64_t)gridDim.x * RPB, it ^= 1) {
+  for (int64_t m0 = (int64_t)blockIdx.x * RPB; m0 < M; m0 += (int64_t)blocks * RPB, it ^= 1) {
     const int64_t m = m0 + (WPR == 1 ? wv : 0);
     const bool live = m < M;
     const T* x = X + m * N;
@@ -144,12 +155,12 @@ __global__ __launch_bounds__(256) void act_quant_rows_kernel(const T* __restrict
 // 32 x 14336 bf16 4.1 -> 2.9 us, 128 x 16384 7.1 -> 3.6, 256 x 14336 7.1 -> 4.6 and, on rows of one chunk per lane, 512 x 4096 3.9 -> 3.4 (back to
 // back in a graph); from three rows per CU on it is level, from four long ones behind (1000 x 14336 11.2 against 11.6).
 template <typename T, int CH, int OC, bool WHOLE>
-__global__ __launch_bounds__(512) void act_quant_parts_kernel(const T* __restrict__ X, int8_t* __restrict__ Y, float* __restrict__ S, int N, int round_scale) {
+__global__ __launch_bounds__(512) void act_quant_parts_kernel(const T* __restrict__ X, int8_t* __restrict__ Y, float* __restrict__ S, int N, int round_scale, int parts) {
   __shared__ float part[8];
   const int tid = threadIdx.x, chunks = N >> 3;
   const int64_t m = blockIdx.x;
   const T* x = X + m * N;
-  const int parts = (int)gridDim.y, own = tid * parts + (int)blockIdx.y;  // the first of the lane's chunks
+  const int own = tid * parts + (int)blockIdx.y;  // the first of the lane's chunks
   Raw8<T> r[CH], mine[WHOLE ? 1 : OC];
 #pragma unroll
   for (int c = 0; c < CH; ++c)
@@ -188,10 +199,10 @@ __global__ __launch_bounds__(512) void act_quant_parts_kernel(const T* __restric
 template <typename T>
 __global__ __launch_bounds__(256) void act_quant_generic_kernel(const T* __restrict__ X, int8_t* __restrict__ Y,
                                                                float* __restrict__ S, int64_t M, int64_t N,
-                                                               int round_scale) {
+                                                               int round_scale, int blocks) {
   const int lane = threadIdx.x & 63;
-  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t waves = (int64_t)blocks * 4;
   for (int64_t m = wave; m < M; m += waves) {
     const T* x = X + m * N;
     float amax = 0.f;
@@ -211,12 +222,14 @@ template <typename T, int WPR>
 static void launch_rows(const T* X, int8_t* Y, float* S, int64_t M, int N, int round_scale, int per_lane,
                         hipStream_t st) {
   // a resident grid (eight work-groups per CU: every wavefront slot) that walks the rows, instead of a work-group per
-  // four rows: 37.0 instead of 40.0 us at M = 16384, N = 4096 (4 and 12 per CU are slower)
+  // four rows: 37.0 instead of 40.0 us at M = 16384, N = 4096 (4 and 12 per CU are slower).  A work-group per row of at most two chunks a
+  // lane is in and out too soon for that: up to four times as many, 4099 x 4096 bf16 11.05 -> 10.8 us, 8192 x 4096 20.0 -> 18.4.
   const int64_t want = ceil_div(M, (int64_t)(4 / WPR));
   int cus = tlq_device_cu_count();
   if (cus <= 0) cus = 256;
-  const int blocks = (int)(want > (int64_t)cus * 8 ? (int64_t)cus * 8 : want);
-#define TLQ_AQ(CH) act_quant_rows_kernel<T, CH, WPR><<<blocks, 256, 0, st>>>(X, Y, S, M, N, round_scale)
+  const int64_t most = (int64_t)cus * (WPR == 4 && per_lane <= 2 ? 32 : 8);
+  const int blocks = (int)(want > most ? most : want);
+#define TLQ_AQ(CH) act_quant_rows_kernel<T, CH, WPR><<<blocks, 256, 0, st>>>(X, Y, S, M, N, round_scale, blocks)
   if (per_lane <= 1) TLQ_AQ(1);
   else if (per_lane <= 2) TLQ_AQ(2);
   else if (per_lane <= 4) TLQ_AQ(4);
@@ -232,8 +245,9 @@ static int run_act_quant(const void* Xv, void* Yv, void* Sv, int64_t M, int64_t 
   float* S = (float*)Sv;
   const bool vec = N % 8 == 0 && ((uintptr_t)X & 15) == 0 && ((uintptr_t)Y & 7) == 0 && N <= 512 * 4 * 16;
   if (vec) {
-    // one wavefront per row while a lane then holds at most 8 chunks and there are rows enough to
-    // fill the chip that way; otherwise the four wavefronts of a work-group split the row
+    // one wavefront per row while a lane then holds at most 4 chunks and there are rows enough to fill the chip that way; otherwise the
+    // four wavefronts of a work-group split the row (bf16, one wavefront against four: 8192 x 1024 6.2 / 8.6 us, 8192 x 2048 11.7 / 11.9,
+    // 4099 x 4096 12.0 / 10.8, 8192 x 4096 18.9 / 18.4)
     int cus = tlq_device_cu_count();
     if (cus <= 0) cus = 256;
     int parts = 8;
@@ -241,7 +255,7 @@ static int run_act_quant(const void* Xv, void* Yv, void* Sv, int64_t M, int64_t 
     const int64_t chunks = N / 8;
     if (M <= (int64_t)2 * cus && N >= 4096 && chunks <= 512 * 4) {
       const dim3 grid((unsigned)M, (unsigned)parts);
-#define TLQ_AQP(CH, OC, WHOLE) act_quant_parts_kernel<T, CH, OC, WHOLE><<<grid, 512, 0, st>>>(X, Y, S, (int)N, round_scale)
+#define TLQ_AQP(CH, OC, WHOLE) act_quant_parts_kernel<T, CH, OC, WHOLE><<<grid, 512, 0, st>>>(X, Y, S, (int)N, round_scale, parts)
       if (chunks <= 512)
         parts == 1 ? TLQ_AQP(1, 1, true) : TLQ_AQP(1, 1, false);
       else if (chunks <= 1024)
@@ -252,14 +266,14 @@ static int run_act_quant(const void* Xv, void* Yv, void* Sv, int64_t M, int64_t 
       return check_launch("tlq_act_quant_i8", "act_quant kernel") ? 0 : 1;
     }
     const int per_lane1 = (int)ceil_div(N, (int64_t)512);
-    const int cap1 = sizeof(T) == 4 ? 4 : 8;
-    if (per_lane1 <= cap1 && M >= 4096)
+    if (per_lane1 <= 4 && M >= 4096)
       launch_rows<T, 1>(X, Y, S, M, (int)N, round_scale, per_lane1, st);
     else
       launch_rows<T, 4>(X, Y, S, M, (int)N, round_scale, (int)ceil_div(N, (int64_t)2048), st);
   } else {
     const int64_t want = ceil_div(M, (int64_t)4);
-    act_quant_generic_kernel<T><<<(int)(want > 65536 ? 65536 : want), 256, 0, st>>>(X, Y, S, M, N, round_scale);
+    const int blocks = (int)(want > 65536 ? 65536 : want);
+    act_quant_generic_kernel<T><<<blocks, 256, 0, st>>>(X, Y, S, M, N, round_scale, blocks);
   }
   return check_launch("tlq_act_quant_i8", "act_quant kernel") ? 0 : 1;
 }
