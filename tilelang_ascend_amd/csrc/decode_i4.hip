@@ -11,8 +11,8 @@ template <bool SIGNED, bool SCALE, int ZMODE>
 __global__ __launch_bounds__(256) void decode_i4_f16_kernel(const uint32_t* __restrict__ words,
                                                             const half_t* __restrict__ scales,
                                                             const void* __restrict__ zeros, uint4_t* __restrict__ out,
-                                                            int64_t n_words, int words_per_group) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_words; i += (int64_t)gridDim.x * blockDim.x) {
+                                                            int64_t n_words, int words_per_group, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_words; i += (int64_t)blocks * 256) {
     uint32_t w = words[i];
     const int64_t g = i / words_per_group;
     uint4_t r;
@@ -45,8 +45,8 @@ __global__ __launch_bounds__(256) void decode_i4_f16_offset_kernel(const uint32_
                                                                    const half_t* __restrict__ scales,
                                                                    const void* __restrict__ zeros, uint4_t* __restrict__ out,
                                                                    int64_t n_words, int words_per_group, int offset,
-                                                                   int zero_offset, int group_offset) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_words; i += (int64_t)gridDim.x * blockDim.x) {
+                                                                   int zero_offset, int group_offset, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_words; i += (int64_t)blocks * 256) {
     uint32_t w = words[i];
     const int64_t g = i / words_per_group;
     uint4_t r;
@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256) void decode_i4_f16_offset_kernel(const uint32_
 
 template <bool SIGNED>
 __global__ __launch_bounds__(256) void decode_i4_i8_kernel(const uint2_t* __restrict__ words, uint4_t* __restrict__ out,
-                                                           int64_t n_pairs) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_pairs; i += (int64_t)gridDim.x * blockDim.x) {
+                                                           int64_t n_pairs, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_pairs; i += (int64_t)blocks * 256) {
     uint2_t w = words[i];
     uint4_t r;
     if (SIGNED)
@@ -112,27 +112,27 @@ extern "C" int tlq_decode_i4_interleaved(const void* words, const void* scales, 
   if (out_dtype == TLQ_I8) {
     const int64_t pairs = n_words / 2;
     if (is_signed)
-      decode_i4_i8_kernel<true><<<grid_for(pairs), 256, 0, st>>>((const uint2_t*)words, o, pairs);
+      decode_i4_i8_kernel<true><<<grid_for(pairs), 256, 0, st>>>((const uint2_t*)words, o, pairs, grid_for(pairs));
     else
-      decode_i4_i8_kernel<false><<<grid_for(pairs), 256, 0, st>>>((const uint2_t*)words, o, pairs);
+      decode_i4_i8_kernel<false><<<grid_for(pairs), 256, 0, st>>>((const uint2_t*)words, o, pairs, grid_for(pairs));
     return check_launch("tlq_decode_i4_interleaved") ? 0 : 1;
   }
   const int g = grid_for(n_words);
   switch (zeros_mode) {
-    case ZEROS_ORIGINAL: decode_i4_f16_kernel<false, true, ZEROS_ORIGINAL><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg); break;
-    case ZEROS_RESCALE: decode_i4_f16_kernel<false, true, ZEROS_RESCALE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg); break;
-    case ZEROS_QUANTIZED: decode_i4_f16_kernel<false, true, ZEROS_QUANTIZED><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg); break;
+    case ZEROS_ORIGINAL: decode_i4_f16_kernel<false, true, ZEROS_ORIGINAL><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, g); break;
+    case ZEROS_RESCALE: decode_i4_f16_kernel<false, true, ZEROS_RESCALE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, g); break;
+    case ZEROS_QUANTIZED: decode_i4_f16_kernel<false, true, ZEROS_QUANTIZED><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, g); break;
     default:
       if (scales) {
         if (is_signed)
-          decode_i4_f16_kernel<true, true, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg);
+          decode_i4_f16_kernel<true, true, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, g);
         else
-          decode_i4_f16_kernel<false, true, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg);
+          decode_i4_f16_kernel<false, true, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, g);
       } else {
         if (is_signed)
-          decode_i4_f16_kernel<true, false, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg);
+          decode_i4_f16_kernel<true, false, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, g);
         else
-          decode_i4_f16_kernel<false, false, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg);
+          decode_i4_f16_kernel<false, false, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, g);
       }
   }
   return check_launch("tlq_decode_i4_interleaved") ? 0 : 1;
@@ -172,19 +172,19 @@ extern "C" int tlq_decode_i4_interleaved_offset(const void* words, const void* s
   const int g = grid_for(n_words), wpg = (int)words_per_group;
   switch (zeros_mode) {
     case ZEROS_ORIGINAL:
-      decode_i4_f16_offset_kernel<false, ZEROS_ORIGINAL><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset);
+      decode_i4_f16_offset_kernel<false, ZEROS_ORIGINAL><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset, g);
       break;
     case ZEROS_RESCALE:
-      decode_i4_f16_offset_kernel<false, ZEROS_RESCALE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset);
+      decode_i4_f16_offset_kernel<false, ZEROS_RESCALE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset, g);
       break;
     case ZEROS_QUANTIZED:
-      decode_i4_f16_offset_kernel<false, ZEROS_QUANTIZED><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset);
+      decode_i4_f16_offset_kernel<false, ZEROS_QUANTIZED><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset, g);
       break;
     default:
       if (is_signed)
-        decode_i4_f16_offset_kernel<true, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset);
+        decode_i4_f16_offset_kernel<true, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset, g);
       else
-        decode_i4_f16_offset_kernel<false, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset);
+        decode_i4_f16_offset_kernel<false, ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n_words, wpg, offset, zero_offset, group_offset, g);
   }
   return check_launch(me) ? 0 : 1;
 }

@@ -11,8 +11,8 @@ enum { LB_ZEROS_NONE = 0, LB_ZEROS_ORIGINAL = 1, LB_ZEROS_RESCALE = 2, LB_ZEROS_
 template <int BITS, bool SIGNED, bool SCALE, int ZMODE>
 __global__ __launch_bounds__(256) void decode_lowbit_f16_kernel(const uint8_t* __restrict__ src, const half_t* __restrict__ scales,
                                                                 const void* __restrict__ zeros, uint4_t* __restrict__ out,
-                                                                int64_t n_units, int units_per_group) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_units; i += (int64_t)gridDim.x * blockDim.x) {
+                                                                int64_t n_units, int units_per_group, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_units; i += (int64_t)blocks * 256) {
     const int64_t g = i / units_per_group;
     uint4_t r;
     if constexpr (BITS == 2) {
@@ -43,8 +43,8 @@ __global__ __launch_bounds__(256) void decode_lowbit_f16_kernel(const uint8_t* _
 }
 
 template <int BITS, bool SIGNED>
-__global__ __launch_bounds__(256) void decode_lowbit_i8_kernel(const uint8_t* __restrict__ src, uint4_t* __restrict__ out, int64_t n_units) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_units; i += (int64_t)gridDim.x * blockDim.x) {
+__global__ __launch_bounds__(256) void decode_lowbit_i8_kernel(const uint8_t* __restrict__ src, uint4_t* __restrict__ out, int64_t n_units, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_units; i += (int64_t)blocks * 256) {
     uint4_t r;
     if constexpr (BITS == 2) {
       uint32_t w = ((const uint32_t*)src)[i];
@@ -58,8 +58,8 @@ __global__ __launch_bounds__(256) void decode_lowbit_i8_kernel(const uint8_t* __
 }
 
 template <bool SIGNED>
-__global__ __launch_bounds__(256) void decode_i2_i4_kernel(const uint32_t* __restrict__ src, uint2_t* __restrict__ out, int64_t n_units) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_units; i += (int64_t)gridDim.x * blockDim.x) {
+__global__ __launch_bounds__(256) void decode_i2_i4_kernel(const uint32_t* __restrict__ src, uint2_t* __restrict__ out, int64_t n_units, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_units; i += (int64_t)blocks * 256) {
     uint32_t w = src[i];
     uint2_t r;
     if (SIGNED) tlq_decode::decode_i2s_to_i4s(&w, &r); else tlq_decode::decode_i2u_to_i4s(&w, &r);
@@ -73,16 +73,16 @@ template <int BITS>
 static void launch_f16(const uint8_t* w, const half_t* s, const void* zeros, uint4_t* o, int64_t n, int upg, bool is_signed, int zmode,
                        hipStream_t st) {
   const int g = lb_grid_for(n);
-  if (zmode == LB_ZEROS_ORIGINAL) { decode_lowbit_f16_kernel<BITS, false, true, LB_ZEROS_ORIGINAL><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg); return; }
-  if (zmode == LB_ZEROS_RESCALE) { decode_lowbit_f16_kernel<BITS, false, true, LB_ZEROS_RESCALE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg); return; }
+  if (zmode == LB_ZEROS_ORIGINAL) { decode_lowbit_f16_kernel<BITS, false, true, LB_ZEROS_ORIGINAL><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg, g); return; }
+  if (zmode == LB_ZEROS_RESCALE) { decode_lowbit_f16_kernel<BITS, false, true, LB_ZEROS_RESCALE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg, g); return; }
   if constexpr (BITS == 2)
-    if (zmode == LB_ZEROS_QUANTIZED) { decode_lowbit_f16_kernel<2, false, true, LB_ZEROS_QUANTIZED><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg); return; }
+    if (zmode == LB_ZEROS_QUANTIZED) { decode_lowbit_f16_kernel<2, false, true, LB_ZEROS_QUANTIZED><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg, g); return; }
   if (s) {
-    if (is_signed) decode_lowbit_f16_kernel<BITS, true, true, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg);
-    else decode_lowbit_f16_kernel<BITS, false, true, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg);
+    if (is_signed) decode_lowbit_f16_kernel<BITS, true, true, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg, g);
+    else decode_lowbit_f16_kernel<BITS, false, true, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg, g);
   } else {
-    if (is_signed) decode_lowbit_f16_kernel<BITS, true, false, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg);
-    else decode_lowbit_f16_kernel<BITS, false, false, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg);
+    if (is_signed) decode_lowbit_f16_kernel<BITS, true, false, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg, g);
+    else decode_lowbit_f16_kernel<BITS, false, false, LB_ZEROS_NONE><<<g, 256, 0, st>>>(w, s, zeros, o, n, upg, g);
   }
 }
 
@@ -120,16 +120,16 @@ extern "C" int tlq_decode_lowbit_interleaved(const void* src, const void* scales
   } else if (out_bits == 8) {
     const int g = lb_grid_for(n_units);
     if (source_bit == 2) {
-      if (is_signed) decode_lowbit_i8_kernel<2, true><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units);
-      else decode_lowbit_i8_kernel<2, false><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units);
+      if (is_signed) decode_lowbit_i8_kernel<2, true><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units, g);
+      else decode_lowbit_i8_kernel<2, false><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units, g);
     } else {
-      if (is_signed) decode_lowbit_i8_kernel<1, true><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units);
-      else decode_lowbit_i8_kernel<1, false><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units);
+      if (is_signed) decode_lowbit_i8_kernel<1, true><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units, g);
+      else decode_lowbit_i8_kernel<1, false><<<g, 256, 0, st>>>((const uint8_t*)src, (uint4_t*)out, n_units, g);
     }
   } else {
     const int g = lb_grid_for(n_units);
-    if (is_signed) decode_i2_i4_kernel<true><<<g, 256, 0, st>>>((const uint32_t*)src, (uint2_t*)out, n_units);
-    else decode_i2_i4_kernel<false><<<g, 256, 0, st>>>((const uint32_t*)src, (uint2_t*)out, n_units);
+    if (is_signed) decode_i2_i4_kernel<true><<<g, 256, 0, st>>>((const uint32_t*)src, (uint2_t*)out, n_units, g);
+    else decode_i2_i4_kernel<false><<<g, 256, 0, st>>>((const uint32_t*)src, (uint2_t*)out, n_units, g);
   }
   return check_launch(me) ? 0 : 1;
 }

@@ -465,7 +465,8 @@ __host__ __device__ inline int ring_younger_rows(int i, int my_rows, int depth) 
 // Wavefront w of W owns the steps small_first(w) .. small_first(w + 1) - 1 of a tile and runs them through a ring of D slots of
 // its own: the first D steps are issued ahead, step i + D once the contents of step i are in registers.  At the top of step i the
 // loads of the steps behind it, small_younger of them, may be outstanding.
-__host__ __device__ inline int small_first(int wave, int waves, int steps) { return (int)(((int64_t)wave * steps) / waves); }
+// (steps < 2^25: a matrix spans less than 4 GiB)
+__host__ __device__ inline int small_first(int wave, int waves, int steps) { return (int)((uint32_t)wave * (uint32_t)steps / (uint32_t)waves); }
 __host__ __device__ inline int small_younger(int i, int n, int D) { return n - 1 - i < D - 1 ? n - 1 - i : D - 1; }
 // gemm_small.h, steps of 128 bytes of K: 2 KB per 16 activation rows, then the weights (kind: SmallW)
 __host__ __device__ constexpr int small_w_tile(int kind, int rt) { return kind == 0 ? rt * 2048 : (kind == 3 ? rt * 1024 : 8192); }

@@ -114,22 +114,23 @@ void w4a16_choice_for_shape(int64_t M, int64_t N, int64_t K, void (*fn)(int algo
 // the row's value is written out once per power-of-two group (the largest power of two that divides K, 1024 at most) into
 // the tail of the workspace and the call runs with that group size -- the same arithmetic per weight, hence the same bits.
 __global__ __launch_bounds__(256) void expand_row_values_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int64_t n_out,
-                                                                int groups) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_out; i += (int64_t)gridDim.x * blockDim.x) out[i] = in[i / groups];
+                                                                int groups, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_out; i += (int64_t)blocks * 256) out[i] = in[i / groups];
 }
 // A matrix of `cols` columns (rows packed) into the first `cols` columns of a matrix whose rows lie `ldc` elements apart.
 template <typename E>
-__global__ __launch_bounds__(256) void copy_into_wider_rows_kernel(const E* __restrict__ in, E* __restrict__ out, int64_t M, int64_t cols, int64_t ldc) {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void copy_into_wider_rows_kernel(const E* __restrict__ in, E* __restrict__ out, int64_t M, int64_t cols, int64_t ldc,
+                                                                    int row_blocks) {
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (c >= cols) return;
-  for (int64_t m = blockIdx.y; m < M; m += gridDim.y) out[m * ldc + c] = in[m * cols + c];
+  for (int64_t m = blockIdx.y; m < M; m += row_blocks) out[m * ldc + c] = in[m * cols + c];
 }
 // The same for 16-bit elements, two at a time: pairs that are aligned in the OUTPUT (a row starts at element m * ldc, whose
 // parity moves the pairs by one column), one 4-byte store each; the first or last column of a row alone where a pair straddles it.
 __global__ __launch_bounds__(256) void copy_pairs_into_wider_rows_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int64_t M,
-                                                                        int64_t cols, int64_t ldc) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (int64_t m = blockIdx.y; m < M; m += gridDim.y) {
+                                                                        int64_t cols, int64_t ldc, int row_blocks) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  for (int64_t m = blockIdx.y; m < M; m += row_blocks) {
     const int64_t o = m * ldc;
     const int64_t c0 = 2 * t - (o & 1);
     if (c0 >= cols) continue;
@@ -839,13 +840,13 @@ static int write_out_row_values(const void* scales, const void* zeros, int64_t M
   const int64_t n_out = N * groups;
   const int grid = (int)((n_out + 255) / 256 > 4096 ? 4096 : (n_out + 255) / 256);
   if (scales) {
-    expand_row_values_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint16_t*)scales, (uint16_t*)base, n_out, (int)groups);
+    expand_row_values_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint16_t*)scales, (uint16_t*)base, n_out, (int)groups, grid);
     if (!check_launch("tlq_gemm_w4a16 (one scale per row, written out per group)", "expand_row_values_kernel")) return -1;
     out.scales = base;
   }
   if (zeros) {
     uint8_t* const zb = base + (scales ? tensor_bytes : 0);
-    expand_row_values_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint16_t*)zeros, (uint16_t*)zb, n_out, (int)groups);
+    expand_row_values_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint16_t*)zeros, (uint16_t*)zb, n_out, (int)groups, grid);
     if (!check_launch("tlq_gemm_w4a16 (one zero point per row, written out per group)", "expand_row_values_kernel")) return -1;
     out.zeros = zb;
   }
@@ -878,10 +879,10 @@ static int run_ragged_rows(const void* A, const void* w_packed, const void* scal
       return rc;
     const dim3 grid((unsigned)ceil_div(head, (int64_t)256), (unsigned)(M > 4096 ? 4096 : M));
     if (out_bytes == 4)
-      copy_into_wider_rows_kernel<uint32_t><<<grid, 256, 0, (hipStream_t)stream>>>((const uint32_t*)packed, (uint32_t*)C, M, head, N);
+      copy_into_wider_rows_kernel<uint32_t><<<grid, 256, 0, (hipStream_t)stream>>>((const uint32_t*)packed, (uint32_t*)C, M, head, N, (int)grid.y);
     else
       copy_pairs_into_wider_rows_kernel<<<dim3((unsigned)ceil_div(head / 2 + 1, (int64_t)256), grid.y), 256, 0, (hipStream_t)stream>>>(
-          (const uint16_t*)packed, (uint16_t*)C, M, head, N);
+          (const uint16_t*)packed, (uint16_t*)C, M, head, N, (int)grid.y);
     if (!check_launch("tlq_gemm_w4a16 (packed result into C)", out_bytes == 4 ? "copy_into_wider_rows_kernel" : "copy_pairs_into_wider_rows_kernel")) return 1;
   }
   const int eb = 2;  // scales and zero points: 16-bit values

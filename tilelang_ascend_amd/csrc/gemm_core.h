@@ -146,9 +146,10 @@ struct RowLoader {
   static_assert(PASSES == 1 || (NT / 8) % 8 == 0, "pass stride must keep the swizzle phase");
   struct Params {
     const uint8_t* base;   // element [0, 0] of batch 0
-    int64_t ld;            // row pitch in bytes
     int64_t batch_stride;  // bytes between batches
-    int64_t k_bytes;       // bytes of K per row (multiple of 16)
+    uint32_t ld;           // row pitch in bytes
+    int k_bytes;           // bytes of K per row (multiple of 16)
+    Params(const uint8_t* base, int64_t ld, int64_t batch_stride, int64_t k_bytes) : base(base), batch_stride(batch_stride), ld((uint32_t)ld), k_bytes((int)k_bytes) {}
   };
   struct Regs {
     uint4_t v[PASSES];
@@ -161,7 +162,7 @@ struct RowLoader {
   bool active;  // this thread has a slot in the (partial) last pass
 
   __device__ __forceinline__ RowLoader(const Params& p, int batch, int row0, int rows_total, int tid)
-      : base(p.base + batch * p.batch_stride + (int64_t)row0 * p.ld), k_bytes((int)p.k_bytes) {
+      : base(p.base + batch * p.batch_stride + (int64_t)row0 * p.ld), k_bytes(p.k_bytes) {
     const int rows_valid = rows_total - row0;
     const int chunk = tid & 7;
     kb_lane = chunk * 16;
@@ -169,7 +170,7 @@ struct RowLoader {
     for (int ps = 0; ps < PASSES; ++ps) {
       int row = (ps * NT + tid) >> 3;
       row = row < rows_valid ? row : rows_valid - 1;  // clamp: loads stay in bounds, results are masked later
-      voff[ps] = (uint32_t)row * (uint32_t)p.ld + (uint32_t)kb_lane;
+      voff[ps] = (uint32_t)row * p.ld + (uint32_t)kb_lane;
     }
     loff = (uint32_t)lds_off(tid >> 3, chunk);
     active = !PARTIAL || ((PASSES - 1) * NT + tid) < SLOTS;
@@ -230,7 +231,7 @@ struct RowLoaderDirect {
   int kb_lane, k_bytes;
 
   __device__ __forceinline__ RowLoaderDirect(const Params& p, int batch, int row0, int rows_total, int tid)
-      : base(p.base + batch * p.batch_stride + (int64_t)row0 * p.ld), k_bytes((int)p.k_bytes) {
+      : base(p.base + batch * p.batch_stride + (int64_t)row0 * p.ld), k_bytes(p.k_bytes) {
     const int rows_valid = rows_total - row0;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -238,7 +239,7 @@ struct RowLoaderDirect {
     lane_off = addr::direct_lds_off(lane, 0, 0, WAVES);
     kb_lane = addr::rd_chunk(lane) * 16;  // rows of one instruction start at a multiple of 8
 #pragma unroll
-    for (int j = 0; j < PER_WAVE; ++j) voff[j] = addr::rd_voff(lane, wave, j, WAVES, rows_valid, (uint32_t)p.ld);
+    for (int j = 0; j < PER_WAVE; ++j) voff[j] = addr::rd_voff(lane, wave, j, WAVES, rows_valid, p.ld);
   }
 
   // The direct loads are written as inline assembly on purpose: while a compiler-visible direct load is
@@ -287,11 +288,12 @@ struct RowLoaderDirect {
 
 // int8 source stored [K, N] (N contiguous): rows of k are copied unchanged into a [128 k][BN] LDS
 // tile; the transposition happens in the operand read (KNFrag8).
-struct I8KNParams {
+struct KNParams {
   const uint8_t* base;  // B[0, 0] of batch 0
-  int64_t ld;           // bytes per k row (= N)
   int64_t batch_stride;
-  int64_t k_total;  // K
+  uint32_t ld;  // bytes per k row (N or 2 N)
+  int k_total;  // K
+  KNParams(const uint8_t* base, int64_t ld, int64_t batch_stride, int64_t k_total) : base(base), batch_stride(batch_stride), ld((uint32_t)ld), k_total((int)k_total) {}
 };
 
 // The tile is filled by direct global -> LDS loads: one wavefront instruction covers
@@ -310,7 +312,7 @@ struct I8KNLoaderDirect {
   static constexpr int PER_WAVE = INSTR / WAVES;
   static constexpr int UNITS = PER_WAVE;
   static_assert(INSTR % WAVES == 0 && PER_WAVE >= 1, "tile does not split into whole wavefront loads");
-  typedef I8KNParams Params;
+  typedef KNParams Params;
   struct Regs {
     uint4_t v[PER_WAVE];
     bool pending;
@@ -322,7 +324,7 @@ struct I8KNLoaderDirect {
   int wave, k_total;
 
   __device__ __forceinline__ I8KNLoaderDirect(const Params& p, int batch, int col0, int cols_total, int tid)
-      : base(p.base + batch * p.batch_stride + col0), k_total((int)p.k_total) {
+      : base(p.base + batch * p.batch_stride + col0), k_total(p.k_total) {
     const int cols_valid = cols_total - col0;
     const int lane = tid & 63;
     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -330,8 +332,8 @@ struct I8KNLoaderDirect {
     lane_off = addr::direct_lds_off(lane, 0, 0, WAVES);
     k_lane = lane / CH;
 #pragma unroll
-    for (int j = 0; j < PER_WAVE; ++j) voff[j] = addr::kn_voff<BN>(lane, wave, j, WAVES, cols_valid, (uint32_t)p.ld);
-    ld_ = (uint32_t)p.ld;
+    for (int j = 0; j < PER_WAVE; ++j) voff[j] = addr::kn_voff<BN>(lane, wave, j, WAVES, cols_valid, p.ld);
+    ld_ = p.ld;
   }
   uint32_t ld_;
 
@@ -378,12 +380,6 @@ struct I8KNLoaderDirect {
 // 16-bit source stored [K, N], N a multiple of 8 (16-byte chunks): the tile is filled by direct global -> LDS loads, one
 // wavefront instruction per 512 / BN consecutive k rows; a partial last stage (rows past K must read as zero) goes
 // through registers.  Other N go through the register loader (H16KNLoader).
-struct H16KNParams {
-  const uint8_t* base;  // B[0, 0] of batch 0
-  int64_t ld;           // bytes per k row (= 2 N)
-  int64_t batch_stride;
-  int64_t k_total;
-};
 template <int BN, int NT>
 struct H16KNLoaderDirect {
   typedef KNFrag16<BN> Frag;
@@ -396,7 +392,7 @@ struct H16KNLoaderDirect {
   static constexpr int PER_WAVE = INSTR / WAVES;
   static constexpr int UNITS = PER_WAVE;
   static_assert(INSTR % WAVES == 0 && PER_WAVE >= 1, "tile does not split into whole wavefront loads");
-  typedef H16KNParams Params;
+  typedef KNParams Params;
   struct Regs {
     uint4_t v[PER_WAVE];
     bool pending;
@@ -406,7 +402,7 @@ struct H16KNLoaderDirect {
   uint32_t wave_off, lane_off, ld_;
   int k_lane, wave, k_total;
   __device__ __forceinline__ H16KNLoaderDirect(const Params& p, int batch, int col0, int cols_total, int tid)
-      : base(p.base + batch * p.batch_stride + (int64_t)col0 * 2), ld_((uint32_t)p.ld), k_total((int)p.k_total) {
+      : base(p.base + batch * p.batch_stride + (int64_t)col0 * 2), ld_(p.ld), k_total(p.k_total) {
     const int lane = tid & 63;
     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     wave_off = addr::direct_lds_off(0, wave, 0, WAVES);
@@ -460,9 +456,9 @@ struct H16KNLoaderDirect {
 struct EpiFloat {  // fp32 accumulators -> f16 / bf16 / f32
   struct Params {
     void* C;
-    int64_t ldc;
     int64_t batch_stride;  // elements
-    int out_dtype;
+    int ldc, out_dtype;
+    __host__ __device__ Params(void* C, int64_t ldc, int64_t batch_stride, int out_dtype) : C(C), batch_stride(batch_stride), ldc((int)ldc), out_dtype(out_dtype) {}
   };
   Params p;
   int64_t boff;
@@ -550,8 +546,9 @@ struct EpiAtomicAddI32 {  // int32 accumulators added into C (split-K; integer a
 struct EpiInt32 {  // raw int32 accumulators
   struct Params {
     int32_t* C;
-    int64_t ldc;
     int64_t batch_stride;
+    int ldc;
+    Params(int32_t* C, int64_t ldc, int64_t batch_stride) : C(C), batch_stride(batch_stride), ldc((int)ldc) {}
   };
   Params p;
   int64_t boff;
@@ -576,20 +573,19 @@ struct EpiInt32 {  // raw int32 accumulators
 // multiply rounds to fp32 on its own (the file is compiled with -ffp-contract=off).
 struct EpiRescale {
   struct Params {
-    void* C;
-    int64_t ldc;
-    int64_t batch_stride;  // elements of C per batch
-    const float* scale_a;  // [batch * M] or null
-    const float* scale_b;  // [n_scale_b] or null
-    int64_t n_scale_b;     // 1 or N
-    int64_t scale_a_batch_stride;
-    int out_dtype;
+    void* C;               // [batch][rows][ldc]
+    const float* scale_a;  // [batch * rows] or null
+    const float* scale_b;  // one value or ldc of them, or null
+    int ldc, rows;
+    int16_t out_dtype, one_scale_b;
+    Params(void* C, int64_t ldc, int64_t rows, const float* scale_a, const float* scale_b, int64_t n_scale_b, int out_dtype)
+        : C(C), scale_a(scale_a), scale_b(scale_b), ldc((int)ldc), rows((int)rows), out_dtype((int16_t)out_dtype), one_scale_b(n_scale_b == 1) {}
   };
   Params p;
   int64_t boff;
   const float* sa;
   __device__ __forceinline__ EpiRescale(const Params& pp, int batch)
-      : p(pp), boff(batch * pp.batch_stride), sa(pp.scale_a ? pp.scale_a + batch * pp.scale_a_batch_stride : nullptr) {}
+      : p(pp), boff((int64_t)batch * pp.rows * pp.ldc), sa(pp.scale_a ? pp.scale_a + (int64_t)batch * pp.rows : nullptr) {}
   // m < M and n < N
   __device__ __forceinline__ float4_t scaled(int m, int n, const int4_t& acc, int N) const {
     float4_t f;
@@ -604,7 +600,7 @@ struct EpiRescale {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int nn = (n + i < N) ? n + i : N - 1;
-        f[i] = f[i] * (p.n_scale_b == 1 ? p.scale_b[0] : p.scale_b[nn]);
+        f[i] = f[i] * (p.one_scale_b ? p.scale_b[0] : p.scale_b[nn]);
       }
     }
     return f;
@@ -641,7 +637,7 @@ struct EpiRescale {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int nn = (n + i < N) ? n + i : N - 1;
-        s.b[tn][i] = p.scale_b ? (p.n_scale_b == 1 ? p.scale_b[0] : p.scale_b[nn]) : 1.0f;
+        s.b[tn][i] = p.scale_b ? (p.one_scale_b ? p.scale_b[0] : p.scale_b[nn]) : 1.0f;
       }
     }
     return s;
@@ -760,7 +756,7 @@ __device__ __forceinline__ void write_tile(const Epi& epi, Acc (&acc)[TN][TM], u
   write_tile_with<Epi, TM, TN>(epi, scales, acc, region, lane, m_base, n_base, M, N);
 }
 
-// Work-group -> tile.  Consecutive hardware ids are dealt round-robin to the 8 XCDs; give
+// Work-group -> tile (`total`: the launch's work-groups).  Consecutive hardware ids are dealt round-robin to the 8 XCDs; give
 // every XCD a contiguous range of logical tiles, and order the tiles of a matrix in bands of four
 // tile rows walked column by column, so that the 32 tiles an XCD runs at a time form a 4 x 8
 // block: they share four activation panels and eight weight panels in that XCD's L2 instead of
@@ -770,8 +766,8 @@ struct TileCoord {
   int batch, m0, n0;
 };
 template <int BM, int BN>
-__device__ __forceinline__ TileCoord tile_of_block(int tiles_m, int tiles_n, int GM) {
-  const int total = gridDim.x;
+__device__ __forceinline__ TileCoord tile_of_block(int total, int M, int N, int GM) {
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   int lid = blockIdx.x;
   if ((total & 7) == 0) lid = (lid & 7) * (total >> 3) + (lid >> 3);
   const int per_batch = tiles_m * tiles_n;
@@ -789,8 +785,9 @@ __device__ __forceinline__ TileCoord tile_of_block(int tiles_m, int tiles_n, int
 // ---- the kernel -----------------------------------------------------------------------------
 template <class Mma, class AL, class WL, class Epi, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(WM* WN * 64, (WM * WN >= 8 ? 2 : 1)) void gemm_mfma_kernel(
-    typename AL::Params pa, typename WL::Params pw, typename Epi::Params pe, int M, int N, int kt_each, int k_tail,
-    int tiles_m, int tiles_n, int band_rows, int kt_total) {
+    typename AL::Params pa, typename WL::Params pw, typename Epi::Params pe, int M, int N, int kt_each, int kt_total,
+    int blocks, int band_and_tail) {
+  const int k_tail = band_and_tail & 1;
   constexpr int TM = BM / WM / 16;  // 16-row activation tiles per wave
   constexpr int TN = BN / WN / 16;  // 16-row weight tiles per wave
   constexpr int A_TILE = BM * kStageBytes, W_TILE = BN * kStageBytes;
@@ -803,7 +800,7 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN >= 8 ? 2 : 1)) void gemm_mfma
   const int q = lane >> 4;
   const int wave_m0 = (wave % WM) * (BM / WM);
   const int wave_n0 = (wave / WM) * (BN / WN);
-  const TileCoord tc = tile_of_block<BM, BN>(tiles_m, tiles_n, band_rows);
+  const TileCoord tc = tile_of_block<BM, BN>(blocks, M, N, band_and_tail >> 1);
   const int m0 = tc.m0, n0 = tc.n0, batch = tc.batch;
   // K slices (the "batches" of a split launch) may be uneven: the last one holds what is left of kt_total stages
   const int KT = kt_total > 0 && kt_total - batch * kt_each < kt_each ? kt_total - batch * kt_each : kt_each;
@@ -1104,8 +1101,8 @@ int launch_gemm(const typename AL::Params& pa, const typename WL::Params& pw, co
     set_error("%s: %lld slices of %d stages do not cover %d stages", what, (long long)batch, KT, kt_total);
     return 1;
   }
-  kern<<<(unsigned)blocks, WM * WN * 64, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, KT, k_tail, (int)tiles_m,
-                                                          (int)tiles_n, g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows, kt_total);
+  kern<<<(unsigned)blocks, WM * WN * 64, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, KT, kt_total, (int)blocks,
+                                                          2 * (g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows) + k_tail);
   char detail[96] = "";
   if (launch_log_on()) snprintf(detail, sizeof(detail), "gemm_mfma_kernel %dx%d tiles, two stages%s", BM, BN, WL::DIRECT ? "" : ", weights through registers");
   return check_launch(what, detail) ? 0 : 1;

@@ -17,12 +17,7 @@ struct H16KNLoader {
   static constexpr int PASSES = (16 * NBLK) / NT;  // 64 k = 16 blocks of 4 rows
   static constexpr int UNITS = PASSES * 4;
   static_assert(PASSES >= 1 && (16 * NBLK) % NT == 0 && NT % NBLK == 0, "bad transposing loader shape");
-  struct Params {
-    const uint8_t* base;  // B[0, 0]
-    int64_t ld;           // bytes per k row (= 2 N)
-    int64_t batch_stride;
-    int64_t k_total;
-  };
+  typedef KNParams Params;
   struct Regs {
     uint4_t v[PASSES][4];
   };
@@ -34,7 +29,7 @@ struct H16KNLoader {
 
   // cols_total must be a multiple of 8 (checked on the host)
   __device__ __forceinline__ H16KNLoader(const Params& p, int batch, int col0, int cols_total, int tid)
-      : base(p.base + batch * p.batch_stride + (int64_t)col0 * 2), ld((uint32_t)p.ld), k_total((int)p.k_total) {
+      : base(p.base + batch * p.batch_stride + (int64_t)col0 * 2), ld(p.ld), k_total(p.k_total) {
     const int cols_valid = cols_total - col0;
     nblk = tid % NBLK;
     kblk0 = tid / NBLK;
@@ -110,10 +105,10 @@ static int run_f16(const void* A, const void* B, void* C, int64_t batch, int64_t
   };
   if (b_layout == TLQ_B_NK) {
     typedef RowLoaderDirect<BN, NT> WL;
-    return launch(Loader<WL>{}, typename WL::Params{(const uint8_t*)B, K * 2, N * K * 2, K * 2});
+    return launch(Loader<WL>{}, typename WL::Params((const uint8_t*)B, K * 2, N * K * 2, K * 2));
   }
   if (N % 8 == 0)  // [K, N] rows are whole 16-byte chunks: copied as they are, transposed by the operand read
-    return launch(Loader<H16KNLoaderDirect<BN, NT>>{}, H16KNParams{(const uint8_t*)B, N * 2, K * N * 2, K});
+    return launch(Loader<H16KNLoaderDirect<BN, NT>>{}, KNParams{(const uint8_t*)B, N * 2, K * N * 2, K});
   if constexpr (!RING) {  // (the ring kernel is not asked for there)
     typedef H16KNLoader<BN, NT> WL;
     return launch(Loader<WL>{}, typename WL::Params{(const uint8_t*)B, N * 2, K * N * 2, K});
@@ -138,7 +133,7 @@ static int run_f16_splitk(const void* A, const void* B, float* C, int64_t M, int
   }
   if (N % 8 == 0) {
     typedef H16KNLoaderDirect<BN, NT> WL;
-    H16KNParams pw{(const uint8_t*)B, N * 2, ks * N * 2, ks};
+    KNParams pw{(const uint8_t*)B, N * 2, ks * N * 2, ks};
     return launch_gemm<Mma, AL, WL, EpiAtomicAdd, BM, BN, WM, WN>(pa, pw, pe, split_k, M, N, ks * 2, st, "tlq_gemm_f16_splitk");
   }
   typedef H16KNLoader<BN, NT> WL;
@@ -187,7 +182,7 @@ static int run_f16_slices(const void* A, const void* B, float* partial, int64_t 
     return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN>(pa, pw, pe, split, M, N, ksb, st, "tlq_gemm_f16 (K slices)", 4, (int)stages);
   }
   typedef H16KNLoaderDirect<BN, NT> WL;  // N % 8 == 0
-  H16KNParams pw{(const uint8_t*)B, N * 2, (ksb / 2) * N * 2, ksb / 2};
+  KNParams pw{(const uint8_t*)B, N * 2, (ksb / 2) * N * 2, ksb / 2};
   return launch_gemm<Mma, AL, WL, EpiFloat, BM, BN, WM, WN>(pa, pw, pe, split, M, N, ksb, st, "tlq_gemm_f16 (K slices)", 4, (int)stages);
 }
 
@@ -227,7 +222,7 @@ static int dispatch_f16(const void* A, const void* B, void* C, int64_t batch, in
   }
   if (g_gemm_slots == 2 && b_layout == TLQ_B_KN && K % 64 == 0 && N % 8 == 0) {  // [K, N] weights, transposed in the operand read
     typename RowLoaderDirect<256, 512>::Params pa{(const uint8_t*)A, K * 2, M * K * 2, K * 2};
-    H16KNParams pw{(const uint8_t*)B, N * 2, K * N * 2, K};
+    KNParams pw{(const uint8_t*)B, N * 2, K * N * 2, K};
     EpiFloat::Params pe{C, N, M * N, out_dtype};
     return launch_gemm_slots<Mma, H16KNLoaderDirect<256, 512>, EpiFloat>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16", 4);
   }

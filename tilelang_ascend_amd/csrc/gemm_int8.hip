@@ -23,9 +23,10 @@ struct W4I8Loader {
   static_assert(PASSES == 1 || (NT / 4) % 8 == 0, "pass stride must keep the swizzle phase");
   struct Params {
     const uint8_t* wp;
-    int64_t row_bytes;  // K / 2
-    int sign_mode;
     int64_t batch_stride;  // bytes between the "batches" (K slices: a slice's packed bytes per row)
+    int row_bytes;         // K / 2
+    int sign_mode;
+    Params(const uint8_t* wp, int64_t row_bytes, int sign_mode, int64_t batch_stride) : wp(wp), batch_stride(batch_stride), row_bytes((int)row_bytes), sign_mode(sign_mode) {}
   };
   struct Regs {
     uint4_t v[PASSES];
@@ -37,7 +38,7 @@ struct W4I8Loader {
   bool active;
 
   __device__ __forceinline__ W4I8Loader(const Params& p, int batch, int row0, int rows_total, int tid)
-      : base(p.wp + batch * p.batch_stride + (int64_t)row0 * p.row_bytes), row_bytes((int)p.row_bytes), sign_mode(p.sign_mode) {
+      : base(p.wp + batch * p.batch_stride + (int64_t)row0 * p.row_bytes), row_bytes(p.row_bytes), sign_mode(p.sign_mode) {
     const int rows_valid = rows_total - row0;
     const int quarter = tid & 3;
     kb_lane = quarter * 16;
@@ -184,7 +185,7 @@ int gemm_i8_i32(const void* A, const void* B, void* C, int64_t batch, int64_t M,
 
 int gemm_w8a8_rescale(const void* A, const void* B, const void* scale_a, const void* scale_b, void* C, int64_t batch,
                       int64_t M, int64_t N, int64_t K, int64_t n_scale_b, int b_layout, int out_dtype, hipStream_t st) {
-  EpiRescale::Params pe{C, N, M * N, (const float*)scale_a, (const float*)scale_b, n_scale_b, M, out_dtype};
+  EpiRescale::Params pe{C, N, M, (const float*)scale_a, (const float*)scale_b, n_scale_b, out_dtype};
   return dispatch_i8<EpiRescale>(A, B, pe, batch, M, N, K, b_layout, st, "tlq_gemm_w8a8");
 }
 
@@ -193,8 +194,8 @@ int gemm_w8a8_rescale(const void* A, const void* B, const void* scale_a, const v
 // bytes one work-group can pull.  Slice z of K is "batch" z of the loaders (the batch strides step along K) and every
 // slice adds its int32 tile into the one accumulator matrix, cleared beforehand: integer adds commute, so the result
 // is the exact sum whatever the order.
-__global__ __launch_bounds__(256) void i32_clear_kernel(int4_t* __restrict__ p, int64_t n4) {
-  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) p[i] = int4_t{0, 0, 0, 0};
+__global__ __launch_bounds__(256) void i32_clear_kernel(int4_t* __restrict__ p, int64_t n4, int blocks) {
+  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)blocks * 256) p[i] = int4_t{0, 0, 0, 0};
 }
 
 // `split` slices of ceil(stages / split) whole stages each, the last one with what is left (at least one stage).
@@ -231,7 +232,8 @@ int gemm_i8_i32_splitk(const void* A, const void* B, int32_t* acc, int64_t M, in
   split = whole_slices(K / kStageBytes, split);
   const int64_t n4 = M * N / 4;  // N % 16 == 0
   const int64_t want = ceil_div(n4, (int64_t)256);
-  i32_clear_kernel<<<(int)(want > 4096 ? 4096 : want), 256, 0, st>>>((int4_t*)acc, n4);
+  const int blocks = (int)(want > 4096 ? 4096 : want);
+  i32_clear_kernel<<<blocks, 256, 0, st>>>((int4_t*)acc, n4, blocks);
   if (!check_launch("tlq_gemm_i8 (clear)")) return 1;
   if (M <= 32) return run_i8_splitk<EpiAtomicAddI32, 32, 128, 1, 4>(A, B, {acc, N}, M, N, K, split, b_layout, st);
   return run_i8_splitk<EpiAtomicAddI32, 128, 128, 2, 2>(A, B, {acc, N}, M, N, K, split, b_layout, st);
@@ -241,8 +243,8 @@ int gemm_i8_i32_splitk(const void* A, const void* B, int32_t* acc, int64_t M, in
 // the arithmetic of EpiRescale on the finished sums (four outputs per thread; N % 16 == 0).
 __global__ __launch_bounds__(256) void i32_sum_rescale_kernel(const int4_t* __restrict__ partial, int split, void* __restrict__ C,
                                                               const float* __restrict__ scale_a, const float* __restrict__ scale_b,
-                                                              int64_t n_scale_b, int64_t n4_total, int n4_row, int out_dtype) {
-  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n4_total; i += (int64_t)gridDim.x * 256) {
+                                                              int64_t n_scale_b, int64_t n4_total, int n4_row, int out_dtype, int blocks) {
+  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n4_total; i += (int64_t)blocks * 256) {
     const int64_t m = i / n4_row;
     const int n = (int)(i - m * n4_row) * 4;
     int4_t a = partial[i];
@@ -282,8 +284,9 @@ int gemm_w8a8_rescale_splitk(const void* A, const void* B, const void* scale_a, 
   if (rc) return rc;
   const int64_t n4 = M * N / 4;
   const int64_t want = ceil_div(n4, (int64_t)256);
-  i32_sum_rescale_kernel<<<(int)(want > 8192 ? 8192 : want), 256, 0, st>>>((const int4_t*)partial, (int)split, C, (const float*)scale_a,
-                                                                            (const float*)scale_b, n_scale_b, n4, (int)(N / 4), out_dtype);
+  const int blocks = (int)(want > 8192 ? 8192 : want);
+  i32_sum_rescale_kernel<<<blocks, 256, 0, st>>>((const int4_t*)partial, (int)split, C, (const float*)scale_a, (const float*)scale_b, n_scale_b, n4, (int)(N / 4),
+                                                 out_dtype, blocks);
   return check_launch("tlq_gemm_w8a8 (sum and rescale)") ? 0 : 1;
 }
 
@@ -310,8 +313,8 @@ int gemm_w4a8_i32(const void* A, const void* Wp, void* C, int64_t M, int64_t N, 
 
 // C = the sum of the slices' int32 matrices (N % 4 == 0)
 __global__ __launch_bounds__(256) void i32_sum_kernel(const int4_t* __restrict__ partial, int split, int4_t* __restrict__ C,
-                                                      int64_t n4_total) {
-  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n4_total; i += (int64_t)gridDim.x * 256) {
+                                                      int64_t n4_total, int blocks) {
+  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n4_total; i += (int64_t)blocks * 256) {
     int4_t a = partial[i];
 #pragma unroll 8
     for (int z = 1; z < split; ++z) a += partial[(int64_t)z * n4_total + i];
@@ -328,7 +331,8 @@ int gemm_w4a8_i32_splitk(const void* A, const void* Wp, void* C, int64_t M, int6
   const int64_t n4 = M * N / 4;  // N % 4 == 0
   const int64_t want = ceil_div(n4, (int64_t)256);
   if (!partial) {
-    i32_clear_kernel<<<(int)(want > 4096 ? 4096 : want), 256, 0, st>>>((int4_t*)C, n4);
+    const int blocks = (int)(want > 4096 ? 4096 : want);
+    i32_clear_kernel<<<blocks, 256, 0, st>>>((int4_t*)C, n4, blocks);
     if (!check_launch("tlq_gemm_w4a8 (clear)")) return 1;
   }
   const int64_t stages = K / kStageBytes;
@@ -348,7 +352,8 @@ int gemm_w4a8_i32_splitk(const void* A, const void* Wp, void* C, int64_t M, int6
     EpiInt32::Params pe{partial, N, M * N};
     if (M <= 32) TLQ_RUN(EpiInt32, pe, 32, 128, 1, 4) else TLQ_RUN(EpiInt32, pe, 128, 128, 2, 2)
     if (rc) return rc;
-    i32_sum_kernel<<<(int)(want > 8192 ? 8192 : want), 256, 0, st>>>((const int4_t*)partial, (int)split, (int4_t*)C, n4);
+    const int blocks = (int)(want > 8192 ? 8192 : want);
+    i32_sum_kernel<<<blocks, 256, 0, st>>>((const int4_t*)partial, (int)split, (int4_t*)C, n4, blocks);
     return check_launch("tlq_gemm_w4a8 (sum)") ? 0 : 1;
   }
   EpiAtomicAddI32::Params pe{(int32_t*)C, N};

@@ -67,10 +67,10 @@ struct RingCfg {
   static_assert(4 * TM * TN * 1024 <= LDS && 8 * (TM / 2) * 16 * kStageBytes <= LDS, "the groups' sums and the staging areas fit the ring");
 };
 
-// KT: whole stages (at least one); k_tail: a partial one follows
+// KT: whole stages (at least one); band_and_tail: 2 x the tile rows of a band, + 1 where a partial stage follows
 template <class Mma, class AL, class WL, class Epi, int BM, int BN>
 __global__ __launch_bounds__(512, 2) void ring_gemm_mfma_kernel(typename AL::Params pa, typename WL::Params pw, typename Epi::Params pe, int M, int N,
-                                                               int KT, int k_tail, int tiles_m, int tiles_n, int band_rows) {
+                                                               int KT, int blocks, int band_and_tail) {
   typedef RingCfg<BM, BN> Cfg;
   typedef typename Mma::acc_t acc_t;
   constexpr int S = Cfg::S, TM = Cfg::TM, TN = Cfg::TN;
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(512, 2) void ring_gemm_mfma_kernel(typename AL::Par
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave_all >> 2, wave = wave_all & 3;  // group: this wavefront's MFMA k-step of every stage
   const int wave_m0 = (wave & 1) * (BM / 2), wave_n0 = (wave >> 1) * (BN / 2);
-  const TileCoord tc = tile_of_block<BM, BN>(tiles_m, tiles_n, band_rows);
+  const TileCoord tc = tile_of_block<BM, BN>(blocks, M, N, band_and_tail >> 1);
   AL al(pa, tc.batch, tc.m0, M, tid);
   WL wl(pw, tc.batch, tc.n0, N, tid);
   typename AL::Regs ra;
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(512, 2) void ring_gemm_mfma_kernel(typename AL::Par
     if (s + S < KT) step(Even{}); else last_steps(Even{});
     if (s < KT) last_steps(Odd{});
   }
-  if (k_tail) {  // the partial stage, with zeros past K: through registers into slot 0 (every load has landed, every fragment is read)
+  if (band_and_tail & 1) {  // the partial stage, with zeros past K: through registers into slot 0 (every load has landed, every fragment is read)
     __syncthreads();
     al.template gload<true>(ra, KT, smem);
     wl.template gload<true>(rw, KT, smem + BM * kStageBytes);
@@ -232,8 +232,8 @@ int launch_ring(const typename AL::Params& pa, const typename WL::Params& pw, co
     set_error("%s: %lld tiles, %lld bytes of K", what, (long long)blocks, (long long)k_bytes);
     return 1;
   }
-  kern<<<(unsigned)blocks, 512, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, (int)(k_bytes / kStageBytes), k_bytes % kStageBytes != 0, (int)tiles_m,
-                                                 (int)tiles_n, g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows);
+  kern<<<(unsigned)blocks, 512, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, (int)(k_bytes / kStageBytes), (int)blocks,
+                                       2 * (g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows) + (k_bytes % kStageBytes != 0));
   char detail[96] = "";
   if (launch_log_on()) snprintf(detail, sizeof(detail), "ring_gemm_mfma_kernel %dx%d tiles, %d stages, K in groups of wavefronts", BM, BN, RingCfg<BM, BN>::S);
   return check_launch(what, detail) ? 0 : 1;

@@ -20,7 +20,7 @@ namespace tlq {
 template <class Mma, class WL, class Epi>
 __global__ __launch_bounds__(512, 2) void gemm_slots_kernel(typename RowLoaderDirect<256, 512>::Params pa,
                                                            typename WL::Params pw, typename Epi::Params pe, int M, int N,
-                                                           int KT, int tiles_m, int tiles_n, int band_rows) {
+                                                           int KT, int blocks, int band_rows) {
   constexpr int BM = 256, BN = 256, WM = 2, WN = 4, TM = 8, TN = 4, SLOTS = 5;
   constexpr int TILE = 256 * kStageBytes;  // one operand, one stage: 32 KB
   typedef RowLoaderDirect<256, 512> Loader;
@@ -29,7 +29,7 @@ __global__ __launch_bounds__(512, 2) void gemm_slots_kernel(typename RowLoaderDi
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave_m0 = (wave % WM) * (BM / WM), wave_n0 = (wave / WM) * (BN / WN);
-  const TileCoord tc = tile_of_block<BM, BN>(tiles_m, tiles_n, band_rows);
+  const TileCoord tc = tile_of_block<BM, BN>(blocks, M, N, band_rows);
   Loader al(pa, tc.batch, tc.m0, M, tid);
   WL wl(pw, tc.batch, tc.n0, N, tid);
   typename Loader::Regs regs;  // unused by full stages (the data never passes through registers)
@@ -115,8 +115,8 @@ int launch_gemm_slots(const typename RowLoaderDirect<256, 512>::Params& pa, cons
     set_error("%s: too many tiles", what);
     return 1;
   }
-  kern<<<(unsigned)blocks, 512, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, (int)(k_bytes / kStageBytes), (int)tiles_m,
-                                                 (int)tiles_n, g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows);
+  kern<<<(unsigned)blocks, 512, lds_bytes, st>>>(pa, pw, pe, (int)M, (int)N, (int)(k_bytes / kStageBytes), (int)blocks,
+                                       g_gemm_band_rows > 0 ? g_gemm_band_rows : band_rows);
   return check_launch(what, "gemm_slots_kernel 256x256 tiles, five slots") ? 0 : 1;
 }
 

@@ -38,7 +38,8 @@ struct SmallParams {
   int64_t a_batch, w_batch;  // bytes between the batches
   int a_row, w_row;          // bytes between rows ([K, N] weights: between k rows)
   int steps;                 // of 128 bytes of K
-  int sign_mode;             // packed weights
+  uint16_t sign_mode;        // packed weights
+  uint16_t waves;            // of a work-group
 };
 
 // four nibbles held one per byte (0 .. 15) -> four int8 under the sign convention; a word of eight -> k order
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(RT* MT <= 4 ? 1024 : 512) void gemm_small_kernel(Sm
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int waves = blockDim.x >> 6;
+  const int waves = p.waves;
   const int r16 = lane & 15, q = lane >> 4;
   uint8_t* const mine = smem + wave * Cfg::LDS;
   const uint32_t mine_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)mine);
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(RT* MT <= 4 ? 1024 : 512) void gemm_small_kernel(Sm
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) red[(wave * (RT * MT) + rt * MT + mt) * 64 + lane] = acc[rt][mt];
   __syncthreads();
-  for (int item = threadIdx.x; item < RT * MT * 64; item += blockDim.x) {
+  for (int item = threadIdx.x; item < RT * MT * 64; item += waves * 64) {
     acc_t sum = red[item];
     for (int w = 1; w < waves; ++w) sum += red[w * (RT * MT * 64) + item];
     const int tile = item >> 6, l = item & 63;  // lane l of a tile holds C[m = l % 16][n = 4 (l / 16) .. + 3]
@@ -255,7 +256,7 @@ constexpr int small_lds(SmallW w, int rt, int mt) {
 }
 
 template <class Mma, SmallW W, class Epi, int RT, int MT, bool TIMES16>
-int launch_one(const SmallParams& p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, int waves, const char* what, hipStream_t st) {
+int launch_one(SmallParams p, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, int waves, const char* what, hipStream_t st) {
   typedef SmallCfg<W, RT, MT> Cfg;
   static_assert(Cfg::LDS == small_lds(W, RT, MT), "the plan's LDS");
   auto kern = gemm_small_kernel<Mma, W, Epi, RT, MT, TIMES16>;
@@ -268,6 +269,7 @@ int launch_one(const SmallParams& p, const typename Epi::Params& pe, int64_t bat
     }
     attr_set = true;
   }
+  p.waves = (uint16_t)waves;
   const dim3 blocks((unsigned)ceil_div(N, (int64_t)16 * RT), (unsigned)ceil_div(M, (int64_t)16 * MT), (unsigned)batch);
   kern<<<blocks, waves * 64, (size_t)waves * Cfg::LDS, st>>>(p, pe, (int)M, (int)N);
   return check_launch(what, "gemm_small_kernel") ? 0 : 1;
@@ -287,7 +289,7 @@ int launch_tile(const SmallTile& t, const SmallParams& p, const typename Epi::Pa
 }
 
 inline SmallParams small_params(const void* A, const void* B, int64_t M, int64_t N, int64_t row_bytes, int64_t w_row, int64_t w_bytes) {
-  return SmallParams{(const uint8_t*)A, (const uint8_t*)B, M * row_bytes, w_bytes, (int)row_bytes, (int)w_row, (int)(row_bytes / 128), 0};
+  return SmallParams{(const uint8_t*)A, (const uint8_t*)B, M * row_bytes, w_bytes, (int)row_bytes, (int)w_row, (int)(row_bytes / 128), 0, 0};
 }
 
 // W4A8 with weights multiplied as 16 times their value (gemm_small_w4a8.hip)

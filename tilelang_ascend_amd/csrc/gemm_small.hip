@@ -71,7 +71,7 @@ int small_i8(const SmallTile& t, const void* A, const void* B, void* C, int64_t 
 
 int small_w8a8(const SmallTile& t, const void* A, const void* B, const void* scale_a, const void* scale_b, void* C, int64_t batch, int64_t M, int64_t N, int64_t K,
                int64_t n_scale_b, int b_layout, int out_dtype, hipStream_t st) {
-  EpiRescale::Params pe{C, N, M * N, (const float*)scale_a, (const float*)scale_b, n_scale_b, M, out_dtype};
+  EpiRescale::Params pe{C, N, M, (const float*)scale_a, (const float*)scale_b, n_scale_b, out_dtype};
   const SmallParams p = small_params(A, B, M, N, K, b_layout == TLQ_B_NK ? K : N, N * K);
   return b_layout == TLQ_B_NK ? launch_tile<MmaI8, kSmallNK, EpiRescale>(t, p, pe, batch, M, N, "tlq_gemm_w8a8", st)
                               : launch_tile<MmaI8, kSmallKN8, EpiRescale>(t, p, pe, batch, M, N, "tlq_gemm_w8a8", st);
@@ -80,7 +80,7 @@ int small_w8a8(const SmallTile& t, const void* A, const void* B, const void* sca
 int small_w4a8(const SmallTile& t, const void* A, const void* Wp, void* C, int64_t M, int64_t N, int64_t K, int sign_mode, hipStream_t st) {
   EpiInt32::Params pe{(int32_t*)C, N, M * N};
   SmallParams p = small_params(A, Wp, M, N, K, K / 2, 0);
-  p.sign_mode = sign_mode;
+  p.sign_mode = (uint16_t)sign_mode;
   if (small_w4a8_times16(sign_mode, K)) return small_w4a8_times16_launch(t, p, pe, M, N, st);
   return launch_tile<MmaI8, kSmallW4, EpiInt32>(t, p, pe, 1, M, N, "tlq_gemm_w4a8", st);
 }

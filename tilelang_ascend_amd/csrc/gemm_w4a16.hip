@@ -39,13 +39,11 @@ struct W4Loader {
     const uint8_t* wp;
     const T* scales;  // never null: the host passes a dummy readable pointer when there are no scales
     const T* zeros;
-    int64_t row_bytes;  // K / 2
-    int groups;         // K / group
-    int group_shift;    // log2(group); group is a power of two here
+    int row_bytes;    // K / 2
+    int slice_bytes;  // split-K: packed bytes of one K slice (whole groups) within a row, 0 without a split; slice z is the kernel's "batch" z
     float zero_scalar;
-    int has_scales, has_zeros;
-    int64_t slice_bytes;  // split-K: packed bytes of one K slice within a row (0 without a split) ...
-    int slice_groups;     // ... and its number of quantisation groups; slice z is the kernel's "batch" z
+    uint8_t group_shift;  // log2(group); group is a power of two here
+    uint8_t has_scales, has_zeros;
   };
   struct Regs {
     uint4_t v[PASSES];
@@ -64,19 +62,20 @@ struct W4Loader {
   NibbleMagic mg;
 
   __device__ __forceinline__ W4Loader(const Params& p, int batch, int row0, int rows_total, int tid)
-      : base(p.wp + (int64_t)row0 * p.row_bytes + batch * p.slice_bytes), group_shift(p.group_shift),
+      : base(p.wp + (int64_t)row0 * p.row_bytes + (int64_t)batch * p.slice_bytes), group_shift(p.group_shift),
         has_s(p.has_scales != 0), has_z(p.has_zeros != 0), one(from_float<T>(1.0f)), zs(from_float<T>(p.zero_scalar)),
         mg(make_nibble_magic()) {
     const int rows_valid = rows_total - row0;
-    sbase = p.scales + (has_s ? (int64_t)row0 * p.groups + batch * p.slice_groups : 0);
-    zbase = p.zeros + (has_z ? (int64_t)row0 * p.groups + batch * p.slice_groups : 0);
+    const int groups = 2 * p.row_bytes >> p.group_shift, slice_groups = 2 * p.slice_bytes >> p.group_shift;
+    sbase = p.scales + (has_s ? (int64_t)row0 * groups + batch * slice_groups : 0);
+    zbase = p.zeros + (has_z ? (int64_t)row0 * groups + batch * slice_groups : 0);
     const int half = tid & 1;
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) {
       int row = (ps * NT + tid) >> 1;
       row = row < rows_valid ? row : rows_valid - 1;  // clamp: loads stay in bounds, results are masked later
       voff[ps] = (uint32_t)row * (uint32_t)p.row_bytes + (uint32_t)(half * 16);
-      goff[ps] = (uint32_t)row * (uint32_t)p.groups + (uint32_t)((half * 32) >> group_shift);
+      goff[ps] = (uint32_t)row * (uint32_t)groups + (uint32_t)((half * 32) >> group_shift);
     }
     const int r0 = tid >> 1;
 #pragma unroll
@@ -154,14 +153,12 @@ static typename W4Loader<T, FOLD, ROWS, NT>::Params w4_params(const W4Args& a) {
   return {(const uint8_t*)a.Wp,
           a.scales ? (const T*)a.scales : dummy,
           a.zeros ? (const T*)a.zeros : dummy,
-          a.K / 2,
-          (int)(a.K / a.group),
-          shift,
+          (int)(a.K / 2),
+          a.split > 1 ? (int)(a.K / a.split / 2) : 0,
           a.zero_scalar,
-          a.scales ? 1 : 0,
-          a.zeros ? 1 : 0,
-          a.split > 1 ? a.K / a.split / 2 : 0,
-          a.split > 1 ? (int)(a.K / a.split / a.group) : 0};
+          (uint8_t)shift,
+          (uint8_t)(a.scales != nullptr),
+          (uint8_t)(a.zeros != nullptr)};
 }
 
 template <typename T, bool FOLD, int BM, int BN, int WM, int WN>
@@ -232,18 +229,17 @@ template <typename T, bool FOLD, int RT, int MT>
 __global__ __launch_bounds__(MT >= 4 ? 512 : 1024) void w4a16_skinny_kernel(const T* __restrict__ A, const uint8_t* __restrict__ Wp,
                                                             const T* __restrict__ scales, const T* __restrict__ zeros,
                                                             void* __restrict__ C, int M, int N, int K, int group,
-                                                            float zero_scalar, int out_dtype) {
+                                                            float zero_scalar, int out_dtype, int waves) {
   typedef typename MmaOf<T>::type Mma;
   extern __shared__ __align__(16) uint8_t smem[];
   float4_t* const red = (float4_t*)smem;  // [waves][RT * MT][64 lanes]
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int waves = blockDim.x >> 6;
   const int r16 = lane & 15, q = lane >> 4;
   const int n_base = blockIdx.x * (16 * RT);
   const int groups = K / group;
   const int KB = K >> 7;
-  const int kb0 = (int)(((int64_t)wave * KB) / waves), kb1 = (int)(((int64_t)(wave + 1) * KB) / waves);
+  const int kb0 = addr::small_first(wave, waves, KB), kb1 = addr::small_first(wave + 1, waves, KB);
   const bool has_s = scales != nullptr, has_z = zeros != nullptr;
   const T one = from_float<T>(1.0f), zs = from_float<T>(zero_scalar);
   const NibbleMagic mg = make_nibble_magic();
@@ -326,7 +322,7 @@ __global__ __launch_bounds__(MT >= 4 ? 512 : 1024) void w4a16_skinny_kernel(cons
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) red[(wave * (RT * MT) + rt * MT + mt) * 64 + lane] = acc[rt][mt];
   __syncthreads();
-  for (int item = threadIdx.x; item < RT * MT * 64; item += blockDim.x) {
+  for (int item = threadIdx.x; item < RT * MT * 64; item += waves * 64) {
     float4_t sum = red[item];
     for (int w = 1; w < waves; ++w) {
       const float4_t v = red[w * (RT * MT * 64) + item];
@@ -368,7 +364,7 @@ static int launch_skinny(const W4Args& a, int waves) {
   const int blocks = (int)ceil_div(a.N, 16 * RT);
   const size_t lds = (size_t)waves * RT * MT * 64 * sizeof(float4_t);
   kern<<<blocks, waves * 64, lds, a.st>>>((const T*)a.A, (const uint8_t*)a.Wp, (const T*)a.scales, (const T*)a.zeros, a.C,
-                                          (int)a.M, (int)a.N, (int)a.K, (int)a.group, a.zero_scalar, a.out_dtype);
+                                          (int)a.M, (int)a.N, (int)a.K, (int)a.group, a.zero_scalar, a.out_dtype, waves);
   return check_launch("tlq_gemm_w4a16(skinny)", "w4a16_skinny_kernel") ? 0 : 1;
 }
 
@@ -430,8 +426,8 @@ int gemm_w4a16_skinny(const void* A, const void* Wp, const void* scales, const v
 // C[i] = round(sum over the K slices of partial[z][i]), slices added in index order (so the result does not
 // depend on which work-group finished first)
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4_t* __restrict__ partial, void* __restrict__ C,
-                                                           int64_t n4, int split, int out_dtype) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
+                                                           int64_t n4, int split, int out_dtype, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)blocks * 256) {
     float4_t v = partial[i];
 #pragma unroll 8  // loads of eight slices in flight (with few outputs the pass is paced by their latency); same order of adds
     for (int z = 1; z < split; ++z) v += partial[(int64_t)z * n4 + i];
@@ -487,7 +483,8 @@ int64_t w4a16_mid_split(int64_t M, int64_t N, int64_t K, int64_t group) {
 
 void launch_splitk_reduce(const float* partial, void* C, int64_t M, int64_t N, int split, int out_dtype, hipStream_t st) {
   const int64_t n4 = M * N / 4, want = ceil_div(n4, (int64_t)256);
-  splitk_reduce_kernel<<<(int)(want > 65536 ? 65536 : want), 256, 0, st>>>((const float4_t*)partial, C, n4, split, out_dtype);
+  const int blocks = (int)(want > 65536 ? 65536 : want);
+  splitk_reduce_kernel<<<blocks, 256, 0, st>>>((const float4_t*)partial, C, n4, split, out_dtype, blocks);
 }
 
 int gemm_w4a16_mfma_splitk(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M,
@@ -504,8 +501,7 @@ int gemm_w4a16_mfma_splitk(const void* A, const void* Wp, const void* scales, co
   else
     rc = fold ? dispatch_w4a16<bf16_t, true>(a) : dispatch_w4a16<bf16_t, false>(a);
   if (rc) return rc;
-  const int64_t n4 = M * N / 4, want = ceil_div(n4, (int64_t)256);
-  splitk_reduce_kernel<<<(int)(want > 65536 ? 65536 : want), 256, 0, st>>>((const float4_t*)partial, C, n4, (int)split, out_dtype);
+  launch_splitk_reduce(partial, C, M, N, (int)split, out_dtype, st);
   return check_launch("tlq_gemm_w4a16(split-K reduce)") ? 0 : 1;
 }
 

@@ -60,8 +60,8 @@ template <typename T, int MT, int LAYOUT>
 __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict__ A, const uint8_t* __restrict__ Wp,
                                                             const T* __restrict__ scales, const T* __restrict__ zeros,
                                                             void* __restrict__ C, float* __restrict__ partial, int M, int N,
-                                                            int K, int gshift, float zero_scalar, int out_dtype, int tiles,
-                                                            int slices) {
+                                                            int K, int gshift, float zero_scalar, int out_dtype, int stride,
+                                                            int waves) {
   typedef typename DecodeMma<T>::type Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
   constexpr int TS = addr::kDecTileSlots;
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int waves = blockDim.x >> 6;
+  const int tiles = (N + 15) >> 4, slices = K / addr::kDecSlice;
   const int r16 = lane & 15, q = lane >> 4;
   uint8_t* const mine = smem + wave * WAVE;
   const uint32_t mine_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)mine);
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
   n_active = n_active < waves ? n_active : waves;
   const int64_t k0 = (int64_t)(active ? slice : 0) * addr::kDecSlice;
   const int groups = K >> gshift;
-  const int first = blockIdx.x, stride = gridDim.x;
+  const int first = blockIdx.x;  // and every stride-th tile after it
   const int my_tiles = (tiles - first + stride - 1) / stride;
   const bool has_s = scales != nullptr, has_z = zeros != nullptr;
   const T one = from_float<T>(1.0f), zs = from_float<T>(zero_scalar);
@@ -345,10 +345,9 @@ static int launch_decode(const void* A, const void* Wp, const void* scales, cons
     }
     attr_set = true;
   }
-  const int tiles = (int)((N + 15) / 16);
   kern<<<dim3(p.grid_x, p.chunks), p.waves * 64, (size_t)p.lds_bytes, st>>>(
       (const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, p.chunks > 1 ? partial : nullptr, (int)M, (int)N, (int)K,
-      gshift, zero_scalar, out_dtype, tiles, (int)(K / addr::kDecSlice));
+      gshift, zero_scalar, out_dtype, p.grid_x, p.waves);
   return check_launch("tlq_gemm_w4a16(decode)", "w4a16_decode_kernel") ? 0 : 1;
 }
 

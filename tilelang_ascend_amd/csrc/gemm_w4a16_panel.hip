@@ -88,7 +88,7 @@ __global__ __launch_bounds__(512, 1) void w4a16_panel_kernel(const T* __restrict
                                                             const T* __restrict__ scales, const T* __restrict__ zeros,
                                                             void* __restrict__ C, float* __restrict__ partial, int M, int N, int K,
                                                             int gshift, float zero_scalar, int out_dtype, int slice_steps,
-                                                            int tiles_m, int tiles_n, int band_rows, uint32_t* __restrict__ flag,
+                                                            int blocks, int band_rows, uint32_t* __restrict__ flag,
                                                             uint32_t epoch) {
   typedef PanelCfg Cfg;
   if constexpr (ZM == 3) {
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(512, 1) void w4a16_panel_kernel(const T* __restrict
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, q = lane >> 4;
-  const TileCoord tc = tile_of_block<Cfg::BM, Cfg::BN>(tiles_m, tiles_n, band_rows);  // batch = K slice
+  const TileCoord tc = tile_of_block<Cfg::BM, Cfg::BN>(blocks, M, N, band_rows);  // batch = K slice
   const int m0 = tc.m0, n0 = tc.n0, slice = tc.batch;
   const int steps_total = K >> 7;
   const int step0 = slice * slice_steps;
@@ -399,7 +399,7 @@ static int launch_panel(const void* A, const void* Wp, const void* scales, const
   }
   const unsigned blocks = (unsigned)((int64_t)p.tiles_m * p.tiles_n * p.split);
   kern<<<blocks, 512, lds_bytes, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, partial, (int)M, (int)N,
-                                       (int)K, gshift, zero_scalar, out_dtype, p.slice_steps, p.tiles_m, p.tiles_n, band_rows, flag, epoch);
+                                       (int)K, gshift, zero_scalar, out_dtype, p.slice_steps, (int)blocks, band_rows, flag, epoch);
   return check_launch("tlq_gemm_w4a16(panel)", ZM == 0 ? "w4a16_panel_kernel, zero-point tensor folded" : (ZM == 3 ? "w4a16_panel_kernel, unfolded behind the flag" : "w4a16_panel_kernel")) ? 0 : 1;
 }
 

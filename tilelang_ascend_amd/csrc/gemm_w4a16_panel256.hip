@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256, 1) void w4a16_panel256_kernel(const T* __restr
                                                                const T* __restrict__ scales, const T* __restrict__ zeros,
                                                                void* __restrict__ C, float* __restrict__ partial, int M, int N, int K,
                                                                int gshift, float zero_scalar, int out_dtype, int slice_steps,
-                                                               int tiles_m, int tiles_n, int band_rows) {
+                                                               int blocks, int band_rows) {
   typedef Panel2Cfg Cfg;
   typedef Panel2Mma<T> Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256, 1) void w4a16_panel256_kernel(const T* __restr
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, q = lane >> 4;
-  const TileCoord tc = tile_of_block<Cfg::BM, Cfg::BN>(tiles_m, tiles_n, band_rows);  // batch = K slice
+  const TileCoord tc = tile_of_block<Cfg::BM, Cfg::BN>(blocks, M, N, band_rows);  // batch = K slice
   const int m0 = tc.m0, n0 = tc.n0, slice = tc.batch;
   const int steps_total = K >> 7;
   const int step0 = slice * slice_steps;
@@ -464,7 +464,7 @@ static int launch_panel256(const void* A, const void* Wp, const void* scales, co
   }
   const unsigned blocks = (unsigned)((int64_t)p.tiles_m * p.tiles_n * p.split);
   kern<<<blocks, 256, lds_bytes, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, partial, (int)M, (int)N,
-                                       (int)K, gshift, zero_scalar, out_dtype, p.slice_steps, p.tiles_m, p.tiles_n, band_rows);
+                                       (int)K, gshift, zero_scalar, out_dtype, p.slice_steps, (int)blocks, band_rows);
   return check_launch("tlq_gemm_w4a16(panel256)", ZM == 0 ? "w4a16_panel256_kernel, zero-point tensor" : "w4a16_panel256_kernel")
              ? 0
              : 1;

@@ -42,7 +42,7 @@ template <typename T, bool FOLD, int LAYOUT, int RT, int MT>
 __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const T* __restrict__ A, const uint8_t* __restrict__ Wp,
                                                                 const T* __restrict__ scales, const T* __restrict__ zeros,
                                                                 void* __restrict__ C, int M, int N, int K, int gshift,
-                                                                float zero_scalar, int out_dtype) {
+                                                                float zero_scalar, int out_dtype, int waves) {
   typedef typename SmallMma<T>::type Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
   constexpr int SLOT = addr::smallw_slot_bytes(RT, MT);  // RT weight tiles + MT activation tiles
@@ -52,7 +52,6 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int waves = blockDim.x >> 6;
   const int r16 = lane & 15, q = lane >> 4;
   uint8_t* const mine = smem + wave * WAVE_LDS;
   const uint32_t mine_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)mine);
@@ -227,7 +226,7 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) red[(wave * (RT * MT) + rt * MT + mt) * 64 + lane] = acc[rt][mt];
   __syncthreads();
-  for (int item = threadIdx.x; item < RT * MT * 64; item += blockDim.x) {
+  for (int item = threadIdx.x; item < RT * MT * 64; item += waves * 64) {
     float4_t sum = red[item];
     for (int w = 1; w < waves; ++w) {
       const float4_t v = red[w * (RT * MT * 64) + item];
@@ -329,7 +328,7 @@ static int launch_small(const SmallArgs& a, int waves) {
   }
   const dim3 blocks((unsigned)ceil_div((int64_t)a.N, (int64_t)16 * RT), (unsigned)ceil_div((int64_t)a.M, (int64_t)16 * MT));
   kern<<<blocks, waves * 64, (size_t)waves * small_wave_lds(RT, MT), a.st>>>((const T*)a.A, (const uint8_t*)a.Wp, (const T*)a.scales, (const T*)a.zeros, a.C,
-                                                                          a.M, a.N, a.K, a.gshift, a.zero_scalar, a.out_dtype);
+                                                                          a.M, a.N, a.K, a.gshift, a.zero_scalar, a.out_dtype, waves);
   return check_launch(a.what, LAYOUT == 1 ? "w4a16_small_kernel, interleaved words" : "w4a16_small_kernel") ? 0 : 1;
 }
 

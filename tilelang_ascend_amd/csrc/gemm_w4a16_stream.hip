@@ -137,7 +137,7 @@ template <typename T, int TB, int KG, int LAYOUT, bool MANY>
 __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restrict__ A, const uint8_t* __restrict__ Wp,
                                                              const T* __restrict__ scales, const T* __restrict__ zeros,
                                                              void* __restrict__ C, float* __restrict__ partial, int M, int N, int K,
-                                                             int gshift, float zero_scalar, int out_dtype, int slice_steps, int by_xcd) {
+                                                             int gshift, float zero_scalar, int out_dtype, int slice_steps, int xcd_slices) {
   typedef StreamCfg<TB, KG> Cfg;
   typedef StreamMma<T> Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
@@ -148,7 +148,10 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
   const int r32 = lane & 31, h = lane >> 5;
   const int kg = wave / WN, wn = wave % WN;  // values 16 KT kg .. of every step; weight rows 64 wn .. 64 wn + 63
   StreamItem item{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
-  if (by_xcd) item = stream_item(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z, true);
+  if (xcd_slices) {  // the launch's K slices, where the order is by XCD
+    const int nb = (N + Cfg::BN - 1) / Cfg::BN, mb = (M + Cfg::BM - 1) / Cfg::BM;
+    item = stream_item(blockIdx.x + nb * (blockIdx.y + xcd_slices * blockIdx.z), nb, xcd_slices, mb, true);
+  }
   const int n0 = item.n * Cfg::BN, m0 = item.m * Cfg::BM, slice = item.slice;
   const int steps_total = K >> 7;
   const int step0 = slice * slice_steps;
@@ -484,7 +487,7 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
   typedef std::integral_constant<int, 0> I0;
   typedef std::integral_constant<int, 1> I1;
   typedef std::integral_constant<int, 2> I2;
-  const bool split = gridDim.y > 1;
+  const bool split = steps_total > slice_steps;
   auto store = [&](auto j0_tag) {  // the wavefront's quarters, from J0 on
     constexpr int J0 = decltype(j0_tag)::value, COUNT = 4 / KG;
     if (split) {
@@ -709,7 +712,7 @@ static int launch_stream(const void* A, const void* Wp, const void* scales, cons
     attr_set = true;
   }
   kern<<<dim3(p.n_blocks, p.split, p.m_blocks), 512, lds_bytes, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, partial, (int)M,
-                                                                     (int)N, (int)K, gshift, zero_scalar, out_dtype, p.slice_steps, p.by_xcd);
+                                                                     (int)N, (int)K, gshift, zero_scalar, out_dtype, p.slice_steps, p.by_xcd ? p.split : 0);
   char detail[80] = "";
   if (launch_log_on()) snprintf(detail, sizeof(detail), "w4a16_stream_kernel, %d activation rows per work-group%s", 32 * TB, p.by_xcd ? ", by XCD" : "");
   return check_launch("tlq_gemm_w4a16(stream)", detail) ? 0 : 1;

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256, 4) void gemv_w4a16_f16_kernel(const half_t* __
                                                                 const half_t* __restrict__ scales,
                                                                 const half_t* __restrict__ zeros,
                                                                 void* __restrict__ C, int m_count, int N, int K,
-                                                                int group_shift, float zero_scalar, int out_dtype) {
+                                                                int group_shift, float zero_scalar, int out_dtype, int blocks, int waves_per_block) {
   extern __shared__ __align__(16) uint8_t smem[];
   const int chunks = K >> 5;
   uint4_t* const lds_pairs = (uint4_t*)smem;                            // [MT][4][chunks]
@@ -251,9 +251,8 @@ __global__ __launch_bounds__(256, 4) void gemv_w4a16_f16_kernel(const half_t* __
   }
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: row pointers stay scalar
-  const int waves_per_block = blockDim.x >> 6;
   const int wave_id = blockIdx.x * waves_per_block + wave;
-  const int wave_count = gridDim.x * waves_per_block;
+  const int wave_count = blocks * waves_per_block;
   const int row_groups = (N + R - 1) / R;
   const int row_bytes = K >> 1;
   const int iters = (chunks + 63) >> 6;  // chunk iterations per row
@@ -312,7 +311,7 @@ __global__ __launch_bounds__(256, 4) void gemv_w4a16_f16_kernel(const half_t* __
 
   for (int m0 = 0; m0 < m_count; m0 += MT) {
     if (m0 > 0) __syncthreads();  // previous pass has finished reading LDS
-    for (int i = threadIdx.x; i < chunks * MT; i += blockDim.x) {
+    for (int i = threadIdx.x; i < chunks * MT; i += waves_per_block * 64) {
       const int m = (MT == 1) ? 0 : i / chunks;
       const int c = i - m * chunks;
       const int mm = (m0 + m < m_count) ? m0 + m : m_count - 1;
@@ -614,14 +613,13 @@ __global__ __launch_bounds__(1024) void gemv_w4a16_ring_kernel(const T* __restri
                                                                              const T* __restrict__ scales,
                                                                              const T* __restrict__ zeros, void* __restrict__ C,
                                                                              int N, int K, int group_shift, float zero_scalar,
-                                                                             int out_dtype, int rows_per_block) {
+                                                                             int out_dtype, int rows_per_block, int nwaves) {
   constexpr bool F16 = __is_same(T, half_t);
   static_assert(MT == 1 || (F16 && MT == 2), "two activation rows: fp16 only");
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nwaves = blockDim.x >> 6;
   const int chunks = K >> 5, row_bytes = K >> 1, groups = K >> group_shift;
   const int r0 = blockIdx.x * rows_per_block;
   const int r1 = r0 + rows_per_block < N ? r0 + rows_per_block : N;
@@ -798,9 +796,9 @@ template <typename T, int R, int MT>
 __global__ __launch_bounds__(256) void gemv_w4a16_kernel(const T* __restrict__ A, const uint8_t* __restrict__ Wp,
                                                          const T* __restrict__ scales, const T* __restrict__ zeros,
                                                          void* __restrict__ C, int m_count, int N, int K, int group,
-                                                         float zero_scalar, int out_dtype) {
+                                                         float zero_scalar, int out_dtype, int waves_per_block) {
   typedef typename ActOf<T>::type Act;
-  // blockIdx.y selects one of gridDim.y independent problems stacked contiguously
+  // blockIdx.y selects one of the independent problems stacked contiguously
   {
     const int64_t b = blockIdx.y;
     const int64_t gsz = (int64_t)N * (K / group);
@@ -813,7 +811,6 @@ __global__ __launch_bounds__(256) void gemv_w4a16_kernel(const T* __restrict__ A
   }
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int waves_per_block = blockDim.x >> 6;
   const int row0 = (blockIdx.x * waves_per_block + wave) * R;
   if (row0 >= N) return;  // whole wavefront leaves together
 
@@ -881,7 +878,7 @@ __global__ __launch_bounds__(256) void w4a16_tail_rows_kernel(const T* __restric
                                                               float zero_scalar, int out_dtype, int64_t ldc, int64_t col0) {
   typedef typename ActOf<T>::type Act;
   const int lane = threadIdx.x & 63;
-  const int64_t m = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int64_t m = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (m >= M) return;  // whole wavefront leaves together
   const int chunks = K >> 5;
   const int groups = K / group;
@@ -934,7 +931,7 @@ static void launch_gemv(const void* A, const void* Wp, const void* scales, const
   const int blocks = (int)ceil_div(N, rows_per_block);
   gemv_w4a16_kernel<T, R, MT><<<dim3(blocks, batch), 64 * waves_per_block, 0, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales,
                                                                      (const T*)zeros, C, M, N, K, group, zero_scalar,
-                                                                     out_dtype);
+                                                                     out_dtype, waves_per_block);
 }
 
 // rows-per-wave / waves-per-block / blocks-per-CU overrides for tuning runs (0 = automatic)
@@ -965,7 +962,7 @@ static int launch_gemv_f16(const void* A, const void* Wp, const void* scales, co
   if (blocks > cap) blocks = cap < 1 ? 1 : cap;
   gemv_w4a16_f16_kernel<R, MT, D><<<dim3(blocks, batch), 64 * waves_per_block, lds, st>>>(
       (const half_t*)A, (const uint8_t*)Wp, (const half_t*)scales, (const half_t*)zeros, C, M, N, K, group_shift,
-      zero_scalar, out_dtype);
+      zero_scalar, out_dtype, blocks, waves_per_block);
   return 0;
 }
 
@@ -1078,7 +1075,7 @@ static int launch_gemv_ring(const void* A, const void* Wp, const void* scales, c
     attr_set = true;
   }
   kern<<<p.blocks, 64 * p.waves, p.lds_bytes, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, N, K,
-                                                  group_shift, zero_scalar, out_dtype, p.rows_per_block);
+                                                  group_shift, zero_scalar, out_dtype, p.rows_per_block, p.waves);
   return check_launch("tlq_gemm_w4a16(gemv)", LAYOUT == 1 ? "gemv_w4a16_ring_kernel, interleaved words" : "gemv_w4a16_ring_kernel") ? 0 : 1;
 }
 

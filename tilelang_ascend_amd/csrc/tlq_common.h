@@ -13,6 +13,10 @@ namespace tlq {
 // ---- error reporting (thread local, read back through tlq_last_error) -------------------
 void set_error(const char* fmt, ...);
 bool check_launch(const char* what, const char* detail = nullptr);
+// Kernel arguments: at most 112 bytes, and no gridDim / blockDim in a kernel, which brings 256 bytes of hidden ones: a work-group count or
+// size that a kernel needs is an argument of its own.  The host writes them to the device on every launch: up to 112 bytes without hidden ones 2.8 us
+// a launch back to back, from 116 on 3.7, 64 with hidden ones 4.1 (empty kernels, median of four).  tlq_gemm_w4a8 on 82 x 1376 x 512 3.8 -> 2.6 us
+// of host time, the whole call from Python 4.6 -> 3.8.
 uint64_t launch_count();
 bool launch_log_on();  // (texts that only the log wants are made only then)
 

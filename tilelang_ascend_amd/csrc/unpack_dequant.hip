@@ -27,11 +27,11 @@ __device__ __forceinline__ bf16_t convert_nibble<bf16_t>(uint32_t u, int sign_mo
 
 template <typename OutT>
 __global__ __launch_bounds__(256) void unpack_int4_vec8(const uint32_t* __restrict__ wp, OutT* __restrict__ out,
-                                                        int64_t n_words, int sign_mode) {
+                                                        int64_t n_words, int sign_mode, int blocks) {
   struct alignas(8 * sizeof(OutT)) Vec {
     OutT v[8];
   };
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_words; i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_words; i += (int64_t)blocks * 256) {
     uint32_t x = wp[i];
     Vec r;
 #pragma unroll
@@ -42,8 +42,8 @@ __global__ __launch_bounds__(256) void unpack_int4_vec8(const uint32_t* __restri
 
 template <typename OutT>
 __global__ __launch_bounds__(256) void unpack_int4_scalar(const uint8_t* __restrict__ wp, OutT* __restrict__ out,
-                                                          int64_t n_elems, int sign_mode) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_elems; i += (int64_t)gridDim.x * blockDim.x) {
+                                                          int64_t n_elems, int sign_mode, int blocks) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_elems; i += (int64_t)blocks * 256) {
     uint32_t b = wp[i >> 1];
     out[i] = convert_nibble<OutT>((b >> (4 * (i & 1))) & 0xF, sign_mode);
   }
@@ -57,11 +57,11 @@ template <typename T, int LAYOUT>
 __global__ __launch_bounds__(256) void dequant_w4_vec8(const uint32_t* __restrict__ wp, const T* __restrict__ scales,
                                                        const T* __restrict__ zeros, T* __restrict__ out,
                                                        int64_t n_words, int words_per_row, int group, int groups_per_row,
-                                                       float zero_scalar) {
+                                                       float zero_scalar, int blocks) {
   const T one = from_float<T>(1.0f);
   const T zs = from_float<T>(zero_scalar);
   const NibbleMagic mg = make_nibble_magic();
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_words; i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_words; i += (int64_t)blocks * 256) {
     int64_t row = i / words_per_row;
     int k = (int)(i - row * words_per_row) * 8;
     int64_t gi = row * groups_per_row + k / group;
@@ -81,12 +81,12 @@ __global__ __launch_bounds__(256) void dequant_w4_vec8(const uint32_t* __restric
 template <typename T>
 __global__ __launch_bounds__(256) void dequant_w4_scalar(const uint8_t* __restrict__ wp, const T* __restrict__ scales,
                                                          const T* __restrict__ zeros, T* __restrict__ out, int64_t N,
-                                                         int64_t K, int group, float zero_scalar) {
+                                                         int64_t K, int group, float zero_scalar, int blocks) {
   const T one = from_float<T>(1.0f);
   const T zs = from_float<T>(zero_scalar);
   int64_t total = N * K;
   int64_t G = K / group;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)blocks * 256) {
     int64_t row = i / K;
     int64_t k = i - row * K;
     int64_t gi = row * G + k / group;
@@ -108,10 +108,12 @@ static int launch_unpack(const void* wp, void* out, int64_t N, int64_t K, int si
   if (N * K == 0) return 0;
   const bool aligned = ((uintptr_t)wp % 4 == 0) && ((uintptr_t)out % (8 * sizeof(OutT)) == 0);
   if (K % 8 == 0 && aligned) {
-    int64_t n_words = N * K / 8;
-    unpack_int4_vec8<OutT><<<grid_for(n_words), 256, 0, st>>>((const uint32_t*)wp, (OutT*)out, n_words, sign_mode);
+    const int64_t n_words = N * K / 8;
+    const int blocks = grid_for(n_words);
+    unpack_int4_vec8<OutT><<<blocks, 256, 0, st>>>((const uint32_t*)wp, (OutT*)out, n_words, sign_mode, blocks);
   } else {
-    unpack_int4_scalar<OutT><<<grid_for(N * K), 256, 0, st>>>((const uint8_t*)wp, (OutT*)out, N * K, sign_mode);
+    const int blocks = grid_for(N * K);
+    unpack_int4_scalar<OutT><<<blocks, 256, 0, st>>>((const uint8_t*)wp, (OutT*)out, N * K, sign_mode, blocks);
   }
   return check_launch("tlq_unpack_int4") ? 0 : 1;
 }
@@ -122,20 +124,22 @@ static int launch_dequant(const void* wp, const void* scales, const void* zeros,
   if (N * K == 0) return 0;
   const bool aligned = ((uintptr_t)wp % 4 == 0) && ((uintptr_t)out % 16 == 0);
   if (K % 8 == 0 && group % 8 == 0 && aligned) {
-    int64_t n_words = N * K / 8;
+    const int64_t n_words = N * K / 8;
+    const int blocks = grid_for(n_words);
     if (w_layout == TLQ_W_INTERLEAVED_F16)
-      dequant_w4_vec8<T, 1><<<grid_for(n_words), 256, 0, st>>>((const uint32_t*)wp, (const T*)scales, (const T*)zeros, (T*)out, n_words,
-                                                              (int)(K / 8), (int)group, (int)(K / group), zero_scalar);
+      dequant_w4_vec8<T, 1><<<blocks, 256, 0, st>>>((const uint32_t*)wp, (const T*)scales, (const T*)zeros, (T*)out, n_words,
+                                                              (int)(K / 8), (int)group, (int)(K / group), zero_scalar, blocks);
     else
-      dequant_w4_vec8<T, 0><<<grid_for(n_words), 256, 0, st>>>((const uint32_t*)wp, (const T*)scales, (const T*)zeros, (T*)out, n_words,
-                                                              (int)(K / 8), (int)group, (int)(K / group), zero_scalar);
+      dequant_w4_vec8<T, 0><<<blocks, 256, 0, st>>>((const uint32_t*)wp, (const T*)scales, (const T*)zeros, (T*)out, n_words,
+                                                              (int)(K / 8), (int)group, (int)(K / group), zero_scalar, blocks);
   } else {
     if (w_layout != TLQ_W_PLAIN) {
       set_error("tlq_dequant_w4_layout: interleaved weights need K %% 8 == 0, group %% 8 == 0, 4-byte aligned words and a 16-byte aligned output");
       return 1;
     }
-    dequant_w4_scalar<T><<<grid_for(N * K), 256, 0, st>>>((const uint8_t*)wp, (const T*)scales, (const T*)zeros, (T*)out,
-                                                         N, K, (int)group, zero_scalar);
+    const int blocks = grid_for(N * K);
+    dequant_w4_scalar<T><<<blocks, 256, 0, st>>>((const uint8_t*)wp, (const T*)scales, (const T*)zeros, (T*)out,
+                                                         N, K, (int)group, zero_scalar, blocks);
   }
   return check_launch("tlq_dequant_w4", "dequant_w4_vec8") ? 0 : 1;
 }
