@@ -20,6 +20,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -118,13 +119,13 @@ int launch(const PlanObject& p, const at::Tensor* const* t, int device, hipStrea
   } else if (p.kind == kF16) {
     ws_bytes = lib.tlq_f16_workspace_bytes(1, v[0], v[1], v[2]);
   }
-  at::Tensor ws;
+  c10::DataPtr ws;  // the allocator's block alone: no tensor around it
   if (ws_bytes > 0) {
-    const int64_t shape[1] = {ws_bytes};
-    ws = new_tensor(shape, at::kByte, device);
-    if (other_stream) ws.record_stream(c10::hip::getStreamFromExternalMasqueradingAsCUDA(stream, (c10::DeviceIndex)device).unwrap());
+    ws = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get()->allocate((size_t)ws_bytes);
+    if (other_stream)
+      c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::recordStreamMasqueradingAsCUDA(ws, c10::hip::getStreamFromExternalMasqueradingAsCUDA(stream, (c10::DeviceIndex)device));
   }
-  void* const w = ws_bytes > 0 ? ws.data_ptr() : nullptr;
+  void* const w = ws.get();
   Released free_lock;
   switch (p.kind) {
     case kW4A16: {

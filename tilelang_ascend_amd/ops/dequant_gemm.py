@@ -241,11 +241,12 @@ def dequant_gemm_fp16_wrapper(M: int, N: int, K: int, block_M: int, block_N: int
         if kernel is None:
             kernel = kernels[key] = w4a16_gemm(M, N, K, block_M, block_N, block_K, input_dtype, output_dtype, group_size,
                                                scales is not None, key[1], algo, weight_layout=weight_layout)
-        args = [A, B_packed]
-        if scales is not None:
-            args.append(scales)
+        args = (A, B_packed) if scales is None else (A, B_packed, scales)
         if z_is_tensor:
-            args.append(zeros)
+            args += (zeros,)
+        out = kernel._fast(*args)  # the ordinary call
+        if out is not NotImplemented:
+            return out
         if A.is_cuda:
             return kernel(*args)
         return kernel(*[a.cuda() for a in args]).cpu()
