@@ -118,10 +118,10 @@ void tlq_tune_gemm_groups(int variant);                       /* the ring kernel
 void tlq_tune_gemm_band(int tile_rows);                       /* tile rows per band of the MFMA kernels' tile order (default 4) */
 void tlq_tune_gemm_tile(int tile);                            /* square tile of the plain 16-bit GEMM (and of the second of the two W4A16 passes):
                                                               * 128 | 256, 0 = by the number of output tiles */
-void tlq_tune_gemm_slots(int mode);                          /* the kernel that cuts LDS into five operand-tile slots (256 x 256 tiles, whole 128-byte
-                                                              * stages of K only): 1 (default) where it measured faster than the two-stage kernel
-                                                              * (int8, several batches of up to 2048 rows), 2 wherever it can run (also the plain
-                                                              * 16-bit GEMMs), 0 never */
+void tlq_tune_gemm_slots(int mode);                          /* 256 x 256 tiles of whole 128-byte stages of K: 1 (default) by the number of stages and
+                                                              * tiles, 0 the two-stage kernel, 2 the one that cuts LDS into five operand-tile slots
+                                                              * (by itself int8, short rows, several batches of up to 2048 rows), 3 the one on four
+                                                              * wavefronts (long rows by itself), each wherever it can run */
 void tlq_tune_w4a16_decode(int on);                          /* 0: the decode kernel is never picked automatically */
 void tlq_tune_w4a16_stream(int on);                          /* 0: tlq_gemm_w4a16_ws never picks the streaming kernel by itself */
 void tlq_tune_w4a16_stream_tiles(int tiles);                 /* 16-row activation tiles per work-group of the streaming kernel, 2, 4, 6 or 8, + 16 for four groups of wavefronts over K (128 weight rows per work-group) instead of two (256); 0 = by its estimate */

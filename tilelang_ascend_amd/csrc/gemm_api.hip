@@ -90,7 +90,7 @@ int gemm_w4a16_decode(const void* A, const void* Wp, const void* scales, const v
 
 thread_local int g_gemm_band_rows = 0;
 thread_local int g_gemm_groups = 0;
-thread_local int g_gemm_slots = 1;  // tlq_tune_gemm_slots: 0 = never the five-slot kernel, 1 = where it measured faster, 2 = wherever it can run
+thread_local int g_gemm_slots = 1;
 extern thread_local int g_gemm_f16_tile;
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // compute units of the current device (256 when it cannot be asked, e.g. without a GPU)
@@ -177,7 +177,7 @@ extern "C" {
 
 void tlq_tune_gemm_groups(int variant) { tlq::tuning_changed(), tlq::g_gemm_groups = variant < 0 || variant > 5 ? 0 : variant; }
 void tlq_tune_gemm_band(int tile_rows) { tlq::g_gemm_band_rows = tile_rows < 0 ? 0 : tile_rows; }
-void tlq_tune_gemm_slots(int mode) { tlq::g_gemm_slots = mode < 0 ? 0 : (mode > 2 ? 2 : mode); }
+void tlq_tune_gemm_slots(int mode) { tlq::tuning_changed(), tlq::g_gemm_slots = mode < 0 ? 0 : (mode > 3 ? 2 : mode); }
 int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused) {
   return tlq::prefer_small_tiles(batch, M, N, fused ? 0.65 : 0.72) ? 128 : 256;
 }

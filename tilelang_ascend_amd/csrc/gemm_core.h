@@ -69,11 +69,11 @@ __device__ __forceinline__ int kn_swz(int k) {
 template <int BN>
 struct KNFrag8 {
   typedef int v2i_t __attribute__((ext_vector_type(2)));
-  uint32_t off[4];
+  uint32_t off[8];
   __device__ __forceinline__ KNFrag8(int lane, int wave_row0) {
     // the swizzle of a k row is unchanged by the +8 (second read) and +64 (k-step) row offsets
 #pragma unroll
-    for (int t = 0; t < 4; ++t) off[t] = addr::knfrag_off<BN>(lane, wave_row0, t);
+    for (int t = 0; t < 8; ++t) off[t] = addr::knfrag_off<BN>(lane, wave_row0, t);
   }
   __device__ __forceinline__ uint4_t read(const uint8_t* tile, int ks, int t) const {
     typedef __attribute__((address_space(3))) v2i_t* lds_ptr;
@@ -89,10 +89,10 @@ struct KNFrag8 {
 template <int BN>
 struct KNFrag16 {
   typedef short v4s_t __attribute__((ext_vector_type(4)));
-  uint32_t off[4];
+  uint32_t off[8];
   __device__ __forceinline__ KNFrag16(int lane, int wave_col0) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) off[t] = addr::kn16frag_off<BN>(lane, wave_col0, t);
+    for (int t = 0; t < 8; ++t) off[t] = addr::kn16frag_off<BN>(lane, wave_col0, t);
   }
   __device__ __forceinline__ uint4_t read(const uint8_t* tile, int ks, int t) const {
     typedef __attribute__((address_space(3))) v4s_t* lds_ptr;
@@ -693,11 +693,18 @@ __device__ __forceinline__ uint4_t pack_with(const Epi& epi, const S& sc, int m,
     return epi.pack(m, n, acc, M, N);
 }
 
-template <class Epi, int TM, int TN, class Acc, class S>
+// TMP: MFMA tile rows that a region holds at a time (16 rows x 128 B each)
+template <class Epi, int TM, int TN, int TMP = TM, class Acc, class S>
 __device__ __forceinline__ void write_tile_with(const Epi& epi, const S& scales, Acc (&acc)[TN][TM], uint8_t* region, int lane, int m_base,
                                                 int n_base, int M, int N) {
   const int r16 = lane & 15, q = lane >> 4;
   const int osz = epi.out_bytes();
+  // 64 accumulator tiles live in the accumulation registers: each is moved where it is used, or the compiler moves many ahead and spills
+  auto taken = [&](const auto& sum) {
+    std::remove_const_t<std::remove_reference_t<decltype(sum)>> v = sum;
+    if constexpr (TM * TN >= 64) asm volatile("" : "+v"(v));
+    return v;
+  };
   bool staged = false;
   // (whole passes of 128 output bytes per row only: a wavefront tile whose width is not a multiple of a pass goes the direct way)
   if constexpr (Epi::STAGED)
@@ -706,7 +713,7 @@ __device__ __forceinline__ void write_tile_with(const Epi& epi, const S& scales,
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) epi.store(m_base + tm * 16 + r16, n_base + tn * 16 + q * 4, acc[tn][tm], M, N);
+      for (int tm = 0; tm < TM; ++tm) epi.store(m_base + tm * 16 + r16, n_base + tn * 16 + q * 4, taken(acc[tn][tm]), M, N);
     return;
   }
   auto run = [&](auto osz_tag) {
@@ -714,15 +721,16 @@ __device__ __forceinline__ void write_tile_with(const Epi& epi, const S& scales,
     constexpr int TNP = 128 / (16 * OSZ);  // MFMA tile columns per pass: 128 bytes of output per row
     if constexpr (TN % TNP == 0) {
 #pragma unroll
-      for (int p0 = 0; p0 < TN; p0 += TNP) {
+      for (int pass = 0; pass < TN / TNP * (TM / TMP); ++pass) {
+        const int p0 = pass / (TM / TMP) * TNP, row0 = pass % (TM / TMP) * TMP * 16;  // the pass's first tile column, and its first row
 #pragma unroll
         for (int t = 0; t < TNP; ++t)
 #pragma unroll
-          for (int tm = 0; tm < TM; ++tm) {
+          for (int tm = row0 / 16; tm < row0 / 16 + TMP; ++tm) {
             const int row = tm * 16 + r16;
-            const uint4_t v = pack_with<Epi>(epi, scales, m_base + row, n_base + (p0 + t) * 16 + q * 4, acc[p0 + t][tm], tm, p0 + t, M, N);
+            const uint4_t v = pack_with<Epi>(epi, scales, m_base + row, n_base + (p0 + t) * 16 + q * 4, taken(acc[p0 + t][tm]), tm, p0 + t, M, N);
             const int byte = (t * 16 + q * 4) * OSZ;  // offset inside the 128-byte row of this pass
-            uint8_t* dst = region + lds_off(row, byte >> 4) + (byte & 15);
+            uint8_t* dst = region + lds_off(row - row0, byte >> 4) + (byte & 15);
             if (OSZ == 2)
               *(uint2_t*)dst = uint2_t{v.x, v.y};
             else
@@ -731,10 +739,10 @@ __device__ __forceinline__ void write_tile_with(const Epi& epi, const S& scales,
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int j = 0; j < 2 * TM; ++j) {
+        for (int j = 0; j < 2 * TMP; ++j) {
           const int row = j * 8 + (lane >> 3), chunk = lane & 7;
           const uint4_t v = *(const uint4_t*)(region + lds_off(row, chunk));
-          const int m = m_base + row, n = n_base + p0 * 16 + chunk * (16 / OSZ);
+          const int m = m_base + row0 + row, n = n_base + p0 * 16 + chunk * (16 / OSZ);
           if (m < M && n < N) *(uint4_t*)epi.addr_of(m, n) = v;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -766,9 +774,8 @@ struct TileCoord {
   int batch, m0, n0;
 };
 template <int BM, int BN>
-__device__ __forceinline__ TileCoord tile_of_block(int total, int M, int N, int GM) {
+__device__ __forceinline__ TileCoord tile_of_index(int lid, int total, int M, int N, int GM) {
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  int lid = blockIdx.x;
   if ((total & 7) == 0) lid = (lid & 7) * (total >> 3) + (lid >> 3);
   const int per_batch = tiles_m * tiles_n;
   TileCoord t;
@@ -780,6 +787,10 @@ __device__ __forceinline__ TileCoord tile_of_block(int total, int M, int N, int 
   t.m0 = (band * GM + r % rows) * BM;
   t.n0 = (r / rows) * BN;
   return t;
+}
+template <int BM, int BN>
+__device__ __forceinline__ TileCoord tile_of_block(int total, int M, int N, int GM) {
+  return tile_of_index<BM, BN>(blockIdx.x, total, M, N, GM);
 }
 
 // ---- the kernel -----------------------------------------------------------------------------
@@ -979,6 +990,27 @@ static constexpr RingCost kRingCost[4][4] = {
     {{5.07, 0.283, 0.262}, {4.70, 0.193, 0.158}, {4.17, 0.224, 0.160}, {4.81, 0.146, 0.097}},
     {{5.94, 0.365, 0.276}, {5.83, 0.291, 0.211}, {5.14, 0.313, 0.167}, {5.28, 0.258, 0.116}},
     {{6.08, 0.287, 0.261}, {6.18, 0.193, 0.171}, {5.10, 0.225, 0.164}, {5.50, 0.147, 0.107}}};
+// ---- 256 x 256 tiles on four wavefronts (gemm_quad.h) ----
+extern thread_local int g_gemm_slots;  // tlq_tune_gemm_slots: 0 = the two-stage kernel alone, 1 = automatic, 2 = five slots, 3 = four wavefronts, wherever either can run
+// In the place of the other kernels of 256 x 256 tiles from so many stages on: 16-bit 17 in one round of tiles, 9 in two, 6 from three on, int8
+// 17, 17, 9.  Its first tile's operands and its last tile's store are four wavefronts' work.  On 480 problems (120 per kind, M 256 .. 8192, N 256 ..
+// 14336, 128 - 28000 bytes of K, one to four batches) time over that of the kernel before, on average, one round: 1.11 - 1.17 on 5 - 8 stages, 0.99 - 1.09 on
+// 9 - 16, 0.90 - 0.97 on 17 - 32, 0.86 - 0.93 beyond; three rounds and more: 16-bit 0.97 - 1.0 from 3 stages on, int8 1.02 - 1.05 on 3 - 8, 0.97 - 0.99 on 9 - 16.
+inline bool quad_takes(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes) {
+  const int64_t stages = k_bytes / kStageBytes;
+  if (k_bytes % kStageBytes != 0 || stages < 2 || (g_gemm_slots != 1 && g_gemm_slots != 3)) return false;
+  if (g_gemm_slots == 3) return true;
+  int cus = tlq_device_cu_count();
+  if (cus <= 0) cus = 256;
+  const int64_t tiles = batch * ceil_div(M, (int64_t)256) * ceil_div(N, (int64_t)256);
+  if (kind >= kTileI8KN) return stages >= (tiles > 2 * cus ? 9 : 17);
+  return stages >= (tiles > 2 * cus ? 6 : (tiles > cus ? 9 : 17));
+}
+// Per round: fixed + stages x step, fitted to the 167 of those problems that it takes (5 - 9 % rms); with every CU busy 1.5 PFLOP/s and 2.4 POP/s.
+struct QuadCost {
+  double launch, fixed, step;
+};
+static constexpr QuadCost kQuadCost[4] = {{0.0, 8.7, 1.07}, {0.0, 9.0, 1.01}, {0.0, 11.6, 1.04}, {3.5, 12.7, 0.88}};
 inline int64_t tile_blocks(int variant, int64_t batch, int64_t M, int64_t N) {  // variant 1 (plain 128 x 128), kGroup*, 6 (256 x 256)
   static constexpr int kRows[6] = {128, 128, 128, 64, 64, 256}, kCols[6] = {128, 128, 64, 128, 64, 256};
   return batch * ceil_div(M, (int64_t)kRows[variant - 1]) * ceil_div(N, (int64_t)kCols[variant - 1]);
@@ -996,6 +1028,11 @@ inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int6
     const double in_round = blocks < cus ? (double)blocks / (double)cus : 1.0;
     const double us = (double)ceil_div(blocks, (int64_t)cus) * (c.fixed + (double)stages * (c.step + c.shared * in_round));
     return us > floor_us ? us : floor_us;
+  }
+  if (variant == 6 && quad_takes(kind, batch, M, N, stages * kStageBytes)) {
+    const QuadCost& c = kQuadCost[kind];
+    const double run = (double)ceil_div(blocks, (int64_t)cus) * (c.fixed + (double)stages * c.step), rate = product * (kind >= kTileI8KN ? 2.1 / 2.4 : 1.45 / 1.5);
+    return c.launch + (run > rate ? (run > memory ? run : memory) : (rate > memory ? rate : memory));
   }
   const TileCost& c = kTileCost[kind][variant == 1 ? 0 : 1];
   const double run = c.fixed + c.step * (double)stages;

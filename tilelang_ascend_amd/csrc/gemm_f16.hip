@@ -1,6 +1,7 @@
 // Plain fp16 / bf16 GEMM with fp32 accumulation: C[b, M, N] = A[b, M, K] . B[b], B[b] stored [K, N]
 // (transposed on the fly) or [N, K]; the matrices of a batch follow each other densely.
 #include "gemm_core.h"
+#include "gemm_quad.h"
 #include "gemm_ring.h"
 #include "gemm_slots.h"
 
@@ -225,6 +226,14 @@ static int dispatch_f16(const void* A, const void* B, void* C, int64_t batch, in
     KNParams pw{(const uint8_t*)B, N * 2, K * N * 2, K};
     EpiFloat::Params pe{C, N, M * N, out_dtype};
     return launch_gemm_slots<Mma, H16KNLoaderDirect<256, 512>, EpiFloat>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16", 4);
+  }
+  if ((b_layout == TLQ_B_NK || N % 8 == 0) && quad_takes(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, batch, M, N, K * 2)) {
+    typedef RowLoaderDirect<256, 256> Rows;
+    const typename Rows::Params pa((const uint8_t*)A, K * 2, M * K * 2, K * 2);
+    const EpiFloat::Params pe(C, N, M * N, out_dtype);
+    if (b_layout == TLQ_B_NK)
+      return launch_quad<Mma, Rows, EpiFloat>(pa, typename Rows::Params((const uint8_t*)B, K * 2, N * K * 2, K * 2), pe, batch, M, N, K * 2, st, "tlq_gemm_f16", 4);
+    return launch_quad<Mma, H16KNLoaderDirect<256, 256>, EpiFloat>(pa, KNParams((const uint8_t*)B, N * 2, K * N * 2, K), pe, batch, M, N, K * 2, st, "tlq_gemm_f16", 4);
   }
   return run_f16<Mma, 256, 256, 2, 4>(A, B, C, batch, M, N, K, out_dtype, b_layout, st);
 }

@@ -4,6 +4,7 @@
 //   * W4A8: packed int4 weights expanded to int8 on the way into LDS
 // The second operand may be stored [K, N] (transposed on the fly) or [N, K].
 #include "gemm_core.h"
+#include "gemm_quad.h"
 #include "gemm_ring.h"
 #include "gemm_slots.h"
 
@@ -127,7 +128,13 @@ template <class Epi>
 static int dispatch_i8(const void* A, const void* B, const typename Epi::Params& pe, int64_t batch, int64_t M,
                        int64_t N, int64_t K, int b_layout, hipStream_t st, const char* what) {
   const int tile = pick_tile(batch, M, N);
-  // The five-slot kernel where it measured ahead of the two-stage loop in alternating runs: several batches of up to
+  if (tile == 256 && quad_takes(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, batch, M, N, K)) {
+    typedef RowLoaderDirect<256, 256> Rows;
+    const typename Rows::Params pa((const uint8_t*)A, K, M * K, K);
+    if (b_layout == TLQ_B_NK) return launch_quad<MmaI8, Rows, Epi>(pa, typename Rows::Params((const uint8_t*)B, K, N * K, K), pe, batch, M, N, K, st, what, 2);
+    return launch_quad<MmaI8, I8KNLoaderDirect<256, 256>, Epi>(pa, KNParams((const uint8_t*)B, N, K * N, K), pe, batch, M, N, K, st, what, 2);
+  }
+  // Short rows: the five-slot kernel where it measured ahead of the two-stage loop in alternating runs: several batches of up to
   // 2048 rows (1 - 3 %); with one batch or longer matrices the two-stage loop is 2 - 14 % ahead.
   const bool slots = g_gemm_slots == 2 || (g_gemm_slots == 1 && batch > 1 && M <= 2048);
   if (b_layout == TLQ_B_KN) {
