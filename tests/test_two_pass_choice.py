@@ -88,3 +88,28 @@ def test_last_fp16_rows_keep_the_gemv_kernels_precision(M, N, K, group, tensor):
         torch.cuda.synchronize()
         assert torch.equal(C[head:], last)
         assert not gemv or bool(((C[head:].double() - want).abs() <= bound).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,group,dt", [(8192, 4096, 4096, 64, torch.float16), (4907, 256, 2048, 64, torch.bfloat16), (881, 528, 3968, 128, torch.bfloat16), (1237, 2912, 2688, 128, torch.bfloat16)])
+def test_two_passes_take_all_rows(M, N, K, group, dt):
+    """Large products, many rows on few weights, and row counts that are no multiple of four where no panel kernel would run: the dequantisation pass and
+    one product over all rows; the same bits as the two passes by name."""
+    lib, P, st = _abi.load(), _abi.ptr, torch.cuda.current_stream().cuda_stream
+    print(f"two passes for all rows M={M} N={N} K={K} g={group} {dt}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A = torch.randn(M, K, device="cuda", generator=g).to(dt)
+    Wp = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device="cuda", generator=g)
+    s = (torch.rand(N, K // group, device="cuda", generator=g) * 0.015 + 0.005).to(dt)
+    z = torch.randint(6, 10, (N, K // group), device="cuda", generator=g).to(dt)
+    size = lib.tlq_w4a16_workspace_bytes_for(M, N, K, _abi.ALGO_AUTO)
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+    t, C = (_abi.F16 if dt == torch.float16 else _abi.BF16), [torch.empty(M, N, dtype=dt, device="cuda") for _ in range(2)]
+    for c, algo in zip(C, (_abi.ALGO_AUTO, _abi.ALGO_TWO_PASS)):
+        lib.tlq_debug_launch_log(1)
+        rc = lib.tlq_gemm_w4a16_ws(P(A), P(Wp), P(s), P(z), P(c), M, N, K, group, 0.0, t, t, algo, P(ws), size, st)
+        log = lib.tlq_debug_launch_log_text().decode()
+        lib.tlq_debug_launch_log(0)
+        _abi.check(rc)
+        assert ("dequant_w4" in log and log.count("tlq_gemm_w4a16") == 0) or lib.tlq_device_cu_count() != 256, log
+    assert torch.equal(C[0], C[1])

@@ -693,28 +693,41 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 }
 
 // Above 512 rows: do the two passes beat what the panel kernels would run?  The dequantisation pass costs 3 us and the weights' bytes, the
-// plain GEMM behind it has smaller tiles and any row count, while the panel kernels have 8 us per round of
+// plain GEMM behind it runs large products at 1.4 - 1.5 PFLOP/s where the 256-row panel kernel reaches 1.2 - 1.3 (8192 x 14336 x 4096 fp16 in groups of
+// 64 774 -> 684 us), has smaller tiles, and takes any row count, while the panel kernels have 8 us per round of
 // work-groups (many rounds of short rows: 4868 x 3152 x 384 bf16 36.9 -> 25.5 us, 6631 x 4608 x 256 38.7 -> 29.8) and leave
-// one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  On 1500 problems
-// (M 513 .. 8192, N 128 .. 14400, K 256 .. 19200, half of the row counts odd) the bar below takes the two passes on 278, ahead by 1.15 - 1.32 x
-// on average, more than 3 % behind on five (12 % at most), on 1500 others 277 and three (4 %); a bar of 0.9 for 0.85 takes 453, 48 of them behind.  The estimates of both
-// panel kernels are 13 - 19 % high there (11 % rms), that of the two passes 4 % (16 - 23 %), which the bar takes in.
+// one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  The panel kernels' estimates
+// are 1.21 x high (11 % rms) short of the rate they reach at best, that of the two passes 0.91 x (7 %) in the kernel of four wavefronts and 1.0 - 1.07
+// elsewhere.  On 650 problems (M 513 .. 8192, N 256 .. 14336, K 256 .. 14336, groups of 64 and 128, both types) the panel kernels or the two passes
+// are the choice on 290: 1.7 % behind the faster of the two on average, 2.9 % by the rule before, of the hundred newly taken four more
+// than 3 % behind.  Where neither panel kernel would run, all rows go through the two passes and none is left over: 132 problems 6.4 % faster, none slower.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
 static double two_passes_us(int64_t M, int64_t N, int64_t K) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(M, N, K); }
 static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
-  const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
-  const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
-  const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
-  if (!p2.ok || N % 8 != 0) return false;
-  double panels;
-  const bool middle = pm.ok && panelm_estimate_wins(head, N, K, group);
-  if (middle)
-    panels = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, head, N, cus_now);
-  else if (panel256_fills(head, N, K, group))
-    panels = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, head, N, cus_now);
-  else
-    panels = two_passes_us(head, N, K);  // they would not run
-  return 1.1 * two_passes_us(M, N, K) < 0.85 * (panels + (head != M ? 5.5 : 0.0));
+  static thread_local PlanTable<bool> known;
+  return known.get(M, N, K, group, [&] {
+    const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
+    const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
+    const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
+    if (!p2.ok || N % 8 != 0) return false;
+    double panels;
+    if (pm.ok && panelm_estimate_wins(head, N, K, group))
+      panels = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, head, N, cus_now);
+    else if (panel256_fills(head, N, K, group))
+      panels = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, head, N, cus_now);
+    else
+      return true;
+    const double best = 2.0 * (double)M * (double)N * (double)K / 1.3e9;  // at 1.3 PFLOP/s
+    panels = panels / 1.21 > best ? panels / 1.21 : best;
+    const bool quad = !prefer_small_tiles(1, M, N) && quad_takes(kTileF16NK, 1, M, N, K * 2);
+    return (quad ? 1.05 : 1.0) * two_passes_us(M, N, K) < panels + (head != M ? 4.5 : 0.0);
+  });
+}
+// Many rows on up to 2^19 weights: the two passes or the tile kernel in one launch.  27 problems above 512 rows where that ran: 13 go to the two passes, 1.28 x
+// on average (4907 x 256 x 2048 38.9 -> 16.8 us), one of them 3 % behind.
+static bool two_passes_beat_tiles(int64_t M, int64_t N, int64_t K) {
+  static thread_local PlanTable<bool> known;
+  return M > 512 && N % 8 == 0 && known.get(M, N, K, 0, [&] { return two_passes_us(M, N, K) < 0.9 * fused_tile_us(M, N, K); });
 }
 
 // Above 512 rows: does the streaming kernel beat the panel kernels (their estimates are 13 - 19 % high, see above; a row count that is no
@@ -1061,7 +1074,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     // (rows of more than 1280 values only where the skinny kernel's work-groups, one per 16 weight rows, run in one round or
     // fill their last round: N = 6144, K = 2048, 384 work-groups: 16 - 22 against 14 - 15 us)
     const bool skinny_fills = ceil_div(N, (int64_t)16) <= cu_count_or_default() || tile_fill(1, 16, N, 16) >= 0.8;
-    if ((M <= 64 && (nk <= ((int64_t)1 << 21) || (nk <= ((int64_t)1 << 24) && (K <= 1280 || (K <= 2048 && skinny_fills))))) || nk <= ((int64_t)1 << 19))
+    if ((M <= 64 && (nk <= ((int64_t)1 << 21) || (nk <= ((int64_t)1 << 24) && (K <= 1280 || (K <= 2048 && skinny_fills))))) || (nk <= ((int64_t)1 << 19) && !(room_for_two_passes && two_passes_beat_tiles(M, N, K))))
       return tlq_gemm_w4a16(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, stream);
     // Short rows, 96 .. 512 activation rows, one round of 128 x 128 tiles: the tile kernel in one launch takes 4.5 us + 1.45 us
     // per 128 values of K whatever M and N, the streaming kernel 11 - 15 us at K = 512 and 19 - 30 us at K = 1024 .. 1536.
