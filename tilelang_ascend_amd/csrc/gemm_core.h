@@ -870,6 +870,14 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN >= 8 ? 2 : 1)) void gemm_mfma
     }
   };
 
+  // Per-row / per-column output scales travel while the main loop runs (int8 NK 160 x 11072 x 768 9.6 -> 9.3 us, KN 4 x 2921 x 11680 x 1024 198 -> 191).  The
+  // ring kernel, which issues several stages at the start, the small-tile kernel and tiles of 32 rows fetch theirs at the end: ahead of their
+  // loads they cost 1 - 3 %.
+  const Epi epi(pe, batch);
+  auto scales_now = [&] { return fetch_scales<Epi, TM, TN>(epi, m0 + wave_m0, n0 + wave_n0, lane, M, N); };
+  std::conditional_t<(BM >= 128), decltype(scales_now()), NoScales> out_scales;
+  if constexpr (BM >= 128) out_scales = scales_now();
+
   // prologue: stage 0 into buffer 0
   if (KT == 1 && k_tail) {
     al.template gload<true>(ra, 0, ldsA0);
@@ -930,12 +938,15 @@ __global__ __launch_bounds__(WM* WN * 64, (WM * WN >= 8 ? 2 : 1)) void gemm_mfma
   }
   if (KT > 0) stage((KT - 1) & 1, std::false_type{});
 
-  Epi epi(pe, batch);
   // the operand tiles are no longer needed once every wavefront is past its last stage: each wavefront then stages its
   // outputs through its own TM * 16 rows x 128 B of LDS
   static_assert(WM * WN * TM * 16 * kStageBytes <= 2 * (A_TILE + W_TILE), "staging area exceeds the operand tiles");
   if constexpr (Epi::STAGED) __syncthreads();
-  write_tile<Epi, TM, TN>(epi, acc, smem + wave * (TM * 16 * kStageBytes), lane, m0 + wave_m0, n0 + wave_n0, M, N);
+  uint8_t* const region = smem + wave * (TM * 16 * kStageBytes);
+  if constexpr (BM >= 128)
+    write_tile_with<Epi, TM, TN>(epi, out_scales, acc, region, lane, m0 + wave_m0, n0 + wave_n0, M, N);
+  else
+    write_tile<Epi, TM, TN>(epi, acc, region, lane, m0 + wave_m0, n0 + wave_n0, M, N);
 }
 
 // Host-side launcher: sets the dynamic LDS size and launches one work-group per tile.
