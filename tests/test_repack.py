@@ -90,6 +90,22 @@ def test_quantize_chunk_counts(dtype, chunks, group):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,words,group", [(1, 1, 8), (1, 63, 8), (3, 43, 8), (1, 130, 16), (5, 102, 24), (7, 73, 584), (2, 256, 128), (3, 343, 56), (9, 128, 1024)])
+def test_dequantize_word_counts(dtype, rows, words, group):
+    """Around the 64 and 128 words of 8 weights that a wavefront takes and the 512 of a work-group, groups that are a power of two and that are not."""
+    from tilelang_ascend_amd import ops
+
+    K, g = 8 * words, torch.Generator().manual_seed(words)
+    assert K % group == 0
+    Wp = torch.randint(0, 256, (rows, K // 2), dtype=torch.uint8, generator=g)
+    s = (torch.rand(rows, K // group, generator=g) * 0.015 + 0.005).to(dtype)
+    for z in (8, torch.randint(0, 16, (rows, K // group), generator=g).to(dtype), (torch.rand(rows, K // group, generator=g) * 15).to(dtype)):
+        got = ops.dequantize_w4(Wp.cuda(), s.cuda(), z.cuda() if isinstance(z, torch.Tensor) else z, group, dtype).cpu()
+        assert torch.equal(got.view(torch.int16), ref.dequant_w4(Wp, s, z, group, dtype).view(torch.int16))
+
+
+@pytest.mark.gpu
 def test_quantize_pack_then_gemm_round_trip():
     """quantise -> pack on the GPU -> W4A16 GEMM with zero point 8 equals the GEMM on the dequantised weights."""
     from tilelang_ascend_amd.ops import w4a16_gemm
