@@ -71,6 +71,35 @@ def test_16_bit(dtype, layout, B, M, N, stages):
             assert bool(((C[0][-1].double() - want).abs() <= K * 2.0 ** -24 * size).all())
 
 
+@pytest.mark.gpu
+def test_in_a_graph():
+    """More tiles than work-groups, captured and replayed with other inputs, eager work in between."""
+    B, M, N, K = 1, 8192, 4096, 1088
+    A, W = torch.randn(M, K, generator=gen(1)).to(torch.bfloat16).cuda(), torch.randn(N, K, generator=gen(2)).to(torch.bfloat16).cuda()
+    C, D, lib, P = torch.empty(M, N, dtype=torch.bfloat16, device="cuda"), torch.empty(M, N, dtype=torch.bfloat16, device="cuda"), _abi.load(), _abi.ptr
+
+    def call(out):
+        _abi.check(lib.tlq_gemm_f16_batched(P(A), P(W), P(out), B, M, N, K, _abi.BF16, _abi.BF16, _abi.B_NK, torch.cuda.current_stream().cuda_stream))
+
+    lib.tlq_debug_launch_log(1)
+    call(C)
+    log = lib.tlq_debug_launch_log_text().decode()
+    lib.tlq_debug_launch_log(0)
+    assert "quad_gemm_mfma_kernel" in log or lib.tlq_device_cu_count() != 256, log
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(C)
+    for seed in (3, 4, 5):
+        A.copy_(torch.randn(M, K, generator=gen(seed)).to(torch.bfloat16))
+        C.fill_(-1)
+        torch.cuda.synchronize()
+        graph.replay()
+        call(D)
+        torch.cuda.synchronize()
+        assert torch.equal(C, D)
+
+
 @pytest.mark.parametrize("source", ["gemm_f16", "gemm_int8"])
 def test_no_spills(tmp_path, source):
     """The waits of the main loop count its loads: nothing may go through scratch memory there."""
