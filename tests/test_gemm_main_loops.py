@@ -93,3 +93,32 @@ def test_w8a8_same_bits_on_both_main_loops(hook, value, layout, B, M, N, K):
     got, got_i = _with_hook(hook, value, run)
     assert torch.equal(got_i, want_i), f"{hook}={value} int32 accumulators differ"
     assert_bit_equal(got, want, f"{hook}={value} {layout} {B}x{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("layout", ["KN", "NK"])
+@pytest.mark.parametrize("tile,groups", [(32, 0), (128, 1), (128, 2), (128, 3), (128, 4), (128, 5), (256, 0)])
+def test_scales_of_every_tiling(tile, groups, layout):
+    """Row scales or none and column scales, one value or a tensor that starts 4 bytes behind a 16-byte boundary, of ragged tiles: two-stage kernels
+    and the ring kernel's tiles (the four wavefronts of 256 x 256 tiles have their own test)."""
+    from tilelang_ascend_amd import _abi
+
+    lib, P, st = _abi.load(), _abi.ptr, torch.cuda.current_stream().cuda_stream
+    M, N, K = 130, 272, 1040
+    print(f"scales tile={tile} groups={groups} {layout}", flush=True)
+    A, W = torch.randint(-127, 128, (M, K), dtype=torch.int8, generator=gen(7)), torch.randint(-127, 128, (K, N), dtype=torch.int8, generator=gen(8))
+    acc = (A.double() @ W.double()).float()  # (sums below 2^24)
+    sa, sb = torch.rand(M, generator=gen(9)) * 0.04 + 0.01, torch.rand(N + 1, generator=gen(10)) * 0.009 + 0.001
+    dA, dW, dsb = A.cuda(), (W if layout == "KN" else W.t().contiguous()).cuda(), sb.cuda()
+    lay = _abi.B_KN if layout == "KN" else _abi.B_NK
+    lib.tlq_tune_i8_tile(tile), lib.tlq_tune_gemm_groups(groups)
+    try:
+        for rows in (None, sa):
+            for lo, n in ((0, N), (1, N), (1, 1)):
+                for dtype, t in ((torch.float16, _abi.F16), (torch.float32, _abi.F32)):
+                    C = torch.full((M, N), float("nan"), dtype=dtype, device="cuda")
+                    drows = None if rows is None else rows.cuda()
+                    _abi.check(lib.tlq_gemm_w8a8(P(dA), P(dW), None if rows is None else P(drows), P(dsb[lo:lo + n]), P(C), 1, M, N, K, n, lay, t, st))
+                    scaled = (acc if rows is None else acc * rows[:, None]) * sb[lo:lo + n]
+                    assert_bit_equal(C.cpu(), scaled.to(dtype), f"tile={tile} groups={groups} {layout} rows={rows is not None} {lo} {n} {dtype}")
+    finally:
+        lib.tlq_tune_i8_tile(0), lib.tlq_tune_gemm_groups(0)

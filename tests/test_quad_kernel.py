@@ -43,11 +43,15 @@ def test_int8(layout, B, M, N, stages):
     C = torch.full((B, M, N), -1, dtype=torch.int32, device="cuda")
     run(3, lambda lib: lib.tlq_gemm_i8(P(A), P(Wd), P(C), B, M, N, K, code, st))
     assert torch.equal(C, want.to(torch.int32))
-    sa, sb = torch.rand(B, M, device="cuda", generator=g) * 0.04 + 0.01, torch.rand(N, device="cuda", generator=g) * 0.009 + 0.001
-    for scale, n in ((sb, N), (sb[:1].contiguous(), 1)):
-        out = torch.empty(B, M, N, dtype=torch.bfloat16, device="cuda")
-        run(3, lambda lib: lib.tlq_gemm_w8a8(P(A), P(Wd), P(sa), P(scale), P(out), B, M, N, K, n, code, _abi.BF16, st))
-        assert torch.equal(out, ((want * sa[:, :, None]) * scale).to(torch.bfloat16))
+    # row scales or none, a scale per column (from a 16-byte boundary and 4 bytes behind one) or one for all, every result type
+    sa, sb = torch.rand(B, M, device="cuda", generator=g) * 0.04 + 0.01, torch.rand(N + 1, device="cuda", generator=g) * 0.009 + 0.001
+    for rows in (sa, None):
+        for scale, n in ((sb[:N], N), (sb[1:], N), (sb[:1], 1)):
+            for dtype, t in ((torch.bfloat16, _abi.BF16), (torch.float16, _abi.F16), (torch.float32, _abi.F32)):
+                out = torch.full((B, M, N), -1, dtype=dtype, device="cuda")
+                run(3, lambda lib: lib.tlq_gemm_w8a8(P(A), P(Wd), None if rows is None else P(rows), P(scale), P(out), B, M, N, K, n, code, t, st))
+                scaled = (want if rows is None else want * rows[:, :, None]) * scale
+                assert torch.equal(out, scaled.to(dtype)), (rows is None, n, dtype)
 
 
 @pytest.mark.gpu
@@ -100,9 +104,7 @@ def test_in_a_graph():
         assert torch.equal(C, D)
 
 
-@pytest.mark.parametrize("source", ["gemm_f16", "gemm_int8"])
-def test_no_spills(tmp_path, source):
-    """The waits of the main loop count its loads: nothing may go through scratch memory there."""
+def code_object(tmp_path, source):
     obj, llvm = os.path.join(build.OBJ_DIR, source + ".o"), "/opt/rocm/llvm/bin"
     if not (os.path.exists(obj) and os.path.exists(f"{llvm}/clang-offload-bundler")):
         pytest.skip("objects of a build and ROCm's LLVM tools wanted")
@@ -110,9 +112,36 @@ def test_no_spills(tmp_path, source):
     subprocess.run([f"{llvm}/llvm-objcopy", "--dump-section", f".hip_fatbin={bundle}", obj, str(tmp_path / "copy.o")], check=True)
     subprocess.run([f"{llvm}/clang-offload-bundler", "--unbundle", "--type=o", f"--input={bundle}", f"--targets=hipv4-amdgcn-amd-amdhsa--{build.ARCH}",
                     f"--output={code}"], check=True)
+    return code, llvm
+
+
+@pytest.mark.parametrize("source", ["gemm_f16", "gemm_int8"])
+def test_no_spills(tmp_path, source):
+    """The waits of the main loop count its loads: nothing may go through scratch memory there."""
+    code, llvm = code_object(tmp_path, source)
     notes = subprocess.run([f"{llvm}/llvm-readelf", "--notes", str(code)], capture_output=True, text=True, check=True).stdout
     kernels = [(re.search(r"\.name:\s+(\S+)", k), k) for k in re.split(r"\n  - \.a(?:gpr_count|rgs)", notes)[1:]]
     quads = [(n[1], k) for n, k in kernels if n and "quad_gemm_mfma_kernel" in n[1]]
     assert len(quads) == 4
     for name, k in quads:
         assert re.search(r"\.vgpr_spill_count: (\d+)", k)[1] == "0" and re.search(r"\.private_segment_fixed_size: (\d+)", k)[1] == "0", name
+
+
+def test_nothing_is_drained_for_the_scales(tmp_path):
+    """A tile's scales are asked for at its start, when the tile before is still being stored and the loads of its own next stages are under way, and
+    have arrived with its first stage: no wait for vector memory stands between the loop's head and its first product, nor ahead of the
+    first output, where the next tile's loads are under way."""
+    code, llvm = code_object(tmp_path, "gemm_int8")
+    listing = subprocess.run([f"{llvm}/llvm-objdump", "-d", "--no-show-raw-insn", str(code)], capture_output=True, text=True, check=True).stdout
+    kernels = [k for k in re.split(r"\n[0-9a-f]{16} (?=<)", listing) if k.startswith("<_ZN3tlq21quad_gemm_mfma_kernel") and "EpiRescale" in k.split("\n", 1)[0]]
+    assert len(kernels) == 2
+    for k in kernels:
+        ops = [line.split("//")[0].strip() for line in k.split("\n")[1:]]
+
+        def at(start, *names):
+            return next(i for i in range(start, len(ops)) if ops[i].startswith(names))
+
+        head, first = at(0, "s_barrier"), at(0, "v_mfma")  # (the tile loop's head lies between them)
+        out = at(first, "v_accvgpr_read")
+        for lo, hi in ((head, first), (out, at(out, "ds_write"))):
+            assert hi > lo and not [op for op in ops[lo:hi] if "vmcnt" in op], ops[lo:hi]

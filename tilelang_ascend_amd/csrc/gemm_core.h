@@ -620,24 +620,46 @@ struct EpiRescale {
   struct Scales {
     float a[TM];
     float4_t b[TN];
+    // the compiler's wait for the loads stands here, not where they are first used
+    __device__ __forceinline__ void arrive() {
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) asm volatile("" : "+v"(a[tm]));
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) asm volatile("" : "+v"(b[tn]));
+    }
   };
+  // One branch for the row scales and one for the column scales, and a 16-byte load per column tile (N is a multiple of 16 wherever results are
+  // rescaled; a float4 of a matrix's last columns is the furthest that is read).  Asked for value by value behind a branch of its own each,
+  // the loads waited for each other's address registers, 71 of them with drains of everything in flight ahead of a wavefront's 128 x 128 products; the
+  // other tiles, which fetch theirs at the end or (128 rows) ahead of the loop, take 1 - 3.5 % less time with it (1500 random problems).
   template <int TM, int TN>
   __device__ __forceinline__ Scales<TM, TN> load_scales(int m_base, int n_base, int lane, int M, int N) const {
+    typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));  // (a scale tensor starts anywhere on 4 bytes)
     Scales<TM, TN> s;
     const int r16 = lane & 15, q = lane >> 4;
+    if (sa) {
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-      int m = m_base + tm * 16 + r16;
-      m = m < M ? m : M - 1;
-      s.a[tm] = sa ? sa[m] : 1.0f;
+      for (int tm = 0; tm < TM; ++tm) {
+        const int m = m_base + tm * 16 + r16;
+        s.a[tm] = *(const float*)((const uint8_t*)sa + 4u * (uint32_t)(m < M ? m : M - 1));
+      }
+    } else {
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) s.a[tm] = 1.0f;
     }
+    if (p.scale_b && !p.one_scale_b) {
 #pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int n = n_base + tn * 16 + q * 4;
+      for (int tn = 0; tn < TN; ++tn) {
+        const int n = n_base + tn * 16 + q * 4;
+        s.b[tn] = *(const float4_any*)((const uint8_t*)p.scale_b + 4u * (uint32_t)(n < N ? n : N - 4));
+      }
+    } else {
+      // (through the scalar cache: its wait drains no vector load)
+      const float b = p.scale_b ? *(const __attribute__((address_space(4))) float*)p.scale_b : 1.0f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int nn = (n + i < N) ? n + i : N - 1;
-        s.b[tn][i] = p.scale_b ? (p.one_scale_b ? p.scale_b[0] : p.scale_b[nn]) : 1.0f;
+      for (int tn = 0; tn < TN; ++tn) {
+        s.b[tn] = float4_t{b, b, b, b};
+        asm volatile("" : "+v"(s.b[tn]));
       }
     }
     return s;
@@ -677,7 +699,9 @@ template <class Epi, typename = void>
 struct EpiHasScales : std::false_type {};
 template <class Epi>
 struct EpiHasScales<Epi, std::enable_if_t<Epi::HAS_SCALES>> : std::true_type {};
-struct NoScales {};
+struct NoScales {
+  __device__ __forceinline__ void arrive() {}
+};
 template <class Epi, int TM, int TN>
 __device__ __forceinline__ auto fetch_scales(const Epi& epi, int m_base, int n_base, int lane, int M, int N) {
   if constexpr (EpiHasScales<Epi>::value)
