@@ -453,9 +453,13 @@ __host__ __device__ inline uint32_t ring_act_voff(int p0, int lane, int pieces) 
   P = P < pieces ? P : pieces - 1;
   return (uint32_t)ring_act_logical(P) * 16u;
 }
-// rows of wavefront `wave`, and the loads it may leave in flight when it reads its i-th row (row i + depth is issued
-// after row i has been read; loads retire in issue order)
-__host__ __device__ inline int ring_my_rows(int rows, int wave, int waves) { return wave < rows ? (rows - wave + waves - 1) / waves : 0; }
+// rows of wavefront `wave` -- (rows - wave) / waves, rounded up, as a multiplication: divided by an argument it is thirty dependent
+// instructions ahead of the first weights' loads (1 x 11008 x 4096 5.80 -> 5.75 us, twelve other shapes 2.7 %); exact for 16 wavefronts and 4096 rows, a plan has at most 1536 --, and the loads it may leave in flight
+// when it reads its i-th row (row i + depth is issued after row i has been read; loads retire in issue order)
+__host__ __device__ constexpr uint32_t ring_inverse(int waves) { return (65536u + (uint32_t)waves - 1u) / (uint32_t)waves; }
+__host__ __device__ inline int ring_my_rows(int rows, int wave, int waves, uint32_t inverse) {
+  return wave < rows ? (int)((uint32_t)(rows - wave + waves - 1) * inverse >> 16) : 0;
+}
 __host__ __device__ inline int ring_younger_rows(int i, int my_rows, int depth) {
   const int y = my_rows - 1 - i;
   return y < depth - 1 ? y : depth - 1;

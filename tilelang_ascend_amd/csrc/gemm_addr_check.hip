@@ -1260,6 +1260,11 @@ int check_gemv_ring(int64_t M, int64_t N, int64_t K, int64_t group, int rows_per
   CHECK_OR_FAIL(M >= 1 && M <= 2 && N >= 1 && K >= 32 && K % 32 == 0 && group >= 32 && K % group == 0 && rows_per_block >= 1 && waves >= 1 &&
                     waves <= 16 && depth >= 1 && depth <= 3,
                 "gemv ring: bad arguments");
+  CHECK_OR_FAIL(rows_per_block <= 4096, "gemv ring: %d rows for a work-group", rows_per_block);
+  for (int rows = 0; rows <= 4096; ++rows)
+    for (int w = 0; w < waves; ++w)
+      CHECK_OR_FAIL(addr::ring_my_rows(rows, w, waves, addr::ring_inverse(waves)) == (w < rows ? (rows - w + waves - 1) / waves : 0),
+                    "gemv ring: rows of wavefront %d of %d, %d rows", w, waves, rows);
   const int chunks = (int)(K / 32), groups = (int)(K / group), iters = (chunks + 63) / 64;
   CHECK_OR_FAIL(iters * depth <= 6, "gemv ring: %d loads per wavefront in flight have no s_waitcnt case", iters * depth);
   CHECK_OR_FAIL(groups % 8 == 0, "gemv ring: %d groups per row are not a whole number of 16-byte pieces", groups);
@@ -1307,7 +1312,7 @@ int check_gemv_ring(int64_t M, int64_t N, int64_t K, int64_t group, int rows_per
     // weights
     std::vector<int> reader((size_t)(r1 - r0), -1);
     for (int w = 0; w < waves; ++w) {
-      const int my_rows = addr::ring_my_rows((int)(r1 - r0), w, waves);
+      const int my_rows = addr::ring_my_rows((int)(r1 - r0), w, waves, addr::ring_inverse(waves));
       std::vector<int> slot(depth, -1);
       std::vector<char> read(my_rows > 0 ? my_rows : 1, 0);
       std::vector<int> queue;  // row index of each outstanding load, oldest first

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
                                                             const T* __restrict__ scales, const T* __restrict__ zeros,
                                                             void* __restrict__ C, float* __restrict__ partial, int M, int N,
                                                             int K, int gshift, float zero_scalar, int out_dtype, int stride,
-                                                            int waves) {
+                                                            int rounds, int waves) {
   typedef typename DecodeMma<T>::type Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
   constexpr int TS = addr::kDecTileSlots;
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tiles = (N + 15) >> 4, slices = K / addr::kDecSlice;
+  const int tiles = (N + 15) >> 4, slices = (int)((uint32_t)K / addr::kDecSlice);
   const int r16 = lane & 15, q = lane >> 4;
   uint8_t* const mine = smem + wave * WAVE;
   const uint32_t mine_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)mine);
@@ -82,8 +82,9 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
   n_active = n_active < waves ? n_active : waves;
   const int64_t k0 = (int64_t)(active ? slice : 0) * addr::kDecSlice;
   const int groups = K >> gshift;
-  const int first = blockIdx.x;  // and every stride-th tile after it
-  const int my_tiles = (tiles - first + stride - 1) / stride;
+  const int first = blockIdx.x;  // and every stride-th tile after it: `rounds` whole rounds (tiles / stride), and one more for the first work-groups
+  const int my_tiles = rounds + (first < tiles - rounds * stride ? 1 : 0);  // (no division ahead of the first
+  // loads, nor one per tile further down: 16 x 14336 x 4096 12.40 -> 12.11 us)
   const bool has_s = scales != nullptr, has_z = zeros != nullptr;
   const T one = from_float<T>(1.0f), zs = from_float<T>(zero_scalar);
   const NibbleMagic mg = make_nibble_magic();
@@ -172,6 +173,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = typename Mma::acc_t{0, 0, 0, 0};
 
+  int turn = 0;  // ts MT modulo waves (waves >= MT)
   for (int ts = 0; ts < my_tiles; ++ts) {
     const int t = first + ts * stride;
     if (active) {
@@ -264,9 +266,10 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
       }
     }
     __syncthreads();  // all partial tiles of tile t are in LDS (two buffers: the other one was read before the previous barrier)
-    int rw = wave - (ts * MT) % waves;
+    int rw = wave - turn;
     rw = rw < 0 ? rw + waves : rw;
-    if (rw < MT) {  // wavefronts (ts MT) % waves .. + MT - 1 add up the MT activation tiles
+    turn = turn + MT < waves ? turn + MT : turn + MT - waves;
+    if (rw < MT) {  // wavefronts turn .. turn + MT - 1 add up the MT activation tiles
       const int mt = rw;
       const uint32_t ro = RED + ((ts % RB) * MT + mt) * 1024 + lane * 16;
       float4_t sum = *(const float4_t*)(smem + ro);
@@ -347,7 +350,7 @@ static int launch_decode(const void* A, const void* Wp, const void* scales, cons
   }
   kern<<<dim3(p.grid_x, p.chunks), p.waves * 64, (size_t)p.lds_bytes, st>>>(
       (const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, p.chunks > 1 ? partial : nullptr, (int)M, (int)N, (int)K,
-      gshift, zero_scalar, out_dtype, p.grid_x, p.waves);
+      gshift, zero_scalar, out_dtype, p.grid_x, (int)(ceil_div(N, (int64_t)16) / p.grid_x), p.waves);
   return check_launch("tlq_gemm_w4a16(decode)", "w4a16_decode_kernel") ? 0 : 1;
 }
 

@@ -613,7 +613,7 @@ __global__ __launch_bounds__(1024) void gemv_w4a16_ring_kernel(const T* __restri
                                                                              const T* __restrict__ scales,
                                                                              const T* __restrict__ zeros, void* __restrict__ C,
                                                                              int N, int K, int group_shift, float zero_scalar,
-                                                                             int out_dtype, int rows_per_block, int nwaves) {
+                                                                             int out_dtype, int rows_per_block, int nwaves, uint32_t inverse) {
   constexpr bool F16 = __is_same(T, half_t);
   static_assert(MT == 1 || (F16 && MT == 2), "two activation rows: fp16 only");
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(1024) void gemv_w4a16_ring_kernel(const T* __restri
     gsel[it] = (cc[it] << 5) >> group_shift;
     voff_w[it] = addr::ring_w_voff(lane, it, chunks);
   }
-  const int my_rows = addr::ring_my_rows(r1 - r0, wave, nwaves);
+  const int my_rows = addr::ring_my_rows(r1 - r0, wave, nwaves, inverse);
   auto issue = [&](int i, int slot) {  // the wavefront's i-th row into ring slot `slot`
     const uint8_t* const base = uniform_ptr(Wp + (int64_t)(r0 + wave + i * nwaves) * row_bytes);
 #pragma unroll
@@ -1075,7 +1075,7 @@ static int launch_gemv_ring(const void* A, const void* Wp, const void* scales, c
     attr_set = true;
   }
   kern<<<p.blocks, 64 * p.waves, p.lds_bytes, st>>>((const T*)A, (const uint8_t*)Wp, (const T*)scales, (const T*)zeros, C, N, K,
-                                                  group_shift, zero_scalar, out_dtype, p.rows_per_block, p.waves);
+                                                  group_shift, zero_scalar, out_dtype, p.rows_per_block, p.waves, addr::ring_inverse(p.waves));
   return check_launch("tlq_gemm_w4a16(gemv)", LAYOUT == 1 ? "gemv_w4a16_ring_kernel, interleaved words" : "gemv_w4a16_ring_kernel") ? 0 : 1;
 }
 
