@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace tlq {
 namespace addr {
 
@@ -131,8 +133,53 @@ __host__ __device__ inline void slots_schedule(int KT, Ops& ops) {
   }
 }
 
-// ---- ring kernel (gemm_ring.h): slots of one stage of both operand tiles in the CU's 160 KB of LDS ----
-constexpr int ring_slots(int slot_bytes) { return 160 * 1024 / slot_bytes; }
+// ---- ring kernel (gemm_ring.h): stage s of both operand tiles lives in slot s % 4 ----
+constexpr int kRingSlots = 4;
+// How many stages the loads are ahead of the products.  What a work-group asks for before its first product it also waits for, until the address unit
+// has taken it: with the whole of LDS ahead (5 - 10 stages) 64 x 64 tiles took 1.34 x as long on 7 - 16 stages, 1.03 x beyond 96, 128 x 128 tiles 1.1 x
+// and 1.01 x.  Three stages against four: 4 - 16 stages 3 - 4 % less time, 17 - 24 level, 48 - 96 8 % more.
+__host__ __device__ inline int ring_ahead(int stages) { return stages <= 16 ? 3 : 4; }
+// The order in which one wavefront issues loads, waits, passes barriers, reads fragments and multiplies, with loads D stages ahead; the kernel and the
+// host-side checker both run this function.  issue(s): the loads of stage s.  wait(n): all but those of its youngest n stages have landed, and its own
+// fragment reads are done (n: an integral_constant in the main loop).  read(): the fragments of stage 0.  stage(parity, reads, loads, s): the products of
+// stage s, among them the reads of the fragments of stage s + 1 and the loads of stage s + D where the tags say so.
+template <int D, class Issue, class Wait, class Barrier, class Read, class Stage>
+__host__ __device__ __forceinline__ void ring_schedule(int KT, const Issue& issue, const Wait& wait, const Barrier& barrier, const Read& read, const Stage& stage) {
+  static_assert(D >= 3 && D <= kRingSlots, "two stages in flight behind the one that is read");
+  typedef std::true_type Yes;
+  typedef std::false_type No;
+  typedef std::integral_constant<int, 0> Even;
+  typedef std::integral_constant<int, 1> Odd;
+  for (int s = 0; s < D && s < KT; ++s) issue(s);
+  wait((KT < D ? KT : D) - 1);
+  barrier();
+  read();
+  int s = 0;
+  auto step = [&](auto parity) {  // s + D < KT
+    wait(std::integral_constant<int, D - 2>{});
+    barrier();
+    stage(parity, Yes{}, Yes{}, s);
+    ++s;
+  };
+  auto last_steps = [&](auto parity) {
+    const int left = KT - s - 2;  // stages behind s + 1
+    wait(left > 0 ? left : 0);
+    barrier();
+    if (s + 1 < KT)
+      stage(parity, Yes{}, No{}, s);
+    else
+      stage(parity, No{}, No{}, s);
+    ++s;
+  };
+  while (s + 1 + D < KT) {
+    step(Even{});
+    step(Odd{});
+  }
+  while (s < KT) {
+    if (s + D < KT) step(Even{}); else last_steps(Even{});
+    if (s < KT) last_steps(Odd{});
+  }
+}
 
 // ---- streaming W4A16 kernel for small and middle M (gemm_w4a16_stream.hip) ---------------------------------------
 // One step is 128 values of K.  A work-group of 8 wavefronts owns 256 or 128 weight rows and 16 * TM activation rows.

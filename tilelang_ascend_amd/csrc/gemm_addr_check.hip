@@ -270,6 +270,57 @@ struct SlotsSim {
   }
 };
 
+// One wavefront of the ring kernel running addr::ring_schedule on `stages` whole stages; `extra` loads more than the kernel's own are left in flight
+// by every wait.
+template <int D>
+int check_ring_schedule(int stages, int loads_per_stage, int extra) {
+  constexpr int S = addr::kRingSlots;
+  std::vector<int> in_flight;                     // stage of each load not known to have landed, oldest first
+  int owner[S], asked = 0, multiplied = 0, fragments = -1;
+  bool landed[S], published[S];
+  std::vector<char> read(stages, 0);              // 1 = asked for, 2 = in registers, 3 = a barrier has passed since: everyone's
+  char msg[160] = "";
+  for (int i = 0; i < S; ++i) owner[i] = -1, landed[i] = published[i] = false;
+  auto fail = [&](const char* what, int s) { if (!msg[0]) snprintf(msg, sizeof(msg), "ring schedule: %s (stage %d of %d)", what, s, stages); };
+  auto issue = [&](int s) {
+    const int slot = s % S;
+    if (s != asked++) fail("stages asked for out of order", s);
+    if (owner[slot] >= 0 && read[owner[slot]] != 3) fail("a load overwrites a stage that someone may still read", owner[slot]);
+    owner[slot] = s, landed[slot] = published[slot] = false;
+    for (int i = 0; i < loads_per_stage; ++i) in_flight.push_back(s);
+  };
+  auto fetch = [&](int s) {
+    if (owner[s % S] != s) fail("the slot of a stage that is read holds another one", s);
+    else if (!published[s % S]) fail("a stage is read before its loads were waited for and published by a barrier", s);
+    read[s] = 1, fragments = s;
+  };
+  auto wait = [&](int n) {
+    while ((int)in_flight.size() > n * loads_per_stage + extra) {
+      const int s = in_flight.front();
+      in_flight.erase(in_flight.begin());
+      bool more = false;
+      for (int u : in_flight) more |= u == s;
+      if (!more) landed[s % S] = true;
+    }
+    for (char& r : read) r = r == 1 ? 2 : r;
+  };
+  auto barrier = [&] {
+    for (int i = 0; i < S; ++i) published[i] = landed[i];
+    for (char& r : read) r = r == 2 ? 3 : r;
+  };
+  addr::ring_schedule<D>(
+      stages, issue, wait, barrier, [&] { fetch(0); },
+      [&](auto parity, auto reads, auto loads, int s) {
+        if (s != multiplied++ || s % 2 != decltype(parity)::value || fragments != s || read[s] != 3) fail("a stage is multiplied out of turn", s);
+        if (s == 0 && asked > 4) fail("more than four stages asked for ahead of the first product", asked);
+        if (decltype(reads)::value) fetch(s + 1);
+        if (decltype(loads)::value) issue(s + D);
+      });
+  if (multiplied != stages || asked != stages) fail("a stage was left out", multiplied);
+  CHECK_OR_FAIL(!msg[0], "%s", msg);
+  return 0;
+}
+
 // The streaming kernel's scales: every load of every window of K slices of `slice_steps` steps, for the first and last blocks of weight rows, and
 // what the reads of the scale area then find.  `shift`: values by which the tensors lie behind a 16-byte boundary.
 int check_stream_scales(int64_t N, int64_t K, int64_t group, int kgs, int slice_steps, int shift) {
@@ -1488,6 +1539,14 @@ int tlq_debug_check_slots_schedule(int stages, int loads_per_tile) {
     return 1;
   }
   return 0;
+}
+
+int tlq_debug_check_ring_schedule(int stages, int loads_per_stage, int extra_in_flight) {
+  if (stages < 1 || loads_per_stage < 1) {
+    set_error("tlq_debug_check_ring_schedule: bad arguments");
+    return 1;
+  }
+  return addr::ring_ahead(stages) == 3 ? check_ring_schedule<3>(stages, loads_per_stage, extra_in_flight) : check_ring_schedule<4>(stages, loads_per_stage, extra_in_flight);
 }
 
 int tlq_debug_check_gemv_ring_addressing(int64_t M, int64_t N, int64_t K, int64_t group, int rows_per_block, int waves, int depth) {

@@ -2,19 +2,19 @@
 //
 // What bounds such a launch is what a CU takes in: a 128 x 128 tile pulls 32 KB per 128-byte stage of K, and a work-group with one stage
 // in flight gets 55 KB per us, with two or more 90 - 97 (direct loads alone, 256 work-groups, row pitches of 4 - 16 KB; one stage of
-// 256 rows on either side: 66 - 71).  So the CU's LDS is a ring of S stages: while stage s is multiplied, s + 1 has landed and
-// s + 2 .. s + S are on their way, and the waits count loads instead of draining them.
+// 256 rows on either side: 66 - 71).  So LDS is a ring of four stages: while stage s is multiplied, s + 1 has landed and s + 2 .. s + 3 or s + 4
+// (addr::ring_ahead) are on their way, and the waits count loads instead of draining them.
 //   * Two groups of four wavefronts (2 x 2 over the tile) take one MFMA k-step of every stage each, so that every SIMD has two wavefronts and a
 //     fragment that is read from LDS still feeds a tile of half the work-group's rows and columns; the groups' sums meet in LDS at the end.
 //   * The fragments of stage s + 1 are read into a second register set while stage s is multiplied.  A slot is therefore free one
-//     barrier after its stage was read: the barrier at the top of iteration s frees the slot of stage s for stage s + S.
+//     barrier after its stage was read: the barrier at the top of iteration s frees the slot of stage s for stage s + 4.
 //   * One barrier per stage: behind it every wavefront's loads of stage s + 1 have landed, and everyone has read stage s.
 //   * The loads and the fragment reads of a stage stand between its products.  Issued together behind the barrier, the loads of eight
 //     wavefronts hold the issue of all of them until the address unit has taken the last one: 989 cycles a stage instead of 706 of
-//     which the products are 523 (128 x 128 tiles, fp16, by the shader's clock).
-// fp16 1000 x 4096 x 4096: 39.5 us with the groups on parts of K in two stages each, which drained the loads in every stage; 37.6 with the ring, 34.1 with
-// the loads between the products.  512 x 4096 x 4096 (64 x 128 tiles) 31.0, 23.8, 23.3; int8 [N, K] 1000 x 4096 x 4096 23.2, 21.6, 19.4.  What is left is
-// power: with the loads between the products the part runs at 1.50 GHz, without the loads at 1.83, without the fragment reads at 1.62,
+//     which the products are 523 (128 x 128 tiles, fp16, by the shader's clock).  No more is asked for ahead of the first product than the lead.
+// fp16 1000 x 4096 x 4096: 39.5 us with the groups on parts of K in two stages each, which drained the loads in every stage; 37.6 with the ring, 33.6 with
+// the loads between the products, 32.9 with a lead of four stages for five.  Over that earlier kernel, the better tile of either, 615 problems: 1.04 x on 4 - 6 stages,
+// 1.06 - 1.09 on 7 - 16, 1.17 on 17 - 24, 1.22 beyond.  What is left is power: with the loads between the products the part runs at 1.50 GHz, without the loads at 1.83, without the fragment reads at 1.62,
 // the products alone at 1.97 (60, 46, 52 and 38 us of a 64 us call).
 #pragma once
 #include "gemm_core.h"
@@ -60,10 +60,10 @@ __device__ __forceinline__ void add_groups_and_write(const Epi& epi, acc_t (&acc
 template <int BM, int BN>
 struct RingCfg {
   static constexpr int SLOT = (BM + BN) * kStageBytes;
-  static constexpr int S = addr::ring_slots(SLOT);
+  static constexpr int S = addr::kRingSlots;
   static constexpr int LDS = S * SLOT;
   static constexpr int TM = BM / 32, TN = BN / 32;  // MFMA tiles of a wavefront: 2 x 2 wavefronts in either group
-  static_assert(S >= 3, "two stages in flight behind the one that is read");
+  static_assert(S == 4 && LDS <= 160 * 1024, "slot of stage s: s % 4");
   static_assert(4 * TM * TN * 1024 <= LDS && 8 * (TM / 2) * 16 * kStageBytes <= LDS, "the groups' sums and the staging areas fit the ring");
 };
 
@@ -149,55 +149,31 @@ __global__ __launch_bounds__(512, 2) void ring_gemm_mfma_kernel(typename AL::Par
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  typedef std::true_type Yes;
+  typedef std::integral_constant<int, 0> Even;
   typedef std::false_type No;
-  // all but the youngest `stages` stages of loads have landed, and this wavefront's fragment reads are done
-  auto wait_but = [&](int stages) {
-    switch (stages) {
+  auto wait_but = [&](auto stages) {
+    if constexpr (std::is_same<decltype(stages), int>::value) {
+      switch (stages) {
 #define TLQ_WAIT(n) \
   case n: asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS * (n)) : "memory"); break;
-      TLQ_WAIT(1) TLQ_WAIT(2) TLQ_WAIT(3) TLQ_WAIT(4) TLQ_WAIT(5) TLQ_WAIT(6) TLQ_WAIT(7) TLQ_WAIT(8) TLQ_WAIT(9)
+        TLQ_WAIT(1) TLQ_WAIT(2) TLQ_WAIT(3)
 #undef TLQ_WAIT
-      default: asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        default: asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      }
+    } else {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS * decltype(stages)::value) : "memory");
     }
   };
-  static_assert(S <= 11, "the waits by name");
-  typedef std::integral_constant<int, 0> Even;
-  typedef std::integral_constant<int, 1> Odd;
-
-  for (int s = 0; s < S && s < KT; ++s) issue(s, s);
-  wait_but((KT < S ? KT : S) - 1);
-  __syncthreads();
-  read(Even{}, 0);
-  int s = 0, slot = 0;  // slot of stage s
-  auto next_of = [&](int x) { return x + 1 == S ? 0 : x + 1; };
-  auto step = [&](auto par) {  // s + S < KT
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS * (S - 2)) : "memory");
-    __syncthreads();
-    const int free_slot = slot;
-    slot = next_of(slot);
-    run_stage(par, Yes{}, Yes{}, slot, s + S, free_slot);
-    ++s;
+  auto run = [&](auto ahead_tag) {
+    constexpr int D = decltype(ahead_tag)::value;
+    addr::ring_schedule<D>(
+        KT, [&](int s) { issue(s, s); }, wait_but, [] { __syncthreads(); }, [&] { read(Even{}, 0); },
+        [&](auto parity, auto reads, auto loads, int s) { run_stage(parity, reads, loads, (s + 1) & (S - 1), s + D, (s + D) & (S - 1)); });
   };
-  auto last_steps = [&](auto par) {
-    const int left = KT - s - 2;  // stages behind s + 1
-    wait_but(left > 0 ? left : 0);
-    __syncthreads();
-    slot = next_of(slot);
-    if (s + 1 < KT)
-      run_stage(par, Yes{}, No{}, slot, 0, 0);
-    else
-      run_stage(par, No{}, No{}, 0, 0, 0);
-    ++s;
-  };
-  while (s + 1 + S < KT) {
-    step(Even{});
-    step(Odd{});
-  }
-  while (s < KT) {
-    if (s + S < KT) step(Even{}); else last_steps(Even{});
-    if (s < KT) last_steps(Odd{});
-  }
+  if (addr::ring_ahead(KT) == 3)
+    run(std::integral_constant<int, 3>{});
+  else
+    run(std::integral_constant<int, 4>{});
   if (band_and_tail & 1) {  // the partial stage, with zeros past K: through registers into slot 0 (every load has landed, every fragment is read)
     __syncthreads();
     al.template gload<true>(ra, KT, smem);
