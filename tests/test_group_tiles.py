@@ -1,5 +1,4 @@
-"""K over groups of wavefronts in the 128-row tiles (gemm_mfma_kernel with KG > 1): every tile, both weight layouts, uneven parts of K, a partial
-last stage, ragged rows and columns, batches, every epilogue -- integers bit for bit, 16-bit results against fp64; the estimate's choice."""
+"""The ring kernel (csrc/gemm_ring.h) in the place of 128-row tiles: every tile, both weight layouts, even and odd stages of K, a partial last stage, ragged rows and columns, batches, every epilogue -- integers bit for bit, 16-bit results against fp64; the estimate's choice."""
 import pytest
 import torch
 
@@ -116,3 +115,28 @@ def test_rows_of_full_rounds_and_the_rest(lib, M, N, K, launches):
             count(lib.tlq_gemm_w8a8(P(A), P(W), None if scale is None else P(scale), P(sb), P(out), 1, M, N, K, N, _abi.B_NK, CODE[dt], st))
             want = ((acc.float() if scale is None else acc.float() * scale[:, None]) * sb).to(dt)
             assert_bit_equal(out.cpu(), want.cpu(), f"rescaled {dt}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op,B,M,N,K,kernel", [
+    ("w8a8 NK", 1, 180, 1456, 512, "gemm_small_kernel"), ("w8a8 NK", 1, 226, 1232, 512, "gemm_small_kernel"),
+    ("f16 KN", 2, 77, 3312, 512, "ring_gemm"), ("f16 KN", 4, 215, 896, 512, "ring_gemm"), ("f16 KN", 4, 210, 720, 640, "ring_gemm")])
+def test_small_tiles_or_the_ring_kernel_on_short_rows(op, B, M, N, K, kernel):
+    """Problems where one of the two is ahead by 15 to 40 % and the choice had it the other way round when it compared the small tiles with another kernel."""
+    lib, P, st = _abi.load(), _abi.ptr, torch.cuda.current_stream().cuda_stream
+    if lib.tlq_device_cu_count() != 256:
+        pytest.skip("the estimates are of 256 compute units")
+    lay = _abi.B_KN if op.endswith("KN") else _abi.B_NK
+    print(f"choice {op} B={B} M={M} N={N} K={K}", flush=True)
+    lib.tlq_debug_launch_log(1)
+    if op.startswith("f16"):
+        A, W, C = torch.zeros(B, M, K, dtype=torch.float16, device="cuda"), torch.zeros(B, K, N, dtype=torch.float16, device="cuda"), torch.empty(B, M, N, dtype=torch.float16, device="cuda")
+        rc = lib.tlq_gemm_f16_batched(P(A), P(W), P(C), B, M, N, K, _abi.F16, _abi.F16, lay, st)
+    else:
+        A, W, C = torch.zeros(B, M, K, dtype=torch.int8, device="cuda"), torch.zeros(B, K, N, dtype=torch.int8, device="cuda"), torch.empty(B, M, N, dtype=torch.bfloat16, device="cuda")
+        sa, sb = torch.ones(B, M, device="cuda"), torch.ones(N, device="cuda")
+        rc = lib.tlq_gemm_w8a8(P(A), P(W), P(sa), P(sb), P(C), B, M, N, K, N, lay, _abi.BF16, st)
+    log = lib.tlq_debug_launch_log_text().decode()
+    lib.tlq_debug_launch_log(0)
+    _abi.check(rc)
+    assert kernel in log, log

@@ -1408,26 +1408,29 @@ static SmallUse w4a8_use(bool two_steps, int sign_mode, int64_t K) {
 // Is the small-tile kernel ahead of what would run in its place?  Two things its own estimate leaves out come on top: the activations' trip from
 // memory (at 2.5 TB/s: every tile of weight rows asks for them again) and, with 16-bit weights, that theirs cannot take less than
 // a copy.  The other side, by what would run: calls that cut K into slices over work-groups (sliced_us), up to 32 rows a fit to the 32-row
-// tiles, else the tiles' own estimates -- plain, of the ring kernel, 256 x 256 --, for W4A8 in two steps behind the
-// unpack pass.  The bars are fitted to problems (M 1 .. 8192, N 64 .. 14400, K 128 .. 14336, one to eight batches) timed with the
-// small-tile kernel, without it and by the choice.  On 9000 others, 1500 per use, it is taken on 5206, ahead by 1.40 - 1.80 x on average
-// and more than 5 % behind on 135 (81 by more than 10 %); the choice is 0.4 - 1.6 % behind the faster of both on average.  (The rule
-// before, without the two additions and with bars of 0.88 - 1.15 of a fit to the plain tiles: 428 of 4693, 2 - 8 % --
-// 8 x 1009 x 160 x 3456 int8 35.8 us against 15.0, W4A8 1374 x 1184 x 5376 47.8 against 28.1.)
+// tiles, else the tiles' own estimates -- plain, of the ring kernel, 256 x 256 --, for W4A8 in two steps behind the unpack pass.
+//   * The ring kernel, one round of its tiles: what the small-tile kernel takes is fitted anew (330 - 520 problems per use, those weighted where the two
+//     are within 1.7 x); the choice is 0.7 - 1.1 % behind the faster of the two on average, more than 5 % on 15 - 31 of them (with bars of 0.88 - 1.2 on its own
+//     estimate 2 - 4 % and 23 - 97).  Behind the unpack pass, and W4A8 by itself, as before.
+//   * Short rows, up to 32 rows and slices keep bars that were fitted to kernels which are still those that run there; on 190 of those problems 1 % behind.
+//   * In more than one round the small-tile kernel is hardly ever ahead (3 of 242 problems) nor taken (3).
 struct SmallBars {
-  double few_sliced, sliced, few, plain, groups;
+  double few_sliced, sliced, few, plain;
+  // against the ring kernel: what the small-tile kernel takes, launch + scale x its estimate + trip x the activations' trip + step x stages + out x
+  // millions of outputs + weights x millions of weights
+  double launch, scale, trip, step, out, weights;
 };
 static constexpr SmallBars kSmallBars[9] = {
-    // <= 32 rows, K slices   K slices   <= 32 rows   tiles   tiles with K in groups
-    {0.84, 1.5, 1.15, 1.03, 0.92},  // int8 [N, K]
-    {0.74, 1.05, 1.05, 1.0, 1.0},   // int8 [K, N]
-    {0.8, 1.04, 1.02, 1.0, 1.0},    // 16-bit [K, N]
-    {1.04, 1.0, 0.93, 0.93, 0.93},  // W4A8
-    {1.04, 1.0, 0.93, 1.0, 1.0},    // W4A8 in two steps
-    {0.84, 0.95, 1.12, 0.9, 0.88},  // W8A8 [N, K]
-    {0.74, 0.9, 1.0, 0.88, 0.92},   // W8A8 [K, N]
-    {1.04, 1.0, 0.93, 0.93, 0.93},  // W4A8 times 16
-    {1.04, 1.0, 0.93, 1.0, 1.0}};   // the same in two steps
+    // <= 32 rows, K slices   K slices   <= 32 rows   tiles   the ring kernel
+    {0.84, 1.5, 1.15, 1.03, -1.54, 0.922, 1.03, 0.040, 0.0, 0.0},  // int8 [N, K]
+    {0.74, 1.05, 1.05, 1.0, -0.67, 0.815, 0.09, 0.102, 0.0, 0.0},  // int8 [K, N]
+    {0.8, 1.04, 1.02, 1.0, 0.55, 0.577, 0.0, 0.071, 1.5, 0.296},    // 16-bit [K, N]
+    {1.04, 1.0, 0.93, 0.93, 0.0, 1.08, 1.08, 0.0, 0.0, 0.0},       // W4A8
+    {1.04, 1.0, 0.93, 1.0, 0.0, 1.0, 1.0, 0.0, 0.0, 0.0},          // W4A8 in two steps
+    {0.84, 0.95, 1.12, 0.9, -1.53, 1.026, 1.0, 0.025, 0.0, 0.0},   // W8A8 [N, K]
+    {0.74, 0.9, 1.0, 0.88, -0.52, 0.868, 0.36, 0.093, 0.0, 0.0},   // W8A8 [K, N]
+    {1.04, 1.0, 0.93, 0.93, 0.0, 1.08, 1.08, 0.0, 0.0, 0.0},       // W4A8 times 16
+    {1.04, 1.0, 0.93, 1.0, 0.0, 1.0, 1.0, 0.0, 0.0, 0.0}};         // the same in two steps
 static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int64_t M, int64_t N, int64_t K) {
   if (!t.ok || small_tile_forced()) return t.ok;
   const SmallW w = small_weights(use);
@@ -1435,7 +1438,8 @@ static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int
   const double g = (double)batch * (double)M * (double)N * (double)K * 1e-9, g32 = (double)batch * (double)ceil_div(M, (int64_t)32) * 32.0 * (double)N * (double)K * 1e-9;
   const double nk = (double)batch * (double)N * (double)K * 1e-6, mn = (double)batch * (double)M * (double)N * 1e-6, k = (double)K * 1e-3;
   const int64_t k_bytes = w == kSmallKN16 ? 2 * K : K, stages = ceil_div(k_bytes, (int64_t)kStageBytes);
-  double us = t.us + (double)batch * (double)M * (double)k_bytes / 2.5e6;
+  const double trip_us = (double)batch * (double)M * (double)k_bytes / 2.5e6;
+  double us = t.us + trip_us;
   if (w == kSmallKN16 && us < 1.05 * nk * 2.0 / 5.0) us = 1.05 * nk * 2.0 / 5.0;
   const bool packed = w == kSmallW4;
   const TileKind tile = w == kSmallKN16 ? kTileF16KN : w == kSmallKN8 ? kTileI8KN : kTileI8NK;
@@ -1452,9 +1456,11 @@ static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int
     return us < bar.sliced * (unpack_us + 2.0 * sliced_us(0, 1, M, N, K));  // (slices that add into the result take twice those with matrices of their own)
   if (!prefer_small_tiles(batch, M, N)) return us < bar.plain * (unpack_us + tile_us(tile, 6, batch, M, N, stages));
   double tiles_us = 0.0;
-  const bool groups = group_tile(tile, batch, M, N, k_bytes, &tiles_us) != 0;
-  if (groups && us < 5.6 && us < 1.1 * (unpack_us + tiles_us)) return true;  // (no more than a launch: nothing to lose)
-  return us < (groups ? bar.groups : bar.plain) * (unpack_us + tiles_us);
+  if (group_tile(tile, batch, M, N, k_bytes, &tiles_us) != 0) {
+    const double mine = bar.launch + bar.scale * t.us + bar.trip * trip_us + bar.step * (double)stages + bar.out * mn + bar.weights * nk;
+    return mine < unpack_us + tiles_us;
+  }
+  return us < bar.plain * (unpack_us + tiles_us);
 }
 static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t K, SmallUse use) {
   const SmallTile t{false, 0, 0, 0, 0.0};

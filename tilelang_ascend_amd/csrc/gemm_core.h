@@ -1013,18 +1013,17 @@ static constexpr TileCost kTileCost[4][2] = {
     {{2.0, 3.4, 1.23, 0.72}, {0.0, 7.3, 1.32, 0}},
     {{0.3, 6.2, 1.02, 0.60}, {0.0, 8.8, 1.13, 0}}};
 // Ring kernel, per round: fixed + stages x (step + shared x the part of the CUs that have a work-group): what the work-groups take from
-// each other, of memory and of the clock, grows with their number.  Fitted to 220 problems per kind (M 33 .. 3000, N 256 .. 14400, 512 ..
-// 28000 bytes of K), every variant that runs in one round forced on each: 7 - 11 % rms; the variant it picks is 2 - 2.6 % behind the best on
-// average.
+// each other, of memory and of the clock, grows with their number.  Fitted to 300 - 700 problems per entry (M 33 .. 3500, N 256 .. 14000, 512 .. 28000 bytes of K,
+// one to eight batches), every variant that runs in one round forced on each: 8 - 13 % rms; the variant it picks is 0.7 - 1.6 % behind the best on average.
 struct RingCost {
   double fixed, step, shared;
 };
 static constexpr RingCost kRingCost[4][4] = {
     // 128 x 128           128 x 64              64 x 128              64 x 64
-    {{5.26, 0.306, 0.276}, {4.78, 0.219, 0.173}, {4.34, 0.254, 0.164}, {4.89, 0.182, 0.093}},
-    {{5.07, 0.283, 0.262}, {4.70, 0.193, 0.158}, {4.17, 0.224, 0.160}, {4.81, 0.146, 0.097}},
-    {{5.94, 0.365, 0.276}, {5.83, 0.291, 0.211}, {5.14, 0.313, 0.167}, {5.28, 0.258, 0.116}},
-    {{6.08, 0.287, 0.261}, {6.18, 0.193, 0.171}, {5.10, 0.225, 0.164}, {5.50, 0.147, 0.107}}};
+    {{4.74, 0.313, 0.201}, {4.01, 0.217, 0.171}, {3.79, 0.246, 0.135}, {3.73, 0.174, 0.076}},
+    {{4.56, 0.288, 0.201}, {4.07, 0.195, 0.124}, {3.71, 0.212, 0.157}, {3.72, 0.146, 0.075}},
+    {{4.73, 0.362, 0.239}, {4.33, 0.287, 0.168}, {3.71, 0.314, 0.123}, {3.65, 0.243, 0.105}},
+    {{4.98, 0.281, 0.218}, {4.28, 0.189, 0.151}, {3.92, 0.206, 0.178}, {3.76, 0.140, 0.094}}};
 // ---- 256 x 256 tiles on four wavefronts (gemm_quad.h) ----
 extern thread_local int g_gemm_slots;  // tlq_tune_gemm_slots: 0 = the two-stage kernel alone, 1 = automatic, 2 = five slots, 3 = four wavefronts, wherever either can run
 // In the place of the other kernels of 256 x 256 tiles from so many stages on: 16-bit 17 in one round of tiles, 9 in two, 6 from three on, int8
@@ -1062,7 +1061,12 @@ inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int6
     const RingCost& c = kRingCost[kind][variant - kGroup128x128];
     const double in_round = blocks < cus ? (double)blocks / (double)cus : 1.0;
     const double us = (double)ceil_div(blocks, (int64_t)cus) * (c.fixed + (double)stages * (c.step + c.shared * in_round));
-    return us > floor_us ? us : floor_us;
+    // several tile rows read the weights again, from memory mostly where the order of tiles is not one by XCD
+    const int64_t tiles_m = ceil_div(M, (int64_t)(variant <= kGroup128x64 ? 128 : 64));
+    const double again = (blocks % 8 != 0 ? 0.9 : 0.3) * (double)((tiles_m < 4 ? tiles_m : 4) - 1);
+    const double trips = memory + again * (double)(batch * N) * (double)(stages * kStageBytes) / 4.8e6;
+    const double most = trips > product ? trips : product;
+    return us > most ? us : most;
   }
   if (variant == 6 && quad_takes(kind, batch, M, N, stages * kStageBytes)) {
     const QuadCost& c = kQuadCost[kind];
