@@ -19,14 +19,16 @@ extern "C" {
  * themselves use (no GPU needed; the reference has no counterpart, its tile addressing is generated by TVM).
  * tlq_debug_check_gemm_addressing walks every tile, thread, load instruction and stage of one operand:
  * source_kind 0 = row-major [rows, row_bytes] operand copied global -> LDS directly in tiles of `tile` rows by
- * `threads` threads; 1 = int8 [K = rows, N = row_bytes] weights in tiles of `tile` (128 | 256) columns; 2 = 16-bit
- * [K = rows, N = row_bytes (the number of columns)] weights in tiles of 128 | 256 columns (N a multiple of 8).  It
+ * `threads` threads; 1 = int8 [K = rows, N = row_bytes] weights in tiles of `tile` (128 | 256 | 64) columns; 2 = 16-bit
+ * [K = rows, N = row_bytes (the number of columns)] weights in tiles of 128 | 256 | 64 columns (N a multiple of 8; 64 for 512 threads).  It
  * checks global extents, LDS extents and coverage, agreement with the (transposing) operand-fragment reads and, for
  * kind 2, that no half-wavefront read meets a bank twice.
  * tlq_debug_check_slots_schedule simulates the five-slot kernel's issue / wait / barrier order over `stages` stages
  * with `loads_per_tile` load instructions per wavefront and tile (the kernel's waits assume 4).
  * tlq_debug_check_ring_schedule does so for the ring kernel's loads, waits, barriers, fragment reads and products over `stages` whole
  * stages; extra_in_flight is added to every wait's count of loads (0 = the kernel's own; more: to see it fail).
+ * tlq_debug_check_quad_schedule does so for the four-wavefront kernel over `tiles` tiles of a work-group, two stages or more each; extra_start is
+ * added to the wait ahead of the first tile, extra_stage to those of the stages.
  * All return 0 when everything holds, else 1 with tlq_last_error() naming the first violation. */
 /* Launch log of the calling thread: tlq_debug_launch_log(1) clears it and starts recording, (0) stops; while it records,
  * every kernel launch of this thread's calls appends "entry point [kernel and variant]" (a repeated entry once), joined
@@ -37,6 +39,7 @@ const char* tlq_debug_launch_log_text(void);
 int tlq_debug_check_gemm_addressing(int source_kind, int64_t rows, int64_t row_bytes, int tile, int threads);
 int tlq_debug_check_slots_schedule(int stages, int loads_per_tile);
 int tlq_debug_check_ring_schedule(int stages, int loads_per_stage, int extra_in_flight);
+int tlq_debug_check_quad_schedule(int stages, int tiles, int extra_start, int extra_stage);
 /* The same walk for the streaming W4A16 kernel (TLQ_ALGO_STREAM): packed weights [N, K / 2] and 2-byte activations [M, K]
  * with 16 * activation_tiles rows per work-group (2 | 4 | 8), and its ring of `ring_depth` steps for 1 .. 40 steps. */
 int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activation_tiles, int ring_depth);

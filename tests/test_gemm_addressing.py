@@ -77,6 +77,20 @@ def test_five_slot_schedule():
 
 
 
+@pytest.mark.parametrize("tile,threads", [(256, 256), (128, 512), (64, 512)])
+def test_operands_of_the_four_wavefront_and_ring_kernels(tile, threads):
+    lib = _abi.load()
+    for M, N, K in SHAPES_16:
+        for rows in (M, N):
+            _ok(lib.tlq_debug_check_gemm_addressing(0, rows, K * 2, tile, threads))
+    for _, M, N, K in W8A8:
+        _ok(lib.tlq_debug_check_gemm_addressing(0, M, K, tile, threads))
+        _ok(lib.tlq_debug_check_gemm_addressing(0, N, K, tile, threads))
+        _ok(lib.tlq_debug_check_gemm_addressing(1, K, N, tile, threads))
+    for K, N in ((64, 8), (64, 256), (128, 264), (256, 1000), (4096, 4096), (192, 40), (72, 264), (1, 8), (40, 72)):
+        _ok(lib.tlq_debug_check_gemm_addressing(2, K, N, tile, threads))
+
+
 @pytest.mark.parametrize("tm,depth", [(2, 5), (4, 4), (6, 3), (8, 3)])
 def test_streaming_kernel_addressing(tm, depth):
     """Streaming W4A16 kernel: every direct load stays inside the packed weights / the activations / the scale tensors (rows past the

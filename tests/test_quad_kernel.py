@@ -104,6 +104,20 @@ def test_in_a_graph():
         assert torch.equal(C, D)
 
 
+def test_schedule():
+    """Walked on the host over several tiles of a work-group: every stage is waited for and published before it is read, loads and outputs overwrite nothing
+    that someone may still read; one load more left in flight by any wait and the walk fails."""
+    lib = _abi.load()
+    for stages in (2, 3, 4, 5, 6, 7, 16, 33):
+        for tiles in (1, 2, 3, 7):
+            assert lib.tlq_debug_check_quad_schedule(stages, tiles, 0, 0) == 0, _abi.last_error()
+            assert lib.tlq_debug_check_quad_schedule(stages, tiles, 1, 0) != 0
+            assert "before its loads were waited for" in _abi.last_error()
+            if stages * tiles > 2:
+                assert lib.tlq_debug_check_quad_schedule(stages, tiles, 0, 1) != 0
+                assert "before its loads were waited for" in _abi.last_error()
+
+
 def code_object(tmp_path, source):
     obj, llvm = os.path.join(build.OBJ_DIR, source + ".o"), "/opt/rocm/llvm/bin"
     if not (os.path.exists(obj) and os.path.exists(f"{llvm}/clang-offload-bundler")):

@@ -65,6 +65,7 @@ SIGNATURES = {
     "tlq_debug_check_gemm_addressing": (_int, [_int, _i64, _i64, _int, _int]),
     "tlq_debug_check_slots_schedule": (_int, [_int, _int]),
     "tlq_debug_check_ring_schedule": (_int, [_int, _int, _int]),
+    "tlq_debug_check_quad_schedule": (_int, [_int, _int, _int, _int]),
     "tlq_debug_stream_plan": (_int, [_i64, _i64, _i64, _i64, _int, _vp]),
     "tlq_debug_check_stream_addressing": (_int, [_i64, _i64, _i64, _int, _int]),
     "tlq_debug_check_stream_schedule": (_int, [_int, _int, _int, _int, _int, _int, _int]),

@@ -3,8 +3,8 @@
 //   * every global byte read lies inside the operand matrix,
 //   * every direct load lands inside its LDS tile, every 16-byte cell of the tile is written exactly once, and holds
 //     the (row, K chunk) that the operand-fragment read of that cell expects,
-//   * the five-slot schedule never overwrites a tile that has not been multiplied and never multiplies a tile whose
-//     loads were not waited for.
+//   * the schedules of the five-slot, the ring and the four-wavefront kernel never overwrite what someone may still read and never
+//     multiply what was not waited for.
 // No GPU is needed: these run in the CPU-only test suite and can be called before a launch.
 #include <utility>
 #include <vector>
@@ -74,13 +74,14 @@ int check_row_direct(int64_t rows_total, int64_t k_bytes, int tile_rows, int thr
     for (int wave_row0 = 0; wave_row0 < tile_rows; wave_row0 += 16)
       for (int lane = 0; lane < 64; ++lane) {
         const uint32_t base = addr::rowfrag_base(lane, wave_row0);
-        for (int ks = 0; ks < 2; ++ks) {
-          const uint32_t off = addr::rowfrag_off(base, ks, 0);
-          CHECK_OR_FAIL(off + 16 <= (uint32_t)tile_rows * addr::kStage, "operand read at %u outside the tile", off);
-          const int want = (wave_row0 + (lane & 15)) * 8 + ks * 4 + (lane >> 4);
-          CHECK_OR_FAIL(cell[off / 16] == want, "operand read (row0 %d lane %d k-step %d) finds cell %d, expects %d", wave_row0, lane, ks,
-                        cell[off / 16], want);
-        }
+        for (int t = 0; t < 8 && wave_row0 + 16 * t < tile_rows; ++t)
+          for (int ks = 0; ks < 2; ++ks) {
+            const uint32_t off = addr::rowfrag_off(base, ks, t);
+            CHECK_OR_FAIL(off + 16 <= (uint32_t)tile_rows * addr::kStage, "operand read at %u outside the tile", off);
+            const int want = (wave_row0 + 16 * t + (lane & 15)) * 8 + ks * 4 + (lane >> 4);
+            CHECK_OR_FAIL(cell[off / 16] == want, "operand read (row0 %d lane %d t %d k-step %d) finds cell %d, expects %d", wave_row0, lane, t, ks,
+                          cell[off / 16], want);
+          }
       }
   }
   return 0;
@@ -129,8 +130,8 @@ int check_kn_direct(int64_t K, int64_t N, int threads) {
     for (size_t c = 0; c < cell.size(); ++c) CHECK_OR_FAIL(cell[c] >= 0, "[K,N] loader: LDS cell %zu never written", c);
     // transposing operand reads: lane (r16, q) of column block t supplies the row of k = 16 q + r16 / 2 (+ 8 for the second
     // read, + 64 for k-step 1) at columns 16 (wave_row0 / 16 + t) + 8 (r16 % 2)
-    for (int wave_row0 = 0; wave_row0 + 64 <= BN; wave_row0 += 64)
-      for (int t = 0; t < 4; ++t)
+    for (int wave_row0 = 0; wave_row0 < BN; wave_row0 += 32)
+      for (int t = 0; t < 8 && wave_row0 + 16 * t < BN; ++t)
         for (int lane = 0; lane < 64; ++lane)
           for (int ks = 0; ks < 2; ++ks)
             for (int h = 0; h < 2; ++h) {
@@ -187,13 +188,13 @@ int check_kn16_direct(int64_t K, int64_t N, int threads) {
           CHECK_OR_FAIL(cell[l / 16] == -1, "[K,N] 16-bit loader: LDS cell %u written twice", l / 16);
           const int pc = lane % (BN / 8);
           CHECK_OR_FAIL(l == (uint32_t)(k * RB + pc * 16), "[K,N] 16-bit loader: lane lands at %u, not on (k %d, chunk %d)", l, k, pc);
-          cell[l / 16] = k * (BN / 8) + (pc ^ addr::kn16_swz(k));  // the logical chunk (8 columns) this cell holds
+          cell[l / 16] = k * (BN / 8) + (pc ^ addr::kn16_swz_of<BN>(k));  // the logical chunk (8 columns) this cell holds
         }
     for (size_t c = 0; c < cell.size(); ++c) CHECK_OR_FAIL(cell[c] >= 0, "[K,N] 16-bit loader: LDS cell %zu never written", c);
     // operand reads: lane (i, q) of column block t supplies the row of k = 8 q + i / 4 (+ 4 for the second read, + 32 for
     // k-step 1) at columns wave_col0 + 16 t + 4 (i % 4) .. + 3
-    for (int wave_col0 = 0; wave_col0 + 64 <= BN; wave_col0 += 64)
-      for (int t = 0; t < 4; ++t)
+    for (int wave_col0 = 0; wave_col0 < BN; wave_col0 += 32)
+      for (int t = 0; t < 8 && wave_col0 + 16 * t < BN; ++t)
         for (int ks = 0; ks < 2; ++ks)
           for (int h = 0; h < 2; ++h) {
             int bank_use[2][64] = {};
@@ -317,6 +318,82 @@ int check_ring_schedule(int stages, int loads_per_stage, int extra) {
         if (decltype(loads)::value) issue(s + D);
       });
   if (multiplied != stages || asked != stages) fail("a stage was left out", multiplied);
+  CHECK_OR_FAIL(!msg[0], "%s", msg);
+  return 0;
+}
+
+// One wavefront of the four-wavefront kernel running addr::quad_start and, for every tile, addr::quad_tile and what the kernel does behind it.  `extra` loads
+// more than the kernel's own are left in flight by the wait ahead of the first tile (extra_start) and by those of the stages (extra_stage).
+int check_quad_schedule(int stages, int tiles, int extra_start, int extra_stage) {
+  const int total = stages * tiles;
+  struct Held { int operand, stage, reads; bool landed, published; };  // stage: of the whole walk; reads: k-steps read, 3 = by everyone
+  Held held[5];
+  int steps_asked[5] = {}, slot[5];
+  for (int i = 0; i < 5; ++i) held[i] = {-1, -1, 3, false, false}, slot[i] = i;
+  const int kStore = -1;
+  std::vector<std::pair<int, int>> in_flight;  // (slot or kStore, stage), oldest first
+  int loaded[2] = {0, 0}, multiplied[2] = {0, 0}, fragments[2] = {-1, -1}, tile = 0, nexts = 0;
+  bool fresh[5] = {};  // (reads that a wait has covered but no barrier yet)
+  char msg[160] = "";
+  auto fail = [&](const char* what, int s) { if (!msg[0]) snprintf(msg, sizeof(msg), "quad schedule: %s (stage %d of %d)", what, s, total); };
+  auto load = [&](int operand, int s, int to) {
+    const int g = loaded[operand]++;
+    if (s != g % stages) fail("stages asked for out of order", g);
+    if (held[to].reads != 3) fail("a load overwrites a slot that someone may still read", g);
+    if (g / stages > nexts && g / stages < tiles) fail("a stage of the next tile asked for by this tile's loader", g);
+    held[to] = {operand, g, 0, false, false}, steps_asked[to] = 0, fresh[to] = false;
+    for (int i = 0; i < addr::kQuadLoads; ++i) in_flight.push_back({to, g});
+  };
+  auto read = [&](int operand, int g, int from, int ks) {
+    if (g >= total) return;  // (behind the last tile, for nobody)
+    if (held[from].operand != operand || held[from].stage != g) fail("the slot of a stage that is read holds something else", g);
+    else if (!held[from].published) fail("a stage is read before its loads were waited for and published by a barrier", g);
+    steps_asked[from] |= 1 << ks;
+  };
+  bool in_start = true;
+  auto wait = [&](auto n) {
+    const size_t left = (size_t)(decltype(n)::value + (in_start ? extra_start : extra_stage));
+    while (in_flight.size() > left) {
+      const std::pair<int, int> e = in_flight.front();
+      in_flight.erase(in_flight.begin());
+      bool more = false;
+      for (const auto& o : in_flight) more |= o == e;
+      if (!more && e.first != kStore && held[e.first].stage == e.second) held[e.first].landed = true;
+    }
+    for (int i = 0; i < 5; ++i) fresh[i] = steps_asked[i] == 3;
+  };
+  auto barrier = [&] {
+    for (int i = 0; i < 5; ++i) {
+      held[i].published = held[i].landed;
+      if (fresh[i]) held[i].reads = 3;
+    }
+  };
+  addr::quad_start(
+      slot, [&](auto operand, int s, int to) { load(decltype(operand)::value, s, to); }, wait, barrier,
+      [&](int a, int w) { read(0, 0, a, 0), read(1, 0, w, 0), fragments[0] = 0; });
+  in_start = false;
+  for (; tile < tiles; ++tile) {
+    addr::quad_tile(
+        stages, slot, [&] { ++nexts; },
+        [&](auto ks_tag, auto first, int a, int w, int s, int to) {
+          constexpr int ks = decltype(ks_tag)::value;
+          const int g = multiplied[ks]++;
+          if (fragments[ks] != g || g != (ks ? multiplied[0] - 1 : multiplied[1])) fail("a k-step is multiplied out of turn", g);
+          if ((decltype(first)::value != 0) != (ks == 0 && g % stages == 0)) fail("the wrong product starts the sums", g);
+          load(ks, s, to);  // (ahead of the reads, the worst place between them)
+          read(0, g + ks, a, 1 - ks), read(1, g + ks, w, 1 - ks), fragments[1 - ks] = g + ks;
+        },
+        wait, barrier);
+    // the outputs go through the free slot and to memory
+    const int last = tile * stages + stages - 1;
+    if (held[slot[4]].reads != 3) fail("the outputs overwrite a slot that someone may still read", last);
+    for (int i = 0; i < 3; ++i) in_flight.push_back({kStore, last});
+    held[slot[4]] = {-1, -1, 0, false, false};
+    if (tile + 1 == tiles) break;
+    steps_asked[slot[4]] = 3, fresh[slot[4]] = true;  // (the kernel's wait for LDS alone)
+    barrier();
+  }
+  if (multiplied[0] != total || multiplied[1] != total || nexts != tiles) fail("a stage was left out", multiplied[1]);
   CHECK_OR_FAIL(!msg[0], "%s", msg);
   return 0;
 }
@@ -1415,13 +1492,15 @@ int tlq_debug_check_gemm_addressing(int source_kind, int64_t rows, int64_t row_b
   if (source_kind == 1) {
     if (tile == 256) return check_kn_direct<256>(rows, row_bytes, threads);
     if (tile == 128) return check_kn_direct<128>(rows, row_bytes, threads);
-    set_error("tlq_debug_check_gemm_addressing: [K,N] tiles are 128 or 256 columns wide (got %d)", tile);
+    if (tile == 64 && threads == 512) return check_kn_direct<64>(rows, row_bytes, threads);
+    set_error("tlq_debug_check_gemm_addressing: [K,N] tiles are 128 or 256 columns wide, 64 for 512 threads (got %d)", tile);
     return 1;
   }
   if (source_kind == 2) {
     if (tile == 256) return check_kn16_direct<256>(rows, row_bytes, threads);
     if (tile == 128) return check_kn16_direct<128>(rows, row_bytes, threads);
-    set_error("tlq_debug_check_gemm_addressing: 16-bit [K,N] tiles are 128 or 256 columns wide (got %d)", tile);
+    if (tile == 64 && threads == 512) return check_kn16_direct<64>(rows, row_bytes, threads);
+    set_error("tlq_debug_check_gemm_addressing: 16-bit [K,N] tiles are 128 or 256 columns wide, 64 for 512 threads (got %d)", tile);
     return 1;
   }
   set_error("tlq_debug_check_gemm_addressing: bad source kind %d", source_kind);
@@ -1547,6 +1626,14 @@ int tlq_debug_check_ring_schedule(int stages, int loads_per_stage, int extra_in_
     return 1;
   }
   return addr::ring_ahead(stages) == 3 ? check_ring_schedule<3>(stages, loads_per_stage, extra_in_flight) : check_ring_schedule<4>(stages, loads_per_stage, extra_in_flight);
+}
+
+int tlq_debug_check_quad_schedule(int stages, int tiles, int extra_start, int extra_stage) {
+  if (stages < 2 || tiles < 1 || extra_start < 0 || extra_stage < 0) {
+    set_error("tlq_debug_check_quad_schedule: bad arguments");
+    return 1;
+  }
+  return check_quad_schedule(stages, tiles, extra_start, extra_stage);
 }
 
 int tlq_debug_check_gemv_ring_addressing(int64_t M, int64_t N, int64_t K, int64_t group, int rows_per_block, int waves, int depth) {

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256, 1) void quad_gemm_mfma_kernel(typename RowLoad
                                                                int M, int N, int KT, int tiles, int grid, int band_rows) {
   constexpr int T = 8, TILE = 256 * kStageBytes;  // MFMA tiles of a wavefront per side; one operand, one stage: 32 KB
   typedef RowLoaderDirect<256, 256> AL;
-  static_assert(AL::PER_WAVE == 8 && WL::PER_WAVE == 8 && WL::DIRECT, "the waits below count eight direct loads per wavefront and tile");
+  static_assert(AL::PER_WAVE == addr::kQuadLoads && WL::PER_WAVE == addr::kQuadLoads && WL::DIRECT, "the waits count the direct loads per wavefront and tile");
   extern __shared__ __align__(16) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -67,16 +67,9 @@ __global__ __launch_bounds__(256, 1) void quad_gemm_mfma_kernel(typename RowLoad
   const typename WL::Frag fragW(lane, wave_n0);
   typename Mma::acc_t acc[T][T];
   uint4_t af[2][T], wf[2][T];  // fragments by k-step of a stage
-  // at the top of stage s: the slots of A(s), W(s), A(s + 1), W(s + 1), and the free one
-  uint8_t* slot[5];
+  uint8_t* slot[5];  // (addr::quad_tile)
 #pragma unroll
   for (int i = 0; i < 5; ++i) slot[i] = smem + i * TILE;
-  auto load_all = [&](const auto& loader, int s, uint8_t* to) {
-    const uint8_t* const src = loader.stage_src(s);
-    const uint32_t dst = loader.stage_dst(to);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) loader.load_one(j, src, dst);
-  };
   // The 64 products of k-step KS; between them the reads of the next k-step's fragments from (ra, rw) and the eight loads of stage s of an operand.
   auto phase = [&](auto ks_tag, auto first_tag, const uint8_t* ra, const uint8_t* rw, const auto& loader, int s, uint8_t* to) {
     constexpr int KS = decltype(ks_tag)::value, OTHER = 1 - KS;
@@ -105,52 +98,50 @@ __global__ __launch_bounds__(256, 1) void quad_gemm_mfma_kernel(typename RowLoad
       __builtin_amdgcn_sched_barrier(0);
     });
   };
-  typedef std::integral_constant<int, 0> K0;
-  typedef std::integral_constant<int, 1> K1;
+  auto wait = [&](auto left) { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(left)::value) : "memory"); };
+  auto barrier = [] { __syncthreads(); };
 
-  load_all(al, 0, slot[0]);
-  load_all(wl, 0, slot[1]);
-  load_all(al, 1, slot[2]);
-  load_all(wl, 1, slot[3]);
-  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-  __syncthreads();
-  wf[0][0] = fragW.read(slot[1], 0, 0);
+  addr::quad_start(
+      slot,
+      [&](auto operand, int s, uint8_t* to) {
+        auto all = [&](const auto& loader) {
+          const uint8_t* const src = loader.stage_src(s);
+          const uint32_t dst = loader.stage_dst(to);
 #pragma unroll
-  for (int t = 0; t < T; ++t) af[0][t] = fragA.read(slot[0], 0, t);
+          for (int j = 0; j < 8; ++j) loader.load_one(j, src, dst);
+        };
+        if constexpr (decltype(operand)::value == 0) all(al); else all(wl);
+      },
+      wait, barrier,
+      [&](const uint8_t* a, const uint8_t* w) {
+        wf[0][0] = fragW.read(w, 0, 0);
 #pragma unroll
-  for (int t = 1; t < T; ++t) wf[0][t] = fragW.read(slot[1], 0, t);
+        for (int t = 0; t < T; ++t) af[0][t] = fragA.read(a, 0, t);
+#pragma unroll
+        for (int t = 1; t < T; ++t) wf[0][t] = fragW.read(w, 0, t);
+      });
   for (;;) {
     const Epi epi(pe, tc.batch);
     const int m_base = tc.m0 + wave_m0, n_base = tc.n0 + wave_n0;
     auto out_scales = fetch_scales<Epi, T, T>(epi, m_base, n_base, lane, M, N);
     tile += grid;
     const bool more = tile < tiles;
-    // stage s: the loads ahead are those of stage s + 2, past the end the first two of the next tile (of this one again, for nobody, behind the last)
-    auto stage = [&](auto first_tag, int s) {
-      int ahead = s + 2;
-      if (ahead >= KT) {
-        ahead -= KT;
-        if (ahead == 0 && more) {
+    addr::quad_tile(
+        KT, slot,
+        [&] {  // (behind the last tile the loads are those of its first stages again, for nobody)
+          if (!more) return;
           tc = tile_of_index<256, 256>(tile, tiles, M, N, band_rows);
           al = AL(pa, tc.batch, tc.m0, M, tid);
           wl = WL(pw, tc.batch, tc.n0, N, tid);
-        }
-      }
-      phase(K0{}, first_tag, slot[0], slot[1], al, ahead, slot[4]);
-      // all but the loads of this phase have landed, and this wavefront has read all of stage s (the first time everything: stores of the tile
-      // before are among what is outstanding, and the count is one of loads in order)
-      if constexpr (decltype(first_tag)::value) {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        out_scales.arrive();  // (the scales are among it; waited for at their use, they would drain the next tile's loads)
-      } else
-        asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-      __syncthreads();
-      phase(K1{}, std::false_type{}, slot[2], slot[3], wl, ahead, slot[0]);
-      uint8_t *const a = slot[0], *const w = slot[1];
-      slot[0] = slot[2], slot[1] = slot[3], slot[2] = slot[4], slot[3] = a, slot[4] = w;
-    };
-    stage(std::true_type{}, 0);
-    for (int s = 1; s < KT; ++s) stage(std::false_type{}, s);
+        },
+        [&](auto ks, auto first, const uint8_t* ra, const uint8_t* rw, int s, uint8_t* to) {
+          if constexpr (decltype(ks)::value == 0) phase(ks, first, ra, rw, al, s, to); else phase(ks, first, ra, rw, wl, s, to);
+        },
+        [&](auto left) {
+          wait(left);
+          if constexpr (decltype(left)::value == 0) out_scales.arrive();  // (the scales are among it; waited for at their use, they would drain the next tile's loads)
+        },
+        barrier);
     // (the wait states between the last MFMAs, which the compiler does not know for what they are, and the first instruction that reads an accumulator)
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     // the free slot was read for the last time in front of the last barrier: the output staging area, 8 KB for each wavefront
