@@ -20,7 +20,7 @@ pytestmark = pytest.mark.skipif(shutil.which("hipcc") is None and not __import__
     ("gemm_w4a16.hip", ["gemm_mfma_kernel", "w4a16_skinny_kernel"]),
     ("gemm_w4a16_small.hip", ["w4a16_small_kernel"]),
     ("gemm_small.hip", ["gemm_small_kernel"]),
-    ("gemm_f16.hip", ["gemm_mfma_kernel"]),  # (among them, here and below, K over groups of wavefronts)
+    ("gemm_f16.hip", ["gemm_mfma_kernel"]),
     ("gemm_int8.hip", ["gemm_mfma_kernel"]),
 ])
 def test_no_register_spills(tmp_path, source, kernels):

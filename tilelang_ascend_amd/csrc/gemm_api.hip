@@ -177,7 +177,7 @@ extern "C" {
 
 void tlq_tune_gemm_groups(int variant) { tlq::tuning_changed(), tlq::g_gemm_groups = variant < 0 || variant > 5 ? 0 : variant; }
 void tlq_tune_gemm_band(int tile_rows) { tlq::g_gemm_band_rows = tile_rows < 0 ? 0 : tile_rows; }
-void tlq_tune_gemm_slots(int mode) { tlq::tuning_changed(), tlq::g_gemm_slots = mode < 0 ? 0 : (mode > 3 ? 2 : mode); }
+void tlq_tune_gemm_slots(int mode) { tlq::tuning_changed(), tlq::g_gemm_slots = mode < 0 ? 0 : (mode > 3 ? 3 : mode); }
 int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused) {
   return tlq::prefer_small_tiles(batch, M, N, fused ? 0.65 : 0.72) ? 128 : 256;
 }

@@ -11,7 +11,7 @@
 // wavefront) outstanding.  Everything else -- wave tiling, LDS tile layout, fragment reads, epilogue -- is the
 // two-stage kernel's.
 //
-// Selected by tlq_tune_gemm_slots(1); whole stages only (K bytes a multiple of 128).
+// Forced by tlq_tune_gemm_slots(2) (modes: gemm_core.h); whole stages only (K bytes a multiple of 128).
 #pragma once
 #include "gemm_core.h"
 
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(512, 2) void gemm_slots_kernel(typename RowLoaderDi
   write_tile_with<Epi, TM, TN>(epi, out_scales, acc, smem + wave * (TM * 16 * kStageBytes), lane, tc.m0 + wave_m0, tc.n0 + wave_n0, M, N);
 }
 
-// tlq_tune_gemm_slots: 0 = the two-stage kernel (default), 1 = this one where it applies
+// (modes: gemm_core.h)
 extern thread_local int g_gemm_slots;
 
 // k_bytes (bytes of K per activation row) a positive multiple of 128: whole stages only.

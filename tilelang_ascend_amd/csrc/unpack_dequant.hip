@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void unpack_int4_scalar(const uint8_t* __restr
 
 // ---- per-group dequantisation -----------------------------------------------------------
 // Rows are whole groups: word i of the matrix is in group i / (group / 8), where there were two divisions of 64 bits a word; and a wavefront takes two
-// words a lane, 64 apart, and is done, as in the quantiser (14336 x 4096 float16 with zero points in groups of 64 24.9 -> 23.1 us, 6.3 TB/s, 4096 x
+// words a lane, 64 apart, and is done, as in the quantiser (14336 x 4096 float16 with zero points in groups of 64 24.9 -> 23.1 us, 6.5 TB/s, 4096 x
 // 4096 bfloat16 9.6 -> 8.7).
 // One lane dequantises a 32-bit word (8 weights) with the expander the GEMM kernels use (bit-identical to the
 // element-wise Dequant<T>::apply, a third of its instructions); a zero point that is a small integer folds into
