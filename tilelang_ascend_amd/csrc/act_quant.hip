@@ -232,9 +232,11 @@ static void launch_rows(const T* X, int8_t* Y, float* S, int64_t M, int N, int r
 #define TLQ_AQ(CH) act_quant_rows_kernel<T, CH, WPR><<<blocks, 256, 0, st>>>(X, Y, S, M, N, round_scale, blocks)
   if (per_lane <= 1) TLQ_AQ(1);
   else if (per_lane <= 2) TLQ_AQ(2);
-  else if (per_lane <= 4) TLQ_AQ(4);
-  else if (per_lane <= 8) TLQ_AQ(8);
-  else TLQ_AQ(16);
+  else if (WPR == 1 || per_lane <= 4) TLQ_AQ(4);  // (one wavefront per row: at most 4, by its caller)
+  else if constexpr (WPR == 4) {
+    if (per_lane <= 8) TLQ_AQ(8);
+    else TLQ_AQ(16);
+  }
 #undef TLQ_AQ
 }
 
