@@ -12,7 +12,7 @@ from helpers import assert_bit_equal, gen
 
 pytestmark = pytest.mark.gpu
 
-HOOKS = [("slots", 0)]
+HOOKS = [("slots", 0), ("slots", 1)]  # the two-stage kernel; the automatic choice, which takes the four-wavefront kernel on long rows
 
 
 def _with_hook(name, value, fn):
