@@ -48,6 +48,8 @@ int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activ
 int tlq_debug_check_stream_schedule(int steps, int depth, int loads, int units, int wait_scales, int wait_first, int wait_step);
 /* Both orders of its work-groups: every block taken once; by XCD, hardly a slice on more XCDs than it needs. */
 int tlq_debug_check_stream_order(int64_t n_blocks, int64_t slices, int64_t m_blocks);
+/* The order of the GEMM kernels' work-groups by XCD: every place taken once, an XCD's places in a row. */
+int tlq_debug_check_xcd_order(int64_t total);
 /* The same walk for the panel kernel (TLQ_ALGO_PANEL) with K slices of `slice_steps` steps of 128 values: every direct load of
  * activations, packed weights and scale windows of every work-group, the LDS map and the operand reads; and the plan the
  * library would choose on a device with `cus` compute units: plan_out is a HOST array of four int64 that receives the tiles

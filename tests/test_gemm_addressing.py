@@ -134,6 +134,12 @@ def test_streaming_kernel_order(n_blocks):
             _ok(_abi.load().tlq_debug_check_stream_order(n_blocks, slices, m_blocks))
 
 
+def test_gemm_kernels_order_by_xcd():
+    """Work-group to place, for totals around multiples of eight and of a round of the machine."""
+    for total in [*range(1, 35), 254, 255, 256, 257, 263, 522, 1031]:
+        _ok(_abi.load().tlq_debug_check_xcd_order(total))
+
+
 @pytest.mark.parametrize("kind", [0, 1, 2, 3, 4])
 def test_small_tile_kernels_addressing_and_schedule(kind):
     """Both small-tile kernels: loads inside their matrices (rows past them clamped), operand reads on the cells that hold what they

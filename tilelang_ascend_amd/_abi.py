@@ -70,6 +70,7 @@ SIGNATURES = {
     "tlq_debug_check_stream_addressing": (_int, [_i64, _i64, _i64, _int, _int]),
     "tlq_debug_check_stream_schedule": (_int, [_int, _int, _int, _int, _int, _int, _int]),
     "tlq_debug_check_stream_order": (_int, [_i64, _i64, _i64]),
+    "tlq_debug_check_xcd_order": (_int, [_i64]),
     "tlq_debug_check_decode_addressing": (_int, [_i64, _i64, _i64, _i64, _int, _int, _int, _int]),
     "tlq_debug_decode_plan": (_int, [_i64, _i64, _i64, _i64, _int, _vp]),
     "tlq_debug_launch_log": (None, [_int]),

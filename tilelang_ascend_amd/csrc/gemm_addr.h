@@ -109,6 +109,13 @@ __host__ __device__ inline uint32_t kn16frag_off(int lane, int wave_col0, int t)
   return (uint32_t)(krow * 2 * BN) + (uint32_t)((chunk ^ kn16_swz_of<BN>(krow)) << 4) + (uint32_t)(8 * (i & 1));
 }
 
+// The place of work-group `id` of `total` in an order in which every XCD (ids are dealt round-robin to the eight of them) has a contiguous range, the
+// first total % 8 XCDs one more than the others.
+__host__ __device__ __forceinline__ int xcd_order(int id, int total) {
+  const int xcd = id & 7, more = total & 7;
+  return xcd * (total >> 3) + (xcd < more ? xcd : more) + (id >> 3);
+}
+
 // ---- five-slot schedule (gemm_slots.h): tile t = 2 * stage (+ 1 for the weights) lives in slot t % 5 ----
 constexpr int kSlots = 5;
 __host__ __device__ inline int slot_of_tile(int t) { return t % kSlots; }

@@ -1534,6 +1534,22 @@ int tlq_debug_check_stream_order(int64_t n_blocks, int64_t slices, int64_t m_blo
   return 0;
 }
 
+int tlq_debug_check_xcd_order(int64_t total) {
+  CHECK_OR_FAIL(total >= 1 && total <= 1 << 24, "order by XCD: bad arguments");
+  std::vector<uint8_t> taken(total, 0);
+  int64_t last[8];
+  for (int x = 0; x < 8; ++x) last[x] = -1;
+  for (int64_t id = 0; id < total; ++id) {
+    const int64_t at = tlq::addr::xcd_order((int)id, (int)total);
+    CHECK_OR_FAIL(at >= 0 && at < total && !taken[at], "order by XCD: work-group %lld of %lld takes place %lld", (long long)id, (long long)total, (long long)at);
+    taken[at] = 1;
+    int64_t& before = last[id & 7];
+    CHECK_OR_FAIL(before < 0 || at == before + 1, "order by XCD: work-group %lld of %lld leaves its XCD's range", (long long)id, (long long)total);
+    before = at;
+  }
+  return 0;
+}
+
 int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activation_tiles, int ring_depth) {
   if (int rc = check_stream(M, N, K, activation_tiles)) return rc;
   // (K slices as the plans cut them: whole groups, or a power-of-two part of one)
