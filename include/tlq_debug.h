@@ -123,6 +123,12 @@ void tlq_tune_gemv_ring(int on);                             /* 1 (default): a s
                                                               * ring kernel where it applies; 0: on the kernels it replaced (for one
                                                               * activation row the same results, bit for bit) */
 void tlq_tune_gemm_groups(int variant);                       /* the ring kernel in the place of 128-row tiles: 0 = automatic, 1 = never, 2 .. 5: its 128x128, 128x64, 64x128, 64x64 tiles */
+/* The kernel and tile that a plain product of one launch gets, by its estimate in microseconds (a double, optional): 1 two-stage kernel 128x128, 2 .. 5 ring kernel
+ * (tlq_tune_gemm_groups), 6 two-stage 256x256, 7 .. 11 four wavefronts (tlq_tune_gemm_quad), 12 the same 256x256.  kind: 0 16-bit weights [K, N], 1 [N, K], 2 int8
+ * [K, N], 3 [N, K].  0: bad arguments. */
+int tlq_debug_gemm_choice(int kind, int64_t batch, int64_t M, int64_t N, int64_t K, void* us_out);
+void tlq_tune_gemm_quad(int variant);                         /* the kernel on four wavefronts, tiles other than 256x256: 0 = automatic, 1 = never, 7 .. 11: its
+                                                              * 192x256, 128x256, 256x128, 192x128, 128x128 tiles wherever they can run */
 void tlq_tune_gemm_band(int tile_rows);                       /* tile rows per band of the MFMA kernels' tile order (default 4) */
 void tlq_tune_gemm_tile(int tile);                            /* square tile of the plain 16-bit GEMM (and of the second of the two W4A16 passes):
                                                               * 128 | 256, 0 = by the number of output tiles */

@@ -94,6 +94,8 @@ SIGNATURES = {
     "tlq_debug_gemv_ring_plan": (_int, [_i64, _i64, _i64, _i64, _int, _vp]),
     "tlq_debug_check_gemv_ring_addressing": (_int, [_i64, _i64, _i64, _i64, _int, _int, _int]),
     "tlq_tune_gemm_groups": (None, [_int]),
+    "tlq_debug_gemm_choice": (_int, [_int, _i64, _i64, _i64, _i64, _vp]),
+    "tlq_tune_gemm_quad": (None, [_int]),
     "tlq_tune_gemm_band": (None, [_int]),
     "tlq_tune_gemm_slots": (None, [_int]),
     "tlq_tune_gemm_tile": (None, [_int]),

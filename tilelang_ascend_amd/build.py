@@ -52,6 +52,8 @@ SOURCES = [
     "gemm_small.hip",
     "gemm_small_w4a8.hip",
     "gemm_f16.hip",
+    "gemm_quad_f16.hip",
+    "gemm_quad_i8.hip",
     "gemm_api.hip",
     "gemm_addr_check.hip",
     "gemm_w4a16_noalloc.hip",

@@ -188,12 +188,12 @@ __host__ __device__ __forceinline__ void ring_schedule(int KT, const Issue& issu
   }
 }
 
-// ---- four wavefronts on 256 x 256 tiles (gemm_quad.h): five slots of one operand tile and stage ----
+// ---- four wavefronts, each on a quarter of a tile (gemm_quad.h): five slots of one operand tile and stage ----
 // slot[]: at the top of stage s those of A(s), W(s), A(s + 1), W(s + 1), and the free one.  The kernel and the host-side checker both run these two functions.
-constexpr int kQuadLoads = 8;  // direct loads of a wavefront per operand and stage
+// LA, LW: direct loads of a wavefront per stage of the activations and of the weights.
 // Ahead of a work-group's first tile.  load(operand, s, slot): the loads of stage s of operand 0 (activations) or 1 (weights).  wait(n): all but the youngest
 // n loads have landed, and the wavefront's own reads of LDS are done.  read(a, w): the fragments of the first k-step.
-template <class Slot, class Load, class Wait, class Barrier, class Read>
+template <int LA, int LW, class Slot, class Load, class Wait, class Barrier, class Read>
 __host__ __device__ __forceinline__ void quad_start(const Slot (&slot)[5], const Load& load, const Wait& wait, const Barrier& barrier, const Read& read) {
   typedef std::integral_constant<int, 0> A;
   typedef std::integral_constant<int, 1> W;
@@ -201,14 +201,14 @@ __host__ __device__ __forceinline__ void quad_start(const Slot (&slot)[5], const
   load(W{}, 0, slot[1]);
   load(A{}, 1, slot[2]);
   load(W{}, 1, slot[3]);
-  wait(std::integral_constant<int, 2 * kQuadLoads>{});
+  wait(std::integral_constant<int, LA + LW>{});
   barrier();
   read(slot[0], slot[1]);
 }
 // The KT stages (two or more) of a tile.  phase(ks, first, a, w, s, to): the products of k-step ks (first: of the tile), between them the reads of the next
 // k-step's fragments from a and w and the loads of stage s of operand ks into slot `to`.  The loads ahead are those of stage s + 2, past the end the first
 // two of the next tile, ahead of which next() is called.
-template <class Slot, class Next, class Phase, class Wait, class Barrier>
+template <int LA, class Slot, class Next, class Phase, class Wait, class Barrier>
 __host__ __device__ __forceinline__ void quad_tile(int KT, Slot (&slot)[5], const Next& next, const Phase& phase, const Wait& wait, const Barrier& barrier) {
   auto stage = [&](auto first, int s) {
     int ahead = s + 2;
@@ -219,7 +219,7 @@ __host__ __device__ __forceinline__ void quad_tile(int KT, Slot (&slot)[5], cons
     phase(std::integral_constant<int, 0>{}, first, slot[0], slot[1], ahead, slot[4]);
     // all but the loads of this phase have landed, and this wavefront has read all of stage s (the first time everything: stores of the tile
     // before are among what is outstanding, and the count is one of loads in order)
-    wait(std::integral_constant<int, decltype(first)::value ? 0 : kQuadLoads>{});
+    wait(std::integral_constant<int, decltype(first)::value ? 0 : LA>{});
     barrier();
     phase(std::integral_constant<int, 1>{}, std::false_type{}, slot[2], slot[3], ahead, slot[0]);
     const Slot a = slot[0], w = slot[1];

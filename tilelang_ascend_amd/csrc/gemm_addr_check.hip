@@ -324,6 +324,7 @@ int check_ring_schedule(int stages, int loads_per_stage, int extra) {
 
 // One wavefront of the four-wavefront kernel running addr::quad_start and, for every tile, addr::quad_tile and what the kernel does behind it.  `extra` loads
 // more than the kernel's own are left in flight by the wait ahead of the first tile (extra_start) and by those of the stages (extra_stage).
+template <int LA, int LW>
 int check_quad_schedule(int stages, int tiles, int extra_start, int extra_stage) {
   const int total = stages * tiles;
   struct Held { int operand, stage, reads; bool landed, published; };  // stage: of the whole walk; reads: k-steps read, 3 = by everyone
@@ -342,7 +343,7 @@ int check_quad_schedule(int stages, int tiles, int extra_start, int extra_stage)
     if (held[to].reads != 3) fail("a load overwrites a slot that someone may still read", g);
     if (g / stages > nexts && g / stages < tiles) fail("a stage of the next tile asked for by this tile's loader", g);
     held[to] = {operand, g, 0, false, false}, steps_asked[to] = 0, fresh[to] = false;
-    for (int i = 0; i < addr::kQuadLoads; ++i) in_flight.push_back({to, g});
+    for (int i = 0; i < (operand == 0 ? LA : LW); ++i) in_flight.push_back({to, g});
   };
   auto read = [&](int operand, int g, int from, int ks) {
     if (g >= total) return;  // (behind the last tile, for nobody)
@@ -368,12 +369,12 @@ int check_quad_schedule(int stages, int tiles, int extra_start, int extra_stage)
       if (fresh[i]) held[i].reads = 3;
     }
   };
-  addr::quad_start(
+  addr::quad_start<LA, LW>(
       slot, [&](auto operand, int s, int to) { load(decltype(operand)::value, s, to); }, wait, barrier,
       [&](int a, int w) { read(0, 0, a, 0), read(1, 0, w, 0), fragments[0] = 0; });
   in_start = false;
   for (; tile < tiles; ++tile) {
-    addr::quad_tile(
+    addr::quad_tile<LA>(
         stages, slot, [&] { ++nexts; },
         [&](auto ks_tag, auto first, int a, int w, int s, int to) {
           constexpr int ks = decltype(ks_tag)::value;
@@ -1649,7 +1650,14 @@ int tlq_debug_check_quad_schedule(int stages, int tiles, int extra_start, int ex
     set_error("tlq_debug_check_quad_schedule: bad arguments");
     return 1;
   }
-  return check_quad_schedule(stages, tiles, extra_start, extra_stage);
+  // (loads of a wavefront per stage: its MFMA tiles along the tile's rows and columns)
+  int failed = 0, rc = 0;
+  for (auto* check : {check_quad_schedule<8, 8>, check_quad_schedule<6, 8>, check_quad_schedule<4, 8>, check_quad_schedule<8, 4>, check_quad_schedule<6, 4>, check_quad_schedule<4, 4>}) {
+    rc = check(stages, tiles, extra_start, extra_stage);
+    failed += rc != 0;
+    if (rc != 0 && extra_start == 0 && extra_stage == 0) return rc;
+  }
+  return failed == 6;  // (with loads left in flight every tile has to fail)
 }
 
 int tlq_debug_check_gemv_ring_addressing(int64_t M, int64_t N, int64_t K, int64_t group, int rows_per_block, int waves, int depth) {

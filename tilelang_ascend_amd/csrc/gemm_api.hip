@@ -90,6 +90,7 @@ int gemm_w4a16_decode(const void* A, const void* Wp, const void* scales, const v
 
 thread_local int g_gemm_band_rows = 0;
 thread_local int g_gemm_groups = 0;
+thread_local int g_gemm_quad = 0;
 thread_local int g_gemm_slots = 1;
 extern thread_local int g_gemm_f16_tile;
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -176,10 +177,17 @@ using namespace tlq;
 extern "C" {
 
 void tlq_tune_gemm_groups(int variant) { tlq::tuning_changed(), tlq::g_gemm_groups = variant < 0 || variant > 5 ? 0 : variant; }
+void tlq_tune_gemm_quad(int variant) { tlq::tuning_changed(), tlq::g_gemm_quad = variant == 1 || (variant >= tlq::kQuad192x256 && variant <= tlq::kQuad128x128) ? variant : 0; }
 void tlq_tune_gemm_band(int tile_rows) { tlq::g_gemm_band_rows = tile_rows < 0 ? 0 : tile_rows; }
 void tlq_tune_gemm_slots(int mode) { tlq::tuning_changed(), tlq::g_gemm_slots = mode < 0 ? 0 : (mode > 3 ? 3 : mode); }
 int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused) {
   return tlq::prefer_small_tiles(batch, M, N, fused ? 0.65 : 0.72) ? 128 : 256;
+}
+int tlq_debug_gemm_choice(int kind, int64_t batch, int64_t M, int64_t N, int64_t K, void* us_out) {
+  if (kind < 0 || kind > 3 || batch < 1 || M < 1 || N < 1 || K < 1 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim) return 0;
+  const tlq::TileChoice c = tlq::tile_choice((tlq::TileKind)kind, batch, M, N, kind >= tlq::kTileI8KN ? K : 2 * K);
+  if (us_out) *(double*)us_out = c.us;
+  return c.variant;
 }
 void tlq_tune_gemm_tile(int tile) { tlq::tuning_changed(), tlq::g_gemm_f16_tile = (tile == 128 || tile == 256) ? tile : 0; }
 void tlq_tune_w4a16_stream(int on) { tlq::tuning_changed(), tlq::g_w4a16_stream = on != 0; }  // (the workspace size above 512 rows follows it)
@@ -696,11 +704,12 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 // plain GEMM behind it runs large products at 1.4 - 1.5 PFLOP/s where the 256-row panel kernel reaches 1.2 - 1.3 (8192 x 14336 x 4096 fp16 in groups of
 // 64 774 -> 684 us), has smaller tiles, and takes any row count, while the panel kernels have 8 us per round of
 // work-groups (many rounds of short rows: 4868 x 3152 x 384 bf16 36.9 -> 25.5 us, 6631 x 4608 x 256 38.7 -> 29.8) and leave
-// one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  The panel kernels' estimates
-// are 1.21 x high (11 % rms) short of the rate they reach at best, that of the two passes 0.91 x (7 %) in the kernel of four wavefronts and 1.0 - 1.07
-// elsewhere.  On 650 problems (M 513 .. 8192, N 256 .. 14336, K 256 .. 14336, groups of 64 and 128, both types) the panel kernels or the two passes
-// are the choice on 290: 1.7 % behind the faster of the two on average, 2.9 % by the rule before, of the hundred newly taken four more
-// than 3 % behind.  Where neither panel kernel would run, all rows go through the two passes and none is left over: 132 problems 6.4 % faster, none slower.
+// one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  With the plain GEMM's tiles between
+// 128 x 128 and 256 x 256 the two passes are ahead of the 256-row kernel on all but 17 of 163 random problems that either takes (M 513 .. 8192, N 256 ..
+// 14336, K 256 .. 14336, groups of 64 and 128, both types): those of fewer than 1024 rows and more than 2000 values, and a few of one partial round.
+// The panel kernels' estimates are 1.21 x high (12 % rms) short of 1.38 PFLOP/s (4096^3 100.5 us, 101.4 in the two passes), that of the two passes within 10 %; the choice by them, with the bars
+// below, is 0.5 % behind the faster of the two.  (The middle-M kernel's bars are those that the tests of the choice ask for, 1003 x 2048 x 4096 in groups of 64
+// 35 us in a launch for 1000 rows and one for three, 29 in the two passes.)  Where neither panel kernel would run, all rows go through the two passes and none is left over.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
 static double two_passes_us(int64_t M, int64_t N, int64_t K) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(M, N, K); }
 static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
@@ -711,16 +720,17 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
     const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
     if (!p2.ok || N % 8 != 0) return false;
     double panels;
-    if (pm.ok && panelm_estimate_wins(head, N, K, group))
+    const bool middle = pm.ok && panelm_estimate_wins(head, N, K, group);
+    if (middle)
       panels = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, head, N, cus_now);
     else if (panel256_fills(head, N, K, group))
       panels = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, head, N, cus_now);
     else
       return true;
-    const double best = 2.0 * (double)M * (double)N * (double)K / 1.3e9;  // at 1.3 PFLOP/s
+    const double best = 2.0 * (double)M * (double)N * (double)K / 1.38e9;  // at 1.38 PFLOP/s
     panels = panels / 1.21 > best ? panels / 1.21 : best;
-    const bool quad = !prefer_small_tiles(1, M, N) && quad_takes(kTileF16NK, 1, M, N, K * 2);
-    return (quad ? 1.05 : 1.0) * two_passes_us(M, N, K) < panels + (head != M ? 4.5 : 0.0);
+    const double two = two_passes_us(M, N, K), with_rest = panels + (head != M ? 4.5 : 0.0);
+    return middle ? two < (head != M ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 0.95 : 1.07) * with_rest;
   });
 }
 // Many rows on up to 2^19 weights: the two passes or the tile kernel in one launch.  27 problems above 512 rows where that ran: 13 go to the two passes, 1.28 x
@@ -752,8 +762,7 @@ static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group) 
       if (us < panels) panels = us;
     }
     panels = 0.87 * panels + (head != M ? 5.5 : 0.0);
-    if (panels < other) other = panels;
-    return sp.us < 0.95 * other;
+    return sp.us < 0.98 * other && sp.us < 0.95 * panels;
   });
 }
 static StreamPlan stream_plan_for(int64_t M, int64_t N, int64_t K, int64_t group, int algo) {  // (by name: 512 rows at most)
@@ -1359,12 +1368,6 @@ int tlq_gemv_w4a16_batched(const void* A, const void* w_packed, const void* scal
                     (hipStream_t)stream);
 }
 
-// The estimate of the ring kernel (gemm_core.h), where it would run; far off otherwise.
-static double group_tile_us(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes) {
-  double us = 0.0;
-  if (M <= 32 || N < 1 || k_bytes < 1 || !prefer_small_tiles(batch, M, N) || group_tile(kind, batch, M, N, k_bytes, &us) == 0) return 1e30;
-  return us;
-}
 // What a call takes that cuts K into slices over work-groups and adds them in a further launch, by SmallW kind: 8 - 9 us before
 // anything is multiplied.
 static double sliced_us(int kind, int64_t batch, int64_t M, int64_t N, int64_t K) {
@@ -1378,19 +1381,14 @@ static double sliced_us(int kind, int64_t batch, int64_t M, int64_t N, int64_t K
     default: return 8.9 + 2.5 * g + 4.7 * mn + 0.24 * k + 6.2 * tiles_k;
   }
 }
-static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes);
-static double plain_nk_us(int64_t M, int64_t N, int64_t K) {  // one 16-bit matrix of [N, K] weights
-  const int64_t stages = ceil_div(K * 2, (int64_t)kStageBytes);
-  if (!prefer_small_tiles(1, M, N)) return tile_us(kTileF16NK, 6, 1, M, N, stages);
-  if (f16_split_choice(1, M, N, K) > 1 && !groups_beat_slices(kTileF16NK, 2, M, N, K, K * 2)) return sliced_us(2, 1, M, N, K);
-  double us = 0.0;
-  group_tile(kTileF16NK, 1, M, N, K * 2, &us);
-  return us;
+// One launch over all of K or slices of it: sliced_us is 1.25 x high on average (0.8 - 2.1), the tiles' estimate 1.05 (0.6 - 1.24); on 78 of the problems that
+// the tiles were fitted to slices had run: 69 go to one launch, 1.17 x faster on average, two of them more than 10 % slower.
+static bool tiles_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes) {
+  return M > 32 && tile_choice(tile, 1, M, N, k_bytes).us < 0.82 * sliced_us(kind, 1, M, N, K);
 }
-static bool groups_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes) {
-  // (rows of more than 48 stages stay with the slices, which their estimate makes too dear: int8 [K, N] 131 x 7568 x 7552 27.6 us in slices, 33 - 51
-  // in the ring kernel's tiles, 1856 x 544 x 24064 52.8 against 74)
-  return k_bytes <= 48 * kStageBytes && group_tile_us(tile, 1, M, N, k_bytes) < 0.9 * sliced_us(kind, 1, M, N, K);
+static double plain_nk_us(int64_t M, int64_t N, int64_t K) {  // one 16-bit matrix of [N, K] weights
+  if (f16_split_choice(1, M, N, K) > 1 && !tiles_beat_slices(kTileF16NK, 2, M, N, K, K * 2)) return sliced_us(2, 1, M, N, K);
+  return tile_choice(kTileF16NK, 1, M, N, K * 2).us;
 }
 // The products that may take the small-tile kernel: weights as stored (the first four: SmallW), int32 results, or rescaled ones
 // (W8A8), W4A8 where the caller brought the room to unpack the weights first (65 to 256 rows: above, that is what runs; the figures
@@ -1445,22 +1443,18 @@ static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int
   const TileKind tile = w == kSmallKN16 ? kTileF16KN : w == kSmallKN8 ? kTileI8KN : kTileI8NK;
   const bool adds = use == kUseI8NK || use == kUseI8KN;  // (their slices add into the result itself)
   if (packed ? M <= 256 && slice_choice(M, N, k_bytes, true, 2.5, 0) > 1
-             : batch == 1 && slice_choice(M, N, k_bytes, !adds, 1.0, 0) > 1 && !groups_beat_slices(tile, w, M, N, K, k_bytes))
+             : batch == 1 && slice_choice(M, N, k_bytes, !adds, 1.0, 0) > 1 && !tiles_beat_slices(tile, w, M, N, K, k_bytes))
     return us < (M <= 32 ? bar.few_sliced : bar.sliced) * sliced_us(w, batch, M, N, K);
   if (packed && use != kUseW4A8TwoSteps && use != kUseW4A8TwoStepsTimes16) return us < bar.few * (4.9 + 0.069 * nk + 1.44 * mn + 5.7 * k + 0.69 * g32);
   if (M <= 32 && w == kSmallNK) return us < bar.few * (5.1 + 1.4 * g + 0.16 * mn + 2.07 * k);
   if (M <= 32 && w == kSmallKN8) return us < bar.few * (4.8 + 1.22 * g + 0.078 * nk + 0.3 * mn + 2.4 * k + 0.38 * g32);
   if (M <= 32 && w == kSmallKN16) return us < bar.few * (3.8 + 0.08 * nk + 0.6 * mn + 9.4 * k + 12.8 * (double)batch * (double)ceil_div(N, (int64_t)128) * (double)K * 1e-6);
   const double unpack_us = packed ? 2.6 + nk * 1.5 / 4.5 : 0.0;
-  if (packed && i8_split_choice(1, M, N, K, false) > 1 && !groups_beat_slices(kTileI8NK, 0, M, N, K, K))
+  if (packed && i8_split_choice(1, M, N, K, false) > 1 && !tiles_beat_slices(kTileI8NK, 0, M, N, K, K))
     return us < bar.sliced * (unpack_us + 2.0 * sliced_us(0, 1, M, N, K));  // (slices that add into the result take twice those with matrices of their own)
-  if (!prefer_small_tiles(batch, M, N)) return us < bar.plain * (unpack_us + tile_us(tile, 6, batch, M, N, stages));
-  double tiles_us = 0.0;
-  if (group_tile(tile, batch, M, N, k_bytes, &tiles_us) != 0) {
-    const double mine = bar.launch + bar.scale * t.us + bar.trip * trip_us + bar.step * (double)stages + bar.out * mn + bar.weights * nk;
-    return mine < unpack_us + tiles_us;
-  }
-  return us < bar.plain * (unpack_us + tiles_us);
+  const double other_us = unpack_us + tile_choice(tile, batch, M, N, k_bytes).us;
+  const double mine = bar.launch + bar.scale * t.us + bar.trip * trip_us + bar.step * (double)stages + bar.out * mn + bar.weights * nk;
+  return mine < other_us && us < 1.5 * other_us;  // (far from the problems of the fit the kernel's own estimate is the better one: fp16 170 x 10656 x 3328 44.8 us, 20.2 in the ring kernel)
 }
 static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t K, SmallUse use) {
   const SmallTile t{false, 0, 0, 0, 0.0};
@@ -1490,7 +1484,9 @@ static SmallTile small_tile_for_f16(int64_t batch, int64_t M, int64_t N, int64_t
 // 62 us.)  Not on rows of fewer than six 128-byte stages, where a launch more is a larger part than the 1.5 us below: 300 random problems
 // that two launches were estimated to win ran, against one, 0.93 as fast on rows of one to three stages (25 of 33 more than 3 % behind;
 // int8 7314 x 2384 x 384 26.7 us for 22.6), 1.01 on four or five (8 of 30 behind), 1.06 on six or seven (1 of 14), 1.1 on eight to
-// fifteen (2 of 55) and 1.2 beyond (none of 168).
+// fifteen (2 of 55) and 1.2 beyond (none of 168).  The tiles between 128 x 128 and 256 x 256 (gemm_core.h) fill most of those rounds in one launch: they are
+// taken where they are estimated to be 12 % ahead of two launches.  (Within that both are about level, 4099 x 4096 x 1024 int8 28.3 us in one launch and 26.2 in two; a test
+// of the two launches names 7314 x 2384 x 768, 23.5 and 27.4.)
 static int64_t rows_of_full_rounds(TileKind kind, int64_t M, int64_t N, int64_t K) {
   if (M <= 512 || N < 256 || K % 128 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_gemm_groups || g_gemm_f16_tile || g_i8_tile || g_gemm_slots == 2) return 0;
   static thread_local PlanTable<int64_t> known;
@@ -1498,24 +1494,23 @@ static int64_t rows_of_full_rounds(TileKind kind, int64_t M, int64_t N, int64_t 
     const bool i8 = kind >= kTileI8KN;
     const int64_t k_bytes = i8 ? K : 2 * K, stages = k_bytes / kStageBytes, cus = cu_count_or_default();
     if (stages < 6) return 0;
-    auto one_us = [&](int64_t rows) {
-      double us = 0.0;
-      if (!prefer_small_tiles(1, rows, N)) return tile_us(kind, 6, 1, rows, N, stages);
-      group_tile(kind, 1, rows, N, k_bytes, &us);
-      return us;
-    };
+    auto one_us = [&](int64_t rows) { return tile_choice(kind, 1, rows, N, k_bytes).us; };
     auto rest_us = [&](int64_t rows) {
       const double us = one_us(rows);
       if (kind == kTileF16NK) return us;
       const SmallTile t = i8 ? small_tile_for_i8(1, rows, N, K, kind == kTileI8NK ? kUseI8NK : kUseI8KN) : small_tile_for_f16(1, rows, N, K, TLQ_B_KN);
       return t.ok && t.us < us ? t.us : us;
     };
-    double best = 0.87 * one_us(M);
+    // (in one launch the tiles in between fill the rounds as a rule; only the others are asked whether two are ahead of them, and those tiles whether
+    // they are ahead of both)
+    const double between_us = 1.13 * one_us(M);
+    double best = 0.97 * tile_choice(kind, 1, M, N, k_bytes, -1).us;
+    if (between_us < best) best = between_us;
     int64_t head = 0;
     for (const int64_t tile : {(int64_t)256, (int64_t)128}) {
       const int64_t across = ceil_div(N, tile), round = tile == 256 ? cus : 2 * cus, rounds = ceil_div(M, tile) * across / round;
       const int64_t rows = rounds * round / across * tile;
-      if (rounds == 0 || rows <= 0 || rows >= M || prefer_small_tiles(1, rows, N) != (tile == 128)) continue;
+      if (rounds == 0 || rows <= 0 || rows >= M) continue;
       const double us = one_us(rows) + 1.5 + rest_us(M - rows);
       if (us < best) best = us, head = rows;
     }
@@ -1569,7 +1564,7 @@ int tlq_gemm_f16_ws(const void* A, const void* B, void* C, void* workspace, int6
     split = f16_split_choice(batch, M, N, K);
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;
   }
-  if (g_f16_split == 0 && split > 1 && (small_tile_for_f16(batch, M, N, K, b_layout).ok || groups_beat_slices(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, 2, M, N, K, K * 2)))
+  if (g_f16_split == 0 && split > 1 && (small_tile_for_f16(batch, M, N, K, b_layout).ok || tiles_beat_slices(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, 2, M, N, K, K * 2)))
     split = 1;
   if (split <= 1) return tlq_gemm_f16_batched(A, B, C, batch, M, N, K, in_dtype, out_dtype, b_layout, stream);
   TLQ_REQUIRE(in_dtype == TLQ_F16 || in_dtype == TLQ_BF16, "tlq_gemm_f16_ws: in_dtype must be float16 or bfloat16 (got %d)",
@@ -1617,7 +1612,7 @@ int tlq_gemm_i8(const void* A, const void* B, void* C, int64_t batch, int64_t M,
   if (const SmallTile t = small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? kUseI8NK : kUseI8KN); t.ok) return small_i8(t, A, B, C, batch, M, N, K, b_layout, (hipStream_t)stream);
   // few activation rows: K slices add into C itself (int32, exact in any order)
   if (const int split = i8_split_choice(batch, M, N, K, false);
-      split > 1 && (g_i8_split || !groups_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
+      split > 1 && (g_i8_split || !tiles_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
     return gemm_i8_i32_splitk(A, B, (int32_t*)C, M, N, K, split, b_layout, (hipStream_t)stream);
   if (const int64_t head = batch == 1 ? rows_of_full_rounds(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, M, N, K) : 0; head > 0) {
     if (const int rc = tlq_gemm_i8(A, B, C, 1, head, N, K, b_layout, stream)) return rc;
@@ -1726,7 +1721,7 @@ int tlq_gemm_w8a8_ws(const void* A, const void* B, const void* scale_a, const vo
     while (split > 1 && (int64_t)split * M * N * 4 > workspace_bytes) split /= 2;  // as many slices as the workspace holds
   }
   if (split <= 1 || small_tile_for_i8(batch, M, N, K, b_layout == TLQ_B_NK ? kUseW8A8NK : kUseW8A8KN).ok ||
-      (!g_i8_split && groups_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
+      (!g_i8_split && tiles_beat_slices(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, b_layout == TLQ_B_NK ? 0 : 1, M, N, K, K)))
     return tlq_gemm_w8a8(A, B, scale_a, scale_b, C, batch, M, N, K, n_scale_b, b_layout, out_dtype, stream);
   TLQ_REQUIRE(b_layout == TLQ_B_KN || b_layout == TLQ_B_NK, "tlq_gemm_w8a8_ws: bad b_layout %d", b_layout);
   TLQ_REQUIRE(out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32, "tlq_gemm_w8a8_ws: bad out_dtype %d",

@@ -22,6 +22,7 @@
 // only on row bits 0..2, so rows 8 apart differ by a constant).
 #pragma once
 
+#include <cmath>
 #include <type_traits>
 
 #include "gemm_addr.h"
@@ -723,10 +724,10 @@ __device__ __forceinline__ void write_tile_with(const Epi& epi, const S& scales,
                                                 int n_base, int M, int N) {
   const int r16 = lane & 15, q = lane >> 4;
   const int osz = epi.out_bytes();
-  // 64 accumulator tiles live in the accumulation registers: each is moved where it is used, or the compiler moves many ahead and spills
+  // (the four-wavefront kernel) accumulators live in the accumulation registers: each is moved where it is used, or the compiler moves many ahead and spills
   auto taken = [&](const auto& sum) {
     std::remove_const_t<std::remove_reference_t<decltype(sum)>> v = sum;
-    if constexpr (TM * TN >= 64) asm volatile("" : "+v"(v));
+    if constexpr (TMP < TM) asm volatile("" : "+v"(v));
     return v;
   };
   bool staged = false;
@@ -998,112 +999,77 @@ inline bool prefer_small_tiles(int64_t batch, int64_t M, int64_t N, double weigh
   return tile_fill(batch, M, N, 128) * weight > tile_fill(batch, M, N, 256);
 }
 
-// ---- launches that give each CU one work-group at most: the ring kernel (gemm_ring.h) ----
-// Its tiles: 128 x 128, and narrower ones where even those would leave CUs idle.
-enum { kGroup128x128 = 2, kGroup128x64 = 3, kGroup64x128 = 4, kGroup64x64 = 5 };
+// ---- the kernel and its tiles ----
+// 128 x 128 tiles of the two-stage kernel, two work-groups to a CU; the ring kernel's (gemm_ring.h); 256 x 256 of the two-stage kernel (five slots
+// where dispatch_i8 says so); those of the kernel on four wavefronts (gemm_quad.h), of which two work-groups of 128 x 128 share a CU.
+enum { kPlain128x128 = 1, kGroup128x128 = 2, kGroup128x64 = 3, kGroup64x128 = 4, kGroup64x64 = 5, kPlain256x256 = 6,
+       kQuad192x256 = 7, kQuad128x256 = 8, kQuad256x128 = 9, kQuad192x128 = 10, kQuad128x128 = 11, kQuad256x256 = 12, kTileVariants = 12 };
 enum TileKind { kTileF16KN = 0, kTileF16NK = 1, kTileI8KN = 2, kTileI8NK = 3 };
 extern thread_local int g_gemm_groups;  // tuning: 0 = automatic, 1 = never, kGroup* = that variant wherever 128-row tiles are taken
-// Microseconds of a launch.  Two-stage kernels: launch + rounds x (fixed + stages x step); `lone`: the step of a plain 128 x 128 work-group
-// that has its CU to itself (260 problems, M 64 .. 8000, N 256 .. 14000, K 256 .. 14336, one to eight batches: 8 - 15 % rms).
+extern thread_local int g_gemm_quad;    // tuning: 0 = automatic, 1 = 256 x 256 alone, kQuad* (but that one) = that tile wherever it can run
+extern thread_local int g_gemm_slots;   // tlq_tune_gemm_slots: 0 = the two-stage kernel alone, 1 = automatic, 2 = five slots, 3 = four wavefronts, wherever either can run
+struct TileShape {
+  int rows, cols, per_cu;
+};
+static constexpr TileShape kTileShape[kTileVariants] = {{128, 128, 2}, {128, 128, 1}, {128, 64, 1}, {64, 128, 1}, {64, 64, 1}, {256, 256, 1},
+                                                        {192, 256, 1}, {128, 256, 1}, {256, 128, 1}, {192, 128, 1}, {128, 128, 2}, {256, 256, 1}};
+// Microseconds of a launch: launch + per round of work-groups fixed + shared x in_round + stages x (step + step_shared x in_round), in_round being the part
+// of the machine's places that have a work-group (what they take from each other, of memory and of the clock, grows with their number); and
+// next to that what the bytes take at 5 TB/s, the products at 2.4 POP/s or 1.52 PFLOP/s and the call by itself.  Fitted to every variant's time on 1120 random problems, 280 per kind (M 33 ..
+// 8192, N 256 .. 14336, 256 - 28000 bytes of K, one to eight batches): 4 - 13 % rms, the int8 ring tiles of 64 rows or columns 16 - 24 %.  The variant of the least
+// estimate is 0.5 - 0.8 % behind the fastest on average on problems that the fit had not seen (more than 5 % on 47 of 1120), and 5 - 8 % ahead of the rules before (128 x 128 or
+// 256 x 256 by how full they make the machine, the ring in one round of tiles, four wavefronts on 256 x 256 tiles by stages), of which the tiles in between are
+// most: 2159 x 2080 x 3072 fp16 44.2 -> 31.0 us in 192 x 128 tiles, 4 x 3620 x 1312 x 9472 445 -> 327 in 192 x 256.
 struct TileCost {
-  double launch, fixed, step, lone;
+  float launch, fixed, shared, step, step_shared;
 };
-static constexpr TileCost kTileCost[4][2] = {
-    // 128 x 128                  256 x 256
-    {{2.4, 1.4, 1.16, 0.74}, {0.0, 5.3, 1.31, 0}},
-    {{2.4, 1.4, 1.10, 0.70}, {0.0, 5.3, 1.25, 0}},
-    {{2.0, 3.4, 1.23, 0.72}, {0.0, 7.3, 1.32, 0}},
-    {{0.3, 6.2, 1.02, 0.60}, {0.0, 8.8, 1.13, 0}}};
-// Ring kernel, per round: fixed + stages x (step + shared x the part of the CUs that have a work-group): what the work-groups take from
-// each other, of memory and of the clock, grows with their number.  Fitted to 300 - 700 problems per entry (M 33 .. 3500, N 256 .. 14000, 512 .. 28000 bytes of K,
-// one to eight batches), every variant that runs in one round forced on each: 8 - 13 % rms; the variant it picks is 0.7 - 1.6 % behind the best on average.
-struct RingCost {
-  double fixed, step, shared;
-};
-static constexpr RingCost kRingCost[4][4] = {
-    // 128 x 128           128 x 64              64 x 128              64 x 64
-    {{4.74, 0.313, 0.201}, {4.01, 0.217, 0.171}, {3.79, 0.246, 0.135}, {3.73, 0.174, 0.076}},
-    {{4.56, 0.288, 0.201}, {4.07, 0.195, 0.124}, {3.71, 0.212, 0.157}, {3.72, 0.146, 0.075}},
-    {{4.73, 0.362, 0.239}, {4.33, 0.287, 0.168}, {3.71, 0.314, 0.123}, {3.65, 0.243, 0.105}},
-    {{4.98, 0.281, 0.218}, {4.28, 0.189, 0.151}, {3.92, 0.206, 0.178}, {3.76, 0.140, 0.094}}};
-// ---- 256 x 256 tiles on four wavefronts (gemm_quad.h) ----
-extern thread_local int g_gemm_slots;  // tlq_tune_gemm_slots: 0 = the two-stage kernel alone, 1 = automatic, 2 = five slots, 3 = four wavefronts, wherever either can run
-// In the place of the other kernels of 256 x 256 tiles from so many stages on: 16-bit 17 in one round of tiles, 9 in two, 6 from three on, int8
-// 17, 17, 9.  Its first tile's operands and its last tile's store are four wavefronts' work.  On 480 problems (120 per kind, M 256 .. 8192, N 256 ..
-// 14336, 128 - 28000 bytes of K, one to four batches) time over that of the kernel before, on average, one round: 1.11 - 1.17 on 5 - 8 stages, 0.99 - 1.09 on
-// 9 - 16, 0.90 - 0.97 on 17 - 32, 0.86 - 0.93 beyond; three rounds and more: 16-bit 0.97 - 1.0 from 3 stages on, int8 1.02 - 1.05 on 3 - 8, 0.97 - 0.99 on 9 - 16.
-inline bool quad_takes(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes) {
-  const int64_t stages = k_bytes / kStageBytes;
-  if (k_bytes % kStageBytes != 0 || stages < 2 || (g_gemm_slots != 1 && g_gemm_slots != 3)) return false;
-  if (g_gemm_slots == 3) return true;
+static constexpr TileCost kTileCost[4][kTileVariants] = {
+    // in the order of the variants
+    {{2.43, 0.37, 2.37, 0.652, 0.439}, {1.46, 2.98, 0.00, 0.283, 0.246}, {1.27, 2.52, 0.00, 0.217, 0.140}, {1.34, 2.08, 0.00, 0.223, 0.132}, {2.76, 0.22, 0.67, 0.164, 0.051}, {0.00, 4.40, 1.50, 1.073, 0.648}, {2.01, 3.79, 1.08, 0.791, 0.362}, {2.40, 2.42, 0.00, 0.586, 0.398}, {2.46, 2.61, 0.33, 0.528, 0.312}, {2.48, 1.94, 0.00, 0.433, 0.297}, {3.05, 0.00, 1.96, 0.388, 0.588}, {2.75, 4.23, 2.45, 0.968, 0.402}},
+    {{2.47, 0.20, 2.68, 0.612, 0.426}, {1.58, 2.54, 0.37, 0.285, 0.223}, {0.94, 2.64, 0.00, 0.214, 0.116}, {1.45, 1.79, 0.31, 0.225, 0.108}, {2.65, 0.30, 0.59, 0.159, 0.039}, {0.90, 3.22, 3.03, 1.111, 0.503}, {2.73, 2.68, 1.84, 0.766, 0.368}, {2.27, 2.22, 0.00, 0.595, 0.358}, {2.01, 2.83, 0.24, 0.514, 0.321}, {2.34, 1.68, 0.23, 0.434, 0.304}, {2.79, 0.00, 2.07, 0.401, 0.549}, {3.29, 3.26, 3.50, 0.951, 0.384}},
+    {{1.93, 1.50, 2.49, 0.652, 0.437}, {1.87, 2.81, 0.25, 0.302, 0.274}, {1.47, 3.21, 0.00, 0.278, 0.154}, {1.90, 2.08, 0.00, 0.238, 0.168}, {3.59, 0.05, 0.60, 0.209, 0.075}, {0.45, 5.44, 2.61, 1.058, 0.510}, {3.03, 4.45, 2.06, 0.776, 0.317}, {2.92, 3.04, 1.39, 0.605, 0.278}, {2.88, 3.55, 0.83, 0.522, 0.283}, {2.75, 2.54, 0.85, 0.451, 0.242}, {3.52, 0.34, 2.92, 0.404, 0.543}, {3.11, 6.06, 2.41, 0.976, 0.379}},
+    {{1.92, 1.61, 2.43, 0.592, 0.445}, {1.80, 2.82, 0.05, 0.280, 0.256}, {1.83, 2.95, 0.13, 0.195, 0.167}, {2.26, 1.64, 0.12, 0.206, 0.175}, {3.27, 0.80, 0.00, 0.128, 0.092}, {0.96, 4.65, 3.36, 1.089, 0.484}, {2.91, 4.49, 2.03, 0.757, 0.320}, {2.73, 3.04, 1.34, 0.595, 0.281}, {2.74, 3.65, 0.76, 0.497, 0.312}, {2.55, 2.86, 0.43, 0.421, 0.257}, {3.24, 0.53, 2.86, 0.387, 0.485}, {3.03, 6.07, 2.69, 0.943, 0.399}}};
+inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int64_t N, int64_t k_bytes) {
   int cus = tlq_device_cu_count();
   if (cus <= 0) cus = 256;
-  const int64_t tiles = batch * ceil_div(M, (int64_t)256) * ceil_div(N, (int64_t)256);
-  if (kind >= kTileI8KN) return stages >= (tiles > 2 * cus ? 9 : 17);
-  return stages >= (tiles > 2 * cus ? 6 : (tiles > cus ? 9 : 17));
+  const TileShape& t = kTileShape[variant - 1];
+  const TileCost& c = kTileCost[kind][variant - 1];
+  const int64_t stages = ceil_div(k_bytes, (int64_t)kStageBytes), blocks = batch * ceil_div(M, (int64_t)t.rows) * ceil_div(N, (int64_t)t.cols), places = (int64_t)cus * t.per_cu;
+  const double rounds = (double)(blocks / places), in_round = (double)(blocks % places) / (double)places;
+  double us = c.launch + rounds * (c.fixed + c.shared + (double)stages * (c.step + c.step_shared));
+  if (in_round > 0.0) us += c.fixed + c.shared * in_round + (double)stages * (c.step + c.step_shared * in_round);
+  const double bytes = (double)(batch * (M + N)) * (double)k_bytes + 2.0 * (double)(batch * M) * (double)N;
+  const double ops = 2.0 * (double)(batch * M) * (double)N * (double)k_bytes;
+  const double memory = bytes / 5.0e6, product = kind >= kTileI8KN ? ops / 2.4e9 : ops / 3.04e9, most = memory < product ? product : memory, least = most < 4.3 ? 4.3 : most;
+  // (the root of the sum of the eighth powers, not the larger of the two: where several tiles reach the rates the one that is there with less work is ahead)
+  const double q = us / least * (us / least), q4 = q * q;
+  return q > 100.0 ? us : least * std::sqrt(std::sqrt(std::sqrt(1.0 + q4 * q4)));
 }
-// Per round: fixed + stages x step, fitted to the 167 of those problems that it takes (5 - 9 % rms); with every CU busy 1.5 PFLOP/s and 2.4 POP/s.
-struct QuadCost {
-  double launch, fixed, step;
+struct TileChoice {
+  int variant;
+  double us;
 };
-static constexpr QuadCost kQuadCost[4] = {{0.0, 8.7, 1.07}, {0.0, 9.0, 1.01}, {0.0, 11.6, 1.04}, {3.5, 12.7, 0.88}};
-inline int64_t tile_blocks(int variant, int64_t batch, int64_t M, int64_t N) {  // variant 1 (plain 128 x 128), kGroup*, 6 (256 x 256)
-  static constexpr int kRows[6] = {128, 128, 128, 64, 64, 256}, kCols[6] = {128, 128, 64, 128, 64, 256};
-  return batch * ceil_div(M, (int64_t)kRows[variant - 1]) * ceil_div(N, (int64_t)kCols[variant - 1]);
-}
-inline double tile_us(TileKind kind, int variant, int64_t batch, int64_t M, int64_t N, int64_t stages) {
-  int cus = tlq_device_cu_count();
-  if (cus <= 0) cus = 256;
-  const int64_t blocks = tile_blocks(variant, batch, M, N);
-  const double memory = (double)(batch * (M + N)) * (double)(stages * kStageBytes) / 4.8e6;  // the rate of a copy, whatever the tiles
-  // a large product with every CU busy runs at the rate the part sustains under that load: 2.1 POP/s int8, 1.45 PFLOP/s 16-bit
-  const double k = (double)(stages * kStageBytes), product = 2.0 * (double)(batch * M) * (double)N * (kind >= kTileI8KN ? k / 2.1e9 : k / 2.9e9);
-  const double floor_us = memory > product ? memory : product;
-  if (variant >= kGroup128x128 && variant <= kGroup64x64) {
-    const RingCost& c = kRingCost[kind][variant - kGroup128x128];
-    const double in_round = blocks < cus ? (double)blocks / (double)cus : 1.0;
-    const double us = (double)ceil_div(blocks, (int64_t)cus) * (c.fixed + (double)stages * (c.step + c.shared * in_round));
-    // several tile rows read the weights again, from memory mostly where the order of tiles is not one by XCD
-    const int64_t tiles_m = ceil_div(M, (int64_t)(variant <= kGroup128x64 ? 128 : 64));
-    const double again = (blocks % 8 != 0 ? 0.9 : 0.3) * (double)((tiles_m < 4 ? tiles_m : 4) - 1);
-    const double trips = memory + again * (double)(batch * N) * (double)(stages * kStageBytes) / 4.8e6;
-    const double most = trips > product ? trips : product;
-    return us > most ? us : most;
-  }
-  if (variant == 6 && quad_takes(kind, batch, M, N, stages * kStageBytes)) {
-    const QuadCost& c = kQuadCost[kind];
-    const double run = (double)ceil_div(blocks, (int64_t)cus) * (c.fixed + (double)stages * c.step), rate = product * (kind >= kTileI8KN ? 2.1 / 2.4 : 1.45 / 1.5);
-    return c.launch + (run > rate ? (run > memory ? run : memory) : (rate > memory ? rate : memory));
-  }
-  const TileCost& c = kTileCost[kind][variant == 1 ? 0 : 1];
-  const double run = c.fixed + c.step * (double)stages;
-  const int64_t rounds = blocks / (2 * cus), rest = blocks % (2 * cus);  // two plain 128 x 128 work-groups share a CU
-  const double us = variant != 1 ? run * (double)ceil_div(blocks, (int64_t)cus)
-                                 : run * (double)rounds + (rest == 0 ? 0.0 : rest > cus ? run : c.fixed + c.lone * (double)stages);
-  return c.launch + (us > floor_us ? us : floor_us);
-}
-// The variant for a problem that would run 128 x 128 tiles: 0 = those, or one of kGroup*, where its work-groups run in one round.  On 880
-// problems (220 per kind, ranges as above) the plain tiles were the fastest on 4, by 3 % at most, so that nothing is asked of the estimate but
-// which of the ring's tiles.  More than one round stays with the plain tiles: two of their work-groups share a CU, and cover each
-// other's barriers (fp16 8 x 780 x 528 x 10752 234 us in two rounds of the 128 x 64 tiles there were before, 160 in plain ones).
-inline int group_tile(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes, double* us = nullptr) {
+// `tile`: 128 or 256: of those square tiles; 0: any; -1: any but the four-wavefront kernel's in between.  The ring kernel takes four stages and more and 33 rows and more (fewer: not measured), the kernel on four
+// wavefronts whole stages, two or more, and on tiles other than 256 x 256 what 64 tiles of 128 x 128 hold (fewer are the small-tile kernel's or the ring's).
+inline TileChoice tile_choice(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes, int tile = 0) {
   const int64_t stages = ceil_div(k_bytes, (int64_t)kStageBytes);
-  if (g_gemm_groups > 1) return stages >= 4 ? g_gemm_groups : 0;
-  int best = 0;
-  double best_us = 0.0;
-  if (g_gemm_groups == 0 && stages >= 4 && M > 32) {  // (up to 32 rows: not measured)
-    int cus = tlq_device_cu_count();
-    if (cus <= 0) cus = 256;
-    for (int v = kGroup128x128; v <= kGroup64x64; ++v) {
-      if (tile_blocks(v, batch, M, N) > cus) continue;
-      const double t = tile_us(kind, v, batch, M, N, stages);
-      if (best == 0 || t < best_us) best = v, best_us = t;
-    }
+  const bool few = batch * M * N < (int64_t)64 * 128 * 128;
+  const bool whole = k_bytes % kStageBytes == 0 && stages >= 2, quad = whole && (g_gemm_slots == 1 || g_gemm_slots == 3);
+  if (g_gemm_quad > 1 && whole) return {g_gemm_quad, 0.0};
+  if (g_gemm_groups > 1 && stages >= 4 && tile != 256) return {g_gemm_groups, 0.0};
+  TileChoice best{0, 0.0};
+  for (int v = 1; v <= kTileVariants; ++v) {
+    if (v >= kGroup128x128 && v <= kGroup64x64 && (tile == 256 || g_gemm_groups == 1 || stages < 4 || M <= 32)) continue;
+    if (v == kPlain128x128 && tile == 256) continue;
+    if (v == kPlain256x256 && (tile == 128 || (tile <= 0 && M <= 128) || (g_gemm_slots == 3 && quad))) continue;
+    if (v >= kQuad192x256 && v <= kQuad128x128 && (tile != 0 || !quad || g_gemm_quad == 1 || M <= 32 || few)) continue;
+    if (v == kQuad256x256 && (tile == 128 || !quad || (tile <= 0 && M <= 128))) continue;
+    const double us = tile_us(kind, v, batch, M, N, k_bytes);
+    if (best.variant == 0 || us < best.us) best = {v, us};
   }
-  if (us) *us = best != 0 ? best_us : tile_us(kind, 1, batch, M, N, stages);
   return best;
 }
-// RUN(tile rows, tile columns, ring kernel or not) for a variant of group_tile()
+// RUN(tile rows, tile columns, ring kernel or not) for 128 x 128 tiles of the two-stage kernel and the ring kernel's
 #define TLQ_GROUP_TILES(variant, RUN)                \
   switch (variant) {                                 \
     case kGroup128x128: RUN(128, 128, true)          \
@@ -1111,6 +1077,15 @@ inline int group_tile(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_
     case kGroup64x128: RUN(64, 128, true)            \
     case kGroup64x64: RUN(64, 64, true)              \
     default: RUN(128, 128, false)                    \
+  }
+// RUN(tile rows, tile columns) for the tiles of the kernel on four wavefronts other than 256 x 256
+#define TLQ_QUAD_TILES(variant, RUN)       \
+  switch (variant) {                       \
+    case kQuad192x256: RUN(192, 256)       \
+    case kQuad128x256: RUN(128, 256)       \
+    case kQuad256x128: RUN(256, 128)       \
+    case kQuad192x128: RUN(192, 128)       \
+    default: RUN(128, 128)                 \
   }
 
 // ---- K slices of a one-batch GEMM with few activation rows ---------------------------------------------

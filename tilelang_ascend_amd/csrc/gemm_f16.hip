@@ -203,16 +203,24 @@ int gemm_f16_slices(const void* A, const void* B, void* C, float* partial, int64
   return check_launch("tlq_gemm_f16 (sum of the slices)") ? 0 : 1;
 }
 
+int quad_gemm_f16(int variant, const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int in_dtype, int out_dtype, int b_layout,
+                  hipStream_t st);
+
 template <class Mma>
 static int dispatch_f16(const void* A, const void* B, void* C, int64_t batch, int64_t M, int64_t N, int64_t K, int out_dtype,
                         int b_layout, hipStream_t st) {
-  const bool small = g_gemm_f16_tile ? g_gemm_f16_tile == 128 : prefer_small_tiles(batch, M, N);
-  if (small) {
-    const int variant = b_layout == TLQ_B_NK || N % 8 == 0 ? group_tile(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, batch, M, N, K * 2) : 0;
+  const TileKind kind = b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN;
+  const bool direct = b_layout == TLQ_B_NK || N % 8 == 0;  // (weights [K, N] in rows that are no whole 16-byte chunks: the two-stage kernel's loader through registers)
+  static thread_local PlanTable<int> known;
+  const int variant = direct ? known.get(batch * 4 + kind, M, N, K, [&] { return tile_choice(kind, batch, M, N, K * 2, g_gemm_f16_tile).variant; })
+                             : (g_gemm_f16_tile ? g_gemm_f16_tile == 128 : prefer_small_tiles(batch, M, N)) ? kPlain128x128 : kPlain256x256;
+  if (variant < kPlain256x256) {
 #define TLQ_RUN(BM, BN, RING) return run_f16<Mma, BM, BN, 2, 2, RING>(A, B, C, batch, M, N, K, out_dtype, b_layout, st);
     TLQ_GROUP_TILES(variant, TLQ_RUN)
 #undef TLQ_RUN
   }
+  if (variant >= kQuad192x256 && variant <= kQuad128x128)
+    return quad_gemm_f16(variant, A, B, C, batch, M, N, K, std::is_same<Mma, MmaF16>::value ? TLQ_F16 : TLQ_BF16, out_dtype, b_layout, st);
   // (the five-slot kernel only on request: alternating runs on one box have the two-stage loop 3 - 14 % ahead on ten of
   // twelve 16-bit shapes, 2 % behind on the other two)
   if (g_gemm_slots == 2 && b_layout == TLQ_B_NK && K % 64 == 0) {  // whole 128-byte stages
@@ -227,7 +235,7 @@ static int dispatch_f16(const void* A, const void* B, void* C, int64_t batch, in
     EpiFloat::Params pe{C, N, M * N, out_dtype};
     return launch_gemm_slots<Mma, H16KNLoaderDirect<256, 512>, EpiFloat>(pa, pw, pe, batch, M, N, K * 2, st, "tlq_gemm_f16", 4);
   }
-  if ((b_layout == TLQ_B_NK || N % 8 == 0) && quad_takes(b_layout == TLQ_B_NK ? kTileF16NK : kTileF16KN, batch, M, N, K * 2)) {
+  if (variant == kQuad256x256) {
     typedef RowLoaderDirect<256, 256> Rows;
     const typename Rows::Params pa((const uint8_t*)A, K * 2, M * K * 2, K * 2);
     const EpiFloat::Params pe(C, N, M * N, out_dtype);

@@ -118,17 +118,26 @@ static int run_i8(const void* A, const typename WL::Params& pw, const typename E
 
 thread_local int g_i8_tile = 0;
 
+// W4A8 through the loader that unpacks into LDS
 static int pick_tile(int64_t batch, int64_t M, int64_t N) {
   if (g_i8_tile) return g_i8_tile;
   if (M <= 32) return 32;
-  return prefer_small_tiles(batch, M, N) ? 128 : 256;  // by machine fill (the rule holds for int8 as measured: twelve shapes, both weight layouts)
+  return prefer_small_tiles(batch, M, N) ? 128 : 256;  // by machine fill
 }
+
+template <class Epi>
+int quad_gemm_i8(int variant, const void* A, const void* B, const typename Epi::Params& pe, int64_t batch, int64_t M, int64_t N, int64_t K, int b_layout, hipStream_t st,
+                 const char* what);
 
 template <class Epi>
 static int dispatch_i8(const void* A, const void* B, const typename Epi::Params& pe, int64_t batch, int64_t M,
                        int64_t N, int64_t K, int b_layout, hipStream_t st, const char* what) {
-  const int tile = pick_tile(batch, M, N);
-  if (tile == 256 && quad_takes(b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN, batch, M, N, K)) {
+  const TileKind kind = b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN;
+  static thread_local PlanTable<int> known;
+  const int variant = g_i8_tile == 32 || (M <= 32 && g_i8_tile == 0) ? 0 : known.get(batch * 4 + kind, M, N, K, [&] { return tile_choice(kind, batch, M, N, K, g_i8_tile).variant; });
+  if (variant >= kQuad192x256 && variant <= kQuad128x128) return quad_gemm_i8<Epi>(variant, A, B, pe, batch, M, N, K, b_layout, st, what);
+  const int tile = variant == 0 ? 32 : variant < kPlain256x256 ? 128 : 256;
+  if (variant == kQuad256x256) {
     typedef RowLoaderDirect<256, 256> Rows;
     const typename Rows::Params pa((const uint8_t*)A, K, M * K, K);
     if (b_layout == TLQ_B_NK) return launch_quad<MmaI8, Rows, Epi>(pa, typename Rows::Params((const uint8_t*)B, K, N * K, K), pe, batch, M, N, K, st, what, 2);
@@ -155,7 +164,7 @@ static int dispatch_i8(const void* A, const void* B, const typename Epi::Params&
         TLQ_RUN(32, 128, 1, 4, false)
       case 128:
 #define TLQ_TILE(BM, BN, RING) TLQ_RUN(BM, BN, 2, 2, RING)
-        TLQ_GROUP_TILES(group_tile(kTileI8KN, batch, M, N, K), TLQ_TILE)
+        TLQ_GROUP_TILES(variant, TLQ_TILE)
       default:
         TLQ_RUN(256, 256, 2, 4, false)
     }
@@ -175,7 +184,7 @@ static int dispatch_i8(const void* A, const void* B, const typename Epi::Params&
       case 32:
         TLQ_RUN(32, 128, 1, 4, false)
       case 128:
-        TLQ_GROUP_TILES(group_tile(kTileI8NK, batch, M, N, K), TLQ_TILE)
+        TLQ_GROUP_TILES(variant, TLQ_TILE)
 #undef TLQ_TILE
       default:
         TLQ_RUN(256, 256, 2, 4, false)

@@ -1,6 +1,6 @@
-// MFMA GEMM over a ring of K stages, for launches that give each CU one work-group at most (group_tile in gemm_core.h).
+// MFMA GEMM over a ring of K stages, for few tiles: launches that give each CU one work-group at most, as a rule (tile_choice in gemm_core.h).
 //
-// What bounds such a launch is what a CU takes in: a 128 x 128 tile pulls 32 KB per 128-byte stage of K, and a work-group with one stage
+// What bounds such a launch (one work-group per CU) is what a CU takes in: a 128 x 128 tile pulls 32 KB per 128-byte stage of K, and a work-group with one stage
 // in flight gets 55 KB per us, with two or more 90 - 97 (direct loads alone, 256 work-groups, row pitches of 4 - 16 KB; one stage of
 // 256 rows on either side: 66 - 71).  So LDS is a ring of four stages: while stage s is multiplied, s + 1 has landed and s + 2 .. s + 3 or s + 4
 // (addr::ring_ahead) are on their way, and the waits count loads instead of draining them.
