@@ -160,3 +160,22 @@ def test_automatic_choice_takes_the_decode_kernel_and_no_workspace_is_needed_for
     finally:
         lib.tlq_tune_w4a16_decode(1)
     check_float_output(c, w4a16_reference(A, Wp, s, z, group), "skinny kernel with the decode kernel off")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16 * 255, 512), (16, 16 * 256 + 8, 4096), (5, 16 * 513 - 4, 3840), (16, 16 * 769, 4096), (16, 16 * 1024, 768), (11, 16 * 1024 + 16, 4096),
+                                   (16, 16 * 1281, 1024), (17, 16 * 1025, 4096), (16, 16 * 300, 8192)])
+@pytest.mark.parametrize("in_dtype", ["float16", "bfloat16"])
+def test_tiles_added_up_together_or_one_by_one(in_dtype, M, N, K):
+    """One to four tiles in a work-group, added up behind the last one, work-groups of four next to work-groups of five (256 CUs), which add theirs up one by
+    one, the last tile cut; sixteen wavefronts and fewer, several chunks of K."""
+    dt = DT[in_dtype]
+    print(f"decode tiles {in_dtype} M={M} N={N} K={K}", flush=True)
+    A = torch.randn(M, K, generator=gen(500 + M)).to(dt)
+    Wp, s, z = make_w4(N, K, 128, dt, "int", seed=501 + N)
+    want = w4a16_reference(A, Wp, s, z, 128)
+    check_float_output(run_decode(A, Wp, s, z, 128), want, f"{in_dtype} {M}x{N}x{K}")
+    hot = torch.zeros(M, K, dtype=dt)
+    rows = torch.arange(M) * (K // M)
+    hot[torch.arange(M), rows] = 1
+    assert_bit_equal(run_decode(hot, Wp, s, z, 128), ref.dequant_w4(Wp, s, z, 128, dt)[:, rows].t().contiguous(), "one-hot rows")

@@ -12,8 +12,8 @@
 //     values of the slice) and one dword gather each, by 16 to 64 lanes, for the scales and zero points of the 16 rows.
 //     Everything else in the loop is kept to a minimum: the kernel is bound by instruction issue (about 100
 //     instructions per 1 KB of packed weights, most of them the dequantisation).
-//   * Per tile the wavefronts' partial tiles meet in LDS (two buffers, one barrier per tile) and are added in
-//     wavefront order by a wavefront that rotates from tile to tile.
+//   * The wavefronts' partial tiles meet in LDS and are added in wavefront order: up to four tiles together at the end, else tile by tile (two
+//     buffers, one barrier per tile) by a wavefront that rotates from tile to tile.
 //
 // The dequantisation skips the four byte permutes per word that put a plain word's values back into k order (the
 // decode of expand8.h for interleaved words, applied to either layout): for plain words the activation operands are
@@ -121,8 +121,9 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
   // ---- activations of this wavefront's K slice -> MFMA operands in registers ----
   // Direct loads of 1 KB into the wavefront's own LDS, one [16 rows][256 B] block (4 KB) at a time, staged in the third
   // ring slot plus the partial-sum area (both idle yet): direct loads move twice as many bytes per clock as loads into
-  // registers, and every work-group has to pull all of A through its CU.  The first two tiles of weights are requested
-  // right behind the first block, so that HBM is busy while the activations (L2 hits) are rearranged.
+  // registers, and every work-group has to pull all of A through its CU.  A tile of weights is requested right behind either of the
+  // first two blocks, so that memory is busy while the activations (L2 hits) are rearranged.  (Both tiles behind the first block: the second
+  // block, and with it the third tile, waited for all of them, and the first wavefronts' requests for the last ones': 16 x 14336 x 4096 11.6 -> 11.3 us.)
   uint4_t af[2][4][MT];
   if (active) {
     constexpr uint32_t STG = 2 * SLOT;
@@ -140,17 +141,15 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
     };
     issue_block(0, 0);
     issue_tile(0);
-    if (my_tiles > 1) issue_tile(1);
 #pragma unroll
     for (int b = 0; b < 2 * MT; ++b) {
       const int kb = b / MT, mt = b % MT;
-      // loads return in issue order: the first block is followed by at most two tiles (eight loads), every later block
+      // loads return in issue order: the first two blocks are followed by a tile (four loads) each, every later block
       // is the youngest load there is
-      if (b == 0) {
-        if (my_tiles > 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      } else {
+      if (b == 0 || (b == 1 && my_tiles > 1))
+        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      else
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint4_t v = *(const uint4_t*)(mine + STG + addr::dec_a_frag(lane, j));
@@ -165,6 +164,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the staging area is free again: next block, or the third tile
       if (b + 1 < 2 * MT) issue_block((b + 1) / MT, (b + 1) % MT);
+      if (b == 0 && my_tiles > 1) issue_tile(1);
     }
     if (my_tiles > 2) issue_tile(2);
   }
@@ -173,9 +173,14 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = typename Mma::acc_t{0, 0, 0, 0};
 
+  // Up to four tiles of one activation tile are added up together behind the last one: a wavefront goes on to its next tile without waiting for the slowest
+  // of the others, which is 8000 cycles behind the first (16 x 14336 x 4096 bf16 12.1 -> 11.6 us).  Their third and fourth partial tiles lie in the slot
+  // of the second tile, which no load follows.
+  const bool at_once = MT == 1 && my_tiles <= 4;
+  static_assert(SLOT >= 2048, "two partial tiles in a slot");
+  auto part_at = [&](int i) { return (i < 2 ? RED : SLOT - 2048u) + (uint32_t)i * 1024u; };
   int turn = 0;  // ts MT modulo waves (waves >= MT)
   for (int ts = 0; ts < my_tiles; ++ts) {
-    const int t = first + ts * stride;
     if (active) {
       if (ts > 0 && ts + 2 < my_tiles) issue_tile(ts + 2);  // into the slot that tile ts - 1 was read from (tile 2: issued above)
       const uint8_t* const slotp = mine + (ts % TS) * SLOT;
@@ -201,7 +206,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
           ok = ok && zf == __builtin_rintf(zf) && zf >= -256.0f && zf <= 256.0f;
         }
         typename Mma::acc_t acc2[2] = {typename Mma::acc_t{0, 0, 0, 0}, typename Mma::acc_t{0, 0, 0, 0}};
-        if (__builtin_amdgcn_ballot_w64(ok) == ~0ull) {  // integer zero points fold into the unpack bias (exact)
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(ok) == ~0ull, 1)) {  // integer zero points fold into the unpack bias (exact)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -237,7 +242,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
           const float zf = to_float(zv);
           const bool ok = zf == __builtin_rintf(zf) && zf >= -256.0f && zf <= 256.0f;
           const uint32_t w[4] = {wf.x, wf.y, wf.z, wf.w};
-          if (__builtin_amdgcn_ballot_w64(ok) == ~0ull) {
+          if (__builtin_expect(__builtin_amdgcn_ballot_w64(ok) == ~0ull, 1)) {
             const Expand8<T, true, 1> ex(sv, zv, mg);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -259,34 +264,47 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
     }
     if (RB == 1 && ts > 0) __syncthreads();  // the single buffer: the wavefronts that added up tile ts - 1 have read it
     if (active) {
-      // partial tile of this wavefront -> its slot of buffer ts % RB
+      // partial tile of this wavefront -> its place, or buffer ts % RB
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        *(float4_t*)(mine + RED + ((ts % RB) * MT + mt) * 1024 + lane * 16) = acc[mt];
-      }
+      for (int mt = 0; mt < MT; ++mt) *(float4_t*)(mine + (at_once ? part_at(ts) : RED + ((ts % RB) * MT + mt) * 1024) + lane * 16) = acc[mt];
     }
+    if (at_once && ts + 1 < my_tiles) continue;
     __syncthreads();  // all partial tiles of tile t are in LDS (two buffers: the other one was read before the previous barrier)
     int rw = wave - turn;
     rw = rw < 0 ? rw + waves : rw;
     turn = turn + MT < waves ? turn + MT : turn + MT - waves;
-    if (rw < MT) {  // wavefronts turn .. turn + MT - 1 add up the MT activation tiles
-      const int mt = rw;
-      const uint32_t ro = RED + ((ts % RB) * MT + mt) * 1024 + lane * 16;
+    // wavefronts turn .. turn + MT - 1 add up the MT activation tiles, or a wavefront each of the tiles
+    for (int i = at_once ? wave : rw; i < (at_once ? my_tiles : MT); i += waves) {
+      const int mt = at_once ? 0 : i, t = first + (at_once ? i : ts) * stride;
+      const uint32_t ro = (at_once ? part_at(i) : RED + ((ts % RB) * MT + mt) * 1024) + lane * 16;
       float4_t sum = *(const float4_t*)(smem + ro);
-      for (int w = 1; w < n_active; ++w) sum += *(const float4_t*)(smem + w * WAVE + ro);
+      // (asked for all at once, or four at a time where the activations leave no registers for more: one by one 16 x 14336 x 4096 took 11.25 for 10.8 us, 32 rows
+      // 15.1 for 14.8)
+      int partials = n_active, cols = N;
+      asm volatile("" : "+s"(partials), "+s"(cols));  // (what is made of them stays behind the tiles: ahead of the first it is 60 instructions more to wait for)
+      if (MT == 1 && partials == 16) {
+        float4_t part[15];
+#pragma unroll
+        for (int w = 1; w < 16; ++w) part[w - 1] = *(const float4_t*)(smem + w * WAVE + ro);
+#pragma unroll
+        for (int w = 1; w < 16; ++w) sum += part[w - 1];
+      } else {
+#pragma unroll 4
+        for (int w = 1; w < partials; ++w) sum += *(const float4_t*)(smem + w * WAVE + ro);
+      }
       // lane l holds D[n = 4 (l / 16) + i][m = l % 16]
       const int m = mt * 16 + r16;
       const int n = t * 16 + 4 * q;
-      if (m < M && n < N) {
-        const int64_t idx = (int64_t)m * N + n;
+      if (m < M && n < cols) {
+        const int64_t idx = (int64_t)m * cols + n;
         if (partial) {
-          float* const P = partial + (int64_t)chunk * M * N;
-          if (n + 3 < N && (N & 3) == 0) {
+          float* const P = partial + (int64_t)chunk * M * cols;
+          if (n + 3 < cols && (cols & 3) == 0) {
             *(float4_t*)(P + idx) = sum;
           } else {
-            for (int i = 0; i < 4 && n + i < N; ++i) P[idx + i] = sum[i];
+            for (int e = 0; e < 4 && n + e < cols; ++e) P[idx + e] = sum[e];
           }
-        } else if (n + 3 < N && (N & 3) == 0) {
+        } else if (n + 3 < cols && (cols & 3) == 0) {
           if (out_dtype == TLQ_F32) {
             *(float4_t*)((float*)C + idx) = sum;
           } else if (out_dtype == TLQ_F16) {
@@ -296,7 +314,7 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
             *(uint2_t*)((uint16_t*)C + idx) = uint2_t{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
           }
         } else {
-          for (int i = 0; i < 4 && n + i < N; ++i) store_out(C, idx + i, sum[i], out_dtype);
+          for (int e = 0; e < 4 && n + e < cols; ++e) store_out(C, idx + e, sum[e], out_dtype);
         }
       }
     }
