@@ -243,7 +243,16 @@ __global__ __launch_bounds__(RT* MT <= 4 ? 1024 : 512) void gemm_small_kernel(Sm
   __syncthreads();
   for (int item = threadIdx.x; item < RT * MT * 64; item += waves * 64) {
     acc_t sum = red[item];
-    for (int w = 1; w < waves; ++w) sum += red[w * (RT * MT * 64) + item];
+    if (waves == 8) {  // (all asked for at once: one by one the reads wait for each other)
+      acc_t part[7];
+#pragma unroll
+      for (int w = 1; w < 8; ++w) part[w - 1] = red[w * (RT * MT * 64) + item];
+#pragma unroll
+      for (int w = 1; w < 8; ++w) sum += part[w - 1];
+    } else {
+#pragma unroll 4
+      for (int w = 1; w < waves; ++w) sum += red[w * (RT * MT * 64) + item];
+    }
     const int tile = item >> 6, l = item & 63;  // lane l of a tile holds C[m = l % 16][n = 4 (l / 16) .. + 3]
     const int rt = tile / MT, mt = tile - rt * MT;
     epi.store(m_base + mt * 16 + (l & 15), n_base + rt * 16 + 4 * (l >> 4), finished(sum), M, N);

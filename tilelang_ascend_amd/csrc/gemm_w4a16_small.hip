@@ -228,12 +228,15 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void w4a16_small_kernel(const
   __syncthreads();
   for (int item = threadIdx.x; item < RT * MT * 64; item += waves * 64) {
     float4_t sum = red[item];
-    for (int w = 1; w < waves; ++w) {
-      const float4_t v = red[w * (RT * MT * 64) + item];
-      sum[0] += v[0];
-      sum[1] += v[1];
-      sum[2] += v[2];
-      sum[3] += v[3];
+    if (waves == 8) {  // (all asked for at once: one by one the reads wait for each other)
+      float4_t part[7];
+#pragma unroll
+      for (int w = 1; w < 8; ++w) part[w - 1] = red[w * (RT * MT * 64) + item];
+#pragma unroll
+      for (int w = 1; w < 8; ++w) sum += part[w - 1];
+    } else {
+#pragma unroll 4
+      for (int w = 1; w < waves; ++w) sum += red[w * (RT * MT * 64) + item];
     }
     const int tile = item >> 6, l = item & 63;
     const int rt = tile / MT, mt = tile - rt * MT;
