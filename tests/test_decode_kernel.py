@@ -164,7 +164,8 @@ def test_automatic_choice_takes_the_decode_kernel_and_no_workspace_is_needed_for
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 16 * 255, 512), (16, 16 * 256 + 8, 4096), (5, 16 * 513 - 4, 3840), (16, 16 * 769, 4096), (16, 16 * 1024, 768), (11, 16 * 1024 + 16, 4096),
-                                   (16, 16 * 1281, 1024), (17, 16 * 1025, 4096), (16, 16 * 300, 8192)])
+                                   (16, 16 * 1281, 1024), (17, 16 * 1025, 4096), (16, 16 * 300, 8192), (32, 16 * 513 - 8, 4096),
+                                   (24, 16 * 1024, 512), (17, 16 * 769, 1024), (32, 16 * 300, 8192)])
 @pytest.mark.parametrize("in_dtype", ["float16", "bfloat16"])
 def test_tiles_added_up_together_or_one_by_one(in_dtype, M, N, K):
     """One to four tiles in a work-group, added up behind the last one, work-groups of four next to work-groups of five (256 CUs), which add theirs up one by

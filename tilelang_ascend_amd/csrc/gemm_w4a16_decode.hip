@@ -173,12 +173,54 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = typename Mma::acc_t{0, 0, 0, 0};
 
-  // Up to four tiles of one activation tile are added up together behind the last one: a wavefront goes on to its next tile without waiting for the slowest
-  // of the others, which is 8000 cycles behind the first (16 x 14336 x 4096 bf16 12.1 -> 11.6 us).  Their third and fourth partial tiles lie in the slot
-  // of the second tile, which no load follows.
-  const bool at_once = MT == 1 && my_tiles <= 4;
-  static_assert(SLOT >= 2048, "two partial tiles in a slot");
-  auto part_at = [&](int i) { return (i < 2 ? RED : SLOT - 2048u) + (uint32_t)i * 1024u; };
+  // Up to four tiles are added up together behind the last one: a wavefront goes on to its next tile without waiting for the slowest
+  // of the others, which is 8000 cycles behind the first (16 x 14336 x 4096 bf16 12.1 -> 11.6 us).  Partial tiles behind the first lie in the slot that
+  // theirs was read from, which no load follows.
+  const bool at_once = my_tiles <= 4;
+  static_assert(SLOT >= MT * 1024 && RB * MT == 2, "the partial tiles of a tile in a slot, or behind the ring");
+  auto part_at = [&](int ts, int mt) { return (ts == 0 ? RED : (uint32_t)(ts % TS) * SLOT) + (uint32_t)mt * 1024u + (uint32_t)lane * 16u; };
+  // Adds up the wavefronts' partial tiles at `ro` in their order, rows 16 mt .. of tile t, and stores them.
+  auto add_up = [&](int t, int mt, uint32_t ro, auto all_tag) {
+    float4_t sum = *(const float4_t*)(smem + ro);
+    // (asked for all at once, or four at a time where the activations leave no registers for more: one by one 16 x 14336 x 4096 took 11.25 for 10.8 us, 32 rows
+    // 15.1 for 14.8)
+    int partials = n_active, cols = N;
+    asm volatile("" : "+s"(partials), "+s"(cols));  // (what is made of them stays behind the tiles: ahead of the first it is 60 instructions more to wait for)
+    if (decltype(all_tag)::value && partials == 16) {
+      float4_t part[15];
+#pragma unroll
+      for (int w = 1; w < 16; ++w) part[w - 1] = *(const float4_t*)(smem + w * WAVE + ro);
+#pragma unroll
+      for (int w = 1; w < 16; ++w) sum += part[w - 1];
+    } else {
+#pragma unroll 4
+      for (int w = 1; w < partials; ++w) sum += *(const float4_t*)(smem + w * WAVE + ro);
+    }
+    // lane l holds D[n = 4 (l / 16) + i][m = l % 16]
+    const int m = mt * 16 + r16;
+    const int n = t * 16 + 4 * q;
+    if (m >= M || n >= cols) return;
+    const int64_t idx = (int64_t)m * cols + n;
+    if (partial) {
+      float* const P = partial + (int64_t)chunk * M * cols;
+      if (n + 3 < cols && (cols & 3) == 0) {
+        *(float4_t*)(P + idx) = sum;
+      } else {
+        for (int e = 0; e < 4 && n + e < cols; ++e) P[idx + e] = sum[e];
+      }
+    } else if (n + 3 < cols && (cols & 3) == 0) {
+      if (out_dtype == TLQ_F32) {
+        *(float4_t*)((float*)C + idx) = sum;
+      } else if (out_dtype == TLQ_F16) {
+        half_t h[4] = {(half_t)sum[0], (half_t)sum[1], (half_t)sum[2], (half_t)sum[3]};
+        *(uint2_t*)((half_t*)C + idx) = bitcast<uint2_t>(h);
+      } else {
+        *(uint2_t*)((uint16_t*)C + idx) = uint2_t{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+      }
+    } else {
+      for (int e = 0; e < 4 && n + e < cols; ++e) store_out(C, idx + e, sum[e], out_dtype);
+    }
+  };
   int turn = 0;  // ts MT modulo waves (waves >= MT)
   for (int ts = 0; ts < my_tiles; ++ts) {
     if (active) {
@@ -262,63 +304,23 @@ __global__ __launch_bounds__(1024) void w4a16_decode_kernel(const T* __restrict_
         }
       }
     }
-    if (RB == 1 && ts > 0) __syncthreads();  // the single buffer: the wavefronts that added up tile ts - 1 have read it
+    if (RB == 1 && ts > 0 && !at_once) __syncthreads();  // the single buffer: the wavefronts that added up tile ts - 1 have read it
     if (active) {
       // partial tile of this wavefront -> its place, or buffer ts % RB
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) *(float4_t*)(mine + (at_once ? part_at(ts) : RED + ((ts % RB) * MT + mt) * 1024) + lane * 16) = acc[mt];
+      for (int mt = 0; mt < MT; ++mt) *(float4_t*)(mine + (at_once ? part_at(ts, mt) : RED + ((ts % RB) * MT + mt) * 1024 + lane * 16)) = acc[mt];
     }
-    if (at_once && ts + 1 < my_tiles) continue;
+    if (at_once) continue;
     __syncthreads();  // all partial tiles of tile t are in LDS (two buffers: the other one was read before the previous barrier)
     int rw = wave - turn;
     rw = rw < 0 ? rw + waves : rw;
     turn = turn + MT < waves ? turn + MT : turn + MT - waves;
-    // wavefronts turn .. turn + MT - 1 add up the MT activation tiles, or a wavefront each of the tiles
-    for (int i = at_once ? wave : rw; i < (at_once ? my_tiles : MT); i += waves) {
-      const int mt = at_once ? 0 : i, t = first + (at_once ? i : ts) * stride;
-      const uint32_t ro = (at_once ? part_at(i) : RED + ((ts % RB) * MT + mt) * 1024) + lane * 16;
-      float4_t sum = *(const float4_t*)(smem + ro);
-      // (asked for all at once, or four at a time where the activations leave no registers for more: one by one 16 x 14336 x 4096 took 11.25 for 10.8 us, 32 rows
-      // 15.1 for 14.8)
-      int partials = n_active, cols = N;
-      asm volatile("" : "+s"(partials), "+s"(cols));  // (what is made of them stays behind the tiles: ahead of the first it is 60 instructions more to wait for)
-      if (MT == 1 && partials == 16) {
-        float4_t part[15];
-#pragma unroll
-        for (int w = 1; w < 16; ++w) part[w - 1] = *(const float4_t*)(smem + w * WAVE + ro);
-#pragma unroll
-        for (int w = 1; w < 16; ++w) sum += part[w - 1];
-      } else {
-#pragma unroll 4
-        for (int w = 1; w < partials; ++w) sum += *(const float4_t*)(smem + w * WAVE + ro);
-      }
-      // lane l holds D[n = 4 (l / 16) + i][m = l % 16]
-      const int m = mt * 16 + r16;
-      const int n = t * 16 + 4 * q;
-      if (m < M && n < cols) {
-        const int64_t idx = (int64_t)m * cols + n;
-        if (partial) {
-          float* const P = partial + (int64_t)chunk * M * cols;
-          if (n + 3 < cols && (cols & 3) == 0) {
-            *(float4_t*)(P + idx) = sum;
-          } else {
-            for (int e = 0; e < 4 && n + e < cols; ++e) P[idx + e] = sum[e];
-          }
-        } else if (n + 3 < cols && (cols & 3) == 0) {
-          if (out_dtype == TLQ_F32) {
-            *(float4_t*)((float*)C + idx) = sum;
-          } else if (out_dtype == TLQ_F16) {
-            half_t h[4] = {(half_t)sum[0], (half_t)sum[1], (half_t)sum[2], (half_t)sum[3]};
-            *(uint2_t*)((half_t*)C + idx) = bitcast<uint2_t>(h);
-          } else {
-            *(uint2_t*)((uint16_t*)C + idx) = uint2_t{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
-          }
-        } else {
-          for (int e = 0; e < 4 && n + e < cols; ++e) store_out(C, idx + e, sum[e], out_dtype);
-        }
-      }
-    }
+    // wavefronts turn .. turn + MT - 1 add up the MT activation tiles
+    if (rw < MT) add_up(first + ts * stride, rw, RED + ((ts % RB) * MT + rw) * 1024 + lane * 16, std::integral_constant<bool, MT == 1>{});
   }
+  if (!at_once) return;
+  __syncthreads();
+  for (int i = wave; i < my_tiles * MT; i += waves) add_up(first + i / MT * stride, i % MT, part_at(i / MT, i % MT), std::true_type{});
 }
 
 }  // namespace
