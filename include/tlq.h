@@ -191,8 +191,8 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
  * any of these on problems that leave the others' tiles few or short, by estimates of both.
  * algo: as tlq_gemm_w4a16, or a family that only this entry point has (TLQ_ALGO_TWO_PASS, _STREAM, _PANEL, _PANEL256, _PANELM).
  * With TLQ_ALGO_AUTO and more than 512 rows, a row count that is no multiple of four runs in one launch of the small-tile kernel or in
- * the two passes where their estimates say so; otherwise as two calls on the stream: the multiple of four below (the panel kernels
- * take such counts only), then the last one to three rows.  Always as two calls where those last rows, run by themselves, go to the
+ * the two passes where their estimates say so; otherwise as two calls on the stream: the multiple of four below, then the last one to
+ * three rows -- bfloat16 rows that lie in the last tile of the first call's kernel go along with it.  Always as two calls where those last rows, run by themselves, go to the
  * fp16 GEMV kernels: they apply scale and zero point to fp32 sums of exact products, and their rows are the only ones of the
  * result whose weights are not rounded to in_dtype.
  * One scale / zero point per weight row (group == K) on rows whose length is no power of two: the kernels over K slices take

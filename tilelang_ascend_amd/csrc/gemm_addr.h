@@ -348,10 +348,12 @@ constexpr uint32_t kPanel2ATile = 16 * kPanel2TM * 256;
 constexpr uint32_t kPanel2Slot = kPanel2ATile + 4 * kPanel2TN * 1024;
 __host__ __device__ inline uint32_t panel2_a_lds(int wave, int j) { return (uint32_t)(j * 4 + wave) * 1024u; }
 __host__ __device__ inline uint32_t panel2_w_lds(int wave, int tn) { return kPanel2ATile + (uint32_t)(wave * kPanel2TN + tn) * 1024u; }
-__host__ __device__ inline int64_t panel2_a_block(int wave, int j, int m0, int M, int K) {
-  int m = m0 + 4 * (j * 4 + wave);
-  m = m + 4 <= M ? m : M - 4;
-  return (int64_t)m * K * 2;
+// Blocks of four rows past the matrix repeat its last, whose lanes past row M - 1 fetch that row.  (Both lane parts are the same for every load, so that a
+// load costs the choice between them.)
+__host__ __device__ inline uint32_t panel2_a_voff(int lane, int wave, int j, int m0, int M, int K) {
+  const int last = (M - 1) & ~3, m = m0 + 4 * (j * 4 + wave) < last ? m0 + 4 * (j * 4 + wave) : last;
+  const int in_last = (lane >> 4) < M - 1 - last ? lane >> 4 : M - 1 - last;
+  return (uint32_t)((int64_t)m * K * 2) + (m + 4 <= M ? panel_a_lane(lane, K) : panel_a_lane(in_last << 4, K)) + panel_a_chunk(lane, wave);
 }
 // byte offsets into a scale / zero-point tensor [N][groups] of 2-byte values: row block of the tile (uniform), the group of
 // step `step` of the matrix (uniform), the lane's row and -- for groups of fewer than 128 values -- its k-group's group

@@ -648,7 +648,7 @@ int check_panel(int64_t M, int64_t N, int64_t K, int64_t group, int slice_steps)
 // activation, weight and scale loads over every step of every slice (and of the steps past the end, which repeat the
 // last), LDS extents and coverage of a slot, agreement of the landing cells with the operand reads.
 int check_panel256(int64_t M, int64_t N, int64_t K, int64_t group, int slice_steps) {
-  CHECK_OR_FAIL(M >= 4 && N >= 16 && M % 4 == 0 && N % 16 == 0 && K >= 128 && K % 128 == 0, "panel256: bad shape");
+  CHECK_OR_FAIL(M >= 1 && N >= 16 && N % 16 == 0 && K >= 128 && K % 128 == 0, "panel256: bad shape");
   CHECK_OR_FAIL(group >= 32 && (group & (group - 1)) == 0 && K % group == 0, "panel256: group %lld on K %lld", (long long)group, (long long)K);
   const int64_t groups = K / group;
   int gshift = 0;
@@ -670,14 +670,14 @@ int check_panel256(int64_t M, int64_t N, int64_t K, int64_t group, int slice_ste
           const uint32_t l0 = addr::panel2_a_lds(wave, j);
           const int I = j * 4 + wave;
           for (int lane = 0; lane < 64; ++lane) {
-            const int64_t voff = addr::panel2_a_block(wave, j, (int)m0, (int)M, (int)K) + addr::panel_a_lane(lane, (int)K) + addr::panel_a_chunk(lane, wave);
+            const int64_t voff = addr::panel2_a_voff(lane, wave, j, (int)m0, (int)M, (int)K);
             CHECK_OR_FAIL(voff >= 0 && voff + (int64_t)(steps_total - 1) * 256 + 16 <= a_extent, "panel256: activation load at %lld of %lld",
                           (long long)voff, (long long)a_extent);
             const uint32_t at = l0 / 16 + lane;
             CHECK_OR_FAIL(at < addr::kPanel2ATile / 16 && cell[at] == -1, "panel256: activation cell %u written twice or outside the tile", at);
             const int row = addr::sa_row(lane, I), chunk = addr::sa_chunk(lane, I);
             CHECK_OR_FAIL((int)at == row * 16 + (lane & 15), "panel256: activation lane lands on cell %u, not on its row", at);
-            if (m0 + 4 * I + 4 <= M)
+            if (m0 + row < M)
               CHECK_OR_FAIL(voff == ((int64_t)(m0 + row) * K) * 2 + chunk * 16, "panel256: activation lane %d of load %d fetches the wrong bytes", lane, I);
             cell[at] = row * 16 + chunk;
           }
@@ -733,7 +733,7 @@ int check_panel256(int64_t M, int64_t N, int64_t K, int64_t group, int slice_ste
 // landing cells with the operand reads.
 int check_panelm(int64_t M, int64_t N, int64_t K, int64_t group, int tm, int slice_steps) {
   CHECK_OR_FAIL(tm == 4 || tm == 8, "panelm: %d activation tiles per work-group", tm);
-  CHECK_OR_FAIL(M >= 4 && N >= 16 && M % 4 == 0 && N % 16 == 0 && K >= 128 && K % 128 == 0, "panelm: bad shape");
+  CHECK_OR_FAIL(M >= 1 && N >= 16 && N % 16 == 0 && K >= 128 && K % 128 == 0, "panelm: bad shape");
   CHECK_OR_FAIL(group >= 32 && (group & (group - 1)) == 0 && K % group == 0 && (K / group) % 8 == 0, "panelm: group %lld on K %lld",
                 (long long)group, (long long)K);
   const int64_t groups = K / group;
@@ -758,14 +758,14 @@ int check_panelm(int64_t M, int64_t N, int64_t K, int64_t group, int tm, int sli
           const uint32_t l0 = addr::panel2_a_lds(wave, j);
           const int I = j * 4 + wave;
           for (int lane = 0; lane < 64; ++lane) {
-            const int64_t voff = addr::panel2_a_block(wave, j, (int)m0, (int)M, (int)K) + addr::panel_a_lane(lane, (int)K) + addr::panel_a_chunk(lane, wave);
+            const int64_t voff = addr::panel2_a_voff(lane, wave, j, (int)m0, (int)M, (int)K);
             CHECK_OR_FAIL(voff >= 0 && voff + (int64_t)(steps_total - 1) * 256 + 16 <= a_extent, "panelm: activation load at %lld of %lld",
                           (long long)voff, (long long)a_extent);
             const uint32_t at = l0 / 16 + lane;
             CHECK_OR_FAIL(at < a_tile / 16 && cell[at] == -1, "panelm: activation cell %u written twice or outside the tile", at);
             const int row = addr::sa_row(lane, I), chunk = addr::sa_chunk(lane, I);
             CHECK_OR_FAIL((int)at == row * 16 + (lane & 15), "panelm: activation lane lands on cell %u, not on its row", at);
-            if (m0 + 4 * I + 4 <= M)
+            if (m0 + row < M)
               CHECK_OR_FAIL(voff == ((int64_t)(m0 + row) * K) * 2 + chunk * 16, "panelm: activation lane %d of load %d fetches the wrong bytes", lane, I);
             cell[at] = row * 16 + chunk;
           }

@@ -712,9 +712,9 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 // 35 us in a launch for 1000 rows and one for three, 29 in the two passes.)  Where neither panel kernel would run, all rows go through the two passes and none is left over.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
 static double two_passes_us(int64_t M, int64_t N, int64_t K) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(M, N, K); }
-static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
+static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group, bool rest_goes_along) {
   static thread_local PlanTable<bool> known;
-  return known.get(M, N, K, group, [&] {
+  return known.get(M, N, K, group * 2 + rest_goes_along, [&] {
     const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
     const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
     const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
@@ -729,8 +729,11 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
       return true;
     const double best = 2.0 * (double)M * (double)N * (double)K / 1.38e9;  // at 1.38 PFLOP/s
     panels = panels / 1.21 > best ? panels / 1.21 : best;
-    const double two = two_passes_us(M, N, K), with_rest = panels + (head != M ? 4.5 : 0.0);
-    return middle ? two < (head != M ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 0.95 : 1.07) * with_rest;
+    // (rows that go along cost no launch.  Above 2048 rows they are counted as one all the same: the panels' estimate is low there, 7 problems of 12 that not counting
+    // it moves are 1 - 13 % slower; up to 2048 rows all 16 are faster, 1.01 - 1.18 x, 518 x 7440 x 1024 24.5 -> 16.4 us)
+    const bool rest = head != M && !(rest_goes_along && M <= 2048 && ceil_div(head, (int64_t)(middle ? 128 : 256)) == ceil_div(M, (int64_t)(middle ? 128 : 256)));
+    const double two = two_passes_us(M, N, K), with_rest = panels + (rest ? 4.5 : 0.0);
+    return middle ? two < (rest ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 0.95 : 1.07) * with_rest;
   });
 }
 // Many rows on up to 2^19 weights: the two passes or the tile kernel in one launch.  27 problems above 512 rows where that ran: 13 go to the two passes, 1.28 x
@@ -780,6 +783,12 @@ static bool stream_args_ok(const void* A, const void* w_packed, const void* scal
          ((uintptr_t)zeros & 1) == 0 && K > 0 && fits32(M, K * 2) && fits32(N, K / 2);
 }
 
+// The one to three rows of the same matrices behind the M (a multiple of four) that the automatic choice is called for: the four-wavefront panel kernels and the streaming kernel take them along
+// where they lie in the last of the tiles that M rows take anyway, and set this to zero.  (One tile row more would cost a round where the head's tiles fill
+// the machine: 4097 x 4096 x 4096 runs 4096 rows in one round and the last row by itself.)
+static thread_local int64_t g_rows_behind = 0;
+static int64_t with_rows_behind(int64_t M, int64_t tile) { return ceil_div(M, tile) == ceil_div(M + g_rows_behind, tile) ? M + g_rows_behind : M; }
+
 // The panel kernel (large M, one launch, weights dequantised on the operand read).  Returns -1 when it does not take the
 // problem (nothing launched, no error set), else the launch's return code.
 static int try_panel(const void* A, const void* w_packed, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
@@ -808,14 +817,17 @@ static int try_panel256(const void* A, const void* w_packed, const void* scales,
   if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return -1;
   const Panel2Plan pp = w4a16_panel256_plan(M, N, K, group, cu_count_or_default());
   if (!pp.ok) return -1;
+  int64_t rows = with_rows_behind(M, 256);
+  auto need = [&] { return pp.split > 1 ? (int64_t)pp.split * rows * N * 4 : (int64_t)0; };
+  if (need() > workspace_bytes || !fits32(rows, K * 2)) rows = M;
   const bool args_ok = A && w_packed && C && aligned16(A) && aligned16(w_packed) && aligned16(C) && ((uintptr_t)scales & 1) == 0 &&
                        ((uintptr_t)zeros & 1) == 0 && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
                        (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) && (M * N) % 4 == 0 &&
                        fits32(M, K * 2) && fits32(N, K / 2) && fits32(N, (K / group) * 2);
   if (!args_ok) return -1;
-  const int64_t need = pp.split > 1 ? (int64_t)pp.split * M * N * 4 : 0;
-  if (need > 0 && !(workspace && aligned16(workspace) && workspace_bytes >= need)) return -1;
-  return gemm_w4a16_panel256(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, pp,
+  if (need() > 0 && !(workspace && aligned16(workspace) && workspace_bytes >= need())) return -1;
+  if (rows != M) g_rows_behind = 0;
+  return gemm_w4a16_panel256(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, pp,
                              (float*)workspace, (hipStream_t)stream);
 }
 
@@ -826,14 +838,17 @@ static int try_panelm(const void* A, const void* w_packed, const void* scales, c
   if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return -1;
   const PanelMPlan pp = w4a16_panelm_plan(M, N, K, group, cu_count_or_default());
   if (!pp.ok) return -1;
+  int64_t rows = with_rows_behind(M, 16 * pp.tm);
+  auto need = [&] { return pp.split > 1 ? (int64_t)pp.split * rows * N * 4 : (int64_t)0; };
+  if (need() > workspace_bytes || !fits32(rows, K * 2)) rows = M;
   const bool args_ok = A && w_packed && C && aligned16(A) && aligned16(w_packed) && aligned16(C) && aligned16(scales) &&
                        aligned16(zeros) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
                        (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) && (M * N) % 4 == 0 &&
                        fits32(M, K * 2) && fits32(N, K / 2) && fits32(N, (K / group) * 2);
   if (!args_ok) return -1;
-  const int64_t need = pp.split > 1 ? (int64_t)pp.split * M * N * 4 : 0;
-  if (need > 0 && !(workspace && aligned16(workspace) && workspace_bytes >= need)) return -1;
-  return gemm_w4a16_panelm(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, pp, (float*)workspace,
+  if (need() > 0 && !(workspace && aligned16(workspace) && workspace_bytes >= need())) return -1;
+  if (rows != M) g_rows_behind = 0;
+  return gemm_w4a16_panelm(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype, pp, (float*)workspace,
                            (hipStream_t)stream);
 }
 
@@ -948,7 +963,9 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // more instead of the two passes for everything (measured: M = 1001, N = 14336, K = 4096: 147 us in one piece, 128 us for
   // 1000 rows; M = 2049, N = K = 8192: 392 against 249 us; M = 601, N = K = 8192: 164 against 120 us; the tail takes 6 - 15 us).
   // One launch or two passes for all rows instead, where their estimates say so -- but not where the last rows belong to the fp16
-  // GEMV kernels, whose results are closer to exact arithmetic.
+  // GEMV kernels, whose results are closer to exact arithmetic.  bfloat16 rows, which every kernel multiplies by the same rounded weights, go along
+  // with the head where they lie in its last tile (with_rows_behind): 45 of 111 problems, 1.03 - 1.24 x (1002 x 8960 x 1152 37.7 -> 32.8 us, 3999 x 4096 x
+  // 4096 117.3 -> 111.9, 1207 x 1024 x 6144 36.2 -> 29.2), none slower.
   const bool head_and_tail = algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && (M & 3) != 0 && M < kMaxDim && N >= 16 && N % 16 == 0 &&
                              N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && C && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
                              (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) &&
@@ -977,7 +994,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // (the estimate first: it is kept per shape, the choice among the others is not and takes 1.8 us of host time)
   if (M > 512 && stream_region && (stream_region = g_stream_tiles > 0 || stream_beats_panels(M, N, K, group))) {
     const int64_t head = M & ~(int64_t)3;
-    const bool two = room_for_two_passes && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
+    const bool two = room_for_two_passes && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
     stream_region = two ? N % 128 == 0 && N > 256 : !head_and_tail;
   }
   if (stream_region) {
@@ -985,7 +1002,9 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     // (129 .. 512 rows where the 256-row kernel's estimate is ahead: on short rows of wide matrices, 472 x 20352 x 1152 in groups of 32 32.0 against
     // 39.7 us, 316 x 24960 x 256 16.8 against 20.2; it runs further down)
     const bool panel = M <= 512 && !g_w4a16_panel && panel256_beats_stream(M, N, K, group, sp);
-    if (!panel && stream_workspace_ok(sp, M, N, workspace, workspace_bytes) && stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype)) {
+    int64_t rows = sp.ok ? with_rows_behind(M, 16 * sp.tm) : M;
+    if (!stream_workspace_ok(sp, rows, N, workspace, workspace_bytes) || !fits32(rows, K * 2)) rows = M;
+    if (!panel && stream_workspace_ok(sp, rows, N, workspace, workspace_bytes) && stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype)) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       // (96 rows and more on short rows, one round of 128 x 128 tiles: the tile kernel, 4.5 us + 1.45 us per 128 values of K -- 264 x 7168 x 256
       // 6.8 against 9.2 us; and, which the tests of the choice ask for, a round that is nearly full, up to 1024 values: 512 x 8192 x 1024
@@ -998,15 +1017,20 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       if (M <= 512 && small_beats_stream(small, sp, M, N, K, group, zeros != nullptr))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
-      return gemm_w4a16_stream(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, sp, (float*)workspace,
+      if (rows != M) g_rows_behind = 0;
+      return gemm_w4a16_stream(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, sp, (float*)workspace,
                                (hipStream_t)stream);
     }
   }
-  if (head_and_tail && (keep_tail || !(room_for_two_passes && two_passes_beat_panels(M, N, K, group)))) {
+  if (head_and_tail && (keep_tail || !(room_for_two_passes && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16)))) {
     const int64_t head = M & ~(int64_t)3;
+    const bool may_go_along = in_dtype == TLQ_BF16;
+    g_rows_behind = may_go_along ? M - head : 0;
     const int rc = tlq_gemm_w4a16_ws(A, w_packed, scales, zeros, C, head, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, workspace,
                                      workspace_bytes, stream);
-    if (rc != 0) return rc;
+    const bool went_along = may_go_along && g_rows_behind == 0;
+    g_rows_behind = 0;
+    if (rc != 0 || went_along) return rc;
     const int64_t out_bytes = out_dtype == TLQ_F32 ? 4 : 2;
     return tlq_gemm_w4a16((const uint8_t*)A + head * K * 2, w_packed, scales, zeros, (uint8_t*)C + head * N * out_bytes, M - head, N, K, group,
                           zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, stream);
@@ -1173,7 +1197,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // 1.50 - 1.56 x), 0.98 - 0.99 on a few of the largest fp16 problems -- and 2 - 21 % behind below that fill (N = K = 4096,
   // M <= 1024: 96 work-groups).  The 128-row kernel is ahead of it nowhere by more than 4 % and stays an explicit choice.
   if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && K > 0 && group > 0 && N >= 1 && N < kMaxDim && K < kMaxDim && M < kMaxDim &&
-      !(have && two_passes_beat_panels(M, N, K, group))) {
+      !(have && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16))) {
     // The middle-M kernel's 128-row tiles first where an estimate of both kernels' times says so: rounds of work-groups x
     // (steps per K slice x the time of a step + a fixed part) + the pass over the slices' partial tiles, with the step
     // times measured at a full machine (2.2 us on 128 rows, 3.3 us on 256) and fixed parts of 6 / 8 us.  On ten (N, K)

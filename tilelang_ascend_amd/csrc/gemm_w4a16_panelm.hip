@@ -97,12 +97,12 @@ __global__ __launch_bounds__(256, 1) void w4a16_panelm_kernel(const T* __restric
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr_t)smem);
 
   // ---- sources of the direct loads: the row block of every load instruction sits in the lane offset (16 weight rows or 4
-  // activation rows per instruction; N % 16 == 0 and M % 4 == 0, blocks past a matrix repeat its last; a matrix spans less
+  // activation rows per instruction; N % 16 == 0, blocks past a matrix repeat its last, activation rows past it its last row; a matrix spans less
   // than 4 GiB), so that a step's loads share one scalar base.
   uint32_t voff_a[TM], voff_w[TN];
 #pragma unroll
   for (int j = 0; j < TM; ++j)
-    voff_a[j] = (uint32_t)addr::panel2_a_block(wave, j, m0, M, K) + addr::panel_a_lane(lane, K) + addr::panel_a_chunk(lane, wave);
+    voff_a[j] = addr::panel2_a_voff(lane, wave, j, m0, M, K);
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn) voff_w[tn] = (uint32_t)addr::panel_w_block(wave, tn, n0, N, K) + addr::panel_w_lane(lane, K);
   const uint32_t voff_sc = addr::panel_sc_voff(lane, wave, n0, N, groups);
