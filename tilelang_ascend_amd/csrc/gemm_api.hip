@@ -470,8 +470,12 @@ static int64_t w4a16_partial_sum_bytes(int64_t M, int64_t N, int64_t K, bool lea
   return split > 1 ? split * M * N * 4 : 0;
 }
 
+// The four-wavefront panel kernels take any row count: rows past the matrix repeat its last.  Asked for by name they take multiples of four, as they
+// always did, and above 512 rows the automatic choice calls them for those (with_rows_behind); up to 512 rows it plans for the next one.
+static int64_t whole_fours(int64_t M) { return (M + 3) & ~(int64_t)3; }
+
 // what the panel kernel may ask of the workspace for any group size: the partial tiles of its K slices and the flag word
-static int64_t panel_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+static int64_t panel_workspace_bytes(int64_t M, int64_t N, int64_t K, bool any_rows = false) {
   if (!(M >= 1 && N >= 1 && K > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return 0;
   int64_t need = 0;
   for (int64_t group = 32; group <= 1024; group *= 2) {
@@ -481,9 +485,9 @@ static int64_t panel_workspace_bytes(int64_t M, int64_t N, int64_t K) {
       const int64_t b = (pp.split > 1 ? (int64_t)pp.split * M * N * 4 : 0) + 16;
       if (b > need) need = b;
     }
-    const Panel2Plan p2 = w4a16_panel256_plan(M, N, K, group, cu_count_or_default());
+    const Panel2Plan p2 = w4a16_panel256_plan(any_rows ? whole_fours(M) : M, N, K, group, cu_count_or_default());
     if (p2.ok) {
-      const int64_t b = (p2.split > 1 ? (int64_t)p2.split * M * N * 4 : 0) + 16;
+      const int64_t b = (p2.split > 1 ? (int64_t)p2.split * M * N * 4 : 0) + (M % 4 == 0 ? 16 : 0);  // (the word is the 128-row kernel's)
       if (b > need) need = b;
     }
   }
@@ -491,12 +495,12 @@ static int64_t panel_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 }
 
 // the same for the middle-M panel kernel
-static int64_t panelm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+static int64_t panelm_workspace_bytes(int64_t M, int64_t N, int64_t K, bool any_rows = false) {
   if (!(M >= 1 && N >= 1 && K > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return 0;
   int64_t need = 0;
   for (int64_t group = 32; group <= 1024; group *= 2) {
     if (K % group != 0) continue;
-    const PanelMPlan pm = w4a16_panelm_plan(M, N, K, group, cu_count_or_default());
+    const PanelMPlan pm = w4a16_panelm_plan(any_rows ? whole_fours(M) : M, N, K, group, cu_count_or_default());
     if (pm.ok && pm.split > 1 && (int64_t)pm.split * M * N * 4 > need) need = (int64_t)pm.split * M * N * 4;
   }
   return need;
@@ -599,11 +603,11 @@ static int64_t w4a16_kernel_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     }
   }
   if (panelm_preferred(M, N, K) || panelm_one_tile(M, N, K) || M > 512 || (M >= 196 && N * K >= ((int64_t)1 << 25))) {  // (above 512 rows: where its estimate beats the 256-row kernel's)
-    const int64_t pm = panelm_workspace_bytes(M, N, K);
+    const int64_t pm = panelm_workspace_bytes(M, N, K, M <= 512);
     if (pm > need) need = pm;
   }
   if (M > 128 || panelm_preferred(M, N, K) || panel_one_round(M, N, K)) {  // (129 .. 512 rows: where the 256-row kernel's estimate beats the middle-M or the streaming kernel's)
-    const int64_t pn = panel_workspace_bytes(M, N, K);
+    const int64_t pn = panel_workspace_bytes(M, N, K, M <= 512);
     if (pn > need) need = pn;
   }
   // two passes (which of the two is taken depends on the group size, so the size covers both): the dequantised matrix,
@@ -643,8 +647,8 @@ static bool panelm_estimate_wins(int64_t M, int64_t N, int64_t K, int64_t group)
 // 256 .. 512 rows: does the 256-row kernel beat the middle-M kernel by the same estimate?
 static bool panel256_estimate_wins(int64_t M, int64_t N, int64_t K, int64_t group) {
   const int64_t cus_now = cu_count_or_default();
-  const PanelMPlan pm = w4a16_panelm_plan(M, N, K, group, (int)cus_now);
-  const Panel2Plan p2 = w4a16_panel256_plan(M, N, K, group, (int)cus_now);
+  const PanelMPlan pm = w4a16_panelm_plan(whole_fours(M), N, K, group, (int)cus_now);
+  const Panel2Plan p2 = w4a16_panel256_plan(whole_fours(M), N, K, group, (int)cus_now);
   if (!pm.ok || !p2.ok) return false;
   const double est_m = panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, pm.tm == 8 ? 2.2 : 1.8, 6.0, M, N, cus_now);
   const double est_2 = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, M, N, cus_now);
@@ -666,25 +670,40 @@ static bool panelm_whole_rounds(int64_t M, int64_t N, int64_t K, int64_t group, 
   return !sp.ok || 0.87 * panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, 2.2, 6.0, M, N, cus_now) < 1.02 * sp.us;
 }
 
-// 129 .. 512 rows: does the 256-row kernel beat the streaming kernel?  It matters where the middle-M kernel does not take K (group
-// counts that are no multiple of eight) and four blocks of 128 rows meet two tiles of 256.  Two prices of the streaming kernel:
-//   * Blocks of 256 weight rows (two groups of wavefronts): rounds x (2.2 us a step of 128 rows, 1.75 of 96, + 8), bar 0.95: 448 x 5120 x
-//     13824 82 against 80 - 84 us, 448 x 18944 x 3584 82 against 100, 144 x 50304 x 4096 in two blocks of 96 rows.
-//   * Blocks of 128 weight rows (four groups) make twice the work-groups at a third of that time a step: by the plan's own estimate, with
-//     the 256-row kernel's at 0.9 (it is 18 % high at the median).  On 434 problems (groups of 32 - 1024, both types) 0.1 % behind the faster
-//     kernel on average, more than 3 % on 6; the price above sent 256 x 11008 x 5504 (44 against 71 us), 512 x 4096 x 11008 (61 against 72)
-//     and 165 others to the slower one (1.11 x on average).  The 256-row kernel is ahead from some 400 rows on 6000 x 12000 on: 512 x 6144 x 14720 88 against 105 us.
+// 129 .. 512 rows: does the 256-row kernel beat the streaming kernel?  By the estimates of both, the panel kernel's at 0.94 (it is 15 % high, the streaming kernel's 2 %):
+// 0.2 % behind the faster of the two on average on 370 problems (matrices of 2^25 - 3e8 weights, groups of 64 and 128, both types).  Between 0.97 and 1.06, and
+// on matrices beyond those, row counts that are no multiple of four stay with the streaming kernel, the others go by its older price, rounds x (2.2 us a step of
+// 128 rows, 1.75 of 96, + 8) for blocks of 256 weight rows (by that price alone 0.6 % behind: 468 x 16768 x 12288 291 -> 241 us, 288 x 26448 x 9216 227 -> 198).
+// 423 x 27904 x 6528 in groups of 32 238 -> 176, 459 x 27136 x 4736 151 -> 127.
 static bool panel256_beats_stream(int64_t M, int64_t N, int64_t K, int64_t group, const StreamPlan& sp) {
   if (M <= 128 || !sp.ok || (sp.tm != 8 && sp.tm != 6)) return false;
   static thread_local PlanTable<bool> known;
   return known.get(M, N, K, group, [&] {
     const int64_t cus_now = cu_count_or_default();
-    const Panel2Plan p2 = w4a16_panel256_plan(M, N, K, group, (int)cus_now);
+    const Panel2Plan p2 = w4a16_panel256_plan(whole_fours(M), N, K, group, (int)cus_now);
     if (!p2.ok) return false;
     const double est_2 = panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, M, N, cus_now);
+    if (0.94 * est_2 < 0.97 * sp.us) return true;
+    if (M % 4 != 0 || (0.94 * est_2 > 1.06 * sp.us && N * K <= 300000000 && N <= 32768)) return false;
     if (sp.kg == 4) return 0.9 * est_2 < sp.us;
-    const double est_s = panel_estimate_us(sp.m_blocks, sp.n_blocks, sp.split, sp.slice_steps, sp.tm == 8 ? 2.2 : 1.75, 8.0, M, N, cus_now);
-    return est_2 < 0.95 * est_s;
+    return est_2 < 0.95 * panel_estimate_us(sp.m_blocks, sp.n_blocks, sp.split, sp.slice_steps, sp.tm == 8 ? 2.2 : 1.75, 8.0, M, N, cus_now);
+  });
+}
+
+// Where panelm_preferred speaks for the middle-M and the 256-row kernel: does the streaming kernel beat both?  By the estimates, the middle-M kernel's at 0.86 (it is
+// 26 % high) and with the same distances: of 30 such problems 14 were 3 % and more behind without this question (288 x 5376 x 13312 71.2 against 54.1 us, 308 x 14720 x
+// 4096 56.7 against 50.8).  Up to 256 binary16 rows, a multiple of four, the middle-M kernel stays (the test of the choice names it: 256 x 14336 x 4096 43.7 against
+// 36.4 us).
+static bool stream_beats_middle(int64_t M, int64_t N, int64_t K, int64_t group, int in_dtype, const StreamPlan& sp) {
+  if (!sp.ok || !g_w4a16_stream || (M <= 256 && M % 4 == 0 && in_dtype == TLQ_F16)) return false;
+  static thread_local PlanTable<bool> known;
+  return known.get(M, N, K, group, [&] {
+    const int64_t cus_now = cu_count_or_default();
+    const double bar = (M % 4 == 0 ? 1.06 : 0.97) * sp.us;
+    const PanelMPlan pm = w4a16_panelm_plan(whole_fours(M), N, K, group, (int)cus_now);
+    const Panel2Plan p2 = w4a16_panel256_plan(whole_fours(M), N, K, group, (int)cus_now);
+    if (pm.ok && 0.86 * panel_estimate_us(pm.tiles_m, pm.tiles_n, pm.split, pm.slice_steps, pm.tm == 8 ? 2.2 : 1.8, 6.0, M, N, cus_now) < bar) return false;
+    return !(p2.ok && 0.94 * panel_estimate_us(p2.tiles_m, p2.tiles_n, p2.split, p2.slice_steps, 3.3, 8.0, M, N, cus_now) < bar);
   });
 }
 
@@ -813,9 +832,9 @@ static int try_panel(const void* A, const void* w_packed, const void* scales, co
 // The 256-row panel kernel: the same contract.
 static int try_panel256(const void* A, const void* w_packed, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                         int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int w_layout, void* workspace,
-                        int64_t workspace_bytes, void* stream) {
+                        int64_t workspace_bytes, void* stream, bool any_rows = false) {
   if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return -1;
-  const Panel2Plan pp = w4a16_panel256_plan(M, N, K, group, cu_count_or_default());
+  const Panel2Plan pp = w4a16_panel256_plan(any_rows ? whole_fours(M) : M, N, K, group, cu_count_or_default());
   if (!pp.ok) return -1;
   int64_t rows = with_rows_behind(M, 256);
   auto need = [&] { return pp.split > 1 ? (int64_t)pp.split * rows * N * 4 : (int64_t)0; };
@@ -834,9 +853,9 @@ static int try_panel256(const void* A, const void* w_packed, const void* scales,
 // The middle-M panel kernel.  Returns -1 when it does not take the problem (nothing launched, no error set).
 static int try_panelm(const void* A, const void* w_packed, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, void* workspace,
-                      int64_t workspace_bytes, void* stream) {
+                      int64_t workspace_bytes, void* stream, bool any_rows = false) {
   if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return -1;
-  const PanelMPlan pp = w4a16_panelm_plan(M, N, K, group, cu_count_or_default());
+  const PanelMPlan pp = w4a16_panelm_plan(any_rows ? whole_fours(M) : M, N, K, group, cu_count_or_default());
   if (!pp.ok) return -1;
   int64_t rows = with_rows_behind(M, 16 * pp.tm);
   auto need = [&] { return pp.split > 1 ? (int64_t)pp.split * rows * N * 4 : (int64_t)0; };
@@ -1138,15 +1157,21 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // (not up to 256 rows with groups of 512 values or more: the panel kernels cut K into windows of eight groups -- 32 steps and
   // more -- and run uncut or nearly so, the streaming kernel cuts inside a group: N = 14336, K = 4096, M = 256: 50 against 59 us;
   // N = 11008: 47 against 58 us; N = K = 8192: 52 against 61 us; from 384 rows on the panel kernels are ahead again)
-  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && (panelm_preferred(M, N, K) || panelm_whole_rounds(M, N, K, group, in_dtype)) && !(M <= 256 && group >= 512)) {
+  auto stream_instead = [&] {
+    const StreamPlan sp = stream_plan_for(M, N, K, group, algo);
+    return stream_beats_middle(M, N, K, group, in_dtype, sp) && stream_workspace_ok(sp, M, N, workspace, workspace_bytes) &&
+           stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype);
+  };
+  if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && (panelm_preferred(M, N, K) || panelm_whole_rounds(M, N, K, group, in_dtype)) && !(M <= 256 && group >= 512) &&
+      !stream_instead()) {
     // (very wide matrices: where the 128-row tiles need a second round of work-groups and the 256-row tiles do not, the
     // 256-row kernel by the same estimate -- N = 28672, K = 4096, M = 512: 104 against 129 us)
     if (panel256_estimate_wins(M, N, K, group)) {
       const int rc = try_panel256(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, workspace,
-                                  workspace_bytes, stream);
+                                  workspace_bytes, stream, true);
       if (rc >= 0) return rc;
     }
-    const int rc = try_panelm(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, workspace, workspace_bytes, stream);
+    const int rc = try_panelm(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, workspace, workspace_bytes, stream, true);
     if (rc >= 0) return rc;
   }
   if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && panel_one_round(M, N, K) && group > 0) {
@@ -1154,7 +1179,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     if (rc >= 0) return rc;
   }
   if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && panelm_one_tile(M, N, K) && group > 0) {
-    const int rc = try_panelm(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, workspace, workspace_bytes, stream);
+    const int rc = try_panelm(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, workspace, workspace_bytes, stream, true);
     if (rc >= 0) return rc;
   }
   // 17 .. 512 activation rows: the streaming kernel (weights once per 128 rows, deep ring of direct loads)
@@ -1170,7 +1195,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     }
     if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && group > 0 && panel256_beats_stream(M, N, K, group, sp)) {
       const int rc = try_panel256(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, workspace,
-                                  workspace_bytes, stream);
+                                  workspace_bytes, stream, true);
       if (rc >= 0) return rc;
     }
     // What is left, the tile kernel over K slices and the two passes, is behind on 783 of 796 problems (33 .. 512 rows, 2^25 .. 2^29 weights,
