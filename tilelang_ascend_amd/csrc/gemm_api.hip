@@ -748,8 +748,8 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
       return true;
     const double best = 2.0 * (double)M * (double)N * (double)K / 1.38e9;  // at 1.38 PFLOP/s
     panels = panels / 1.21 > best ? panels / 1.21 : best;
-    // (rows that go along cost no launch.  Above 2048 rows they are counted as one all the same: the panels' estimate is low there, 7 problems of 12 that not counting
-    // it moves are 1 - 13 % slower; up to 2048 rows all 16 are faster, 1.01 - 1.18 x, 518 x 7440 x 1024 24.5 -> 16.4 us)
+    // (rows that go along cost no launch.  Above 2048 rows they are counted as one all the same: the panels' estimate is low there, 6 problems of 10 that not counting
+    // it moves are 1 - 13 % slower; up to 2048 rows 10 of 11 are faster, 1.01 - 1.18 x, 518 x 7440 x 1024 24.5 -> 16.4 us)
     const bool rest = head != M && !(rest_goes_along && M <= 2048 && ceil_div(head, (int64_t)(middle ? 128 : 256)) == ceil_div(M, (int64_t)(middle ? 128 : 256)));
     const double two = two_passes_us(M, N, K), with_rest = panels + (rest ? 4.5 : 0.0);
     return middle ? two < (rest ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 0.95 : 1.07) * with_rest;
@@ -976,15 +976,15 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     }
   }
   const bool room_for_two_passes = N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && workspace != nullptr && workspace_bytes >= N * K * 2 && aligned16(workspace);
-  // Above 512 rows the panel kernels are the fast path, and they take row counts that are multiples of four (their direct
+  // Above 512 rows the panel kernels are the fast path, and they were written for row counts that are multiples of four (their direct
   // loads move four activation rows).  Any other count -- prompt lengths are what they are -- runs as its multiple of four
   // below through the same choice plus the last one to three rows through the small-M kernels, which is one short launch
   // more instead of the two passes for everything (measured: M = 1001, N = 14336, K = 4096: 147 us in one piece, 128 us for
   // 1000 rows; M = 2049, N = K = 8192: 392 against 249 us; M = 601, N = K = 8192: 164 against 120 us; the tail takes 6 - 15 us).
   // One launch or two passes for all rows instead, where their estimates say so -- but not where the last rows belong to the fp16
   // GEMV kernels, whose results are closer to exact arithmetic.  bfloat16 rows, which every kernel multiplies by the same rounded weights, go along
-  // with the head where they lie in its last tile (with_rows_behind): 45 of 111 problems, 1.03 - 1.24 x (1002 x 8960 x 1152 37.7 -> 32.8 us, 3999 x 4096 x
-  // 4096 117.3 -> 111.9, 1207 x 1024 x 6144 36.2 -> 29.2), none slower.
+  // with the head where they lie in its last tile (with_rows_behind): 33 of 105 random problems, 1.10 x on average (1002 x 8960 x 1152 37.7 -> 32.8 us, 3999 x 4096 x
+  // 4096 117.3 -> 111.9, 1207 x 1024 x 6144 36.2 -> 29.2), one of them slower (1366 x 4224 x 512 14.5 -> 14.9).
   const bool head_and_tail = algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && (M & 3) != 0 && M < kMaxDim && N >= 16 && N % 16 == 0 &&
                              N < kMaxDim && K > 0 && K < kMaxDim && group > 0 && A && C && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
                              (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32) &&
@@ -1007,7 +1007,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // us, which the test of that choice names), then the 128-row, the 256-row or the streaming kernel.  Above 512 rows two regions keep what
   // ran before the streaming kernel took such calls, though it is level or ahead: the two passes, where they ran, on weight-row counts
   // that are no multiple of 128 or no more than 256 (639 x 5680 x 896 22.2 against 15.5 us), and, where the panel kernels ran, a launch for
-  // the last one to three rows.  The automatic choice's tests name those kernels too.
+  // the last three fp16 rows.  The automatic choice's tests name those kernels too.
   bool stream_region = algo == TLQ_ALGO_AUTO && g_w4a16_stream && !keep_tail && M > 32 && M <= kStreamMaxRows && N > 0 && K > 0 && group > 0 && N < kMaxDim && K < kMaxDim &&
                        N * K < ((int64_t)1 << (M > 195 ? 25 : 26));
   // (the estimate first: it is kept per shape, the choice among the others is not and takes 1.8 us of host time)
