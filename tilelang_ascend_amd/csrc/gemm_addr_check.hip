@@ -401,8 +401,8 @@ int check_quad_schedule(int stages, int tiles, int extra_start, int extra_stage)
 
 // The streaming kernel's scales: every load of every window of K slices of `slice_steps` steps, for the first and last blocks of weight rows, and
 // what the reads of the scale area then find.  `shift`: values by which the tensors lie behind a 16-byte boundary.
-int check_stream_scales(int64_t N, int64_t K, int64_t group, int kgs, int slice_steps, int shift) {
-  const int mg = kgs == 4 ? 32 : 16, bn = 512 / kgs, groups = (int)(K / group), steps_total = (int)(K / 128);
+int check_stream_scales(int64_t N, int64_t K, int64_t group, int kgs, int mg, int slice_steps, int shift) {
+  const int bn = 512 / kgs, groups = (int)(K / group), steps_total = (int)(K / 128);
   CHECK_OR_FAIL(N >= 4 && N % 4 == 0 && K % group == 0 && group >= 32 && N * groups * 2 < ((int64_t)1 << 32) && slice_steps >= 1, "stream scales: bad arguments");
   int gshift = 0;
   while (((int64_t)1 << gshift) < group) ++gshift;
@@ -496,7 +496,7 @@ int check_stream(int64_t M, int64_t N, int64_t K, int tm) {
         for (int t = 0; t < kt; ++t) ++taken[2 * kt * kg + kt * h + t];
     for (int w = 0; w < 16; ++w) CHECK_OR_FAIL(taken[w] == 1, "stream: word %d of a step is taken %d times", w, taken[w]);
     // the scale area: what a read finds is the value it wants, whether pieces or dwords brought it (a dword read may start one value on)
-    const int mg = kgs == 4 ? 32 : 16;
+    for (int mg = kgs == 4 ? 32 : 16; mg <= 32; mg *= 2)
     for (int cells : {mg / 8, mg / 2}) {
       std::vector<int> value(32 * mg, -1);
       for (int i = 0; i < 32 * cells / 64; ++i)
@@ -1566,7 +1566,8 @@ int tlq_debug_check_stream_addressing(int64_t M, int64_t N, int64_t K, int activ
       for (int kgs = 2; kgs <= 4; kgs += 2)
         for (int shift : {0, 2})
           if (N % 4 == 0)
-            if (int rc = check_stream_scales(N, K, group, kgs, ss, shift)) return rc;
+            for (int mg = kgs == 4 ? 32 : 16; mg <= 32; mg *= 2)  // (256 weight rows: 16, and 32 in a slice of several windows)
+              if (int rc = check_stream_scales(N, K, group, kgs, mg, ss, shift)) return rc;
     }
   }
   const int l = activation_tiles / 2;

@@ -13,7 +13,7 @@
 //     instruction for 4 (v_fma_mixlo / mixhi_f16: 8), while the products take 32 (16) cycles of the matrix pipeline: with 16 x 16 x 32
 //     operands the port is the bound, 3745 cycles a step of 128 rows against 2749 (matrix pipeline: 2048).  At full load the clock
 //     gives way in turn (1.6 - 1.9 GHz): the step of 128 rows takes 1.8 us, 2.1 before.
-//   * The scales and zero points of 32 weight rows are fetched 16 (KG = 2) or 32 groups at a time into LDS: a slice longer than that
+//   * The scales and zero points of 32 weight rows are fetched 16 (KG = 2; 32 where a longer slice has room for them) or 32 groups at a time into LDS: a slice longer than that
 //     runs in windows, each of which fetches its scales and restarts the ring.
 // K slices write fp32 partial sums as [slice][N / 4][M][4] (two runs of 512 bytes per store), added up in slice order by
 // w4a16_stream_reduce_kernel.  All together, against the kernel with 16 x 16 operands and no groups: 211 x 4096 x 11008 37.0 -> 33.0 us,
@@ -48,11 +48,14 @@ struct StreamMma<bf16_t> {
   }
 };
 
-// quantisation groups per window of a K slice: what the scale area holds (few weight rows leave room for twice as many)
-constexpr int stream_max_groups(int kg) { return kg == 4 ? 32 : 16; }
+// quantisation groups per window of a K slice: what the scale area holds (few weight rows leave room for twice as many).  A slice of several windows (`many`) takes
+// twice as many of 256 weight rows too, where that leaves the ring as deep as it is: 19 of 96 random problems with 33 - 511 rows 1.05 x on average (163 x 5888 x 13952
+// 48.2 -> 44.9 us, 173 x 19328 x 2688 in groups of 32 41.3 -> 36.6, 36 x 12544 x 11904 in groups of 64 44.0 -> 41.1), the others level but for one plan that this
+// moves (296 x 5888 x 6656 in groups of 32 49.6 -> 50.9).
+constexpr int stream_max_groups(int kg, int tb = 0, bool many = false) { return kg == 4 || (many && (tb == 2 || tb == 3)) ? 32 : 16; }
 
-// TB: 32-row activation blocks per work-group; KG: groups of wavefronts, each with 128 / KG values of every step
-template <int TB, int KG>
+// TB: 32-row activation blocks per work-group; KG: groups of wavefronts, each with 128 / KG values of every step; MANY: several windows
+template <int TB, int KG, bool MANY>
 struct StreamCfg {
   static_assert(TB >= 1 && TB <= 4 && (KG == 2 || KG == 4), "32-row activation blocks and groups of wavefronts");
   static constexpr int WN = 8 / KG, BM = 32 * TB, BN = 64 * WN;
@@ -61,7 +64,7 @@ struct StreamCfg {
   static constexpr int A_TILE = BM * 256;                     // bytes of activations per step
   static constexpr int W_TILE = BN * 64;                      // packed weights per step
   static constexpr int SLOT = A_TILE + W_TILE;
-  static constexpr int MG = stream_max_groups(KG);
+  static constexpr int MG = stream_max_groups(KG, TB, MANY);
   static constexpr int SZ = 2 * 32 * MG * 2;                  // per 32 weight rows: scales [32][MG groups], then zero points, 2 bytes each
   static constexpr int FITS = (160 * 1024 - BN / 32 * SZ) / SLOT;
   static constexpr int D = FITS > 6 ? 6 : FITS;               // ring depth, one work-group per CU
@@ -138,7 +141,7 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
                                                              const T* __restrict__ scales, const T* __restrict__ zeros,
                                                              void* __restrict__ C, float* __restrict__ partial, int M, int N, int K,
                                                              int gshift, float zero_scalar, int out_dtype, int slice_steps, int xcd_slices) {
-  typedef StreamCfg<TB, KG> Cfg;
+  typedef StreamCfg<TB, KG, MANY> Cfg;
   typedef StreamMma<T> Mma;
   typedef __attribute__((address_space(3))) uint8_t* lptr_t;
   constexpr int D = Cfg::D, LA = Cfg::LA, WN = Cfg::WN, KT = Cfg::T, NU = Cfg::NU, MG = Cfg::MG;
@@ -232,7 +235,7 @@ __global__ __launch_bounds__(512, 2) void w4a16_stream_kernel(const T* __restric
   const uint32_t sz_lane = lds0 + (uint32_t)(Cfg::RING + 2 * wn * Cfg::SZ);
 
   // The slice runs in windows of as many steps as the scale area holds groups for (16 groups: 4, 8, 16 steps for groups
-  // of 32, 64, 128 values, more for larger groups; 32 groups, twice as many, with four groups of wavefronts).  Every window fetches its scales and restarts the ring: a memory
+  // of 32, 64, 128 values, more for larger groups; 32 groups, twice as many, with four groups of wavefronts and where stream_max_groups says so).  Every window fetches its scales and restarts the ring: a memory
   // round trip without multiplications per window, which costs less than a further K slice (a partial tile to write
   // and add, and more work-groups than CUs).
   const int window = __builtin_amdgcn_readfirstlane(gshift >= 7 ? MG << (gshift - 7) : MG >> (7 - gshift));
@@ -632,11 +635,11 @@ thread_local int g_stream_slice_steps = 0;  // tuning and tests: steps of 128 va
 // its best on average (22 % at most, more than 5 % on 19 of 158); on 3338 others (M 17 .. 512, N .. 33000, K .. 18944) 5 % high and 7.9 % rms.
 // Rounds are whole: counted half by how full the last one is, as they were, plans with a few work-groups in a second round looked 15 - 20 % shorter
 // than they are (188 x 18128 x 3200 284 work-groups in 49.6 us, 142 in 35.0): 575 problems that this moves 1.08 x on average, 27 of them 3 % and more behind.
-static double stream_us(int64_t M, int64_t N, int64_t K, int tm, int kg, int64_t m_blocks, int64_t n_blocks, int64_t slice_steps, int64_t slices, int64_t windows, int64_t cus) {
+static double stream_us(int64_t M, int64_t N, int64_t K, int tm, int kg, int64_t m_blocks, int64_t n_blocks, int64_t slice_steps, int64_t slices, double windows, int64_t cus) {
   static const double kStep[2][4] = {{0.73, 0.83, 0.95, 1.15}, {0.355, 0.47, 0.61, 0.68}};  // us per step of 128 values of K: [groups][32-row blocks]
   const int64_t blocks = m_blocks * n_blocks * slices;
   const double rounds = (double)ceil_div(blocks, cus);
-  return 1.95 + rounds * ((kg == 4 ? 4.45 : 3.0) + (double)slice_steps * kStep[kg == 4][tm / 2 - 1] + 2.9 * (double)(windows - 1)) +
+  return 1.95 + rounds * ((kg == 4 ? 4.45 : 3.0) + (double)slice_steps * kStep[kg == 4][tm / 2 - 1] + 2.9 * (windows - 1.0)) +
          (slices > 1 ? 2.36 + 1.7e-6 * (double)slices * (double)M * (double)N : 0.0) + 0.385e-9 * (double)(m_blocks * tm * 16) * (double)(n_blocks * (512 / kg)) * (double)K +
          0.6e-6 * (double)M * (double)N + 0.022e-6 * (double)N * (double)K + 0.086e-6 * (double)M * (double)K;
 }
@@ -671,7 +674,9 @@ static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group
     for (int tm = 2; tm <= 8; tm += 2) {
       if (g_stream_tiles > 0 ? (tm != (g_stream_tiles & 15) || kg != (g_stream_tiles >= 16 ? 4 : 2)) : (tm > 2 && M <= 16 * (tm - 2)) || (tm < 6 && M > 16 * tm)) continue;
       const int64_t m_blocks = ceil_div(M, (int64_t)16 * tm), n_blocks = ceil_div(N, (int64_t)(512 / kg));
-      const int64_t window = (int64_t)stream_max_groups(kg) * group / 128;  // steps whose groups the scale area holds
+      const int64_t window = (int64_t)stream_max_groups(kg) * group / 128;  // steps whose groups the scale area holds; and in a slice of several windows (where those hold
+      // more: 0.6 of a restart more, for the control flow of several windows and their longer fetch)
+      const int64_t of_many = (int64_t)stream_max_groups(kg, tm / 2, true) * group / 128;
       for (int64_t want = 1; want <= 16; ++want) {
         int64_t ss = whole_or_part(ceil_div(steps_total, want));
         if (g_stream_slice_steps > 0) {
@@ -683,7 +688,7 @@ static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group
         if (ss > steps_total) ss = steps_total;
         const int64_t slices = ceil_div(steps_total, ss);
         if (slices > 16) continue;  // too many partial sums to add up: the tile kernel with longer slices takes it
-        const double us = stream_us(M, N, K, tm, kg, m_blocks, n_blocks, ss, slices, ceil_div(ss, window), cus);
+        const double us = stream_us(M, N, K, tm, kg, m_blocks, n_blocks, ss, slices, ss <= window ? 1.0 : (double)ceil_div(ss, of_many) + (of_many > window ? 0.6 : 0.0), cus);
         if (!best.ok || us < best.us) best = StreamPlan{true, tm, (int)m_blocks, (int)n_blocks, (int)slices, (int)ss, kg, us, false};
       }
     }
@@ -701,7 +706,7 @@ static int launch_stream(const void* A, const void* Wp, const void* scales, cons
                          int64_t M, int64_t N, int64_t K, int gshift, float zero_scalar, int out_dtype, const StreamPlan& p,
                          hipStream_t st) {
   auto kern = w4a16_stream_kernel<T, TB, KG, LAYOUT, MANY>;
-  constexpr int lds_bytes = StreamCfg<TB, KG>::LDS;
+  constexpr int lds_bytes = StreamCfg<TB, KG, MANY>::LDS;
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
