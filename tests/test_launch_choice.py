@@ -1,0 +1,67 @@
+"""What the library would launch, asked without a GPU: its calls of the HIP runtime go to tests/launch_recorder.c (256 compute units, every launch succeeds),
+and its own launch log says which kernels ran.  In a process of its own, which never loads the runtime proper."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+from tilelang_ascend_amd import _abi
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes, json, sys
+rec = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+i64, i32, f32, p = ctypes.c_int64, ctypes.c_int, ctypes.c_float, ctypes.c_void_p
+lib.tlq_debug_launch_log_text.restype = lib.tlq_last_error.restype = ctypes.c_char_p
+lib.tlq_gemm_i8.argtypes = [p] * 3 + [i64] * 4 + [i32, p]
+lib.tlq_gemm_w4a16_ws.argtypes = [p] * 5 + [i64] * 4 + [f32] + [i32] * 3 + [p, i64, p]
+lib.tlq_w4a16_choice_set.argtypes = [i64] * 4 + [i32] * 2
+A, W, C, S, WS = (i << 40 for i in range(1, 6))  # (addresses that nothing reads)
+def log(call):
+    lib.tlq_debug_launch_log(1)
+    rc = call()
+    text = lib.tlq_debug_launch_log_text().decode()
+    lib.tlq_debug_launch_log(0)
+    return [rc, text, lib.tlq_last_error().decode() if rc else ""]
+def i8(B, M, N, K, layout):
+    return log(lambda: lib.tlq_gemm_i8(A, W, C, B, M, N, K, layout, None))
+"""
+
+
+@pytest.fixture(scope="module")
+def recorder(tmp_path_factory):
+    if not shutil.which("gcc"):
+        pytest.skip("a C compiler wanted")
+    out = str(tmp_path_factory.mktemp("recorder") / "launch_recorder.so")
+    subprocess.run(["gcc", "-O1", "-Wall", "-Wextra", "-shared", "-fPIC", os.path.join(HERE, "launch_recorder.c"), "-o", out], check=True)
+    return out
+
+
+def ask(recorder, code):
+    """`code` behind the prelude in a process of its own; what it leaves in `result`."""
+    done = subprocess.run([sys.executable, "-c", PRELUDE + code + "\nprint(json.dumps(result))", recorder, _abi.library_path()], capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0, done.stderr
+    return json.loads(done.stdout)
+
+
+# 128-row tiles are the two-stage or the ring kernel's, 256-row ones those of four wavefronts or of the two-stage kernel
+@pytest.mark.parametrize("B,M,N,K", [(8, 2048, 4096, 4096), (8, 3072, 4096, 4096), (1, 513, 1040, 1024), (1, 100, 272, 400)])
+@pytest.mark.parametrize("layout", [_abi.B_KN, _abi.B_NK])
+def test_a_forced_int8_tile_holds_and_ends(recorder, B, M, N, K, layout):
+    """Forced tiles and the automatic choice in turn on one shape, on one thread: each call by the tile that is set for it, and by none that was."""
+    def each(tiles):
+        return ask(recorder, f"""
+result = []
+for tile in {tiles}:
+    lib.tlq_tune_i8_tile(tile)
+    result.append(i8({B}, {M}, {N}, {K}, {layout}))
+""")
+    fresh = {tile: each([tile])[0] for tile in (0, 32, 128, 256)}
+    assert all(rc == 0 for rc, _, _ in fresh.values()), fresh
+    assert "256x256" in fresh[256][1] and "256" not in fresh[128][1] and "32x128" in fresh[32][1], fresh
+    order = [0, 128, 256, 0, 256, 128, 0, 32, 0]
+    assert each(order) == [fresh[tile] for tile in order]

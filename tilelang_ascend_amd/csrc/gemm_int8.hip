@@ -134,7 +134,9 @@ static int dispatch_i8(const void* A, const void* B, const typename Epi::Params&
                        int64_t N, int64_t K, int b_layout, hipStream_t st, const char* what) {
   const TileKind kind = b_layout == TLQ_B_NK ? kTileI8NK : kTileI8KN;
   static thread_local PlanTable<int> known;
-  const int variant = g_i8_tile == 32 || (M <= 32 && g_i8_tile == 0) ? 0 : known.get(batch * 4 + kind, M, N, K, [&] { return tile_choice(kind, batch, M, N, K, g_i8_tile).variant; });
+  // (a forced tile is part of the key: it is set and reset around single calls, and leaves what is known of the others alone)
+  const int forced = g_i8_tile == 0 || g_i8_tile == 128 ? g_i8_tile : 256;
+  const int variant = g_i8_tile == 32 || (M <= 32 && g_i8_tile == 0) ? 0 : known.get((batch * 4 + kind) * 3 + forced / 128, M, N, K, [&] { return tile_choice(kind, batch, M, N, K, forced).variant; });
   if (variant >= kQuad192x256 && variant <= kQuad128x128) return quad_gemm_i8<Epi>(variant, A, B, pe, batch, M, N, K, b_layout, st, what);
   const int tile = variant == 0 ? 32 : variant < kPlain256x256 ? 128 : 256;
   if (variant == kQuad256x256) {
