@@ -65,3 +65,17 @@ for tile in {tiles}:
     assert "256x256" in fresh[256][1] and "256" not in fresh[128][1] and "32x128" in fresh[32][1], fresh
     order = [0, 128, 256, 0, 256, 128, 0, 32, 0]
     assert each(order) == [fresh[tile] for tile in order]
+
+
+@pytest.mark.parametrize("M,N,K", [(8202, 960, 3200), (1182, 6944, 6656), (6715, 1168, 3072)])
+def test_forced_int8_slices_end_too(recorder, M, N, K):
+    """Rows of full rounds and the rest: the rest is not asked of the small-tile kernel while K slices are forced, and is again afterwards."""
+    one = f"i8(1, {M}, {N}, {K}, {_abi.B_NK})"
+    auto, never = (ask(recorder, f"lib.tlq_tune_i8_split({split}); result = {one}") for split in (0, 1))
+    assert auto != never  # (else the shape says nothing)
+    assert ask(recorder, f"""
+result = []
+for split in (0, 1, 0, 1):
+    lib.tlq_tune_i8_split(split)
+    result.append({one})
+""") == [auto, never, auto, never]

@@ -1539,7 +1539,7 @@ static SmallTile small_tile_for_f16(int64_t batch, int64_t M, int64_t N, int64_t
 static int64_t rows_of_full_rounds(TileKind kind, int64_t M, int64_t N, int64_t K) {
   if (M <= 512 || N < 256 || K % 128 != 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || g_gemm_groups || g_gemm_f16_tile || g_i8_tile || g_gemm_slots == 2) return 0;
   static thread_local PlanTable<int64_t> known;
-  return known.get(M, N, K, kind, [&]() -> int64_t {
+  return known.get(M, N, K, kind + 4 * (g_i8_split != 0), [&]() -> int64_t {  // (forced K slices: small_tile_for_i8 refuses the rest)
     const bool i8 = kind >= kTileI8KN;
     const int64_t k_bytes = i8 ? K : 2 * K, stages = k_bytes / kStageBytes, cus = cu_count_or_default();
     if (stages < 6) return 0;
