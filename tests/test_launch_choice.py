@@ -79,3 +79,20 @@ for split in (0, 1, 0, 1):
     lib.tlq_tune_i8_split(split)
     result.append({one})
 """) == [auto, never, auto, never]
+
+
+W4A16 = """
+def w4a16(M, N, K, group, ws=0):
+    return log(lambda: lib.tlq_gemm_w4a16_ws(A, W, S, None, C, M, N, K, group, 8.0, 1, 1, 0, WS if ws else None, ws, None))
+"""
+
+
+@pytest.mark.parametrize("M,N,K,group", [(1207, 720, 3200, 128), (602, 2432, 2176, 64), (767, 1328, 1536, 64), (1005, 496, 2688, 128)])
+def test_last_rows_behind_a_tuned_kernel_that_gets_no_lds(recorder, M, N, K, group):
+    """bfloat16 rows that would go along with the tuned 256-row kernel: where its launch fails, the rules decide for the head, and the last one to three rows are theirs too."""
+    call = f"w4a16({M}, {N}, {K}, {group})"
+    rules = ask(recorder, W4A16 + f"result = {call}")
+    tuned = W4A16 + f"lib.tlq_w4a16_choice_set({M & ~3}, {N}, {K}, {group}, {_abi.BF16}, {_abi.ALGO_PANEL256})\n"
+    assert rules[0] == 0 and " + " in rules[1], rules  # (the head and the rest, by different kernels)
+    assert ask(recorder, tuned + f"result = {call}") == [0, "tlq_gemm_w4a16(panel256) [w4a16_panel256_kernel]", ""]
+    assert ask(recorder, tuned + f"rec.recorder_refuse(b'panel256')\nresult = {call}") == rules

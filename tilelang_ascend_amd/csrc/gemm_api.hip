@@ -803,10 +803,14 @@ static bool stream_args_ok(const void* A, const void* w_packed, const void* scal
 }
 
 // The one to three rows of the same matrices behind the M (a multiple of four) that the automatic choice is called for: the four-wavefront panel kernels and the streaming kernel take them along
-// where they lie in the last of the tiles that M rows take anyway, and set this to zero.  (One tile row more would cost a round where the head's tiles fill
+// where they lie in the last of the tiles that M rows take anyway, and set this to zero once they are launched (not ahead of it: a tuned kernel that fails leaves them to the rules).  (One tile row more would cost a round where the head's tiles fill
 // the machine: 4097 x 4096 x 4096 runs 4096 rows in one round and the last row by itself.)
 static thread_local int64_t g_rows_behind = 0;
 static int64_t with_rows_behind(int64_t M, int64_t tile) { return ceil_div(M, tile) == ceil_div(M + g_rows_behind, tile) ? M + g_rows_behind : M; }
+static int rows_behind_done(int rc, bool along) {
+  if (rc == 0 && along) g_rows_behind = 0;
+  return rc;
+}
 
 // The panel kernel (large M, one launch, weights dequantised on the operand read).  Returns -1 when it does not take the
 // problem (nothing launched, no error set), else the launch's return code.
@@ -845,9 +849,9 @@ static int try_panel256(const void* A, const void* w_packed, const void* scales,
                        fits32(M, K * 2) && fits32(N, K / 2) && fits32(N, (K / group) * 2);
   if (!args_ok) return -1;
   if (need() > 0 && !(workspace && aligned16(workspace) && workspace_bytes >= need())) return -1;
-  if (rows != M) g_rows_behind = 0;
-  return gemm_w4a16_panel256(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, pp,
-                             (float*)workspace, (hipStream_t)stream);
+  const int rc = gemm_w4a16_panel256(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype,
+                                     w_layout, pp, (float*)workspace, (hipStream_t)stream);
+  return rows_behind_done(rc, rows != M);
 }
 
 // The middle-M panel kernel.  Returns -1 when it does not take the problem (nothing launched, no error set).
@@ -866,9 +870,9 @@ static int try_panelm(const void* A, const void* w_packed, const void* scales, c
                        fits32(M, K * 2) && fits32(N, K / 2) && fits32(N, (K / group) * 2);
   if (!args_ok) return -1;
   if (need() > 0 && !(workspace && aligned16(workspace) && workspace_bytes >= need())) return -1;
-  if (rows != M) g_rows_behind = 0;
-  return gemm_w4a16_panelm(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype, pp, (float*)workspace,
-                           (hipStream_t)stream);
+  const int rc = gemm_w4a16_panelm(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype,
+                                   pp, (float*)workspace, (hipStream_t)stream);
+  return rows_behind_done(rc, rows != M);
 }
 
 // One group per weight row on rows whose length is no power of two (K = 11008, 5120, 3584 ...): only the oldest kernels take
@@ -1036,9 +1040,9 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       if (M <= 512 && small_beats_stream(small, sp, M, N, K, group, zeros != nullptr))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                                 (hipStream_t)stream);
-      if (rows != M) g_rows_behind = 0;
-      return gemm_w4a16_stream(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, sp, (float*)workspace,
-                               (hipStream_t)stream);
+      const int rc = gemm_w4a16_stream(A, w_packed, scales, zeros, C, rows, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, sp, (float*)workspace,
+                                       (hipStream_t)stream);
+      return rows_behind_done(rc, rows != M);
     }
   }
   if (head_and_tail && (keep_tail || !(room_for_two_passes && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16)))) {
