@@ -96,3 +96,21 @@ def test_last_rows_behind_a_tuned_kernel_that_gets_no_lds(recorder, M, N, K, gro
     assert rules[0] == 0 and " + " in rules[1], rules  # (the head and the rest, by different kernels)
     assert ask(recorder, tuned + f"result = {call}") == [0, "tlq_gemm_w4a16(panel256) [w4a16_panel256_kernel]", ""]
     assert ask(recorder, tuned + f"rec.recorder_refuse(b'panel256')\nresult = {call}") == rules
+
+
+# The least workspaces with which the streaming kernel took these problems while every window of its scale area held 16 groups: the plans that the
+# longer windows choose cut K into more slices, which do not fit.
+@pytest.mark.parametrize("M,N,K,group,workspace", [(413, 664, 12672, 32, 10969280), (472, 3040, 4224, 64, 11479040), (499, 3488, 4224, 32, 13924096),
+                                                   (464, 4912, 18944, 32, 27350016), (265, 4544, 4352, 32, 12087872)])
+def test_streaming_kernel_in_the_workspaces_that_held_its_slices(recorder, M, N, K, group, workspace):
+    def call(ws, layout, algo):
+        return ask(recorder, f"""
+lib.tlq_gemm_w4a16_layout_ws.argtypes = [p] * 5 + [i64] * 4 + [f32] + [i32] * 4 + [p, i64, p]
+result = log(lambda: lib.tlq_gemm_w4a16_layout_ws(A, W, S, None, C, {M}, {N}, {K}, {group}, 8.0, 0, 0, {algo}, {layout}, WS, {ws}, None))
+""")
+    for layout in (_abi.W_PLAIN, _abi.W_INTERLEAVED_F16):
+        for algo in (_abi.ALGO_AUTO, _abi.ALGO_STREAM):
+            rc, text, error = call(workspace, layout, algo)
+            assert rc == 0 and "w4a16_stream_kernel" in text, (layout, algo, text, error)
+        rc, _, error = call(1 << 16, layout, _abi.ALGO_STREAM)  # (no plan's slices: refused, as ever)
+        assert rc == 1 and "workspace" in error, error

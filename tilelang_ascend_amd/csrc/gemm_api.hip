@@ -787,13 +787,18 @@ static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group) 
     return sp.us < 0.98 * other && sp.us < 0.95 * panels;
   });
 }
-static StreamPlan stream_plan_for(int64_t M, int64_t N, int64_t K, int64_t group, int algo) {  // (by name: 512 rows at most)
-  if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return StreamPlan{};
-  if (M > 512 && !(g_stream_tiles > 0 || (algo == TLQ_ALGO_AUTO && stream_beats_panels(M, N, K, group)))) return StreamPlan{};
-  return w4a16_stream_plan(M, N, K, group, cu_count_or_default());
-}
 static bool stream_workspace_ok(const StreamPlan& sp, int64_t M, int64_t N, const void* workspace, int64_t workspace_bytes) {
   return sp.ok && (sp.split == 1 || (workspace && aligned16(workspace) && workspace_bytes >= (int64_t)sp.split * M * N * 4));
+}
+// By name: 512 rows at most.  Where the workspace does not hold the K slices of the best plan, the plan by short windows, which cuts fewer on some problems: its
+// slices are what such calls were sized for before windows were longer (472 x 3040 x 4224 in groups of 64: two slices for three).
+static StreamPlan stream_plan_for(int64_t M, int64_t N, int64_t K, int64_t group, int algo, const void* workspace, int64_t workspace_bytes) {
+  if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return StreamPlan{};
+  if (M > 512 && !(g_stream_tiles > 0 || (algo == TLQ_ALGO_AUTO && stream_beats_panels(M, N, K, group)))) return StreamPlan{};
+  const StreamPlan best = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
+  if (!best.ok || stream_workspace_ok(best, M, N, workspace, workspace_bytes)) return best;
+  const StreamPlan other = w4a16_stream_plan(M, N, K, group, cu_count_or_default(), true);
+  return stream_workspace_ok(other, M, N, workspace, workspace_bytes) ? other : best;
 }
 static bool stream_args_ok(const void* A, const void* w_packed, const void* scales, const void* zeros, const void* C, int64_t M, int64_t N, int64_t K, int in_dtype,
                            int out_dtype) {
@@ -1021,7 +1026,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     stream_region = two ? N % 128 == 0 && N > 256 : !head_and_tail;
   }
   if (stream_region) {
-    const StreamPlan sp = stream_plan_for(M, N, K, group, algo);
+    const StreamPlan sp = stream_plan_for(M, N, K, group, algo, workspace, workspace_bytes);
     // (129 .. 512 rows where the 256-row kernel's estimate is ahead: on short rows of wide matrices, 472 x 20352 x 1152 in groups of 32 32.0 against
     // 39.7 us, 316 x 24960 x 256 16.8 against 20.2; it runs further down)
     const bool panel = M <= 512 && !g_w4a16_panel && panel256_beats_stream(M, N, K, group, sp);
@@ -1162,7 +1167,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // more -- and run uncut or nearly so, the streaming kernel cuts inside a group: N = 14336, K = 4096, M = 256: 50 against 59 us;
   // N = 11008: 47 against 58 us; N = K = 8192: 52 against 61 us; from 384 rows on the panel kernels are ahead again)
   auto stream_instead = [&] {
-    const StreamPlan sp = stream_plan_for(M, N, K, group, algo);
+    const StreamPlan sp = stream_plan_for(M, N, K, group, algo, workspace, workspace_bytes);
     return stream_beats_middle(M, N, K, group, in_dtype, sp) && stream_workspace_ok(sp, M, N, workspace, workspace_bytes) &&
            stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype);
   };
@@ -1188,7 +1193,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   }
   // 17 .. 512 activation rows: the streaming kernel (weights once per 128 rows, deep ring of direct loads)
   if ((algo == TLQ_ALGO_AUTO && g_w4a16_stream) || algo == TLQ_ALGO_STREAM) {
-    const StreamPlan sp = M <= 512 || g_stream_tiles > 0 ? stream_plan_for(M, N, K, group, algo) : StreamPlan{};
+    const StreamPlan sp = M <= 512 || g_stream_tiles > 0 ? stream_plan_for(M, N, K, group, algo, workspace, workspace_bytes) : StreamPlan{};
     const bool args_ok = stream_args_ok(A, w_packed, scales, zeros, C, M, N, K, in_dtype, out_dtype);
     const bool ws_ok = stream_workspace_ok(sp, M, N, workspace, workspace_bytes);
     if (algo == TLQ_ALGO_AUTO && sp.ok && args_ok) {
@@ -1370,7 +1375,7 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
     if (rc >= 0) return rc;
   }
   if (algo != TLQ_ALGO_TWO_PASS) {
-    const StreamPlan sp = M <= 512 ? stream_plan_for(M, N, K, group, algo) : StreamPlan{};
+    const StreamPlan sp = M <= 512 ? stream_plan_for(M, N, K, group, algo, workspace, workspace_bytes) : StreamPlan{};
     const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));
     const bool room_for_two_passes = ws_aligned && workspace_bytes >= N * K * 2;
     // (no tile kernel reads this layout: the alternative is the two passes, which are behind: 512 x 8192 x 4096 39 against 56 us)

@@ -656,7 +656,7 @@ static bool stream_by_xcd(const StreamPlan& p, int64_t M, int64_t N, int64_t K) 
   const double meet = 8.0 / gcd8((int64_t)p.n_blocks * p.split), w = 0.5e-6 * (double)N * (double)K * ((p.m_blocks < meet ? p.m_blocks : meet) - 1.0);
   return a + w > (p.split > 1 ? 40.0 : 12.0);  // MB
 }
-static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group, int64_t cus) {
+static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group, int64_t cus, bool short_windows) {
   StreamPlan best{false, 0, 0, 0, 0, 0, 2, 0.0, false};
   if (M < 17 || M > kStreamMaxRows || N < 1 || K < 128 || K % 128 != 0 || group < 32 || (group & (group - 1)) != 0 || K % group != 0) return best;
   if (N % 4 != 0) return best;
@@ -676,7 +676,7 @@ static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group
       const int64_t m_blocks = ceil_div(M, (int64_t)16 * tm), n_blocks = ceil_div(N, (int64_t)(512 / kg));
       const int64_t window = (int64_t)stream_max_groups(kg) * group / 128;  // steps whose groups the scale area holds; and in a slice of several windows (where those hold
       // more: 0.6 of a restart more, for the control flow of several windows and their longer fetch)
-      const int64_t of_many = (int64_t)stream_max_groups(kg, tm / 2, true) * group / 128;
+      const int64_t of_many = short_windows ? window : (int64_t)stream_max_groups(kg, tm / 2, true) * group / 128;
       for (int64_t want = 1; want <= 16; ++want) {
         int64_t ss = whole_or_part(ceil_div(steps_total, want));
         if (g_stream_slice_steps > 0) {
@@ -695,10 +695,10 @@ static StreamPlan stream_plan_now(int64_t M, int64_t N, int64_t K, int64_t group
   if (best.ok) best.by_xcd = stream_by_xcd(best, M, N, K);
   return best;
 }
-StreamPlan w4a16_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus) {
+StreamPlan w4a16_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, bool short_windows) {
   static thread_local PlanTable<StreamPlan> known;
   const int64_t n = cus > 0 ? cus : 256;
-  return known.get(M, N, K, group * 4096 + n, [&] { return stream_plan_now(M, N, K, group, n); });
+  return known.get(M, N, K, (group * 2 + short_windows) * 4096 + n, [&] { return stream_plan_now(M, N, K, group, n, short_windows); });
 }
 
 template <typename T, int TB, int KG, int LAYOUT, bool MANY>

@@ -27,7 +27,8 @@ __host__ __device__ inline StreamItem stream_item(uint32_t id, uint32_t n_blocks
   const uint32_t at = xcd * (total >> 3) + (xcd < rest ? xcd : rest) + (id >> 3), t = at / m_blocks;
   return StreamItem{(int)(t % n_blocks), (int)(t / n_blocks), (int)(at % m_blocks)};
 }
-StreamPlan w4a16_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus);
+// short_windows: the plan as it is if no window of the scale area holds more groups than those of a slice of one window (fewer K slices on some problems).
+StreamPlan w4a16_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, bool short_windows = false);
 int gemm_w4a16_stream(const void* A, const void* Wp, const void* scales, const void* zeros, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t group, float zero_scalar, int in_dtype, int out_dtype, int w_layout, const StreamPlan& p,
                       float* partial, hipStream_t st);
