@@ -87,7 +87,7 @@ def w4a16(M, N, K, group, ws=0):
 """
 
 
-@pytest.mark.parametrize("M,N,K,group", [(1207, 720, 3200, 128), (602, 2432, 2176, 64), (767, 1328, 1536, 64), (1005, 496, 2688, 128)])
+@pytest.mark.parametrize("M,N,K,group", [(1635, 272, 3584, 128), (1295, 560, 2816, 64), (2442, 224, 2944, 128), (1759, 496, 3072, 64)])
 def test_last_rows_behind_a_tuned_kernel_that_gets_no_lds(recorder, M, N, K, group):
     """bfloat16 rows that would go along with the tuned 256-row kernel: where its launch fails, the rules decide for the head, and the last one to three rows are theirs too."""
     call = f"w4a16({M}, {N}, {K}, {group})"
@@ -114,3 +114,15 @@ result = log(lambda: lib.tlq_gemm_w4a16_layout_ws(A, W, S, None, C, {M}, {N}, {K
             assert rc == 0 and "w4a16_stream_kernel" in text, (layout, algo, text, error)
         rc, _, error = call(1 << 16, layout, _abi.ALGO_STREAM)  # (no plan's slices: refused, as ever)
         assert rc == 1 and "workspace" in error, error
+
+
+# (bfloat16, groups of 64; a workspace too small for the dequantised weights, and none)
+@pytest.mark.parametrize("M,N,K", [(2308, 1328, 4224), (2174, 1152, 3840), (2528, 2688, 4608), (4020, 576, 3584), (1059, 2416, 4736), (926, 1888, 3328), (565, 1040, 640)])
+def test_calls_without_room_for_the_two_passes_are_not_decided_by_them(recorder, M, N, K):
+    """What runs above 512 rows without the room that the two passes take does not follow the estimate of their plain GEMM, here made very low
+    (tlq_tune_gemm_quad) and high (its oldest kernel alone)."""
+    for ws in (0, N * K):
+        auto, fast, slow = (ask(recorder, W4A16 + f"{tune}; result = w4a16({M}, {N}, {K}, 64, {ws})")
+                            for tune in ("pass", "lib.tlq_tune_gemm_quad(11)", "lib.tlq_tune_gemm_groups(1); lib.tlq_tune_gemm_slots(0)"))
+        assert auto[0] == 0 and "dequant" not in auto[1], auto
+        assert auto == fast == slow

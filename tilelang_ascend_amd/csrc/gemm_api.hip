@@ -301,11 +301,11 @@ static bool small_beats_stream(const SmallTile& p, const StreamPlan& sp, int64_t
 // above 512 rows: the tile kernel on up to 2^19 weights -- and the launch for the last M % 4 rows, 4 us, where they run apart --, else the
 // two passes or the panel kernels, which are level with them or ahead; only while the whole call stays short
 static double two_passes_us(int64_t M, int64_t N, int64_t K);
-static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group);
-static bool small_beats_panels(const SmallTile& p, int64_t M, int64_t N, int64_t K, bool head_and_tail) {
+static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group, bool two_passes);
+static bool small_beats_panels(const SmallTile& p, int64_t M, int64_t N, int64_t K, bool head_and_tail, bool two_passes) {
   if (!p.ok || p.us >= 13.0) return false;
   const double us = small_us(p, M, N, K);
-  return us < (N * K <= ((int64_t)1 << 19) ? 0.95 * (fused_tile_us(M, N, K) + (head_and_tail ? 4.0 : 0.0)) : 0.95 * two_passes_us(M, N, K));
+  return us < 0.95 * (two_passes && N * K > ((int64_t)1 << 19) ? two_passes_us(M, N, K) : fused_tile_us(M, N, K) + (head_and_tail ? 4.0 : 0.0));
 }
 // the decode kernel over chunks of K, whose second launch adds the chunks
 static bool small_beats_decode_chunks(const SmallTile& p, int64_t M, int64_t N, int64_t K) {
@@ -597,7 +597,7 @@ static int64_t w4a16_kernel_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (tuned[0] > need) need = tuned[0];
   if (M > 512 && M <= kStreamMaxRows) {  // partial sums of the streaming kernel, where it is the choice for some group size
     for (int64_t group = 32; group <= K && K % group == 0; group *= 2) {
-      if (!stream_beats_panels(M, N, K, group)) continue;
+      if (!stream_beats_panels(M, N, K, group, true)) continue;
       const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
       if (sp.split > 1 && (int64_t)sp.split * M * N * 4 > need) need = (int64_t)sp.split * M * N * 4;
     }
@@ -755,6 +755,9 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
     return middle ? two < (rest ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 0.95 : 1.07) * with_rest;
   });
 }
+static bool room_for_two_passes(int64_t N, int64_t K, const void* workspace, int64_t workspace_bytes) {
+  return N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && workspace != nullptr && workspace_bytes >= N * K * 2 && aligned16(workspace);
+}
 // Many rows on up to 2^19 weights: the two passes or the tile kernel in one launch.  27 problems above 512 rows where that ran: 13 go to the two passes, 1.28 x
 // on average (4907 x 256 x 2048 38.9 -> 16.8 us), one of them 3 % behind.
 static bool two_passes_beat_tiles(int64_t M, int64_t N, int64_t K) {
@@ -766,15 +769,19 @@ static bool two_passes_beat_tiles(int64_t M, int64_t N, int64_t K) {
 // multiple of four costs them a launch) and the two passes?  On 300 random problems (M 513 .. 4096, up to 2e11 operations) where the rule
 // alone decided, 1.13 x on average over what ran before (1.9 x at most: 663 x 4096 x 1792 34.1 -> 17.5 us), more than 5 % behind on 7;
 // with the regions that the entry point leaves to the others 1.06 x.
-static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group) {
+static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group, bool two_passes) {
   static thread_local PlanTable<bool> known;
-  return g_w4a16_stream && known.get(M, N, K, group, [&] {
+  return g_w4a16_stream && known.get(M, N, K, group * 2 + two_passes, [&] {
     const StreamPlan sp = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
     if (!sp.ok) return false;
     const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
-    double other = N % 8 == 0 ? two_passes_us(M, N, K) : fused_tile_us(M, N, K);
+    const int64_t tiles = ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128);
+    // (without room for the two passes it is the tile kernel that would run: 1.05 x its estimate in one round of tiles, 1.2 - 1.3 x in two, 1.4 x beyond; by an
+    // estimate of passes that cannot run 2308 x 1328 x 4224 took 80 us in the tile kernel for 44 here; 1138 random calls that either moves 1.22 x on average)
+    double other = fused_tile_us(M, N, K) * (two_passes || (tiles <= cus_now && K <= 512) ? 1.0 : tiles <= cus_now ? 1.05 : tiles <= 2 * cus_now ? 1.25 : 1.4);
+    if (two_passes && N % 8 == 0) other = two_passes_us(M, N, K);
     // (short rows in one round of 128 x 128 tiles: the tile kernel, 3388 x 384 x 384 8.5 against 9.9 us)
-    if (K <= 512 && ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)128) <= cus_now && fused_tile_us(M, N, K) < other) other = fused_tile_us(M, N, K);
+    if (K <= 512 && tiles <= cus_now && fused_tile_us(M, N, K) < other) other = fused_tile_us(M, N, K);
     const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
     const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
     double panels = 1e30;
@@ -784,7 +791,7 @@ static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group) 
       if (us < panels) panels = us;
     }
     panels = 0.87 * panels + (head != M ? 5.5 : 0.0);
-    return sp.us < 0.98 * other && sp.us < 0.95 * panels;
+    return sp.us < (two_passes || K > 512 ? 0.98 : 0.95) * other && sp.us < 0.95 * panels;
   });
 }
 static bool stream_workspace_ok(const StreamPlan& sp, int64_t M, int64_t N, const void* workspace, int64_t workspace_bytes) {
@@ -794,7 +801,7 @@ static bool stream_workspace_ok(const StreamPlan& sp, int64_t M, int64_t N, cons
 // slices are what such calls were sized for before windows were longer (472 x 3040 x 4224 in groups of 64: two slices for three).
 static StreamPlan stream_plan_for(int64_t M, int64_t N, int64_t K, int64_t group, int algo, const void* workspace, int64_t workspace_bytes) {
   if (!(M >= 1 && N >= 1 && K > 0 && group > 0 && M < kMaxDim && N < kMaxDim && K < kMaxDim)) return StreamPlan{};
-  if (M > 512 && !(g_stream_tiles > 0 || (algo == TLQ_ALGO_AUTO && stream_beats_panels(M, N, K, group)))) return StreamPlan{};
+  if (M > 512 && !(g_stream_tiles > 0 || (algo == TLQ_ALGO_AUTO && stream_beats_panels(M, N, K, group, room_for_two_passes(N, K, workspace, workspace_bytes))))) return StreamPlan{};
   const StreamPlan best = w4a16_stream_plan(M, N, K, group, cu_count_or_default());
   if (!best.ok || stream_workspace_ok(best, M, N, workspace, workspace_bytes)) return best;
   const StreamPlan other = w4a16_stream_plan(M, N, K, group, cu_count_or_default(), true);
@@ -984,7 +991,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       set_error("%s", "");
     }
   }
-  const bool room_for_two_passes = N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && workspace != nullptr && workspace_bytes >= N * K * 2 && aligned16(workspace);
+  const bool two_passes_fit = room_for_two_passes(N, K, workspace, workspace_bytes);
   // Above 512 rows the panel kernels are the fast path, and they were written for row counts that are multiples of four (their direct
   // loads move four activation rows).  Any other count -- prompt lengths are what they are -- runs as its multiple of four
   // below through the same choice plus the last one to three rows through the small-M kernels, which is one short launch
@@ -1005,7 +1012,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       aligned16(w_packed) && aligned16(C) && (in_dtype == TLQ_F16 || in_dtype == TLQ_BF16) &&
       (out_dtype == TLQ_F16 || out_dtype == TLQ_BF16 || out_dtype == TLQ_F32)) {
     const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
-    if (small_beats_panels(small, M, N, K, head_and_tail))
+    if (small_beats_panels(small, M, N, K, head_and_tail, two_passes_fit))
       return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_W_PLAIN, small, "tlq_gemm_w4a16(small)",
                               (hipStream_t)stream);
   }
@@ -1020,9 +1027,9 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   bool stream_region = algo == TLQ_ALGO_AUTO && g_w4a16_stream && !keep_tail && M > 32 && M <= kStreamMaxRows && N > 0 && K > 0 && group > 0 && N < kMaxDim && K < kMaxDim &&
                        N * K < ((int64_t)1 << (M > 195 ? 25 : 26));
   // (the estimate first: it is kept per shape, the choice among the others is not and takes 1.8 us of host time)
-  if (M > 512 && stream_region && (stream_region = g_stream_tiles > 0 || stream_beats_panels(M, N, K, group))) {
+  if (M > 512 && stream_region && (stream_region = g_stream_tiles > 0 || stream_beats_panels(M, N, K, group, two_passes_fit))) {
     const int64_t head = M & ~(int64_t)3;
-    const bool two = room_for_two_passes && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
+    const bool two = two_passes_fit && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
     stream_region = two ? N % 128 == 0 && N > 256 : !head_and_tail;
   }
   if (stream_region) {
@@ -1050,7 +1057,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       return rows_behind_done(rc, rows != M);
     }
   }
-  if (head_and_tail && (keep_tail || !(room_for_two_passes && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16)))) {
+  if (head_and_tail && (keep_tail || !(two_passes_fit && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16)))) {
     const int64_t head = M & ~(int64_t)3;
     const bool may_go_along = in_dtype == TLQ_BF16;
     g_rows_behind = may_go_along ? M - head : 0;
@@ -1135,7 +1142,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
     // (rows of more than 1280 values only where the skinny kernel's work-groups, one per 16 weight rows, run in one round or
     // fill their last round: N = 6144, K = 2048, 384 work-groups: 16 - 22 against 14 - 15 us)
     const bool skinny_fills = ceil_div(N, (int64_t)16) <= cu_count_or_default() || tile_fill(1, 16, N, 16) >= 0.8;
-    if ((M <= 64 && (nk <= ((int64_t)1 << 21) || (nk <= ((int64_t)1 << 24) && (K <= 1280 || (K <= 2048 && skinny_fills))))) || (nk <= ((int64_t)1 << 19) && !(room_for_two_passes && two_passes_beat_tiles(M, N, K))))
+    if ((M <= 64 && (nk <= ((int64_t)1 << 21) || (nk <= ((int64_t)1 << 24) && (K <= 1280 || (K <= 2048 && skinny_fills))))) || (nk <= ((int64_t)1 << 19) && !(two_passes_fit && two_passes_beat_tiles(M, N, K))))
       return tlq_gemm_w4a16(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, TLQ_ALGO_AUTO, stream);
     // Short rows, 96 .. 512 activation rows, one round of 128 x 128 tiles: the tile kernel in one launch takes 4.5 us + 1.45 us
     // per 128 values of K whatever M and N, the streaming kernel 11 - 15 us at K = 512 and 19 - 30 us at K = 1024 .. 1536.
@@ -1377,10 +1384,9 @@ int tlq_gemm_w4a16_layout_ws(const void* A, const void* w_packed, const void* sc
   if (algo != TLQ_ALGO_TWO_PASS) {
     const StreamPlan sp = M <= 512 ? stream_plan_for(M, N, K, group, algo, workspace, workspace_bytes) : StreamPlan{};
     const bool ws_ok = sp.ok && (M * N) % 4 == 0 && (sp.split == 1 || (ws_aligned && workspace_bytes >= (int64_t)sp.split * M * N * 4));
-    const bool room_for_two_passes = ws_aligned && workspace_bytes >= N * K * 2;
     // (no tile kernel reads this layout: the alternative is the two passes, which are behind: 512 x 8192 x 4096 39 against 56 us)
     // the small-tile kernel in the place of either, for calls that bring the workspace those want: without it they are refused
-    if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (ws_ok || (room_for_two_passes && N % 8 == 0))) {
+    if (algo == TLQ_ALGO_AUTO && sp.ok && (M * N) % 4 == 0 && (ws_ok || (room_for_two_passes(N, K, workspace, workspace_bytes) && N % 8 == 0))) {
       const SmallTile small = w4a16_small_plan(M, N, K, group, scales, zeros, 0, 0, 0);
       if (small_beats_stream(small, sp, M, N, K, group, zeros != nullptr))
         return gemm_w4a16_small(A, w_packed, scales, zeros, C, M, N, K, group, zero_scalar, in_dtype, out_dtype, w_layout, small, "tlq_gemm_w4a16(small)",
