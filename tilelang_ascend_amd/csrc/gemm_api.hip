@@ -1445,10 +1445,11 @@ static double sliced_us(int kind, int64_t batch, int64_t M, int64_t N, int64_t K
     default: return 8.9 + 2.5 * g + 4.7 * mn + 0.24 * k + 6.2 * tiles_k;
   }
 }
-// One launch over all of K or slices of it: sliced_us is 1.25 x high on average (0.8 - 2.1), the tiles' estimate 1.05 (0.6 - 1.24); on 78 of the problems that
-// the tiles were fitted to slices had run: 69 go to one launch, 1.17 x faster on average, two of them more than 10 % slower.
+// One launch over all of K, or slices of it?  By both estimates (on rows of up to 64 stages 0.91 and 1.0 x what is measured, 13 - 14 % rms); longer rows stay with the
+// slices, which they make too dear.  On 3284 random [N, K] 16-bit products that have a cut 2.2 % behind the faster of the two, 2.8 % by a bar of 0.82 on rows of any length
+// (496 x 2496 x 11520 47 us in slices, 73 in one launch, which that took; 1111 x 240 x 2496 10.0 in one launch, 13.8 in slices).
 static bool tiles_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes) {
-  return M > 32 && tile_choice(tile, 1, M, N, k_bytes).us < 0.82 * sliced_us(kind, 1, M, N, K);
+  return M > 32 && k_bytes <= 64 * kStageBytes && tile_choice(tile, 1, M, N, k_bytes).us < 0.9 * sliced_us(kind, 1, M, N, K);
 }
 static double plain_nk_us(int64_t M, int64_t N, int64_t K) {  // one 16-bit matrix of [N, K] weights
   if (f16_split_choice(1, M, N, K) > 1 && !tiles_beat_slices(kTileF16NK, 2, M, N, K, K * 2)) return sliced_us(2, 1, M, N, K);
