@@ -137,3 +137,18 @@ lib.tlq_gemm_f16_ws.argtypes = [p] * 4 + [i64] * 5 + [i32] * 3 + [p]
 result = log(lambda: lib.tlq_gemm_f16_ws(A, W, C, WS, 1 << 32, 1, {M}, {N}, {K}, 0, 0, {_abi.B_NK}, None))
 """)
     assert rc == 0 and ("K slices" in text) == slices, (text, error)
+
+
+# The small-tile kernel against the tiles, measured: narrow results and long rows 15.6 / 24.3, 19.2 / 29.8, 22.5 / 34.7, 5.6 / 12.1, 6.0 / 8.7 us; two stages of K 8.3 / 5.8, 8.1 / 5.7
+@pytest.mark.parametrize("kind,B,M,N,K,layout,small", [("w8a8", 9, 269, 64, 9344, _abi.B_KN, True), ("i8", 8, 464, 64, 11520, _abi.B_KN, True), ("f16", 4, 52, 512, 6080, _abi.B_KN, True),
+                                                       ("w8a8", 5, 399, 16, 7424, _abi.B_NK, True), ("f16", 1, 3791, 64, 1856, _abi.B_KN, True),
+                                                       ("w8a8", 1, 227, 3760, 256, _abi.B_KN, False), ("w8a8", 1, 99, 7264, 256, _abi.B_NK, False)])
+def test_small_tiles_or_tiles(recorder, kind, B, M, N, K, layout, small):
+    call = {"i8": f"lib.tlq_gemm_i8(A, W, C, {B}, {M}, {N}, {K}, {layout}, None)", "f16": f"lib.tlq_gemm_f16_batched(A, W, C, {B}, {M}, {N}, {K}, 0, 0, {layout}, None)",
+            "w8a8": f"lib.tlq_gemm_w8a8(A, W, S, S, C, {B}, {M}, {N}, {K}, {N}, {layout}, 0, None)"}[kind]
+    rc, text, error = ask(recorder, f"""
+lib.tlq_gemm_f16_batched.argtypes = [p] * 3 + [i64] * 4 + [i32] * 3 + [p]
+lib.tlq_gemm_w8a8.argtypes = [p] * 5 + [i64] * 5 + [i32] * 2 + [p]
+result = log(lambda: {call})
+""")
+    assert rc == 0 and ("gemm_small_kernel" in text) == small, (text, error)
