@@ -152,3 +152,14 @@ lib.tlq_gemm_w8a8.argtypes = [p] * 5 + [i64] * 5 + [i32] * 2 + [p]
 result = log(lambda: {call})
 """)
     assert rc == 0 and ("gemm_small_kernel" in text) == small, (text, error)
+
+
+# an odd number of tile rows of 64, 128 x 64 against 64 x 128 tiles: 22.1 / 28.1, 26.8 / 33.5, 50.7 / 63.2, 28.6 / 34.8, 13.9 / 17.2 us
+@pytest.mark.parametrize("kind,B,M,N,K", [("i8", 1, 416, 3456, 5040), ("i8", 1, 436, 2656, 9216), ("i8", 1, 694, 2624, 11440), ("w8a8", 1, 287, 4128, 7232), ("w8a8", 5, 140, 1536, 2704)])
+def test_ring_tiles_that_leave_fewer_units_idle(recorder, kind, B, M, N, K):
+    call = {"i8": f"lib.tlq_gemm_i8(A, W, C, {B}, {M}, {N}, {K}, {_abi.B_NK}, None)", "w8a8": f"lib.tlq_gemm_w8a8(A, W, S, S, C, {B}, {M}, {N}, {K}, {N}, {_abi.B_NK}, 0, None)"}[kind]
+    rc, text, error = ask(recorder, f"""
+lib.tlq_gemm_w8a8.argtypes = [p] * 5 + [i64] * 5 + [i32] * 2 + [p]
+result = log(lambda: {call})
+""")
+    assert rc == 0 and "ring_gemm_mfma_kernel 128x64" in text, (text, error)

@@ -1468,34 +1468,6 @@ static SmallUse w4a8_use(bool two_steps, int sign_mode, int64_t K) {
   if (small_w4a8_times16(sign_mode, K)) return two_steps ? kUseW4A8TwoStepsTimes16 : kUseW4A8Times16;
   return two_steps ? kUseW4A8TwoSteps : kUseW4A8;
 }
-// The ring kernel in one round of its tiles, as the small-tile kernel's bars against it were fitted (0.0: none of its tiles runs in one): fixed + stages x (step + shared x the part
-// of the CUs that have a work-group), no less than the trips of the operands from memory, several tile rows reading the weights again, and the products take.
-// (Against the estimates of tile_choice, which are fitted without regard to the small-tile kernel, those bars go wrong on narrow results and long rows: 8 x 237 x 16 x 12928 W8A8
-// 11.0 -> 27.2 us, 3106 x 64 x 2048 4.8 -> 7.7.  3932 random products of 6 us and more: 88 of them more than 10 % behind what ran before those estimates, 25 by these.)
-static double one_round_ring_us(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes) {
-  struct RingCost {
-    double fixed, step, shared;
-  };
-  static constexpr RingCost kRingCost[4][4] = {
-      // 128 x 128           128 x 64              64 x 128              64 x 64
-      {{4.74, 0.313, 0.201}, {4.01, 0.217, 0.171}, {3.79, 0.246, 0.135}, {3.73, 0.174, 0.076}},
-      {{4.56, 0.288, 0.201}, {4.07, 0.195, 0.124}, {3.71, 0.212, 0.157}, {3.72, 0.146, 0.075}},
-      {{4.73, 0.362, 0.239}, {4.33, 0.287, 0.168}, {3.71, 0.314, 0.123}, {3.65, 0.243, 0.105}},
-      {{4.98, 0.281, 0.218}, {4.28, 0.189, 0.151}, {3.92, 0.206, 0.178}, {3.76, 0.140, 0.094}}};
-  const int64_t stages = ceil_div(k_bytes, (int64_t)kStageBytes), cus = cu_count_or_default();
-  const double row = (double)(stages * kStageBytes), memory = (double)(batch * (M + N)) * row / 4.8e6, product = (double)(batch * M) * (double)N * row / (kind >= kTileI8KN ? 1.05e9 : 1.45e9);
-  double best = 0.0;
-  for (int v = kGroup128x128; v <= kGroup64x64 && g_gemm_groups != 1 && stages >= 4 && M > 32; ++v) {
-    const int64_t tiles_m = ceil_div(M, (int64_t)kTileShape[v - 1].rows), blocks = batch * tiles_m * ceil_div(N, (int64_t)kTileShape[v - 1].cols);
-    if (blocks > cus) continue;
-    const RingCost& c = kRingCost[kind][v - kGroup128x128];
-    double us = c.fixed + (double)stages * (c.step + c.shared * (double)blocks / (double)cus);
-    const double trips = memory + (blocks % 8 != 0 ? 0.9 : 0.3) * (double)((tiles_m < 4 ? tiles_m : 4) - 1) * (double)(batch * N) * row / 4.8e6, most = trips > product ? trips : product;
-    if (us < most) us = most;
-    if (best == 0.0 || us < best) best = us;
-  }
-  return best;
-}
 // Is the small-tile kernel ahead of what would run in its place?  Two things its own estimate leaves out come on top: the activations' trip from
 // memory (at 2.5 TB/s: every tile of weight rows asks for them again) and, with 16-bit weights, that theirs cannot take less than
 // a copy.  The other side, by what would run: calls that cut K into slices over work-groups (sliced_us), up to 32 rows a fit to the 32-row
@@ -1547,7 +1519,7 @@ static bool small_tile_wins(const SmallTile& t, SmallUse use, int64_t batch, int
   if (packed && i8_split_choice(1, M, N, K, false) > 1 && !tiles_beat_slices(kTileI8NK, 0, M, N, K, K))
     return us < bar.sliced * (unpack_us + 2.0 * sliced_us(0, 1, M, N, K));  // (slices that add into the result take twice those with matrices of their own)
   const double mine = bar.launch + bar.scale * t.us + bar.trip * trip_us + bar.step * (double)stages + bar.out * mn + bar.weights * nk;
-  const double ring_us = one_round_ring_us(tile, batch, M, N, k_bytes);
+  const double ring_us = one_round_ring(tile, batch, M, N, k_bytes).us;
   return ring_us > 0.0 ? mine < unpack_us + ring_us : mine < bar.plain * (unpack_us + tile_choice(tile, batch, M, N, k_bytes).us);
 }
 static SmallTile small_tile_for_i8(int64_t batch, int64_t M, int64_t N, int64_t K, SmallUse use) {

@@ -1049,6 +1049,34 @@ struct TileChoice {
   int variant;
   double us;
 };
+// The ring kernel's tile of `from` .. `to` that is the fastest in one round of work-groups (variant 0: none runs in one), by the estimate that the small-tile kernel's bars against it
+// were fitted with: fixed + stages x (step + shared x the part of the CUs that have a work-group), no less than the trips of the operands from memory, several tile rows reading the weights again, and the products take.
+// (Against the estimates of tile_choice, which are fitted without regard to the small-tile kernel, those bars go wrong on narrow results and long rows: 8 x 237 x 16 x 12928 W8A8
+// 11.0 -> 27.2 us, 3106 x 64 x 2048 4.8 -> 7.7.  3932 random products of 6 us and more: 88 of them more than 10 % behind what ran before those estimates, 25 by these.)
+inline TileChoice one_round_ring(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes, int from = kGroup128x128, int to = kGroup64x64) {
+  struct RingCost {
+    double fixed, step, shared;
+  };
+  static constexpr RingCost kRingCost[4][4] = {
+      // 128 x 128           128 x 64              64 x 128              64 x 64
+      {{4.74, 0.313, 0.201}, {4.01, 0.217, 0.171}, {3.79, 0.246, 0.135}, {3.73, 0.174, 0.076}},
+      {{4.56, 0.288, 0.201}, {4.07, 0.195, 0.124}, {3.71, 0.212, 0.157}, {3.72, 0.146, 0.075}},
+      {{4.73, 0.362, 0.239}, {4.33, 0.287, 0.168}, {3.71, 0.314, 0.123}, {3.65, 0.243, 0.105}},
+      {{4.98, 0.281, 0.218}, {4.28, 0.189, 0.151}, {3.92, 0.206, 0.178}, {3.76, 0.140, 0.094}}};
+  const int64_t stages = ceil_div(k_bytes, (int64_t)kStageBytes), cus = tlq_device_cu_count() > 0 ? tlq_device_cu_count() : 256;
+  const double row = (double)(stages * kStageBytes), memory = (double)(batch * (M + N)) * row / 4.8e6, product = (double)(batch * M) * (double)N * row / (kind >= kTileI8KN ? 1.05e9 : 1.45e9);
+  TileChoice best{0, 0.0};
+  for (int v = from; v <= to && g_gemm_groups != 1 && stages >= 4 && M > 32; ++v) {
+    const int64_t tiles_m = ceil_div(M, (int64_t)kTileShape[v - 1].rows), blocks = batch * tiles_m * ceil_div(N, (int64_t)kTileShape[v - 1].cols);
+    if (blocks > cus) continue;
+    const RingCost& c = kRingCost[kind][v - kGroup128x128];
+    double us = c.fixed + (double)stages * (c.step + c.shared * (double)blocks / (double)cus);
+    const double trips = memory + (blocks % 8 != 0 ? 0.9 : 0.3) * (double)((tiles_m < 4 ? tiles_m : 4) - 1) * (double)(batch * N) * row / 4.8e6, most = trips > product ? trips : product;
+    if (us < most) us = most;
+    if (best.variant == 0 || us < best.us) best = {v, us};
+  }
+  return best;
+}
 // `tile`: 128 or 256: of those square tiles; 0: any; -1: any but the four-wavefront kernel's in between.  The ring kernel takes four stages and more and 33 rows and more (fewer: not measured), the kernel on four
 // wavefronts whole stages, two or more, and on tiles other than 256 x 256 what 64 tiles of 128 x 128 hold (fewer are the small-tile kernel's or the ring's).
 inline TileChoice tile_choice(TileKind kind, int64_t batch, int64_t M, int64_t N, int64_t k_bytes, int tile = 0) {
@@ -1067,6 +1095,10 @@ inline TileChoice tile_choice(TileKind kind, int64_t batch, int64_t M, int64_t N
     const double us = tile_us(kind, v, batch, M, N, k_bytes);
     if (best.variant == 0 || us < best.us) best = {v, us};
   }
+  // (64 x 128 tiles that are fewer than those of 128 x 64, an odd number of tile rows: the estimates above do not see the CUs that they leave idle, by which 51 of 204 random products were
+  // 1.06 x slower on average, 27 of them 5 % and more, 148 x 7920 x 2288 W8A8 12.1 -> 15.3 us; with this question 25 of 464 are, for 51)
+  if (best.variant == kGroup64x128 && g_gemm_groups == 0 && ceil_div(M, (int64_t)64) * ceil_div(N, (int64_t)128) < ceil_div(M, (int64_t)128) * ceil_div(N, (int64_t)64))
+    if (const TileChoice two = one_round_ring(kind, batch, M, N, k_bytes, kGroup128x64, kGroup64x128); two.variant != 0) best.variant = two.variant;
   return best;
 }
 // RUN(tile rows, tile columns, ring kernel or not) for 128 x 128 tiles of the two-stage kernel and the ring kernel's
