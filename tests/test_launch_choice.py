@@ -163,3 +163,13 @@ lib.tlq_gemm_w8a8.argtypes = [p] * 5 + [i64] * 5 + [i32] * 2 + [p]
 result = log(lambda: {call})
 """)
     assert rc == 0 and "ring_gemm_mfma_kernel 128x64" in text, (text, error)
+
+
+# 16-bit products of one and a half rounds of the ring kernel's tiles, two-stage kernel / ring kernel: 109 / 154, 146 / 189, 194 / 269 us
+@pytest.mark.parametrize("B,M,N,K", [(1, 2797, 2192, 6896), (1, 2464, 1728, 9456), (8, 564, 1600, 8224)])
+def test_two_stages_or_more_than_one_round_of_the_ring(recorder, B, M, N, K):
+    rc, text, error = ask(recorder, f"""
+lib.tlq_gemm_f16_batched.argtypes = [p] * 3 + [i64] * 4 + [i32] * 3 + [p]
+result = log(lambda: lib.tlq_gemm_f16_batched(A, W, C, {B}, {M}, {N}, {K}, 0, 0, {_abi.B_NK}, None))
+""")
+    assert rc == 0 and "[gemm_mfma_kernel" in text, (text, error)
