@@ -730,7 +730,16 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 // below, is 0.5 % behind the faster of the two.  (The middle-M kernel's bars are those that the tests of the choice ask for, 1003 x 2048 x 4096 in groups of 64
 // 35 us in a launch for 1000 rows and one for three, 29 in the two passes.)  Where neither panel kernel would run, all rows go through the two passes and none is left over.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
-static double two_passes_us(int64_t M, int64_t N, int64_t K) { return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(M, N, K); }
+static bool tiles_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes);
+// (fitted to 1900 calls of 6 - 100 us, 7 % rms: right behind the dequantisation the ring kernel takes 19 % more than on its own, the kernels of larger tiles do not.
+// Without that the passes looked 12 % too fast and took calls from the streaming and the small-tile kernel: 564 x 3328 x 1280 19.9 for 12.9 us, 801 x 384 x 2176
+// 13.9 for 9.6)
+static double two_passes_us(int64_t M, int64_t N, int64_t K) {
+  if (f16_split_choice(1, M, N, K) > 1 && !tiles_beat_slices(kTileF16NK, 2, M, N, K, K * 2)) return 2.6 + (double)N * (double)K * 2.5 / 4.8e6 + plain_nk_us(M, N, K);
+  const TileChoice c = tile_choice(kTileF16NK, 1, M, N, K * 2);
+  const bool ring = c.variant >= kGroup128x128 && c.variant <= kGroup64x64;
+  return ring ? 2.7 + 0.31e-6 * (double)N * (double)K + 1.19 * c.us : 4.6 + 0.645e-6 * (double)N * (double)K + 0.93 * c.us;
+}
 static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group, bool rest_goes_along) {
   static thread_local PlanTable<bool> known;
   return known.get(M, N, K, group * 2 + rest_goes_along, [&] {
@@ -752,7 +761,7 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
     // it moves are 1 - 13 % slower; up to 2048 rows 10 of 11 are faster, 1.01 - 1.18 x, 518 x 7440 x 1024 24.5 -> 16.4 us)
     const bool rest = head != M && !(rest_goes_along && M <= 2048 && ceil_div(head, (int64_t)(middle ? 128 : 256)) == ceil_div(M, (int64_t)(middle ? 128 : 256)));
     const double two = two_passes_us(M, N, K), with_rest = panels + (rest ? 4.5 : 0.0);
-    return middle ? two < (rest ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 0.95 : 1.07) * with_rest;
+    return middle ? two < (rest ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 1.05 : 1.12) * with_rest;
   });
 }
 static bool room_for_two_passes(int64_t N, int64_t K, const void* workspace, int64_t workspace_bytes) {
@@ -762,7 +771,7 @@ static bool room_for_two_passes(int64_t N, int64_t K, const void* workspace, int
 // on average (4907 x 256 x 2048 38.9 -> 16.8 us), one of them 3 % behind.
 static bool two_passes_beat_tiles(int64_t M, int64_t N, int64_t K) {
   static thread_local PlanTable<bool> known;
-  return M > 512 && N % 8 == 0 && known.get(M, N, K, 0, [&] { return two_passes_us(M, N, K) < 0.9 * fused_tile_us(M, N, K); });
+  return M > 512 && N % 8 == 0 && known.get(M, N, K, 0, [&] { return two_passes_us(M, N, K) < fused_tile_us(M, N, K); });
 }
 
 // Above 512 rows: does the streaming kernel beat the panel kernels (their estimates are 13 - 19 % high, see above; a row count that is no
@@ -779,9 +788,10 @@ static bool stream_beats_panels(int64_t M, int64_t N, int64_t K, int64_t group, 
     // (without room for the two passes it is the tile kernel that would run: 1.05 x its estimate in one round of tiles, 1.2 - 1.3 x in two, 1.4 x beyond; by an
     // estimate of passes that cannot run 2308 x 1328 x 4224 took 80 us in the tile kernel for 44 here; 1138 random calls that either moves 1.22 x on average)
     double other = fused_tile_us(M, N, K) * (two_passes || (tiles <= cus_now && K <= 512) ? 1.0 : tiles <= cus_now ? 1.05 : tiles <= 2 * cus_now ? 1.25 : 1.4);
-    if (two_passes && N % 8 == 0) other = two_passes_us(M, N, K);
-    // (short rows in one round of 128 x 128 tiles: the tile kernel, 3388 x 384 x 384 8.5 against 9.9 us)
-    if (K <= 512 && tiles <= cus_now && fused_tile_us(M, N, K) < other) other = fused_tile_us(M, N, K);
+    if (two_passes && N % 8 == 0) other = 1.04 * two_passes_us(M, N, K);
+    // (short rows in one round of 128 x 128 tiles: the tile kernel, 3388 x 384 x 384 8.5 against 9.9 us, 2816 x 1792 x 128 7.1 against 9.2, which its estimate is
+    // some 10 % above)
+    if (K <= 512 && tiles <= cus_now && 0.9 * fused_tile_us(M, N, K) < other) other = 0.9 * fused_tile_us(M, N, K);
     const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
     const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
     double panels = 1e30;
