@@ -181,3 +181,16 @@ result = log(lambda: lib.tlq_gemm_f16_batched(A, W, C, {B}, {M}, {N}, {K}, 0, 0,
 def test_two_passes_or_one_kernel(recorder, M, N, K, group, kernel):
     rc, text, error = ask(recorder, W4A16 + f"result = w4a16({M}, {N}, {K}, {group}, 1 << 32)")
     assert rc == 0 and kernel in text and "dequant" not in text, (text, error)
+
+
+# (bfloat16, groups, the workspace asked for; the sizes at which the GPU test of these rows compares results)
+@pytest.mark.parametrize("M,N,K,group,kernels", [(1002, 8960, 1152, 64, ["w4a16_panel256"]), (1023, 8960, 1152, 64, ["w4a16_panel256"]), (2209, 14224, 1536, 128, ["w4a16_panel256"]),
+                                                 (601, 11008, 4096, 128, ["w4a16_panelm"]), (639, 11008, 4096, 128, ["w4a16_panelm"]),
+                                                 (641, 11008, 4096, 128, ["w4a16_panelm", "gemv"]), (839, 6144, 2048, 64, ["w4a16_stream"]), (641, 7936, 4224, 128, ["w4a16_stream"]),
+                                                 (590, 1664, 5120, 128, ["w4a16_stream", "reduce"]), (1207, 1024, 6144, 64, ["w4a16_stream", "reduce"])])
+def test_which_kernel_takes_the_last_rows(recorder, M, N, K, group, kernels):
+    """The last one to three rows lie in a tile of the kernel that takes the others, each kernel without and with K slices, or have a launch of their own."""
+    ws = _abi.load().tlq_w4a16_workspace_bytes(M, N, K)
+    rc, text, error = ask(recorder, W4A16 + f"result = w4a16({M}, {N}, {K}, {group}, {ws})")
+    launches = text.split(" + ")
+    assert rc == 0 and len(launches) == len(kernels) and all(k in l for k, l in zip(kernels, launches)), (text, error)
