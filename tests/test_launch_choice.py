@@ -175,9 +175,10 @@ result = log(lambda: lib.tlq_gemm_f16_batched(A, W, C, {B}, {M}, {N}, {K}, 0, 0,
     assert rc == 0 and "[gemm_mfma_kernel" in text, (text, error)
 
 
-# A full workspace: the kernel named against the two passes, measured 12.9 / 19.9, 11.1 / 16.0, 9.1 / 12.9, 13.7 / 18.6, 12.6 / 17.2, 21.0 / 30.7 us
+# A full workspace: the kernel named against the two passes, measured 12.9 / 19.9, 11.1 / 16.0, 9.1 / 12.9, 13.7 / 18.6, 12.6 / 17.2, 21.0 / 30.7, 101.7 / 104.3, 204 / 229 us
 @pytest.mark.parametrize("M,N,K,group,kernel", [(564, 3328, 1280, 128, "w4a16_stream"), (872, 512, 2688, 128, "w4a16_small"), (875, 320, 2048, 256, "w4a16_small"),
-                                                (864, 512, 3328, 64, "w4a16_small"), (1086, 5376, 384, 128, "w4a16_stream"), (2872, 384, 3328, 64, "w4a16_stream")])
+                                                (864, 512, 3328, 64, "w4a16_small"), (1086, 5376, 384, 128, "w4a16_stream"), (2872, 384, 3328, 64, "w4a16_stream"),
+                                                (4096, 4096, 4096, 128, "w4a16_panel256"), (2816, 10752, 4096, 128, "w4a16_panel256")])
 def test_two_passes_or_one_kernel(recorder, M, N, K, group, kernel):
     rc, text, error = ask(recorder, W4A16 + f"result = w4a16({M}, {N}, {K}, {group}, 1 << 32)")
     assert rc == 0 and kernel in text and "dequant" not in text, (text, error)

@@ -726,8 +726,9 @@ static bool panel256_fills(int64_t M, int64_t N, int64_t K, int64_t group) {
 // one to three rows to a launch of their own (639 x 5680 x 896 29.2 -> 22.6 us, 7671 x 512 x 3200 49.0 -> 35.9).  With the plain GEMM's tiles between
 // 128 x 128 and 256 x 256 the two passes are ahead of the 256-row kernel on all but 17 of 163 random problems that either takes (M 513 .. 8192, N 256 ..
 // 14336, K 256 .. 14336, groups of 64 and 128, both types): those of fewer than 1024 rows and more than 2000 values, and a few of one partial round.
-// The panel kernels' estimates are 1.21 x high (12 % rms) short of 1.38 PFLOP/s (4096^3 100.5 us, 101.4 in the two passes), that of the two passes within 10 %; the choice by them, with the bars
-// below, is 0.5 % behind the faster of the two.  (The middle-M kernel's bars are those that the tests of the choice ask for, 1003 x 2048 x 4096 in groups of 64
+// The 256-row kernel's time against its estimate / 1.21, or 1.38 PFLOP/s: 1.05 (8 % rms) on 420 random problems and 1.07 on 264 of round sizes (M 768 .. 8192, N 1024 .. 14336), 7 % less
+// of it without a tensor of zero points where K is long; that of the two passes 1.0 (7 %).  With the bars below the choice is 0.5 % behind the faster of the two on either set
+// (4096^3 bf16, scalar zero point, 101.7 - 104.9 us here, 104.3 - 107.9 in the two passes; with a tensor 111.6 and 103.2).  (The middle-M kernel's bars are those that the tests of the choice ask for, 1003 x 2048 x 4096 in groups of 64
 // 35 us in a launch for 1000 rows and one for three, 29 in the two passes.)  Where neither panel kernel would run, all rows go through the two passes and none is left over.
 static double plain_nk_us(int64_t M, int64_t N, int64_t K);
 static bool tiles_beat_slices(TileKind tile, int kind, int64_t M, int64_t N, int64_t K, int64_t k_bytes);
@@ -740,9 +741,9 @@ static double two_passes_us(int64_t M, int64_t N, int64_t K) {
   const bool ring = c.variant >= kGroup128x128 && c.variant <= kGroup64x64;
   return ring ? 2.7 + 0.31e-6 * (double)N * (double)K + 1.19 * c.us : 4.6 + 0.645e-6 * (double)N * (double)K + 0.93 * c.us;
 }
-static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group, bool rest_goes_along) {
+static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t group, bool rest_goes_along, bool zero_points) {
   static thread_local PlanTable<bool> known;
-  return known.get(M, N, K, group * 2 + rest_goes_along, [&] {
+  return known.get(M, N, K, group * 4 + rest_goes_along * 2 + zero_points, [&] {
     const int64_t cus_now = cu_count_or_default(), head = M & ~(int64_t)3;
     const PanelMPlan pm = w4a16_panelm_plan(head, N, K, group, (int)cus_now);
     const Panel2Plan p2 = w4a16_panel256_plan(head, N, K, group, (int)cus_now);
@@ -761,7 +762,7 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
     // it moves are 1 - 13 % slower; up to 2048 rows 10 of 11 are faster, 1.01 - 1.18 x, 518 x 7440 x 1024 24.5 -> 16.4 us)
     const bool rest = head != M && !(rest_goes_along && M <= 2048 && ceil_div(head, (int64_t)(middle ? 128 : 256)) == ceil_div(M, (int64_t)(middle ? 128 : 256)));
     const double two = two_passes_us(M, N, K), with_rest = panels + (rest ? 4.5 : 0.0);
-    return middle ? two < (rest ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 1.05 : 1.12) * with_rest;
+    return middle ? two < (rest ? 0.9 : 1.0) * with_rest : two < (M <= 1024 ? 1.05 : zero_points || K <= 512 ? 1.13 : 1.08) * with_rest;
   });
 }
 static bool room_for_two_passes(int64_t N, int64_t K, const void* workspace, int64_t workspace_bytes) {
@@ -1039,7 +1040,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // (the estimate first: it is kept per shape, the choice among the others is not and takes 1.8 us of host time)
   if (M > 512 && stream_region && (stream_region = g_stream_tiles > 0 || stream_beats_panels(M, N, K, group, two_passes_fit))) {
     const int64_t head = M & ~(int64_t)3;
-    const bool two = two_passes_fit && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
+    const bool two = two_passes_fit && N % 8 == 0 && (two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16, zeros != nullptr) || !(panelm_estimate_wins(head, N, K, group) || panel256_fills(head, N, K, group)));
     stream_region = two ? N % 128 == 0 && N > 256 : !head_and_tail;
   }
   if (stream_region) {
@@ -1067,7 +1068,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
       return rows_behind_done(rc, rows != M);
     }
   }
-  if (head_and_tail && (keep_tail || !(two_passes_fit && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16)))) {
+  if (head_and_tail && (keep_tail || !(two_passes_fit && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16, zeros != nullptr)))) {
     const int64_t head = M & ~(int64_t)3;
     const bool may_go_along = in_dtype == TLQ_BF16;
     g_rows_behind = may_go_along ? M - head : 0;
@@ -1248,7 +1249,7 @@ int tlq_gemm_w4a16_ws(const void* A, const void* w_packed, const void* scales, c
   // 1.50 - 1.56 x), 0.98 - 0.99 on a few of the largest fp16 problems -- and 2 - 21 % behind below that fill (N = K = 4096,
   // M <= 1024: 96 work-groups).  The 128-row kernel is ahead of it nowhere by more than 4 % and stays an explicit choice.
   if (algo == TLQ_ALGO_AUTO && !g_w4a16_panel && M > 512 && K > 0 && group > 0 && N >= 1 && N < kMaxDim && K < kMaxDim && M < kMaxDim &&
-      !(have && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16))) {
+      !(have && two_passes_beat_panels(M, N, K, group, in_dtype == TLQ_BF16, zeros != nullptr))) {
     // The middle-M kernel's 128-row tiles first where an estimate of both kernels' times says so: rounds of work-groups x
     // (steps per K slice x the time of a step + a fixed part) + the pass over the slices' partial tiles, with the step
     // times measured at a full machine (2.2 us on 128 rows, 3.3 us on 256) and fixed parts of 6 / 8 us.  On ten (N, K)
