@@ -104,9 +104,10 @@ int tlq_debug_gemv_rows_plan(int64_t batch, int64_t N, int64_t K, int64_t group,
  * tlq_debug_check_gemv_ring_addressing walks, on the host, every load of the first, middle and last work-groups of such a
  * launch (bounds of every global read and LDS write, coverage of the staging data and of the rows, ring order against the
  * kernel's wait counts); 0 = consistent.  No counterpart in the reference. */
-/* Output tile (128 or 256, square) the MFMA GEMMs take for `batch` problems of M x N outputs on the current device (256 CUs
- * when there is none): by machine fill, see tlq_tune_gemm_tile.  fused = 1: the fused W4A16 tile kernel's rule.  Host only;
- * no counterpart in the reference (its block_M / block_N are arguments, example_dequant_gemm_fine_grained.py:437). */
+/* Output tile (128 or 256, square) by machine fill, for `batch` problems of M x N outputs on the current device (256 CUs when there is none).  fused = 0: the
+ * rule of the kernels whose weights pass through registers (16-bit [K, N] with N % 8 != 0, W4A8 unpacked into LDS) and of K slices added by atomics; the other
+ * plain products go by tlq_debug_gemm_choice.  fused = 1: that of the fused W4A16 tile kernel.  Host only; no counterpart in the reference (its block_M / block_N are arguments,
+ * example_dequant_gemm_fine_grained.py:437). */
 int tlq_debug_gemm_tile(int64_t batch, int64_t M, int64_t N, int fused);
 int tlq_debug_gemv_ring_plan(int64_t M, int64_t N, int64_t K, int64_t group, int cus, void* plan_out);
 int tlq_debug_check_gemv_ring_addressing(int64_t M, int64_t N, int64_t K, int64_t group, int rows_per_block, int waves, int depth);

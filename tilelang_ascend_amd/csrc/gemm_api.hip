@@ -768,8 +768,8 @@ static bool two_passes_beat_panels(int64_t M, int64_t N, int64_t K, int64_t grou
 static bool room_for_two_passes(int64_t N, int64_t K, const void* workspace, int64_t workspace_bytes) {
   return N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && workspace != nullptr && workspace_bytes >= N * K * 2 && aligned16(workspace);
 }
-// Many rows on up to 2^19 weights: the two passes or the tile kernel in one launch.  27 problems above 512 rows where that ran: 13 go to the two passes, 1.28 x
-// on average (4907 x 256 x 2048 38.9 -> 16.8 us), one of them 3 % behind.
+// Many rows on up to 2^19 weights: the two passes or the tile kernel in one launch (4907 x 256 x 2048 16.8 against 38.9 us).  By the estimate before this one, at 0.9, 13 of 27
+// problems above 512 rows went to the two passes, 1.28 x on average, one of them 3 % behind; 112 calls between a bar of 0.9 and this one are 1.17 x faster in them.
 static bool two_passes_beat_tiles(int64_t M, int64_t N, int64_t K) {
   static thread_local PlanTable<bool> known;
   return M > 512 && N % 8 == 0 && known.get(M, N, K, 0, [&] { return two_passes_us(M, N, K) < fused_tile_us(M, N, K); });

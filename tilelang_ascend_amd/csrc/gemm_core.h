@@ -987,6 +987,8 @@ extern thread_local int g_gemm_band_rows;
 // a launch with 128 of them leaves half the machine idle.  Fill = tiles / (rounds x CUs); the small tiles are taken
 // when their fill, weighted by 0.72, beats the large tiles' (measured on fifteen shapes: every choice this rule makes
 // was the faster one, e.g. M = 2048, N = 4096: 248 against 322 us; M = 3072, N = 4096: 99 (large) against 111 us).
+// The rule of the kernels whose weights pass through registers, of K slices added by atomics and of the fused W4A16 tile kernel; the other products have more
+// kernels to choose from (tile_choice below).
 inline double tile_fill(int64_t batch, int64_t M, int64_t N, int64_t tile) {
   int cus = tlq_device_cu_count();
   if (cus <= 0) cus = 256;
