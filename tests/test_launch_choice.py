@@ -116,6 +116,18 @@ result = log(lambda: lib.tlq_gemm_w4a16_layout_ws(A, W, S, None, C, {M}, {N}, {K
         assert rc == 1 and "workspace" in error, error
 
 
+# One group per row, written out per 128 values: the room for that is in the built-in scratch array where it holds the least workspace that the shape can use, and
+# that size follows the plan with the fewer slices (51.8 MiB for the first, 69.0 by the other plan), and of two the one that cuts at all.
+@pytest.mark.parametrize("M,N,K,most", [(376, 12032, 18816, 54288384), (458, 10192, 11648, 56015232), (407, 9376, 9344, 45792384)])
+def test_least_workspace_counts_the_plan_with_the_fewer_slices(recorder, M, N, K, most):
+    assert 0 < _abi.load().tlq_w4a16_workspace_bytes_min(M, N, K) <= most
+    rc, text, error = ask(recorder, f"""
+lib.tlq_gemm_w4a16_noalloc.argtypes = [p] * 5 + [i64] * 4 + [f32] + [i32] * 3 + [p]
+result = log(lambda: lib.tlq_gemm_w4a16_noalloc(A, W, S, WS, C, {M}, {N}, {K}, {K}, 8.0, 1, 1, 0, None))
+""")
+    assert rc == 0 and "w4a16_stream_kernel" in text, (text, error)
+
+
 # (bfloat16, groups of 64; a workspace too small for the dequantised weights, and none)
 @pytest.mark.parametrize("M,N,K", [(2308, 1328, 4224), (2174, 1152, 3840), (2528, 2688, 4608), (4020, 576, 3584), (1059, 2416, 4736), (926, 1888, 3328), (565, 1040, 640)])
 def test_calls_without_room_for_the_two_passes_are_not_decided_by_them(recorder, M, N, K):

@@ -425,13 +425,18 @@ int tlq_gemm_w4a16(const void* A, const void* w_packed, const void* scales, cons
 // N = 14336, K = 4096 and 20-40 % ahead from there on and for N = 4096, K = 14336)
 static const int64_t kTwoPassMinM = 256;
 
-// most K slices the streaming kernel cuts for any group size (the smallest group allows the shortest slices)
-static int64_t stream_max_split(int64_t M, int64_t N, int64_t K) {
+// most K slices the streaming kernel cuts for any group size (the smallest group allows the shortest slices).  least: those of the plan of short windows where it cuts
+// fewer, since a call whose workspace does not hold the best plan's runs by it (stream_plan_for), or where the best one does not cut at all: a size that no kernel
+// asks for would be that of the two passes then, and keep callers with less from the scratch that the rows' own scales want
+static int64_t stream_max_split(int64_t M, int64_t N, int64_t K, bool least = false) {
   int64_t most = 0;
   for (int64_t group = 32; group <= K; group *= 2) {
     if (K % group) continue;
     const StreamPlan p = w4a16_stream_plan(M, N, K, group, cu_count_or_default());  // (the count the launch plans with)
-    if (p.ok && p.split > most) most = p.split;
+    int64_t split = p.ok ? p.split : 0;
+    if (least && p.ok)
+      if (const StreamPlan other = w4a16_stream_plan(M, N, K, group, cu_count_or_default(), true); other.ok && (other.split < split || split == 1)) split = other.split;
+    if (split > most) most = split;
   }
   return most;
 }
@@ -461,7 +466,7 @@ static int plain_gemm_on_workspace(const void* A, void* workspace, int64_t works
 // most slices); 0 when none of them cuts K
 static int64_t w4a16_partial_sum_bytes(int64_t M, int64_t N, int64_t K, bool least = false) {
   int64_t split = w4a16_mid_split(M, N, K, 32);
-  const int64_t ssplit = M > 512 ? 0 : (least ? stream_max_split(M, N, K) : stream_promised_split(M, N, K));
+  const int64_t ssplit = M > 512 ? 0 : (least ? stream_max_split(M, N, K, true) : stream_promised_split(M, N, K));
   if (ssplit > split) split = ssplit;
   if (M <= 32) {  // the decode kernel cuts rows longer than 4096 values into chunks
     const DecodePlan dp = w4a16_decode_plan(M, N, K, 32, cu_count_or_default());
